@@ -5,19 +5,24 @@
 One shared object, `csrc/libmobula_hip.so`, holds the runtime and every
 operator's entry points.  It stays in the source tree (next to the code that
 loads it).  Replaces the per-call JIT of the reference
-(mobula/building/build.py:64-146) with one explicit hipcc invocation.
+(mobula/building/build.py:64-146) with one explicit hipcc invocation.  A second
+one, `csrc/_torch_direct.so` (host code only), is the bundled operators' way from
+torch tensors into that library; it is built where torch is installed.
 """
 import glob
+import importlib.util
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 from .config import config
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, 'csrc')
 LIB_PATH = os.path.join(CSRC, 'libmobula_hip.so')
+TORCH_LIB_PATH = os.path.join(CSRC, '_torch_direct.so')
 
 
 def sources():
@@ -67,6 +72,35 @@ def build_library(verbose=False):
     return LIB_PATH
 
 
+def build_torch_direct(verbose=False):
+    """The torch side (csrc/torch_direct.cpp) against the launcher library; None where
+    torch is not installed."""
+    if importlib.util.find_spec('torch') is None:
+        return None
+    torch_dir = os.path.dirname(importlib.util.find_spec('torch').origin)
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(shutil.which(config.HIPCC) or '/opt/rocm/bin/hipcc')))
+    tmp = TORCH_LIB_PATH + '.tmp.{}'.format(os.getpid())
+    cmd = (['g++', '-O2', '-std=c++17', '-fPIC', '-shared', '-Wall',
+            # how torch's own headers ask for the ROCm build they are part of
+            '-D__HIP_PLATFORM_AMD__=1', '-DUSE_ROCM=1',
+            '-I' + os.path.join(_HERE, '..', 'include'), '-I' + sysconfig.get_paths()['include'],
+            '-I' + os.path.join(torch_dir, 'include'),
+            '-I' + os.path.join(torch_dir, 'include', 'torch', 'csrc', 'api', 'include'),
+            '-I' + os.path.join(rocm, 'include'), '-o', tmp, os.path.join(CSRC, 'torch_direct.cpp'),
+            '-L' + CSRC, '-lmobula_hip', '-L' + os.path.join(torch_dir, 'lib'), '-lc10', '-lc10_hip', '-ltorch_cpu',
+            '-ltorch_python', '-Wl,-rpath,$ORIGIN'])
+    if verbose or config.SHOW_BUILDING_COMMAND:
+        print(' '.join(cmd), flush=True)
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if proc.returncode != 0:
+        if os.path.exists(tmp):
+            os.remove(tmp)
+        raise RuntimeError('g++ failed:\n' + proc.stdout)
+    os.replace(tmp, TORCH_LIB_PATH)
+    return TORCH_LIB_PATH
+
+
 if __name__ == '__main__':
     print(build_library(verbose=True))
+    print(build_torch_direct(verbose=True))
     sys.exit(0)

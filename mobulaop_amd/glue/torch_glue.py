@@ -13,8 +13,9 @@ import ctypes
 
 import torch
 
-from .common import (MobulaTensor, INPUT_FUNCS, assign, get_in_data, get_in_shape,
+from .common import (CUSTOM_OP_LIST, MobulaTensor, INPUT_FUNCS, assign, get_in_data, get_in_shape,
                      get_varnames)
+from .. import native
 from ..dtype import c_bfloat16, c_half
 
 # int32 / float32 / float64 are the reference's (mobula/glue/torch_glue.py:6-9); the
@@ -131,7 +132,16 @@ class OpGen(object):
         if self.name not in self.cache:
             self.cache[self.name] = self.register()
         inputs, (ctor_args, ctor_kwargs) = get_in_data(op=self.op, *args, **kwargs)
+        self._offer_direct_call(inputs)
         return self.cache[self.name](*ctor_args, **ctor_kwargs)(*inputs)
+
+    def _offer_direct_call(self, inputs):
+        """From the first call on GPU tensors on, an operator class that names a native call
+        (`torch_direct`) is asked for through it: see csrc/torch_direct.cpp."""
+        name, handle = getattr(self.op, 'torch_direct', None), CUSTOM_OP_LIST.get(self.name)
+        if (name is not None and handle is not None and getattr(handle.op, 'torch_direct', None) == name and
+                not handle.attrs and handle.direct is None and any(t.is_cuda for t in inputs)):
+            handle.direct = getattr(native.torch_direct(), name)
 
     def register(self):
         return _make_module(self.op, self.name, _make_function(self.op, self.name))

@@ -14,6 +14,7 @@ There is no CPU implementation behind this module: if the library is missing
 (and cannot be built) every call raises.
 """
 import ctypes
+import importlib.util
 import os
 
 from .config import config
@@ -68,6 +69,30 @@ def set_option(name, value):
 
 def get_option(name):
     return int(library().mobula_hip_get_option(name.encode()))
+
+
+_torch_direct = None
+
+
+def torch_direct():
+    """The module that takes the bundled operators' calls on torch GPU tensors straight to
+    the library (csrc/torch_direct.cpp); builds it first if it is absent and can be."""
+    global _torch_direct
+    if _torch_direct is None:
+        library()   # (the module is linked against it)
+        from . import build as _build
+        if not os.path.exists(_build.TORCH_LIB_PATH):
+            _build.build_torch_direct()
+        import torch  # noqa: F401  (its libraries have to be loaded first)
+        spec = importlib.util.spec_from_file_location('_torch_direct', _build.TORCH_LIB_PATH)
+        try:
+            module = importlib.util.module_from_spec(spec)
+        except ImportError as exc:
+            raise RuntimeError('cannot load {}: {} -- build it with `python -m mobulaop_amd.build`'.format(
+                _build.TORCH_LIB_PATH, exc))
+        spec.loader.exec_module(module)
+        _torch_direct = module
+    return _torch_direct
 
 
 def symbol(name):

@@ -39,6 +39,7 @@ def _nhwc(t):
 @mobula.op.register
 class ROIAlign:
     follows_channels_last = True   # the torch glue allocates y in the memory format of data
+    torch_direct = 'ROIAlign'      # calls on torch GPU tensors go straight to the library
 
     def __init__(self, pooled_size, spatial_scale, sampling_ratio):
         self.pooled_size = pooled_size

@@ -199,3 +199,55 @@ def test_double_tensors_through_the_operator(mobula):
     out = np.zeros((3, 3, 4, 4))
     mobula.func.roi_align_forward(out.size, xh, 0.25, 3, 12, 14, 4, 4, 0, rh, out)
     np.testing.assert_array_equal(out, oracle.forward_f64(xh, rh, (4, 4), 0.25, 0))
+
+
+@pytest.mark.parametrize('form', ['plain', 'channels_last', 'transposed', 'channels_last_odd', 'one_bin'])
+def test_direct_calls_agree_with_the_operator_class(mobula, form):
+    """Calls on torch GPU tensors go straight to the library; the operator class gives the same values,
+    formats and gradients (also for strided maps, expanded gradients and boxes that want one)."""
+    torch.manual_seed(7)
+    C, pooled = (6, (3, 5)) if form == 'channels_last_odd' else (8, (1, 1) if form == 'one_bin' else (3, 5))
+    x = torch.randn(2, C, 12, 9, device='cuda')
+    if form.startswith('channels_last') or form == 'one_bin':
+        x = x.contiguous(memory_format=torch.channels_last)
+    elif form == 'transposed':
+        x = x.transpose(2, 3)
+    rois = torch.tensor([[0, 1, 2, 30, 20], [1, -4, 3, 25, 40], [1, 8, 8, 9, 9]], device='cuda', dtype=torch.float32)
+    rois.requires_grad_(True)
+    kw = dict(pooled_size=pooled, spatial_scale=0.25, sampling_ratio=2)
+    handle, results = mobula.op.ROIAlign, []
+    handle(x, rois, **kw)
+    direct = handle.direct
+    assert direct is not None
+    for call in (direct, None):
+        handle.direct = call
+        xi = x.detach().requires_grad_(True)
+        y = handle(data=xi, rois=rois, **kw)
+        results.append((y,) + torch.autograd.grad((2 * y).sum(), (xi, rois)))
+    handle.direct = direct
+    for a, b in zip(*results):
+        assert a.stride() == b.stride() and torch.equal(a, b)
+
+
+@pytest.mark.parametrize('bias,image_grad', [(True, True), (False, True), (True, False)])
+def test_direct_convolution_agrees_with_the_operator_class(mobula, bias, image_grad):
+    mobula.op.load('Convolution')
+    torch.manual_seed(8)
+    x = torch.randn(2, 5, 9, 7, device='cuda').contiguous(memory_format=torch.channels_last)
+    w = torch.randn(6, 5, 3, 2, device='cuda', requires_grad=True)
+    b = torch.randn(6, device='cuda', requires_grad=True)
+    x.requires_grad_(image_grad)
+    inputs = [x, w] + ([b] if bias else [])
+    wanted = [t for t in inputs if t.requires_grad]
+    handle, results = mobula.op.Conv2D, []
+    kw = dict(channels=6, kernel_size=(3, 2), strides=(2, 1), padding=(1, 0), dilation=(1, 2))
+    handle(*inputs, **kw)
+    direct = handle.direct
+    assert direct is not None
+    for call in (direct, None):
+        handle.direct = call
+        y = handle(*inputs, **kw)
+        results.append((y,) + torch.autograd.grad(y, wanted, torch.ones_like(y).expand_as(y)))
+    handle.direct = direct
+    for a, b in zip(*results):
+        assert a.stride() == b.stride() and torch.equal(a, b)
