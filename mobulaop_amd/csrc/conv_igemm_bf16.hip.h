@@ -26,9 +26,9 @@
 // per matrix instruction, half of what 128 x 128 tiles need.
 //
 // Operands go from memory straight into LDS (buffer loads with the LDS flag,
-// 16 bytes per lane: one instruction moves sixteen 64-byte rows), three stages
-// deep: while step s is multiplied, step s + 1 has landed or is landing and
-// step s + 2 is requested.  No register staging, no LDS store instructions.
+// 16 bytes per lane: one instruction moves sixteen 64-byte rows), three or four
+// stages deep: while step s is multiplied, the steps up to the last stage but one
+// have landed or are landing and the next one is requested.  No register staging, no LDS store instructions.
 // A column in the padding loads from beyond the buffer, which writes zeros.
 // LDS rows are 64 bytes with no padding; the four 16-byte chunks of row r sit
 // in slots chunk ^ ((r >> 2) & 3), which puts the 16-byte fragment reads of
@@ -49,7 +49,7 @@
 namespace conv {
 
 struct TileB16 {
-  static constexpr int BN = 256, BK = 32, STAGES = 3;
+  static constexpr int BN = 256, BK = 32;
 };
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
@@ -470,20 +470,32 @@ __device__ __forceinline__ void wait_for_loads_but() {
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
 }
 
+// The barrier alone.  __syncthreads() would also wait for every load in flight (they write LDS),
+// and with them for the stages that are only wanted steps later; what has to have landed is
+// counted by wait_for_loads_but().  No memory access moves across it.
+__device__ __forceinline__ void workgroup_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 __host__ __device__ inline int k_steps_b16(int K) { return (K + TileB16::BK - 1) / TileB16::BK; }
 
 // A tile of ROWS x COLS results and the WAVES wavefronts that share it, each NI x NJ fragments of
 // 32 x 32.  A stage in LDS always has room for 256 columns.
-template <int ROWS_, int COLS_, int WAVES_, int NI_>
+template <int ROWS_, int COLS_, int WAVES_, int NI_, int STAGES_>
 struct ShapeB16 {
-  static constexpr int ROWS = ROWS_, COLS = COLS_, WAVES = WAVES_, NI = NI_;
+  static constexpr int ROWS = ROWS_, COLS = COLS_, WAVES = WAVES_, NI = NI_, STAGES = STAGES_;
   static constexpr int WM = ROWS / (32 * NI), WN = WAVES / WM;   // wavefronts down and across the tile
   static constexpr int NJ = COLS / WN / 32;
   static_assert(WM * NI * 32 == ROWS && WN * NJ * 32 == COLS && COLS <= TileB16::BN, "the wavefronts cover the tile");
   static constexpr int STAGE_HALVES = (ROWS + TileB16::BN) * TileB16::BK;
 };
-typedef ShapeB16<256, 256, 8, 4> WideShapeB16;     // 2 x 4 wavefronts of 128 x 64: two to a SIMD
-typedef ShapeB16<128, 256, 4, 4> LowShapeB16;      // 1 x 4 wavefronts of 128 x 64, for products of at most 128 rows
+// Stages of a tile in LDS: four where a CU holds one workgroup anyway (128 KB), so that a step's
+// operands are requested three steps ahead (forward + backward at 32 x 256 x 56 x 56, 3 x 3: 537 us
+// with three stages and a full wait per step, 521 so); three where two workgroups share a CU.
+typedef ShapeB16<256, 256, 8, 4, 4> WideShapeB16;  // 2 x 4 wavefronts of 128 x 64: two to a SIMD
+typedef ShapeB16<128, 256, 4, 4, 3> LowShapeB16;   // 1 x 4 wavefronts of 128 x 64, for products of at most 128 rows
 
 // C[M, Ncols] = A[M, K] x B[K, Ncols], the tile of shape S at (m0, n0) over the K steps
 // s_begin .. s_end - 1 (s_begin < s_end).  piece == nullptr: results go through ops.store;
@@ -495,7 +507,7 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
   constexpr int ROWS = S::ROWS, WAVES = S::WAVES, NI = S::NI, NJ = S::NJ, WN = S::WN;
   constexpr int A_LOADS = ROWS / 16 / WAVES, B_LOADS = T::BN / 16 / WAVES, LOADS = A_LOADS + B_LOADS;
   constexpr int STAGE = S::STAGE_HALVES;
-  __shared__ __attribute__((aligned(1024))) unsigned short lds[T::STAGES * STAGE];
+  __shared__ __attribute__((aligned(1024))) unsigned short lds[S::STAGES * STAGE];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = (wave / WN) * (32 * NI), wn = (wave % WN) * (32 * NJ);   // the wavefront's part of the tile
 
@@ -533,7 +545,7 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
   auto step_requested = [&]() {
     ops.advance(cur);
     ++s_issue;
-    stage_issue = stage_issue + 1 == T::STAGES ? 0 : stage_issue + 1;
+    stage_issue = stage_issue + 1 == S::STAGES ? 0 : stage_issue + 1;
   };
 
   float16v acc[NI][NJ];
@@ -580,18 +592,18 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
   //                stage s + 1
   constexpr int SLOTS = NI * NJ, ITEMS = LOADS + READS;   // products of a half step; what the second half issues besides
 #pragma unroll
-  for (int k = 0; k < T::STAGES - 1; ++k) {
+  for (int k = 0; k < S::STAGES - 1; ++k) {
 #pragma unroll
     for (int q = 0; q < LOADS; ++q) request(q);
     step_requested();
   }
-  wait_for_loads_but<(T::STAGES - 2) * LOADS>();
+  wait_for_loads_but<(S::STAGES - 2) * LOADS>();
   __syncthreads();
   int stage = 0;
 #pragma unroll
   for (int k = 0; k < READS; ++k) read_fragment(0, 0, k);
   for (int s = s_begin; s < s_end; ++s) {
-    const int next = stage + 1 == T::STAGES ? 0 : stage + 1;
+    const int next = stage + 1 == S::STAGES ? 0 : stage + 1;
 #pragma unroll
     for (int k = 0; k < SLOTS; ++k) {
       multiply(0, k);
@@ -599,8 +611,8 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
       for (int q = k * READS / SLOTS; q < (k + 1) * READS / SLOTS; ++q) read_fragment(stage, 1, q);
       __builtin_amdgcn_sched_barrier(0);
     }
-    wait_for_loads_but<(T::STAGES - 3) * LOADS>();
-    __syncthreads();
+    wait_for_loads_but<(S::STAGES - 3) * LOADS>();
+    workgroup_barrier();
 #pragma unroll
     for (int k = 0; k < SLOTS; ++k) {
       multiply(1, k);
