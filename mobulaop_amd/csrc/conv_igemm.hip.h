@@ -576,34 +576,61 @@ igemm_weight_kernel(BackwardWeightOps ops, int k_per_slice, int k_total, int row
                                       k_steps(ops.K), StoreResult<BackwardWeightOps>{ops, nullptr});
 }
 
-// out[i] (+)= sum over slices of partial[s][i]
+// out[i] (+)= sum over slices of partial[s][i].  `groups` (a power of two) threads share an output: each
+// adds a contiguous run of slices, the runs are added in order.  V: outputs per thread (one 16-byte load
+// per slice for four).
+template <int V>
 __global__ void __launch_bounds__(256)
 reduce_slices_kernel(const float* __restrict__ partial, float* __restrict__ out, long long count,
-                     int slices, int accumulate) {
-  const long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
+                     int slices, int groups, int accumulate) {
+  typedef float vec __attribute__((ext_vector_type(V)));
+  __shared__ vec sums[256];
+  const int per_block = 256 / groups, local = threadIdx.x % per_block, group = threadIdx.x / per_block;
+  const long long i = (static_cast<long long>(blockIdx.x) * per_block + local) * V;
+  const int run = (slices + groups - 1) / groups, z0 = group * run, z1 = min(slices, z0 + run);
+  vec s = 0.0f;
+  if (i < count) {
+#pragma unroll 8
+    for (int z = z0; z < z1; ++z) s += *reinterpret_cast<const vec*>(partial + static_cast<long long>(z) * count + i);
+  }
+  if (groups > 1) {
+    sums[threadIdx.x] = s;
+    __syncthreads();
+    if (group != 0) return;
+    for (int q = 1; q < groups; ++q) s += sums[q * per_block + local];
+  }
   if (i >= count) return;
-  float s = 0.0f;
-  for (int z = 0; z < slices; ++z) s += partial[static_cast<long long>(z) * count + i];
-  out[i] = accumulate ? out[i] + s : s;
+  vec* const to = reinterpret_cast<vec*>(out + i);
+  *to = accumulate ? *to + s : s;
 }
 
-// db[d] (+)= sum over images and pixels of dy[img, d, :, :]; one workgroup per filter.
+// sums[part][d] (+)= sum of dy[img, d, :, :] over the images of the part (img = part, part + parts, ...);
+// grid (filters, parts).  V: pixels per load.
+template <int V>
 __global__ void __launch_bounds__(256)
-bias_grad_kernel(const float* __restrict__ dy, float* __restrict__ db, int N, int D, int ohw, int accumulate) {
+bias_grad_kernel(const float* __restrict__ dy, float* __restrict__ sums, int N, int D, int ohw, int accumulate) {
+  typedef float vec __attribute__((ext_vector_type(V)));
   __shared__ float part[256];
   const int d = blockIdx.x;
-  float s = 0.0f;
-  for (int img = 0; img < N; ++img) {
+  vec v = 0.0f;
+  for (int img = blockIdx.y; img < N; img += gridDim.y) {
     const float* p = dy + (static_cast<size_t>(img) * D + d) * ohw;
-    for (int i = threadIdx.x; i < ohw; i += 256) s += p[i];
+#pragma unroll 4
+    for (int i = threadIdx.x * V; i < ohw; i += 256 * V) v += *reinterpret_cast<const vec*>(p + i);
   }
+  float s = 0.0f;
+#pragma unroll
+  for (int k = 0; k < V; ++k) s += v[k];
   part[threadIdx.x] = s;
   __syncthreads();
   for (int off = 128; off > 0; off >>= 1) {
     if (threadIdx.x < off) part[threadIdx.x] += part[threadIdx.x + off];
     __syncthreads();
   }
-  if (threadIdx.x == 0) db[d] = accumulate ? db[d] + part[0] : part[0];
+  if (threadIdx.x == 0) {
+    float* const to = sums + static_cast<size_t>(blockIdx.y) * D + d;
+    *to = accumulate ? *to + part[0] : part[0];
+  }
 }
 
 // The reference's unfold and fold (opzoo/Convolution/Convolution.cpp:13-90), one

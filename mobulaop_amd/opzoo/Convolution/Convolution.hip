@@ -8,10 +8,12 @@
 // (opzoo/Convolution/Convolution.py:17-57), computed on the matrix cores
 // without a column buffer.
 #include <algorithm>
+#include <vector>
 
 #include "runtime.h"
 #include "conv_igemm.hip.h"
 #include "conv_igemm_bf16.hip.h"
+#include "conv_patch_f32.hip.h"
 
 namespace {
 
@@ -136,6 +138,8 @@ void launch_igemm_b16(const Ops& ops, float* piece_buffer, hipStream_t stream) {
 
 // workgroups the weight gradient aims at: four per CU of a 256-CU device
 constexpr long long kWeightSlots = 1024;
+
+size_t align_to_256(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
 int blocks_for(long long n) { return static_cast<int>(std::min<long long>((n + 255) / 256, 256ll * 32)); }
 // (for kernels that take one element per thread and do not stride)
@@ -280,6 +284,361 @@ bool plan_gather_b16(conv::GatheredB16* ops, float** pieces, const char* what, c
   return true;
 }
 
+// ---- fp32 products from patches (conv_patch_f32.hip.h) -----------------------
+
+constexpr size_t kLdsOfCu = 160 * 1024;
+
+// Workgroups of `kernel` the device holds at a time, with `lds` bytes of dynamic LDS each.
+template <typename Kernel>
+int resident_with_lds(Kernel* kernel, size_t lds) {
+  static thread_local int cached_device = -1, cached = 0;
+  static thread_local size_t cached_lds = 0;
+  static thread_local Kernel* cached_kernel = nullptr;
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess) return 0;
+  if (device != cached_device || lds != cached_lds || kernel != cached_kernel) {
+    int per_cu = 0, cus = 0;
+    const void* const f = reinterpret_cast<const void*>(kernel);
+    if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kLdsOfCu)) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, 256, lds) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
+      (void)hipGetLastError();
+      return 0;
+    }
+    cached = per_cu * cus;
+    cached_device = device; cached_lds = lds; cached_kernel = kernel;
+  }
+  return cached;
+}
+
+// A product of the forward form: what PatchOps and ArrangePatchArgs describe, before the choice of
+// tiles and chunks.
+struct PatchProduct {
+  conv::PatchOps ops;
+  conv::ArrangePatchArgs arrange;
+};
+
+// How a tile's patch is cut: rows of the patch, columns per image, channels per chunk.
+struct PatchCut { int rows, npx, cc; size_t lds; double cost; };
+
+// Rows a tile of BN columns needs at most.  Columns are numbered through all images (a tile may
+// cross into the next one, which costs the patch another image's margin rows), or every image's
+// are padded to whole tiles.
+template <typename T>
+PatchCut cut_patch(const conv::PatchOps& o, int taps, bool crossing) {
+  const long long pix = static_cast<long long>(o.Ho) * o.Wo;
+  const bool aligned = T::BN % o.Wo == 0, inside = o.Wo % T::BN == 0 && !crossing;
+  const int nr = aligned ? T::BN / o.Wo : inside ? 1 : (T::BN - 2) / o.Wo + 2;
+  PatchCut cut{};
+  cut.npx = static_cast<int>(crossing ? pix : (pix + T::BN - 1) / T::BN * T::BN);
+  cut.rows = (std::min(nr, o.Ho) - 1) * o.sh + o.reach;
+  if (crossing) {
+    const int q = static_cast<int>(std::min<long long>({(T::BN - 2) / pix + 2, o.N, nr}));
+    // (linear in the number of images a tile meets: two of them, or as many as fit)
+    for (const int k : {std::min(2, q), q}) cut.rows = std::max(cut.rows, (nr - k) * o.sh + k * o.reach);
+  }
+  const long long plane = static_cast<long long>(cut.rows) * o.pitch;
+  cut.cost = -1.0;
+  if (plane >= (1 << 16)) return cut;
+  for (int j = 1; j <= std::min(o.C, 256); ++j) {
+    const int cc = (o.C + j - 1) / j, chunks = (o.C + cc - 1) / cc, sub = (cc * taps + 15) / 16;
+    const size_t lds = conv::patch_lds_bytes<T>(chunks > 1 ? 2 : 1, plane * cc, static_cast<int>(plane), sub * 16);
+    if (lds > kLdsOfCu || (chunks > 1 && sub < 2)) continue;   // (the next patch is loaded a step behind the chunk's first)
+    // clocks of a K step: the matrix instructions of a wavefront (64 clocks each, 2048 with two rows of
+    // fragments) and what they do not hide -- measured with two workgroups to a CU: 10 % and 250
+    // clocks, 30 for every piece of the patch; one workgroup to a CU hides less
+    const double loads = static_cast<double>(cc) * ((plane + 63) / 64) / sub;
+    const double step = T::NI * 1126.0 + 250.0 + 30.0 * loads + (2 * lds > kLdsOfCu ? 700.0 : 0.0);
+    const double cost = step * sub * chunks * ((static_cast<double>(o.N) * cut.npx + T::BN - 1) / T::BN);
+    if (cut.cost < 0 || cost < cut.cost) { cut.cost = cost; cut.cc = cc; cut.lds = lds; }
+  }
+  return cut;
+}
+
+// The cheaper of the two ways to number columns; false: neither fits LDS.
+template <typename T>
+bool cut_product(const PatchProduct& p, PatchCut* cut) {
+  const int taps = p.arrange.KHp * p.arrange.KWp;
+  const PatchCut a = cut_patch<T>(p.ops, taps, true), b = cut_patch<T>(p.ops, taps, false);
+  if (a.cost < 0 && b.cost < 0) return false;
+  *cut = b.cost >= 0 && (a.cost < 0 || b.cost < a.cost) ? b : a;
+  return true;
+}
+
+template <typename T>
+size_t product_bytes(const PatchProduct& p, const PatchCut& cut, int* mpad, int* sub) {
+  const int taps = p.arrange.KHp * p.arrange.KWp, chunks = (p.ops.C + cut.cc - 1) / cut.cc;
+  *mpad = (p.ops.M + T::BM - 1) / T::BM * T::BM;
+  *sub = (cut.cc * taps + 15) / 16;
+  return align_to_256(sizeof(float) * 16ull * *sub * chunks * *mpad) + align_to_256(sizeof(int) * 16ull * *sub);
+}
+
+template <typename T>
+void launch_product(PatchProduct p, const PatchCut& cut, char* at, float* pieces, hipStream_t stream) {
+  int mpad = 0, sub = 0;
+  const size_t bytes = product_bytes<T>(p, cut, &mpad, &sub);
+  conv::PatchOps& o = p.ops;
+  conv::ArrangePatchArgs& a = p.arrange;
+  o.npx = cut.npx; o.cols = o.N * cut.npx; o.mpad = mpad; o.cc = cut.cc; o.sub = sub;
+  o.chunks = (o.C + cut.cc - 1) / cut.cc; o.plane = cut.rows * o.pitch;
+  float* const wp = reinterpret_cast<float*>(at);
+  int* const koff = reinterpret_cast<int*>(at + bytes - align_to_256(sizeof(int) * 16ull * sub));
+  o.wp = wp; o.koff = koff;
+  a.wp = wp; a.koff = koff; a.M = o.M; a.mpad = mpad; a.C = o.C; a.cc = o.cc; a.sub = sub; a.chunks = o.chunks;
+  a.plane = o.plane; a.pitch = o.pitch;
+  conv::arrange_patch_weights_kernel<<<blocks_for(16ll * sub * o.chunks * mpad), 256, 0, stream>>>(a);
+  const int row_tiles = mpad / T::BM, count = row_tiles * static_cast<int>((static_cast<long long>(o.cols) + T::BN - 1) / T::BN);
+  // tiles are cut along K at whole chunks where there are several (a piece loads whole patches)
+  const int unit = o.chunks > 1 ? sub : 1, steps = o.chunks * sub;
+  conv::TileSplit split = split_tiles(count, steps / unit, resident_with_lds(conv::patch_kernel<T>, cut.lds));
+  split.steps_per_piece *= unit;
+  const int rest = count - split.whole;
+  const dim3 grid(conv::tile_blocks(split.whole) + rest * split.pieces);
+  conv::patch_kernel<T><<<grid, T::NT, cut.lds, stream>>>(o, row_tiles, split, pieces);
+  if (rest > 0)
+    conv::reduce_patch_pieces_kernel<T><<<rest * (T::BM * T::BN / 256), 256, 0, stream>>>(o, row_tiles, split, pieces);
+}
+
+// The tiles of a product by its number of rows; f<T>(cut) if a cut of T fits, else false.
+template <typename T, typename F>
+bool with_cut(const PatchProduct& p, const F& f) {
+  PatchCut cut{};
+  int mpad = 0, sub = 0;
+  return cut_product<T>(p, &cut) && product_bytes<T>(p, cut, &mpad, &sub) < (1ull << 31) && f(cut, T());
+}
+template <typename F>
+bool with_tiles(const PatchProduct& p, const F& f) {
+  const conv::PatchOps& o = p.ops;
+  const long long image = static_cast<long long>(o.C) * o.Hs * o.Ws, pix = static_cast<long long>(o.Ho) * o.Wo;
+  // a tile's columns span this many images at most; their byte offsets must stay below 2^31
+  if ((256 / std::max<long long>(pix, 1) + 2) * image * 4 >= (1ll << 31)) return false;
+  if (static_cast<long long>(o.N) * (pix + 256) >= (1ll << 31)) return false;
+  if (o.M > 64) return with_cut<conv::PatchTile128>(p, f);
+  if (o.M > 32) return with_cut<conv::PatchTile64>(p, f);
+  return with_cut<conv::PatchTile32>(p, f);
+}
+
+// Clocks of a K step of igemm_kernel (three workgroups to a CU, whole tiles of 128 x 128).
+constexpr double kGatherStep = 2750.0;
+
+// CU clocks of the product from patches; < 0: it does not fit.
+double patch_product_cost(const PatchProduct& p) {
+  double cost = -1.0;
+  with_tiles(p, [&](const PatchCut& cut, auto tiles) {
+    typedef decltype(tiles) T;
+    cost = cut.cost * ((p.ops.M + T::BM - 1) / T::BM);
+    return true;
+  });
+  return cost;
+}
+
+// CU clocks of a gathered product of M rows over `channels` (conv_igemm.hip.h: K steps of sixteen
+// channels of one tap).
+double gathered_product_cost(int M, int channels, int taps, long long columns) {
+  return kGatherStep * taps * ((channels + 15) / 16) * ((M + conv::Tile::BM - 1) / conv::Tile::BM) *
+         ((columns + conv::Tile::BN - 1) / conv::Tile::BN);
+}
+
+// One product of the forward form (patch_product_cost said that it fits).
+void run_patch_product(const PatchProduct& p, hipStream_t stream) {
+  with_tiles(p, [&](const PatchCut& cut, auto tiles) {
+    typedef decltype(tiles) T;
+    int mpad = 0, sub = 0;
+    const size_t bytes = product_bytes<T>(p, cut, &mpad, &sub);
+    const size_t piece_bytes = sizeof(float) * kMaxPieceBlocks * conv::Tile::BM * conv::Tile::BN;
+    char* const ws = static_cast<char*>(mobula_hip::workspace(bytes + piece_bytes));
+    if (!failed()) launch_product<T>(p, cut, ws, reinterpret_cast<float*>(ws + bytes), stream);
+    return true;
+  });
+  MOBULA_HIP_TRY(hipGetLastError());
+}
+
+// A pointwise product without padding or strides reads pixel n for output pixel n: with the plane as
+// one column of pixels a tile's patch is exactly its columns.
+void flatten_pointwise(conv::PatchOps* o) {
+  if (o->reach != 1 || o->pitch != o->Wo || o->sh != 1 || o->sw != 1 || o->ph != 0 || o->pw != 0 || o->Hs != o->Ho ||
+      o->Ws != o->Wo || o->os_h != 1 || o->os_w != 1)
+    return;
+  o->Hs *= o->Ws; o->Ws = 1;
+  o->Ho *= o->Wo; o->Wo = 1;
+  o->out_h *= o->out_w; o->out_w = 1;
+  o->pitch = 1;
+}
+
+bool forward_from_patches(const conv::Geometry& g, const float* x, const float* weight, const float* bias, float* y,
+                          hipStream_t stream) {
+  PatchProduct p{};
+  p.ops = conv::PatchOps{x, nullptr, nullptr, bias, y, g.N, g.C, g.H, g.W, g.D, g.OH, g.OW, g.stride_h, g.stride_w,
+                         g.pad_h, g.pad_w, (g.KH - 1) * g.dil_h + 1, 0, 0, 0, 0, 0, 0, 0,
+                         (g.OW - 1) * g.stride_w + (g.KW - 1) * g.dil_w + 1, 0, g.OH, g.OW, 1, 1, 0, 0};
+  const long long taps = g.KH * g.KW;
+  p.arrange = conv::ArrangePatchArgs{weight, nullptr, nullptr, 0, 0, 0, 0, 0, 0, g.KH, g.KW, g.KW, 0, 1, 0, 1,
+                                     g.C * taps, taps, 0, 0, g.dil_h, g.dil_w};
+  flatten_pointwise(&p.ops);
+  // Patches win where a step of sixteen channels of one tap is mostly padding (few channels), where
+  // a tile of 128 rows is, and at strides; large layers of round sizes stay with the gathered tiles.
+  const double cost = patch_product_cost(p);
+  if (cost < 0 || cost > gathered_product_cost(g.D, g.C, g.KH * g.KW, static_cast<long long>(g.N) * g.OH * g.OW))
+    return false;
+  run_patch_product(p, stream);
+  return true;
+}
+
+// Filter taps k that reach the pixels of a class: (offset + pad - k * dil) % stride == 0.  They are
+// first, first + inc, ...: `count` of them; neighbours lie `step` source pixels apart, and pixel
+// i of the class reads source pixel i + shift for the first of them.
+struct TapsOfClass { int first, inc, count, step, shift; };
+TapsOfClass taps_of_class(int K, int dil, int stride, int pad, int offset) {
+  TapsOfClass t{0, 1, 0, 1, 0};
+  int common = dil, rest = stride;
+  while (rest != 0) { const int r = common % rest; common = rest; rest = r; }
+  t.inc = stride / common;
+  t.step = dil / common;
+  for (int k = 0; k < std::min(K, t.inc); ++k)
+    if ((offset + pad - k * dil) % stride == 0) {
+      t.first = k;
+      t.count = (K - 1 - k) / t.inc + 1;
+      t.shift = (offset + pad - k * dil) / stride;
+      break;
+    }
+  return t;
+}
+
+bool data_gradient_from_patches(const conv::Geometry& g, const float* dy, const float* weight, float* dx,
+                                int accumulate, hipStream_t stream) {
+  if (g.stride_h > g.H || g.stride_w > g.W || g.stride_h * g.stride_w > 16) return false;
+  const long long taps = g.KH * g.KW;
+  std::vector<PatchProduct> classes;
+  double cost = 0.0;
+  for (int a = 0; a < g.stride_h; ++a)
+    for (int b = 0; b < g.stride_w; ++b) {
+      const TapsOfClass th = taps_of_class(g.KH, g.dil_h, g.stride_h, g.pad_h, a);
+      const TapsOfClass tw = taps_of_class(g.KW, g.dil_w, g.stride_w, g.pad_w, b);
+      const int Ho = (g.H - 1 - a) / g.stride_h + 1, Wo = (g.W - 1 - b) / g.stride_w + 1;
+      if (th.count == 0 || tw.count == 0) continue;
+      // taps in reverse order walk forward over dy: the last one reads pixel i + shift - (count - 1) * step
+      PatchProduct p{};
+      p.ops = conv::PatchOps{dy, nullptr, nullptr, nullptr, dx, g.N, g.D, g.OH, g.OW, g.C, Ho, Wo, 1, 1,
+                             (th.count - 1) * th.step - th.shift, (tw.count - 1) * tw.step - tw.shift,
+                             (th.count - 1) * th.step + 1, 0, 0, 0, 0, 0, 0, 0, Wo + (tw.count - 1) * tw.step,
+                             accumulate, g.H, g.W, g.stride_h, g.stride_w, a, b};
+      p.arrange = conv::ArrangePatchArgs{weight, nullptr, nullptr, 0, 0, 0, 0, 0, 0, th.count, tw.count, g.KW,
+                                         th.first + (th.count - 1) * th.inc, -th.inc,
+                                         tw.first + (tw.count - 1) * tw.inc, -tw.inc, taps, g.C * taps, 0, 0,
+                                         th.step, tw.step};
+      flatten_pointwise(&p.ops);
+      const double product = patch_product_cost(p);
+      if (product < 0) return false;
+      cost += product;
+      classes.push_back(p);
+    }
+  if (cost > gathered_product_cost(g.C, g.D, g.KH * g.KW, static_cast<long long>(g.N) * g.H * g.W)) return false;
+  for (int a = 0; a < g.stride_h && !accumulate; ++a)
+    for (int b = 0; b < g.stride_w; ++b) {
+      if (taps_of_class(g.KH, g.dil_h, g.stride_h, g.pad_h, a).count != 0 &&
+          taps_of_class(g.KW, g.dil_w, g.stride_w, g.pad_w, b).count != 0)
+        continue;
+      const int Ho = (g.H - 1 - a) / g.stride_h + 1, Wo = (g.W - 1 - b) / g.stride_w + 1;
+      const long long count = static_cast<long long>(g.N) * g.C * Ho * Wo;
+      conv::zero_class_kernel<<<blocks_for(count), 256, 0, stream>>>(dx, count, g.H, g.W, Ho, Wo, g.stride_h, g.stride_w,
+                                                                     a, b);
+    }
+  for (const PatchProduct& p : classes)
+    if (!failed()) run_patch_product(p, stream);
+  return true;
+}
+
+// Weight gradient from patches: how its chunks are cut; cost < 0: it does not fit.
+struct WeightCut { int px, plane, channels; size_t lds; double cost; };
+template <typename T>
+WeightCut cut_weight(const conv::Geometry& g) {
+  const int taps = g.KH * g.KW, ohw = g.OH * g.OW, pitch = (g.OW - 1) * g.stride_w + (g.KW - 1) * g.dil_w + 1;
+  const int reach = (g.KH - 1) * g.dil_h + 1;
+  WeightCut best{0, 0, 0, 0, -1.0};
+  if (g.W >= (1 << 16)) return best;
+  const int channels = std::min(g.C, (T::BN - 1) / taps + 2);
+  for (int px = 32; px <= 512 && px < ohw + 32; px += 16) {
+    const int nr = std::min(g.OH, px % g.OW == 0 ? px / g.OW : g.OW % px == 0 ? 1 : (px - 2) / g.OW + 2);
+    const long long plane = static_cast<long long>((nr - 1) * g.stride_h + reach) * pitch;
+    if (plane >= (1 << 15)) break;
+    const size_t lds = conv::patch_lds_bytes<T>(2, plane * channels, static_cast<int>(plane), 2 * px);
+    if (lds > kLdsOfCu) break;
+    const double loads = static_cast<double>(channels) * ((plane + 63) / 64);
+    // (as in cut_patch; the right operand's reads meet bank conflicts)
+    const double chunk = px / 16 * (T::NI * 1126.0 + 550.0 + (2 * lds > kLdsOfCu ? 700.0 : 0.0)) + 30.0 * loads;
+    const double cost = chunk * ((ohw + px - 1) / px);
+    if (best.cost < 0 || cost < best.cost) best = WeightCut{px, static_cast<int>(plane), channels, lds, cost};
+  }
+  return best;
+}
+
+void reduce_slices(const float* partial, float* out, long long count, int slices, int accumulate, hipStream_t stream) {
+  // groups of threads share an output's slices until the device has work; four outputs a thread
+  // where they lie on 16-byte boundaries
+  const int wide = count % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 ? 4 : 1;
+  int groups = 1;
+  while (groups < 32 && 2 * groups <= slices && count / wide * groups < 128 * 1024) groups *= 2;
+  const dim3 grid(static_cast<unsigned>((count / wide + 256 / groups - 1) / (256 / groups)));
+  if (wide == 4)
+    conv::reduce_slices_kernel<4><<<grid, 256, 0, stream>>>(partial, out, count, slices, groups, accumulate);
+  else
+    conv::reduce_slices_kernel<1><<<grid, 256, 0, stream>>>(partial, out, count, slices, groups, accumulate);
+}
+
+template <typename T>
+bool weight_gradient_with(const conv::Geometry& g, const float* dy, const float* x, int accumulate, float* dw,
+                          hipStream_t stream) {
+  const WeightCut cut = cut_weight<T>(g);
+  const int ohw = g.OH * g.OW, chunks_per_image = cut.cost < 0 ? 1 : (ohw + cut.px - 1) / cut.px;
+  // (planes that fill their chunks badly -- a few pixels -- go to the kernel whose K steps span images)
+  if (cut.cost < 0 || static_cast<long long>(chunks_per_image) * cut.px * 3 > 4ll * ohw) return false;
+  if (static_cast<long long>(g.D) * ohw * 4 >= (1ll << 31) || static_cast<long long>(g.N) * chunks_per_image >= (1ll << 31))
+    return false;
+  const int cols = g.C * g.KH * g.KW, row_tiles = (g.D + T::BM - 1) / T::BM;
+  const long long tiles = static_cast<long long>(row_tiles) * ((cols + T::BN - 1) / T::BN);
+  if (tiles >= (1ll << 20)) return false;
+  // CU clocks against those of igemm_weight_kernel: its steps span images and cost a little less,
+  // but it needs a padded copy of x at unit stride along a row, and tests every pixel at others
+  const double here = cut.cost * g.N * static_cast<double>(tiles);
+  const long long padded = static_cast<long long>(g.N) * g.C * (g.H + 2 * g.pad_h) * (g.W + 2 * g.pad_w);
+  const double there = (g.stride_w == 1 ? 2670.0 : 5000.0) * conv::k_steps(g.N * ohw) *
+                           ((g.D + conv::Tile::BM - 1) / conv::Tile::BM) * ((cols + conv::Tile::BN - 1) / conv::Tile::BN) +
+                       (g.stride_w == 1 ? 8.0 * padded / 4.5e12 * 2.4e9 * 256.0 : 0.0);
+  if (here > there) return false;
+  const int chunks = g.N * chunks_per_image;
+  const bool wide = ohw % 4 == 0;
+  const int resident = wide ? resident_with_lds(conv::patch_weight_kernel<T, true>, cut.lds)
+                            : resident_with_lds(conv::patch_weight_kernel<T, false>, cut.lds);
+  int slices = static_cast<int>(std::max<long long>(1, std::min<long long>(chunks, resident / tiles)));
+  const int per_slice = (chunks + slices - 1) / slices;
+  slices = (chunks + per_slice - 1) / per_slice;
+  const long long wt = static_cast<long long>(g.D) * cols;
+  char* const ws = static_cast<char*>(mobula_hip::workspace(sizeof(float) * slices * wt));
+  if (failed()) return true;
+  conv::PatchWeightOps o{dy, x, reinterpret_cast<float*>(ws), g.N, g.C, g.H, g.W, g.D, g.OH, g.OW, g.stride_h, g.stride_w,
+                         g.pad_h, g.pad_w, g.dil_h, g.dil_w, g.KH, g.KW, cols, cut.px, chunks_per_image, cut.channels,
+                         cut.plane, (g.OW - 1) * g.stride_w + (g.KW - 1) * g.dil_w + 1};
+  const int count = static_cast<int>(tiles) * slices;
+  const dim3 grid(conv::tile_blocks(count));
+  if (wide)
+    conv::patch_weight_kernel<T, true><<<grid, T::NT, cut.lds, stream>>>(o, per_slice, chunks, row_tiles,
+                                                                        static_cast<int>(tiles), count);
+  else
+    conv::patch_weight_kernel<T, false><<<grid, T::NT, cut.lds, stream>>>(o, per_slice, chunks, row_tiles,
+                                                                         static_cast<int>(tiles), count);
+  reduce_slices(o.partial, dw, wt, slices, accumulate, stream);
+  MOBULA_HIP_TRY(hipGetLastError());
+  return true;
+}
+
+bool weight_gradient_from_patches(const conv::Geometry& g, const float* dy, const float* x, int accumulate, float* dw,
+                                  hipStream_t stream) {
+  if (g.N == 0) return false;
+  if (g.D > 64) return weight_gradient_with<conv::PatchTile128>(g, dy, x, accumulate, dw, stream);
+  if (g.D > 32) return weight_gradient_with<conv::PatchTile64>(g, dy, x, accumulate, dw, stream);
+  return weight_gradient_with<conv::PatchTile32>(g, dy, x, accumulate, dw, stream);
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -361,6 +720,7 @@ MOBULA_KERNEL conv2d_forward_kernel(const int n, const T* x, const T* weight, co
   }
   {
     mobula_hip::KernelTimer timer("conv2d_forward", stream);
+    if (compute_mode() == conv::kFp32 && forward_from_patches(g, x, weight, ops.bias, y, stream)) return;
     GatherPlan plan;
     const long long taps = g.KH * g.KW;
     if (!plan_gather(&plan, "conv2d_forward", g, weight, g.D, g.C, static_cast<long long>(g.C) * g.H * g.W,
@@ -416,6 +776,7 @@ MOBULA_KERNEL conv2d_backward_data_kernel(const int n, const T* dy, const T* wei
   }
   {
     mobula_hip::KernelTimer timer("conv2d_backward_data", stream);
+    if (compute_mode() == conv::kFp32 && data_gradient_from_patches(g, dy, weight, dx, accumulate, stream)) return;
     GatherPlan plan;
     const long long taps = g.KH * g.KW;
     // row m of the left operand is input channel m: element [m][tap][d] = weight[d][m][tap]
@@ -510,6 +871,10 @@ MOBULA_KERNEL conv2d_backward_weight_kernel(const int n, const T* dy, const T* x
       return;
     }
   }
+  if (compute_mode() == conv::kFp32 && wt > 0) {
+    mobula_hip::KernelTimer timer("conv2d_backward_weight", stream);
+    if (weight_gradient_from_patches(g, dy, x, accumulate, dw, stream)) return;
+  }
   conv::BackwardWeightOps ops;
   ops.dy = dy; ops.x = x; ops.g = g;
   ops.M = g.D; ops.Ncols = g.C * g.KH * g.KW; ops.K = 0; ops.k_begin = 0;
@@ -558,7 +923,7 @@ MOBULA_KERNEL conv2d_backward_weight_kernel(const int n, const T* dy, const T* x
         conv::igemm_weight_kernel<conv::kFp32><<<grid, conv::Tile::NT, 0, stream>>>(
             ops, static_cast<int>(k_per_slice), static_cast<int>(k_total), row_tiles, tps, count);
     }
-    conv::reduce_slices_kernel<<<blocks_for(wt), 256, 0, stream>>>(ops.partial, dw, wt, static_cast<int>(slices), accumulate);
+    reduce_slices(ops.partial, dw, wt, static_cast<int>(slices), accumulate, stream);
   }
   MOBULA_HIP_TRY(hipGetLastError());
 }
@@ -572,7 +937,20 @@ MOBULA_KERNEL conv2d_backward_bias_kernel(const int n, const T* dy, const int ac
   if (!fits("conv2d_backward_bias", 1, static_cast<long long>(batch) * n * pixels) ||
       !fits("conv2d_backward_bias", 5, n))
     return;
-  conv::bias_grad_kernel<<<n, 256, 0, call_state().stream>>>(dy, db, batch, n, pixels, accumulate);
+  // planes of a filter dealt to as many workgroups as give the device about a thousand, their
+  // sums added in order by a second kernel (one workgroup per filter: 95 us for 64 filters of
+  // 8 x 112 x 112, the memory has 26 MB to give)
+  hipStream_t stream = call_state().stream;
+  const int parts = std::max(1, std::min(batch, 1024 / n));
+  const bool wide = pixels % 4 == 0 && reinterpret_cast<uintptr_t>(dy) % 16 == 0;
+  float* sums = db;
+  if (parts > 1) {
+    sums = static_cast<float*>(mobula_hip::workspace(sizeof(float) * static_cast<size_t>(parts) * n));
+    if (failed()) return;
+  }
+  (wide ? conv::bias_grad_kernel<4> : conv::bias_grad_kernel<1>)<<<dim3(n, parts), 256, 0, stream>>>(
+      dy, sums, batch, n, pixels, parts > 1 ? 0 : accumulate);
+  if (parts > 1) reduce_slices(sums, db, n, parts, accumulate, stream);
   MOBULA_HIP_TRY(hipGetLastError());
 }
 

@@ -421,3 +421,43 @@ def test_errors_surface_as_exceptions():
         native.end_call('conv2d_forward')
     # the library stays usable
     _call('conv2d_forward_c6a7aa85', ctypes.c_int(4), _ptr(x), _ptr(w), _ptr(w), ctypes.c_int(0), *geo, _ptr(y))
+
+
+@pytest.mark.parametrize('shape', [
+    # the fp32 kernels that stage patches of the map: tiles of 32, 64 and 128 rows, their edges, and what chunks,
+    # strides and image borders do to them  (N, C, H, W, D, kernel, pad, stride, dilation)
+    (2, 3, 40, 37, 64, (7, 7), (3, 3), (2, 2), (1, 1)),     # a first layer; planes that are no multiple of four
+    (9, 3, 5, 6, 65, (3, 3), (1, 1), (1, 1), (1, 1)),       # tiles span images; one row past a tile
+    (3, 1, 33, 64, 32, (5, 1), (2, 0), (1, 1), (1, 1)),     # one channel, rows that divide a tile
+    (2, 19, 24, 30, 33, (3, 3), (1, 1), (2, 3), (1, 1)),    # strides that differ: six classes of dx
+    (1, 40, 21, 26, 24, (3, 2), (2, 1), (3, 2), (2, 3)),    # dilation against stride: classes without taps
+    (2, 8, 16, 16, 130, (1, 1), (0, 0), (2, 2), (1, 1)),    # pointwise at a stride: three classes of dx are zero
+    (5, 33, 11, 11, 17, (1, 1), (0, 0), (1, 1), (1, 1)),    # pointwise, few rows
+    (1, 5, 60, 250, 40, (3, 9), (0, 4), (1, 1), (1, 1)),    # rows longer than a tile
+])
+def test_fp32_products_from_patches(shape):
+    N, C, H, W, D, kernel, pad, stride, dil = shape
+    g = torch.Generator().manual_seed(77)
+    x, w = torch.randn(N, C, H, W, generator=g), torch.randn(D, C, *kernel, generator=g)
+    b = torch.randn(D, generator=g)
+    xr, wr = x.double().requires_grad_(True), w.double().requires_grad_(True)
+    y_ref = F.conv2d(xr, wr, b.double(), stride=stride, padding=pad, dilation=dil)
+    dy = torch.randn(y_ref.shape, generator=g)
+    y_ref.backward(dy.double())
+    xd, wd, bd, dyd = x.cuda(), w.cuda(), b.cuda(), dy.cuda()
+    geo = _ci(N, C, H, W, D, kernel[0], kernel[1], pad[0], pad[1], stride[0], stride[1], dil[0], dil[1])
+    y = torch.full(y_ref.shape, float('nan'), device='cuda')
+    _call('conv2d_forward_c6a7aa85', ctypes.c_int(y.numel()), _ptr(xd), _ptr(wd), _ptr(bd), ctypes.c_int(1), *geo, _ptr(y))
+    _close(y, y_ref, 'y', 1e-5)
+    for start, accumulate in ((float('nan'), 0), (1.0, 1)):
+        dx, dw = torch.full(x.shape, start, device='cuda'), torch.full(w.shape, start, device='cuda')
+        _call('conv2d_backward_data_ecf81c91', ctypes.c_int(dx.numel()), _ptr(dyd), _ptr(wd), ctypes.c_int(accumulate),
+              *geo, _ptr(dx))
+        _call('conv2d_backward_weight_ecf81c91', ctypes.c_int(dw.numel()), _ptr(dyd), _ptr(xd), ctypes.c_int(accumulate),
+              *geo, _ptr(dw))
+        _close(dx - accumulate, xr.grad, 'dx', 1e-5)
+        _close(dw - accumulate, wr.grad, 'dw', 1e-5)
+    db = torch.empty(D, device='cuda')
+    _call('conv2d_backward_bias_cd239a08', ctypes.c_int(D), _ptr(dyd), ctypes.c_int(0), ctypes.c_int(N),
+          ctypes.c_int(y.shape[2] * y.shape[3]), _ptr(db))
+    _close(db, dy.double().sum((0, 2, 3)), 'db', 1e-5)
