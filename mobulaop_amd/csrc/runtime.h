@@ -12,6 +12,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <initializer_list>
 #include <string>
 #include <vector>
 
@@ -62,10 +63,17 @@ class DeviceScope {
   bool ok_ = true;
 };
 
-// Device mirrors of host buffers for calls that arrive with device id -1.
+// Device mirrors of host buffers for calls that arrive with device id -1 (host_copy.hip).  The
+// mirrors of a call lie in a grow-only block of the calling thread and device (of at most 1 GiB;
+// larger ones are allocated for the call), which release_staging() and the thread's end give back.
 class HostStaging {
  public:
+  HostStaging();
   ~HostStaging();
+  HostStaging(const HostStaging&) = delete;
+  HostStaging& operator=(const HostStaging&) = delete;
+  // Makes room for mirrors of these sizes (optional, before the first of them).
+  void reserve(std::initializer_list<size_t> sizes);
   // Device copy of `bytes` bytes at `host` (uploaded when `upload`).
   void* in(const void* host, size_t bytes, bool upload = true);
   // Device buffer that is downloaded to `host` by flush().
@@ -73,9 +81,12 @@ class HostStaging {
   bool flush(hipStream_t stream);  // download outputs, wait for completion
 
  private:
-  struct Item { void* dev; void* host; size_t bytes; bool download; };
+  struct Item { void* dev; void* host; size_t bytes; bool download, own; };
   std::vector<Item> items_;
+  size_t mark_ = 0;
+  bool unfinished_ = false;
 };
+void release_staging();   // frees the calling thread's block on the current device and the pinned ring
 
 // Every entry point starts a call with begin_call() -- the error text of the
 // thread's previous call is dropped, so an error is reported for the call that

@@ -174,35 +174,6 @@ DeviceScope::~DeviceScope() {
   if (changed_) (void)hipSetDevice(previous_);
 }
 
-HostStaging::~HostStaging() {
-  for (auto& it : items_) (void)hipFree(it.dev);
-}
-
-void* HostStaging::in(const void* host, size_t bytes, bool upload) {
-  void* dev = inout(const_cast<void*>(host), bytes, upload);
-  items_.back().download = false;
-  return dev;
-}
-
-void* HostStaging::inout(void* host, size_t bytes, bool upload) {
-  Item item{nullptr, host, bytes, true};
-  MOBULA_HIP_TRY(hipMalloc(&item.dev, bytes > 0 ? bytes : 1));
-  if (!failed() && upload && bytes > 0)
-    MOBULA_HIP_TRY(hipMemcpy(item.dev, host, bytes, hipMemcpyHostToDevice));
-  items_.push_back(item);
-  return item.dev;
-}
-
-bool HostStaging::flush(hipStream_t stream) {
-  MOBULA_HIP_TRY(hipStreamSynchronize(stream));
-  for (auto& it : items_) {
-    if (failed()) break;
-    if (it.download && it.bytes > 0)
-      MOBULA_HIP_TRY(hipMemcpy(it.host, it.dev, it.bytes, hipMemcpyDeviceToHost));
-  }
-  return !failed();
-}
-
 namespace {
 struct SideState { hipStream_t stream = nullptr; hipEvent_t fork = nullptr, join = nullptr; bool tried = false; };
 SideState& side_state(int device) {
@@ -361,6 +332,7 @@ double mobula_hip_last_kernel_ms(const char** name) {
 long long mobula_hip_workspace_bytes(void) { return mobula_hip::workspace_bytes(); }
 long long mobula_hip_release_workspace(void) {
   mobula_hip::begin_call();
+  mobula_hip::release_staging();
   return mobula_hip::release_workspace();
 }
 // The calling thread's workspace on the current device is no longer used by any recorded graph.

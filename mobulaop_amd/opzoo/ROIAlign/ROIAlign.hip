@@ -788,6 +788,7 @@ void forward_entry(int device_id, int nthreads, const T* x, B scale, int C, int 
     st.extents.assign(11, -1);
     st.extents[1] = p.N * C * H * W;
     mobula_hip::HostStaging stage;
+    stage.reserve({sizeof(T) * p.N * C * H * W, sizeof(B) * 5 * p.R, sizeof(T) * p.n_out});
     const T* dx = static_cast<const T*>(stage.in(x, sizeof(T) * p.N * C * H * W));
     const B* dr = static_cast<const B*>(stage.in(rois, sizeof(B) * 5 * p.R));
     T* dy = static_cast<T*>(stage.inout(y, sizeof(T) * p.n_out, /*upload=*/false));
@@ -826,6 +827,7 @@ void backward_entry(int device_id, int nthreads, const T* dy, B scale, int C, in
                              PW, S, e_map, e_rois, 1, assign ? num_images : -1)) {
     if (p.N < 0) p.N = host_images(rois, p.R, (1ll << 31) / (static_cast<long long>(C) * H * W));
     mobula_hip::HostStaging stage;
+    stage.reserve({sizeof(T) * p.n_out, sizeof(B) * 5 * p.R, sizeof(T) * p.N * C * H * W});
     const T* ddy = static_cast<const T*>(stage.in(dy, sizeof(T) * p.n_out));
     const B* dr = static_cast<const B*>(stage.in(rois, sizeof(B) * 5 * p.R));
     T* ddx = static_cast<T*>(stage.inout(dx, sizeof(T) * p.N * C * H * W, /*upload=*/!assign));

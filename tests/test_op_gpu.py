@@ -251,3 +251,36 @@ def test_direct_convolution_agrees_with_the_operator_class(mobula, bias, image_g
     handle.direct = direct
     for a, b in zip(*results):
         assert a.stride() == b.stride() and torch.equal(a, b)
+
+
+@pytest.mark.parametrize('shape', [(1, 3, 8, 9), (2, 64, 90, 91), (3, 256, 100, 120)])   # one copy; a few pieces; rounds of the ring
+def test_host_arrays_of_several_sizes_and_from_several_threads(mobula, shape):
+    """Arrays in host memory go through pinned slots in pieces: every element arrives, also when threads
+    use the ring at once and after its memory was given back."""
+    import threading
+    from mobulaop_amd import native
+    rng = np.random.default_rng(3)
+    N, C, H, W = shape
+    rois = np.array([[n % N, 3 * n % 40, 5, 3 * n % 40 + 30.5, 60] for n in range(100)], dtype=np.float32)
+    kw = dict(pooled_size=(7, 7), spatial_scale=0.5, sampling_ratio=2)
+    x = rng.random(shape, dtype=np.float32)
+    dy = rng.standard_normal((100, C, 7, 7), dtype=np.float32)
+    xt = torch.from_numpy(x).cuda().requires_grad_(True)
+    yt = mobula.op.ROIAlign(xt, torch.from_numpy(rois).cuda(), **kw)
+    yt.backward(torch.from_numpy(dy).cuda())
+    wrong = []
+
+    def work():
+        op = mobula.op.ROIAlign[np.ndarray](**kw)
+        for _ in range(2):
+            y = op(x, rois)
+            dx, _ = op.backward(dy)
+            if not (np.array_equal(y, yt.detach().cpu().numpy()) and np.array_equal(dx, xt.grad.cpu().numpy())):
+                wrong.append(1)
+            native.release_workspace()
+    threads = [threading.Thread(target=work) for _ in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
