@@ -78,7 +78,7 @@ __global__ void __launch_bounds__(FwdMerged::NW * 64, 4)
 forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
                       const int* __restrict__ order, T* __restrict__ y, float scale, int C, int H,
                       int W, int PH, int PW, int S, long long num_images, int cblk,
-                      int rows_per_pass, int R) {
+                      int rows_per_pass, int rois_listed, int parts) {
   using K = FwdBlocked;
   using M = FwdMerged;
   constexpr int CPL = BlockOf<T>::CPL, CB = BlockOf<T>::CB, STAGE = BlockOf<T>::STAGE_MERGED;
@@ -94,6 +94,8 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
   auto uni_i = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
   auto uni_f = [](float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); };
   // job decode: as in forward_blocked_kernel
+  // (with few ROIs the pooled rows of one are dealt to `parts` wavefronts, neighbours in this order)
+  const int R = rois_listed * parts;
   const int xcd = blockIdx.x & 7;
   const long long wi = static_cast<long long>(blockIdx.x >> 3) * M::NW + wave;
   long long slot;
@@ -118,6 +120,9 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
     slot = part * range + wi;
   }
   if (slot >= R) return;
+  const int ph_first = static_cast<int>(slot % parts) * ((PH + parts - 1) / parts);
+  const int ph_end = min(PH, ph_first + (PH + parts - 1) / parts);
+  slot /= parts;
   const int roi = uni_i(order != nullptr ? order[slot] : static_cast<int>(slot));   // no order: as listed
   const int c0 = cb * CB, nch = min(CB, C - c0);
   const int grp = lane >> 3, quad = lane & 7;
@@ -178,8 +183,8 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
     }
   };
 
-  for (int ph0 = 0; ph0 < PH; ph0 += rows_per_pass) {
-    const int rp = min(rows_per_pass, PH - ph0), seg = rp * PW;
+  for (int ph0 = ph_first; ph0 < ph_end; ph0 += rows_per_pass) {
+    const int rp = min(rows_per_pass, ph_end - ph0), seg = rp * PW;
     for (int pwb = 0; pwb < PW; pwb += K::PWB) {
       const int pw = pwb + grp;
       const bool bin_on = pw < PW && quad_on;

@@ -172,65 +172,103 @@ __device__ __forceinline__ WindowCount count_windows(const RoiGeom& g, int PH, i
   return c;
 }
 
-// Window items, step 1: counts[r] = windows of ROI r (-1: its grid has more than kMergedGrid
-// points along an axis), work[r] = an upper bound of the work entries of its items.
-__global__ void __launch_bounds__(256)
-window_counts_kernel(const float* __restrict__ rois, int R, float scale, int PH, int PW, int S, int H, int W,
-                     int tw, int* __restrict__ counts, long long* __restrict__ work) {
-  for (long long r = blockIdx.x * 256ll + threadIdx.x; r < R; r += 256ll * gridDim.x) {
-    const RoiGeom g = roi_geometry(rois + r * 5, scale, PH, PW, S);
-    if (g.grid_h > kMergedGrid || g.grid_w > kMergedGrid || g.grid_h < 1 || g.grid_w < 1) {
-      counts[r] = -1;
-      work[r] = 0;
-      continue;
-    }
-    const WindowCount c = count_windows(g, PH, PW, H, W, tw);
-    counts[r] = c.windows;
-    work[r] = static_cast<long long>(c.windows) * c.tiles_x * c.taps;
-  }
+// Windows of ROI r (-1: its grid has more than kMergedGrid points along an axis) and an upper
+// bound of the work entries of its items.
+__device__ __forceinline__ int windows_of_roi(const float* __restrict__ rois, long long r, float scale, int PH, int PW,
+                                              int S, int H, int W, int tw, long long* work) {
+  const RoiGeom g = roi_geometry(rois + r * 5, scale, PH, PW, S);
+  *work = 0;
+  if (g.grid_h > kMergedGrid || g.grid_w > kMergedGrid || g.grid_h < 1 || g.grid_w < 1) return -1;
+  const WindowCount c = count_windows(g, PH, PW, H, W, tw);
+  *work = static_cast<long long>(c.windows) * c.tiles_x * c.taps;
+  return c.windows;
 }
 
-// Step 2: offsets[r] = number of the first window item of ROI r, offsets[R] = their total
-// (offsets may be the array of counts: every thread reads its share before any writes);
-// info[0] = the total, info[1] = 1 if some ROI's grid is too large to merge (the caller
-// then takes another path), info[2] = an upper bound of the work entries of all items
-// (saturating at 2^30).  One workgroup of 1024 threads.
+struct WindowArgs { const float* rois; int R; float scale; int PH, PW, S, H, W, tw; };
+
+// Window items, step 1 (many ROIs): their counts and work bounds, one thread per ROI.
+__global__ void __launch_bounds__(256)
+window_counts_kernel(WindowArgs a, int* __restrict__ counts, long long* __restrict__ work) {
+  for (long long r = blockIdx.x * 256ll + threadIdx.x; r < a.R; r += 256ll * gridDim.x)
+    counts[r] = windows_of_roi(a.rois, r, a.scale, a.PH, a.PW, a.S, a.H, a.W, a.tw, &work[r]);
+}
+
+// Up to this many ROIs are counted by the workgroup that adds the counts up: one launch less.
+constexpr int kCountedInOffsets = 2048;
+
+// Step 2: offsets[r] = number of the first window item of ROI r, offsets[R] = their total;
+// told[0] = the total, told[1] = 1 if some ROI's grid is too large to merge (the caller then takes
+// another path), told[2] = an upper bound of the work entries of all items (saturating at 2^30),
+// told[3] = ticket, written last: `told` is pinned host memory that the calling thread watches.
+// One workgroup of 1024 threads; every thread reads its share of the counts before any writes
+// (offsets may be that array).
 __global__ void __launch_bounds__(1024)
-window_offsets_kernel(const int* __restrict__ counts, const long long* __restrict__ work, int R,
-                      int* __restrict__ offsets, int* __restrict__ info) {
-  __shared__ int part[1024];
-  __shared__ long long entries[1024];
+window_offsets_kernel(WindowArgs a, const int* __restrict__ counts, const long long* __restrict__ work,
+                      int* __restrict__ offsets, volatile int* told, int ticket) {
+  __shared__ int part[16];
+  __shared__ long long entries[16];
   __shared__ int too_big;
-  const int t = threadIdx.x, share = (R + 1023) / 1024;
-  const int first = min(R, t * share), last = min(R, first + share);
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, share = (a.R + 1023) / 1024;
+  const int first = min(a.R, t * share), last = min(a.R, first + share);
+  const bool counted = a.R > kCountedInOffsets;
   if (t == 0) too_big = 0;
   __syncthreads();
+  int few[kCountedInOffsets / 1024];
   int sum = 0;
   long long all = 0;
-  for (int r = first; r < last; ++r) {
-    const int c = counts[r];
+  auto take = [&](int c, long long w) {
     if (c < 0) too_big = 1;
     sum += max(c, 0);
-    all += work[r];
+    all += w;
+  };
+  if (counted) {
+    for (int r = first; r < last; ++r) take(counts[r], work[r]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < kCountedInOffsets / 1024; ++k) {
+      few[k] = 0;
+      if (first + k < last) {
+        long long w = 0;
+        few[k] = windows_of_roi(a.rois, first + k, a.scale, a.PH, a.PW, a.S, a.H, a.W, a.tw, &w);
+        take(few[k], w);
+      }
+    }
   }
-  part[t] = sum;
-  entries[t] = all;
-  __syncthreads();
-  if (t == 0) {   // exclusive prefix over the threads
-    int run = 0;
-    long long total = 0;
-    for (int i = 0; i < 1024; ++i) { const int c = part[i]; part[i] = run; run += c; total += entries[i]; }
-    offsets[R] = run;
-    info[0] = run;
-    info[1] = too_big;
-    info[2] = static_cast<int>(min(total, 1ll << 30));
+  int upto = sum;   // inclusive sum over the wavefront's lanes
+  for (int off = 1; off < 64; off <<= 1) {
+    const int up = __shfl_up(upto, off);
+    if (lane >= off) upto += up;
+    all += __shfl_xor(all, off);
   }
+  if (lane == 63) { part[wave] = upto; entries[wave] = all; }
   __syncthreads();
-  int at = part[t];
-  for (int r = first; r < last; ++r) {
-    const int c = max(counts[r], 0);
-    offsets[r] = at;
-    at += c;
+  int at = upto - sum;
+  for (int w = 0; w < wave; ++w) at += part[w];
+  if (counted) {
+    for (int r = first; r < last; ++r) {
+      const int c = max(counts[r], 0);
+      offsets[r] = at;
+      at += c;
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < kCountedInOffsets / 1024; ++k)
+      if (first + k < last) {
+        offsets[first + k] = at;
+        at += max(few[k], 0);
+      }
+  }
+  if (t == 1023) {
+    offsets[a.R] = at;
+    if (told != nullptr) {
+      long long total = 0;
+      for (int w = 0; w < 16; ++w) total += entries[w];
+      told[0] = at;
+      told[1] = too_big;
+      told[2] = static_cast<int>(min(total, 1ll << 30));
+      __threadfence_system();
+      told[3] = ticket;
+    }
   }
 }
 

@@ -1,6 +1,7 @@
 // See runtime.h.
 #include "runtime.h"
 
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -151,6 +152,44 @@ void unpin_workspace() {
 long long workspace_bytes() {
   Scratch* const s = scratch_of_current_device();
   return s == nullptr ? 0 : static_cast<long long>(s->bytes);
+}
+
+namespace {
+struct MailboxOfThread {
+  Mailbox box;
+  ~MailboxOfThread() {
+    if (box.words != nullptr) (void)hipHostFree(box.words);
+  }
+};
+}  // namespace
+
+Mailbox* mailbox() {
+  static thread_local MailboxOfThread mine;
+  if (mine.box.words == nullptr) {
+    void* p = nullptr;
+    MOBULA_HIP_TRY(hipHostMalloc(&p, 64, hipHostMallocPortable | hipHostMallocCoherent));
+    if (!failed()) {
+      std::memset(p, 0, 64);
+      mine.box.words = static_cast<int*>(p);
+    }
+  }
+  return &mine.box;
+}
+
+bool wait_for_mail(Mailbox* box, hipStream_t stream) {
+  const volatile int* const words = box->words;
+  for (unsigned spins = 0; words[3] != box->ticket; ++spins) {
+    __builtin_ia32_pause();
+    if (spins % 4096 != 4095) continue;
+    // (the stream has nothing left to do, or has failed: the mail is there, or will never be)
+    const hipError_t state = hipStreamQuery(stream);
+    if (state == hipErrorNotReady) continue;
+    MOBULA_HIP_TRY(state);
+    if (!failed() && words[3] != box->ticket) set_error("a kernel ended without its message to the host");
+    break;
+  }
+  std::atomic_thread_fence(std::memory_order_acquire);
+  return !failed();
 }
 
 long long option(const char* name, long long fallback) {

@@ -163,7 +163,8 @@ bool use_tiled();
 // straightforward fallback: the caller converts to NCHW instead).
 template <typename T>
 bool nhwc_forward_supported(const Problem& p) {
-  return roialign::blocked_rows_per_pass<T>(p.C, p.H, p.W, p.PH, p.PW, p.S != 1 && p.S != 2) > 0 &&
+  return p.C % roialign::BlockOf<T>::CPL == 0 &&   // (a lane's sixteen bytes of channels, aligned)
+         roialign::blocked_rows_per_pass<T>(p.C, p.H, p.W, p.PH, p.PW, p.S != 1 && p.S != 2) > 0 &&
          static_cast<long long>(p.H) * p.W * p.C * static_cast<long long>(sizeof(T)) < (1ll << 31);
 }
 
@@ -177,7 +178,8 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
   const bool small_grid = p.S == 1 || p.S == 2;   // else: sampling grids above 2 x 2, merged lists
   const int rpp = roialign::blocked_rows_per_pass<T>(p.C, p.H, p.W, p.PH, p.PW, !small_grid);
   const int nw = small_grid ? FB::NW : roialign::FwdMerged::NW;   // wavefronts per workgroup of the gather
-  const long long grid = roialign::blocked_grid(p.R, cblk, nw);
+  const int parts = roialign::forward_row_parts(p.R, cblk, p.PH, !small_grid);
+  const long long grid = roialign::blocked_grid(static_cast<long long>(p.R) * parts, cblk, nw);
   const bool fits = rpp > 0 && p.N > 0 && p.N < 65536 && cblk < 65536 && grid < (1ll << 31);
   if (p.nhwc) {
     // the map is read where it lies: no copy, only the ROI ordering before the gather
@@ -193,16 +195,16 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
       if (failed()) return;
       roialign::roi_order_kernel<<<1, 1024, 0, stream>>>(rois, p.R, p.scale, p.H, p.W, p.N, order);
     }
-    const long long grid = roialign::blocked_grid_nhwc(p.R, cblk, nw);
+    const long long grid = roialign::blocked_grid_nhwc(static_cast<long long>(p.R) * parts, cblk, nw);
     if (small_grid) {
       mobula_hip::KernelTimer timer("forward_blocked_kernel", stream);
       roialign::forward_blocked_kernel<T, true><<<static_cast<unsigned>(grid), FB::NW * 64, 0, stream>>>(
-          x, rois, order, y, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, p.N, cblk, p.PH, p.R);
+          x, rois, order, y, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, p.N, cblk, p.PH, p.R, parts);
     } else {
       {
         mobula_hip::KernelTimer timer("forward_merged_kernel", stream);
         roialign::forward_merged_kernel<T, true><<<static_cast<unsigned>(grid), nw * 64, 0, stream>>>(
-            x, rois, order, y, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, p.N, cblk, p.PH, p.R);
+            x, rois, order, y, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, p.N, cblk, p.PH, p.R, parts);
       }
       // the boxes that kernel leaves out (sampling grids of more than 64 points per axis)
       if (p.S <= 0 || p.S > roialign::kSearchedGrid)
@@ -212,10 +214,12 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
     MOBULA_HIP_TRY(hipGetLastError());
     return;
   }
-  if (use_tiled() && fits) {
+  const size_t xt_bytes = (sizeof(T) * p.N * cblk * CB * pixels + 255) / 256 * 256;
+  const bool fixed = p.fixed_scratch != nullptr;
+  // (with fixed scratch a map whose padded channels do not fit it takes the straightforward kernel)
+  const bool padded_beyond = fixed && p.C % roialign::BlockOf<T>::CPL != 0 && xt_bytes + sizeof(int) * p.R > p.fixed_scratch_bytes;
+  if (use_tiled() && fits && !padded_beyond) {
     // channel-blocked copy of the map, spatial ROI order, then the gather
-    const size_t xt_bytes = (sizeof(T) * p.N * cblk * CB * pixels + 255) / 256 * 256;
-    const bool fixed = p.fixed_scratch != nullptr;
     if (fixed && xt_bytes + sizeof(int) * p.R > p.fixed_scratch_bytes) {
       set_error("roi_align_forward_noalloc: the problem needs %zu bytes of scratch memory, the library's fixed "
                 "buffer holds %zu (feature map too large for the entry point that allocates nothing)",
@@ -250,13 +254,13 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
     if (small_grid) {
       mobula_hip::KernelTimer timer("forward_blocked_kernel", stream, !fixed);   // (its events are allocations)
       roialign::forward_blocked_kernel<T, false><<<static_cast<unsigned>(grid), FB::NW * 64, 0, stream>>>(
-          xt, rois, order, y, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, p.N, cblk, rpp, p.R);
+          xt, rois, order, y, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, p.N, cblk, rpp, p.R, parts);
     } else {
       // every pixel of a bin is loaded once
       {
         mobula_hip::KernelTimer timer("forward_merged_kernel", stream, !fixed);
         roialign::forward_merged_kernel<T, false><<<static_cast<unsigned>(grid), nw * 64, 0, stream>>>(
-            xt, rois, order, y, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, p.N, cblk, rpp, p.R);
+            xt, rois, order, y, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, p.N, cblk, rpp, p.R, parts);
       }
       // the boxes that kernel leaves out (sampling grids of more than 64 points per axis), from the map itself
       if (p.S <= 0 || p.S > roialign::kSearchedGrid)
@@ -321,18 +325,18 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
   // not while the stream is being captured into a graph).
   const bool windows = roialign::lists_in_windows(p.S);
   long long items = p.R, window_entries = 0;
-  // the head of the workspace: offsets[R + 1], info[3], counts[R], work[R] (see window_offsets_kernel)
-  const size_t b_offsets = windows ? align_up(sizeof(int) * (p.R + 4) + sizeof(int) * p.R + 8, 256) +
+  // the head of the workspace: offsets[R + 1], counts[R], work[R] (see window_offsets_kernel)
+  const size_t b_offsets = windows ? align_up(sizeof(int) * (2 * p.R + 1), 256) +
                                          align_up(sizeof(long long) * p.R, 256) : 0;
   char* head = nullptr;
-  auto number_windows = [&](char* at) {
+  const roialign::WindowArgs wa{rois, p.R, p.scale, p.PH, p.PW, p.S, p.H, p.W, tw};
+  auto number_windows = [&](char* at, int* told, int ticket) {
     int* const offsets = reinterpret_cast<int*>(at);
-    int* const counts = offsets + p.R + 4;
-    long long* const work = reinterpret_cast<long long*>(at + align_up(sizeof(int) * (2 * p.R + 4) + 8, 256));
-    if (p.R > 0)
-      roialign::window_counts_kernel<<<grid_for(p.R, 256), 256, 0, stream>>>(rois, p.R, p.scale, p.PH, p.PW, p.S, p.H,
-                                                                            p.W, tw, counts, work);
-    roialign::window_offsets_kernel<<<1, 1024, 0, stream>>>(counts, work, p.R, offsets, offsets + p.R + 1);
+    int* const counts = offsets + p.R + 1;
+    long long* const work = reinterpret_cast<long long*>(at + align_up(sizeof(int) * (2 * p.R + 1), 256));
+    if (p.R > roialign::kCountedInOffsets)
+      roialign::window_counts_kernel<<<grid_for(p.R, 256), 256, 0, stream>>>(wa, counts, work);
+    roialign::window_offsets_kernel<<<1, 1024, 0, stream>>>(wa, counts, work, offsets, told, ticket);
   };
   if (p.S > roialign::kSearchedGrid) return false;   // (fixed grids of that size are not merged)
   if (windows) {
@@ -342,13 +346,15 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
       return false;
     }
     head = static_cast<char*>(mobula_hip::workspace(b_offsets));
+    mobula_hip::Mailbox* const box = mobula_hip::mailbox();
     if (failed()) return false;
-    number_windows(head);
-    int info[3] = {0, 1, 0};
-    MOBULA_HIP_TRY(hipMemcpyAsync(info, reinterpret_cast<int*>(head) + p.R + 1, sizeof(info), hipMemcpyDeviceToHost,
-                                  stream));
-    MOBULA_HIP_TRY(hipStreamSynchronize(stream));
-    if (failed() || info[1] != 0) return false;   // an adaptive grid too large to merge
+    // the numbers come back through pinned memory that this thread watches (a copy and a wait for
+    // the stream take some 25 us longer, with the device idle)
+    number_windows(head, box->words, ++box->ticket);
+    MOBULA_HIP_TRY(hipGetLastError());
+    if (failed() || !mobula_hip::wait_for_mail(box, stream)) return false;
+    const volatile int* const info = box->words;
+    if (info[1] != 0) return false;   // an adaptive grid too large to merge
     items = info[0];
     window_entries = info[2];
   }
@@ -388,7 +394,7 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
   if (failed()) return false;
   int* offsets = nullptr;
   if (windows) {
-    if (base != head) number_windows(base);   // the workspace has grown: it is another buffer now
+    if (base != head) number_windows(base, nullptr, 0);   // the workspace has grown: it is another buffer now
     offsets = reinterpret_cast<int*>(base);
     base += b_offsets;
   }
@@ -444,8 +450,9 @@ int row_split(const Problem& p) {
   return roialign::backward_row_split(p.N, p.H, p.W, (p.C + BB::CB - 1) / BB::CB);
 }
 
-// The tile owner for a problem: tile columns tw, nsplit wavefronts per tile row (lists of
-// merged windows are not split), sample lists or windows.
+// The tile owner for a problem: tile columns tw, nsplit wavefronts per tile row, sample lists or
+// windows of merged weights (which are not split: 47 us against 71 in four parts, 301 boxes on
+// 3 x 81 x 75 x 113).
 template <bool NHWC, typename T>
 auto owner_kernel(int tw, int* nsplit, bool windows) {
   using BB = roialign::BwdBlocked;

@@ -1064,3 +1064,23 @@ def test_fp16_full_size_subset():
     want = oracle.forward(w['data'].astype(np.float32), w['rois'][pick], pooled, scale, S)
     got = y[torch.from_numpy(pick).cuda()].float().cpu().numpy()
     assert_parity(got, want.astype(np.float16).astype(np.float32), FP16_TOL, 'cfg4 subset')
+
+
+@pytest.mark.parametrize('S', [2, 0])
+@pytest.mark.parametrize('R,C,pooled', [(1, 5, (7, 7)), (9, 33, (5, 9)), (40, 81, (3, 20)), (300, 62, (14, 14))])
+def test_few_boxes_share_their_pooled_rows_among_wavefronts(R, C, pooled, S):
+    """Few boxes: the pooled rows of one are dealt to several wavefronts, as many as there are rows or only
+    some of them; channel counts that end inside a lane's quad (fp32 and fp16)."""
+    abi.set_impl('tiled')
+    rng = np.random.default_rng(R + C)
+    N, H, W, scale = 2, 27, 43, 0.25
+    x = rng.standard_normal((N, C, H, W)).astype(np.float32)
+    c = np.stack([rng.uniform(0, W / scale, R), rng.uniform(0, H / scale, R)], 1)
+    wh = np.exp(rng.uniform(np.log(2), np.log(1.5 * W / scale), (R, 2)))
+    rois = np.concatenate([rng.integers(0, N, (R, 1)), c - wh / 2, c + wh / 2], 1).astype(np.float32)
+    y = abi.forward(abi.to_dev(x), abi.to_dev(rois), pooled, scale, S).cpu().numpy()
+    assert_parity(y, oracle.forward(x, rois, pooled, scale, S), FWD_TOL, 'fp32')
+    x16 = x.astype(np.float16)
+    y16 = abi.forward(abi.to_dev(x16), abi.to_dev(rois), pooled, scale, S).cpu().numpy()
+    want = oracle.forward(x16.astype(np.float32), rois, pooled, scale, S).astype(np.float16)
+    assert_parity(y16.astype(np.float32), want.astype(np.float32), FP16_TOL, 'fp16')
