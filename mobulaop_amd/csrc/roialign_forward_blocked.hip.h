@@ -56,40 +56,42 @@ inline int blocked_rows_per_pass(int C, long long H, long long W, int PH, int PW
   return min(PH, stage / (B::CB * PW));
 }
 
-struct OrderArgs { const float* rois; int* order; int R; float scale; int H, W; long long num_images; };
+struct OrderArgs { const float* rois; int* order; int R; float scale; int H, W; long long num_images; int PH, PW, S; };
 
 template <int NT, int MAXC>
 __device__ __forceinline__ void roi_order_body(int* hist, int* wave_sum, int* carry, const float* __restrict__ rois,
                                                int R, float scale, int H, int W, long long num_images,
                                                int* __restrict__ order);
 
-// out[n][cb][p][CB] = in[n][cb*CB + k][p]; channels past C are written as zero.
-// With oa.order set the launch has one more column of workgroups, the first of which sorts the
-// ROIs (roi_order_body with the cells that fit the tile's LDS) while the others copy: the
-// ordering of a few thousand ROIs then costs nothing beside a copy that takes several times as long.
+// True if no sample of any ROI can touch the pixels p0 .. p0 + 63 of image n (asked by a whole workgroup
+// of 256 threads, each looks at every 256th ROI).  A box's pixels lie between the cells of its two
+// corners, the interpolation's neighbours and a cell to spare included.
+__device__ __forceinline__ bool pixels_untouched(const OrderArgs& oa, int n, int p0) {
+  const int last = min(p0 + 63, oa.H * oa.W - 1), y0 = p0 / oa.W, y1 = last / oa.W;
+  const int x0 = y0 == y1 ? p0 - y0 * oa.W : 0, x1 = y0 == y1 ? last - y1 * oa.W : oa.W - 1;
+  bool hit = false;
+  for (int r = threadIdx.x; r < oa.R; r += 256) {
+    const RoiGeom g = roi_geometry(oa.rois + static_cast<long long>(r) * 5, oa.scale, oa.PH, oa.PW, oa.S);
+    if (g.batch != n) continue;
+    const float end_h = g.start_h + g.bin_h * static_cast<float>(oa.PH);
+    const float end_w = g.start_w + g.bin_w * static_cast<float>(oa.PW);
+    // (samples in [-1, 0] and in [size - 1, size] use the border cells; what is not a number touches everything)
+    const bool miss = end_h < static_cast<float>(y0) - 2.0f - (y0 == 0 ? 2.0f : 0.0f) ||
+                      g.start_h > static_cast<float>(y1) + 2.0f + (y1 == oa.H - 1 ? 2.0f : 0.0f) ||
+                      end_w < static_cast<float>(x0) - 2.0f - (x0 == 0 ? 2.0f : 0.0f) ||
+                      g.start_w > static_cast<float>(x1) + 2.0f + (x1 == oa.W - 1 ? 2.0f : 0.0f);
+    hit = hit || !miss;
+  }
+  return __syncthreads_or(hit) == 0;
+}
+
+// dst[p][CB] = src[c0 + k][p] for the 64 pixels from p0 on (one channel block of one image); channels past C
+// are written as zero.
 template <typename T, bool VEC>
-__global__ void __launch_bounds__(256)
-transpose_to_blocked_kernel(const T* __restrict__ in, T* __restrict__ out, int C, int P, OrderArgs oa) {
+__device__ __forceinline__ void transpose_pixels(const T* __restrict__ src, T* __restrict__ dst, int C, int P, int c0,
+                                                 int p0, T (&tile)[BlockOf<T>::CB][65]) {
   constexpr int CB = BlockOf<T>::CB;
   struct alignas(4 * sizeof(T)) V4 { T v[4]; };
-  __shared__ T tile[CB][65];
-  int bx = blockIdx.x;
-  if (oa.order != nullptr) {
-    if (bx == 0) {
-      if (blockIdx.y == 0 && blockIdx.z == 0) {
-        constexpr int WORDS = static_cast<int>(sizeof(tile) / 4), MAXC = WORDS - 24;
-        int* const words = reinterpret_cast<int*>(&tile[0][0]);
-        roi_order_body<256, MAXC>(words, words + MAXC + 1, words + MAXC + 20, oa.rois, oa.R, oa.scale, oa.H, oa.W,
-                                  oa.num_images, oa.order);
-      }
-      return;
-    }
-    --bx;
-  }
-  const int n = blockIdx.z, cb = blockIdx.y, cblk = gridDim.y;
-  const int p0 = bx * 64, c0 = cb * CB;
-  const T* src = in + static_cast<size_t>(n) * C * P;
-  T* dst = out + (static_cast<size_t>(n) * cblk + cb) * P * CB;
   if (VEC) {
     const int q = threadIdx.x & 15, r = threadIdx.x >> 4;   // 16 quads of pixels, 16 channels per pass
 #pragma unroll
@@ -132,6 +134,46 @@ transpose_to_blocked_kernel(const T* __restrict__ in, T* __restrict__ out, int C
       for (int i = 0; i < 4; ++i) v.v[i] = tile[4 * cq + i][pl];
       *reinterpret_cast<V4*>(dst + static_cast<size_t>(p0 + pl) * CB + 4 * cq) = v;
     }
+  }
+}
+
+// out[n][cb][p][CB] = in[n][cb*CB + k][p].
+// With oa.order set the launch has one more column of workgroups, the first of which sorts the
+// ROIs (roi_order_body with the cells that fit the tile's LDS) while the others copy: the
+// ordering of a few thousand ROIs then costs nothing beside a copy that takes several times as long.
+// sparse != 0 (few ROIs on a large map): a workgroup takes a run of 64 pixels of every gridDim.y-th of the
+// cblk channel blocks, and leaves the copy unwritten where no box reaches.
+template <typename T, bool VEC>
+__global__ void __launch_bounds__(256)
+transpose_to_blocked_kernel(const T* __restrict__ in, T* __restrict__ out, int C, int P, int cblk, int sparse,
+                            OrderArgs oa) {
+  constexpr int CB = BlockOf<T>::CB;
+  __shared__ T tile[CB][65];
+  int bx = blockIdx.x;
+  if (oa.order != nullptr) {
+    if (bx == 0) {
+      if (blockIdx.y == 0 && blockIdx.z == 0) {
+        constexpr int WORDS = static_cast<int>(sizeof(tile) / 4), MAXC = WORDS - 24;
+        int* const words = reinterpret_cast<int*>(&tile[0][0]);
+        roi_order_body<256, MAXC>(words, words + MAXC + 1, words + MAXC + 20, oa.rois, oa.R, oa.scale, oa.H, oa.W,
+                                  oa.num_images, oa.order);
+      }
+      return;
+    }
+    --bx;
+  }
+  const int n = blockIdx.z, p0 = bx * 64;
+  const T* const src = in + static_cast<size_t>(n) * C * P;
+  T* const dst = out + static_cast<size_t>(n) * cblk * P * CB;
+  int cb = blockIdx.y;
+  if (sparse == 0) {
+    transpose_pixels<T, VEC>(src, dst + static_cast<size_t>(cb) * P * CB, C, P, cb * CB, p0, tile);
+    return;
+  }
+  if (pixels_untouched(oa, n, p0)) return;
+  for (; cb < cblk; cb += gridDim.y) {
+    transpose_pixels<T, VEC>(src, dst + static_cast<size_t>(cb) * P * CB, C, P, cb * CB, p0, tile);
+    __syncthreads();   // the tile has been read
   }
 }
 

@@ -218,7 +218,15 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
   const bool fixed = p.fixed_scratch != nullptr;
   // (with fixed scratch a map whose padded channels do not fit it takes the straightforward kernel)
   const bool padded_beyond = fixed && p.C % roialign::BlockOf<T>::CPL != 0 && xt_bytes + sizeof(int) * p.R > p.fixed_scratch_bytes;
-  if (use_tiled() && fits && !padded_beyond) {
+  // Few outputs of a fixed grid: one thread each, straight from the map, takes less time than the copy
+  // (microseconds by size, measured: 13.5 per million outputs at 2 x 2 points, 2.7 for the gather from the
+  // copy; the copy moves 6 TB/s).  Eight boxes of 64 channels on 32 x 32 pixels: 8.1 us a launch less;
+  // 32 of 256 channels on 4 x 200 x 336: 88 -> 11 us, 512 of them 112 -> 107.  (A map too large for fixed scratch
+  // stays an error.)
+  const double copied_us = 3.0 + 2.0 * xt_bytes / 6.0e6 + 2.7e-6 * p.n_out;
+  const bool direct = (!fixed || xt_bytes + sizeof(int) * p.R <= p.fixed_scratch_bytes) && p.S >= 1 && p.S <= 4 && mobula_hip::option("roialign_impl", kAuto) == kAuto &&
+                      13.5e-6 * p.n_out * p.S * p.S / 4 < copied_us;
+  if (use_tiled() && fits && !padded_beyond && !direct) {
     // channel-blocked copy of the map, spatial ROI order, then the gather
     if (fixed && xt_bytes + sizeof(int) * p.R > p.fixed_scratch_bytes) {
       set_error("roi_align_forward_noalloc: the problem needs %zu bytes of scratch memory, the library's fixed "
@@ -240,16 +248,21 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
     mobula_hip::SideStream side(stream, !fixed && order != nullptr && !order_in_copy && p.R > kSideStreamRois);
     if (order != nullptr && !order_in_copy)
       roialign::roi_order_kernel<<<1, 1024, 0, side.get()>>>(rois, p.R, p.scale, p.H, p.W, p.N, order);
-    const roialign::OrderArgs oa{rois, order_in_copy ? order : nullptr, static_cast<int>(p.R), p.scale, p.H, p.W, p.N};
+    const roialign::OrderArgs oa{rois, order_in_copy ? order : nullptr, static_cast<int>(p.R), p.scale, p.H, p.W, p.N,
+                                 p.PH, p.PW, p.S};
+    // Few boxes on a large map: only what they can touch is copied (4 x 256 x 200 x 336 in fp32, adaptive
+    // grid: 97 -> 34 us with two boxes, 99 -> 53 with 32, 119 -> 107 with 128; beyond some 32 boxes an
+    // image, and on maps the caches hold, looking at the boxes costs more than it saves).
+    const bool sparse = xt_bytes > kSortedAboveBytes && p.R <= 32 * p.N;
     const dim3 tgrid(static_cast<unsigned>((pixels + 63) / 64) + (order_in_copy ? 1u : 0u),
-                     static_cast<unsigned>(cblk), static_cast<unsigned>(p.N));
+                     static_cast<unsigned>(sparse ? std::min(cblk, 2) : cblk), static_cast<unsigned>(p.N));
     const bool vec = pixels % 4 == 0 && reinterpret_cast<size_t>(x) % (4 * sizeof(T)) == 0;
     if (vec)
       roialign::transpose_to_blocked_kernel<T, true><<<tgrid, 256, 0, stream>>>(
-          x, xt, p.C, static_cast<int>(pixels), oa);
+          x, xt, p.C, static_cast<int>(pixels), cblk, sparse ? 1 : 0, oa);
     else
       roialign::transpose_to_blocked_kernel<T, false><<<tgrid, 256, 0, stream>>>(
-          x, xt, p.C, static_cast<int>(pixels), oa);
+          x, xt, p.C, static_cast<int>(pixels), cblk, sparse ? 1 : 0, oa);
     side.join();
     if (small_grid) {
       mobula_hip::KernelTimer timer("forward_blocked_kernel", stream, !fixed);   // (its events are allocations)

@@ -1084,3 +1084,28 @@ def test_few_boxes_share_their_pooled_rows_among_wavefronts(R, C, pooled, S):
     y16 = abi.forward(abi.to_dev(x16), abi.to_dev(rois), pooled, scale, S).cpu().numpy()
     want = oracle.forward(x16.astype(np.float32), rois, pooled, scale, S).astype(np.float16)
     assert_parity(y16.astype(np.float32), want.astype(np.float32), FP16_TOL, 'fp16')
+
+
+@pytest.mark.parametrize('W', [200, 203])
+@pytest.mark.parametrize('dtype', [np.float32, np.float16])
+def test_few_boxes_on_a_large_map_copy_only_what_they_touch(W, dtype):
+    """Up to 32 boxes an image on a map beyond the caches: pixels no box reaches are not copied.  The workspace
+    holds NaN beforehand; boxes at every border, past it, of no extent, and one that covers the map."""
+    abi.set_impl('auto')
+    rng = np.random.default_rng(W)
+    N, C, H, scale, pooled = 3, 64 if dtype == np.float32 else 128, 260, 0.5, (5, 4)
+    x = rng.standard_normal((N, C, H, W)).astype(dtype)
+    E, F = W / scale, H / scale   # the image
+    rois = np.array([[0, -30, -30, 12, 9], [0, E - 20, F - 9, E + 40, F + 40], [1, E - 1, 3, E + 9, 60],
+                     [1, 100, F - 0.5, 160, F + 3], [2, 50, 50, 50, 50], [2, 63.9, 128, 64.1, 300], [2, 2, 2, 1, 1],
+                     [1, -500, -500, -400, -400], [5, 0, 0, 9, 9]] +
+                    [[n % N, a, b, a + 37.5, b + 21] for n, (a, b) in
+                     enumerate(zip(rng.uniform(0, E - 40, 20), rng.uniform(0, F - 30, 20)))], dtype=np.float32)
+    poison = torch.full((N, C, H + 64, W), float('nan'), device='cuda')
+    abi.forward(poison, abi.to_dev(np.array([[n, 0, 0, E, F + 128] for n in range(N)], dtype=np.float32)), (1, 1), scale, 0)
+    for some in (rois, np.concatenate([rois, [[0, 0, 0, E, F]]]).astype(np.float32)):
+        got = abi.forward(abi.to_dev(x), abi.to_dev(some), pooled, scale, 0).cpu().numpy()
+        keep = some[:, 0] < N
+        want = oracle.forward(x.astype(np.float32), some[keep], pooled, scale, 0).astype(dtype)
+        assert_parity(got[keep].astype(np.float32), want.astype(np.float32), FWD_TOL if dtype == np.float32 else FP16_TOL, 'y')
+        assert not got[~keep].any()
