@@ -338,9 +338,13 @@ forward_blocked_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
     slot = part * range + wi;
   }
   if (slot >= R) return;
-  const int ph_first = static_cast<int>(slot % parts) * ((PH + parts - 1) / parts);
-  const int ph_end = min(PH, ph_first + (PH + parts - 1) / parts);
-  slot /= parts;
+  int ph_first = 0, ph_end = PH;
+  if (parts > 1) {
+    const int rows = (PH + parts - 1) / parts;
+    ph_first = static_cast<int>(slot % parts) * rows;
+    ph_end = min(PH, ph_first + rows);
+    slot /= parts;
+  }
   const int roi = uni_i(order != nullptr ? order[slot] : static_cast<int>(slot));   // no order: as listed
   const int c0 = cb * CB, nch = min(CB, C - c0);
   const int grp = lane >> 3, quad = lane & 7;   // pooled column within a step, channel quad
