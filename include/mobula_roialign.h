@@ -270,6 +270,13 @@ void conv2d_backward_weight_ecf81c91(const int device_id, const int n, const flo
                                      const int kernel_h, const int kernel_w, const int pad_h,
                                      const int pad_w, const int stride_h, const int stride_w,
                                      const int dilation_h, const int dilation_w, float* dw);
+/* dx and dw of one backward pass in one call (overwritten; a null pointer: not wanted), with the
+ * conversions of their operands shared where the option "conv_compute" asks for bf16 products. */
+void mobula_hip_conv2d_backward(const int device_id, const float* dy, const float* x, const float* weight,
+                                const int batch, const int channels, const int height, const int width,
+                                const int filters, const int kernel_h, const int kernel_w, const int pad_h,
+                                const int pad_w, const int stride_h, const int stride_w,
+                                const int dilation_h, const int dilation_w, float* dx, float* dw);
 /* db[filters] (+)= sum of dy over images and pixels; n = filters. */
 void conv2d_backward_bias_cd239a08(const int device_id, const int n, const float* dy,
                                    const int accumulate, const int batch, const int pixels, float* db);

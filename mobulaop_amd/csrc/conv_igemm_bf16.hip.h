@@ -72,13 +72,25 @@ __device__ __forceinline__ unsigned pack_bf16_parts(float lo, float hi, int part
 // once: its loads leave the caches to the copy that is about to be read.
 // tail != 0: a second copy, `tail` halves after the first, holds the tails of the values (what
 // their bf16 heads leave).
+struct BlockedJob {
+  const float* src; unsigned short* dst;
+  int C, Cpad, P; size_t tail;
+  int vec;                         // P is a multiple of four and src 16-byte aligned
+  unsigned tiles_p, tiles_c, blocks;   // workgroups: (pixels / 64) x (channels / 64) x images
+};
+
+constexpr int kPrepLdsWords = 64 * 65;   // what a job of prepare_b16_kernel finds in LDS
+
 template <bool VEC>
-__global__ void __launch_bounds__(256)
-to_blocked_bf16_kernel(const float* __restrict__ src, unsigned short* __restrict__ dst, int C, int Cpad, int P,
-                       size_t tail) {
+__device__ __forceinline__ void to_blocked_bf16(const BlockedJob& job, unsigned block, float* lds) {
   typedef float f32x4 __attribute__((ext_vector_type(4)));
-  __shared__ float tile[64][65];
-  const int n = blockIdx.z, c0 = blockIdx.y * 64, p0 = blockIdx.x * 64;
+  float (*const tile)[65] = reinterpret_cast<float (*)[65]>(lds);
+  const int C = job.C, Cpad = job.Cpad, P = job.P;
+  const size_t tail = job.tail;
+  const float* const src = job.src;
+  unsigned short* const dst = job.dst;
+  const unsigned row = block / job.tiles_p;
+  const int n = row / job.tiles_c, c0 = (row - n * job.tiles_c) * 64, p0 = (block - row * job.tiles_p) * 64;
   const float* in = src + static_cast<size_t>(n) * C * P;
   if (VEC) {
     const int q = threadIdx.x & 15, r = threadIdx.x >> 4;   // 16 quads of pixels, 16 channels per pass
@@ -124,21 +136,25 @@ to_blocked_bf16_kernel(const float* __restrict__ src, unsigned short* __restrict
 // c < C, else 0 (m < Mpad, c < Cpad).  tail != 0: three copies `tail` halves apart, heads, heads
 // again and tails (what the bf16 heads leave): the weights of the three passes of a product with
 // split operands, one after the other like the K steps that read them.
-__global__ void __launch_bounds__(256)
-arrange_weights_bf16_kernel(const float* __restrict__ w, unsigned short* __restrict__ out, int M, int Mpad,
-                            int C, int Cpad, int taps, long long stride_m, long long stride_c, size_t tail) {
-  const long long total = static_cast<long long>(Mpad) * taps * Cpad / 2;   // pairs of channels
-  const long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
+struct ArrangeJob {
+  const float* w; unsigned short* out;
+  int M, Mpad, C, Cpad, taps; long long stride_m, stride_c; size_t tail;
+  unsigned blocks;
+};
+
+__device__ __forceinline__ void arrange_weights_bf16(const ArrangeJob& job, unsigned block) {
+  const long long total = static_cast<long long>(job.Mpad) * job.taps * job.Cpad / 2;   // pairs of channels
+  const long long i = static_cast<long long>(block) * 256 + threadIdx.x;
   if (i >= total) return;
-  const int j = 2 * static_cast<int>(i % 16), m = static_cast<int>((i / 16) % Mpad);
-  const int s = static_cast<int>(i / (16ll * Mpad));
-  const int cb = s / taps, tap = s - cb * taps, c = cb * 32 + j;
-  const float lo = (m < M && c < C) ? w[m * stride_m + c * stride_c + tap] : 0.0f;
-  const float hi = (m < M && c + 1 < C) ? w[m * stride_m + (c + 1) * stride_c + tap] : 0.0f;
-  reinterpret_cast<unsigned*>(out)[i] = pack_bf16(lo, hi);
-  if (tail != 0) {
-    reinterpret_cast<unsigned*>(out + tail)[i] = pack_bf16(lo, hi);
-    reinterpret_cast<unsigned*>(out + 2 * tail)[i] = pack_bf16_parts(lo, hi, 1);
+  const int j = 2 * static_cast<int>(i % 16), m = static_cast<int>((i / 16) % job.Mpad);
+  const int s = static_cast<int>(i / (16ll * job.Mpad));
+  const int cb = s / job.taps, tap = s - cb * job.taps, c = cb * 32 + j;
+  const float lo = (m < job.M && c < job.C) ? job.w[m * job.stride_m + c * job.stride_c + tap] : 0.0f;
+  const float hi = (m < job.M && c + 1 < job.C) ? job.w[m * job.stride_m + (c + 1) * job.stride_c + tap] : 0.0f;
+  reinterpret_cast<unsigned*>(job.out)[i] = pack_bf16(lo, hi);
+  if (job.tail != 0) {
+    reinterpret_cast<unsigned*>(job.out + job.tail)[i] = pack_bf16(lo, hi);
+    reinterpret_cast<unsigned*>(job.out + 2 * job.tail)[i] = pack_bf16_parts(lo, hi, 1);
   }
 }
 
@@ -313,14 +329,26 @@ struct BackwardDataOpsB16 : GatheredB16 {
 // 8, at most kPaddedSpan; blockIdx.y counts the spans of a plane); neighbouring lanes read
 // neighbouring positions, the bf16 values go through LDS and leave 16 bytes per lane.
 constexpr int kPaddedSpan = 4096;
-__global__ void __launch_bounds__(256)
-to_padded_bf16_kernel(const float* __restrict__ src, unsigned short* __restrict__ dst,
-                      unsigned short* __restrict__ shifted, int H, int W, int off_h, int off_w, int Hg, int Wg,
-                      int Gp, int span, size_t tail) {
+struct PaddedJob {
+  const float* src; unsigned short* dst; unsigned short* shifted;
+  int H, W, off_h, off_w, Hg, Wg, Gp;
+  int span;      // positions, or grid rows, of a workgroup
+  int rows;      // 1: whole grid rows, sixteen bytes per load (to_padded_bf16_rows)
+  size_t tail;
+  unsigned planes, blocks;   // workgroups: planes x spans of a plane
+};
+static_assert(2 * (kPaddedSpan + 8) * sizeof(unsigned short) <= kPrepLdsWords * sizeof(float), "fits the jobs' LDS");
+
+__device__ __forceinline__ void to_padded_bf16(const PaddedJob& job, unsigned block, float* lds) {
   // (tail != 0: the tails of the values as a second set of planes, `tail` halves after the heads)
-  __shared__ __attribute__((aligned(16))) unsigned short vals_s[2][kPaddedSpan + 8];
-  const int plane = blockIdx.x, base = blockIdx.y * span;
-  const float* in = src + static_cast<size_t>(plane) * H * W;
+  unsigned short (*const vals_s)[kPaddedSpan + 8] = reinterpret_cast<unsigned short (*)[kPaddedSpan + 8]>(lds);
+  const int H = job.H, W = job.W, off_h = job.off_h, off_w = job.off_w, Hg = job.Hg, Wg = job.Wg, Gp = job.Gp;
+  const int span = job.span;
+  const size_t tail = job.tail;
+  unsigned short* const dst = job.dst;
+  unsigned short* const shifted = job.shifted;
+  const int plane = block % job.planes, base = (block / job.planes) * span;
+  const float* in = job.src + static_cast<size_t>(plane) * H * W;
   auto value_at = [&](int gh, int gw) {
     const int ih = gh - off_h, iw = gw - off_w;
     const bool inside = (gh < Hg) & (static_cast<unsigned>(ih) < static_cast<unsigned>(H)) &
@@ -357,25 +385,28 @@ to_padded_bf16_kernel(const float* __restrict__ src, unsigned short* __restrict_
 }
 
 // The same copy for planes whose rows are a multiple of four elements long and 16-byte aligned
-// (VEC4 of the launcher): a workgroup takes `rows` whole grid rows (rows * Wg <= kPaddedSpan; the
+// (`rows` of the job): a workgroup takes `rows` whole grid rows (rows * Wg <= kPaddedSpan; the
 // last span also the tail up to Gp), reads the source rows under them sixteen bytes per lane --
 // they are one contiguous run -- and drops the values at their grid positions in LDS, which was
 // zeroed first; LDS then leaves as above.  (With 4-byte loads the copy runs at 3.5 TB/s, with
 // 16-byte loads as fast as the other layout copies.)
-__global__ void __launch_bounds__(256)
-to_padded_bf16_rows_kernel(const float* __restrict__ src, unsigned short* __restrict__ dst,
-                           unsigned short* __restrict__ shifted, int H, int W, int off_h, int off_w, int Hg,
-                           int Wg, int Gp, int rows, size_t tail) {
+__device__ __forceinline__ void to_padded_bf16_rows(const PaddedJob& job, unsigned block, float* lds) {
   typedef float f32x4 __attribute__((ext_vector_type(4)));
-  __shared__ __attribute__((aligned(16))) unsigned short vals_s[2][kPaddedSpan + 8];
-  const int plane = blockIdx.x, r0 = blockIdx.y * rows, r1 = min(r0 + rows, Hg);
-  const bool last = (blockIdx.y + 1) * rows >= Hg;
+  unsigned short (*const vals_s)[kPaddedSpan + 8] = reinterpret_cast<unsigned short (*)[kPaddedSpan + 8]>(lds);
+  const int H = job.H, W = job.W, off_h = job.off_h, off_w = job.off_w, Hg = job.Hg, Wg = job.Wg, Gp = job.Gp;
+  const int rows = job.span;
+  const size_t tail = job.tail;
+  unsigned short* const dst = job.dst;
+  unsigned short* const shifted = job.shifted;
+  const int plane = block % job.planes, part_of_plane = block / job.planes;
+  const int r0 = part_of_plane * rows, r1 = min(r0 + rows, Hg);
+  const bool last = (part_of_plane + 1) * rows >= Hg;
   const int base = r0 * Wg, end = last ? Gp : r1 * Wg, count = end - base;   // (multiples of 8: the launcher sees to it)
   const int parts = tail != 0 ? 2 : 1;
   for (int part = 0; part < parts; ++part)
     for (int j = 4 * threadIdx.x; j < count + 8; j += 4 * 256) *reinterpret_cast<unsigned long long*>(vals_s[part] + j) = 0ull;
   __syncthreads();
-  const float* in = src + static_cast<size_t>(plane) * H * W;
+  const float* in = job.src + static_cast<size_t>(plane) * H * W;
   const int ih0 = max(r0 - off_h, 0), ih1 = min(r1 - off_h, H);   // source rows under the span
   for (int i = ih0 * W + 4 * threadIdx.x; i < ih1 * W; i += 4 * 256) {
     const f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(in + i));
@@ -411,6 +442,32 @@ to_padded_bf16_rows_kernel(const float* __restrict__ src, unsigned short* __rest
       }
     }
   }
+}
+
+// Everything a product's operands need, in one launch: the jobs do not depend on each other, and a small
+// layer's conversions take less time than their launches (a job with blocks == 0 is absent).
+__global__ void __launch_bounds__(256)
+prepare_b16_kernel(ArrangeJob weights, BlockedJob gathered, PaddedJob rows, PaddedJob columns) {
+  __shared__ __attribute__((aligned(16))) float lds[kPrepLdsWords];
+  unsigned block = blockIdx.x;
+  if (block < gathered.blocks) {
+    if (gathered.vec) to_blocked_bf16<true>(gathered, block, lds);
+    else to_blocked_bf16<false>(gathered, block, lds);
+    return;
+  }
+  block -= gathered.blocks;
+  if (block < columns.blocks) {
+    if (columns.rows) to_padded_bf16_rows(columns, block, lds);
+    else to_padded_bf16(columns, block, lds);
+    return;
+  }
+  block -= columns.blocks;
+  if (block < rows.blocks) {
+    if (rows.rows) to_padded_bf16_rows(rows, block, lds);
+    else to_padded_bf16(rows, block, lds);
+    return;
+  }
+  arrange_weights_bf16(weights, block - rows.blocks);
 }
 
 // Rows: filters d; columns: (tap, channel), tap-major; K: (image, grid position).
@@ -489,13 +546,18 @@ struct ShapeB16 {
   static constexpr int WM = ROWS / (32 * NI), WN = WAVES / WM;   // wavefronts down and across the tile
   static constexpr int NJ = COLS / WN / 32;
   static_assert(WM * NI * 32 == ROWS && WN * NJ * 32 == COLS && COLS <= TileB16::BN, "the wavefronts cover the tile");
-  static constexpr int STAGE_HALVES = (ROWS + TileB16::BN) * TileB16::BK;
+  // rows of the left operand a stage has room for: every wavefront brings the same number of pieces of
+  // sixteen (those past the tile bring zeros)
+  static constexpr int A_ROWS = (ROWS + 16 * WAVES - 1) / (16 * WAVES) * (16 * WAVES);
+  static constexpr int STAGE_HALVES = (A_ROWS + TileB16::BN) * TileB16::BK;
 };
 // Stages of a tile in LDS: four where a CU holds one workgroup anyway (128 KB), so that a step's
 // operands are requested three steps ahead (forward + backward at 32 x 256 x 56 x 56, 3 x 3: 537 us
 // with three stages and a full wait per step, 521 so); three where two workgroups share a CU.
 typedef ShapeB16<256, 256, 8, 4, 4> WideShapeB16;  // 2 x 4 wavefronts of 128 x 64: two to a SIMD
-typedef ShapeB16<128, 256, 4, 4, 3> LowShapeB16;   // 1 x 4 wavefronts of 128 x 64, for products of at most 128 rows
+typedef ShapeB16<192, 256, 8, 3, 4> MidShapeB16;   // 2 x 4 of 96 x 64: products whose rows leave the last 256 half empty
+typedef ShapeB16<128, 256, 4, 4, 3> LowShapeB16;   // 1 x 4 of 128 x 64, for products of at most 128 rows ...
+typedef ShapeB16<64, 256, 4, 2, 3> FlatShapeB16;   // ... and 1 x 4 of 64 x 64 for at most 64
 
 // C[M, Ncols] = A[M, K] x B[K, Ncols], the tile of shape S at (m0, n0) over the K steps
 // s_begin .. s_end - 1 (s_begin < s_end).  piece == nullptr: results go through ops.store;
@@ -505,7 +567,7 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
                                                float* __restrict__ piece) {
   using T = TileB16;
   constexpr int ROWS = S::ROWS, WAVES = S::WAVES, NI = S::NI, NJ = S::NJ, WN = S::WN;
-  constexpr int A_LOADS = ROWS / 16 / WAVES, B_LOADS = T::BN / 16 / WAVES, LOADS = A_LOADS + B_LOADS;
+  constexpr int A_ROWS = S::A_ROWS, A_LOADS = A_ROWS / 16 / WAVES, B_LOADS = T::BN / 16 / WAVES, LOADS = A_LOADS + B_LOADS;
   constexpr int STAGE = S::STAGE_HALVES;
   __shared__ __attribute__((aligned(1024))) unsigned short lds[S::STAGES * STAGE];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -534,11 +596,12 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
     const int dead = s_issue < s_end ? 0 : kDead;
     const typename Ops::Step e = ops.step_at(cur, s_issue);
     if (k < A_LOADS) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_buf, base + 16 * (A_LOADS * wave + k) * 32, 16, a_off | dead,
+      const int past = A_ROWS > ROWS && 16 * (A_LOADS * wave + k) >= ROWS ? kDead : 0;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_buf, base + 16 * (A_LOADS * wave + k) * 32, 16, a_off | dead | past,
                                                (s_issue < s_end ? e.a_delta : 0) + k * ops.a_offset(16), 0, 0);
     } else {
       const int kb = k - A_LOADS;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(b_buf, base + (ROWS + 16 * (B_LOADS * wave + kb)) * 32, 16,
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(b_buf, base + (A_ROWS + 16 * (B_LOADS * wave + kb)) * 32, 16,
                                                ops.b_offset(bctx[kb], e, l_chunk) | dead, 0, 0, 0);
     }
   };
@@ -563,7 +626,7 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
   for (int kc = 0; kc < 2; ++kc) {
     const int slot = (2 * kc + half) ^ sw;
     rd_a[kc] = (wm + col) * 32 + slot * 8;
-    rd_b[kc] = (ROWS + wn + col) * 32 + slot * 8;
+    rd_b[kc] = (A_ROWS + wn + col) * 32 + slot * 8;
   }
   bf16x8 fa[2][NI], fb[2][NJ];
   // fragment reads of a chunk in the order the products below first need them: a0 b0 b1 .. a1 a2 ..
@@ -637,8 +700,10 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
 #pragma unroll
       for (int i = 0; i < NI; ++i)
 #pragma unroll
-        for (int v = 0; v < 16; ++v)
-          piece[(wm + i * 32 + 8 * (v >> 2) + 4 * half + (v & 3)) * T::BN + column] = acc[i][j][v];
+        for (int v = 0; v < 16; ++v) {   // (what lies past the product is not read back either)
+          const int row = wm + i * 32 + 8 * (v >> 2) + 4 * half + (v & 3);
+          if (m0 + row < ops.M && n0 + column < ops.Ncols) piece[row * T::BN + column] = acc[i][j][v];
+        }
     } else {
       const typename Ops::Column out = ops.column(n0 + column);
 #pragma unroll
@@ -678,11 +743,13 @@ reduce_pieces_b16_kernel(Ops ops, int row_tiles, int n_base, TileSplit split, co
   constexpr int TILE = S::ROWS * TileB16::BN;
   const int local = blockIdx.x / (TILE / 256), e = (blockIdx.x % (TILE / 256)) * 256 + threadIdx.x;
   const int t = split.whole + local, column = e % TileB16::BN;
-  if (column >= S::COLS) return;
+  const int m = (t % row_tiles) * S::ROWS + e / TileB16::BN, n = n_base + (t / row_tiles) * S::COLS + column;
+  if (column >= S::COLS || m >= ops.M || n >= ops.Ncols) return;
   const float* p = piece_buffer + static_cast<size_t>(local) * split.pieces * TILE + e;
   float sum = 0.0f;
+#pragma unroll 8
   for (int i = 0; i < split.pieces; ++i) sum += p[static_cast<size_t>(i) * TILE];
-  ops.store(ops.column(n_base + (t / row_tiles) * S::COLS + column), (t % row_tiles) * S::ROWS + e / TileB16::BN, sum);
+  ops.store(ops.column(n), m, sum);
 }
 
 }  // namespace conv

@@ -241,22 +241,19 @@ struct Conv2DBackward : public Node {
     const Tensor dy = grads[0].contiguous();
     const ConvArgs& a = args;
     const int dev = dy.device().index();
-    if (task_should_compute_output(0))
-      out[0] = filled_like(x, [&](const Tensor& dx) {
-        const Tensor w = weight.contiguous();
-        begin(dy, {-1, dy.numel(), w.numel(), -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, dx.numel()});
-        conv2d_backward_data_ecf81c91(dev, static_cast<int>(dx.numel()), dy.data_ptr<float>(), w.data_ptr<float>(), 0,
-                                      GEOMETRY_OF(x, a), dx.data_ptr<float>());
-        raise_if_failed("conv2d_backward_data");
-      });
-    if (task_should_compute_output(1))
-      out[1] = filled_like(weight, [&](const Tensor& dw) {
-        const Tensor xd = x.contiguous();
-        begin(dy, {-1, dy.numel(), xd.numel(), -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, dw.numel()});
-        conv2d_backward_weight_ecf81c91(dev, static_cast<int>(dw.numel()), dy.data_ptr<float>(), xd.data_ptr<float>(), 0,
-                                        GEOMETRY_OF(x, a), dw.data_ptr<float>());
-        raise_if_failed("conv2d_backward_weight");
-      });
+    const bool want_x = task_should_compute_output(0), want_w = task_should_compute_output(1);
+    if (want_x || want_w) {
+      if (want_x) out[0] = at::empty_like(x);
+      if (want_w) out[1] = at::empty_like(weight);
+      auto dense = [](const Tensor& t) { return !t.defined() || t.is_contiguous() ? t : at::empty(t.sizes(), t.options()); };
+      const Tensor dx = dense(out[0]), dw = dense(out[1]), xd = x.contiguous(), w = weight.contiguous();
+      begin(dy, {});
+      mobula_hip_conv2d_backward(dev, dy.data_ptr<float>(), xd.data_ptr<float>(), w.data_ptr<float>(), GEOMETRY_OF(x, a),
+                                 want_x ? dx.data_ptr<float>() : nullptr, want_w ? dw.data_ptr<float>() : nullptr);
+      raise_if_failed("conv2d_backward");
+      if (want_x && !dx.is_same(out[0])) out[0].copy_(dx);
+      if (want_w && !dw.is_same(out[1])) out[1].copy_(dw);
+    }
     if (bias.defined() && task_should_compute_output(2))
       out[2] = filled_like(bias, [&](const Tensor& db) {
         begin(dy, {-1, dy.numel(), -1, -1, -1, db.numel()});

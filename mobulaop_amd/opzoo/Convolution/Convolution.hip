@@ -126,13 +126,22 @@ void launch_igemm_b16_shape(const Ops& ops, int n_base, int columns, float* piec
         ops, row_tiles, n_base, split, piece_buffer);
 }
 
-// Tiles of 256 x 256, or 128 x 256 for products of at most 128 rows.  (Tried for a last round that
+// Tiles by the number of rows: the height whose tiles cover them with the least in all, a tile costing
+// its rows and (the columns' operand is loaded for any height) some 64 more.  (Tried for a last round that
 // fills between half and three quarters of the device: one round of narrower tiles, 256 x 160,
 // over the same columns.  The two rounds then take as long as before -- the full round alone runs
 // slower than beside a half-empty one -- so there is one shape per product.)
 template <typename Ops>
 void launch_igemm_b16(const Ops& ops, float* piece_buffer, hipStream_t stream) {
-  if (ops.M <= 128) launch_igemm_b16_shape<Ops, conv::LowShapeB16>(ops, 0, ops.Ncols, piece_buffer, stream);
+  int best = 0;
+  long long least = 0;
+  for (const int rows : {256, 192, 128, 64}) {
+    const long long cost = static_cast<long long>((ops.M + rows - 1) / rows) * (rows + 64);
+    if (best == 0 || cost < least) { best = rows; least = cost; }
+  }
+  if (best == 64) launch_igemm_b16_shape<Ops, conv::FlatShapeB16>(ops, 0, ops.Ncols, piece_buffer, stream);
+  else if (best == 128) launch_igemm_b16_shape<Ops, conv::LowShapeB16>(ops, 0, ops.Ncols, piece_buffer, stream);
+  else if (best == 192) launch_igemm_b16_shape<Ops, conv::MidShapeB16>(ops, 0, ops.Ncols, piece_buffer, stream);
   else launch_igemm_b16_shape<Ops, conv::WideShapeB16>(ops, 0, ops.Ncols, piece_buffer, stream);
 }
 
@@ -230,59 +239,143 @@ bool plan_gather(GatherPlan* plan, const char* what, const conv::Geometry& g, co
   return true;
 }
 
-// Workspace of a gathered product with bf16 operands in memory (conv_igemm_bf16.hip.h): the
-// weights as [K step][Mpad][32] bf16, the gathered tensor `src` ([images][channels][src_pixels]
-// fp32) as [images][channel block][src_pixels][32] bf16, the piece buffer.  Fills in the
-// fields of `ops` that describe them.  split: two sets of each, heads then tails of the fp32
-// values, and three passes over K.  *taken = false (and no error): the shape does not fit this
-// path's 32-bit offsets with split operands; the caller has other kernels for that mode.
-bool plan_gather_b16(conv::GatheredB16* ops, float** pieces, const char* what, const conv::Geometry& g,
-                     const float* w, int M, int channels, const float* src, int images, int src_pixels,
-                     int columns_per_image, long long stride_m, long long stride_c, bool split, bool* taken,
-                     hipStream_t stream) {
-  *taken = true;
+// ---- products with bf16 operands in memory (conv_igemm_bf16.hip.h) ---------
+
+// The operands of a call's products: what they need of the workspace, and the jobs that write them.
+struct PrepB16 {
+  size_t bytes = 0;
+  conv::ArrangeJob weights{};
+  conv::BlockedJob gathered{};
+  conv::PaddedJob rows{}, columns{};
+  void launch(hipStream_t stream) const {
+    const unsigned blocks = gathered.blocks + columns.blocks + rows.blocks + weights.blocks;
+    if (blocks > 0) conv::prepare_b16_kernel<<<blocks, 256, 0, stream>>>(weights, gathered, rows, columns);
+  }
+};
+constexpr size_t kPieceBytes = sizeof(float) * kMaxPieceBlocks * conv::Tile::BM * conv::Tile::BN;
+
+enum Fit { kFits, kOther, kError };   // kOther: the shape is for the caller's other kernels
+
+// A gathered product: the weights as [K step][Mpad][32] bf16, the gathered tensor `src`
+// ([images][channels][src_pixels] fp32) as [images][channel block][src_pixels][32] bf16.  Fills in the
+// fields of `ops` and `prep` but for the addresses (place_gather_b16).  split: two sets of each, heads then
+// tails of the fp32 values, and three passes over K.
+Fit plan_gather_b16(conv::GatheredB16* ops, PrepB16* prep, const char* what, const conv::Geometry& g, const float* w,
+                    int M, int channels, const float* src, int images, int src_pixels, int columns_per_image,
+                    long long stride_m, long long stride_c, bool split) {
   const int sets = split ? 2 : 1;
   const int taps = g.KH * g.KW, cpad = (channels + 31) / 32 * 32;
   const long long image_bytes = static_cast<long long>(src_pixels) * cpad * 2;
   // a tile's columns span this many images at most; their byte offsets must stay below 2^31
   const long long span = (conv::TileB16::BN - 1) / std::max(columns_per_image, 1) + 2;
-  if (split && (span + images) * image_bytes >= (1ll << 31)) { *taken = false; return false; }
+  if (split && (span + images) * image_bytes >= (1ll << 31)) return kOther;
   if (span * image_bytes >= (1ll << 31)) {
     set_error("%s: images of %lld bytes are too large for the 32-bit offsets of the gather", what, image_bytes);
-    return false;
+    return kError;
   }
-  const int mpad = (M + 255) / 256 * 256;   // (covers row tiles of 128 and of 256)
+  const int mpad = (M + 63) / 64 * 64;   // (rows of a tile past these are read from the next step's and not stored)
   const long long k = static_cast<long long>(taps) * cpad, wcount = k * mpad;
   const int weight_sets = split ? 3 : 1;   // (heads, heads again, tails: one per pass)
   if (3 * k >= (1ll << 31) || 2 * weight_sets * wcount >= (1ll << 31)) {
-    if (split) { *taken = false; return false; }
+    if (split) return kOther;
     set_error("%s: weights too large", what);
-    return false;
+    return kError;
   }
-  const size_t weight_bytes = (2 * weight_sets * wcount + 255) / 256 * 256;
-  const size_t source_bytes = (static_cast<size_t>(sets) * images * image_bytes + 255) / 256 * 256;
-  const size_t piece_bytes = sizeof(float) * kMaxPieceBlocks * conv::Tile::BM * conv::Tile::BN;
-  char* ws = static_cast<char*>(mobula_hip::workspace(weight_bytes + source_bytes + piece_bytes));
-  if (failed()) return false;
-  unsigned short* const weights = reinterpret_cast<unsigned short*>(ws);
-  unsigned short* const source = reinterpret_cast<unsigned short*>(ws + weight_bytes);
-  *pieces = reinterpret_cast<float*>(ws + weight_bytes + source_bytes);
-  ops->wp = weights; ops->src = source; ops->g = g; ops->M = M;
-  ops->K = static_cast<int>((split ? 3 : 1) * k); ops->cpad = cpad; ops->mpad = mpad;
+  ops->g = g; ops->M = M; ops->cpad = cpad; ops->mpad = mpad;
+  ops->K = static_cast<int>((split ? 3 : 1) * k);
   ops->source_tail = split ? static_cast<int>(images * image_bytes) : 0;
-  const size_t weight_tail = split ? static_cast<size_t>(wcount) : 0;                      // (in halves)
-  const size_t source_tail = split ? static_cast<size_t>(images) * image_bytes / 2 : 0;
-  conv::arrange_weights_bf16_kernel<<<blocks_for_all(wcount / 2), 256, 0, stream>>>(
-      w, weights, M, mpad, channels, cpad, taps, stride_m, stride_c, weight_tail);
-  const dim3 tgrid((src_pixels + 63) / 64, (cpad + 63) / 64, images);
-  if (src_pixels % 4 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0)
-    conv::to_blocked_bf16_kernel<true><<<tgrid, 256, 0, stream>>>(src, source, channels, cpad, src_pixels,
-                                                                  source_tail);
-  else
-    conv::to_blocked_bf16_kernel<false><<<tgrid, 256, 0, stream>>>(src, source, channels, cpad, src_pixels,
-                                                                   source_tail);
-  return true;
+  const unsigned tiles_p = (src_pixels + 63) / 64, tiles_c = (cpad + 63) / 64;
+  prep->weights = conv::ArrangeJob{w, nullptr, M, mpad, channels, cpad, taps, stride_m, stride_c,
+                                   split ? static_cast<size_t>(wcount) : 0,   // (in halves)
+                                   static_cast<unsigned>(blocks_for_all(wcount / 2))};
+  prep->gathered = conv::BlockedJob{src, nullptr, channels, cpad, src_pixels,
+                                    split ? static_cast<size_t>(images) * image_bytes / 2 : 0,
+                                    src_pixels % 4 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0, tiles_p, tiles_c,
+                                    tiles_p * tiles_c * images};
+  prep->bytes += align_to_256(2 * weight_sets * wcount) + align_to_256(static_cast<size_t>(sets) * images * image_bytes);
+  return kFits;
 }
+
+// Takes the product's operands from the workspace at `at`; returns what follows them.
+char* place_gather_b16(conv::GatheredB16* ops, PrepB16* prep, char* at) {
+  const conv::ArrangeJob& a = prep->weights;
+  const size_t wcount = static_cast<size_t>(a.Mpad) * a.taps * a.Cpad;
+  unsigned short* const weights = reinterpret_cast<unsigned short*>(at);
+  at += align_to_256(2 * (a.tail != 0 ? 3 : 1) * wcount);
+  unsigned short* const source = reinterpret_cast<unsigned short*>(at);
+  const size_t images = prep->gathered.blocks / (prep->gathered.tiles_p * prep->gathered.tiles_c);
+  at += align_to_256((a.tail != 0 ? 2 : 1) * images * prep->gathered.P * a.Cpad * 2);
+  ops->wp = prep->weights.out = weights;
+  ops->src = prep->gathered.dst = source;
+  return at;
+}
+
+// The weight gradient at unit strides: bf16 copies of dy and x on a common padded grid, one plain product
+// per tap.  With split operands (head + tail, two bf16 for every fp32) the copies hold two sets of
+// planes, heads then tails, and the product walks the images three times: head x head, head x tail, tail x head.
+Fit plan_weight_b16(conv::WeightGradOpsB16* ops, PrepB16* prep, const conv::Geometry& g, const float* dy, const float* x,
+                    bool split) {
+  if (g.stride_h != 1 || g.stride_w != 1 || g.N == 0) return kOther;
+  const int sets = split ? 2 : 1;
+  const int Hg = g.H + 2 * g.pad_h, Wg = g.W + 2 * g.pad_w;
+  const long long G = static_cast<long long>(Hg) * Wg, Gp = (G + 31) / 32 * 32;
+  const long long dy_set = 2ll * g.N * g.D * Gp, x_set = 2ll * g.N * g.C * Gp;   // bytes of one set of planes
+  const long long dy_bytes = sets * dy_set, x_bytes = sets * x_set;
+  if (dy_bytes >= (1ll << 31) || 2 * x_bytes >= (1ll << 31) || 3ll * g.N * Gp >= (1ll << 31) || g.OH > Hg || g.OW > Wg)
+    return kOther;
+  ops->g = g; ops->M = g.D; ops->Ncols = g.C * g.KH * g.KW;
+  ops->split = split ? 1 : 0;
+  ops->K = static_cast<int>((split ? 3 : 1) * g.N * Gp); ops->Gp = static_cast<int>(Gp); ops->Wg = Wg;
+  ops->copy_bytes = static_cast<unsigned>(x_bytes);
+  // whole grid rows per workgroup and 16-byte loads where rows of both tensors allow it (a span
+  // of rows must be a multiple of 8 positions: Wg even and four rows, or any rows if Wg % 8 == 0)
+  int rows = (conv::kPaddedSpan - 32) / Wg;   // (the last span also takes the tail of the plane: up to 31 positions)
+  if (Wg % 8 != 0) rows = Wg % 2 == 0 ? rows / 4 * 4 : 0;
+  const bool vec = rows > 0 && g.W % 4 == 0 && g.OW % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+                   reinterpret_cast<uintptr_t>(dy) % 16 == 0;
+  int spans, span;
+  if (vec) {
+    span = std::min(rows, (Hg + 3) / 4 * 4);
+    spans = (Hg + span - 1) / span;
+  } else {   // a plane in as few, equally long spans as fit the kernel's LDS
+    spans = static_cast<int>((Gp + conv::kPaddedSpan - 1) / conv::kPaddedSpan);
+    span = static_cast<int>((Gp / 8 + spans - 1) / spans * 8);
+  }
+  const unsigned rows_planes = static_cast<unsigned>(g.N) * g.D, columns_planes = static_cast<unsigned>(g.N) * g.C;
+  prep->rows = conv::PaddedJob{dy, nullptr, nullptr, g.OH, g.OW, 0, 0, Hg, Wg, static_cast<int>(Gp), span, vec ? 1 : 0,
+                               split ? static_cast<size_t>(dy_set / 2) : 0, rows_planes, rows_planes * spans};
+  prep->columns = conv::PaddedJob{x, nullptr, nullptr, g.H, g.W, g.pad_h, g.pad_w, Hg, Wg, static_cast<int>(Gp), span,
+                                  vec ? 1 : 0, split ? static_cast<size_t>(x_set / 2) : 0, columns_planes,
+                                  columns_planes * spans};
+  prep->bytes += align_to_256(dy_bytes) + align_to_256(2 * x_bytes);
+  return kFits;
+}
+
+char* place_weight_b16(conv::WeightGradOpsB16* ops, PrepB16* prep, char* at) {
+  const size_t sets = ops->split ? 2 : 1;
+  unsigned short* const dyg = reinterpret_cast<unsigned short*>(at);
+  at += align_to_256(sets * 2 * ops->g.N * ops->g.D * ops->Gp);
+  unsigned short* const xg = reinterpret_cast<unsigned short*>(at);
+  // the shifted copy follows the first one directly (its bytes are a multiple of 64): the reads of
+  // the last plane that run past its end then land in the other copy or beyond the buffer
+  // (zeros), never in workspace bytes that nothing wrote
+  prep->columns.shifted = reinterpret_cast<unsigned short*>(at + ops->copy_bytes);
+  at += align_to_256(2 * static_cast<size_t>(ops->copy_bytes));
+  ops->dyg = prep->rows.dst = dyg;
+  ops->xg = prep->columns.dst = xg;
+  return at;
+}
+
+Fit plan_data_b16(conv::BackwardDataOpsB16* ops, PrepB16* prep, const conv::Geometry& g, const float* dy, const float* w,
+                  int accumulate, float* dx) {
+  ops->dx = dx; ops->accumulate = accumulate; ops->Ncols = g.N * g.H * g.W;
+  const long long taps = g.KH * g.KW;
+  // row m of the left operand is input channel m: element [m][tap][d] = weight[d][m][tap]
+  return plan_gather_b16(ops, prep, "conv2d_backward_data", g, w, g.C, g.D, dy, g.N, g.OH * g.OW, g.H * g.W, taps,
+                         g.C * taps, compute_mode() == conv::kBf16x3);
+}
+
+bool bf16_mode() { return compute_mode() == conv::kBf16 || compute_mode() == conv::kBf16x3; }
 
 // ---- fp32 products from patches (conv_patch_f32.hip.h) -----------------------
 
@@ -699,24 +792,26 @@ MOBULA_KERNEL conv2d_forward_kernel(const int n, const T* x, const T* weight, co
   conv::ForwardOps ops;
   ops.x = x; ops.bias = has_bias ? bias : nullptr; ops.y = y; ops.g = g;
   ops.M = g.D; ops.Ncols = g.N * g.OH * g.OW;
-  if ((compute_mode() == conv::kBf16 || compute_mode() == conv::kBf16x3) && g.N < 65536) {
+  if (bf16_mode() && g.N < 65536) {
     // operands as bf16 in memory: channel-blocked copy of x, weights by K step (heads and tails
     // of both with split operands)
-    bool taken = true;
-    {
+    conv::ForwardOpsB16 ob;
+    ob.bias = ops.bias; ob.y = y; ob.Ncols = ops.Ncols;
+    PrepB16 prep;
+    const long long taps = g.KH * g.KW;
+    const Fit fit = plan_gather_b16(&ob, &prep, "conv2d_forward", g, weight, g.D, g.C, x, g.N, g.H * g.W, g.OH * g.OW,
+                                    g.C * taps, taps, compute_mode() == conv::kBf16x3);
+    if (fit == kError) return;
+    if (fit == kFits) {
       mobula_hip::KernelTimer timer("conv2d_forward", stream);
-      conv::ForwardOpsB16 ob;
-      ob.bias = ops.bias; ob.y = y; ob.Ncols = ops.Ncols;
-      float* pieces = nullptr;
-      const long long taps = g.KH * g.KW;
-      if (plan_gather_b16(&ob, &pieces, "conv2d_forward", g, weight, g.D, g.C, x, g.N, g.H * g.W, g.OH * g.OW,
-                          g.C * taps, taps, compute_mode() == conv::kBf16x3, &taken, stream)) {
-        launch_igemm_b16(ob, pieces, stream);
-        MOBULA_HIP_TRY(hipGetLastError());
-        return;
-      }
-    }
-    if (taken) return;   // (with an error; not taken: the kernels below split fp32 operands themselves)
+      char* const ws = static_cast<char*>(mobula_hip::workspace(prep.bytes + kPieceBytes));
+      if (failed()) return;
+      char* const pieces = place_gather_b16(&ob, &prep, ws);
+      prep.launch(stream);
+      launch_igemm_b16(ob, reinterpret_cast<float*>(pieces), stream);
+      MOBULA_HIP_TRY(hipGetLastError());
+      return;
+    }   // (else the kernels below split fp32 operands themselves)
   }
   {
     mobula_hip::KernelTimer timer("conv2d_forward", stream);
@@ -756,23 +851,21 @@ MOBULA_KERNEL conv2d_backward_data_kernel(const int n, const T* dy, const T* wei
   conv::BackwardDataOps ops;
   ops.dy = dy; ops.dx = dx; ops.g = g; ops.accumulate = accumulate;
   ops.M = g.C; ops.Ncols = g.N * g.H * g.W;
-  if ((compute_mode() == conv::kBf16 || compute_mode() == conv::kBf16x3) && g.N < 65536) {
-    bool taken = true;
-    {
+  if (bf16_mode() && g.N < 65536) {
+    conv::BackwardDataOpsB16 ob;
+    PrepB16 prep;
+    const Fit fit = plan_data_b16(&ob, &prep, g, dy, weight, accumulate, dx);
+    if (fit == kError) return;
+    if (fit == kFits) {
       mobula_hip::KernelTimer timer("conv2d_backward_data", stream);
-      conv::BackwardDataOpsB16 ob;
-      ob.dx = dx; ob.accumulate = accumulate; ob.Ncols = ops.Ncols;
-      float* pieces = nullptr;
-      const long long taps = g.KH * g.KW;
-      // row m of the left operand is input channel m: element [m][tap][d] = weight[d][m][tap]
-      if (plan_gather_b16(&ob, &pieces, "conv2d_backward_data", g, weight, g.C, g.D, dy, g.N, g.OH * g.OW,
-                          g.H * g.W, taps, g.C * taps, compute_mode() == conv::kBf16x3, &taken, stream)) {
-        launch_igemm_b16(ob, pieces, stream);
-        MOBULA_HIP_TRY(hipGetLastError());
-        return;
-      }
+      char* const ws = static_cast<char*>(mobula_hip::workspace(prep.bytes + kPieceBytes));
+      if (failed()) return;
+      char* const pieces = place_gather_b16(&ob, &prep, ws);
+      prep.launch(stream);
+      launch_igemm_b16(ob, reinterpret_cast<float*>(pieces), stream);
+      MOBULA_HIP_TRY(hipGetLastError());
+      return;
     }
-    if (taken) return;
   }
   {
     mobula_hip::KernelTimer timer("conv2d_backward_data", stream);
@@ -813,60 +906,17 @@ MOBULA_KERNEL conv2d_backward_weight_kernel(const int n, const T* dy, const T* x
     return;
   }
   hipStream_t stream = call_state().stream;
-  if ((compute_mode() == conv::kBf16 || compute_mode() == conv::kBf16x3) && g.stride_h == 1 && g.stride_w == 1 &&
-      wt > 0 && g.N > 0) {
-    // bf16 operands in memory on a common padded grid, one plain product per tap.  With split
-    // operands (head + tail, two bf16 for every fp32) the copies hold two sets of planes, heads
-    // then tails, and the product walks the images three times: head x head, head x tail, tail x head.
-    const bool split = compute_mode() == conv::kBf16x3;
-    const int sets = split ? 2 : 1;
-    const int Hg = g.H + 2 * g.pad_h, Wg = g.W + 2 * g.pad_w;
-    const long long G = static_cast<long long>(Hg) * Wg, Gp = (G + 31) / 32 * 32;
-    const long long dy_set = 2ll * g.N * g.D * Gp, x_set = 2ll * g.N * g.C * Gp;   // bytes of one set of planes
-    const long long dy_bytes = sets * dy_set, x_bytes = sets * x_set;
-    if (dy_bytes < (1ll << 31) && 2 * x_bytes < (1ll << 31) && 3ll * g.N * Gp < (1ll << 31) && g.OH <= Hg &&
-        g.OW <= Wg) {
+  if (bf16_mode() && wt > 0) {
+    conv::WeightGradOpsB16 ob;
+    PrepB16 prep;
+    ob.dw = dw; ob.accumulate = accumulate;
+    if (plan_weight_b16(&ob, &prep, g, dy, x, compute_mode() == conv::kBf16x3) == kFits) {
       mobula_hip::KernelTimer timer("conv2d_backward_weight", stream);
-      const size_t dy_room = (dy_bytes + 255) / 256 * 256, x_room = (x_bytes + 255) / 256 * 256;
-      const size_t piece_bytes = sizeof(float) * kMaxPieceBlocks * conv::Tile::BM * conv::Tile::BN;
-      char* ws = static_cast<char*>(mobula_hip::workspace(dy_room + 2 * x_room + piece_bytes));
+      char* const ws = static_cast<char*>(mobula_hip::workspace(prep.bytes + kPieceBytes));
       if (failed()) return;
-      conv::WeightGradOpsB16 ob;
-      unsigned short* const dyg = reinterpret_cast<unsigned short*>(ws);
-      unsigned short* const xg = reinterpret_cast<unsigned short*>(ws + dy_room);
-      ob.dyg = dyg; ob.xg = xg; ob.dw = dw; ob.g = g; ob.M = g.D; ob.Ncols = g.C * g.KH * g.KW;
-      ob.split = split ? 1 : 0;
-      ob.K = static_cast<int>((split ? 3 : 1) * g.N * Gp); ob.Gp = static_cast<int>(Gp); ob.Wg = Wg;
-      ob.accumulate = accumulate;
-      // the shifted copy follows the first one directly (x_bytes is a multiple of 64): the reads of
-      // the last plane that run past its end then land in the other copy or beyond the buffer
-      // (zeros), never in workspace bytes that nothing wrote
-      ob.copy_bytes = static_cast<unsigned>(x_bytes);
-      unsigned short* const xg1 = reinterpret_cast<unsigned short*>(ws + dy_room + x_bytes);
-      const size_t dy_tail = split ? static_cast<size_t>(dy_set / 2) : 0, x_tail = split ? static_cast<size_t>(x_set / 2) : 0;
-      // whole grid rows per workgroup and 16-byte loads where rows of both tensors allow it (a span
-      // of rows must be a multiple of 8 positions: Wg even and four rows, or any rows if Wg % 8 == 0)
-      int rows = (conv::kPaddedSpan - 32) / Wg;   // (the last span also takes the tail of the plane: up to 31 positions)
-      if (Wg % 8 != 0) rows = Wg % 2 == 0 ? rows / 4 * 4 : 0;
-      const bool vec = rows > 0 && g.W % 4 == 0 && g.OW % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
-                       reinterpret_cast<uintptr_t>(dy) % 16 == 0;
-      if (vec) {
-        rows = std::min(rows, (Hg + 3) / 4 * 4);
-        const unsigned spans = static_cast<unsigned>((Hg + rows - 1) / rows);
-        conv::to_padded_bf16_rows_kernel<<<dim3(g.N * g.D, spans), 256, 0, stream>>>(
-            dy, dyg, nullptr, g.OH, g.OW, 0, 0, Hg, Wg, static_cast<int>(Gp), rows, dy_tail);
-        conv::to_padded_bf16_rows_kernel<<<dim3(g.N * g.C, spans), 256, 0, stream>>>(
-            x, xg, xg1, g.H, g.W, g.pad_h, g.pad_w, Hg, Wg, static_cast<int>(Gp), rows, x_tail);
-      } else {
-        // a plane in as few, equally long spans as fit the kernel's LDS
-        const int spans = static_cast<int>((Gp + conv::kPaddedSpan - 1) / conv::kPaddedSpan);
-        const int span = static_cast<int>((Gp / 8 + spans - 1) / spans * 8);
-        conv::to_padded_bf16_kernel<<<dim3(g.N * g.D, spans), 256, 0, stream>>>(dy, dyg, nullptr, g.OH, g.OW, 0, 0, Hg,
-                                                                               Wg, static_cast<int>(Gp), span, dy_tail);
-        conv::to_padded_bf16_kernel<<<dim3(g.N * g.C, spans), 256, 0, stream>>>(
-            x, xg, xg1, g.H, g.W, g.pad_h, g.pad_w, Hg, Wg, static_cast<int>(Gp), span, x_tail);
-      }
-      launch_igemm_b16(ob, reinterpret_cast<float*>(ws + dy_room + 2 * x_room), stream);
+      char* const pieces = place_weight_b16(&ob, &prep, ws);
+      prep.launch(stream);
+      launch_igemm_b16(ob, reinterpret_cast<float*>(pieces), stream);
       MOBULA_HIP_TRY(hipGetLastError());
       return;
     }
@@ -959,6 +1009,28 @@ MOBULA_KERNEL conv2d_backward_bias_kernel(const int n, const T* dy, const int ac
 // buffers (device id -1 is an error here).
 // ---------------------------------------------------------------------------
 namespace {
+// True if the gradients were taken here (or the call has failed).
+bool both_gradients_b16(const conv::Geometry& g, const float* dy, const float* x, const float* weight, float* dx,
+                        float* dw) {
+  if (!bf16_mode() || g.N == 0 || g.N >= 65536) return false;
+  conv::BackwardDataOpsB16 data;
+  conv::WeightGradOpsB16 wgrad;
+  PrepB16 prep;
+  wgrad.dw = dw; wgrad.accumulate = 0;
+  if (plan_weight_b16(&wgrad, &prep, g, dy, x, compute_mode() == conv::kBf16x3) != kFits) return false;
+  const Fit fit = plan_data_b16(&data, &prep, g, dy, weight, 0, dx);
+  if (fit != kFits) return fit == kError;
+  hipStream_t stream = call_state().stream;
+  char* const ws = static_cast<char*>(mobula_hip::workspace(prep.bytes + kPieceBytes));
+  if (failed()) return true;
+  float* const pieces = reinterpret_cast<float*>(place_weight_b16(&wgrad, &prep, place_gather_b16(&data, &prep, ws)));
+  prep.launch(stream);
+  launch_igemm_b16(data, pieces, stream);
+  launch_igemm_b16(wgrad, pieces, stream);
+  MOBULA_HIP_TRY(hipGetLastError());
+  return true;
+}
+
 bool on_device(const char* what, int device_id) {
   mobula_hip::begin_call();
   if (device_id >= 0) return true;
@@ -1023,6 +1095,24 @@ void conv2d_backward_weight_ecf81c91(const int device_id, const int n, const flo
   if (!on_device("conv2d_backward_weight", device_id)) return;
   mobula_hip::DeviceScope scope(device_id);
   if (scope.ok()) conv2d_backward_weight_kernel<float>(n, dy, x, accumulate, CONV_GEOMETRY_ARGS, dw);
+  mobula_hip::finish_call();
+}
+
+// Both gradients of a backward pass (a null dx or dw: not wanted), which share the conversions of
+// their operands where the products have bf16 ones: one launch prepares dy for both, x and the weights.
+void mobula_hip_conv2d_backward(const int device_id, const float* dy, const float* x, const float* weight,
+                                CONV_GEOMETRY_PARAMS, float* dx, float* dw) {
+  if (!on_device("conv2d_backward", device_id)) return;
+  mobula_hip::DeviceScope scope(device_id);
+  conv::Geometry g;
+  if (scope.ok() && describe(&g, "conv2d_backward", CONV_GEOMETRY_ARGS) &&
+      !(dx != nullptr && dw != nullptr && both_gradients_b16(g, dy, x, weight, dx, dw)) && !failed()) {
+    call_state().extents.clear();
+    if (dx != nullptr)
+      conv2d_backward_data_kernel<float>(g.N * g.C * g.H * g.W, dy, weight, 0, CONV_GEOMETRY_ARGS, dx);
+    if (dw != nullptr && !failed())
+      conv2d_backward_weight_kernel<float>(g.D * g.C * g.KH * g.KW, dy, x, 0, CONV_GEOMETRY_ARGS, dw);
+  }
   mobula_hip::finish_call();
 }
 
