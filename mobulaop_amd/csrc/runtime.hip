@@ -183,7 +183,10 @@ bool wait_for_mail(Mailbox* box, hipStream_t stream) {
     if (spins % 4096 != 4095) continue;
     // (the stream has nothing left to do, or has failed: the mail is there, or will never be)
     const hipError_t state = hipStreamQuery(stream);
-    if (state == hipErrorNotReady) continue;
+    if (state == hipErrorNotReady) {
+      (void)hipGetLastError();   // (an answer, no error of the call)
+      continue;
+    }
     MOBULA_HIP_TRY(state);
     if (!failed() && words[3] != box->ticket) set_error("a kernel ended without its message to the host");
     break;
