@@ -9,7 +9,7 @@
 // per call, and the interpreter lock handed to the engine's thread and back.
 //
 // A call this file does not take (other tensor types, arguments it cannot read, shapes
-// the operator class would refuse) is answered with NotImplemented, and the operator
+// the operator class would refuse, calls under a transform of torch's) is answered with NotImplemented, and the operator
 // class takes it as before: what is an error stays the error it was.
 //
 // Semantics are those of opzoo/ROIAlign/ROIAlign.py and opzoo/Convolution/Convolution.py
@@ -25,7 +25,9 @@
 #include <vector>
 
 #include <ATen/ATen.h>
+#include <ATen/TracerMode.h>
 #include <ATen/core/grad_mode.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
@@ -53,6 +55,13 @@ void raise_if_failed(const char* what) {
   const std::string message = std::string(what) + ": " + text;
   mobula_hip_clear_error();
   throw std::runtime_error(message);
+}
+
+// A gradient whose values lie in memory of its own (a batched one, or one without values, has none).
+const Tensor& with_values(const Tensor& dy) {
+  TORCH_CHECK(dy.has_storage() && (dy.numel() == 0 || dy.const_data_ptr() != nullptr),
+              "the gradient of the output has no values in memory: batched and fake tensors are not taken");
+  return dy;
 }
 
 bool is_channels_last(const Tensor& t) {
@@ -164,7 +173,7 @@ struct RoiAlignBackward : public Node {
     at::AutoDispatchBelowADInplaceOrView guard;
     variable_list out(2);
     if (!grads[0].defined()) return out;
-    if (task_should_compute_output(0)) out[0] = data_gradient(grads[0]);
+    if (task_should_compute_output(0)) out[0] = data_gradient(with_values(grads[0]));
     if (task_should_compute_output(1)) out[1] = at::zeros_like(rois);   // no gradient flows to the boxes
     return out;
   }
@@ -238,7 +247,7 @@ struct Conv2DBackward : public Node {
     at::AutoDispatchBelowADInplaceOrView guard;
     variable_list out(bias.defined() ? 3 : 2);
     if (!grads[0].defined()) return out;
-    const Tensor dy = grads[0].contiguous();
+    const Tensor dy = with_values(grads[0]).contiguous();
     const ConvArgs& a = args;
     const int dev = dy.device().index();
     const bool want_x = task_should_compute_output(0), want_w = task_should_compute_output(1);
@@ -328,11 +337,20 @@ bool read_pair(PyObject* o, int (&out)[2]) {
   return read_int(PySequence_Fast_GET_ITEM(o, 0), &out[0]) && read_int(PySequence_Fast_GET_ITEM(o, 1), &out[1]);
 }
 
-// A plain tensor (or parameter) on a GPU.
+// A call that torch watches or transforms (torch.func, tracing, a dispatch mode): what it needs to
+// see is the operator class's autograd function.
+bool is_watched() {
+  return at::tracer::impl::is_dispatch_enabled() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+         c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
+
+// A plain tensor (or parameter) on a GPU, with memory of its own and no forward-mode tangent.
 bool read_tensor(PyObject* o, Tensor* out) {
   if (o == nullptr || !THPVariable_CheckExact(o)) return false;
   const Tensor& t = THPVariable_Unpack(o);
-  if (!t.is_cuda() || t.layout() != at::kStrided || t.is_conj() || t.is_neg() || t.numel() > INT_MAX) return false;
+  if (!t.is_cuda() || t.layout() != at::kStrided || t.is_conj() || t.is_neg() || !t.has_storage() ||
+      t.numel() > INT_MAX || t._fw_grad(0).defined())
+    return false;
   *out = t;
   return true;
 }
@@ -346,7 +364,7 @@ PyObject* py_roi_align(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObj
   Tensor x, rois;
   RoiAlignArgs a;
   int pooled[2];
-  if (!by_name(names, 5, args, nargs, kwnames, v) || !read_tensor(v[0], &x) || !read_tensor(v[1], &rois) ||
+  if (is_watched() || !by_name(names, 5, args, nargs, kwnames, v) || !read_tensor(v[0], &x) || !read_tensor(v[1], &rois) ||
       !read_pair(v[2], pooled) || v[3] == nullptr || !(PyFloat_Check(v[3]) || PyLong_CheckExact(v[3])) ||
       !read_int(v[4], &a.S))
     return not_taken();
@@ -375,7 +393,7 @@ PyObject* py_conv2d(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObject
   PyObject* v[8];
   // positional values are taken for the tensors only: how many of them are inputs is a question
   // for the operator class otherwise
-  if (nargs > 3 || !by_name(names, 8, args, nargs, kwnames, v)) return not_taken();
+  if (nargs > 3 || is_watched() || !by_name(names, 8, args, nargs, kwnames, v)) return not_taken();
   Tensor x, weight, bias;
   ConvArgs a;
   a.stride[0] = a.stride[1] = a.dil[0] = a.dil[1] = 1;

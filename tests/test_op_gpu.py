@@ -5,7 +5,7 @@ import pytest
 
 torch = pytest.importorskip('torch')
 
-from mobulaop_amd import workloads  # noqa: E402
+from mobulaop_amd import native, workloads  # noqa: E402
 from mobulaop_amd.testing import assert_parity  # noqa: E402
 from oracle import roialign as oracle  # noqa: E402
 
@@ -229,6 +229,68 @@ def test_direct_calls_agree_with_the_operator_class(mobula, form):
         assert a.stride() == b.stride() and torch.equal(a, b)
 
 
+@pytest.mark.parametrize('context', ['grad', 'vmap', 'vmap_of_another', 'forward_ad', 'trace', 'fake', 'mode'])
+def test_direct_calls_leave_transformed_calls_to_the_operator_class(mobula, context):
+    """torch.func, tracing, forward mode and dispatch modes have to see the autograd function."""
+    from torch.autograd import forward_ad
+    from torch.utils.flop_counter import FlopCounterMode
+    direct = native.torch_direct().ROIAlign
+    x = torch.randn(1, 4, 8, 9, device='cuda')
+    rois = torch.tensor([[0, 1, 2, 30, 20]], device='cuda', dtype=torch.float32)
+    kw = dict(pooled_size=(2, 2), spatial_scale=0.25, sampling_ratio=2)
+    seen = []
+
+    def call(a):
+        seen.append(direct(a, rois, **kw))
+        return a.sum()
+
+    def call_on_captured(a):
+        seen.append(direct(x, rois, **kw))
+        return a.sum()
+    if context == 'grad':
+        torch.func.grad(call)(x)
+    elif context == 'vmap':
+        torch.func.vmap(call)(x[None])
+    elif context == 'vmap_of_another':
+        torch.func.vmap(call_on_captured)(x)
+    elif context == 'forward_ad':
+        with forward_ad.dual_level():
+            call(forward_ad.make_dual(x, torch.ones_like(x)))
+    elif context == 'trace':
+        torch.jit.trace(call, (x,), check_trace=False)
+    elif context == 'fake':
+        from torch._subclasses.fake_tensor import FakeTensorMode
+        with FakeTensorMode() as mode:
+            call(mode.from_tensor(x))
+    else:
+        with FlopCounterMode(display=False):
+            call(x)
+    assert seen == [NotImplemented]
+
+
+def test_direct_backward_refuses_batched_gradients(mobula):
+    x = torch.randn(1, 4, 8, 9, device='cuda', requires_grad=True)
+    rois = torch.tensor([[0, 1, 2, 30, 20]], device='cuda', dtype=torch.float32)
+    y = native.torch_direct().ROIAlign(x, rois, (2, 2), 0.25, 2)
+    with pytest.raises(RuntimeError):
+        torch.autograd.grad(y, x, torch.ones((3,) + y.shape, device='cuda'), is_grads_batched=True)
+
+
+def test_adaptive_backward_waits_behind_a_busy_stream(mobula):
+    """The number of weight windows is awaited by the host: as long as the stream is busy, and without
+    leaving an error behind."""
+    x = torch.randn(1, 4, 24, 25, device='cuda', requires_grad=True)
+    rois = torch.tensor([[0, 1, 2, 80, 90]], device='cuda', dtype=torch.float32)
+    a = torch.randn(4096, 4096, device='cuda')
+    kw = dict(pooled_size=(2, 2), spatial_scale=0.25, sampling_ratio=0)
+    (want,) = torch.autograd.grad(mobula.op.ROIAlign(x, rois, **kw).sum(), x)
+    y = mobula.op.ROIAlign(x, rois, **kw).sum()
+    for _ in range(30):
+        a = (a @ a) * 1e-3
+    (got,) = torch.autograd.grad(y, x)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize('bias,image_grad', [(True, True), (False, True), (True, False)])
 def test_direct_convolution_agrees_with_the_operator_class(mobula, bias, image_grad):
     mobula.op.load('Convolution')
@@ -258,7 +320,6 @@ def test_host_arrays_of_several_sizes_and_from_several_threads(mobula, shape):
     """Arrays in host memory go through pinned slots in pieces: every element arrives, also when threads
     use the ring at once and after its memory was given back."""
     import threading
-    from mobulaop_amd import native
     rng = np.random.default_rng(3)
     N, C, H, W = shape
     rois = np.array([[n % N, 3 * n % 40, 5, 3 * n % 40 + 30.5, 60] for n in range(100)], dtype=np.float32)
