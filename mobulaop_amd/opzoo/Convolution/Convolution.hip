@@ -145,8 +145,11 @@ void launch_igemm_b16(const Ops& ops, float* piece_buffer, hipStream_t stream) {
   else launch_igemm_b16_shape<Ops, conv::WideShapeB16>(ops, 0, ops.Ncols, piece_buffer, stream);
 }
 
-// workgroups the weight gradient aims at: four per CU of a 256-CU device
-constexpr long long kWeightSlots = 1024;
+// workgroups the weight gradient aims at: two rounds of what a 256-CU device holds at a time, three to a
+// CU (256 channels and filters, 32 x 56 x 56, 3 x 3: 928 us and 17 for adding the slices up, one round
+// 928 and 9; with two to a CU 967 and 7, four, whose loop has too few registers, 993 and 11).  Longer sums
+// lose more: 3.3e-7 of the result against 64 bits, 4.4e-7 with one round.
+constexpr long long kWeightSlots = 1536;
 
 size_t align_to_256(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
@@ -511,8 +514,9 @@ bool with_tiles(const PatchProduct& p, const F& f) {
   return with_cut<conv::PatchTile32>(p, f);
 }
 
-// Clocks of a K step of igemm_kernel (three workgroups to a CU, whole tiles of 128 x 128).
-constexpr double kGatherStep = 2750.0;
+// Clocks of a K step of igemm_kernel (whole tiles of 128 x 128; 905 us at 2.3 GHz for 6.1 tiles of 144
+// steps to a CU, and a last round).
+constexpr double kGatherStep = 2500.0;
 
 // CU clocks of the product from patches; < 0: it does not fit.
 double patch_product_cost(const PatchProduct& p) {
@@ -694,7 +698,7 @@ bool weight_gradient_with(const conv::Geometry& g, const float* dy, const float*
   // but it needs a padded copy of x at unit stride along a row, and tests every pixel at others
   const double here = cut.cost * g.N * static_cast<double>(tiles);
   const long long padded = static_cast<long long>(g.N) * g.C * (g.H + 2 * g.pad_h) * (g.W + 2 * g.pad_w);
-  const double there = (g.stride_w == 1 ? 2670.0 : 5000.0) * conv::k_steps(g.N * ohw) *
+  const double there = (g.stride_w == 1 ? 2540.0 : 4870.0) * conv::k_steps(g.N * ohw) *
                            ((g.D + conv::Tile::BM - 1) / conv::Tile::BM) * ((cols + conv::Tile::BN - 1) / conv::Tile::BN) +
                        (g.stride_w == 1 ? 8.0 * padded / 4.5e12 * 2.4e9 * 256.0 : 0.0);
   if (here > there) return false;
@@ -929,7 +933,7 @@ MOBULA_KERNEL conv2d_backward_weight_kernel(const int n, const T* dy, const T* x
   ops.dy = dy; ops.x = x; ops.g = g;
   ops.M = g.D; ops.Ncols = g.C * g.KH * g.KW; ops.K = 0; ops.k_begin = 0;
   // K = N*OH*OW is long and the result small: K is cut into slices of whole K
-  // steps, as many as give every CU four workgroups; the partial sums of the
+  // steps, as many as give every CU six workgroups; the partial sums of the
   // slices are added in a fixed order afterwards.
   const int row_tiles = (ops.M + conv::Tile::BM - 1) / conv::Tile::BM;
   const long long per_slice_tiles = static_cast<long long>(row_tiles) * ((ops.Ncols + conv::Tile::BN - 1) / conv::Tile::BN);

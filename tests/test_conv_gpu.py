@@ -461,3 +461,28 @@ def test_fp32_products_from_patches(shape):
     _call('conv2d_backward_bias_cd239a08', ctypes.c_int(D), _ptr(dyd), ctypes.c_int(0), ctypes.c_int(N),
           ctypes.c_int(y.shape[2] * y.shape[3]), _ptr(db))
     _close(db, dy.double().sum((0, 2, 3)), 'db', 1e-5)
+
+
+@pytest.mark.parametrize('channels,filters', [(16, 128), (32, 130), (48, 100), (128, 16), (130, 32), (100, 48)])
+def test_fp32_gathered_products_of_few_steps(channels, filters):
+    """Tiles of one, two and three K steps (the loop requests two ahead), rows and columns that end
+    within a tile; the weight gradient's slices are one K step each."""
+    g = torch.Generator().manual_seed(78)
+    x, w = torch.randn(3, channels, 9, 15, generator=g), torch.randn(filters, channels, 1, 1, generator=g)
+    dy = torch.randn(3, filters, 9, 15, generator=g)
+    xr, wr = x.double().requires_grad_(True), w.double().requires_grad_(True)
+    y_ref = F.conv2d(xr, wr)
+    y_ref.backward(dy.double())
+    geo = _ci(3, channels, 9, 15, filters, 1, 1, 0, 0, 1, 1, 1, 1)
+    xd, wd, dyd = x.cuda(), w.cuda(), dy.cuda()
+    y = torch.full(dy.shape, float('nan'), device='cuda')
+    _call('conv2d_forward_c6a7aa85', ctypes.c_int(y.numel()), _ptr(xd), _ptr(wd), _ptr(wd), ctypes.c_int(0), *geo, _ptr(y))
+    _close(y, y_ref, 'y', 1e-5)
+    for start, accumulate in ((float('nan'), 0), (1.0, 1)):
+        dx, dw = torch.full(x.shape, start, device='cuda'), torch.full(w.shape, start, device='cuda')
+        _call('conv2d_backward_data_ecf81c91', ctypes.c_int(dx.numel()), _ptr(dyd), _ptr(wd), ctypes.c_int(accumulate),
+              *geo, _ptr(dx))
+        _call('conv2d_backward_weight_ecf81c91', ctypes.c_int(dw.numel()), _ptr(dyd), _ptr(xd), ctypes.c_int(accumulate),
+              *geo, _ptr(dw))
+        _close(dx - accumulate, xr.grad, 'dx', 1e-5)
+        _close(dw - accumulate, wr.grad, 'dw', 1e-5)
