@@ -419,6 +419,11 @@ __device__ __forceinline__ void igemm_tile(const Ops& ops, int m0, int n0, int s
       ops.fetch_b(bctx, step, b_k, rb);
     }
   };
+  auto stage4 = [&](int buf, int b, int h) {   // fp32: half h of what this thread fetched of A (b = 0) or B
+    const float* const r = (b ? rb : ra) + 4 * h;
+    *reinterpret_cast<f32x4*>(b ? &Bs[buf][b_n * T::PITCH + b_k + 4 * h] : &As[buf][a_m * T::PITCH + a_k + 4 * h]) =
+        f32x4{r[0], r[1], r[2], r[3]};
+  };
   auto stage = [&](int buf) {
     if (BF16) {
       typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
@@ -443,10 +448,7 @@ __device__ __forceinline__ void igemm_tile(const Ops& ops, int m0, int n0, int s
       }
     } else {
 #pragma unroll
-      for (int j = 0; j < 8; j += 4) {
-        *reinterpret_cast<f32x4*>(&As[buf][a_m * T::PITCH + a_k + j]) = f32x4{ra[j], ra[j + 1], ra[j + 2], ra[j + 3]};
-        *reinterpret_cast<f32x4*>(&Bs[buf][b_n * T::PITCH + b_k + j]) = f32x4{rb[j], rb[j + 1], rb[j + 2], rb[j + 3]};
-      }
+      for (int q = 0; q < 4; ++q) stage4(buf, q >> 1, q & 1);
     }
   };
 
@@ -463,7 +465,7 @@ __device__ __forceinline__ void igemm_tile(const Ops& ops, int m0, int n0, int s
     // 32 x 256 x 56 x 56, 256 filters 3 x 3, with fetch, products, stage and barrier one after the other,
     // forward / data gradient / weight gradient: 1011 / 1014 / 974 us; LDS accesses under products 984 /
     // 982 / 937; loads between them 924 / 916 / 937; results written without a test per element 914 / 894 /
-    // 928 (without any load after the first steps it is 868 / 870 / 825).
+    // 928; the LDS writes where they stand 880 / 873 / 915 (without any load after the first steps it is 868 / 870 / 825).
     f32x4 fa[2][2], fb[2][2];
     auto read = [&](int buf, int h) {
 #pragma unroll
@@ -497,11 +499,27 @@ __device__ __forceinline__ void igemm_tile(const Ops& ops, int m0, int n0, int s
       if constexpr (Ops::kGathered) step = ops.load_step(ahead);
       __builtin_amdgcn_sched_barrier(0);
       multiply(0, 1);
-      multiply(0, 2);
       __builtin_amdgcn_sched_barrier(0);
-      stage(buf ^ 1);
-      if constexpr (!Ops::kGathered)
+      if constexpr (Ops::kGathered) {
+        // (behind four more products it takes 911 / 880 us instead of 880 / 873)
+        stage(buf ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(0, 2);
+        __builtin_amdgcn_sched_barrier(0);
+      } else {
+        // one LDS write between two matrix instructions (933 -> 915 us; the gathered products lose by
+        // it: 880 -> 984)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            stage4(buf ^ 1, i, j);
+            __builtin_amdgcn_sched_barrier(0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[0][i][2], fb[0][j][2], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+          }
         if (s + 2 < steps) step = ops.next_step(step, s + 2);
+      }
       ops.fetch_a(m0 + a_m, step, ahead, a_k, ra);
       __builtin_amdgcn_sched_barrier(0);
       multiply(0, 3);

@@ -515,7 +515,7 @@ bool with_tiles(const PatchProduct& p, const F& f) {
 }
 
 // Clocks of a K step of igemm_kernel (whole tiles of 128 x 128; 905 us at 2.3 GHz for 6.1 tiles of 144
-// steps to a CU, and a last round).
+// steps to a CU, and a last round; 880 since).
 constexpr double kGatherStep = 2500.0;
 
 // CU clocks of the product from patches; < 0: it does not fit.
