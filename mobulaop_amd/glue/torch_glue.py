@@ -137,9 +137,10 @@ class OpGen(object):
 
     def _offer_direct_call(self, inputs):
         """From the first call on GPU tensors on, an operator class that names a native call
-        (`torch_direct`) is asked for through it: see csrc/torch_direct.cpp."""
-        name, handle = getattr(self.op, 'torch_direct', None), CUSTOM_OP_LIST.get(self.name)
-        if (name is not None and handle is not None and getattr(handle.op, 'torch_direct', None) == name and
+        (`torch_direct`) is asked for through it: see csrc/torch_direct.cpp.  The class itself has to
+        name it: a subclass may do something else, in code of its own."""
+        name, handle = vars(self.op).get('torch_direct'), CUSTOM_OP_LIST.get(self.name)
+        if (name is not None and handle is not None and vars(handle.op).get('torch_direct') == name and
                 not handle.attrs and handle.direct is None and any(t.is_cuda for t in inputs)):
             handle.direct = getattr(native.torch_direct(), name)
 

@@ -148,6 +148,33 @@ def test_torch_cpu_tensor_goes_through_torch_glue(mobula):
         mobula.op._Twice(a, other=np.zeros(3))  # two frameworks in one call
 
 
+class _TensorOnAGpu:
+    """Stands for a torch tensor on a GPU where the glue asks whether one is among a call's inputs."""
+    is_cuda = True
+
+
+def test_only_classes_that_name_a_native_call_are_routed_to_it(mobula, monkeypatch):
+    """Calls of the bundled class go to the native module from the first GPU tensors on; a registered
+    subclass with passes of its own keeps running these."""
+    import types
+    from mobulaop_amd import native
+    from mobulaop_amd.glue import common, torch_glue
+    monkeypatch.setattr(native, 'torch_direct', lambda: types.SimpleNamespace(ROIAlign=lambda *a, **k: 'native'))
+    base = mobula.op.ROIAlign
+
+    class _Doubled(base.op):
+        def forward(self, data, rois):
+            return 2 * data
+    handles = [mobula.op.register('_DoubledROIAlign')(_Doubled),
+               mobula.op.register('_SameROIAlign')(type('_Same', (base.op,), {'torch_direct': 'ROIAlign'}))]
+    for handle, routed in zip([base] + handles, [True, False, True]):
+        monkeypatch.setattr(handle, 'direct', None)
+        torch_glue.OpGen(handle.op, handle.name)._offer_direct_call([_TensorOnAGpu()])
+        assert (handle.direct is not None) == routed, handle.name
+    for handle in handles:
+        del common.CUSTOM_OP_LIST[handle.name]
+
+
 def test_roialign_infer_shape_and_req_null(mobula):
     op = mobula.op.ROIAlign[np.ndarray](pooled_size=(7, 5), spatial_scale=0.5, sampling_ratio=2)
     ins, outs = op.infer_shape([(2, 3, 8, 9), (4, 5)])
