@@ -142,7 +142,7 @@ class OpGen(object):
         name, handle = vars(self.op).get('torch_direct'), CUSTOM_OP_LIST.get(self.name)
         if (name is not None and handle is not None and vars(handle.op).get('torch_direct') == name and
                 not handle.attrs and handle.direct is None and any(t.is_cuda for t in inputs)):
-            handle.direct = getattr(native.torch_direct(), name)
+            handle.direct = getattr(native.torch_direct(), name, None)   # (no module: the class goes on)
 
     def register(self):
         return _make_module(self.op, self.name, _make_function(self.op, self.name))

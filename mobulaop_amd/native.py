@@ -16,6 +16,7 @@ There is no CPU implementation behind this module: if the library is missing
 import ctypes
 import importlib.util
 import os
+import warnings
 
 from .config import config
 from .dtype import CTYPENAME2CTYPE
@@ -72,26 +73,30 @@ def get_option(name):
 
 
 _torch_direct = None
+_torch_direct_error = None   # why it cannot be had (asked for once)
 
 
 def torch_direct():
     """The module that takes the bundled operators' calls on torch GPU tensors straight to
-    the library (csrc/torch_direct.cpp); builds it first if it is absent and can be."""
-    global _torch_direct
-    if _torch_direct is None:
-        library()   # (the module is linked against it)
+    the library (csrc/torch_direct.cpp); builds it first if it is absent and can be.  Only a
+    shorter way: None, after one warning, where it cannot be built or loaded (no compiler, no
+    Python headers, a tree that cannot be written), and the operator classes take the calls."""
+    global _torch_direct, _torch_direct_error
+    if _torch_direct is None and _torch_direct_error is None:
+        library()   # (the module is linked against it; without it nothing runs)
         from . import build as _build
-        if not os.path.exists(_build.TORCH_LIB_PATH):
-            _build.build_torch_direct()
-        import torch  # noqa: F401  (its libraries have to be loaded first)
-        spec = importlib.util.spec_from_file_location('_torch_direct', _build.TORCH_LIB_PATH)
         try:
+            if not os.path.exists(_build.TORCH_LIB_PATH):
+                _build.build_torch_direct()
+            import torch  # noqa: F401  (its libraries have to be loaded first)
+            spec = importlib.util.spec_from_file_location('_torch_direct', _build.TORCH_LIB_PATH)
             module = importlib.util.module_from_spec(spec)
-        except ImportError as exc:
-            raise RuntimeError('cannot load {}: {} -- build it with `python -m mobulaop_amd.build`'.format(
-                _build.TORCH_LIB_PATH, exc))
-        spec.loader.exec_module(module)
-        _torch_direct = module
+            spec.loader.exec_module(module)
+            _torch_direct = module
+        except (ImportError, OSError, RuntimeError) as exc:
+            _torch_direct_error = exc
+            warnings.warn('{} cannot be built or loaded: torch calls go through the operator classes, which '
+                          'cost the host more ({})'.format(_build.TORCH_LIB_PATH, exc))
     return _torch_direct
 
 

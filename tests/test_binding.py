@@ -175,6 +175,30 @@ def test_only_classes_that_name_a_native_call_are_routed_to_it(mobula, monkeypat
         del common.CUSTOM_OP_LIST[handle.name]
 
 
+@pytest.mark.parametrize('fault', ['no compiler', 'compiler fails', 'does not load'])
+def test_calls_go_on_without_the_native_torch_module(mobula, monkeypatch, tmp_path, fault):
+    """Where the module cannot be had the operator class keeps the call: one warning, one attempt."""
+    from mobulaop_amd import build, native
+    from mobulaop_amd.glue import torch_glue
+    attempts = []
+
+    def build_torch_direct():
+        attempts.append(1)
+        if fault != 'does not load':
+            raise FileNotFoundError('g++') if fault == 'no compiler' else RuntimeError('g++ failed')
+        (tmp_path / '_torch_direct.so').write_bytes(b'not a shared object')
+    monkeypatch.setattr(build, 'TORCH_LIB_PATH', str(tmp_path / '_torch_direct.so'))
+    monkeypatch.setattr(build, 'build_torch_direct', build_torch_direct)
+    monkeypatch.setattr(native, '_torch_direct', None)
+    monkeypatch.setattr(native, '_torch_direct_error', None, raising=False)
+    monkeypatch.setattr(mobula.op.ROIAlign, 'direct', None)
+    gen = torch_glue.OpGen(mobula.op.ROIAlign.op, 'ROIAlign')
+    with pytest.warns(UserWarning, match='operator classes'):
+        gen._offer_direct_call([_TensorOnAGpu()])
+    gen._offer_direct_call([_TensorOnAGpu()])
+    assert mobula.op.ROIAlign.direct is None and attempts == [1]
+
+
 def test_roialign_infer_shape_and_req_null(mobula):
     op = mobula.op.ROIAlign[np.ndarray](pooled_size=(7, 5), spatial_scale=0.5, sampling_ratio=2)
     ins, outs = op.infer_shape([(2, 3, 8, 9), (4, 5)])
