@@ -6,10 +6,11 @@ One shared object, `csrc/libmobula_hip.so`, holds the runtime and every
 operator's entry points.  It stays in the source tree (next to the code that
 loads it).  Replaces the per-call JIT of the reference
 (mobula/building/build.py:64-146) with one explicit hipcc invocation.  A second
-one, `csrc/_torch_direct.so` (host code only), is the bundled operators' way from
+one, `csrc/_torch_direct.<key>.so` (host code only), is the bundled operators' way from
 torch tensors into that library; it is built where torch is installed.
 """
 import glob
+import hashlib
 import importlib.util
 import os
 import shutil
@@ -22,7 +23,7 @@ from .config import config
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, 'csrc')
 LIB_PATH = os.path.join(CSRC, 'libmobula_hip.so')
-TORCH_LIB_PATH = os.path.join(CSRC, '_torch_direct.so')
+TORCH_SOURCES = (os.path.join(CSRC, 'torch_direct.cpp'), os.path.join(_HERE, '..', 'include', 'mobula_roialign.h'))
 
 
 def sources():
@@ -72,21 +73,34 @@ def build_library(verbose=False):
     return LIB_PATH
 
 
+def torch_lib_path():
+    """Where the torch side lies, named by all that it was compiled against -- its sources, this torch
+    and this Python: a file left by another torch, whose C++ types may differ, is not found."""
+    import torch
+    digest = hashlib.sha256(repr((torch.__version__, torch.version.git_version, torch.compiled_with_cxx11_abi(),
+                                  sysconfig.get_config_var('SOABI'))).encode())
+    for path in TORCH_SOURCES:
+        with open(path, 'rb') as f:
+            digest.update(f.read())
+    return os.path.join(CSRC, '_torch_direct.{}.so'.format(digest.hexdigest()[:12]))
+
+
 def build_torch_direct(verbose=False):
     """The torch side (csrc/torch_direct.cpp) against the launcher library; None where
-    torch is not installed."""
+    torch is not installed.  (One file per torch_lib_path(): environments that share a tree keep theirs.)"""
     if importlib.util.find_spec('torch') is None:
         return None
     torch_dir = os.path.dirname(importlib.util.find_spec('torch').origin)
+    path = torch_lib_path()
     rocm = os.path.dirname(os.path.dirname(os.path.realpath(shutil.which(config.HIPCC) or '/opt/rocm/bin/hipcc')))
-    tmp = TORCH_LIB_PATH + '.tmp.{}'.format(os.getpid())
+    tmp = path + '.tmp.{}'.format(os.getpid())
     cmd = (['g++', '-O2', '-std=c++17', '-fPIC', '-shared', '-Wall',
             # how torch's own headers ask for the ROCm build they are part of
             '-D__HIP_PLATFORM_AMD__=1', '-DUSE_ROCM=1',
             '-I' + os.path.join(_HERE, '..', 'include'), '-I' + sysconfig.get_paths()['include'],
             '-I' + os.path.join(torch_dir, 'include'),
             '-I' + os.path.join(torch_dir, 'include', 'torch', 'csrc', 'api', 'include'),
-            '-I' + os.path.join(rocm, 'include'), '-o', tmp, os.path.join(CSRC, 'torch_direct.cpp'),
+            '-I' + os.path.join(rocm, 'include'), '-o', tmp, TORCH_SOURCES[0],
             '-L' + CSRC, '-lmobula_hip', '-L' + os.path.join(torch_dir, 'lib'), '-lc10', '-lc10_hip', '-ltorch_cpu',
             '-ltorch_python', '-Wl,-rpath,$ORIGIN'])
     if verbose or config.SHOW_BUILDING_COMMAND:
@@ -96,8 +110,8 @@ def build_torch_direct(verbose=False):
         if os.path.exists(tmp):
             os.remove(tmp)
         raise RuntimeError('g++ failed:\n' + proc.stdout)
-    os.replace(tmp, TORCH_LIB_PATH)
-    return TORCH_LIB_PATH
+    os.replace(tmp, path)
+    return path
 
 
 if __name__ == '__main__':

@@ -78,7 +78,7 @@ _torch_direct_error = None   # why it cannot be had (asked for once)
 
 def torch_direct():
     """The module that takes the bundled operators' calls on torch GPU tensors straight to
-    the library (csrc/torch_direct.cpp); builds it first if it is absent and can be.  Only a
+    the library (csrc/torch_direct.cpp); builds it first if none for this torch is there.  Only a
     shorter way: None, after one warning, where it cannot be built or loaded (no compiler, no
     Python headers, a tree that cannot be written), and the operator classes take the calls."""
     global _torch_direct, _torch_direct_error
@@ -86,17 +86,17 @@ def torch_direct():
         library()   # (the module is linked against it; without it nothing runs)
         from . import build as _build
         try:
-            if not os.path.exists(_build.TORCH_LIB_PATH):
+            path = _build.torch_lib_path()   # (imports torch: its libraries have to be loaded first)
+            if not os.path.exists(path):
                 _build.build_torch_direct()
-            import torch  # noqa: F401  (its libraries have to be loaded first)
-            spec = importlib.util.spec_from_file_location('_torch_direct', _build.TORCH_LIB_PATH)
+            spec = importlib.util.spec_from_file_location('_torch_direct', path)
             module = importlib.util.module_from_spec(spec)
             spec.loader.exec_module(module)
             _torch_direct = module
         except (ImportError, OSError, RuntimeError) as exc:
             _torch_direct_error = exc
-            warnings.warn('{} cannot be built or loaded: torch calls go through the operator classes, which '
-                          'cost the host more ({})'.format(_build.TORCH_LIB_PATH, exc))
+            warnings.warn('csrc/torch_direct.cpp cannot be built or loaded: torch calls go through the operator '
+                          'classes, which cost the host more ({})'.format(exc))
     return _torch_direct
 
 

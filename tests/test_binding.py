@@ -187,7 +187,7 @@ def test_calls_go_on_without_the_native_torch_module(mobula, monkeypatch, tmp_pa
         if fault != 'does not load':
             raise FileNotFoundError('g++') if fault == 'no compiler' else RuntimeError('g++ failed')
         (tmp_path / '_torch_direct.so').write_bytes(b'not a shared object')
-    monkeypatch.setattr(build, 'TORCH_LIB_PATH', str(tmp_path / '_torch_direct.so'))
+    monkeypatch.setattr(build, 'torch_lib_path', lambda: str(tmp_path / '_torch_direct.so'))
     monkeypatch.setattr(build, 'build_torch_direct', build_torch_direct)
     monkeypatch.setattr(native, '_torch_direct', None)
     monkeypatch.setattr(native, '_torch_direct_error', None, raising=False)
@@ -197,6 +197,21 @@ def test_calls_go_on_without_the_native_torch_module(mobula, monkeypatch, tmp_pa
         gen._offer_direct_call([_TensorOnAGpu()])
     gen._offer_direct_call([_TensorOnAGpu()])
     assert mobula.op.ROIAlign.direct is None and attempts == [1]
+
+
+def test_the_native_torch_module_belongs_to_one_torch_and_its_sources(monkeypatch, tmp_path):
+    import torch
+    from mobulaop_amd import build
+    paths = [build.torch_lib_path()]
+    assert build.torch_lib_path() == paths[0]
+    monkeypatch.setattr(torch, '__version__', '0.0')
+    paths.append(build.torch_lib_path())
+    monkeypatch.undo()
+    other = tmp_path / 'torch_direct.cpp'
+    other.write_text('// another source')
+    monkeypatch.setattr(build, 'TORCH_SOURCES', (str(other),) + build.TORCH_SOURCES[1:])
+    paths.append(build.torch_lib_path())
+    assert len(set(paths)) == 3
 
 
 def test_roialign_infer_shape_and_req_null(mobula):
