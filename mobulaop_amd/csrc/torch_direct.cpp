@@ -1,6 +1,6 @@
 // The bundled operators for torch tensors on a GPU, without Python between the call
 // and the launcher: `mobula.op.ROIAlign(...)` and `mobula.op.Conv2D(...)` hand their
-// arguments here (glue/torch_glue.py: direct_calls), forward runs at once, backward is
+// arguments here (glue/torch_glue.py: _offer_direct_call), forward runs at once, backward is
 // a node of torch's graph that runs on the engine's thread without the interpreter.
 //
 // What it saves: a forward + backward of eight boxes keeps the GPU busy for 34 us, and
@@ -9,8 +9,9 @@
 // per call, and the interpreter lock handed to the engine's thread and back.
 //
 // A call this file does not take (other tensor types, arguments it cannot read, shapes
-// the operator class would refuse, calls under a transform of torch's) is answered with NotImplemented, and the operator
-// class takes it as before: what is an error stays the error it was.
+// the operator class would refuse, calls under a transform of torch's or with hooks on all
+// modules) is answered with NotImplemented, and the operator class takes it as before: what is
+// an error stays the error it was.
 //
 // Semantics are those of opzoo/ROIAlign/ROIAlign.py and opzoo/Convolution/Convolution.py
 // under the torch glue: fresh outputs and gradients, boxes get zeros, channels-last maps
@@ -337,11 +338,26 @@ bool read_pair(PyObject* o, int (&out)[2]) {
   return read_int(PySequence_Fast_GET_ITEM(o, 0), &out[0]) && read_int(PySequence_Fast_GET_ITEM(o, 1), &out[1]);
 }
 
-// A call that torch watches or transforms (torch.func, tracing, a dispatch mode): what it needs to
-// see is the operator class's autograd function.
+// Hooks on every module's calls (torch.nn.modules.module.register_module_*_hook): the operator class's
+// call is one, of an nn.Module.
+bool has_module_hooks() {
+  static PyObject* const module = PyImport_ImportModule("torch.nn.modules.module");
+  static PyObject* const names[] = {
+      PyUnicode_InternFromString("_global_forward_pre_hooks"), PyUnicode_InternFromString("_global_forward_hooks"),
+      PyUnicode_InternFromString("_global_backward_pre_hooks"), PyUnicode_InternFromString("_global_backward_hooks")};
+  if (module == nullptr) { PyErr_Clear(); return true; }
+  for (PyObject* const name : names) {
+    PyObject* const hooks = name == nullptr ? nullptr : PyDict_GetItem(PyModule_GetDict(module), name);
+    if (hooks == nullptr || !PyDict_Check(hooks) || PyDict_Size(hooks) != 0) return true;
+  }
+  return false;
+}
+
+// A call that torch watches or transforms (torch.func, tracing, a dispatch mode, hooks): what it needs to
+// see is the operator class's module and autograd function.
 bool is_watched() {
   return at::tracer::impl::is_dispatch_enabled() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
-         c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+         c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) || has_module_hooks();
 }
 
 // A plain tensor (or parameter) on a GPU, with memory of its own and no forward-mode tangent.

@@ -268,6 +268,25 @@ def test_direct_calls_leave_transformed_calls_to_the_operator_class(mobula, cont
     assert seen == [NotImplemented]
 
 
+@pytest.mark.parametrize('kind', ['forward_pre', 'forward', 'full_backward_pre', 'full_backward'])
+def test_hooks_on_all_modules_see_direct_calls(mobula, kind):
+    """The operator class's call is a module's: with such a hook registered it keeps the call."""
+    from torch.nn.modules import module
+    x = torch.randn(1, 4, 8, 9, device='cuda', requires_grad=True)
+    rois = torch.tensor([[0, 1, 2, 30, 20]], device='cuda', dtype=torch.float32)
+    kw = dict(pooled_size=(2, 2), spatial_scale=0.25, sampling_ratio=2)
+    for _ in range(2):
+        mobula.op.ROIAlign(x, rois, **kw)
+    seen = []
+    hook = getattr(module, 'register_module_{}_hook'.format(kind))(lambda m, *a: seen.append(type(m).__name__))
+    try:
+        mobula.op.ROIAlign(x, rois, **kw).sum().backward()
+    finally:
+        hook.remove()
+    assert seen == ['_ROIAlign_TORCH_NN_MODULE']
+    assert isinstance(native.torch_direct().ROIAlign(x, rois, **kw), torch.Tensor)   # (and not without one)
+
+
 def test_direct_backward_refuses_batched_gradients(mobula):
     x = torch.randn(1, 4, 8, 9, device='cuda', requires_grad=True)
     rois = torch.tensor([[0, 1, 2, 30, 20]], device='cuda', dtype=torch.float32)
