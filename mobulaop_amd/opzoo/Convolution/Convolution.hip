@@ -237,8 +237,8 @@ bool plan_gather(GatherPlan* plan, const char* what, const conv::Geometry& g, co
   plan->K = static_cast<int>(k);
   conv::build_gather_steps_kernel<<<(count + 255) / 256, 256, 0, stream>>>(plan->steps, count, per_tap, g.KW,
                                                                           g.dil_h, g.dil_w, plane_row, sign);
-  conv::arrange_weights_kernel<<<blocks_for(wcount), 256, 0, stream>>>(w, plan->weights, M, mpad, channels, cpad,
-                                                                       taps, stride_m, stride_c);
+  conv::arrange_weights_kernel<<<blocks_for_all(wcount), 256, 0, stream>>>(w, plan->weights, M, mpad, channels, cpad,
+                                                                           taps, stride_m, stride_c);
   return true;
 }
 

@@ -16,6 +16,7 @@ import torch.nn.functional as F
 
 from mobulaop_amd import native
 from oracle import conv as oracle
+import abi_util as abi
 
 pytestmark = pytest.mark.gpu
 CONV_TOL = 1e-3
@@ -486,3 +487,24 @@ def test_fp32_gathered_products_of_few_steps(channels, filters):
               *geo, _ptr(dw))
         _close(dx - accumulate, xr.grad, 'dx', 1e-5)
         _close(dw - accumulate, wr.grad, 'dw', 1e-5)
+
+
+@pytest.mark.parametrize('channels,filters,kernel', [(512, 512, 3), (256, 256, 7)])
+def test_weights_of_more_than_two_million_elements(channels, filters, kernel):
+    """The gathered products read a rearranged copy of the weights from the workspace: all of it is written."""
+    g = torch.Generator().manual_seed(79)
+    x = torch.randn(1, channels, 14, 14, generator=g)
+    w = torch.randn(filters, channels, kernel, kernel, generator=g)
+    dy = torch.randn(1, filters, 14, 14, generator=g)
+    xr = x.double().requires_grad_(True)
+    y_ref = F.conv2d(xr, w.double(), padding=kernel // 2)
+    y_ref.backward(dy.double())
+    geo = _ci(1, channels, 14, 14, filters, kernel, kernel, kernel // 2, kernel // 2, 1, 1, 1, 1)
+    xd, wd, dyd = x.cuda(), w.cuda(), dy.cuda()
+    y, dx = torch.empty(dy.shape, device='cuda'), torch.empty(x.shape, device='cuda')
+    abi.poison_workspace(128 << 20)
+    _call('conv2d_forward_c6a7aa85', ctypes.c_int(y.numel()), _ptr(xd), _ptr(wd), _ptr(wd), ctypes.c_int(0), *geo, _ptr(y))
+    _close(y, y_ref, 'y', 1e-5)
+    abi.poison_workspace(128 << 20)
+    _call('conv2d_backward_data_ecf81c91', ctypes.c_int(dx.numel()), _ptr(dyd), _ptr(wd), ctypes.c_int(0), *geo, _ptr(dx))
+    _close(dx, xr.grad, 'dx', 1e-5)
