@@ -42,6 +42,10 @@ long long arg_extent(int index);
 // between asynchronous calls is ordered behind its previous call; every entry
 // point ends with finish_call(), which keeps the book for that.
 void* workspace(size_t bytes);
+// The same for a caller that has another way: null, without an error, where the buffer cannot be had
+// (it would have to grow while the stream is being captured or a recorded graph uses it, or the
+// device has no memory for it).
+void* workspace_if_possible(size_t bytes);
 long long release_workspace();   // frees the calling thread's buffer on the current device
 // A call recorded into a HIP graph pins the buffer (replays use its address): it is then
 // neither grown nor released (an error instead) until unpin_workspace().

@@ -62,9 +62,9 @@ Scratch* scratch_of_current_device() {
 }
 std::mutex g_mutex;
 std::map<std::string, long long> g_options;
-}  // namespace
 
-void* workspace(size_t bytes) {
+// `required`: what keeps the buffer from being had is an error of the call.
+void* take_workspace(size_t bytes, bool required) {
   Scratch* const s = scratch_of_current_device();
   if (s == nullptr) return nullptr;
   CallState& st = call_state();
@@ -93,6 +93,7 @@ void* workspace(size_t bytes) {
           hipStreamWaitEvent(st.stream, s->idle, 0) != hipSuccess) {
         (void)hipGetLastError();
         if (capturing) {   // (a device-wide wait would break the recording)
+          if (!required) return nullptr;
           set_error("the previous call of this thread ran on another stream and cannot be waited for while "
                     "this stream is being captured: synchronise that stream before recording");
           return nullptr;
@@ -101,9 +102,10 @@ void* workspace(size_t bytes) {
       }
       if (failed()) return nullptr;
     }
-    s->busy = false;   // ordered behind it from here on (finish_call marks the new call)
+    // (`last` names this stream once the call has the buffer; a call that does not get it leaves the book as it is)
   }
   if (s->bytes < bytes && (capturing || s->pinned)) {
+    if (!required) return nullptr;
     set_error("the workspace of this thread (%zu bytes) is too small for the call (%zu bytes) and cannot be "
               "replaced %s: make one ordinary call of the largest shape before recording, or call "
               "mobula_hip_unpin_workspace() once the graphs are gone", s->bytes, bytes,
@@ -116,14 +118,23 @@ void* workspace(size_t bytes) {
     s->ptr = nullptr;
     s->bytes = 0;
     size_t want = bytes + bytes / 4 + (1u << 20);
-    MOBULA_HIP_TRY(hipMalloc(&s->ptr, want));
-    if (failed()) { s->ptr = nullptr; return nullptr; }
+    const hipError_t status = hipMalloc(&s->ptr, want);
+    if (status != hipSuccess) {
+      if (required) MOBULA_HIP_TRY(status);
+      else (void)hipGetLastError();
+      s->ptr = nullptr;
+      return nullptr;
+    }
     s->bytes = want;
   }
   s->last = st.stream;
   st.used_workspace = true;
   return s->ptr;
 }
+}  // namespace
+
+void* workspace(size_t bytes) { return take_workspace(bytes, true); }
+void* workspace_if_possible(size_t bytes) { return take_workspace(bytes, false); }
 
 // Frees the calling thread's scratch buffer on the current device (hipFree waits
 // for the work that still uses it); returns the bytes given back.

@@ -216,8 +216,12 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
   }
   const size_t xt_bytes = (sizeof(T) * p.N * cblk * CB * pixels + 255) / 256 * 256;
   const bool fixed = p.fixed_scratch != nullptr;
-  // (with fixed scratch a map whose padded channels do not fit it takes the straightforward kernel)
-  const bool padded_beyond = fixed && p.C % roialign::BlockOf<T>::CPL != 0 && xt_bytes + sizeof(int) * p.R > p.fixed_scratch_bytes;
+  // A channel count that no lane's sixteen bytes divide: the copy is padded, to seven times the map's
+  // size at worst.  Where its memory cannot be had (fixed scratch too small, a stream being captured or a recorded graph
+  // with a smaller workspace, a full device) the straightforward kernel, which needs none, takes the call.
+  const bool padded = p.C % roialign::BlockOf<T>::CPL != 0;
+  const bool padded_beyond = fixed && padded && xt_bytes + sizeof(int) * p.R > p.fixed_scratch_bytes;
+  char* ws = nullptr;   // for the copy and the ROI order; null: the straightforward kernel
   // Few outputs of a fixed grid: one thread each, straight from the map, takes less time than the copy
   // (microseconds by size, measured: 13.5 per million outputs at 2 x 2 points, 2.7 for the gather from the
   // copy; the copy moves 6 TB/s).  Eight boxes of 64 channels on 32 x 32 pixels: 8.1 us a launch less;
@@ -234,8 +238,12 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
                 xt_bytes + sizeof(int) * p.R, p.fixed_scratch_bytes);
       return;
     }
-    char* const ws = fixed ? p.fixed_scratch : static_cast<char*>(mobula_hip::workspace(xt_bytes + sizeof(int) * p.R));
+    ws = static_cast<char*>(fixed    ? p.fixed_scratch
+                            : padded ? mobula_hip::workspace_if_possible(xt_bytes + sizeof(int) * p.R)
+                                     : mobula_hip::workspace(xt_bytes + sizeof(int) * p.R));
     if (failed()) return;
+  }
+  if (ws != nullptr) {
     T* const xt = reinterpret_cast<T*>(ws);
     // ROIs are visited in spatial order when the map is larger than the L2 caches
     // hold; a small map is read in the caller's order and the ordering kernel is left out

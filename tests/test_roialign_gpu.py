@@ -1109,3 +1109,48 @@ def test_few_boxes_on_a_large_map_copy_only_what_they_touch(W, dtype):
         want = oracle.forward(x.astype(np.float32), some[keep], pooled, scale, 0).astype(dtype)
         assert_parity(got[keep].astype(np.float32), want.astype(np.float32), FWD_TOL if dtype == np.float32 else FP16_TOL, 'y')
         assert not got[~keep].any()
+
+
+@pytest.mark.parametrize('S', [2, 0])
+@pytest.mark.parametrize('dtype,C', [(np.float32, 5), (np.float16, 81)])
+def test_odd_channel_counts_are_taken_without_a_workspace(dtype, C, S):
+    """Their blocked copy is padded to many times the map; where the workspace cannot be had -- nothing may be
+    allocated while a stream is being captured, a recorded graph holds a small one where it is -- the call
+    runs as it did without the copy."""
+    rng = np.random.default_rng(C)
+    x = rng.standard_normal((2, C, 30, 41)).astype(dtype)
+    rois = np.array([[n % 2, 3 * n, 2 * n, 5 * n + 20.5, 3 * n + 30] for n in range(40)], dtype=np.float32)
+    abi.set_impl('tiled')   # (the copy is made for any size)
+    want = oracle.forward(x.astype(np.float32), rois, (3, 4), 0.25, S).astype(dtype).astype(np.float32)
+    xd, rd, stream = abi.to_dev(x), abi.to_dev(rois), torch.cuda.Stream()
+    tol = FWD_TOL if dtype == np.float32 else FP16_TOL
+    torch.cuda.synchronize()
+    native.unpin_workspace()
+    native.release_workspace()
+    graphs = []
+    for pin in (False, True):
+        if pin:   # a graph of a call that needs a little of the workspace
+            native.release_workspace()
+            few, y_few = abi.to_dev(x[:1, :8 if C == 81 else 4, :5, :5]), []
+            abi.forward(few, rd[:1], (3, 4), 0.25, S)
+            graphs.append(torch.cuda.CUDAGraph())
+            with torch.cuda.graph(graphs[-1], stream=stream):
+                y_few.append(abi.forward(few, rd[:1], (3, 4), 0.25, S, stream=torch.cuda.current_stream().cuda_stream))
+            held = native.workspace_bytes()
+            big = abi.to_dev(np.tile(x, (1, 1, 8, 8)))
+            y = abi.forward(big, rd, (3, 4), 0.25, S)
+            assert native.workspace_bytes() == held
+            assert_parity(y.float().cpu().numpy(), oracle.forward(big.float().cpu().numpy(), rois, (3, 4), 0.25, S), tol, 'pinned')
+        else:
+            graphs.append(torch.cuda.CUDAGraph())
+            with torch.cuda.graph(graphs[-1], stream=stream):
+                y = abi.forward(xd, rd, (3, 4), 0.25, S, stream=torch.cuda.current_stream().cuda_stream)
+            for _ in range(3):
+                y.fill_(7.0)
+                graphs[-1].replay()
+                torch.cuda.synchronize()
+                assert_parity(y.float().cpu().numpy(), want, tol, 'captured')
+                assert_parity(abi.forward(xd, rd, (3, 4), 0.25, 2 if S == 0 else 1).float().cpu().numpy(),
+                              oracle.forward(x.astype(np.float32), rois, (3, 4), 0.25, 2 if S == 0 else 1), tol, 'between')
+    graphs.clear()
+    native.unpin_workspace()
