@@ -995,12 +995,13 @@ MOBULA_KERNEL conv2d_backward_bias_kernel(const int n, const T* dy, const int ac
   // sums added in order by a second kernel (one workgroup per filter: 95 us for 64 filters of
   // 8 x 112 x 112, the memory has 26 MB to give)
   hipStream_t stream = call_state().stream;
-  const int parts = std::max(1, std::min(batch, 1024 / n));
+  int parts = std::max(1, std::min(batch, 1024 / n));
   const bool wide = pixels % 4 == 0 && reinterpret_cast<uintptr_t>(dy) % 16 == 0;
   float* sums = db;
   if (parts > 1) {
-    sums = static_cast<float*>(mobula_hip::workspace(sizeof(float) * static_cast<size_t>(parts) * n));
+    sums = static_cast<float*>(mobula_hip::workspace_if_possible(sizeof(float) * static_cast<size_t>(parts) * n));
     if (failed()) return;
+    if (sums == nullptr) { sums = db; parts = 1; }   // (a first call under capture: one workgroup per filter needs none)
   }
   (wide ? conv::bias_grad_kernel<4> : conv::bias_grad_kernel<1>)<<<dim3(n, parts), 256, 0, stream>>>(
       dy, sums, batch, n, pixels, parts > 1 ? 0 : accumulate);

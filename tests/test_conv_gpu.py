@@ -508,3 +508,23 @@ def test_weights_of_more_than_two_million_elements(channels, filters, kernel):
     abi.poison_workspace(128 << 20)
     _call('conv2d_backward_data_ecf81c91', ctypes.c_int(dx.numel()), _ptr(dyd), _ptr(wd), ctypes.c_int(0), *geo, _ptr(dx))
     _close(dx, xr.grad, 'dx', 1e-5)
+
+
+def test_bias_gradient_can_be_recorded_first():
+    """Without a workspace, which cannot be had while a stream is being captured, one workgroup per filter
+    adds the images up."""
+    dy = torch.randn(5, 3, 7, 9, generator=torch.Generator().manual_seed(80))
+    dyd, db, stream = dy.cuda(), torch.zeros(3, device='cuda'), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    native.release_workspace()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        native.begin_call(torch.cuda.current_stream().cuda_stream, [])
+        native.library().conv2d_backward_bias_cd239a08(ctypes.c_int(0), *_ci(3), _ptr(dyd), *_ci(0, 5, 63), _ptr(db))
+        native.end_call('conv2d_backward_bias')
+    for _ in range(3):
+        db.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        _close(db, dy.double().sum((0, 2, 3)), 'db', 1e-5)
+        dyd.add_(0)   # (ordinary work between the replays)
