@@ -1026,8 +1026,9 @@ bool both_gradients_b16(const conv::Geometry& g, const float* dy, const float* x
   const Fit fit = plan_data_b16(&data, &prep, g, dy, weight, 0, dx);
   if (fit != kFits) return fit == kError;
   hipStream_t stream = call_state().stream;
-  char* const ws = static_cast<char*>(mobula_hip::workspace(prep.bytes + kPieceBytes));
-  if (failed()) return true;
+  // (both products' operands at a time; where there is no room for that, one product after the other)
+  char* const ws = static_cast<char*>(mobula_hip::workspace_if_possible(prep.bytes + kPieceBytes));
+  if (ws == nullptr) return failed();
   float* const pieces = reinterpret_cast<float*>(place_weight_b16(&wgrad, &prep, place_gather_b16(&data, &prep, ws)));
   prep.launch(stream);
   launch_igemm_b16(data, pieces, stream);

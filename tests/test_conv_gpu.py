@@ -528,3 +528,49 @@ def test_bias_gradient_can_be_recorded_first():
         torch.cuda.synchronize()
         _close(db, dy.double().sum((0, 2, 3)), 'db', 1e-5)
         dyd.add_(0)   # (ordinary work between the replays)
+
+
+@pytest.mark.parametrize('mode', ['bf16', 'bf16x3'])
+def test_both_gradients_in_a_workspace_that_holds_the_operands_of_one(mode):
+    """The gradients of one call share their operands where the workspace can hold both; where it cannot
+    grow they are made one after the other, with the same bits."""
+    native.set_option('conv_compute', MODES[mode][0])
+    N, C, H, W, D = 24 if mode == 'bf16' else 12, 32, 56, 56, 512
+    g = torch.Generator(device='cuda').manual_seed(81)
+    x, w = torch.randn(N, C, H, W, generator=g, device='cuda'), torch.randn(D, C, 3, 3, generator=g, device='cuda')
+    dy = torch.randn(N, D, H, W, generator=g, device='cuda')
+    geo = _ci(N, C, H, W, D, 3, 3, 1, 1, 1, 1, 1, 1)
+    lib, stream = native.library(), torch.cuda.Stream()
+
+    def both(dx, dw, on=None):
+        native.begin_call(on, [])
+        lib.mobula_hip_conv2d_backward(ctypes.c_int(0), _ptr(dy), _ptr(x), _ptr(w), *geo, _ptr(dx), _ptr(dw))
+        native.end_call('conv2d_backward')
+    try:
+        want, single, got = ([torch.full_like(t, float('nan')) for t in (x, w)] for _ in range(3))
+        torch.cuda.synchronize()
+        both(*want)
+        roomy = native.workspace_bytes()
+        native.release_workspace()
+        _call('conv2d_backward_data_ecf81c91', ctypes.c_int(x.numel()), _ptr(dy), _ptr(w), ctypes.c_int(0), *geo,
+              _ptr(single[0]))
+        _call('conv2d_backward_weight_ecf81c91', ctypes.c_int(w.numel()), _ptr(dy), _ptr(x), ctypes.c_int(0), *geo,
+              _ptr(single[1]))
+        held = native.workspace_bytes()
+        assert held < roomy / 1.25   # (a workspace is made a quarter larger than asked for)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            both(*got, on=torch.cuda.current_stream().cuda_stream)
+        for _ in range(3):
+            for t in got:
+                t.fill_(float('nan'))
+            graph.replay()
+            torch.cuda.synchronize()
+            for a, b, c in zip(got, want, single):
+                assert torch.equal(a, b) and torch.equal(a, c)
+            both(*single)   # an ordinary call between the replays: the recorded graph holds the workspace where it is
+            assert native.workspace_bytes() == held
+        del graph
+    finally:
+        native.unpin_workspace()
+        native.set_option('conv_compute', 0)
