@@ -475,7 +475,7 @@ void launch_product(PatchProduct p, const PatchCut& cut, char* at, float* pieces
   const size_t bytes = product_bytes<T>(p, cut, &mpad, &sub);
   conv::PatchOps& o = p.ops;
   conv::ArrangePatchArgs& a = p.arrange;
-  o.npx = cut.npx; o.cols = o.N * cut.npx; o.mpad = mpad; o.cc = cut.cc; o.sub = sub;
+  o.npx = cut.npx; o.cols = o.N * cut.npx; o.mpad = mpad; o.cc = cut.cc; o.sub = sub; o.taps = a.KHp * a.KWp;
   o.chunks = (o.C + cut.cc - 1) / cut.cc; o.plane = cut.rows * o.pitch;
   float* const wp = reinterpret_cast<float*>(at);
   int* const koff = reinterpret_cast<int*>(at + bytes - align_to_256(sizeof(int) * 16ull * sub));

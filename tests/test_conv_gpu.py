@@ -574,3 +574,49 @@ def test_both_gradients_in_a_workspace_that_holds_the_operands_of_one(mode):
     finally:
         native.unpin_workspace()
         native.set_option('conv_compute', 0)
+
+
+@pytest.mark.parametrize('shape', [
+    # K steps of the products from patches that end in padding: taps x channels that fill no whole step, chunks of
+    # channels that end past the last one, chunks of pixels that end past the plane
+    (2, 3, 20, 21, 64, (7, 7), (3, 3), (2, 2), (1, 1)),
+    (3, 1, 33, 64, 32, (5, 1), (2, 0), (1, 1), (1, 1)),
+    (2, 32, 24, 26, 33, (3, 3), (1, 1), (2, 2), (1, 1)),
+    (2, 50, 19, 23, 40, (3, 3), (1, 1), (1, 1), (1, 1)),
+    (5, 33, 11, 11, 17, (1, 1), (0, 0), (1, 1), (1, 1)),
+])
+def test_an_infinity_stays_an_infinity_in_fp32_products(shape):
+    """What pads a K step is zero times zero: one infinite element of an operand makes the results that it
+    belongs to infinite, of the right sign, and no other."""
+    N, C, H, W, D, kernel, pad, stride, dil = shape
+    g = torch.Generator().manual_seed(82)
+    x, w = torch.randn(N, C, H, W, generator=g), torch.randn(D, C, *kernel, generator=g)
+    geo = _ci(N, C, H, W, D, kernel[0], kernel[1], pad[0], pad[1], stride[0], stride[1], dil[0], dil[1])
+
+    def check(got, want, what):
+        got = got.cpu().double()
+        assert not got.isnan().any(), what
+        assert torch.equal(got == float('inf'), want == float('inf')) and torch.equal(got == -float('inf'), want == -float('inf')), what
+        finite = want.isfinite()
+        if finite.any():
+            _close(got[finite], want[finite], what, 1e-5)
+    for at in ((0, 0, 0, 0), (N - 1, C - 1, H - 1, W - 1), (N // 2, C // 2, H // 2, W // 2), (0, C - 1, 1, 2)):
+        xi = x.clone()
+        xi[at] = float('inf')
+        xr, wr = x.double().requires_grad_(True), w.double().requires_grad_(True)
+        conv = lambda a, b: F.conv2d(a, b, stride=stride, padding=pad, dilation=dil)   # noqa: E731
+        y_ref = conv(xi.double(), wr)
+        dy = torch.randn(y_ref.shape, generator=g)
+        (dw_ref,) = torch.autograd.grad(y_ref, wr, dy.double())
+        y, dw, dx = torch.empty(dy.shape, device='cuda'), torch.empty(w.shape, device='cuda'), torch.empty(x.shape, device='cuda')
+        xd, wd, dyd = xi.cuda(), w.cuda(), dy.cuda()
+        _call('conv2d_forward_c6a7aa85', ctypes.c_int(y.numel()), _ptr(xd), _ptr(wd), _ptr(wd), ctypes.c_int(0), *geo, _ptr(y))
+        check(y, y_ref.detach(), 'y')
+        _call('conv2d_backward_weight_ecf81c91', ctypes.c_int(dw.numel()), _ptr(dyd), _ptr(xd), ctypes.c_int(0), *geo, _ptr(dw))
+        check(dw, dw_ref, 'dw')
+        dyi = dy.clone()
+        dyi[at[0], at[1] % D, min(at[2], dy.shape[2] - 1), min(at[3], dy.shape[3] - 1)] = float('inf')
+        (dx_ref,) = torch.autograd.grad(conv(xr, w.double()), xr, dyi.double())
+        dyd = dyi.cuda()
+        _call('conv2d_backward_data_ecf81c91', ctypes.c_int(dx.numel()), _ptr(dyd), _ptr(wd), ctypes.c_int(0), *geo, _ptr(dx))
+        check(dx, dx_ref, 'dx')
