@@ -328,14 +328,22 @@ int mobula_hip_device_count(void);
 
 /* The calls keep one grow-only scratch buffer per calling thread and device for
  * their intermediate tables (no counterpart in the reference, whose kernels use
- * none).  workspace_bytes: its current size for the calling thread on the
- * current device.  release_workspace: gives it back to the device (waits for the
- * work that still uses it) and returns the bytes freed; the next call allocates
- * afresh.  A HIP graph recorded from calls of this thread refers to the buffer
- * by address: a call on a capturing stream pins it, and a pinned buffer is
- * neither released nor replaced by a larger one (such a call fails with an
- * error instead) until unpin_workspace() says the graphs are gone.  Replays are
- * not ordered against the thread's calls on other streams (the caller orders those). */
+ * none).  Calls with host buffers (device id -1) also keep the device copies of
+ * these, at most 1 GiB per calling thread and device, and, shared by all
+ * threads, 24 MB of pinned host memory through which larger arrays are copied
+ * with the help of up to seven threads (no more than half of the process's
+ * processors; they end after two seconds without a copy).
+ * workspace_bytes: device memory that the calling thread holds in this way on
+ * the current device, scratch buffer and copies.  release_workspace: gives it
+ * back to the device (waits for the work that still uses it), and the pinned
+ * memory unless a copy is using it, and returns the device bytes freed; the next
+ * call allocates afresh.  A thread that ends gives back its own.  A HIP graph
+ * recorded from calls of this thread refers to the scratch buffer by address: a
+ * call on a capturing stream pins it, and a pinned buffer is neither released nor
+ * replaced by a larger one (such a call runs without it where it can, and fails
+ * with an error where it cannot) until unpin_workspace() says the graphs are gone.
+ * Replays are not ordered against the thread's calls on other streams (the
+ * caller orders those). */
 long long mobula_hip_workspace_bytes(void);
 long long mobula_hip_release_workspace(void);
 void mobula_hip_unpin_workspace(void);

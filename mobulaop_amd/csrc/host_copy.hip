@@ -389,12 +389,19 @@ bool HostStaging::flush(hipStream_t stream) {
   return !failed();
 }
 
-void release_staging() {
+long long staging_bytes() {
+  const Arena* const a = arena_of_current_device();
+  return a == nullptr ? 0 : static_cast<long long>(a->bytes);
+}
+
+long long release_staging() {
   Copier::get().release();
   Arena* const a = arena_of_current_device();
-  if (a == nullptr || a->base == nullptr || a->used != 0) return;
+  if (a == nullptr || a->base == nullptr || a->used != 0) return 0;
+  const long long bytes = static_cast<long long>(a->bytes);
   (void)hipFree(a->base);
   *a = Arena();
+  return bytes;
 }
 
 }  // namespace mobula_hip

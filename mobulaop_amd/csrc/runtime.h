@@ -97,7 +97,8 @@ class HostStaging {
   size_t mark_ = 0;
   bool unfinished_ = false;
 };
-void release_staging();   // frees the calling thread's block on the current device and the pinned ring
+long long staging_bytes();     // size of the calling thread's block on the current device
+long long release_staging();   // frees that block (the bytes are returned) and the pinned ring
 
 // Every entry point starts a call with begin_call() -- the error text of the
 // thread's previous call is dropped, so an error is reported for the call that

@@ -382,11 +382,11 @@ double mobula_hip_last_kernel_ms(const char** name) {
   return ms;
 }
 
-long long mobula_hip_workspace_bytes(void) { return mobula_hip::workspace_bytes(); }
+long long mobula_hip_workspace_bytes(void) { return mobula_hip::workspace_bytes() + mobula_hip::staging_bytes(); }
 long long mobula_hip_release_workspace(void) {
   mobula_hip::begin_call();
-  mobula_hip::release_staging();
-  return mobula_hip::release_workspace();
+  const long long mirrors = mobula_hip::release_staging();
+  return mirrors + mobula_hip::release_workspace();
 }
 // The calling thread's workspace on the current device is no longer used by any recorded graph.
 void mobula_hip_unpin_workspace(void) { mobula_hip::unpin_workspace(); }

@@ -136,15 +136,16 @@ def device_can_read(address):
 
 
 def workspace_bytes():
-    """Size of the calling thread's scratch buffer on the current device."""
+    """Device memory the library holds for the calling thread on the current device between
+    calls: its scratch buffer and, after calls with host arrays, their device copies."""
     fn = library().mobula_hip_workspace_bytes
     fn.restype = ctypes.c_longlong
     return int(fn())
 
 
 def release_workspace():
-    """Give the calling thread's scratch buffer back to the device; returns the
-    bytes freed.  The next call allocates what it needs.  Refused (RuntimeError)
+    """Give the calling thread's scratch buffer and copies of host arrays back to the device, and
+    the pinned host memory these are copied through; returns the device bytes freed.  The next call allocates what it needs.  Refused (RuntimeError)
     while a recorded HIP graph uses the buffer: see unpin_workspace()."""
     lib = library()
     fn = lib.mobula_hip_release_workspace

@@ -268,6 +268,20 @@ def test_direct_calls_leave_transformed_calls_to_the_operator_class(mobula, cont
     assert seen == [NotImplemented]
 
 
+def test_memory_kept_after_host_arrays_is_counted_and_given_back(mobula):
+    """The device copies of host arrays outlive a call: they are part of what the library says it holds."""
+    native.release_workspace()
+    assert native.workspace_bytes() == 0
+    x = np.ones((2, 64, 90, 91), dtype=np.float32)
+    y = np.empty((3, 64, 2, 2), dtype=np.float32)
+    rois = np.zeros((3, 5), dtype=np.float32)
+    mobula.func.roi_align_forward(y.size, x, 1.0, 64, 90, 91, 2, 2, 2, rois, y)
+    held = native.workspace_bytes()
+    assert held >= x.nbytes + y.nbytes + rois.nbytes
+    assert native.release_workspace() == held
+    assert native.workspace_bytes() == 0 and native.release_workspace() == 0
+
+
 @pytest.mark.parametrize('kind', ['forward_pre', 'forward', 'full_backward_pre', 'full_backward'])
 def test_hooks_on_all_modules_see_direct_calls(mobula, kind):
     """The operator class's call is a module's: with such a hook registered it keeps the call."""
