@@ -56,7 +56,10 @@ inline int blocked_rows_per_pass(int C, long long H, long long W, int PH, int PW
   return min(PH, stage / (B::CB * PW));
 }
 
-struct OrderArgs { const float* rois; int* order; int R; float scale; int H, W; long long num_images; int PH, PW, S; };
+struct OrderArgs {
+  const float* rois; int* order; int R; float scale; int H, W; long long num_images; int PH, PW, S;
+  const int* direct;   // not null: nothing is copied where *direct is not 0 (choose_direct_kernel)
+};
 
 template <int NT, int MAXC>
 __device__ __forceinline__ void roi_order_body(int* hist, int* wave_sum, int* carry, const float* __restrict__ rois,
@@ -149,6 +152,7 @@ transpose_to_blocked_kernel(const T* __restrict__ in, T* __restrict__ out, int C
                             OrderArgs oa) {
   constexpr int CB = BlockOf<T>::CB;
   __shared__ T tile[CB][65];
+  if (oa.direct != nullptr && *oa.direct != 0) return;
   int bx = blockIdx.x;
   if (oa.order != nullptr) {
     if (bx == 0) {

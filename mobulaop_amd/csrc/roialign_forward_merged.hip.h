@@ -78,7 +78,7 @@ __global__ void __launch_bounds__(FwdMerged::NW * 64, 4)
 forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
                       const int* __restrict__ order, T* __restrict__ y, float scale, int C, int H,
                       int W, int PH, int PW, int S, long long num_images, int cblk,
-                      int rows_per_pass, int rois_listed, int parts) {
+                      int rows_per_pass, int rois_listed, int parts, const int* __restrict__ direct) {
   using K = FwdBlocked;
   using M = FwdMerged;
   constexpr int CPL = BlockOf<T>::CPL, CB = BlockOf<T>::CB, STAGE = BlockOf<T>::STAGE_MERGED;
@@ -88,6 +88,7 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
   __shared__ int rown_s[M::NW][M::RPH];
   __shared__ int coln_s[M::NW][K::PWB];
   __shared__ __attribute__((aligned(16))) T stage_s[M::NW][STAGE];
+  if (direct != nullptr && *direct != 0) return;   // (forward_naive_kernel does the call: choose_direct_kernel)
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

@@ -8,11 +8,34 @@
 
 namespace roialign {
 
+// *direct = 1 if the boxes' sample points on an adaptive grid (points per bin, summed over the boxes) are
+// at most `most`, else 0.  One workgroup: the boxes are on the device, and so is the choice between two ways
+// to do a call.  (A box without extent has a point; one that is not a number counts as whatever the
+// conversion makes of it: either way takes it.)
+__global__ void __launch_bounds__(1024)
+choose_direct_kernel(const float* __restrict__ rois, int R, float scale, int PH, int PW, float most,
+                     int* __restrict__ direct) {
+  __shared__ float sums[16];
+  float points = 0.0f;
+  for (int r = threadIdx.x; r < R; r += 1024) {
+    const RoiGeom g = roi_geometry(rois + static_cast<long long>(r) * 5, scale, PH, PW, 0);
+    points += static_cast<float>(g.grid_h) * static_cast<float>(g.grid_w);
+  }
+  for (int off = 32; off > 0; off >>= 1) points += __shfl_xor(points, off);
+  if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = points;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int w = 1; w < 16; ++w) points += sums[w];
+  *direct = points <= most ? 1 : 0;
+}
+
+// only != null: nothing is done where *only is 0 (choose_direct_kernel).
 template <typename T>
 __global__ void __launch_bounds__(256)
 forward_naive_kernel(long long n_out, const T* __restrict__ x, float scale, int C, int H, int W,
                      int PH, int PW, int S, const float* __restrict__ rois, T* __restrict__ y,
-                     long long num_images) {
+                     long long num_images, const int* __restrict__ only) {
+  if (only != nullptr && *only == 0) return;
   const long long stride = static_cast<long long>(gridDim.x) * blockDim.x;
   const int bins = PH * PW;
   for (long long idx = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; idx < n_out;

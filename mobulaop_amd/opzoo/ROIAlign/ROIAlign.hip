@@ -204,7 +204,7 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
       {
         mobula_hip::KernelTimer timer("forward_merged_kernel", stream);
         roialign::forward_merged_kernel<T, true><<<static_cast<unsigned>(grid), nw * 64, 0, stream>>>(
-            x, rois, order, y, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, p.N, cblk, p.PH, p.R, parts);
+            x, rois, order, y, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, p.N, cblk, p.PH, p.R, parts, nullptr);
       }
       // the boxes that kernel leaves out (sampling grids of more than 64 points per axis)
       if (p.S <= 0 || p.S > roialign::kSearchedGrid)
@@ -228,8 +228,19 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
   // 32 of 256 channels on 4 x 200 x 336: 88 -> 11 us, 512 of them 112 -> 107.  (A map too large for fixed scratch
   // stays an error.)
   const double copied_us = 3.0 + 2.0 * xt_bytes / 6.0e6 + 2.7e-6 * p.n_out;
-  const bool direct = (!fixed || xt_bytes + sizeof(int) * p.R <= p.fixed_scratch_bytes) && p.S >= 1 && p.S <= 4 && mobula_hip::option("roialign_impl", kAuto) == kAuto &&
-                      13.5e-6 * p.n_out * p.S * p.S / 4 < copied_us;
+  const bool automatic = mobula_hip::option("roialign_impl", kAuto) == kAuto;
+  const bool direct = (!fixed || xt_bytes + sizeof(int) * p.R <= p.fixed_scratch_bytes) && p.S >= 1 &&
+                      (p.S <= 4 || padded) && automatic && 13.5e-6 * p.n_out * p.S * p.S / 4 < copied_us;
+  // The same question for a padded copy and an adaptive grid: how many points there are only the device knows.
+  // A point of a million outputs takes one thread per output 3.6 us.  Where the copy takes much longer than a
+  // point per bin would, the device is asked, which costs a call 5 us (and what it then leaves out 10), and
+  // the copy is made if the boxes have more points than it takes.  Measured without and with the question, 81
+  // fp32 channels, 7 x 7 bins of 1, 4, 16 and 64 points: 4 x 200 x 336, 150 boxes 43 / 45 / 50 / 66 and 19 / 23 / 55 /
+  // 71 us (one thread per output alone 9 / 12 / 41 / 187); 8 x 200 x 336, 400 boxes 74 / 76 / 92 / 144 and 31 / 43 / 98 /
+  // 149 (14 / 25 / 95 / 449).  Not asked: 4 x 200 x 336, 1000 boxes 56 / 59 / 83 / 159 (29 / 57 / 222 / 1088); 1 x 200 x
+  // 336, 300 boxes 24 / 29 / 37 / 53 (10 / 19 / 71 / 335).
+  const double copy_us = 3.0 + 2.0 * xt_bytes / 6.0e6, point_us = 3.6e-6;
+  const bool ask = padded && p.S <= 0 && !fixed && automatic && copy_us > 20.0 + 2.0 * point_us * p.n_out;
   if (use_tiled() && fits && !padded_beyond && !direct) {
     // channel-blocked copy of the map, spatial ROI order, then the gather
     if (fixed && xt_bytes + sizeof(int) * p.R > p.fixed_scratch_bytes) {
@@ -238,13 +249,18 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
                 xt_bytes + sizeof(int) * p.R, p.fixed_scratch_bytes);
       return;
     }
+    const size_t bytes = xt_bytes + sizeof(int) * (p.R + 1);
     ws = static_cast<char*>(fixed    ? p.fixed_scratch
-                            : padded ? mobula_hip::workspace_if_possible(xt_bytes + sizeof(int) * p.R)
-                                     : mobula_hip::workspace(xt_bytes + sizeof(int) * p.R));
+                            : padded ? mobula_hip::workspace_if_possible(bytes)
+                                     : mobula_hip::workspace(bytes));
     if (failed()) return;
   }
   if (ws != nullptr) {
     T* const xt = reinterpret_cast<T*>(ws);
+    int* const choice = ask ? reinterpret_cast<int*>(ws + xt_bytes) + p.R : nullptr;
+    if (ask)
+      roialign::choose_direct_kernel<<<1, 1024, 0, stream>>>(
+          rois, p.R, p.scale, p.PH, p.PW, static_cast<float>((copy_us - 8.0) / (point_us * p.C * p.PH * p.PW)), choice);
     // ROIs are visited in spatial order when the map is larger than the L2 caches
     // hold; a small map is read in the caller's order and the ordering kernel is left out
     int* const order = xt_bytes > kSortedAboveBytes ? reinterpret_cast<int*>(ws + xt_bytes) : nullptr;
@@ -257,7 +273,7 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
     if (order != nullptr && !order_in_copy)
       roialign::roi_order_kernel<<<1, 1024, 0, side.get()>>>(rois, p.R, p.scale, p.H, p.W, p.N, order);
     const roialign::OrderArgs oa{rois, order_in_copy ? order : nullptr, static_cast<int>(p.R), p.scale, p.H, p.W, p.N,
-                                 p.PH, p.PW, p.S};
+                                 p.PH, p.PW, p.S, choice};
     // Few boxes on a large map: only what they can touch is copied (4 x 256 x 200 x 336 in fp32, adaptive
     // grid: 97 -> 34 us with two boxes, 99 -> 53 with 32, 119 -> 107 with 128; beyond some 32 boxes an
     // image, and on maps the caches hold, looking at the boxes costs more than it saves).
@@ -281,18 +297,21 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
       {
         mobula_hip::KernelTimer timer("forward_merged_kernel", stream, !fixed);
         roialign::forward_merged_kernel<T, false><<<static_cast<unsigned>(grid), nw * 64, 0, stream>>>(
-            xt, rois, order, y, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, p.N, cblk, rpp, p.R, parts);
+            xt, rois, order, y, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, p.N, cblk, rpp, p.R, parts, choice);
       }
       // the boxes that kernel leaves out (sampling grids of more than 64 points per axis), from the map itself
       if (p.S <= 0 || p.S > roialign::kSearchedGrid)
         roialign::forward_large_grid_kernel<T, false><<<static_cast<unsigned>(p.R), 64, 0, stream>>>(
           x, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, rois, y, p.N);
     }
+    if (choice != nullptr)
+      roialign::forward_naive_kernel<T><<<std::min(2048, grid_for(p.n_out, 256)), 256, 0, stream>>>(
+          p.n_out, x, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, rois, y, p.N, choice);
     MOBULA_HIP_TRY(hipGetLastError());
     return;
   }
   roialign::forward_naive_kernel<T><<<grid_for(p.n_out, 256), 256, 0, stream>>>(
-      p.n_out, x, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, rois, y, p.N);
+      p.n_out, x, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, rois, y, p.N, nullptr);
   MOBULA_HIP_TRY(hipGetLastError());
 }
 

@@ -1154,3 +1154,27 @@ def test_odd_channel_counts_are_taken_without_a_workspace(dtype, C, S):
                               oracle.forward(x.astype(np.float32), rois, (3, 4), 0.25, 2 if S == 0 else 1), tol, 'between')
     graphs.clear()
     native.unpin_workspace()
+
+
+@pytest.mark.parametrize('side,ways', [(5, 'naive'), (60, 'tiled'), (None, 'tiled')])
+def test_the_device_chooses_between_the_padded_copy_and_none(side, ways):
+    """An odd channel count on a large map with an adaptive grid: a kernel adds the boxes' sample points up, and
+    the call takes the copy and the gather, or one thread per output, with the bits of whichever it is.  The
+    workspace holds NaN beforehand; None: boxes that are no numbers, infinite, or of no image among them."""
+    rng = np.random.default_rng(12)
+    N, C, H, W, R, pooled = 4, 33, 240, 240, 140, (3, 4)
+    x = rng.standard_normal((N, C, H, W)).astype(np.float32)
+    c, half = rng.uniform(0, W, (R, 2)), (side or 5) / 2
+    rois = np.concatenate([rng.integers(0, N, (R, 1)), c - half, c + half], 1).astype(np.float32)
+    if side is None:
+        rois[:6] = [[0, 1, 2, np.nan, 9], [1, -np.inf, 0, np.inf, 9], [7, 0, 0, 9, 9], [-1, 0, 0, 9, 9], [2, 9, 9, 3, 3],
+                    [3, -1e9, -1e9, 1e9, 1e9]]
+    xd, rd, got = abi.to_dev(x), abi.to_dev(rois), {}
+    for impl in ('naive', 'tiled', 'auto'):
+        abi.set_impl(impl)
+        abi.poison_workspace(160 << 20)
+        got[impl] = abi.forward(xd, rd, pooled, 1.0, 0)
+    assert torch.equal(got['auto'].nan_to_num(123.0), got[ways].nan_to_num(123.0))
+    assert not torch.equal(got['naive'].nan_to_num(123.0), got['tiled'].nan_to_num(123.0))
+    first = 0 if side else 6
+    assert_parity(got['auto'][first:].cpu().numpy(), oracle.forward(x, rois[first:], pooled, 1.0, 0), FWD_TOL, 'y')
