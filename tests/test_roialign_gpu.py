@@ -1178,3 +1178,26 @@ def test_the_device_chooses_between_the_padded_copy_and_none(side, ways):
     assert not torch.equal(got['naive'].nan_to_num(123.0), got['tiled'].nan_to_num(123.0))
     first = 0 if side else 6
     assert_parity(got['auto'][first:].cpu().numpy(), oracle.forward(x, rois[first:], pooled, 1.0, 0), FWD_TOL, 'y')
+
+
+@pytest.mark.parametrize('S', [2, 0])
+@pytest.mark.parametrize('W', [116, 117])
+@pytest.mark.parametrize('dtype', [np.float32, np.float16])
+def test_partly_copied_maps_of_several_channel_blocks(W, dtype, S):
+    """Both gathers over a copy that holds only what the boxes touch: five channel blocks, of which a workgroup of
+    the copy takes two or three, one after the other; with the fixed grid too many outputs for one thread each.
+    The workspace holds NaN beforehand."""
+    abi.set_impl('auto')
+    rng = np.random.default_rng(W)
+    N, C, H, scale, pooled, R = 3, 160 if dtype == np.float32 else 320, 125, 0.5, (14, 14), 60
+    x = rng.standard_normal((N, C, H, W)).astype(dtype)
+    # (no box in the last image nor in the lower half of the others, but for two at the borders)
+    c = np.stack([rng.uniform(20, 2 * W - 20, R), rng.uniform(0, H - 70, R)], 1)
+    wh = rng.uniform(5, 60, (R, 2))
+    rois = np.concatenate([rng.integers(0, N - 1, (R, 1)), c - wh / 2, c + wh / 2], 1).astype(np.float32)
+    rois[:2] = [[0, 2 * W - 30, 2 * H - 20, 2 * W + 9, 2 * H + 9], [1, -9, 2 * H - 12.5, 13, 2 * H]]
+    assert x.nbytes > 24 << 20 and R <= 32 * N   # (else everything is copied)
+    abi.poison_workspace(48 << 20)
+    y = abi.forward(abi.to_dev(x), abi.to_dev(rois), pooled, scale, S).cpu().numpy()
+    want = oracle.forward(x.astype(np.float32), rois, pooled, scale, S).astype(dtype)
+    assert_parity(y.astype(np.float32), want.astype(np.float32), FWD_TOL if dtype == np.float32 else FP16_TOL, 'y')
