@@ -27,12 +27,12 @@
 // one chunk ahead.  A lane's four k of a matrix instruction group are neighbours in the left
 // operand (k = 8 g + 4 half + e for instruction e), so that it reads them as sixteen bytes.
 //
-// Bound: the matrix cores, 72 % busy.  Per K step and wavefront 32 instructions of 64 clocks, against
-// four 16-byte and sixteen 4-byte LDS reads and about five loads; two workgroups to a CU cover each
-// other's barriers.  An image of three channels (8 x 3 x 224 x 224, 7 x 7 at stride 2, 64 filters):
-// forward 259 -> 38 us (44 with a test per element in the write-out), weight gradient 208 -> 46 us with its
-// reduction, where the gathered tiles
-// multiply 13 padding channels of 16 and 64 padding rows of 128.
+// Bound: per K step and wavefront 32 matrix instructions of 64 clocks, against four 16-byte and sixteen 4-byte
+// LDS reads and about five loads; two workgroups to a CU cover each other's barriers.  An image of three
+// channels (8 x 3 x 224 x 224, 7 x 7 at stride 2, 64 filters): forward 259 -> 39 us (44 with a test per element
+// in the write-out), 40 % of its clocks in matrix instructions -- 392 tiles on 512 slots, of ten steps each, that
+// all load their patch, then all multiply, then all write --, weight gradient 208 -> 42 and 5 for adding the slices
+// up, 57 %; the gathered tiles multiply 13 padding channels of 16 and 64 padding rows of 128.
 #pragma once
 #include <type_traits>
 
@@ -55,7 +55,7 @@ typedef PatchTile<1, 1, 4> PatchTile32;    // 32 x 256
 struct PatchOps {
   const float* __restrict__ src;   // [N][C][Hs][Ws]
   const float* __restrict__ wp;    // [K step][mpad][16] (arrange_patch_weights_kernel)
-  const int* __restrict__ koff;    // [sub * 16] byte offsets within a patch buffer
+  const int* __restrict__ koff;    // [sub * 16] byte offsets within a patch buffer, -1 for padding
   const float* __restrict__ bias; float* __restrict__ out;
   int N, C, Hs, Ws, M, Ho, Wo, sh, sw, ph, pw;
   int reach;             // source rows an output row needs: (KH - 1) * step + 1
@@ -64,7 +64,7 @@ struct PatchOps {
   int plane, pitch;      // positions of a channel in the patch, of a patch row
   int accumulate;
   int out_h, out_w, os_h, os_w, oo_h, oo_w;   // where pixel (oh, ow) lies in an output plane of out_h x out_w
-  int taps;
+  int zeros;   // positions of LDS that hold zeros for the k that pad a chunk: as far as a column's base reaches
 };
 
 // wp[t][m][kk] for K step t = chunk * sub + s: k = 16 s + kk within the chunk is (tap, channel), channel
@@ -96,7 +96,7 @@ arrange_patch_weights_kernel(ArrangePatchArgs a) {
     if (i < a.sub * 16) {
       const int k0 = static_cast<int>(i), tap0 = k0 / a.cc, jh0 = tap0 / a.KWp;
       a.koff[i] = tap0 < taps ? ((k0 - tap0 * a.cc) * a.plane + jh0 * a.step_h * a.pitch +
-                                 (tap0 - jh0 * a.KWp) * a.step_w) * 4 : 0;
+                                 (tap0 - jh0 * a.KWp) * a.step_w) * 4 : -1;
     }
   }
 }
@@ -122,13 +122,15 @@ __device__ __forceinline__ void wait_for_memory() { __builtin_amdgcn_s_waitcnt(0
 //   second half:  products of group 1 | fragment reads of group 0 of step t + 1 | requests for the left
 //                 operand of step t + 2 and for a share of the next chunk's patch
 // (Requests and reads in front of the products, a full wait per step: 1079 us instead of 1046 for the
-// forward product of 32 x 256 x 56 x 56, 3 x 3; 246 us of matrix instructions take 342.)
+// forward product of 32 x 256 x 56 x 56, 3 x 3, which igemm_kernel does in 903.)
 // f: where things are.  f.request(stage) asks for the next step's left operand, f.request_patch() for a
 // share of the next patch; f.patch(), f.offsets(), f.valid() are those of the step to read, f.next() goes on.
-// Of a step's sixteen k the first f.valid() exist (all of them for f.full_steps() from here).  The others meet
-// zeros in the left operand, and what the patch holds for them (the values of some other k) is made zero
-// as well: an infinity there would be NaN.
-template <typename T, typename F>
+// The k that pad a step meet zeros in the left operand, and have to meet zeros here as well: some other k's value,
+// were it infinite, would make them NaN.  Either their offsets lead to zeros (ZEROS: as many as a column's base
+// reaches; twelve forward and data products of 3 to 200 channels take 0-1 % longer for it, 1-9 % with cleared
+// registers), or of a step's sixteen k the first f.valid() exist (all of them for f.full_steps() from here) and
+// the others are cleared (weight gradient, whose columns reach all over the patch: no slower).
+template <typename T, bool ZEROS, typename F>
 __device__ __forceinline__ void patch_pipeline(F& f, int steps, const int (&base)[2], int wm, float16v (&acc)[T::NI][2]) {
   typedef int i32x4 __attribute__((ext_vector_type(4)));
   typedef PatchFragments<T> Fragments;
@@ -174,9 +176,10 @@ __device__ __forceinline__ void patch_pipeline(F& f, int steps, const int (&base
   workgroup_barrier();
   read(f0, 0, 0);
   int stage = 0, t = 0;
-  auto step = [&](auto padded) {
-    const int next = stage == 2 ? 0 : stage + 1, valid = padded ? f.valid() : 16;
-    if (padded) clear_padding(f0, 0, valid);
+  auto step = [&](auto& f, auto padded) {
+    const int next = stage == 2 ? 0 : stage + 1;
+    int valid = 16;
+    if constexpr (decltype(padded)::value) { valid = f.valid(); clear_padding(f0, 0, valid); }
     multiply(f0, 0);
     read(f1, stage, 1);
     __builtin_amdgcn_sched_barrier(0);
@@ -185,7 +188,7 @@ __device__ __forceinline__ void patch_pipeline(F& f, int steps, const int (&base
     multiply(f0, 3);
     wait_for_memory();
     workgroup_barrier();
-    if (padded) clear_padding(f1, 1, valid);
+    if constexpr (decltype(padded)::value) clear_padding(f1, 1, valid);
     multiply(f1, 0);
     f.next();
     if (t + 1 < steps) read(f0, next, 0);
@@ -199,11 +202,14 @@ __device__ __forceinline__ void patch_pipeline(F& f, int steps, const int (&base
     multiply(f1, 3);
     stage = next;
   };
-  // (steps without padding in a loop of their own: with the question in every step the forward and weight
-  // gradient of an image of three channels, 7 x 7 at stride 2, took 1 % longer)
-  while (t < steps) {
-    for (const int end = min(steps, t + f.full_steps()); t < end; ++t) step(std::false_type());
-    if (t < steps) { step(std::true_type()); ++t; }
+  if constexpr (ZEROS) {
+    for (; t < steps; ++t) step(f, std::false_type());
+  } else {
+    // (steps without padding in a loop of their own: no question in each of them)
+    while (t < steps) {
+      for (const int end = min(steps, t + f.full_steps()); t < end; ++t) step(f, std::false_type());
+      if (t < steps) { step(f, std::true_type()); ++t; }
+    }
   }
 }
 
@@ -220,11 +226,11 @@ struct PatchPieces {
   __device__ __forceinline__ void advance() { piece += 4; settle(); }
 };
 
-// Bytes of LDS: three stages of the left operand, one or two patches, the table of patch positions
+// Bytes of LDS: three stages of the left operand, one or two patches, zeros, the table of patch positions
 // (whole pieces of 64) and of koff.
 template <typename T>
-__host__ __device__ inline size_t patch_lds_bytes(int buffers, long long patch_floats, int positions, int ko_entries) {
-  return sizeof(float) * (3 * T::BM * T::BK + buffers * ((patch_floats + 3) & ~3ll) + ((positions + 63) & ~63) + ko_entries);
+__host__ __device__ inline size_t patch_lds_bytes(int buffers, long long patch_floats, int zeros, int positions, int ko_entries) {
+  return sizeof(float) * (3 * T::BM * T::BK + buffers * ((patch_floats + 3) & ~3ll) + zeros + ((positions + 63) & ~63) + ko_entries);
 }
 
 // The tile at (m0, n0) over the K steps t_begin .. t_end - 1; results through ops, or (piece !=
@@ -238,8 +244,9 @@ __device__ __forceinline__ void patch_tile(const PatchOps& ops, int m0, int n0, 
   const int patch_floats = (ops.cc * ops.plane + 3) & ~3, buffers = ops.chunks > 1 ? 2 : 1;
   float* const As = patch_lds;
   float* const Bs = As + 3 * T::BM * T::BK;
-  int* const pos = reinterpret_cast<int*>(Bs + buffers * patch_floats);
-  int* const ko = pos + ((ops.plane + 63) & ~63);
+  float* const zeros = Bs + buffers * patch_floats;
+  int* const pos = reinterpret_cast<int*>(zeros + ops.zeros);
+  int* const ko = pos + ((ops.plane + 63) & ~63);   // [buffer][sub * 16]
 
   // The patch: for the first image the source rows from its first output row of the tile to its
   // last, then all rows of each further image, one after the other.
@@ -259,7 +266,11 @@ __device__ __forceinline__ void patch_tile(const PatchOps& ops, int m0, int n0, 
                     static_cast<unsigned>(iw) < static_cast<unsigned>(ops.Ws);
     pos[p] = in ? ((img - first) * image + ih * ops.Ws + iw) * 4 : kDead;
   }
-  for (int k = tid; k < ops.sub * 16; k += T::NT) ko[k] = ops.koff[k];
+  for (int k = tid; k < buffers * ops.sub * 16; k += T::NT) {
+    const int buffer = k >= ops.sub * 16 ? 1 : 0, at = ops.koff[k - buffer * ops.sub * 16];
+    ko[k] = at >= 0 ? at : (buffers - buffer) * patch_floats * 4;   // (the zeros follow the last buffer)
+  }
+  for (int p = tid; p < ops.zeros; p += T::NT) zeros[p] = 0.0f;
 
   int base[2];
 #pragma unroll
@@ -272,14 +283,13 @@ __device__ __forceinline__ void patch_tile(const PatchOps& ops, int m0, int n0, 
 
   const size_t skip = static_cast<size_t>(first) * image;
   const size_t left = (static_cast<size_t>(ops.N) * image - skip) * sizeof(float);
-  const __amdgpu_buffer_rsrc_t src = buffer_of(ops.src + skip, static_cast<unsigned>(left < kRecordLimit ? left : kRecordLimit));
   const __amdgpu_buffer_rsrc_t wp =
       buffer_of(ops.wp, static_cast<unsigned>(ops.chunks * ops.sub) * static_cast<unsigned>(ops.mpad) * 64u);
   const int a_off = (m0 + (lane >> 2)) * 64 + ((lane & 3) ^ ((lane >> 4) & 3)) * 16;
   struct {
-    const PatchOps& ops; __amdgpu_buffer_rsrc_t src, wp;
+    const PatchOps& ops; const float* src; unsigned src_bytes; __amdgpu_buffer_rsrc_t wp;
     float *As, *Bs; const int* ko;
-    int wave, lane, a_off, plane_bytes, patch_floats, tail, portion;
+    int wave, lane, a_off, plane_bytes, patch_floats, portion;
     PatchPieces pieces;
     int t_request, chunk, last_chunk, s, buf;
     __device__ __forceinline__ void request(int stage) {
@@ -294,10 +304,12 @@ __device__ __forceinline__ void patch_tile(const PatchOps& ops, int m0, int n0, 
     }
     __device__ __forceinline__ void load_patch(int of_chunk, float* to, int count) {
       for (; count > 0 && pieces.channel < ops.cc; --count) {
-        const int c = of_chunk * ops.cc + pieces.channel;   // (channels past the last one are zeros)
+        // (channels past the last one are zeros: no byte of the source is theirs)
+        const int c = of_chunk * ops.cc + pieces.channel;
+        const __amdgpu_buffer_rsrc_t from = buffer_of(src, c < ops.C ? src_bytes : 0u);
         if (pieces.piece * 64 + lane < ops.plane)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(src, to + pieces.channel * ops.plane + pieces.piece * 64, 4,
-                                                   c < ops.C ? pieces.at : kDead, min(c, ops.C - 1) * plane_bytes, 0, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(from, to + pieces.channel * ops.plane + pieces.piece * 64, 4, pieces.at,
+                                                   c * plane_bytes, 0, 0);
         pieces.advance();
       }
     }
@@ -307,13 +319,11 @@ __device__ __forceinline__ void patch_tile(const PatchOps& ops, int m0, int n0, 
       else if (chunk < last_chunk) load_patch(chunk + 1, Bs + (buf ^ 1) * patch_floats, portion);
     }
     __device__ __forceinline__ const char* patch() const { return reinterpret_cast<const char*>(Bs + buf * patch_floats); }
-    __device__ __forceinline__ const int* offsets() const { return ko + 16 * s; }
-    __device__ __forceinline__ int valid() const { return s == ops.sub - 1 ? tail : 16; }
-    __device__ __forceinline__ int full_steps() const { return tail == 16 ? ops.chunks * ops.sub : ops.sub - 1 - s; }
+    __device__ __forceinline__ const int* offsets() const { return ko + 16 * (buf * ops.sub + s); }
     __device__ __forceinline__ void next() {
       if (++s == ops.sub) { s = 0; ++chunk; buf ^= 1; }
     }
-  } f{ops, src, wp, As, Bs, ko, wave, lane, a_off, ops.Hs * ops.Ws * 4, patch_floats, ops.cc * ops.taps - 16 * (ops.sub - 1), 0,
+  } f{ops, ops.src + skip, static_cast<unsigned>(left < kRecordLimit ? left : kRecordLimit), wp, As, Bs, ko, wave, lane, a_off, ops.Hs * ops.Ws * 4, patch_floats, 0,
       PatchPieces{0, 0, (ops.plane + 63) / 64, 0, pos}, t_begin, t_begin / ops.sub, (t_end - 1) / ops.sub, 0, 0};
   f.s = t_begin - f.chunk * ops.sub;
   const int count = (ops.cc * f.pieces.per_channel + 3) / 4;   // pieces of a wavefront, at most
@@ -323,7 +333,7 @@ __device__ __forceinline__ void patch_tile(const PatchOps& ops, int m0, int n0, 
   f.load_patch(f.chunk, Bs, count);
   f.pieces.restart();
   float16v acc[T::NI][2];
-  patch_pipeline<T>(f, t_end - t_begin, base, wm, acc);
+  patch_pipeline<T, true>(f, t_end - t_begin, base, wm, acc);
 
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -536,7 +546,7 @@ __device__ __forceinline__ void patch_weight_tile(const PatchWeightOps& ops, int
   f.load_patch(q_begin, Bs, count);
   f.pieces.restart();
   float16v acc[T::NI][2];
-  patch_pipeline<T>(f, (q_end - q_begin) * f.sub, base, wm, acc);
+  patch_pipeline<T, false>(f, (q_end - q_begin) * f.sub, base, wm, acc);
 
 #pragma unroll
   for (int j = 0; j < 2; ++j) {

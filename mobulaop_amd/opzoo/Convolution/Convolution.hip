@@ -415,7 +415,7 @@ struct PatchProduct {
 };
 
 // How a tile's patch is cut: rows of the patch, columns per image, channels per chunk.
-struct PatchCut { int rows, npx, cc; size_t lds; double cost; };
+struct PatchCut { int rows, npx, cc, zeros; size_t lds; double cost; };
 
 // Rows a tile of BN columns needs at most.  Columns are numbered through all images (a tile may
 // cross into the next one, which costs the patch another image's margin rows), or every image's
@@ -438,7 +438,10 @@ PatchCut cut_patch(const conv::PatchOps& o, int taps, bool crossing) {
   if (plane >= (1 << 16)) return cut;
   for (int j = 1; j <= std::min(o.C, 256); ++j) {
     const int cc = (o.C + j - 1) / j, chunks = (o.C + cc - 1) / cc, sub = (cc * taps + 15) / 16;
-    const size_t lds = conv::patch_lds_bytes<T>(chunks > 1 ? 2 : 1, plane * cc, static_cast<int>(plane), sub * 16);
+    // (where channels and taps of a chunk fill no whole steps: zeros as far as a column's base reaches)
+    const int buffers = chunks > 1 ? 2 : 1;
+    const int zeros = cc * taps % 16 == 0 ? 0 : ((cut.rows - o.reach) * o.pitch + (o.Wo - 1) * o.sw + 4) & ~3;
+    const size_t lds = conv::patch_lds_bytes<T>(buffers, plane * cc, zeros, static_cast<int>(plane), buffers * sub * 16);
     if (lds > kLdsOfCu || (chunks > 1 && sub < 2)) continue;   // (the next patch is loaded a step behind the chunk's first)
     // clocks of a K step: the matrix instructions of a wavefront (64 clocks each, 2048 with two rows of
     // fragments) and what they do not hide -- measured with two workgroups to a CU: 10 % and 250
@@ -446,7 +449,7 @@ PatchCut cut_patch(const conv::PatchOps& o, int taps, bool crossing) {
     const double loads = static_cast<double>(cc) * ((plane + 63) / 64) / sub;
     const double step = T::NI * 1126.0 + 250.0 + 30.0 * loads + (2 * lds > kLdsOfCu ? 700.0 : 0.0);
     const double cost = step * sub * chunks * ((static_cast<double>(o.N) * cut.npx + T::BN - 1) / T::BN);
-    if (cut.cost < 0 || cost < cut.cost) { cut.cost = cost; cut.cc = cc; cut.lds = lds; }
+    if (cut.cost < 0 || cost < cut.cost) { cut.cost = cost; cut.cc = cc; cut.zeros = zeros; cut.lds = lds; }
   }
   return cut;
 }
@@ -475,7 +478,7 @@ void launch_product(PatchProduct p, const PatchCut& cut, char* at, float* pieces
   const size_t bytes = product_bytes<T>(p, cut, &mpad, &sub);
   conv::PatchOps& o = p.ops;
   conv::ArrangePatchArgs& a = p.arrange;
-  o.npx = cut.npx; o.cols = o.N * cut.npx; o.mpad = mpad; o.cc = cut.cc; o.sub = sub; o.taps = a.KHp * a.KWp;
+  o.npx = cut.npx; o.cols = o.N * cut.npx; o.mpad = mpad; o.cc = cut.cc; o.sub = sub; o.zeros = cut.zeros;
   o.chunks = (o.C + cut.cc - 1) / cut.cc; o.plane = cut.rows * o.pitch;
   float* const wp = reinterpret_cast<float*>(at);
   int* const koff = reinterpret_cast<int*>(at + bytes - align_to_256(sizeof(int) * 16ull * sub));
@@ -514,8 +517,8 @@ bool with_tiles(const PatchProduct& p, const F& f) {
   return with_cut<conv::PatchTile32>(p, f);
 }
 
-// Clocks of a K step of igemm_kernel (whole tiles of 128 x 128; 905 us at 2.3 GHz for 6.1 tiles of 144
-// steps to a CU, and a last round; 880 since).
+// Clocks of a K step of igemm_kernel on a CU, whole tiles of 128 x 128 (905 us at 2.3 GHz for 6.1 tiles of
+// 144 steps to a CU, and a last round).
 constexpr double kGatherStep = 2500.0;
 
 // CU clocks of the product from patches; < 0: it does not fit.
@@ -658,7 +661,7 @@ WeightCut cut_weight(const conv::Geometry& g) {
     const int nr = std::min(g.OH, px % g.OW == 0 ? px / g.OW : g.OW % px == 0 ? 1 : (px - 2) / g.OW + 2);
     const long long plane = static_cast<long long>((nr - 1) * g.stride_h + reach) * pitch;
     if (plane >= (1 << 15)) break;
-    const size_t lds = conv::patch_lds_bytes<T>(2, plane * channels, static_cast<int>(plane), 2 * px);
+    const size_t lds = conv::patch_lds_bytes<T>(2, plane * channels, 0, static_cast<int>(plane), 2 * px);
     if (lds > kLdsOfCu) break;
     const double loads = static_cast<double>(channels) * ((plane + 63) / 64);
     // (as in cut_patch; the right operand's reads meet bank conflicts)
