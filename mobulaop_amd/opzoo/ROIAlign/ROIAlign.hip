@@ -361,7 +361,7 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
                 hipStream_t stream, TilePlan* plan, const T* fuse_dy = nullptr) {
   // List items: the ROIs, or for sampling grids of more than 2 x 2 points the
   // windows of merged weights their bins are cut into.  How many depends on the
-  // boxes, so their number has to come back from the device (one blocking copy:
+  // boxes, so their number has to come back from the device (the host waits for it:
   // not while the stream is being captured into a graph).
   const bool windows = roialign::lists_in_windows(p.S);
   long long items = p.R, window_entries = 0;

@@ -87,8 +87,8 @@ class ROIAlign:
             except RuntimeError:
                 # Sampling grids other than 1 or 2 points are merged into lists whose size
                 # depends on the boxes: an adaptive grid of more than 2^15 points per bin, or
-                # a stream that is being captured (the size comes back through a blocking
-                # copy), is refused there.  The NCHW entry point below takes every grid.
+                # a stream that is being captured (the host waits for the size), is refused
+                # there.  The NCHW entry point below takes every grid.
                 if self.sampling_ratio in (1, 2):
                     raise
                 taken = False
