@@ -57,8 +57,8 @@ __device__ __forceinline__ float buffer_load1(__amdgpu_buffer_rsrc_t r, int voff
 // and the 16 channels are 16 loads from one address with scalar plane offsets.
 // The left operand is a copy of the weights in that order, [Mpad][taps][Cpad],
 // zero where a row or channel is padding (arrange_weights_kernel), so that its
-// loads need no guards; the gathered operand re-reads the last real channel
-// for padding channels (times zero).
+// loads need no guards; padding channels of the gathered operand are loaded
+// through a descriptor of no bytes: zeros.
 
 // One K step of a gathered product.
 struct GatherStep {
@@ -107,7 +107,7 @@ struct ForwardOps {
   Geometry g; int M, Ncols, K;   // K = taps * Cpad
   static constexpr bool kGathered = true;
   typedef GatherStep Step;
-  struct BCtx { __amdgpu_buffer_rsrc_t src; int anchor; int ih0, iw0; bool ok; };
+  struct BCtx { const float* src; unsigned bytes; int anchor; int ih0, iw0; bool ok; };
   __device__ Step load_step(int s) const { return steps[s]; }
   __device__ Step next_step(const Step&, int s) const { return steps[s]; }
   __device__ void fetch_a(int m, const Step&, int s, int ak, float (&out)[8]) const {
@@ -124,7 +124,8 @@ struct ForwardOps {
     const int img = n / ohw, r = n - img * ohw, oh = r / g.OW, ow = r - oh * g.OW;
     const size_t skip = static_cast<size_t>(first) * image;
     const size_t left = (static_cast<size_t>(g.N) * image - skip) * sizeof(float);
-    c.src = buffer_of(x + skip, static_cast<unsigned>(left < kRecordLimit ? left : kRecordLimit));
+    c.src = x + skip;
+    c.bytes = static_cast<unsigned>(left < kRecordLimit ? left : kRecordLimit);
     c.ih0 = oh * g.stride_h - g.pad_h;
     c.iw0 = ow * g.stride_w - g.pad_w;
     c.anchor = ((img - first) * image + c.ih0 * g.W + c.iw0) * 4;
@@ -137,7 +138,7 @@ struct ForwardOps {
     return in ? c.anchor + e.delta : kDead;
   }
   __device__ float load_b(const BCtx& c, const Step& e, int at, int k) const {
-    return buffer_load1(c.src, at, min(e.c0 + k, g.C - 1) * (g.H * g.W * 4));
+    return buffer_load1(buffer_of(c.src, e.c0 + k < g.C ? c.bytes : 0u), at, (e.c0 + k) * (g.H * g.W * 4));
   }
   __device__ float* column(int n) const {
     const int ohw = g.OH * g.OW, img = n / ohw, r = n - img * ohw;
@@ -157,7 +158,7 @@ struct BackwardDataOps {
   Geometry g; int M, Ncols, K; int accumulate;
   static constexpr bool kGathered = true;
   typedef GatherStep Step;
-  struct BCtx { __amdgpu_buffer_rsrc_t src; int anchor; int ihp, iwp; bool ok; };
+  struct BCtx { const float* src; unsigned bytes; int anchor; int ihp, iwp; bool ok; };
   __device__ Step load_step(int s) const { return steps[s]; }
   __device__ Step next_step(const Step&, int s) const { return steps[s]; }
   __device__ void fetch_a(int m, const Step&, int s, int ak, float (&out)[8]) const {
@@ -174,7 +175,8 @@ struct BackwardDataOps {
     const int img = n / hw, r = n - img * hw, ih = r / g.W, iw = r - ih * g.W;
     const size_t skip = static_cast<size_t>(first) * image;
     const size_t left = (static_cast<size_t>(g.N) * image - skip) * sizeof(float);
-    c.src = buffer_of(dy + skip, static_cast<unsigned>(left < kRecordLimit ? left : kRecordLimit));
+    c.src = dy + skip;
+    c.bytes = static_cast<unsigned>(left < kRecordLimit ? left : kRecordLimit);
     c.ihp = ih + g.pad_h; c.iwp = iw + g.pad_w;
     // stride 1: byte offset of dy[img, 0, ihp, iwp]; otherwise of dy[img, 0, 0, 0]
     const bool unit = g.stride_h == 1 && g.stride_w == 1;
@@ -194,7 +196,7 @@ struct BackwardDataOps {
     return in ? c.anchor + (oh * g.OW + ow) * 4 : kDead;
   }
   __device__ float load_b(const BCtx& c, const Step& e, int at, int k) const {
-    return buffer_load1(c.src, at, min(e.c0 + k, g.D - 1) * (g.OH * g.OW * 4));
+    return buffer_load1(buffer_of(c.src, e.c0 + k < g.D ? c.bytes : 0u), at, (e.c0 + k) * (g.OH * g.OW * 4));
   }
   __device__ float* column(int n) const {
     const int hw = g.H * g.W, img = n / hw, r = n - img * hw;

@@ -584,6 +584,9 @@ def test_both_gradients_in_a_workspace_that_holds_the_operands_of_one(mode):
     (2, 32, 24, 26, 33, (3, 3), (1, 1), (2, 2), (1, 1)),
     (2, 50, 19, 23, 40, (3, 3), (1, 1), (1, 1), (1, 1)),
     (5, 33, 11, 11, 17, (1, 1), (0, 0), (1, 1), (1, 1)),
+    # gathered products: channels (of dy: filters) that fill no whole step of sixteen
+    (2, 69, 9, 15, 250, (3, 3), (1, 1), (1, 1), (1, 1)),
+    (3, 130, 9, 15, 140, (1, 1), (0, 0), (1, 1), (1, 1)),
 ])
 def test_an_infinity_stays_an_infinity_in_fp32_products(shape):
     """What pads a K step is zero times zero: one infinite element of an operand makes the results that it
