@@ -346,9 +346,13 @@ bool has_module_hooks() {
       PyUnicode_InternFromString("_global_forward_pre_hooks"), PyUnicode_InternFromString("_global_forward_hooks"),
       PyUnicode_InternFromString("_global_backward_pre_hooks"), PyUnicode_InternFromString("_global_backward_hooks")};
   if (module == nullptr) { PyErr_Clear(); return true; }
+  PyObject* const scope = PyModule_GetDict(module);
   for (PyObject* const name : names) {
-    PyObject* const hooks = name == nullptr ? nullptr : PyDict_GetItem(PyModule_GetDict(module), name);
-    if (hooks == nullptr || !PyDict_Check(hooks) || PyDict_Size(hooks) != 0) return true;
+    PyObject* const hooks = name == nullptr ? nullptr : PyDict_GetItemWithError(scope, name);
+    if (hooks == nullptr || !PyDict_Check(hooks) || PyDict_Size(hooks) != 0) {
+      PyErr_Clear();
+      return true;
+    }
   }
   return false;
 }
