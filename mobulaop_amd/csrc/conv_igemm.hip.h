@@ -469,8 +469,8 @@ __device__ __forceinline__ void igemm_tile(const Ops& ops, int m0, int n0, int s
     // forward / data gradient / weight gradient: 1011 / 1014 / 974 us; LDS accesses under products 984 /
     // 982 / 937; loads between them 924 / 916 / 937; results written without a test per element 914 / 894 /
     // 928; the LDS writes where they stand 880 / 873 / 915 (without any load after the first steps it is 868 / 870 / 825).
-    // (Steps back to back on one device; in a profile of whole steps the clock is a little lower and these are 903 / 898 /
-    // 939, 87, 88 and 84 % of their clocks in matrix instructions.)
+    // (Back to back on one device; devices and runs differ by 4 %, and profiles/conv2d_cfg5_mfma.txt has some 3 % more: 87,
+    // 87 and 84 % of the clocks in matrix instructions.)
     f32x4 fa[2][2], fb[2][2];
     auto read = [&](int buf, int h) {
 #pragma unroll

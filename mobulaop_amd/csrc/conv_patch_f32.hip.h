@@ -122,7 +122,7 @@ __device__ __forceinline__ void wait_for_memory() { __builtin_amdgcn_s_waitcnt(0
 //   second half:  products of group 1 | fragment reads of group 0 of step t + 1 | requests for the left
 //                 operand of step t + 2 and for a share of the next chunk's patch
 // (Requests and reads in front of the products, a full wait per step: 1079 us instead of 1046 for the
-// forward product of 32 x 256 x 56 x 56, 3 x 3, which igemm_kernel does in 903.)
+// forward product of 32 x 256 x 56 x 56, 3 x 3, which igemm_kernel does in some 900.)
 // f: where things are.  f.request(stage) asks for the next step's left operand, f.request_patch() for a
 // share of the next patch; f.patch(), f.offsets(), f.valid() are those of the step to read, f.next() goes on.
 // The k that pad a step meet zeros in the left operand, and have to meet zeros here as well: some other k's value,

@@ -47,3 +47,12 @@ def test_traffic_of_a_summary_for_other_sources_is_not_quoted(tmp_path):
     stale.write_text(open(TRAFFIC).read().replace(bench.kernel_source_digest(), '0' * 16))
     assert bench.measured_traffic(str(stale), 'backward_blocked_kernel') is None
     assert bench.measured_traffic(str(tmp_path / 'absent.txt'), 'backward_blocked_kernel') is None
+
+
+def test_every_conv_summary_names_the_kernel_sources_of_this_tree():
+    import glob
+    files = sorted(glob.glob(os.path.join(ROOT, 'profiles', 'conv2d_*.txt')))
+    assert len(files) >= 2
+    for f in files:
+        assert 'kernel sources: ' + bench.conv_source_digest() in open(f).read(), (
+            os.path.basename(f) + ' was measured on other kernel sources: run its commands again')
