@@ -260,10 +260,6 @@ void conv2d_backward_data_ecf81c91(const int device_id, const int n, const float
                                    const int pad_h, const int pad_w, const int stride_h,
                                    const int stride_w, const int dilation_h, const int dilation_w,
                                    float* dx);
-/* (With the option "conv_compute" set to 1 or 2 and unit strides the weight gradient is formed
- * from whole zero-padded planes: a non-finite value of x then also meets zeros of dy that belong
- * to a neighbouring channel's or image's positions, and 0 x inf = NaN ends up in the gradient of
- * that neighbouring channel's weights.  Mode 0 confines a non-finite x to its own channel.) */
 void conv2d_backward_weight_ecf81c91(const int device_id, const int n, const float* dy, const float* x,
                                      const int accumulate, const int batch, const int channels,
                                      const int height, const int width, const int filters,
@@ -271,7 +267,7 @@ void conv2d_backward_weight_ecf81c91(const int device_id, const int n, const flo
                                      const int pad_w, const int stride_h, const int stride_w,
                                      const int dilation_h, const int dilation_w, float* dw);
 /* dx and dw of one backward pass in one call (overwritten; a null pointer: not wanted), with the
- * conversions of their operands shared where the option "conv_compute" asks for bf16 products. */
+ * conversions of their operands shared where the products have bf16 operands or fp32 ones in bf16 parts. */
 void mobula_hip_conv2d_backward(const int device_id, const float* dy, const float* x, const float* weight,
                                 const int batch, const int channels, const int height, const int width,
                                 const int filters, const int kernel_h, const int kernel_w, const int pad_h,
@@ -302,10 +298,14 @@ void mobula_hip_clear_error(void);
  * lets helper kernels of a call run on a second stream of the device, 0 keeps
  * everything on the caller's stream; "conv_compute": 0 (default) multiplies the
  * convolution's fp32 operands as they are, 1 rounds them to bf16 and accumulates
- * in fp32 (results about 2e-3 off; a non-finite value in x can make the weight
- * gradient of a neighbouring channel NaN, see conv2d_backward_weight), 2 splits
- * every operand into two bf16 and forms three bf16 products per multiply-add
- * (results about 5e-6 off; non-finite values as in mode 1);
+ * in fp32 (results about 2e-3 off), 2 splits every operand into two bf16 and
+ * forms three bf16 products per multiply-add (results about 5e-6 off; an
+ * infinity gives NaN);
+ * "conv_fp32_split": 1 (default) lets fp32 products of large layers be formed
+ * from three bf16 parts of every operand, six products of parts for one of
+ * fp32, where that is faster (results as near to exact ones as the fp32
+ * kernels'; tensors with infinities, NaN, subnormals or products near the
+ * ends of the range take those), 0 never, 2 wherever a product fits;
  * "roialign_tile_columns": 0 (default) lets the backward pass choose its tile
  * width from the size of the map, 56 or 28 fixes it; "roialign_row_split": 0
  * (default) lets it choose how many wavefronts share a tile row's work list,

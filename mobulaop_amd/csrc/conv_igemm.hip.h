@@ -56,7 +56,7 @@ __device__ __forceinline__ float buffer_load1(__amdgpu_buffer_rsrc_t r, int voff
 // and whether it falls into the padding is worked out once per step and lane,
 // and the 16 channels are 16 loads from one address with scalar plane offsets.
 // The left operand is a copy of the weights in that order, [Mpad][taps][Cpad],
-// zero where a row or channel is padding (arrange_weights_kernel), so that its
+// zero where a row or channel is padding (gather_tables_kernel), so that its
 // loads need no guards; padding channels of the gathered operand are loaded
 // through a descriptor of no bytes: zeros.
 
@@ -67,29 +67,50 @@ struct GatherStep {
   int c0;         // first channel of the step
 };
 
-// steps[s] for s = tap * (Cpad / 16) + c0 / 16; sign = +1: taps walk forward over
-// the source (forward pass), -1: backward (data gradient, source = dy).
-__global__ void __launch_bounds__(256)
-build_gather_steps_kernel(GatherStep* __restrict__ steps, int count, int per_tap, int KW, int dil_h,
-                          int dil_w, int row, int sign) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= count) return;
-  const int tap = s / per_tap, kh = tap / KW, kw = tap - kh * KW;
-  steps[s] = GatherStep{kh * dil_h, kw * dil_w, sign * (kh * dil_h * row + kw * dil_w) * 4,
-                        (s - tap * per_tap) * 16};
-}
+// Three bf16 parts stand for an fp32 value exactly, and their products for fp32 products, while no part
+// and no product of two parts leaves the normal range: biased exponents of 24 to 247 in either
+// operand, and the smallest two together at least 2^-100 (a product's last counted part is 2^-24 of it).
+// Infinities and NaN are outside, so are subnormals.  The fp32 kernels take the product otherwise; both
+// are launched, and the tensors' words decide on the device which of them returns at once.
+struct SplitRange {
+  const unsigned* a; const unsigned* b;   // exponent words of the operands; null: no choice to make
+  __device__ bool inside() const {
+    const unsigned ea = *a, eb = *b, both = ea | eb;
+    const int low_a = ea == 0u ? 31 : __builtin_ctz(ea), low_b = eb == 0u ? 31 : __builtin_ctz(eb);
+    return (both & 0x80000007u) == 0u && 8 * (low_a + low_b) >= 2 * 127 - 100;
+  }
+  __device__ bool leaves_split() const { return a != nullptr && !inside(); }
+  __device__ bool leaves_fp32() const { return a != nullptr && inside(); }
+};
 
-// out[m][tap][c] = w[m * stride_m + c * stride_c + tap] for m < M and c < C, else 0
-// (m < Mpad, c < Cpad).
+// What a gathered product reads besides the gathered tensor, in one launch: out[m][tap][c] =
+// w[m * stride_m + c * stride_c + tap] for m < M and c < C, else 0 (m < Mpad, c < Cpad), and, by the
+// workgroups past these, steps[s] for s = tap * (Cpad / 16) + c0 / 16; sign = +1: taps walk forward over
+// the source (forward pass), -1: backward (data gradient, source = dy).
+struct GatherTables {
+  const float* w; float* out;
+  int M, Mpad, C, Cpad, taps; long long stride_m, stride_c;
+  GatherStep* steps;
+  int KW, dil_h, dil_w, row, sign;
+  unsigned weight_blocks, step_blocks;
+};
 __global__ void __launch_bounds__(256)
-arrange_weights_kernel(const float* __restrict__ w, float* __restrict__ out, int M, int Mpad, int C,
-                       int Cpad, int taps, long long stride_m, long long stride_c) {
-  const long long total = static_cast<long long>(Mpad) * taps * Cpad;
-  const long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
+gather_tables_kernel(GatherTables t, SplitRange range) {
+  if (range.leaves_fp32()) return;
+  if (blockIdx.x >= t.weight_blocks) {
+    const int s = (blockIdx.x - t.weight_blocks) * 256 + threadIdx.x, per_tap = t.Cpad / 16;
+    if (s >= t.taps * per_tap) return;
+    const int tap = s / per_tap, kh = tap / t.KW, kw = tap - kh * t.KW;
+    t.steps[s] = GatherStep{kh * t.dil_h, kw * t.dil_w, t.sign * (kh * t.dil_h * t.row + kw * t.dil_w) * 4,
+                            (s - tap * per_tap) * 16};
+    return;
+  }
+  const long long total = static_cast<long long>(t.Mpad) * t.taps * t.Cpad;
+  const long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
   if (i >= total) return;
-  const int c = static_cast<int>(i % Cpad), tap = static_cast<int>((i / Cpad) % taps);
-  const int m = static_cast<int>(i / (static_cast<long long>(Cpad) * taps));
-  out[i] = (m < M && c < C) ? w[m * stride_m + c * stride_c + tap] : 0.0f;
+  const int c = static_cast<int>(i % t.Cpad), tap = static_cast<int>((i / t.Cpad) % t.taps);
+  const int m = static_cast<int>(i / (static_cast<long long>(t.Cpad) * t.taps));
+  t.out[i] = (m < t.M && c < t.C) ? t.w[m * t.stride_m + c * t.stride_c + tap] : 0.0f;
 }
 
 // ---- operand functors -------------------------------------------------------
@@ -224,7 +245,8 @@ build_taps_kernel(Tap* __restrict__ taps, int count, int KH, int KW, int plane, 
 // (W + 2 pad_w), in which every tap of every output pixel is an element (no range tests).
 __global__ void __launch_bounds__(256)
 pad_planes_kernel(const float* __restrict__ x, float* __restrict__ xp, int H, int W, int pad_h, int pad_w,
-                  int Hp, int Wp) {
+                  int Hp, int Wp, SplitRange range) {
+  if (range.leaves_fp32()) return;
   const float* in = x + static_cast<size_t>(blockIdx.x) * H * W;
   float* out = xp + static_cast<size_t>(blockIdx.x) * Hp * Wp;
   const int step_h = 256 / Wp, step_w = 256 - step_h * Wp;   // 256 elements further on
@@ -643,7 +665,8 @@ struct TileSplit {
 // and read the same gathered operand.
 template <typename Ops, int MODE>
 __global__ void __launch_bounds__(Tile::NT, 2)
-igemm_kernel(Ops ops, int row_tiles, TileSplit split, float* __restrict__ piece_buffer) {
+igemm_kernel(Ops ops, int row_tiles, TileSplit split, float* __restrict__ piece_buffer, SplitRange range) {
+  if (range.leaves_fp32()) return;
   const int whole_blocks = tile_blocks(split.whole);
   int t, s_begin = 0, s_end = k_steps(ops.K);
   float* piece = nullptr;
@@ -664,7 +687,8 @@ igemm_kernel(Ops ops, int row_tiles, TileSplit split, float* __restrict__ piece_
 // Results of the split tiles: sum of their pieces, in piece order.
 template <typename Ops>
 __global__ void __launch_bounds__(256)
-reduce_pieces_kernel(Ops ops, int row_tiles, TileSplit split, const float* __restrict__ piece_buffer) {
+reduce_pieces_kernel(Ops ops, int row_tiles, TileSplit split, const float* __restrict__ piece_buffer, SplitRange range) {
+  if (range.leaves_fp32()) return;
   constexpr int TILE = Tile::BM * Tile::BN;
   const int local = blockIdx.x / (TILE / 256), e = (blockIdx.x % (TILE / 256)) * 256 + threadIdx.x;
   const int t = split.whole + local;
@@ -679,7 +703,8 @@ reduce_pieces_kernel(Ops ops, int row_tiles, TileSplit split, const float* __res
 template <int MODE>
 __global__ void __launch_bounds__(Tile::NT)
 igemm_weight_kernel(BackwardWeightOps ops, int k_per_slice, int k_total, int row_tiles,
-                    int tiles_per_slice, int count) {
+                    int tiles_per_slice, int count, SplitRange range) {
+  if (range.leaves_fp32()) return;
   const int t = tile_of_block(count);
   if (t < 0) return;
   const int slice = t / tiles_per_slice, tile = t - slice * tiles_per_slice;
@@ -696,7 +721,8 @@ igemm_weight_kernel(BackwardWeightOps ops, int k_per_slice, int k_total, int row
 template <int V>
 __global__ void __launch_bounds__(256)
 reduce_slices_kernel(const float* __restrict__ partial, float* __restrict__ out, long long count,
-                     int slices, int groups, int accumulate) {
+                     int slices, int groups, int accumulate, SplitRange range) {
+  if (range.leaves_fp32()) return;
   typedef float vec __attribute__((ext_vector_type(V)));
   __shared__ vec sums[256];
   const int per_block = 256 / groups, local = threadIdx.x % per_block, group = threadIdx.x / per_block;

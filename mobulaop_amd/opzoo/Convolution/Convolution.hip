@@ -8,6 +8,7 @@
 // (opzoo/Convolution/Convolution.py:17-57), computed on the matrix cores
 // without a column buffer.
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "runtime.h"
@@ -53,9 +54,9 @@ int resident_workgroups() {
 // device holds at a time, and no device is assumed to hold more than this.
 constexpr int kMaxPieceBlocks = 2048;
 
-conv::TileSplit split_tiles(int count, int steps, int resident) {
+conv::TileSplit split_tiles(int count, int steps, int resident, int room = kMaxPieceBlocks) {
   conv::TileSplit split{count, 1, steps};
-  resident = std::min(resident, kMaxPieceBlocks);
+  resident = std::min(resident, room);
   if (resident <= 0 || steps < 2) return split;
   const int rest = count % resident;
   // a last round that fills less than half of the device is cut along K
@@ -69,24 +70,24 @@ conv::TileSplit split_tiles(int count, int steps, int resident) {
 }
 
 template <typename Ops, int MODE>
-void launch_igemm_mode(const Ops& ops, float* piece_buffer, hipStream_t stream) {
+void launch_igemm_mode(const Ops& ops, float* piece_buffer, conv::SplitRange range, hipStream_t stream) {
   const int row_tiles = (ops.M + conv::Tile::BM - 1) / conv::Tile::BM;
   const int count = row_tiles * ((ops.Ncols + conv::Tile::BN - 1) / conv::Tile::BN);
   const conv::TileSplit split = split_tiles(count, conv::k_steps(ops.K), resident_workgroups<Ops, MODE>());
   const int rest = count - split.whole;
   const dim3 grid(conv::tile_blocks(split.whole) + rest * split.pieces);
-  conv::igemm_kernel<Ops, MODE><<<grid, conv::Tile::NT, 0, stream>>>(ops, row_tiles, split, piece_buffer);
+  conv::igemm_kernel<Ops, MODE><<<grid, conv::Tile::NT, 0, stream>>>(ops, row_tiles, split, piece_buffer, range);
   if (rest > 0)
     conv::reduce_pieces_kernel<Ops><<<rest * (conv::Tile::BM * conv::Tile::BN / 256), 256, 0, stream>>>(
-        ops, row_tiles, split, piece_buffer);
+        ops, row_tiles, split, piece_buffer, range);
 }
 
 template <typename Ops>
-void launch_igemm(const Ops& ops, float* piece_buffer, hipStream_t stream) {
+void launch_igemm(const Ops& ops, float* piece_buffer, hipStream_t stream, conv::SplitRange range = {}) {
   switch (compute_mode()) {
-    case conv::kBf16: launch_igemm_mode<Ops, conv::kBf16>(ops, piece_buffer, stream); break;
-    case conv::kBf16x3: launch_igemm_mode<Ops, conv::kBf16x3>(ops, piece_buffer, stream); break;
-    default: launch_igemm_mode<Ops, conv::kFp32>(ops, piece_buffer, stream);
+    case conv::kBf16: launch_igemm_mode<Ops, conv::kBf16>(ops, piece_buffer, range, stream); break;
+    case conv::kBf16x3: launch_igemm_mode<Ops, conv::kBf16x3>(ops, piece_buffer, range, stream); break;
+    default: launch_igemm_mode<Ops, conv::kFp32>(ops, piece_buffer, range, stream);
   }
 }
 
@@ -110,39 +111,79 @@ int resident_workgroups_b16() {
   return cached;
 }
 
-// The columns from n_base on (`columns` of them) of a bf16 product in tiles of shape S.  Pieces of
-// these products are ROWS x 256 floats; the piece buffer holds kMaxPieceBlocks pieces of 128 x 128.
+// How a bf16 product is cut into tiles of shape S and, where that is faster, the last round's along K; about
+// how long it takes (us).
 template <typename Ops, typename S>
-void launch_igemm_b16_shape(const Ops& ops, int n_base, int columns, float* piece_buffer, hipStream_t stream) {
-  const int row_tiles = (ops.M + S::ROWS - 1) / S::ROWS, count = row_tiles * ((columns + S::COLS - 1) / S::COLS);
-  const int room = kMaxPieceBlocks * conv::Tile::BM * conv::Tile::BN / (S::ROWS * conv::TileB16::BN);
-  const int resident = std::min(resident_workgroups_b16<Ops, S>(), room);
-  const conv::TileSplit split = split_tiles(count, conv::k_steps_b16(ops.K), resident);
-  const int rest = count - split.whole;
-  const dim3 grid(conv::tile_blocks(split.whole) + rest * split.pieces);
-  conv::igemm_b16_kernel<Ops, S><<<grid, 64 * S::WAVES, 0, stream>>>(ops, row_tiles, n_base, split, piece_buffer);
-  if (rest > 0)
-    conv::reduce_pieces_b16_kernel<Ops, S><<<rest * (S::ROWS * conv::TileB16::BN / 256), 256, 0, stream>>>(
-        ops, row_tiles, n_base, split, piece_buffer);
+conv::TileSplit split_b16(const Ops& ops, double* cost) {
+  const int row_tiles = (ops.M + S::ROWS - 1) / S::ROWS, count = row_tiles * ((ops.Ncols + S::COLS - 1) / S::COLS);
+  const int room = kMaxPieceBlocks * conv::Tile::BM * conv::Tile::BN / (S::ROWS * S::COLS);   // (of the piece buffer)
+  const int resident = resident_workgroups_b16<Ops, S>(), steps = ops.k_steps(), cus = std::max(resident / S::PER_CU, 1);
+  // a step of 256 rows: 0.97 us with one part, 1.1 with two (32 x 256 x 56 x 56, 256 filters 3 x 3); lower tiles: loads
+  // and barriers that nothing hides cost what 64 rows do, 40 where two workgroups share a CU (and halve its
+  // rate; one alone: a third more); three parts: 1.2 us for 128 rows, 0.68 for 64; two steps more to fill the
+  // stages and write results
+  const double base = Ops::PARTS == 1 ? 0.97 : 1.1;
+  const double step = Ops::PARTS == 3 ? 2.24 * (S::ROWS + 20) / 276.0 : base * (S::ROWS + (S::PER_CU == 2 ? 40 : 64)) / 320.0;
+  auto time = [&](int workgroups, int length) {
+    return step * (length + 2) * (workgroups <= cus && S::PER_CU == 2 ? 1.33 : static_cast<double>((workgroups + cus - 1) / cus));
+  };
+  const conv::TileSplit whole{count, 1, steps}, cut = split_tiles(count, steps, resident, room);
+  const double whole_time = time(count, steps);
+  const int rest = count - cut.whole, pieces = rest * cut.pieces;
+  // pieces are written and read again at some 4 TB/s, and added up by a kernel of their own
+  const double cut_time = (cut.whole > 0 ? time(cut.whole, steps) : 0.0) + time(pieces, cut.steps_per_piece) +
+                          static_cast<double>(pieces) * S::ROWS * S::COLS * 8 / 4e6 + 5.0;
+  const bool cut_wins = rest > 0 && cut_time < whole_time;
+  if (cost != nullptr) *cost = cut_wins ? cut_time : whole_time;
+  return cut_wins ? cut : whole;
 }
 
-// Tiles by the number of rows: the height whose tiles cover them with the least in all, a tile costing
-// its rows and (the columns' operand is loaded for any height) some 64 more.  (Tried for a last round that
-// fills between half and three quarters of the device: one round of narrower tiles, 256 x 160,
+// A bf16 product in tiles of shape S; returns the pieces that are left to be added up.
+template <typename Ops, typename S>
+conv::PiecesB16 launch_igemm_b16_shape(const Ops& ops, float* piece_buffer, conv::SplitRange range, hipStream_t stream) {
+  const conv::TileSplit split = split_b16<Ops, S>(ops, nullptr);
+  const int row_tiles = (ops.M + S::ROWS - 1) / S::ROWS;
+  const int rest = row_tiles * ((ops.Ncols + S::COLS - 1) / S::COLS) - split.whole;
+  const dim3 grid(conv::tile_blocks(split.whole) + rest * split.pieces);
+  conv::igemm_b16_kernel<Ops, S><<<grid, 64 * S::WAVES, 0, stream>>>(ops, row_tiles, split, piece_buffer, range);
+  return conv::PiecesB16{piece_buffer, split, row_tiles, S::ROWS, static_cast<unsigned>(rest) * S::ROWS, range};
+}
+
+// Tiles of the height that takes least: high ones where there are many, lower ones where the last row of tiles
+// would be mostly empty or whole tiles fill the device that high ones would have to be cut along K for
+// (130 rows, 15075 columns, K = 864, two parts: 46 us with 256 rows, 40 with 192, 32 with 64).  (Tried for a last
+// round that fills between half and three quarters of the device: one round of narrower tiles, 256 x 160,
 // over the same columns.  The two rounds then take as long as before -- the full round alone runs
 // slower than beside a half-empty one -- so there is one shape per product.)
 template <typename Ops>
-void launch_igemm_b16(const Ops& ops, float* piece_buffer, hipStream_t stream) {
-  int best = 0;
-  long long least = 0;
-  for (const int rows : {256, 192, 128, 64}) {
-    const long long cost = static_cast<long long>((ops.M + rows - 1) / rows) * (rows + 64);
-    if (best == 0 || cost < least) { best = rows; least = cost; }
+int rows_b16(const Ops& ops, double* least) {
+  double cost[4] = {1e30, 1e30, 0.0, 0.0};
+  if constexpr (Ops::PARTS < 3) {
+    split_b16<Ops, conv::ShapeB16<256, Ops::PARTS>>(ops, cost);
+    split_b16<Ops, conv::ShapeB16<192, Ops::PARTS>>(ops, cost + 1);
   }
-  if (best == 64) launch_igemm_b16_shape<Ops, conv::FlatShapeB16>(ops, 0, ops.Ncols, piece_buffer, stream);
-  else if (best == 128) launch_igemm_b16_shape<Ops, conv::LowShapeB16>(ops, 0, ops.Ncols, piece_buffer, stream);
-  else if (best == 192) launch_igemm_b16_shape<Ops, conv::MidShapeB16>(ops, 0, ops.Ncols, piece_buffer, stream);
-  else launch_igemm_b16_shape<Ops, conv::WideShapeB16>(ops, 0, ops.Ncols, piece_buffer, stream);
+  split_b16<Ops, conv::ShapeB16<128, Ops::PARTS>>(ops, cost + 2);
+  split_b16<Ops, conv::ShapeB16<64, Ops::PARTS>>(ops, cost + 3);
+  const int best = static_cast<int>(std::min_element(cost, cost + 4) - cost);
+  if (least != nullptr) *least = cost[best];
+  return 256 - 64 * best;
+}
+template <typename Ops>
+conv::PiecesB16 launch_igemm_b16(const Ops& ops, float* piece_buffer, hipStream_t stream, conv::SplitRange range = {}) {
+  const int rows = rows_b16(ops, nullptr);
+  if constexpr (Ops::PARTS < 3) {
+    if (rows == 256)
+      return launch_igemm_b16_shape<Ops, conv::ShapeB16<256, Ops::PARTS>>(ops, piece_buffer, range, stream);
+    if (rows == 192)
+      return launch_igemm_b16_shape<Ops, conv::ShapeB16<192, Ops::PARTS>>(ops, piece_buffer, range, stream);
+  }
+  if (rows == 128)
+    return launch_igemm_b16_shape<Ops, conv::ShapeB16<128, Ops::PARTS>>(ops, piece_buffer, range, stream);
+  return launch_igemm_b16_shape<Ops, conv::ShapeB16<64, Ops::PARTS>>(ops, piece_buffer, range, stream);
+}
+template <typename Ops>
+void reduce_b16(const Ops& ops, const conv::PiecesB16& pieces, hipStream_t stream) {
+  if (pieces.blocks > 0) conv::reduce_pieces_b16_kernel<Ops><<<pieces.blocks, 256, 0, stream>>>(ops, pieces);
 }
 
 // workgroups the weight gradient aims at: two rounds of what a 256-CU device holds at a time, three to a
@@ -196,50 +237,41 @@ bool describe(conv::Geometry* g, const char* what, int N, int C, int H, int W, i
   return true;
 }
 
-conv::Tap* make_taps(int count, int KH, int KW, int plane, int dil_h, int dil_w, size_t extra_bytes,
-                     char** extra, hipStream_t stream) {
-  const size_t tap_bytes = (sizeof(conv::Tap) * count + 255) / 256 * 256;
-  char* ws = static_cast<char*>(mobula_hip::workspace(tap_bytes + extra_bytes));
-  if (failed()) return nullptr;
-  conv::Tap* taps = reinterpret_cast<conv::Tap*>(ws);
-  if (extra != nullptr) *extra = ws + tap_bytes;
-  conv::build_taps_kernel<<<(count + 255) / 256, 256, 0, stream>>>(taps, count, KH, KW, plane, dil_h, dil_w);
-  return taps;
-}
+constexpr size_t kPieceBytes = sizeof(float) * kMaxPieceBlocks * conv::Tile::BM * conv::Tile::BN;
 
-// Workspace of a gathered product (forward, data gradient): the table of K
-// steps and the weights in [Mpad][taps][Cpad] order.  channels = what K runs
-// over besides the taps, plane_row = row length of the gathered tensor.
-struct GatherPlan { conv::GatherStep* steps; float* weights; float* pieces; int K; };
+// A gathered product (forward, data gradient): its table of K steps and its weights in [Mpad][taps][Cpad]
+// order, `bytes` of workspace.  channels = what K runs over besides the taps, plane_row = row length of
+// the gathered tensor.
+struct GatherPlan { conv::GatherTables tables; int K; size_t step_bytes, bytes; };
 
 bool plan_gather(GatherPlan* plan, const char* what, const conv::Geometry& g, const float* w, int M,
                  int channels, long long image_elems, int columns_per_image, int plane_row, int sign,
-                 long long stride_m, long long stride_c, hipStream_t stream) {
+                 long long stride_m, long long stride_c) {
   // a tile's columns span this many images at most; their byte offsets must stay below 2^31
   const long long span = (conv::Tile::BN - 1) / std::max(columns_per_image, 1) + 2;
   if (span * image_elems * 4 >= (1ll << 31)) {
     set_error("%s: images of %lld elements are too large for the 32-bit offsets of the gather", what, image_elems);
     return false;
   }
-  const int taps = g.KH * g.KW, cpad = (channels + 15) / 16 * 16, per_tap = cpad / 16;
+  const int taps = g.KH * g.KW, cpad = (channels + 15) / 16 * 16, count = taps * (cpad / 16);
   const int mpad = (M + conv::Tile::BM - 1) / conv::Tile::BM * conv::Tile::BM;
   const long long k = static_cast<long long>(taps) * cpad, wcount = k * mpad;
   if (k >= (1ll << 31) || wcount >= (1ll << 31)) { set_error("%s: weights too large", what); return false; }
-  const int count = taps * per_tap;
-  const size_t step_bytes = (sizeof(conv::GatherStep) * count + 255) / 256 * 256;
-  const size_t weight_bytes = (sizeof(float) * wcount + 255) / 256 * 256;
-  const size_t piece_bytes = sizeof(float) * kMaxPieceBlocks * conv::Tile::BM * conv::Tile::BN;
-  char* ws = static_cast<char*>(mobula_hip::workspace(step_bytes + weight_bytes + piece_bytes));
-  if (failed()) return false;
-  plan->steps = reinterpret_cast<conv::GatherStep*>(ws);
-  plan->weights = reinterpret_cast<float*>(ws + step_bytes);
-  plan->pieces = reinterpret_cast<float*>(ws + step_bytes + weight_bytes);
+  plan->tables = conv::GatherTables{w, nullptr, M, mpad, channels, cpad, taps, stride_m, stride_c, nullptr, g.KW, g.dil_h,
+                                    g.dil_w, plane_row, sign, static_cast<unsigned>(blocks_for_all(wcount)),
+                                    static_cast<unsigned>((count + 255) / 256)};
   plan->K = static_cast<int>(k);
-  conv::build_gather_steps_kernel<<<(count + 255) / 256, 256, 0, stream>>>(plan->steps, count, per_tap, g.KW,
-                                                                          g.dil_h, g.dil_w, plane_row, sign);
-  conv::arrange_weights_kernel<<<blocks_for_all(wcount), 256, 0, stream>>>(w, plan->weights, M, mpad, channels, cpad,
-                                                                           taps, stride_m, stride_c);
+  plan->step_bytes = align_to_256(sizeof(conv::GatherStep) * count);
+  plan->bytes = plan->step_bytes + align_to_256(sizeof(float) * wcount);
   return true;
+}
+
+// Fills the plan's tables, in the workspace at `at`; returns what follows them.
+char* build_gather(GatherPlan* plan, char* at, hipStream_t stream, conv::SplitRange range = {}) {
+  plan->tables.steps = reinterpret_cast<conv::GatherStep*>(at);
+  plan->tables.out = reinterpret_cast<float*>(at + plan->step_bytes);
+  conv::gather_tables_kernel<<<plan->tables.weight_blocks + plan->tables.step_blocks, 256, 0, stream>>>(plan->tables, range);
+  return at + plan->bytes;
 }
 
 // ---- products with bf16 operands in memory (conv_igemm_bf16.hip.h) ---------
@@ -248,137 +280,136 @@ bool plan_gather(GatherPlan* plan, const char* what, const conv::Geometry& g, co
 struct PrepB16 {
   size_t bytes = 0;
   conv::ArrangeJob weights{};
-  conv::BlockedJob gathered{};
-  conv::PaddedJob rows{}, columns{};
-  void launch(hipStream_t stream) const {
-    const unsigned blocks = gathered.blocks + columns.blocks + rows.blocks + weights.blocks;
-    if (blocks > 0) conv::prepare_b16_kernel<<<blocks, 256, 0, stream>>>(weights, gathered, rows, columns);
+  conv::BlockedJob first{}, second{};   // x of a forward pass; dy and x of a backward pass
+  template <int PARTS>
+  void launch(hipStream_t stream, conv::ExponentWords exponents = {}) const {
+    const unsigned blocks = first.blocks + second.blocks + weights.blocks;
+    if (blocks > 0) conv::prepare_b16_kernel<PARTS><<<blocks, 256, 0, stream>>>(weights, first, second, exponents);
   }
 };
-constexpr size_t kPieceBytes = sizeof(float) * kMaxPieceBlocks * conv::Tile::BM * conv::Tile::BN;
 
 enum Fit { kFits, kOther, kError };   // kOther: the shape is for the caller's other kernels
 
-// A gathered product: the weights as [K step][Mpad][32] bf16, the gathered tensor `src`
-// ([images][channels][src_pixels] fp32) as [images][channel block][src_pixels][32] bf16.  Fills in the
-// fields of `ops` and `prep` but for the addresses (place_gather_b16).  split: two sets of each, heads then
-// tails of the fp32 values, and three passes over K.
-Fit plan_gather_b16(conv::GatheredB16* ops, PrepB16* prep, const char* what, const conv::Geometry& g, const float* w,
-                    int M, int channels, const float* src, int images, int src_pixels, int columns_per_image,
-                    long long stride_m, long long stride_c, bool split) {
-  const int sets = split ? 2 : 1;
-  const int taps = g.KH * g.KW, cpad = (channels + 31) / 32 * 32;
+// A tensor as [part][images][channel block][pixels][16] bf16 (channels padded to whole K steps).
+template <int PARTS>
+int padded_channels(int channels) { return PARTS == 1 ? (channels + 31) / 32 * 32 : (channels + 15) / 16 * 16; }
+template <int PARTS>
+size_t blocked_bytes(int images, int channels, int pixels) {
+  return 2ull * PARTS * images * padded_channels<PARTS>(channels) * pixels;
+}
+template <int PARTS>
+conv::BlockedJob blocked_job(const float* src, int images, int channels, int pixels) {
+  const int cpad = padded_channels<PARTS>(channels);
+  const unsigned tiles_p = (pixels + 63) / 64, tiles_c = (cpad + 63) / 64;
+  return conv::BlockedJob{src, nullptr, channels, cpad, pixels, static_cast<size_t>(images) * cpad * pixels,
+                          pixels % 4 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0, tiles_p, tiles_c,
+                          tiles_p * tiles_c * images};
+}
+char* place_blocked(conv::BlockedJob* job, size_t bytes, char* at) {
+  job->dst = reinterpret_cast<unsigned short*>(at);
+  return at + align_to_256(bytes);
+}
+
+// A gathered product of M rows over `channels` of the gathered tensor ([images][channels][src_pixels]): fills in
+// the fields of `ops` and `prep` but for the addresses and the tensor itself.
+template <int PARTS>
+Fit plan_gather_b16(conv::GatheredB16<PARTS>* ops, PrepB16* prep, const char* what, const conv::Geometry& g,
+                    const float* w, int M, int channels, int images, int src_pixels, int columns_per_image,
+                    long long stride_m, long long stride_c) {
+  const int taps = g.KH * g.KW, cpad = padded_channels<PARTS>(channels);
   const long long image_bytes = static_cast<long long>(src_pixels) * cpad * 2;
   // a tile's columns span this many images at most; their byte offsets must stay below 2^31
-  const long long span = (conv::TileB16::BN - 1) / std::max(columns_per_image, 1) + 2;
-  if (split && (span + images) * image_bytes >= (1ll << 31)) return kOther;
+  const long long span = 255 / std::max(columns_per_image, 1) + 2;
+  if (PARTS > 1 && (span + PARTS * images) * image_bytes >= (1ll << 31)) return kOther;
   if (span * image_bytes >= (1ll << 31)) {
     set_error("%s: images of %lld bytes are too large for the 32-bit offsets of the gather", what, image_bytes);
     return kError;
   }
-  const int mpad = (M + 63) / 64 * 64;   // (rows of a tile past these are read from the next step's and not stored)
-  const long long k = static_cast<long long>(taps) * cpad, wcount = k * mpad;
-  const int weight_sets = split ? 3 : 1;   // (heads, heads again, tails: one per pass)
-  if (3 * k >= (1ll << 31) || 2 * weight_sets * wcount >= (1ll << 31)) {
-    if (split) return kOther;
+  const int mpad = (M + 63) / 64 * 64;   // (rows of a tile past these are read from what follows and not stored)
+  const long long wcount = static_cast<long long>(taps) * cpad * mpad;
+  if (2 * PARTS * wcount >= (1ll << 31)) {
+    if (PARTS > 1) return kOther;
     set_error("%s: weights too large", what);
     return kError;
   }
   ops->g = g; ops->M = M; ops->cpad = cpad; ops->mpad = mpad;
-  ops->K = static_cast<int>((split ? 3 : 1) * k);
-  ops->source_tail = split ? static_cast<int>(images * image_bytes) : 0;
-  const unsigned tiles_p = (src_pixels + 63) / 64, tiles_c = (cpad + 63) / 64;
+  ops->source_part = PARTS > 1 ? static_cast<int>(images * image_bytes) : 0;
   prep->weights = conv::ArrangeJob{w, nullptr, M, mpad, channels, cpad, taps, stride_m, stride_c,
-                                   split ? static_cast<size_t>(wcount) : 0,   // (in halves)
                                    static_cast<unsigned>(blocks_for_all(wcount / 2))};
-  prep->gathered = conv::BlockedJob{src, nullptr, channels, cpad, src_pixels,
-                                    split ? static_cast<size_t>(images) * image_bytes / 2 : 0,
-                                    src_pixels % 4 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0, tiles_p, tiles_c,
-                                    tiles_p * tiles_c * images};
-  prep->bytes += align_to_256(2 * weight_sets * wcount) + align_to_256(static_cast<size_t>(sets) * images * image_bytes);
+  prep->bytes += align_to_256(2 * PARTS * wcount);
   return kFits;
 }
-
-// Takes the product's operands from the workspace at `at`; returns what follows them.
-char* place_gather_b16(conv::GatheredB16* ops, PrepB16* prep, char* at) {
+template <int PARTS>
+char* place_weights(conv::GatheredB16<PARTS>* ops, PrepB16* prep, char* at) {
   const conv::ArrangeJob& a = prep->weights;
-  const size_t wcount = static_cast<size_t>(a.Mpad) * a.taps * a.Cpad;
-  unsigned short* const weights = reinterpret_cast<unsigned short*>(at);
-  at += align_to_256(2 * (a.tail != 0 ? 3 : 1) * wcount);
-  unsigned short* const source = reinterpret_cast<unsigned short*>(at);
-  const size_t images = prep->gathered.blocks / (prep->gathered.tiles_p * prep->gathered.tiles_c);
-  at += align_to_256((a.tail != 0 ? 2 : 1) * images * prep->gathered.P * a.Cpad * 2);
-  ops->wp = prep->weights.out = weights;
-  ops->src = prep->gathered.dst = source;
-  return at;
+  ops->wp = prep->weights.out = reinterpret_cast<unsigned short*>(at);
+  return at + align_to_256(2ull * PARTS * a.Mpad * a.taps * a.Cpad);
 }
 
-// The weight gradient at unit strides: bf16 copies of dy and x on a common padded grid, one plain product
-// per tap.  With split operands (head + tail, two bf16 for every fp32) the copies hold two sets of
-// planes, heads then tails, and the product walks the images three times: head x head, head x tail, tail x head.
-Fit plan_weight_b16(conv::WeightGradOpsB16* ops, PrepB16* prep, const conv::Geometry& g, const float* dy, const float* x,
-                    bool split) {
-  if (g.stride_h != 1 || g.stride_w != 1 || g.N == 0) return kOther;
-  const int sets = split ? 2 : 1;
-  const int Hg = g.H + 2 * g.pad_h, Wg = g.W + 2 * g.pad_w;
-  const long long G = static_cast<long long>(Hg) * Wg, Gp = (G + 31) / 32 * 32;
-  const long long dy_set = 2ll * g.N * g.D * Gp, x_set = 2ll * g.N * g.C * Gp;   // bytes of one set of planes
-  const long long dy_bytes = sets * dy_set, x_bytes = sets * x_set;
-  if (dy_bytes >= (1ll << 31) || 2 * x_bytes >= (1ll << 31) || 3ll * g.N * Gp >= (1ll << 31) || g.OH > Hg || g.OW > Wg)
-    return kOther;
-  ops->g = g; ops->M = g.D; ops->Ncols = g.C * g.KH * g.KW;
-  ops->split = split ? 1 : 0;
-  ops->K = static_cast<int>((split ? 3 : 1) * g.N * Gp); ops->Gp = static_cast<int>(Gp); ops->Wg = Wg;
-  ops->copy_bytes = static_cast<unsigned>(x_bytes);
-  // whole grid rows per workgroup and 16-byte loads where rows of both tensors allow it (a span
-  // of rows must be a multiple of 8 positions: Wg even and four rows, or any rows if Wg % 8 == 0)
-  int rows = (conv::kPaddedSpan - 32) / Wg;   // (the last span also takes the tail of the plane: up to 31 positions)
-  if (Wg % 8 != 0) rows = Wg % 2 == 0 ? rows / 4 * 4 : 0;
-  const bool vec = rows > 0 && g.W % 4 == 0 && g.OW % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
-                   reinterpret_cast<uintptr_t>(dy) % 16 == 0;
-  int spans, span;
-  if (vec) {
-    span = std::min(rows, (Hg + 3) / 4 * 4);
-    spans = (Hg + span - 1) / span;
-  } else {   // a plane in as few, equally long spans as fit the kernel's LDS
-    spans = static_cast<int>((Gp + conv::kPaddedSpan - 1) / conv::kPaddedSpan);
-    span = static_cast<int>((Gp / 8 + spans - 1) / spans * 8);
+// The products of a call and the operands they share.
+template <int PARTS>
+struct ForwardB16 {
+  conv::ForwardOpsB16<PARTS> ops;
+  PrepB16 prep;
+  size_t x_bytes;
+  Fit plan(const conv::Geometry& g, const float* x, const float* w, const float* bias, float* y) {
+    const long long taps = g.KH * g.KW;
+    ops.bias = bias; ops.y = y; ops.Ncols = g.N * g.OH * g.OW;
+    prep.first = blocked_job<PARTS>(x, g.N, g.C, g.H * g.W);
+    x_bytes = blocked_bytes<PARTS>(g.N, g.C, g.H * g.W);
+    prep.bytes = align_to_256(x_bytes);
+    return plan_gather_b16<PARTS>(&ops, &prep, "conv2d_forward", g, w, g.D, g.C, g.N, g.H * g.W, g.OH * g.OW, g.C * taps,
+                                  taps);
   }
-  const unsigned rows_planes = static_cast<unsigned>(g.N) * g.D, columns_planes = static_cast<unsigned>(g.N) * g.C;
-  prep->rows = conv::PaddedJob{dy, nullptr, nullptr, g.OH, g.OW, 0, 0, Hg, Wg, static_cast<int>(Gp), span, vec ? 1 : 0,
-                               split ? static_cast<size_t>(dy_set / 2) : 0, rows_planes, rows_planes * spans};
-  prep->columns = conv::PaddedJob{x, nullptr, nullptr, g.H, g.W, g.pad_h, g.pad_w, Hg, Wg, static_cast<int>(Gp), span,
-                                  vec ? 1 : 0, split ? static_cast<size_t>(x_set / 2) : 0, columns_planes,
-                                  columns_planes * spans};
-  prep->bytes += align_to_256(dy_bytes) + align_to_256(2 * x_bytes);
-  return kFits;
-}
+  char* place(char* at) {
+    at = place_blocked(&prep.first, x_bytes, at);
+    ops.src = prep.first.dst;
+    return place_weights<PARTS>(&ops, &prep, at);
+  }
+};
 
-char* place_weight_b16(conv::WeightGradOpsB16* ops, PrepB16* prep, char* at) {
-  const size_t sets = ops->split ? 2 : 1;
-  unsigned short* const dyg = reinterpret_cast<unsigned short*>(at);
-  at += align_to_256(sets * 2 * ops->g.N * ops->g.D * ops->Gp);
-  unsigned short* const xg = reinterpret_cast<unsigned short*>(at);
-  // the shifted copy follows the first one directly (its bytes are a multiple of 64): the reads of
-  // the last plane that run past its end then land in the other copy or beyond the buffer
-  // (zeros), never in workspace bytes that nothing wrote
-  prep->columns.shifted = reinterpret_cast<unsigned short*>(at + ops->copy_bytes);
-  at += align_to_256(2 * static_cast<size_t>(ops->copy_bytes));
-  ops->dyg = prep->rows.dst = dyg;
-  ops->xg = prep->columns.dst = xg;
-  return at;
-}
-
-Fit plan_data_b16(conv::BackwardDataOpsB16* ops, PrepB16* prep, const conv::Geometry& g, const float* dy, const float* w,
-                  int accumulate, float* dx) {
-  ops->dx = dx; ops->accumulate = accumulate; ops->Ncols = g.N * g.H * g.W;
-  const long long taps = g.KH * g.KW;
-  // row m of the left operand is input channel m: element [m][tap][d] = weight[d][m][tap]
-  return plan_gather_b16(ops, prep, "conv2d_backward_data", g, w, g.C, g.D, dy, g.N, g.OH * g.OW, g.H * g.W, taps,
-                         g.C * taps, compute_mode() == conv::kBf16x3);
-}
-
-bool bf16_mode() { return compute_mode() == conv::kBf16 || compute_mode() == conv::kBf16x3; }
+template <int PARTS>
+struct BackwardB16 {
+  conv::BackwardDataOpsB16<PARTS> data;
+  conv::WeightGradOpsB16<PARTS> weight;
+  PrepB16 prep;
+  size_t dy_bytes, x_bytes;
+  bool with_dx, with_dw;
+  // (dx, dw: null where they are not wanted)
+  Fit plan(const conv::Geometry& g, const float* dy, const float* x, const float* w, int accumulate, float* dx, float* dw) {
+    const long long taps = g.KH * g.KW;
+    with_dx = dx != nullptr; with_dw = dw != nullptr;
+    prep.first = blocked_job<PARTS>(dy, g.N, g.D, g.OH * g.OW);
+    dy_bytes = blocked_bytes<PARTS>(g.N, g.D, g.OH * g.OW);
+    x_bytes = 0;
+    prep.bytes = align_to_256(dy_bytes);
+    if (with_dw) {
+      x_bytes = blocked_bytes<PARTS>(g.N, g.C, g.H * g.W);
+      const long long cols = taps * ((g.C + 15) / 16 * 16), k = static_cast<long long>(g.N) * g.OH * g.OW;
+      if (std::max(x_bytes, dy_bytes) >= (1ull << 31) || cols >= (1ll << 28) || g.N == 0) return kOther;
+      prep.second = blocked_job<PARTS>(x, g.N, g.C, g.H * g.W);
+      prep.bytes += align_to_256(x_bytes);
+      weight.dw = dw; weight.accumulate = accumulate; weight.g = g; weight.M = g.D; weight.Ncols = static_cast<int>(cols);
+      weight.dblocks = padded_channels<PARTS>(g.D) / 16; weight.cblocks = padded_channels<PARTS>(g.C) / 16;
+      weight.ctiles = (g.C + 15) / 16;
+      const int step = conv::WeightGradOpsB16<PARTS>::STEP, rest = step % (g.OH * g.OW);
+      weight.step_n = step / (g.OH * g.OW); weight.step_h = rest / g.OW; weight.step_w = rest % g.OW;
+      if (k + 4 * step >= (1ll << 31)) return kOther;   // (pixels past the last are counted too)
+    }
+    if (!with_dx) return kFits;
+    data.dx = dx; data.accumulate = accumulate; data.Ncols = g.N * g.H * g.W;
+    // row m of the left operand is input channel m: element [m][tap][d] = weight[d][m][tap]
+    return plan_gather_b16<PARTS>(&data, &prep, "conv2d_backward_data", g, w, g.C, g.D, g.N, g.OH * g.OW, g.H * g.W, taps,
+                                  g.C * taps);
+  }
+  char* place(char* at) {
+    at = place_blocked(&prep.first, dy_bytes, at);
+    data.src = weight.dys = prep.first.dst;
+    if (with_dw) at = place_blocked(&prep.second, x_bytes, at);
+    weight.xs = prep.second.dst;
+    return with_dx ? place_weights<PARTS>(&data, &prep, at) : at;
+  }
+};
 
 // ---- fp32 products from patches (conv_patch_f32.hip.h) -----------------------
 
@@ -565,8 +596,7 @@ void flatten_pointwise(conv::PatchOps* o) {
   o->pitch = 1;
 }
 
-bool forward_from_patches(const conv::Geometry& g, const float* x, const float* weight, const float* bias, float* y,
-                          hipStream_t stream) {
+PatchProduct forward_patches(const conv::Geometry& g, const float* x, const float* weight, const float* bias, float* y) {
   PatchProduct p{};
   p.ops = conv::PatchOps{x, nullptr, nullptr, bias, y, g.N, g.C, g.H, g.W, g.D, g.OH, g.OW, g.stride_h, g.stride_w,
                          g.pad_h, g.pad_w, (g.KH - 1) * g.dil_h + 1, 0, 0, 0, 0, 0, 0, 0,
@@ -575,13 +605,21 @@ bool forward_from_patches(const conv::Geometry& g, const float* x, const float* 
   p.arrange = conv::ArrangePatchArgs{weight, nullptr, nullptr, 0, 0, 0, 0, 0, 0, g.KH, g.KW, g.KW, 0, 1, 0, 1,
                                      g.C * taps, taps, 0, 0, g.dil_h, g.dil_w};
   flatten_pointwise(&p.ops);
-  // Patches win where a step of sixteen channels of one tap is mostly padding (few channels), where
-  // a tile of 128 rows is, and at strides; large layers of round sizes stay with the gathered tiles.
-  const double cost = patch_product_cost(p);
-  if (cost < 0 || cost > gathered_product_cost(g.D, g.C, g.KH * g.KW, static_cast<long long>(g.N) * g.OH * g.OW))
-    return false;
-  run_patch_product(p, stream);
-  return true;
+  return p;
+}
+
+// Patches win where a step of sixteen channels of one tap is mostly padding (few channels), where
+// a tile of 128 rows is, and at strides; large layers of round sizes stay with the gathered tiles.
+// *cost: CU clocks of the cheaper way.
+bool patches_win(double patches, double gathered, double* cost) {
+  const bool win = patches >= 0 && patches <= gathered;
+  *cost = win ? patches : gathered;
+  return win;
+}
+
+bool forward_patches_win(const conv::Geometry& g, const PatchProduct& p, double* cost) {
+  return patches_win(patch_product_cost(p),
+                     gathered_product_cost(g.D, g.C, g.KH * g.KW, static_cast<long long>(g.N) * g.OH * g.OW), cost);
 }
 
 // Filter taps k that reach the pixels of a class: (offset + pad - k * dil) % stride == 0.  They are
@@ -604,11 +642,13 @@ TapsOfClass taps_of_class(int K, int dil, int stride, int pad, int offset) {
   return t;
 }
 
-bool data_gradient_from_patches(const conv::Geometry& g, const float* dy, const float* weight, float* dx,
-                                int accumulate, hipStream_t stream) {
-  if (g.stride_h > g.H || g.stride_w > g.W || g.stride_h * g.stride_w > 16) return false;
+// The data gradient by classes of pixels that meet the same taps (one per phase of the strides); cost < 0: it does
+// not fit.
+struct DataPatches { std::vector<PatchProduct> classes; double cost; };
+DataPatches data_patches(const conv::Geometry& g, const float* dy, const float* weight, float* dx, int accumulate) {
+  DataPatches d{{}, -1.0};
+  if (g.stride_h > g.H || g.stride_w > g.W || g.stride_h * g.stride_w > 16) return d;
   const long long taps = g.KH * g.KW;
-  std::vector<PatchProduct> classes;
   double cost = 0.0;
   for (int a = 0; a < g.stride_h; ++a)
     for (int b = 0; b < g.stride_w; ++b) {
@@ -628,11 +668,19 @@ bool data_gradient_from_patches(const conv::Geometry& g, const float* dy, const 
                                          th.step, tw.step};
       flatten_pointwise(&p.ops);
       const double product = patch_product_cost(p);
-      if (product < 0) return false;
+      if (product < 0) return d;
       cost += product;
-      classes.push_back(p);
+      d.classes.push_back(p);
     }
-  if (cost > gathered_product_cost(g.C, g.D, g.KH * g.KW, static_cast<long long>(g.N) * g.H * g.W)) return false;
+  d.cost = cost;
+  return d;
+}
+
+bool data_patches_win(const conv::Geometry& g, const DataPatches& d, double* cost) {
+  return patches_win(d.cost, gathered_product_cost(g.C, g.D, g.KH * g.KW, static_cast<long long>(g.N) * g.H * g.W), cost);
+}
+
+void run_data_patches(const conv::Geometry& g, const DataPatches& d, float* dx, int accumulate, hipStream_t stream) {
   for (int a = 0; a < g.stride_h && !accumulate; ++a)
     for (int b = 0; b < g.stride_w; ++b) {
       if (taps_of_class(g.KH, g.dil_h, g.stride_h, g.pad_h, a).count != 0 &&
@@ -643,9 +691,8 @@ bool data_gradient_from_patches(const conv::Geometry& g, const float* dy, const 
       conv::zero_class_kernel<<<blocks_for(count), 256, 0, stream>>>(dx, count, g.H, g.W, Ho, Wo, g.stride_h, g.stride_w,
                                                                      a, b);
     }
-  for (const PatchProduct& p : classes)
+  for (const PatchProduct& p : d.classes)
     if (!failed()) run_patch_product(p, stream);
-  return true;
 }
 
 // Weight gradient from patches: how its chunks are cut; cost < 0: it does not fit.
@@ -672,7 +719,8 @@ WeightCut cut_weight(const conv::Geometry& g) {
   return best;
 }
 
-void reduce_slices(const float* partial, float* out, long long count, int slices, int accumulate, hipStream_t stream) {
+void reduce_slices(const float* partial, float* out, long long count, int slices, int accumulate, hipStream_t stream,
+                   conv::SplitRange range = {}) {
   // groups of threads share an output's slices until the device has work; four outputs a thread
   // where they lie on 16-byte boundaries
   const int wide = count % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 ? 4 : 1;
@@ -680,31 +728,43 @@ void reduce_slices(const float* partial, float* out, long long count, int slices
   while (groups < 32 && 2 * groups <= slices && count / wide * groups < 128 * 1024) groups *= 2;
   const dim3 grid(static_cast<unsigned>((count / wide + 256 / groups - 1) / (256 / groups)));
   if (wide == 4)
-    conv::reduce_slices_kernel<4><<<grid, 256, 0, stream>>>(partial, out, count, slices, groups, accumulate);
+    conv::reduce_slices_kernel<4><<<grid, 256, 0, stream>>>(partial, out, count, slices, groups, accumulate, range);
   else
-    conv::reduce_slices_kernel<1><<<grid, 256, 0, stream>>>(partial, out, count, slices, groups, accumulate);
+    conv::reduce_slices_kernel<1><<<grid, 256, 0, stream>>>(partial, out, count, slices, groups, accumulate, range);
+}
+
+// CU clocks of igemm_weight_kernel: its steps span images and cost a little less than those from patches,
+// but it needs a padded copy of x at unit stride along a row, and tests every pixel at others.
+double weight_gathered_cost(const conv::Geometry& g) {
+  const double padded = static_cast<double>(g.N) * g.C * (g.H + 2 * g.pad_h) * (g.W + 2 * g.pad_w);
+  const int cols = g.C * g.KH * g.KW;
+  return (g.stride_w == 1 ? 2540.0 : 4870.0) * conv::k_steps(g.N * g.OH * g.OW) *
+             ((g.D + conv::Tile::BM - 1) / conv::Tile::BM) * ((cols + conv::Tile::BN - 1) / conv::Tile::BN) +
+         (g.stride_w == 1 ? 8.0 * padded / 4.5e12 * 2.4e9 * 256.0 : 0.0);
+}
+
+// CU clocks of the weight gradient from patches; < 0: it does not fit, or is the dearer way.
+template <typename T>
+double weight_patch_cost(const conv::Geometry& g, const WeightCut& cut) {
+  const int ohw = g.OH * g.OW, chunks_per_image = cut.cost < 0 ? 1 : (ohw + cut.px - 1) / cut.px;
+  // (planes that fill their chunks badly -- a few pixels -- go to the kernel whose K steps span images)
+  if (g.N == 0 || cut.cost < 0 || static_cast<long long>(chunks_per_image) * cut.px * 3 > 4ll * ohw) return -1.0;
+  if (static_cast<long long>(g.D) * ohw * 4 >= (1ll << 31) || static_cast<long long>(g.N) * chunks_per_image >= (1ll << 31))
+    return -1.0;
+  const long long tiles = static_cast<long long>((g.D + T::BM - 1) / T::BM) * ((g.C * g.KH * g.KW + T::BN - 1) / T::BN);
+  if (tiles >= (1ll << 20)) return -1.0;
+  const double here = cut.cost * g.N * static_cast<double>(tiles);
+  return here <= weight_gathered_cost(g) ? here : -1.0;
 }
 
 template <typename T>
 bool weight_gradient_with(const conv::Geometry& g, const float* dy, const float* x, int accumulate, float* dw,
                           hipStream_t stream) {
   const WeightCut cut = cut_weight<T>(g);
-  const int ohw = g.OH * g.OW, chunks_per_image = cut.cost < 0 ? 1 : (ohw + cut.px - 1) / cut.px;
-  // (planes that fill their chunks badly -- a few pixels -- go to the kernel whose K steps span images)
-  if (cut.cost < 0 || static_cast<long long>(chunks_per_image) * cut.px * 3 > 4ll * ohw) return false;
-  if (static_cast<long long>(g.D) * ohw * 4 >= (1ll << 31) || static_cast<long long>(g.N) * chunks_per_image >= (1ll << 31))
-    return false;
+  if (weight_patch_cost<T>(g, cut) < 0) return false;
+  const int ohw = g.OH * g.OW, chunks_per_image = (ohw + cut.px - 1) / cut.px;
   const int cols = g.C * g.KH * g.KW, row_tiles = (g.D + T::BM - 1) / T::BM;
   const long long tiles = static_cast<long long>(row_tiles) * ((cols + T::BN - 1) / T::BN);
-  if (tiles >= (1ll << 20)) return false;
-  // CU clocks against those of igemm_weight_kernel: its steps span images and cost a little less,
-  // but it needs a padded copy of x at unit stride along a row, and tests every pixel at others
-  const double here = cut.cost * g.N * static_cast<double>(tiles);
-  const long long padded = static_cast<long long>(g.N) * g.C * (g.H + 2 * g.pad_h) * (g.W + 2 * g.pad_w);
-  const double there = (g.stride_w == 1 ? 2540.0 : 4870.0) * conv::k_steps(g.N * ohw) *
-                           ((g.D + conv::Tile::BM - 1) / conv::Tile::BM) * ((cols + conv::Tile::BN - 1) / conv::Tile::BN) +
-                       (g.stride_w == 1 ? 8.0 * padded / 4.5e12 * 2.4e9 * 256.0 : 0.0);
-  if (here > there) return false;
   const int chunks = g.N * chunks_per_image;
   const bool wide = ohw % 4 == 0;
   const int resident = wide ? resident_with_lds(conv::patch_weight_kernel<T, true>, cut.lds)
@@ -731,12 +791,359 @@ bool weight_gradient_with(const conv::Geometry& g, const float* dy, const float*
   return true;
 }
 
+double weight_fp32_cost(const conv::Geometry& g) {
+  double patches;
+  if (g.D > 64) patches = weight_patch_cost<conv::PatchTile128>(g, cut_weight<conv::PatchTile128>(g));
+  else if (g.D > 32) patches = weight_patch_cost<conv::PatchTile64>(g, cut_weight<conv::PatchTile64>(g));
+  else patches = weight_patch_cost<conv::PatchTile32>(g, cut_weight<conv::PatchTile32>(g));
+  return patches >= 0 ? patches : weight_gathered_cost(g);
+}
+
 bool weight_gradient_from_patches(const conv::Geometry& g, const float* dy, const float* x, int accumulate, float* dw,
                                   hipStream_t stream) {
-  if (g.N == 0) return false;
   if (g.D > 64) return weight_gradient_with<conv::PatchTile128>(g, dy, x, accumulate, dw, stream);
   if (g.D > 32) return weight_gradient_with<conv::PatchTile64>(g, dy, x, accumulate, dw, stream);
   return weight_gradient_with<conv::PatchTile32>(g, dy, x, accumulate, dw, stream);
+}
+
+// ---- fp32 weight gradient in slices of K (igemm_weight_kernel) --------------------------
+
+// K = N*OH*OW is long and the result small: K is cut into slices of whole K steps, as many as give
+// every CU six workgroups; the partial sums of the slices are added in a fixed order afterwards.
+struct WeightPlan {
+  int row_tiles, tiles, slices, k_per_slice, k_total, Hp, Wp;
+  bool padded;
+  size_t tap_bytes, partial_bytes, bytes;
+};
+
+bool plan_weight(WeightPlan* plan, const conv::Geometry& g) {
+  const long long wt = static_cast<long long>(g.D) * g.C * g.KH * g.KW, cols = static_cast<long long>(g.C) * g.KH * g.KW;
+  const int row_tiles = (g.D + conv::Tile::BM - 1) / conv::Tile::BM;
+  const long long tiles = row_tiles * ((cols + conv::Tile::BN - 1) / conv::Tile::BN);
+  const long long k_total = static_cast<long long>(g.N) * g.OH * g.OW;   // < 2^31: checked by describe()
+  if (tiles >= (1ll << 20)) { set_error("conv2d_backward_weight: too many tiles"); return false; }
+  const long long k_steps = std::max<long long>(1, (k_total + conv::Tile::BK - 1) / conv::Tile::BK);
+  long long slices = std::min<long long>(k_steps, std::max<long long>(1, kWeightSlots / tiles));
+  const long long k_per_slice = (k_steps + slices - 1) / slices * conv::Tile::BK;
+  slices = std::max<long long>(1, (k_total + k_per_slice - 1) / k_per_slice);
+  // a zero-padded copy of x saves the gathered operand its range tests where eight output pixels
+  // of a row are eight neighbouring inputs (unit stride along a row); 32-bit offsets within an image
+  const int Hp = g.H + 2 * g.pad_h, Wp = g.W + 2 * g.pad_w;
+  const long long plane_p = static_cast<long long>(Hp) * Wp;
+  const bool padded = g.stride_w == 1 && g.N > 0 && plane_p * g.C * 4 < (1ll << 31) && plane_p < (1ll << 22);
+  const size_t tap_bytes = align_to_256(sizeof(conv::Tap) * cols);
+  const size_t partial_bytes = align_to_256(sizeof(float) * static_cast<size_t>(slices) * wt);
+  *plan = WeightPlan{row_tiles, static_cast<int>(tiles), static_cast<int>(slices), static_cast<int>(k_per_slice),
+                     static_cast<int>(k_total), Hp, Wp, padded, tap_bytes, partial_bytes,
+                     tap_bytes + partial_bytes + (padded ? sizeof(float) * static_cast<size_t>(g.N) * g.C * plane_p : 0)};
+  return true;
+}
+
+void run_weight(const WeightPlan& plan, const conv::Geometry& g, const float* dy, const float* x, int accumulate,
+                float* dw, char* ws, hipStream_t stream, conv::SplitRange range = {}) {
+  conv::BackwardWeightOps ops;
+  ops.dy = dy; ops.x = x; ops.g = g;
+  ops.M = g.D; ops.Ncols = g.C * g.KH * g.KW; ops.K = 0; ops.k_begin = 0;
+  conv::Tap* const taps = reinterpret_cast<conv::Tap*>(ws);
+  conv::build_taps_kernel<<<(ops.Ncols + 255) / 256, 256, 0, stream>>>(
+      taps, ops.Ncols, g.KH, g.KW, plan.padded ? plan.Hp * plan.Wp : g.H * g.W, g.dil_h, g.dil_w);
+  ops.taps = taps;
+  ops.partial = reinterpret_cast<float*>(ws + plan.tap_bytes);
+  ops.xp = nullptr; ops.Hp = plan.Hp; ops.Wp = plan.Wp;
+  if (plan.padded) {
+    float* const xp = reinterpret_cast<float*>(ws + plan.tap_bytes + plan.partial_bytes);
+    conv::pad_planes_kernel<<<dim3(g.N * g.C, static_cast<unsigned>((plan.Hp * plan.Wp + 2047) / 2048)), 256, 0, stream>>>(
+        x, xp, g.H, g.W, g.pad_h, g.pad_w, plan.Hp, plan.Wp, range);
+    ops.xp = xp;
+  }
+  const int count = plan.tiles * plan.slices;
+  const dim3 grid(conv::tile_blocks(count));
+  auto launch = [&](auto kernel) {
+    kernel<<<grid, conv::Tile::NT, 0, stream>>>(ops, plan.k_per_slice, plan.k_total, plan.row_tiles, plan.tiles, count, range);
+  };
+  switch (compute_mode()) {
+    case conv::kBf16: launch(conv::igemm_weight_kernel<conv::kBf16>); break;
+    case conv::kBf16x3: launch(conv::igemm_weight_kernel<conv::kBf16x3>); break;
+    default: launch(conv::igemm_weight_kernel<conv::kFp32>);
+  }
+  reduce_slices(ops.partial, dw, static_cast<long long>(g.D) * ops.Ncols, plan.slices, accumulate, stream, range);
+}
+
+// ---- products with bf16 operands, or operands of two bf16 ---------------------------------
+// (true: taken, or the call has failed)
+
+template <int PARTS>
+bool forward_b16(const conv::Geometry& g, const float* x, const float* weight, const float* bias, float* y,
+                 hipStream_t stream) {
+  ForwardB16<PARTS> f;
+  const Fit fit = f.plan(g, x, weight, bias, y);
+  if (fit != kFits) return fit == kError;
+  char* const ws = static_cast<char*>(mobula_hip::workspace(f.prep.bytes + kPieceBytes));
+  if (failed()) return true;
+  char* const pieces = f.place(ws);
+  f.prep.template launch<PARTS>(stream);
+  reduce_b16(f.ops, launch_igemm_b16(f.ops, reinterpret_cast<float*>(pieces), stream), stream);
+  MOBULA_HIP_TRY(hipGetLastError());
+  return true;
+}
+
+// Launches the wanted products of a backward pass (operands prepared): one after the other, the pieces of both
+// added up by one kernel behind them.
+template <int PARTS>
+void launch_gradients_b16(const BackwardB16<PARTS>& b, char* piece_buffers, hipStream_t stream,
+                          conv::SplitRange data_range = {}, conv::SplitRange weight_range = {}) {
+  float* const first = reinterpret_cast<float*>(piece_buffers);
+  float* const second = b.with_dx ? first + kPieceBytes / sizeof(float) : first;
+  conv::PiecesB16 data{}, weight{};
+  if (b.with_dx) data = launch_igemm_b16(b.data, first, stream, data_range);
+  if (b.with_dw) weight = launch_igemm_b16(b.weight, second, stream, weight_range);
+  if (data.blocks > 0 && weight.blocks > 0)
+    conv::reduce_gradients_b16_kernel<PARTS><<<data.blocks + weight.blocks, 256, 0, stream>>>(b.data, data, b.weight, weight);
+  else if (data.blocks > 0) reduce_b16(b.data, data, stream);
+  else reduce_b16(b.weight, weight, stream);
+}
+
+// The gradients that are wanted (null: not).  Both share the copy of dy; where the workspace cannot hold what both
+// need the caller takes one after the other.
+template <int PARTS>
+bool gradients_b16(const conv::Geometry& g, const float* dy, const float* x, const float* weight, int accumulate,
+                   float* dx, float* dw, hipStream_t stream) {
+  BackwardB16<PARTS> b;
+  const Fit fit = b.plan(g, dy, x, weight, accumulate, dx, dw);
+  if (fit != kFits) return fit == kError;
+  const size_t bytes = b.prep.bytes + (dx != nullptr && dw != nullptr ? 2 : 1) * kPieceBytes;
+  char* const ws = static_cast<char*>(dx != nullptr && dw != nullptr ? mobula_hip::workspace_if_possible(bytes)
+                                                                     : mobula_hip::workspace(bytes));
+  if (ws == nullptr || failed()) return failed();
+  char* const pieces = b.place(ws);
+  b.prep.template launch<PARTS>(stream);
+  launch_gradients_b16<PARTS>(b, pieces, stream);
+  MOBULA_HIP_TRY(hipGetLastError());
+  return true;
+}
+
+// ---- fp32 products from three bf16 parts per operand ---------------------------------------
+//
+// An fp32 value is three bf16 exactly, and six products of parts make an fp32 product but for terms of 2^-26
+// of it; sums are fp32 as before, with fewer roundings.  The matrix cores do sixteen times the bf16
+// products per clock, so six cost less than one of fp32; the parts are written by a pass over the
+// tensors first.  At 32 x 256 x 56 x 56, 256 filters 3 x 3: forward 911 -> 600 us, both gradients 1890 -> 1166
+// (the products 535 to 580 us, 1.2 to 1.3 PFLOP/s of bf16, what a large bf16 product of a library
+// reaches on this device; the passes 45 and 90), errors against 64 bits 5.0e-7 -> 2.9e-7 (3.3e-7 -> 2.5e-7
+// for the weights' gradient).  The fp32 kernels follow every such product and return at once unless a
+// tensor holds values the parts do not stand for (conv::SplitRange).
+
+// option "conv_fp32_split": 1 = where it pays (default), 0 = never, 2 = wherever a product fits
+int split_choice() { return mobula_hip::option("conv_fp32_split", 1); }
+
+// Exponent words of x (or dy), the weights, and dy beside x, ahead of a call's operands.
+constexpr size_t kWordBytes = 256;
+
+// Microseconds of the fp32 ways from the CU clocks of their kernels (which know nothing of rounds that are not full)
+// and of what the split ways take besides their products: the passes over the tensors, and the
+// launches that clear words and find nothing to do.  Fitted to some fifty layers of 10 us to 3 ms.
+double forward_fp32_us(double clocks) { return clocks / (256 * 2300.0) + 15.0; }
+double data_fp32_us(double clocks, size_t classes) {
+  return clocks / (256 * 2300.0) + 15.0 * std::max<size_t>(classes, 1);
+}
+double weight_fp32_us(double clocks) { return 1.1 * clocks / (256 * 2300.0) + 30.0; }
+double parts_us(long long elements) { return elements * 10 / 4.0e6; }
+constexpr double kSplitOverhead = 28.0;
+
+// Which of the wanted products split operands are faster for: those of some thirty us and more whose channels and
+// filters fill the tiles (forward, fp32 against split: 25 x 416 x 55 x 56, 168 filters 3 x 3: 1180 -> 563 us;
+// 5 x 96 x 119 x 109, 256: 263 -> 182; 8 x 432 x 8 x 9, 384: 50 against 93; 23 x 256 x 72 x 64, 32: 221
+// against 236).
+struct SplitChoice { bool dx, dw; };
+SplitChoice choose_split(const conv::Geometry& g, bool dx, bool dw);
+
+// True where the product is taken (or the call has failed).
+bool forward_split(const conv::Geometry& g, const float* x, const float* weight, const float* bias, float* y,
+                   double fp32_cost, hipStream_t stream) {
+  ForwardB16<3> f;
+  if (split_choice() != 2 && forward_fp32_us(fp32_cost) < kSplitOverhead) return false;
+  if (f.plan(g, x, weight, bias, y) != kFits) return false;
+  if (split_choice() != 2) {
+    double product = 0.0;
+    rows_b16(f.ops, &product);
+    if (product + parts_us(static_cast<long long>(g.N) * g.C * g.H * g.W) + kSplitOverhead > forward_fp32_us(fp32_cost)) return false;
+  }
+  GatherPlan plan;
+  const long long taps = g.KH * g.KW;
+  if (!plan_gather(&plan, "conv2d_forward", g, weight, g.D, g.C, static_cast<long long>(g.C) * g.H * g.W,
+                   g.OH * g.OW, g.W, +1, g.C * taps, taps))
+    return true;
+  char* const ws = static_cast<char*>(mobula_hip::workspace_if_possible(kWordBytes + f.prep.bytes + plan.bytes + kPieceBytes));
+  if (ws == nullptr) return failed();
+  unsigned* const words = reinterpret_cast<unsigned*>(ws);
+  const conv::SplitRange range{words, words + 1};
+  char* const tables = f.place(ws + kWordBytes);
+  float* const pieces = reinterpret_cast<float*>(tables + plan.bytes);
+  conv::clear_words_kernel<<<1, 64, 0, stream>>>(words, 2);
+  f.prep.launch<3>(stream, conv::ExponentWords{words + 1, words, nullptr});
+  reduce_b16(f.ops, launch_igemm_b16(f.ops, pieces, stream, range), stream);
+  build_gather(&plan, tables, stream, range);
+  conv::ForwardOps ops;
+  ops.x = x; ops.bias = bias; ops.y = y; ops.g = g; ops.M = g.D; ops.Ncols = f.ops.Ncols;
+  ops.wp = plan.tables.out; ops.steps = plan.tables.steps; ops.K = plan.K;
+  launch_igemm_mode<conv::ForwardOps, conv::kFp32>(ops, pieces, range, stream);
+  MOBULA_HIP_TRY(hipGetLastError());
+  return true;
+}
+
+// The gradients that are wanted (null: not).
+bool gradients_split(const conv::Geometry& g, const float* dy, const float* x, const float* weight, int accumulate,
+                     float* dx, float* dw, hipStream_t stream) {
+  BackwardB16<3> b;
+  GatherPlan plan{};
+  WeightPlan weight_plan{};
+  const long long taps = g.KH * g.KW;
+  if (b.plan(g, dy, x, weight, accumulate, dx, dw) != kFits) return false;
+  if (dx != nullptr && !plan_gather(&plan, "conv2d_backward_data", g, weight, g.C, g.D,
+                                    static_cast<long long>(g.D) * g.OH * g.OW, g.H * g.W, g.OW, -1, taps, g.C * taps))
+    return true;
+  if (dw != nullptr && !plan_weight(&weight_plan, g)) return true;
+  // (the fp32 weight gradient comes last: what it needs takes the place of the operands)
+  const size_t operands = b.prep.bytes + plan.bytes + (dx != nullptr && dw != nullptr ? 2 : 1) * kPieceBytes;
+  char* const ws = static_cast<char*>(
+      mobula_hip::workspace_if_possible(kWordBytes + std::max(operands, weight_plan.bytes)));
+  if (ws == nullptr) return failed();
+  unsigned* const words = reinterpret_cast<unsigned*>(ws);   // dy, weights, x
+  char* const tables = b.place(ws + kWordBytes);
+  const conv::SplitRange data_range{words, words + 1}, weight_range{words, words + 2};
+  conv::clear_words_kernel<<<1, 64, 0, stream>>>(words, 3);
+  b.prep.launch<3>(stream, conv::ExponentWords{words + 1, words, words + 2});
+  launch_gradients_b16<3>(b, tables + plan.bytes, stream, data_range, weight_range);
+  if (dx != nullptr) {
+    build_gather(&plan, tables, stream, data_range);
+    conv::BackwardDataOps ops;
+    ops.dy = dy; ops.dx = dx; ops.g = g; ops.accumulate = accumulate; ops.M = g.C; ops.Ncols = b.data.Ncols;
+    ops.wp = plan.tables.out; ops.steps = plan.tables.steps; ops.K = plan.K;
+    launch_igemm_mode<conv::BackwardDataOps, conv::kFp32>(ops, reinterpret_cast<float*>(tables + plan.bytes), data_range,
+                                                          stream);
+  }
+  if (dw != nullptr) run_weight(weight_plan, g, dy, x, accumulate, dw, ws + kWordBytes, stream, weight_range);
+  MOBULA_HIP_TRY(hipGetLastError());
+  return true;
+}
+
+SplitChoice choose_split(const conv::Geometry& g, bool dx, bool dw) {
+  if (split_choice() == 0 || g.N == 0 || g.N >= 65536) return SplitChoice{false, false};
+  if (split_choice() == 2) return SplitChoice{dx, dw};
+  // (what the fp32 ways take at most: most small layers end here)
+  const double most_dx = data_fp32_us(gathered_product_cost(g.C, g.D, g.KH * g.KW, static_cast<long long>(g.N) * g.H * g.W),
+                                      static_cast<size_t>(g.stride_h) * g.stride_w);
+  const double most_dw = weight_fp32_us(weight_gathered_cost(g));
+  dx = dx && most_dx > kSplitOverhead;
+  dw = dw && most_dw > kSplitOverhead + 10.0;
+  if (!dx && !dw) return SplitChoice{false, false};
+  BackwardB16<3> b;
+  float any;   // (for its address: nothing is written)
+  if (b.plan(g, &any, &any, &any, 0, dx ? &any : nullptr, dw ? &any : nullptr) != kFits) return SplitChoice{false, false};
+  const double dy_parts = parts_us(static_cast<long long>(g.N) * g.D * g.OH * g.OW);
+  const double x_parts = parts_us(static_cast<long long>(g.N) * g.C * g.H * g.W);
+  double data = 0.0, weight = 0.0, data_fp32 = 0.0, weight_fp32 = 0.0;
+  if (dx) {
+    rows_b16(b.data, &data);
+    const DataPatches patches = data_patches(g, nullptr, nullptr, nullptr, 0);
+    const size_t classes = data_patches_win(g, patches, &data_fp32) ? patches.classes.size() : 1;
+    data_fp32 = data_fp32_us(data_fp32, classes);
+  }
+  if (dw) {
+    rows_b16(b.weight, &weight);
+    weight_fp32 = weight_fp32_us(weight_fp32_cost(g));
+  }
+  const double only_dx = data + dy_parts + kSplitOverhead, only_dw = weight + dy_parts + x_parts + kSplitOverhead;
+  SplitChoice best{dx && only_dx < data_fp32, dw && only_dw < weight_fp32};
+  if (dx && dw) {   // the parts of dy are shared
+    const double both = data + weight + dy_parts + x_parts + 1.3 * kSplitOverhead, none = data_fp32 + weight_fp32;
+    const double one_dx = only_dx + weight_fp32, one_dw = only_dw + data_fp32;
+    best.dx = std::min(both, one_dx) < std::min(none, one_dw);
+    best.dw = std::min(both, one_dw) < std::min(none, one_dx);
+  }
+  return best;
+}
+
+// Both gradients in one go, sharing what prepares their operands; false: not taken, or only as far as *done says.
+bool both_gradients(const conv::Geometry& g, const float* dy, const float* x, const float* weight, float* dx, float* dw,
+                    SplitChoice* done) {
+  hipStream_t stream = call_state().stream;
+  if (compute_mode() == conv::kBf16) return gradients_b16<1>(g, dy, x, weight, 0, dx, dw, stream);
+  if (compute_mode() == conv::kBf16x3) return gradients_b16<2>(g, dy, x, weight, 0, dx, dw, stream);
+  const SplitChoice split = choose_split(g, true, true);
+  if ((split.dx || split.dw) &&
+      gradients_split(g, dy, x, weight, 0, split.dx ? dx : nullptr, split.dw ? dw : nullptr, stream))
+    *done = split;
+  return done->dx && done->dw;
+}
+
+// dx (+)= and dw (+)= as the launchers below say; allow_split: whether products of parts have yet to be weighed.
+void data_gradient(const conv::Geometry& g, const float* dy, const float* weight, int accumulate, float* dx,
+                   bool allow_split) {
+  if (static_cast<long long>(g.N) * g.C * g.H * g.W == 0) return;
+  hipStream_t stream = call_state().stream;
+  mobula_hip::KernelTimer timer("conv2d_backward_data", stream);
+  if (g.N < 65536) {
+    bool taken = false;
+    if (compute_mode() == conv::kBf16) taken = gradients_b16<1>(g, dy, nullptr, weight, accumulate, dx, nullptr, stream);
+    if (compute_mode() == conv::kBf16x3) taken = gradients_b16<2>(g, dy, nullptr, weight, accumulate, dx, nullptr, stream);
+    if (taken) return;
+  }
+  if (compute_mode() == conv::kFp32) {
+    if (allow_split && choose_split(g, true, false).dx &&
+        gradients_split(g, dy, nullptr, weight, accumulate, dx, nullptr, stream))
+      return;
+    const DataPatches patches = data_patches(g, dy, weight, dx, accumulate);
+    double cost = 0.0;
+    if (data_patches_win(g, patches, &cost)) {
+      run_data_patches(g, patches, dx, accumulate, stream);
+      return;
+    }
+  }
+  GatherPlan plan;
+  const long long taps = g.KH * g.KW;
+  // row m of the left operand is input channel m: element [m][tap][d] = weight[d][m][tap]
+  if (!plan_gather(&plan, "conv2d_backward_data", g, weight, g.C, g.D,
+                   static_cast<long long>(g.D) * g.OH * g.OW, g.H * g.W, g.OW, -1, taps, g.C * taps))
+    return;
+  char* const ws = static_cast<char*>(mobula_hip::workspace(plan.bytes + kPieceBytes));
+  if (failed()) return;
+  float* const pieces = reinterpret_cast<float*>(build_gather(&plan, ws, stream));
+  conv::BackwardDataOps ops;
+  ops.dy = dy; ops.dx = dx; ops.g = g; ops.accumulate = accumulate;
+  ops.M = g.C; ops.Ncols = g.N * g.H * g.W;
+  ops.wp = plan.tables.out; ops.steps = plan.tables.steps; ops.K = plan.K;
+  launch_igemm(ops, pieces, stream);
+  MOBULA_HIP_TRY(hipGetLastError());
+}
+
+void weight_gradient(const conv::Geometry& g, const float* dy, const float* x, int accumulate, float* dw,
+                     bool allow_split) {
+  const long long wt = static_cast<long long>(g.D) * g.C * g.KH * g.KW;
+  if (static_cast<long long>(g.C) * g.H * g.W * 4 >= (1ll << 31)) {
+    set_error("conv2d_backward_weight: images too large for 32-bit byte offsets");
+    return;
+  }
+  hipStream_t stream = call_state().stream;
+  mobula_hip::KernelTimer timer("conv2d_backward_weight", stream);
+  if (wt > 0) {
+    bool taken = false;
+    if (compute_mode() == conv::kBf16) taken = gradients_b16<1>(g, dy, x, nullptr, accumulate, nullptr, dw, stream);
+    if (compute_mode() == conv::kBf16x3) taken = gradients_b16<2>(g, dy, x, nullptr, accumulate, nullptr, dw, stream);
+    if (taken) return;
+  }
+  if (compute_mode() == conv::kFp32 && wt > 0) {
+    if (allow_split && choose_split(g, false, true).dw &&
+        gradients_split(g, dy, x, nullptr, accumulate, nullptr, dw, stream))
+      return;
+    if (weight_gradient_from_patches(g, dy, x, accumulate, dw, stream)) return;
+  }
+  WeightPlan plan;
+  if (!plan_weight(&plan, g)) return;
+  char* const ws = static_cast<char*>(mobula_hip::workspace(plan.bytes));
+  if (failed()) return;
+  run_weight(plan, g, dy, x, accumulate, dw, ws, stream);
+  MOBULA_HIP_TRY(hipGetLastError());
 }
 
 }  // namespace
@@ -796,41 +1203,37 @@ MOBULA_KERNEL conv2d_forward_kernel(const int n, const T* x, const T* weight, co
     return;
   if (out == 0) return;
   hipStream_t stream = call_state().stream;
+  if (!has_bias) bias = nullptr;
+  mobula_hip::KernelTimer timer("conv2d_forward", stream);
+  if (g.N < 65536) {
+    bool taken = false;
+    if (compute_mode() == conv::kBf16) taken = forward_b16<1>(g, x, weight, bias, y, stream);
+    if (compute_mode() == conv::kBf16x3) taken = forward_b16<2>(g, x, weight, bias, y, stream);
+    if (taken) return;
+  }   // (else the kernels below round or split fp32 operands themselves)
+  if (compute_mode() == conv::kFp32) {
+    const PatchProduct patches = forward_patches(g, x, weight, bias, y);
+    double cost = 0.0;
+    const bool from_patches = forward_patches_win(g, patches, &cost);
+    if (split_choice() != 0 && forward_split(g, x, weight, bias, y, cost, stream)) return;
+    if (from_patches) {
+      run_patch_product(patches, stream);
+      return;
+    }
+  }
+  GatherPlan plan;
+  const long long taps = g.KH * g.KW;
+  if (!plan_gather(&plan, "conv2d_forward", g, weight, g.D, g.C, static_cast<long long>(g.C) * g.H * g.W,
+                   g.OH * g.OW, g.W, +1, g.C * taps, taps))
+    return;
+  char* const ws = static_cast<char*>(mobula_hip::workspace(plan.bytes + kPieceBytes));
+  if (failed()) return;
+  float* const pieces = reinterpret_cast<float*>(build_gather(&plan, ws, stream));
   conv::ForwardOps ops;
-  ops.x = x; ops.bias = has_bias ? bias : nullptr; ops.y = y; ops.g = g;
+  ops.x = x; ops.bias = bias; ops.y = y; ops.g = g;
   ops.M = g.D; ops.Ncols = g.N * g.OH * g.OW;
-  if (bf16_mode() && g.N < 65536) {
-    // operands as bf16 in memory: channel-blocked copy of x, weights by K step (heads and tails
-    // of both with split operands)
-    conv::ForwardOpsB16 ob;
-    ob.bias = ops.bias; ob.y = y; ob.Ncols = ops.Ncols;
-    PrepB16 prep;
-    const long long taps = g.KH * g.KW;
-    const Fit fit = plan_gather_b16(&ob, &prep, "conv2d_forward", g, weight, g.D, g.C, x, g.N, g.H * g.W, g.OH * g.OW,
-                                    g.C * taps, taps, compute_mode() == conv::kBf16x3);
-    if (fit == kError) return;
-    if (fit == kFits) {
-      mobula_hip::KernelTimer timer("conv2d_forward", stream);
-      char* const ws = static_cast<char*>(mobula_hip::workspace(prep.bytes + kPieceBytes));
-      if (failed()) return;
-      char* const pieces = place_gather_b16(&ob, &prep, ws);
-      prep.launch(stream);
-      launch_igemm_b16(ob, reinterpret_cast<float*>(pieces), stream);
-      MOBULA_HIP_TRY(hipGetLastError());
-      return;
-    }   // (else the kernels below split fp32 operands themselves)
-  }
-  {
-    mobula_hip::KernelTimer timer("conv2d_forward", stream);
-    if (compute_mode() == conv::kFp32 && forward_from_patches(g, x, weight, ops.bias, y, stream)) return;
-    GatherPlan plan;
-    const long long taps = g.KH * g.KW;
-    if (!plan_gather(&plan, "conv2d_forward", g, weight, g.D, g.C, static_cast<long long>(g.C) * g.H * g.W,
-                     g.OH * g.OW, g.W, +1, g.C * taps, taps, stream))
-      return;
-    ops.wp = plan.weights; ops.steps = plan.steps; ops.K = plan.K;
-    launch_igemm(ops, plan.pieces, stream);
-  }
+  ops.wp = plan.tables.out; ops.steps = plan.tables.steps; ops.K = plan.K;
+  launch_igemm(ops, pieces, stream);
   MOBULA_HIP_TRY(hipGetLastError());
 }
 
@@ -853,40 +1256,7 @@ MOBULA_KERNEL conv2d_backward_data_kernel(const int n, const T* dy, const T* wei
       !fits("conv2d_backward_data", 2, static_cast<long long>(g.D) * g.C * g.KH * g.KW) ||
       !fits("conv2d_backward_data", 17, in))
     return;
-  if (in == 0) return;
-  hipStream_t stream = call_state().stream;
-  conv::BackwardDataOps ops;
-  ops.dy = dy; ops.dx = dx; ops.g = g; ops.accumulate = accumulate;
-  ops.M = g.C; ops.Ncols = g.N * g.H * g.W;
-  if (bf16_mode() && g.N < 65536) {
-    conv::BackwardDataOpsB16 ob;
-    PrepB16 prep;
-    const Fit fit = plan_data_b16(&ob, &prep, g, dy, weight, accumulate, dx);
-    if (fit == kError) return;
-    if (fit == kFits) {
-      mobula_hip::KernelTimer timer("conv2d_backward_data", stream);
-      char* const ws = static_cast<char*>(mobula_hip::workspace(prep.bytes + kPieceBytes));
-      if (failed()) return;
-      char* const pieces = place_gather_b16(&ob, &prep, ws);
-      prep.launch(stream);
-      launch_igemm_b16(ob, reinterpret_cast<float*>(pieces), stream);
-      MOBULA_HIP_TRY(hipGetLastError());
-      return;
-    }
-  }
-  {
-    mobula_hip::KernelTimer timer("conv2d_backward_data", stream);
-    if (compute_mode() == conv::kFp32 && data_gradient_from_patches(g, dy, weight, dx, accumulate, stream)) return;
-    GatherPlan plan;
-    const long long taps = g.KH * g.KW;
-    // row m of the left operand is input channel m: element [m][tap][d] = weight[d][m][tap]
-    if (!plan_gather(&plan, "conv2d_backward_data", g, weight, g.C, g.D,
-                     static_cast<long long>(g.D) * g.OH * g.OW, g.H * g.W, g.OW, -1, taps, g.C * taps, stream))
-      return;
-    ops.wp = plan.weights; ops.steps = plan.steps; ops.K = plan.K;
-    launch_igemm(ops, plan.pieces, stream);
-  }
-  MOBULA_HIP_TRY(hipGetLastError());
+  data_gradient(g, dy, weight, accumulate, dx, true);
 }
 
 // dw[D, C, KH, KW] (+)= the gradient with respect to the weights.  n is the
@@ -908,81 +1278,7 @@ MOBULA_KERNEL conv2d_backward_weight_kernel(const int n, const T* dy, const T* x
       !fits("conv2d_backward_weight", 2, static_cast<long long>(g.N) * g.C * g.H * g.W) ||
       !fits("conv2d_backward_weight", 17, wt))
     return;
-  if (static_cast<long long>(g.C) * g.H * g.W * 4 >= (1ll << 31)) {
-    set_error("conv2d_backward_weight: images too large for 32-bit byte offsets");
-    return;
-  }
-  hipStream_t stream = call_state().stream;
-  if (bf16_mode() && wt > 0) {
-    conv::WeightGradOpsB16 ob;
-    PrepB16 prep;
-    ob.dw = dw; ob.accumulate = accumulate;
-    if (plan_weight_b16(&ob, &prep, g, dy, x, compute_mode() == conv::kBf16x3) == kFits) {
-      mobula_hip::KernelTimer timer("conv2d_backward_weight", stream);
-      char* const ws = static_cast<char*>(mobula_hip::workspace(prep.bytes + kPieceBytes));
-      if (failed()) return;
-      char* const pieces = place_weight_b16(&ob, &prep, ws);
-      prep.launch(stream);
-      launch_igemm_b16(ob, reinterpret_cast<float*>(pieces), stream);
-      MOBULA_HIP_TRY(hipGetLastError());
-      return;
-    }
-  }
-  if (compute_mode() == conv::kFp32 && wt > 0) {
-    mobula_hip::KernelTimer timer("conv2d_backward_weight", stream);
-    if (weight_gradient_from_patches(g, dy, x, accumulate, dw, stream)) return;
-  }
-  conv::BackwardWeightOps ops;
-  ops.dy = dy; ops.x = x; ops.g = g;
-  ops.M = g.D; ops.Ncols = g.C * g.KH * g.KW; ops.K = 0; ops.k_begin = 0;
-  // K = N*OH*OW is long and the result small: K is cut into slices of whole K
-  // steps, as many as give every CU six workgroups; the partial sums of the
-  // slices are added in a fixed order afterwards.
-  const int row_tiles = (ops.M + conv::Tile::BM - 1) / conv::Tile::BM;
-  const long long per_slice_tiles = static_cast<long long>(row_tiles) * ((ops.Ncols + conv::Tile::BN - 1) / conv::Tile::BN);
-  const long long k_total = static_cast<long long>(g.N) * g.OH * g.OW;   // < 2^31: checked by describe()
-  if (per_slice_tiles >= (1ll << 20)) { set_error("conv2d_backward_weight: too many tiles"); return; }
-  const long long k_steps = std::max<long long>(1, (k_total + conv::Tile::BK - 1) / conv::Tile::BK);
-  long long slices = std::min<long long>(k_steps, std::max<long long>(1, kWeightSlots / per_slice_tiles));
-  const long long k_per_slice = (k_steps + slices - 1) / slices * conv::Tile::BK;
-  slices = std::max<long long>(1, (k_total + k_per_slice - 1) / k_per_slice);
-  // a zero-padded copy of x saves the gathered operand its range tests where eight output pixels
-  // of a row are eight neighbouring inputs (unit stride along a row); 32-bit offsets within an image
-  const int Hp = g.H + 2 * g.pad_h, Wp = g.W + 2 * g.pad_w;
-  const long long plane_p = static_cast<long long>(Hp) * Wp;
-  const bool padded = g.stride_w == 1 && g.N > 0 && plane_p * g.C * 4 < (1ll << 31) && plane_p < (1ll << 22);
-  const size_t partial_bytes = (sizeof(float) * static_cast<size_t>(slices) * wt + 255) / 256 * 256;
-  const size_t padded_bytes = padded ? sizeof(float) * static_cast<size_t>(g.N) * g.C * plane_p : 0;
-  char* extra = nullptr;
-  ops.taps = make_taps(ops.Ncols, g.KH, g.KW, padded ? static_cast<int>(plane_p) : g.H * g.W, g.dil_h, g.dil_w,
-                       partial_bytes + padded_bytes, &extra, stream);
-  if (failed()) return;
-  ops.partial = reinterpret_cast<float*>(extra);
-  ops.xp = nullptr; ops.Hp = Hp; ops.Wp = Wp;
-  {
-    mobula_hip::KernelTimer timer("conv2d_backward_weight", stream);
-    if (padded) {
-      float* const xp = reinterpret_cast<float*>(extra + partial_bytes);
-      conv::pad_planes_kernel<<<dim3(g.N * g.C, static_cast<unsigned>((plane_p + 2047) / 2048)), 256, 0, stream>>>(
-          x, xp, g.H, g.W, g.pad_h, g.pad_w, Hp, Wp);
-      ops.xp = xp;
-    }
-    const int tps = static_cast<int>(per_slice_tiles), count = tps * static_cast<int>(slices);
-    const dim3 grid(conv::tile_blocks(count));
-    switch (compute_mode()) {
-      case conv::kBf16:
-        conv::igemm_weight_kernel<conv::kBf16><<<grid, conv::Tile::NT, 0, stream>>>(
-            ops, static_cast<int>(k_per_slice), static_cast<int>(k_total), row_tiles, tps, count); break;
-      case conv::kBf16x3:
-        conv::igemm_weight_kernel<conv::kBf16x3><<<grid, conv::Tile::NT, 0, stream>>>(
-            ops, static_cast<int>(k_per_slice), static_cast<int>(k_total), row_tiles, tps, count); break;
-      default:
-        conv::igemm_weight_kernel<conv::kFp32><<<grid, conv::Tile::NT, 0, stream>>>(
-            ops, static_cast<int>(k_per_slice), static_cast<int>(k_total), row_tiles, tps, count);
-    }
-    reduce_slices(ops.partial, dw, wt, static_cast<int>(slices), accumulate, stream);
-  }
-  MOBULA_HIP_TRY(hipGetLastError());
+  weight_gradient(g, dy, x, accumulate, dw, true);
 }
 
 // db[D] (+)= sum of dy over images and pixels.  n = D.
@@ -1017,29 +1313,6 @@ MOBULA_KERNEL conv2d_backward_bias_kernel(const int n, const T* dy, const int ac
 // buffers (device id -1 is an error here).
 // ---------------------------------------------------------------------------
 namespace {
-// True if the gradients were taken here (or the call has failed).
-bool both_gradients_b16(const conv::Geometry& g, const float* dy, const float* x, const float* weight, float* dx,
-                        float* dw) {
-  if (!bf16_mode() || g.N == 0 || g.N >= 65536) return false;
-  conv::BackwardDataOpsB16 data;
-  conv::WeightGradOpsB16 wgrad;
-  PrepB16 prep;
-  wgrad.dw = dw; wgrad.accumulate = 0;
-  if (plan_weight_b16(&wgrad, &prep, g, dy, x, compute_mode() == conv::kBf16x3) != kFits) return false;
-  const Fit fit = plan_data_b16(&data, &prep, g, dy, weight, 0, dx);
-  if (fit != kFits) return fit == kError;
-  hipStream_t stream = call_state().stream;
-  // (both products' operands at a time; where there is no room for that, one product after the other)
-  char* const ws = static_cast<char*>(mobula_hip::workspace_if_possible(prep.bytes + kPieceBytes));
-  if (ws == nullptr) return failed();
-  float* const pieces = reinterpret_cast<float*>(place_weight_b16(&wgrad, &prep, place_gather_b16(&data, &prep, ws)));
-  prep.launch(stream);
-  launch_igemm_b16(data, pieces, stream);
-  launch_igemm_b16(wgrad, pieces, stream);
-  MOBULA_HIP_TRY(hipGetLastError());
-  return true;
-}
-
 bool on_device(const char* what, int device_id) {
   mobula_hip::begin_call();
   if (device_id >= 0) return true;
@@ -1114,13 +1387,16 @@ void mobula_hip_conv2d_backward(const int device_id, const float* dy, const floa
   if (!on_device("conv2d_backward", device_id)) return;
   mobula_hip::DeviceScope scope(device_id);
   conv::Geometry g;
+  SplitChoice done{false, false};
   if (scope.ok() && describe(&g, "conv2d_backward", CONV_GEOMETRY_ARGS) &&
-      !(dx != nullptr && dw != nullptr && both_gradients_b16(g, dy, x, weight, dx, dw)) && !failed()) {
-    call_state().extents.clear();
-    if (dx != nullptr)
-      conv2d_backward_data_kernel<float>(g.N * g.C * g.H * g.W, dy, weight, 0, CONV_GEOMETRY_ARGS, dx);
-    if (dw != nullptr && !failed())
-      conv2d_backward_weight_kernel<float>(g.D * g.C * g.KH * g.KW, dy, x, 0, CONV_GEOMETRY_ARGS, dw);
+      !(dx != nullptr && dw != nullptr && g.N > 0 && g.N < 65536 && both_gradients(g, dy, x, weight, dx, dw, &done)) &&
+      !failed()) {
+    // (what was weighed for both together is not weighed again)
+    const bool weighed = dx != nullptr && dw != nullptr && compute_mode() == conv::kFp32;
+    if (dx != nullptr && !done.dx)
+      data_gradient(g, dy, weight, 0, dx, !weighed);
+    if (dw != nullptr && !done.dw && !failed())
+      weight_gradient(g, dy, x, 0, dw, !weighed);
   }
   mobula_hip::finish_call();
 }

@@ -623,3 +623,91 @@ def test_an_infinity_stays_an_infinity_in_fp32_products(shape):
         dyd = dyi.cuda()
         _call('conv2d_backward_data_ecf81c91', ctypes.c_int(dx.numel()), _ptr(dyd), _ptr(wd), ctypes.c_int(0), *geo, _ptr(dx))
         check(dx, dx_ref, 'dx')
+
+
+@pytest.fixture
+def split_always():
+    native.set_option('conv_fp32_split', 2)
+    yield
+    native.set_option('conv_fp32_split', 1)
+
+
+def _three_products(geo, x, w, dy, dx0=None, dw0=None):
+    """y, dx, dw through the C-ABI; dx0, dw0: added to."""
+    y = torch.full(dy.shape, float('nan'), device='cuda')
+    dx = torch.full(x.shape, float('nan'), device='cuda') if dx0 is None else dx0.clone()
+    dw = torch.full(w.shape, float('nan'), device='cuda') if dw0 is None else dw0.clone()
+    _call('conv2d_forward_c6a7aa85', ctypes.c_int(y.numel()), _ptr(x), _ptr(w), _ptr(w), ctypes.c_int(0), *geo, _ptr(y))
+    _call('conv2d_backward_data_ecf81c91', ctypes.c_int(dx.numel()), _ptr(dy), _ptr(w), ctypes.c_int(dx0 is not None), *geo,
+          _ptr(dx))
+    _call('conv2d_backward_weight_ecf81c91', ctypes.c_int(dw.numel()), _ptr(dy), _ptr(x), ctypes.c_int(dw0 is not None), *geo,
+          _ptr(dw))
+    return y, dx, dw
+
+
+@pytest.mark.parametrize('shape', [
+    # N, C, H, W, D, kernel, pad, stride, dilation
+    (1, 1, 1, 1, 1, (1, 1), (0, 0), (1, 1), (1, 1)),         # one multiply-add
+    (3, 16, 5, 3, 64, (1, 1), (0, 0), (1, 1), (1, 1)),       # 15 pixels an image: a step of K meets two and three images
+    (40, 17, 2, 2, 65, (2, 2), (1, 1), (1, 1), (1, 1)),      # 9 pixels, rows and channels one past a tile and a block
+    (2, 15, 16, 16, 128, (3, 3), (1, 1), (1, 1), (1, 1)),    # whole steps of pixels and rows of two workgroups' tiles
+    (2, 33, 19, 21, 193, (3, 2), (2, 0), (1, 1), (1, 1)),    # odd planes: the element-wise conversion
+    (4, 64, 24, 28, 256, (3, 3), (1, 1), (1, 1), (1, 1)),    # columns in whole tiles, rows too
+    (3, 48, 23, 17, 257, (3, 3), (0, 1), (2, 2), (1, 1)),    # strides: taps that reach no pixel
+    (2, 24, 30, 22, 40, (3, 2), (2, 1), (2, 1), (1, 2)),     # strides and dilation
+    (5, 20, 7, 9, 130, (5, 5), (6, 2), (1, 3), (1, 1)),      # padding beyond the kernel
+])
+def test_fp32_products_of_three_parts(shape, split_always):
+    """fp32 products from three bf16 parts per operand: exact products but for 2^-26 of them, and at most six fp32
+    roundings for sixteen of K, each of 2^-24 of a sum no larger than the result's own scale."""
+    N, C, H, W, D, kernel, pad, stride, dil = shape
+    g = torch.Generator().manual_seed(91)
+    x, w = torch.randn(N, C, H, W, generator=g), torch.randn(D, C, *kernel, generator=g)
+    xr, wr = x.double().requires_grad_(True), w.double().requires_grad_(True)
+    y_ref = F.conv2d(xr, wr, None, stride=stride, padding=pad, dilation=dil)
+    dy = torch.randn(y_ref.shape, generator=g)
+    y_ref.backward(dy.double())
+    geo = _ci(N, C, H, W, D, kernel[0], kernel[1], pad[0], pad[1], stride[0], stride[1], dil[0], dil[1])
+    _leave_nan_patterns_in_the_workspace()
+    xd, wd, dyd = x.cuda(), w.cuda(), dy.cuda()
+    got = _three_products(geo, xd, wd, dyd)
+    terms = C * kernel[0] * kernel[1], D * kernel[0] * kernel[1], dy[:, 0].numel()
+    for a, b, k, what in zip(got, (y_ref.detach(), xr.grad, wr.grad), terms, ('y', 'dx', 'dw')):
+        error = ((a.cpu().double() - b).norm() / b.norm()).item()
+        assert error <= 2.0 ** -24 * (1 + (6 * (k / 16 + 1)) ** 0.5), (what, error)
+    # added to what is there; the same bits a second time
+    start = torch.randn(x.shape, generator=g).cuda(), torch.randn(w.shape, generator=g).cuda()
+    again = _three_products(geo, xd, wd, dyd, *start)
+    assert torch.equal(again[0], got[0])
+    assert torch.equal(again[1], start[0] + got[1]) and torch.equal(again[2], start[1] + got[2])
+
+
+@pytest.mark.parametrize('scale_x,scale_w,odd', [
+    (1.0, 1.0, float('inf')), (1.0, 1.0, -float('inf')), (1.0, 1.0, float('nan')),
+    (1.0, 1.0, 3e38), (1.0, 1.0, 1e-40), (1.0, 1.0, 2.0 ** -110),
+    (2.0 ** -60, 2.0 ** -60, None),     # every operand in range, the products' last parts not
+    (2.0 ** 60, 2.0 ** 55, None), (2.0 ** -96, 2.0 ** 40, None), (0.0, 1.0, None),
+])
+def test_values_that_three_parts_do_not_stand_for(scale_x, scale_w, odd, split_always):
+    """Operands outside the range of the parts are multiplied by the fp32 kernels: the results are those that the option
+    gives without parts, which in these sizes take the same kernels."""
+    N, C, H, W, D = 2, 64, 24, 28, 128
+    geo = _ci(N, C, H, W, D, 3, 3, 1, 1, 1, 1, 1, 1)
+    g = torch.Generator(device='cuda').manual_seed(92)
+    x = torch.randn(N, C, H, W, generator=g, device='cuda') * scale_x
+    w = torch.randn(D, C, 3, 3, generator=g, device='cuda') * scale_w
+    dy = torch.randn(N, D, H, W, generator=g, device='cuda') * scale_x
+    if odd is not None:
+        x[1, 3, 5, 7] = odd
+        dy[0, 9, 20, 1] = odd
+    got = _three_products(geo, x, w, dy)
+    native.set_option('conv_fp32_split', 0)
+    want = _three_products(geo, x, w, dy)
+    for a, b, what in zip(got, want, ('y', 'dx', 'dw')):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf()), what
+        fine = b.isfinite()
+        if fine.any() and b[fine].abs().max() > 0:
+            scale = b[fine].double().norm()
+            assert ((a[fine].double() - b[fine].double()).norm() / scale).item() <= 2e-6, what
+        else:
+            assert torch.equal(a[fine], b[fine]), what
