@@ -28,6 +28,7 @@ struct FwdBlocked {
   static constexpr int PWB = 8;        // pooled columns per step (one per group of 8 lanes)
   static constexpr int CELL = 32;      // side of the sorting cells in pixels
   static constexpr int MAXCELLS = 8192;
+  static constexpr int CLASSES = 4;    // of boxes by their work, adaptive grids (roi_order_body)
 };
 
 // Per element type: channels per lane (16 bytes), channels per block of the
@@ -63,8 +64,8 @@ struct OrderArgs {
 
 template <int NT, int MAXC>
 __device__ __forceinline__ void roi_order_body(int* hist, int* wave_sum, int* carry, const float* __restrict__ rois,
-                                               int R, float scale, int H, int W, long long num_images,
-                                               int* __restrict__ order);
+                                               int R, float scale, int H, int W, long long num_images, int PH, int PW,
+                                               int S, int* __restrict__ order);
 
 // True if no sample of any ROI can touch the pixels p0 .. p0 + 63 of image n (asked by a whole workgroup
 // of 256 threads, each looks at every 256th ROI).  A box's pixels lie between the cells of its two
@@ -160,7 +161,7 @@ transpose_to_blocked_kernel(const T* __restrict__ in, T* __restrict__ out, int C
         constexpr int WORDS = static_cast<int>(sizeof(tile) / 4), MAXC = WORDS - 24;
         int* const words = reinterpret_cast<int*>(&tile[0][0]);
         roi_order_body<256, MAXC>(words, words + MAXC + 1, words + MAXC + 20, oa.rois, oa.R, oa.scale, oa.H, oa.W,
-                                  oa.num_images, oa.order);
+                                  oa.num_images, oa.PH, oa.PW, oa.S, oa.order);
       }
       return;
     }
@@ -183,26 +184,36 @@ transpose_to_blocked_kernel(const T* __restrict__ in, T* __restrict__ out, int C
 
 // order[] = ROI indices sorted by (image, 32x32-pixel cell of the box centre,
 // rows of cells walked in alternating direction): consecutive wavefronts then
-// read neighbouring parts of the map.  One workgroup; counting sort with the
+// read neighbouring parts of the map.  With an adaptive grid a box of large bins takes many times as long as a
+// small one, and one that starts last keeps the device waiting: boxes are then sorted by classes of work first, the
+// longest in front (6000 boxes, 7 x 7, on 100 x 100: 2.8 of four wavefronts a SIMD in flight on average, then 3.5;
+// 580 -> 526 us).  One workgroup; counting sort with the
 // histogram in LDS.  ROIs that name no image sort last.
 // (the body: NT threads of one workgroup, at most MAXC cells; hist holds MAXC + 1 counters)
 template <int NT, int MAXC>
 __device__ __forceinline__ void roi_order_body(int* hist, int* wave_sum, int* carry, const float* __restrict__ rois,
-                                               int R, float scale, int H, int W, long long num_images,
-                                               int* __restrict__ order) {
+                                               int R, float scale, int H, int W, long long num_images, int PH, int PW,
+                                               int S, int* __restrict__ order) {
   using K = FwdBlocked;
+  const int classes = S <= 0 ? K::CLASSES : 1;
   int cell = K::CELL;
   long long cy = (H + cell - 1) / cell, cx = (W + cell - 1) / cell;
-  while (cy * cx * num_images > MAXC && cell < (1 << 20)) {
+  while (classes * cy * cx * num_images > MAXC && cell < (1 << 20)) {
     cell *= 2;
     cy = (H + cell - 1) / cell; cx = (W + cell - 1) / cell;
   }
-  const int cells = cy * cx * num_images > MAXC ? 1 : static_cast<int>(cy * cx * num_images);
-  auto key_of = [&](int r) {
-    const float* q = rois + static_cast<long long>(r) * 5;
-    const int b = static_cast<int>(q[0]);
+  const int cells = classes * cy * cx * num_images > MAXC ? 1 : static_cast<int>(classes * cy * cx * num_images);
+  struct Box { float v[5]; };
+  auto key_of = [&](const Box& box) {
+    const float* const q = box.v;
+    int b = static_cast<int>(q[0]);
     if (b < 0 || b >= num_images) return cells;
     if (cells == 1) return 0;
+    if (classes > 1) {   // pixels of a bin, its border included
+      const float work = ((q[4] - q[2]) * scale / static_cast<float>(PH) + 2.0f) *
+                         ((q[3] - q[1]) * scale / static_cast<float>(PW) + 2.0f);
+      b += static_cast<int>(num_images) * (work >= 128.0f ? 0 : work >= 64.0f ? 1 : work >= 32.0f ? 2 : 3);
+    }
     const float mx = 0.5f * (q[1] + q[3]) * scale, my = 0.5f * (q[2] + q[4]) * scale;
     const int ix = min(max(static_cast<int>(mx), 0), W - 1) / cell;
     const int iy = min(max(static_cast<int>(my), 0), H - 1) / cell;
@@ -212,7 +223,21 @@ __device__ __forceinline__ void roi_order_body(int* hist, int* wave_sum, int* ca
   for (int i = threadIdx.x; i <= cells; i += NT) hist[i] = 0;
   if (threadIdx.x == 0) *carry = 0;
   __syncthreads();
-  for (int r = threadIdx.x; r < R; r += NT) atomicAdd(&hist[key_of(r)], 1);
+  // (Eight boxes of a thread at a time, all of their loads first: beside a copy that saturates the memory a load takes
+  // microseconds.  6000 boxes: 46 us until they are sorted, 27 where the loads overlap.)
+  auto every_box = [&](auto use) {
+    for (int r0 = threadIdx.x; r0 < R; r0 += 8 * NT) {
+      Box box[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+#pragma unroll
+        for (int i = 0; i < 5; ++i) box[k].v[i] = rois[static_cast<long long>(min(r0 + k * NT, R - 1)) * 5 + i];
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        if (r0 + k * NT < R) use(r0 + k * NT, key_of(box[k]));
+    }
+  };
+  every_box([&](int, int key) { atomicAdd(&hist[key], 1); });
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int base = 0; base <= cells; base += NT) {
@@ -232,16 +257,17 @@ __device__ __forceinline__ void roi_order_body(int* hist, int* wave_sum, int* ca
     if (threadIdx.x == NT - 1) *carry = before + incl;
     __syncthreads();
   }
-  for (int r = threadIdx.x; r < R; r += NT) order[atomicAdd(&hist[key_of(r)], 1)] = r;
+  every_box([&](int r, int key) { order[atomicAdd(&hist[key], 1)] = r; });
 }
 
 __global__ void __launch_bounds__(1024)
 roi_order_kernel(const float* __restrict__ rois, int R, float scale, int H, int W,
-                 long long num_images, int* __restrict__ order) {
+                 long long num_images, int PH, int PW, int S, int* __restrict__ order) {
   __shared__ int hist[FwdBlocked::MAXCELLS + 1];
   __shared__ int wave_sum[16];
   __shared__ int carry;
-  roi_order_body<1024, FwdBlocked::MAXCELLS>(hist, wave_sum, &carry, rois, R, scale, H, W, num_images, order);
+  roi_order_body<1024, FwdBlocked::MAXCELLS>(hist, wave_sum, &carry, rois, R, scale, H, W, num_images, PH, PW, S,
+                                                   order);
 }
 
 // A row sample: byte offsets of its low and high row in a channel block's
@@ -291,6 +317,50 @@ inline long long blocked_grid_nhwc(long long R, int cblk, int nw = FwdBlocked::N
 inline int forward_row_parts(long long R, int cblk, int PH, bool merged) {
   const long long jobs = R * cblk, wanted = merged ? 8192 : 4096;
   return jobs <= 0 ? 1 : static_cast<int>(std::min<long long>(PH, std::max<long long>(1, wanted / jobs)));
+}
+
+// Some pooled rows of every channel leave LDS: `seg` contiguous elements per channel, `pitch` apart there and
+// `bins` apart in y, whose element `dst` is the first.  Lanes take pieces of WIDTH elements, one division a lane.
+template <typename T, int WIDTH>
+__device__ __forceinline__ void store_pooled_rows(T* __restrict__ dst, const T* stage, int lane, int nch, int seg,
+                                                  int pitch, int bins) {
+  struct alignas(WIDTH * sizeof(T)) Piece { T v[WIDTH]; };
+  const int pieces = seg / WIDTH;   // of a channel
+  if (pieces <= 64) {
+    // as many channels at a time as the lanes cover
+    const int chans = 64 / pieces, cl = lane / pieces, j = (lane - cl * pieces) * WIDTH;
+    if (cl < chans) {
+      // (the same base for every lane: scalar registers; 32-bit offsets per lane)
+      int to = cl * bins + j, from = cl * pitch + j;
+#pragma nounroll
+      for (int c = cl; c < nch; c += chans, to += chans * bins, from += chans * pitch)
+        *reinterpret_cast<Piece*>(dst + to) = *reinterpret_cast<const Piece*>(stage + from);
+    }
+  } else {
+    for (int c = 0; c < nch; ++c)
+      for (int i = lane; i < pieces; i += 64)
+        reinterpret_cast<Piece*>(dst + static_cast<size_t>(c) * bins)[i] =
+            reinterpret_cast<const Piece*>(stage + c * pitch)[i];
+  }
+}
+
+// The same with the widest pieces that the places allow: channels and rows that start at multiples of four
+// elements (14 x 14 and 28 x 28 pooled maps) go 16 bytes a lane, a quarter of the instructions (8192 boxes of 256
+// channels, 14 x 14: 840 -> 820 us; straight from the lanes, 32 bytes at a time, 1262).
+template <typename T>
+__device__ __forceinline__ void store_pooled_rows(T* __restrict__ dst, const T* stage, int lane, int nch, int seg,
+                                                  int pitch, int bins) {
+  const bool fours = ((seg | pitch | bins) & 3) == 0 && reinterpret_cast<size_t>(dst) % (4 * sizeof(T)) == 0;
+  if (fours) store_pooled_rows<T, 4>(dst, stage, lane, nch, seg, pitch, bins);
+  else store_pooled_rows<T, 1>(dst, stage, lane, nch, seg, pitch, bins);
+}
+
+// Elements between the channels of a wavefront's staged rows: four more than they are where those fit, else
+// the eight channel quads of 56 elements each lie in two banks.
+template <typename T>
+__device__ __forceinline__ int staged_pitch(int rows_per_pass, int PH, int PW, int stage) {
+  const int seg = rows_per_pass * PW;
+  return rows_per_pass < PH && BlockOf<T>::CB * (seg + 4) <= stage ? seg + 4 : seg;
 }
 
 template <typename T, bool NHWC>
@@ -408,8 +478,9 @@ forward_blocked_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
     }
   };
 
+  const int staged = staged_pitch<T>(rows_per_pass, PH, PW, STAGE);
   for (int ph0 = ph_first; ph0 < ph_end; ph0 += rows_per_pass) {
-    const int rp = min(rows_per_pass, ph_end - ph0), seg = rp * PW;
+    const int rp = min(rows_per_pass, ph_end - ph0), seg = rp * PW, pitch = rp == PH ? seg : staged;
     for (int pwb = 0; pwb < PW; pwb += K::PWB) {
       const int pw = pwb + grp;
       const bool bin_on = pw < PW && quad_on;
@@ -566,7 +637,7 @@ forward_blocked_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
           } else if (bin_on) {
 #pragma unroll
             for (int i = 0; i < CPL; ++i)
-              stage[(CPL * quad + i) * seg + (ph - ph0) * PW + pw] = from_float<T>(acc[i]);
+              stage[(CPL * quad + i) * pitch + (ph - ph0) * PW + pw] = from_float<T>(acc[i]);
           }
         }
       };
@@ -593,22 +664,7 @@ forward_blocked_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
         for (int i = lane_now; i < total; i += 64) dst[i] = stage[i];
       }
     } else {
-      // some pooled rows of every channel: seg contiguous elements per channel, the lanes cover
-      // as many channels at a time as fit (one division per pass, none per element)
-      const int chans = max(1, 64 / seg), cl = lane_now / seg, j0 = lane_now - cl * seg;
-      if (seg <= 64) {
-        if (cl < chans) {
-          // (the same base for every lane: scalar registers; 32-bit offsets per lane)
-          T* const base = y + (static_cast<size_t>(roi) * C + c0) * bins + ph0 * PW;
-          int to = cl * bins + j0, from = cl * seg + j0;
-#pragma nounroll
-          for (int c = cl; c < nch; c += chans, to += chans * bins, from += chans * seg) base[to] = stage[from];
-        }
-      } else {
-        for (int c = 0; c < nch; ++c)
-          for (int j = lane_now; j < seg; j += 64)
-            y[(static_cast<size_t>(roi) * C + c0 + c) * bins + ph0 * PW + j] = stage[c * seg + j];
-      }
+      store_pooled_rows<T>(y + (static_cast<size_t>(roi) * C + c0) * bins + ph0 * PW, stage, lane_now, nch, seg, pitch, bins);
     }
   }
 }

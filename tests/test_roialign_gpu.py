@@ -1086,6 +1086,29 @@ def test_few_boxes_share_their_pooled_rows_among_wavefronts(R, C, pooled, S):
     assert_parity(y16.astype(np.float32), want.astype(np.float32), FP16_TOL, 'fp16')
 
 
+@pytest.mark.parametrize('pooled', [(7, 7), (3, 9), (12, 5), (14, 14)])
+@pytest.mark.parametrize('dtype,C', [(np.float32, 36), (np.float16, 72)])
+def test_adaptive_grids_at_the_edges_of_the_lists(dtype, C, pooled):
+    """Bins of one to 17 pixels an axis: merged lists of 14 samples and one more, more pooled rows and columns than are
+    listed at a time, rows staged in several passes; enough boxes for all of their pooled rows to stay with
+    one wavefront, on a map that is read in order of work and place."""
+    abi.set_impl('auto')
+    rng = np.random.default_rng(C + pooled[1])
+    N, H, W = 2, 17 * pooled[0] + 2, 17 * pooled[1] + 2
+    N += (24 << 20) // (N * H * W * 128) if pooled == (7, 7) else 0
+    bins = np.array([[h, w] for h in (1, 4, 5, 13.5, 14, 14.25, 17) for w in (0.5, 4, 8, 9, 13.75, 14, 15, 17)])
+    at = rng.uniform(-3, 3, bins.shape)
+    rois = np.stack([rng.integers(0, N, len(bins)), at[:, 0], at[:, 1], at[:, 0] + bins[:, 1] * pooled[1],
+                     at[:, 1] + bins[:, 0] * pooled[0]], 1).astype(np.float32)
+    x = rng.standard_normal((N, C, H, W)).astype(dtype)
+    want = oracle.forward(x.astype(np.float32), rois, pooled, 1.0, 0).astype(dtype).astype(np.float32)
+    tol = FWD_TOL if dtype == np.float32 else FP16_TOL
+    many = np.tile(rois, (80 if pooled == (7, 7) else 1, 1))
+    y = abi.forward(abi.to_dev(x), abi.to_dev(many), pooled, 1.0, 0)
+    for part in (y[:len(rois)], y[-len(rois):]):
+        assert_parity(part.float().cpu().numpy(), want, tol, 'y')
+
+
 @pytest.mark.parametrize('W', [200, 203])
 @pytest.mark.parametrize('dtype', [np.float32, np.float16])
 def test_few_boxes_on_a_large_map_copy_only_what_they_touch(W, dtype):
