@@ -200,7 +200,8 @@ __device__ __forceinline__ float lane_value(const unsigned __attribute__((ext_ve
 template <bool NHWC, typename TO, int TW, int NSPLIT = 1, bool WIN = false>
 __global__ void __launch_bounds__(BwdBlocked::NT * NSPLIT)
 backward_blocked_kernel(const void* __restrict__ dy_any, TO* __restrict__ dx_any,
-                        const WorkRange* __restrict__ ranges, const WorkEntry* __restrict__ entries,
+                        const WorkRange* __restrict__ ranges, const SortedRow* __restrict__ sorted,
+                        const int* __restrict__ class_counts, const WorkEntry* __restrict__ entries,
                         const AxisUnit* __restrict__ lists, TileGrid tg, ListLayout ll, int C, int H,
                         int W, int PH, int PW, int cblk, unsigned dyb_bytes, unsigned list_bytes,
                         int assign) {   // assign: bit 0 = overwrite dx (else add to it), bit 1 = rows may be written four columns at a time
@@ -228,9 +229,19 @@ backward_blocked_kernel(const void* __restrict__ dy_any, TO* __restrict__ dx_any
     const int part = xcd / cblk;
     const long long range = (tg.total * K::BANDS + parts - 1) / parts;
     if (part >= parts || wi >= range) return;
-    tile = part * range + wi;
+    tile = sorted != nullptr ? wi * parts + part : part * range + wi;
   }
   if (tile >= tg.total * K::BANDS) return;
+  static_assert(K::TH == 1 && K::BANDS == kTileRows, "a band is a tile row");
+  WorkRange wr;
+  if (sorted != nullptr) {   // the longest lists first (many boxes to a pixel)
+    const SortedRow r = sorted_row(sorted, class_counts, tg.total * kTileRows, tile);
+    if (r.row < 0) return;
+    tile = __builtin_amdgcn_readfirstlane(r.row);
+    wr = WorkRange{__builtin_amdgcn_readfirstlane(r.begin), __builtin_amdgcn_readfirstlane(r.count)};
+  } else {
+    wr = ranges[tile];
+  }
   const int band = static_cast<int>(tile % K::BANDS);
   tile /= K::BANDS;
   const int n = static_cast<int>(tile / tg.per_image);
@@ -249,7 +260,6 @@ backward_blocked_kernel(const void* __restrict__ dy_any, TO* __restrict__ dx_any
   for (int i = lane; i < RS * K::CS / 4; i += 64)
     reinterpret_cast<float4*>(row)[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 
-  const WorkRange wr = ranges[tile * kTileRows + band * K::TH + wave];
   const int n_entries = wr.count;   // a multiple of 2 * G, and G more entries follow: the lists are padded
   const int16v* const wl = reinterpret_cast<const int16v*>(entries + wr.begin);
   // this part's share: the items that start in [first_entry, end_entry), whole groups of 2 * G entries

@@ -291,6 +291,7 @@ __device__ __forceinline__ AxisUnit clip_unit(int bin, const AxisSample& a, int 
 // The wavefront also finds the ROI's box (the pixels any valid sample touches),
 // and stores it as tile ranges for build_tile_work_kernel.
 // `block`: index among the workgroups (of 256 threads) that build lists.
+constexpr int kWorkClasses = 8;   // of tile rows by the length of their work lists (SortedRow)
 struct ListsArgs {
   const float* rois;
   int items, R;
@@ -315,8 +316,8 @@ __device__ __forceinline__ void build_lists_body(unsigned block, const ListsArgs
   TileBox* __restrict__ boxes = a.boxes;
   int* __restrict__ cursors = a.cursors;
   AxisUnit* __restrict__ lists = a.lists;
-  // the two bump pointers of build_tile_work_kernel, which runs after this one
-  if (block == 0 && threadIdx.x < 2) cursors[threadIdx.x] = 0;
+  // the counters of build_tile_work_kernel, which runs after this one
+  if (block == 0 && threadIdx.x < 2 + kWorkClasses) cursors[threadIdx.x] = 0;
   const int item = static_cast<int>((block * 256u + threadIdx.x) >> 6);
   if (item >= items) return;
   const int lane = threadIdx.x & 63;
@@ -463,7 +464,7 @@ __device__ __forceinline__ void build_window_lists_body(unsigned block, const Li
   const int items = a.items, R = a.R, PH = a.PH, PW = a.PW, H = a.H, W = a.W;
   const TileGrid tg = a.tg;
   const ListLayout ll = a.ll;
-  if (block == 0 && threadIdx.x < 2) a.cursors[threadIdx.x] = 0;
+  if (block == 0 && threadIdx.x < 2 + kWorkClasses) a.cursors[threadIdx.x] = 0;
   const int item = static_cast<int>((block * 256u + threadIdx.x) >> 6);
   if (item >= items) return;
   const int lane = threadIdx.x & 63;
@@ -592,6 +593,25 @@ struct alignas(16) WorkEntry {
 };
 struct WorkRange { int begin; int count; };
 
+// The tile rows sorted by the length of their work lists, the longest first: classes a factor sqrt(2) apart, from
+// 256 entries down to 32.  Rows differ by three to ten times (boxes cluster), and one that starts last keeps the device
+// waiting.  A class is an array of its own; its rows stand in the order in which they were found.
+struct alignas(16) SortedRow { int row, begin, count, unused; };   // row: tile * kTileRows + row of the tile
+__device__ __forceinline__ int work_class(int count) {
+  return min(max(static_cast<int>(2.0f * (8.0f - __log2f(static_cast<float>(max(count, 1))))), 0), kWorkClasses - 1);
+}
+// Row `at` of all in that order (row < 0: there are no more).  counts: rows of each class.
+__device__ __forceinline__ SortedRow sorted_row(const SortedRow* __restrict__ sorted, const int* __restrict__ counts,
+                                                long long capacity, long long at) {
+#pragma unroll
+  for (int c = 0; c < kWorkClasses; ++c) {
+    const int n = counts[c];
+    if (at < n) return sorted[c * capacity + at];
+    at -= n;
+  }
+  return SortedRow{-1, 0, 0, 0};
+}
+
 // One workgroup per tile, one wavefront per tile row.
 // First the tile's ROI list: every wavefront takes a sixteenth of the ROIs,
 // counts those whose box covers the tile, and after one exchange writes them,
@@ -610,7 +630,7 @@ __global__ void __launch_bounds__(kTileRows * 64)
 build_tile_work_kernel(const TileBox* __restrict__ boxes, int R, int* __restrict__ tile_rois,
                        const AxisUnit* __restrict__ lists, TileGrid tg, ListLayout ll,
                        int* __restrict__ cursors, WorkRange* __restrict__ ranges,
-                       WorkEntry* __restrict__ entries) {
+                       WorkEntry* __restrict__ entries, SortedRow* __restrict__ sorted, int H) {
   __shared__ int hits[kTileRows];
   __shared__ int row_total[kTileRows];
   __shared__ int list_base, tile_base;
@@ -729,7 +749,14 @@ build_tile_work_kernel(const TileBox* __restrict__ boxes, int R, int* __restrict
   __syncthreads();
   int out = tile_base;
   for (int r = 0; r < row; ++r) out += row_total[r];
-  if (lane == 0) ranges[tile * kTileRows + row] = WorkRange{out, padded};
+  if (lane == 0) {
+    ranges[tile * kTileRows + row] = WorkRange{out, padded};
+    if (sorted != nullptr && ty * tg.th + row < H) {
+      const int c = work_class(padded);
+      const int at = atomicAdd(cursors + 2 + c, 1);
+      sorted[c * tg.total * kTileRows + at] = SortedRow{static_cast<int>(tile) * kTileRows + row, out, padded, 0};
+    }
+  }
   for (int base = 0; base < count; base += 64) {
     int c = first_c, roi = first_item, owner = 0;
     const RowTap* taps = first_taps;

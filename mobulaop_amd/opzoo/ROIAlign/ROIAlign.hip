@@ -35,6 +35,16 @@ constexpr long long kSideStreamBytes = 64ll << 20;
 // L2 caches (4 MB) then holds its eighth of the map's channel blocks whole.
 constexpr size_t kSortedAboveBytes = 24u << 20;
 
+// Tile rows of a backward pass that are sorted by the length of their work lists.
+constexpr long long kSortedRows = 1 << 17;
+// Pooled elements to an element of the map from which on they are: the owners' time is then that of their lists, and
+// ending together pays more than writing neighbouring pieces of a map row (224 bytes) together.  Whole passes of
+// 256 channels, natural and sorted order: 14 x 14, 8 x 128 x 128, 1024 / 2048 / 4096 / 8192 boxes (1.5 / 3 / 6 / 12 to one)
+// 424 / 701 / 1211 / 2177 and 413 / 658 / 1148 / 2105 us; 7 x 7, 2 x 64 x 64, 512 / 1024 / 2048 (3 / 6 / 12) 84.6 / 132 /
+// 235 and 85.4 / 125 / 225; 7 x 7, 4 x 200 x 336, 4000 / 8000 / 16000 / 24000 (0.7 / 1.5 / 2.9 / 4.4) 542 / 828 / 1431 /
+// 2050 and 584 / 848 / 1424 / 2027.  Channels-last rows, 24000 boxes in bf16: 1361 and 1397, so never.
+constexpr long long kSortedAbove = 4;
+
 struct Problem {
   long long n_out;  // R*C*PH*PW
   int R, C, H, W, PH, PW, S;
@@ -320,13 +330,15 @@ struct TilePlan {
   bool dy_transposed = false;   // the pre-pass also wrote dyb (plan_tiles was given dy)
   roialign::TileGrid grid;
   roialign::TileBox* boxes;
-  int* cursors;                // bump pointers: [0] ROI lists, [1] work lists
+  int* cursors;                // bump pointers: [0] ROI lists, [1] work lists; then rows of each class of `sorted`
   int* tile_rois;
   roialign::ListLayout layout;
   roialign::AxisUnit* lists;
   float* dyb;                  // channel-blocked copy of dy (null for channels-last tensors)
   size_t dyb_bytes, list_bytes;   // dyb_bytes: of one channel block's slab
   roialign::WorkRange* ranges; // per (tile, tile row)
+  roialign::SortedRow* sorted; // the same by length (null: not sorted)
+  const int* class_counts() const { return cursors + 2; }
   roialign::WorkEntry* entries;
 };
 
@@ -408,7 +420,7 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
   const long long list_cap = items * g.per_image;  // every item in every tile
   if (g.total <= 0 || g.total > (1ll << 24) || list_cap > (1ll << 27)) return false;
   const size_t b_recs = align_up(sizeof(roialign::TileBox) * std::max<long long>(items, 1), 256);
-  const size_t b_cnt = 256;   // the two bump pointers
+  const size_t b_cnt = 256;   // the counters
   const size_t b_list = align_up(sizeof(int) * std::max<long long>(list_cap, 1), 256);
   plan->layout = roialign::make_list_layout(g, p.PH, p.PW, p.S);
   const long long n_units = plan->layout.roi_stride * items;
@@ -429,8 +441,14 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
   plan->dyb_bytes = b_slab; plan->list_bytes = b_units;
   const size_t b_ranges = align_up(sizeof(roialign::WorkRange) * g.total * roialign::kTileRows, 256);
   const size_t b_entries = align_up(sizeof(roialign::WorkEntry) * n_entries, 256) + 512;
+  // (beyond kSortedRows the device is refilled so often that the last rows hardly count, and the classes' arrays
+  // would take 16 MB)
+  const long long sort_option = mobula_hip::option("roialign_sort_rows", 1);
+  const bool sort_rows = g.total * roialign::kTileRows <= kSortedRows && sort_option != 0 &&
+                         (sort_option == 2 || (!p.nhwc && p.n_out >= kSortedAbove * p.N * p.C * p.H * p.W));
+  const size_t b_sorted = sort_rows ? sizeof(roialign::SortedRow) * roialign::kWorkClasses * g.total * roialign::kTileRows : 0;
   char* base = static_cast<char*>(mobula_hip::workspace(b_offsets + b_recs + b_cnt + b_list + b_units + b_dyt +
-                                                        b_ranges + b_entries + 256));
+                                                        b_ranges + b_entries + b_sorted + 256));
   if (failed()) return false;
   int* offsets = nullptr;
   if (windows) {
@@ -449,6 +467,7 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
   cur += b_ranges;
   plan->entries = reinterpret_cast<roialign::WorkEntry*>(cur);
   cur += b_entries;
+  plan->sorted = sort_rows ? reinterpret_cast<roialign::SortedRow*>(cur) : nullptr;
   // two kernels: per-item tables (which also resets the bump pointers), then per-tile lists
   const int n_items = static_cast<int>(items);
   const roialign::ListsArgs la{rois, n_items, p.R, p.scale, p.PH, p.PW, p.S, p.H, p.W, p.N, g, plan->layout,
@@ -465,7 +484,7 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
   (windows ? roialign::build_tile_work_kernel<true> : roialign::build_tile_work_kernel<false>)
       <<<static_cast<unsigned>(g.total), roialign::kTileRows * 64, 0, stream>>>(
           plan->boxes, n_items, plan->tile_rois, plan->lists, g, plan->layout, plan->cursors, plan->ranges,
-          plan->entries);
+          plan->entries, plan->sorted, p.H);
   MOBULA_HIP_TRY(hipGetLastError());
   return !failed();
 }
@@ -543,7 +562,7 @@ void backward_device(const Problem& p, const T* dy, const float* rois, T* dx, bo
     int nsplit = row_split(p);
     const auto kernel = owner_kernel<true, T>(tw, &nsplit, plan.layout.windows != 0);
     kernel<<<static_cast<unsigned>(roialign::backward_blocked_grid(plan.grid.total, cblk)), BB::NT * nsplit, 0, stream>>>(
-        dy, dx, plan.ranges, plan.entries, plan.lists,
+        dy, dx, plan.ranges, plan.sorted, plan.class_counts(), plan.entries, plan.lists,
         plan.grid, plan.layout, p.C, p.H, p.W, p.PH, p.PW, cblk, dy_bytes,
         static_cast<unsigned>(plan.list_bytes), assign ? 1 : 0);
     MOBULA_HIP_TRY(hipGetLastError());
@@ -584,7 +603,7 @@ void backward_device(const Problem& p, const T* dy, const float* rois, T* dx, bo
                            mobula_hip::option("roialign_row_quads", 1) != 0;
         const auto kernel = owner_kernel<false, T>(tw, &nsplit, plan.layout.windows != 0);
         kernel<<<static_cast<unsigned>(grid), BB::NT * nsplit, 0, stream>>>(
-            plan.dyb, dx, plan.ranges, plan.entries, plan.lists, plan.grid, plan.layout, p.C, p.H,
+            plan.dyb, dx, plan.ranges, plan.sorted, plan.class_counts(), plan.entries, plan.lists, plan.grid, plan.layout, p.C, p.H,
             p.W, p.PH, p.PW, cblk, static_cast<unsigned>(plan.dyb_bytes),
             static_cast<unsigned>(plan.list_bytes), (assign ? 1 : 0) | (quads ? 2 : 0));
       }

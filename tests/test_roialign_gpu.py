@@ -1086,6 +1086,38 @@ def test_few_boxes_share_their_pooled_rows_among_wavefronts(R, C, pooled, S):
     assert_parity(y16.astype(np.float32), want.astype(np.float32), FP16_TOL, 'fp16')
 
 
+@pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
+@pytest.mark.parametrize('shape', [   # N, C, H, W, R, pooled, S
+    (2, 256, 33, 60, 90, (7, 7), 2), (1, 300, 16, 57, 40, (14, 14), 1), (3, 36, 47, 29, 250, (5, 9), 0),
+    (2, 64, 100, 64, 400, (7, 7), 2), (1, 4, 5, 7, 3, (2, 3), 2)])
+def test_rows_sorted_by_their_work_give_the_same_gradient(shape, layout):
+    """The tile owners in the order of their lists' lengths and in natural order: the same sums bit for bit, with
+    fewer and more than eight channel blocks, rows past the map's end, split rows, windows, boxes off the map."""
+    N, C, H, W, R, pooled, S = shape
+    abi.set_impl('tiled')
+    rng = np.random.default_rng(R)
+    scale = 0.5
+    c = np.stack([rng.normal(W / 2, W / 3, R) / scale, rng.normal(H / 2, H / 4, R) / scale], 1)
+    wh = np.exp(rng.uniform(np.log(2), np.log(W / scale), (R, 2)))
+    rois = np.concatenate([rng.integers(0, N, (R, 1)), c - wh / 2, c + wh / 2], 1).astype(np.float32)
+    dy = rng.standard_normal((R, C) + pooled).astype(np.float32)
+    want = oracle.backward(dy, rois, (N, C, H, W), scale, S, impl='ordered')
+    got = []
+    try:
+        for order in (0, 2):
+            native.set_option('roialign_sort_rows', order)
+            if layout == 'nchw':
+                dx = abi.backward(abi.to_dev(dy), abi.to_dev(rois), (N, C, H, W), scale, S, assign=True)
+            else:
+                dx = abi.backward_nhwc(abi.to_dev(np.ascontiguousarray(dy.transpose(0, 2, 3, 1))), abi.to_dev(rois),
+                                       (N, H, W, C), scale, S, assign=True).permute(0, 3, 1, 2)
+            got.append(dx.cpu())
+    finally:
+        native.set_option('roialign_sort_rows', 1)
+    assert torch.equal(got[0], got[1])
+    assert_parity(got[1].numpy(), want, BWD_TOL, 'dx')
+
+
 @pytest.mark.parametrize('pooled', [(7, 7), (3, 9), (12, 5), (14, 14)])
 @pytest.mark.parametrize('dtype,C', [(np.float32, 36), (np.float16, 72)])
 def test_adaptive_grids_at_the_edges_of_the_lists(dtype, C, pooled):
