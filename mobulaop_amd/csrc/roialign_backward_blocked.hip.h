@@ -68,14 +68,16 @@ inline int backward_row_split(long long images, int H, int W, int cblk) {
 // not exist.  One workgroup per (ROI, group of `per` channel blocks): the input words of the
 // group are contiguous and so are the output words of each of its blocks.
 // LDS holds the input as it is; the transposition happens in the reads.
-// T is the element type of dy (float or __half); dyb is fp32 either way.
+// dyb has dy's element type T: a 16-bit dy is widened where the owners use it, which halves what is written here and
+// read there (with fp32 in between: 4000 boxes, 7 x 7, on 4 x 256 x 200 x 336 fp16, both passes, 371 us against 349; 2048,
+// 28 x 28, on 8 x 256 x 128 x 128, 1872 against 1530, a part of it the order of the rows).
 // `block`: index among the workgroups (of 256 threads) that transpose.
 // `cap`: channels LDS holds at a time.  With per >= 1 whole blocks fit (cap is not used);
 // per == 0 says that not even one block does (large pooled sizes): the workgroup then takes one
 // channel block in passes of `cap` channels (a multiple of 4).
 template <typename T>
 __device__ __forceinline__ void transpose_dy_blocked_body(unsigned block, const T* __restrict__ dy,
-                                                          float* __restrict__ dyb, int C, int PH, int PW,
+                                                          T* __restrict__ dyb, int C, int PH, int PW,
                                                           int cblk, int per, int R, int cap) {
   constexpr int CB = BwdBlocked::CB;
   constexpr int VEC = 16 / sizeof(T);   // elements per 16-byte word
@@ -88,7 +90,11 @@ __device__ __forceinline__ void transpose_dy_blocked_body(unsigned block, const 
   const int c0 = cb0 * CB, nch = min(nblk * CB, C - c0);
   const int bins = PH * PW;
   const int pass_ch = per > 0 ? nch : cap;
-  typedef float f32x4s __attribute__((ext_vector_type(4)));
+  // four channels of a bin: written once, read by another kernel
+  typedef unsigned Four __attribute__((ext_vector_type(sizeof(T))));
+  auto store_four = [](T* to, const T (&v)[4]) {
+    __builtin_nontemporal_store(__builtin_bit_cast(Four, v), reinterpret_cast<Four*>(to));
+  };
   for (int pc = 0; pc < nch; pc += pass_ch) {
     const int pn = min(pass_ch, nch - pc);
     const T* src = dy + (static_cast<size_t>(r) * C + c0 + pc) * bins;
@@ -108,33 +114,28 @@ __device__ __forceinline__ void transpose_dy_blocked_body(unsigned block, const 
     if (per > 0) {
       for (int blk = 0; blk < nblk; ++blk) {
         // every channel block has a slab of its own (all ROIs): its owners address it with 32-bit offsets
-        float* const dst = dyb + (static_cast<size_t>(cb0 + blk) * R + r) * bins * CB;
+        T* const dst = dyb + (static_cast<size_t>(cb0 + blk) * R + r) * bins * CB;
         for (int p = threadIdx.x; p < per_blk; p += 256) {
           const int cq = p & 7, cell = p >> 3, c = blk * CB + 4 * cq;   // channel quad, bin, first channel
           const T* in = tbuf + c * bins + cell;
-          float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-          if (c + 0 < nch) v.x = to_float(in[0]);
-          if (c + 1 < nch) v.y = to_float(in[bins]);
-          if (c + 2 < nch) v.z = to_float(in[2 * bins]);
-          if (c + 3 < nch) v.w = to_float(in[3 * bins]);
-          __builtin_nontemporal_store(f32x4s{v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4s*>(dst + static_cast<size_t>(p) * 4));
+          T v[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = c + i < nch ? in[i * bins] : from_float<T>(0.0f);
+          store_four(dst + static_cast<size_t>(p) * 4, v);
         }
       }
     } else {
       // the channel quads pc / 4 .. of the one block: 16-byte pieces, the quads of a cell side by side;
       // the last pass also writes the zero quads of channels that do not exist
-      float* const dst = dyb + (static_cast<size_t>(cb0) * R + r) * bins * CB;
+      T* const dst = dyb + (static_cast<size_t>(cb0) * R + r) * bins * CB;
       const int q0 = pc / 4, nq = pc + pass_ch >= nch ? CB / 4 - q0 : pn / 4;
       for (int q = threadIdx.x; q < nq * bins; q += 256) {
         const int cell = q / nq, qi = q - cell * nq, c = 4 * qi;   // bin, channel quad and first channel within the pass
         const T* in = tbuf + c * bins + cell;
-        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (c + 0 < pn) v.x = to_float(in[0]);
-        if (c + 1 < pn) v.y = to_float(in[bins]);
-        if (c + 2 < pn) v.z = to_float(in[2 * bins]);
-        if (c + 3 < pn) v.w = to_float(in[3 * bins]);
-        __builtin_nontemporal_store(f32x4s{v.x, v.y, v.z, v.w},
-                                    reinterpret_cast<f32x4s*>(dst + (static_cast<size_t>(cell) * 8 + q0 + qi) * 4));
+        T v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = c + i < pn ? in[i * bins] : from_float<T>(0.0f);
+        store_four(dst + (static_cast<size_t>(cell) * 8 + q0 + qi) * 4, v);
       }
     }
   }
@@ -142,7 +143,7 @@ __device__ __forceinline__ void transpose_dy_blocked_body(unsigned block, const 
 
 template <typename T>
 __global__ void __launch_bounds__(256)
-transpose_dy_blocked_kernel(const T* __restrict__ dy, float* __restrict__ dyb, int C, int PH,
+transpose_dy_blocked_kernel(const T* __restrict__ dy, T* __restrict__ dyb, int C, int PH,
                             int PW, int cblk, int per, int R, int cap) {
   transpose_dy_blocked_body<T>(blockIdx.x, dy, dyb, C, PH, PW, cblk, per, R, cap);
 }
@@ -154,7 +155,7 @@ transpose_dy_blocked_kernel(const T* __restrict__ dy, float* __restrict__ dyb, i
 // dependencies than in work.  Dynamic LDS as for transpose_dy_blocked_kernel.
 template <typename T>
 __global__ void __launch_bounds__(256)
-lists_and_dy_kernel(ListsArgs lists, unsigned list_blocks, const T* __restrict__ dy, float* __restrict__ dyb,
+lists_and_dy_kernel(ListsArgs lists, unsigned list_blocks, const T* __restrict__ dy, T* __restrict__ dyb,
                     int cblk, int per, int C) {
   if (blockIdx.x < list_blocks) {
     if (lists.window_offsets != nullptr) build_window_lists_body(blockIdx.x, lists);
@@ -195,8 +196,8 @@ __device__ __forceinline__ float lane_value(const unsigned __attribute__((ext_ve
 // way out -- for maps that give the SIMDs too few tile rows to keep them busy.
 // WIN: the list items are windows of merged column weights (sampling grids of more than two
 // points per bin and axis) instead of pairs of sample columns.
-// dy_any: the blocked fp32 copy dyb, or for channels-last tensors the caller's
-// dy[R][PH][PW][C] itself, of dx's element type.
+// dy_any: the blocked copy dyb, or for channels-last tensors the caller's dy[R][PH][PW][C] itself; of
+// dx's element type.
 template <bool NHWC, typename TO, int TW, int NSPLIT = 1, bool WIN = false>
 __global__ void __launch_bounds__(BwdBlocked::NT * NSPLIT)
 backward_blocked_kernel(const void* __restrict__ dy_any, TO* __restrict__ dx_any,
@@ -270,7 +271,7 @@ backward_blocked_kernel(const void* __restrict__ dy_any, TO* __restrict__ dx_any
 
   // dyb and the sample lists as raw buffers: a scalar byte offset per entry
   // plus a fixed lane offset
-  typedef typename std::conditional<NHWC, TO, float>::type TI;   // element type of what dy_any points to
+  typedef TO TI;   // element type of what dy_any points to
   constexpr unsigned E = sizeof(TI);
   const unsigned dy_pw = (NHWC ? C : K::CB) * E;
   const unsigned dy_ph = static_cast<unsigned>(PW) * dy_pw;

@@ -142,12 +142,12 @@ __device__ __forceinline__ void transpose_pixels(const T* __restrict__ src, T* _
 }
 
 // out[n][cb][p][CB] = in[n][cb*CB + k][p].
-// With oa.order set the launch has one more column of workgroups, the first of which sorts the
+// ORDER (oa.order set): the launch has one more column of workgroups, the first of which sorts the
 // ROIs (roi_order_body with the cells that fit the tile's LDS) while the others copy: the
 // ordering of a few thousand ROIs then costs nothing beside a copy that takes several times as long.
 // sparse != 0 (few ROIs on a large map): a workgroup takes a run of 64 pixels of every gridDim.y-th of the
 // cblk channel blocks, and leaves the copy unwritten where no box reaches.
-template <typename T, bool VEC>
+template <typename T, bool VEC, bool ORDER>
 __global__ void __launch_bounds__(256)
 transpose_to_blocked_kernel(const T* __restrict__ in, T* __restrict__ out, int C, int P, int cblk, int sparse,
                             OrderArgs oa) {
@@ -155,7 +155,7 @@ transpose_to_blocked_kernel(const T* __restrict__ in, T* __restrict__ out, int C
   __shared__ T tile[CB][65];
   if (oa.direct != nullptr && *oa.direct != 0) return;
   int bx = blockIdx.x;
-  if (oa.order != nullptr) {
+  if constexpr (ORDER) {
     if (bx == 0) {
       if (blockIdx.y == 0 && blockIdx.z == 0) {
         constexpr int WORDS = static_cast<int>(sizeof(tile) / 4), MAXC = WORDS - 24;

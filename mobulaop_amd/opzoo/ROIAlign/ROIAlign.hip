@@ -291,12 +291,11 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
     const dim3 tgrid(static_cast<unsigned>((pixels + 63) / 64) + (order_in_copy ? 1u : 0u),
                      static_cast<unsigned>(sparse ? std::min(cblk, 2) : cblk), static_cast<unsigned>(p.N));
     const bool vec = pixels % 4 == 0 && reinterpret_cast<size_t>(x) % (4 * sizeof(T)) == 0;
-    if (vec)
-      roialign::transpose_to_blocked_kernel<T, true><<<tgrid, 256, 0, stream>>>(
-          x, xt, p.C, static_cast<int>(pixels), cblk, sparse ? 1 : 0, oa);
-    else
-      roialign::transpose_to_blocked_kernel<T, false><<<tgrid, 256, 0, stream>>>(
-          x, xt, p.C, static_cast<int>(pixels), cblk, sparse ? 1 : 0, oa);
+    const auto transpose = order_in_copy ? (vec ? roialign::transpose_to_blocked_kernel<T, true, true>
+                                                : roialign::transpose_to_blocked_kernel<T, false, true>)
+                                         : (vec ? roialign::transpose_to_blocked_kernel<T, true, false>
+                                                : roialign::transpose_to_blocked_kernel<T, false, false>);
+    transpose<<<tgrid, 256, 0, stream>>>(x, xt, p.C, static_cast<int>(pixels), cblk, sparse ? 1 : 0, oa);
     side.join();
     if (small_grid) {
       mobula_hip::KernelTimer timer("forward_blocked_kernel", stream, !fixed);   // (its events are allocations)
@@ -334,7 +333,7 @@ struct TilePlan {
   int* tile_rois;
   roialign::ListLayout layout;
   roialign::AxisUnit* lists;
-  float* dyb;                  // channel-blocked copy of dy (null for channels-last tensors)
+  char* dyb;                   // channel-blocked copy of dy, of its type (null for channels-last tensors)
   size_t dyb_bytes, list_bytes;   // dyb_bytes: of one channel block's slab
   roialign::WorkRange* ranges; // per (tile, tile row)
   roialign::SortedRow* sorted; // the same by length (null: not sorted)
@@ -428,8 +427,8 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
   const size_t b_units = align_up(sizeof(roialign::AxisUnit) * n_units, 256) + 256;  // blocks are read whole
   const int cblk = (p.C + 31) / 32;
   // dyb: one slab per channel block (all ROIs), 256-byte aligned
-  // (a multiple of 128 bytes; the slabs follow each other as the transposition writes them)
-  const size_t b_slab = with_dyb ? sizeof(float) * 32 * p.PW * p.R * p.PH : 0;
+  // (a multiple of 64 bytes; the slabs follow each other as the transposition writes them)
+  const size_t b_slab = with_dyb ? sizeof(T) * 32 * p.PW * p.R * p.PH : 0;
   const size_t b_dyt = align_up(b_slab * cblk, 256);
   // work lists: every tap of every ROI once per tile column it spans
   // (windows: the bound that came back with their number)
@@ -461,7 +460,7 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
   plan->tile_rois = reinterpret_cast<int*>(base + b_recs + b_cnt);
   plan->lists = reinterpret_cast<roialign::AxisUnit*>(base + b_recs + b_cnt + b_list);
   char* cur = base + b_recs + b_cnt + b_list + b_units;
-  plan->dyb = with_dyb ? reinterpret_cast<float*>(cur) : nullptr;
+  plan->dyb = with_dyb ? cur : nullptr;
   cur += b_dyt;
   plan->ranges = reinterpret_cast<roialign::WorkRange*>(cur);
   cur += b_ranges;
@@ -476,7 +475,7 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
   const DyLaunch dl = dy_launch<T>(p);
   if (fuse_dy != nullptr && with_dyb && dl.per > 0 && dl.blocks > 0 && dl.blocks + list_blocks < (1ll << 31)) {
     roialign::lists_and_dy_kernel<T><<<static_cast<unsigned>(dl.blocks + list_blocks), 256, dl.lds, stream>>>(
-        la, static_cast<unsigned>(list_blocks), fuse_dy, plan->dyb, cblk, dl.per, p.C);
+        la, static_cast<unsigned>(list_blocks), fuse_dy, reinterpret_cast<T*>(plan->dyb), cblk, dl.per, p.C);
     plan->dy_transposed = true;
   } else {
     roialign::build_lists_kernel<<<static_cast<unsigned>(list_blocks), 256, 0, stream>>>(la);
@@ -593,7 +592,7 @@ void backward_device(const Problem& p, const T* dy, const float* rois, T* dx, bo
     if (grid < (1ll << 31) && dl.blocks < (1ll << 31) && (dl.per > 0 || dl.cap >= 4)) {
       if (p.R > 0 && !plan.dy_transposed)
         roialign::transpose_dy_blocked_kernel<T><<<static_cast<unsigned>(dl.blocks), 256, dl.lds, side.get()>>>(
-            dy, plan.dyb, p.C, p.PH, p.PW, cblk, dl.per, p.R, dl.cap);
+            dy, reinterpret_cast<T*>(plan.dyb), p.C, p.PH, p.PW, cblk, dl.per, p.R, dl.cap);
       side.join();
       {
         mobula_hip::KernelTimer timer("backward_blocked_kernel", stream);

@@ -1086,6 +1086,25 @@ def test_few_boxes_share_their_pooled_rows_among_wavefronts(R, C, pooled, S):
     assert_parity(y16.astype(np.float32), want.astype(np.float32), FP16_TOL, 'fp16')
 
 
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('C,pooled,S', [(36, (7, 7), 2), (300, (3, 5), 1), (64, (32, 32), 2), (4, (9, 2), 0)])
+def test_sixteen_bit_gradients_through_the_blocked_copy(dtype, C, pooled, S):
+    """A 16-bit dy is copied as it is and widened by the tile owners: the same sums, bit for bit, as from the
+    channels-last tensor they read directly; last channel blocks in part, rows at odd 16-bit places."""
+    abi.set_impl('tiled')
+    rng = np.random.default_rng(C)
+    N, H, W, R, scale = 2, 35, 59, 23, 0.5
+    c = np.stack([rng.uniform(0, W, R), rng.uniform(0, H, R)], 1) / scale
+    wh = np.exp(rng.uniform(np.log(3), np.log(W / scale), (R, 2)))
+    rois = abi.to_dev(np.concatenate([rng.integers(0, N, (R, 1)), c - wh / 2, c + wh / 2], 1).astype(np.float32))
+    dy = abi.to_dev(rng.standard_normal((R, C) + pooled).astype(np.float32)).to(dtype)
+    got = abi.backward(dy, rois, (N, C, H, W), scale, S, assign=True)
+    same = abi.backward_nhwc(dy.permute(0, 2, 3, 1).contiguous(), rois, (N, H, W, C), scale, S, assign=True)
+    assert torch.equal(got, same.permute(0, 3, 1, 2))
+    want = oracle.backward(dy.float().cpu().numpy(), rois.cpu().numpy(), (N, C, H, W), scale, S, impl='ordered')
+    assert_parity(got.float().cpu().numpy(), want, FP16_TOL if dtype == torch.float16 else 2.0 ** -8, 'dx')
+
+
 @pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
 @pytest.mark.parametrize('shape', [   # N, C, H, W, R, pooled, S
     (2, 256, 33, 60, 90, (7, 7), 2), (1, 300, 16, 57, 40, (14, 14), 1), (3, 36, 47, 29, 250, (5, 9), 0),
