@@ -42,7 +42,11 @@ constexpr long long kSortedRows = 1 << 17;
 // 256 channels, natural and sorted order: 14 x 14, 8 x 128 x 128, 1024 / 2048 / 4096 / 8192 boxes (1.5 / 3 / 6 / 12 to one)
 // 424 / 701 / 1211 / 2177 and 413 / 658 / 1148 / 2105 us; 7 x 7, 2 x 64 x 64, 512 / 1024 / 2048 (3 / 6 / 12) 84.6 / 132 /
 // 235 and 85.4 / 125 / 225; 7 x 7, 4 x 200 x 336, 4000 / 8000 / 16000 / 24000 (0.7 / 1.5 / 2.9 / 4.4) 542 / 828 / 1431 /
-// 2050 and 584 / 848 / 1424 / 2027.  Channels-last rows, 24000 boxes in bf16: 1361 and 1397, so never.
+// 2050 and 584 / 848 / 1424 / 2027.  Channels-last rows, 24000 boxes in bf16: 1361 and 1397, so never.  And never with
+// fewer than five channel blocks: several XCDs then share one and each takes a part of the map in natural order, whose
+// dy stays in its L2; sorted, every one of them reads all of it.  14 x 14, 4096 boxes, 32 / 64 / 96 / 128 / 192 channels:
+// 234 / 396 / 613 / 686 / 1073 and 284 / 444 / 596 / 665 / 994; 28 x 28, 4 x 69 x 230, 1041 boxes, 64 / 96 / 256 channels:
+// 634 / 1075 / 2013 and 745 / 1267 / 1990.
 constexpr long long kSortedAbove = 4;
 
 struct Problem {
@@ -444,7 +448,7 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
   // would take 16 MB)
   const long long sort_option = mobula_hip::option("roialign_sort_rows", 1);
   const bool sort_rows = g.total * roialign::kTileRows <= kSortedRows && sort_option != 0 &&
-                         (sort_option == 2 || (!p.nhwc && p.n_out >= kSortedAbove * p.N * p.C * p.H * p.W));
+                         (sort_option == 2 || (!p.nhwc && cblk >= 5 && p.n_out >= kSortedAbove * p.N * p.C * p.H * p.W));
   const size_t b_sorted = sort_rows ? sizeof(roialign::SortedRow) * roialign::kWorkClasses * g.total * roialign::kTileRows : 0;
   char* base = static_cast<char*>(mobula_hip::workspace(b_offsets + b_recs + b_cnt + b_list + b_units + b_dyt +
                                                         b_ranges + b_entries + b_sorted + 256));
