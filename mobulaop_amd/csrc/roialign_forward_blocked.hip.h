@@ -28,7 +28,6 @@ struct FwdBlocked {
   static constexpr int PWB = 8;        // pooled columns per step (one per group of 8 lanes)
   static constexpr int CELL = 32;      // side of the sorting cells in pixels
   static constexpr int MAXCELLS = 8192;
-  static constexpr int CLASSES = 4;    // of boxes by their work, adaptive grids (roi_order_body)
 };
 
 // Per element type: channels per lane (16 bytes), channels per block of the
@@ -64,8 +63,8 @@ struct OrderArgs {
 
 template <int NT, int MAXC>
 __device__ __forceinline__ void roi_order_body(int* hist, int* wave_sum, int* carry, const float* __restrict__ rois,
-                                               int R, float scale, int H, int W, long long num_images, int PH, int PW,
-                                               int S, int* __restrict__ order);
+                                               int R, float scale, int H, int W, long long num_images,
+                                               int* __restrict__ order);
 
 // True if no sample of any ROI can touch the pixels p0 .. p0 + 63 of image n (asked by a whole workgroup
 // of 256 threads, each looks at every 256th ROI).  A box's pixels lie between the cells of its two
@@ -161,7 +160,7 @@ transpose_to_blocked_kernel(const T* __restrict__ in, T* __restrict__ out, int C
         constexpr int WORDS = static_cast<int>(sizeof(tile) / 4), MAXC = WORDS - 24;
         int* const words = reinterpret_cast<int*>(&tile[0][0]);
         roi_order_body<256, MAXC>(words, words + MAXC + 1, words + MAXC + 20, oa.rois, oa.R, oa.scale, oa.H, oa.W,
-                                  oa.num_images, oa.PH, oa.PW, oa.S, oa.order);
+                                  oa.num_images, oa.order);
       }
       return;
     }
@@ -184,36 +183,29 @@ transpose_to_blocked_kernel(const T* __restrict__ in, T* __restrict__ out, int C
 
 // order[] = ROI indices sorted by (image, 32x32-pixel cell of the box centre,
 // rows of cells walked in alternating direction): consecutive wavefronts then
-// read neighbouring parts of the map.  With an adaptive grid a box of large bins takes many times as long as a
-// small one, and one that starts last keeps the device waiting: boxes are then sorted by classes of work first, the
-// longest in front (6000 boxes, 7 x 7, on 100 x 100: 2.8 of four wavefronts a SIMD in flight on average, then 3.5;
-// 580 -> 526 us).  One workgroup; counting sort with the
+// read neighbouring parts of the map.  (Longest boxes first, for adaptive grids: 2 % on a map whose eighth
+// an L2 nearly holds, and up to twice the time where XCDs take ranges of the order: one then has all the long ones.)
+// One workgroup; counting sort with the
 // histogram in LDS.  ROIs that name no image sort last.
 // (the body: NT threads of one workgroup, at most MAXC cells; hist holds MAXC + 1 counters)
 template <int NT, int MAXC>
 __device__ __forceinline__ void roi_order_body(int* hist, int* wave_sum, int* carry, const float* __restrict__ rois,
-                                               int R, float scale, int H, int W, long long num_images, int PH, int PW,
-                                               int S, int* __restrict__ order) {
+                                               int R, float scale, int H, int W, long long num_images,
+                                               int* __restrict__ order) {
   using K = FwdBlocked;
-  const int classes = S <= 0 ? K::CLASSES : 1;
   int cell = K::CELL;
   long long cy = (H + cell - 1) / cell, cx = (W + cell - 1) / cell;
-  while (classes * cy * cx * num_images > MAXC && cell < (1 << 20)) {
+  while (cy * cx * num_images > MAXC && cell < (1 << 20)) {
     cell *= 2;
     cy = (H + cell - 1) / cell; cx = (W + cell - 1) / cell;
   }
-  const int cells = classes * cy * cx * num_images > MAXC ? 1 : static_cast<int>(classes * cy * cx * num_images);
+  const int cells = cy * cx * num_images > MAXC ? 1 : static_cast<int>(cy * cx * num_images);
   struct Box { float v[5]; };
   auto key_of = [&](const Box& box) {
     const float* const q = box.v;
-    int b = static_cast<int>(q[0]);
+    const int b = static_cast<int>(q[0]);
     if (b < 0 || b >= num_images) return cells;
     if (cells == 1) return 0;
-    if (classes > 1) {   // pixels of a bin, its border included
-      const float work = ((q[4] - q[2]) * scale / static_cast<float>(PH) + 2.0f) *
-                         ((q[3] - q[1]) * scale / static_cast<float>(PW) + 2.0f);
-      b += static_cast<int>(num_images) * (work >= 128.0f ? 0 : work >= 64.0f ? 1 : work >= 32.0f ? 2 : 3);
-    }
     const float mx = 0.5f * (q[1] + q[3]) * scale, my = 0.5f * (q[2] + q[4]) * scale;
     const int ix = min(max(static_cast<int>(mx), 0), W - 1) / cell;
     const int iy = min(max(static_cast<int>(my), 0), H - 1) / cell;
@@ -262,12 +254,11 @@ __device__ __forceinline__ void roi_order_body(int* hist, int* wave_sum, int* ca
 
 __global__ void __launch_bounds__(1024)
 roi_order_kernel(const float* __restrict__ rois, int R, float scale, int H, int W,
-                 long long num_images, int PH, int PW, int S, int* __restrict__ order) {
+                 long long num_images, int* __restrict__ order) {
   __shared__ int hist[FwdBlocked::MAXCELLS + 1];
   __shared__ int wave_sum[16];
   __shared__ int carry;
-  roi_order_body<1024, FwdBlocked::MAXCELLS>(hist, wave_sum, &carry, rois, R, scale, H, W, num_images, PH, PW, S,
-                                                   order);
+  roi_order_body<1024, FwdBlocked::MAXCELLS>(hist, wave_sum, &carry, rois, R, scale, H, W, num_images, order);
 }
 
 // A row sample: byte offsets of its low and high row in a channel block's

@@ -20,9 +20,9 @@
 // Bound by vector instructions and the L1 path about alike (4 x 512 x 100 x 100 fp16, 6000 boxes, 7 x 7: busy 80 % and 78 % of
 // the time): a multiply-add per pixel and channel, a 16-byte load per pixel and eight channels.  What is not
 // one of these is kept out of the loops: lists end in entries that load nothing, so a column takes a read and an
-// add; a row's entry is fetched from a lane that holds it; both axes' lists are made in one go; windows of 14
-// samples, so that only bins beyond 14 pixels are listed twice (4999 -> 4054 vector instructions a wavefront);
-// and the ROIs are ordered so that the longest start first (roi_order_body).  Together 582 -> 455 us a call.
+// add; a row's entry is fetched from a lane that holds it; both axes' lists are made in one go; grids of up to
+// 14 points in one window, so that only bins beyond 14 pixels are listed twice (4999 -> 4054 vector instructions a wavefront,
+// 573 -> 473 us a call).
 #pragma once
 #include <type_traits>
 
@@ -31,8 +31,10 @@
 namespace roialign {
 
 struct FwdMerged {
-  static constexpr int LCAP = 28;   // entries per merged list
-  static constexpr int WS = 14;     // samples merged per list at a time: at most 2 * WS entries
+  static constexpr int LCAP = 28;   // entries per merged list: two a sample
+  // Samples merged per list at a time: all of a grid of up to 14, else 11 (grids of up to 22 in two windows; in windows of
+  // 14 they take 7 % longer: 3000 boxes with bins of up to 23 pixels on 8 x 96 x 160 x 160, 499 and 534 us).
+  static constexpr int WHOLE = 14, WS = 11;
   static constexpr int RPH = 8;     // pooled rows whose lists are held at a time
   // One wavefront per workgroup: the wavefronts are independent, and a slot is refilled as soon
   // as its wavefront ends instead of when the slowest of four does (boxes differ a lot in work
@@ -143,6 +145,7 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
   const int batch = uni_i(g.batch);
   const bool image_ok = batch >= 0 && batch < num_images;
   const int gh = uni_i(g.grid_h), gw = uni_i(g.grid_w);
+  const int ws_h = gh <= M::WHOLE ? M::WHOLE : M::WS, ws_w = gw <= M::WHOLE ? M::WHOLE : M::WS;
   // A box far larger than the map (or infinite) has up to 2^31 sample points per
   // bin, nearly all outside the map: forward_large_grid_kernel does those boxes.
   if (gh > kSearchedGrid || gw > kSearchedGrid) return;
@@ -173,7 +176,7 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
     if (i0 != row_i0 || ph < row_p0 || ph >= row_p0 + M::RPH) {
       row_p0 = ph; row_i0 = i0;
       if (lane < M::RPH && ph + lane < PH)
-        rown[lane] = merge_axis_samples(rowm[lane], g.start_h, ph + lane, g.bin_h, i0, min(M::WS, gh - i0),
+        rown[lane] = merge_axis_samples(rowm[lane], g.start_h, ph + lane, g.bin_h, i0, min(ws_h, gh - i0),
                                         gh, H, row_bytes);
     }
   };
@@ -189,7 +192,7 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
       col_p0 = pwb; col_i0 = i0;
       int n = 0;
       if (lane < K::PWB && pwb + lane < PW) {
-        n = merge_axis_samples(colm[lane], g.start_w, pwb + lane, g.bin_w, i0, min(M::WS, gw - i0), gw, W,
+        n = merge_axis_samples(colm[lane], g.start_w, pwb + lane, g.bin_w, i0, min(ws_w, gw - i0), gw, W,
                                px_bytes);
       }
       const int own = n;
@@ -207,7 +210,7 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
     int n = 0;
     if (lane < 16 && p < (is_col ? PW : PH))
       n = merge_axis_samples(is_col ? colm[lane & 7] : rowm[lane & 7], is_col ? g.start_w : g.start_h, p,
-                             is_col ? g.bin_w : g.bin_h, 0, min(M::WS, grid), grid, is_col ? W : H,
+                             is_col ? g.bin_w : g.bin_h, 0, min(is_col ? ws_w : ws_h, grid), grid, is_col ? W : H,
                              is_col ? px_bytes : row_bytes);
     if (lane < 8) rown[lane] = n;
     const int own = __shfl(n, (lane & 7) + 8);
@@ -230,12 +233,12 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
         for (int i = 0; i < CPL; ++i) acc[i] = 0.0f;
         if (image_ok) {
 #pragma nounroll
-          for (int iyw = 0; iyw < gh; iyw += M::WS) {
+          for (int iyw = 0; iyw < gh; iyw += ws_h) {
             need_rows(ph, iyw);
             const int nr = uni_i(rown[ph - row_p0]);
             const MergedEntry row_of_lane = rowm[ph - row_p0][min(lane, M::LCAP - 1)];   // an entry a lane
 #pragma nounroll
-            for (int ixw = 0; ixw < gw; ixw += M::WS) {
+            for (int ixw = 0; ixw < gw; ixw += ws_w) {
               need_cols(pwb, ixw);
               const MergedEntry* const clist = colm[grp];
               // blocks of four map rows (scalar) x four or two map columns (per lane): the columns

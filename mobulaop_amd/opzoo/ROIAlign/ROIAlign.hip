@@ -207,7 +207,7 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
     if (sizeof(T) * p.N * pixels * p.C > kSortedAboveBytes) {
       order = static_cast<int*>(mobula_hip::workspace(sizeof(int) * p.R));
       if (failed()) return;
-      roialign::roi_order_kernel<<<1, 1024, 0, stream>>>(rois, p.R, p.scale, p.H, p.W, p.N, p.PH, p.PW, p.S, order);
+      roialign::roi_order_kernel<<<1, 1024, 0, stream>>>(rois, p.R, p.scale, p.H, p.W, p.N, order);
     }
     const long long grid = roialign::blocked_grid_nhwc(static_cast<long long>(p.R) * parts, cblk, nw);
     if (small_grid) {
@@ -285,7 +285,7 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
     const bool order_in_copy = order != nullptr && p.R <= kOrderInCopyRois;
     mobula_hip::SideStream side(stream, !fixed && order != nullptr && !order_in_copy && p.R > kSideStreamRois);
     if (order != nullptr && !order_in_copy)
-      roialign::roi_order_kernel<<<1, 1024, 0, side.get()>>>(rois, p.R, p.scale, p.H, p.W, p.N, p.PH, p.PW, p.S, order);
+      roialign::roi_order_kernel<<<1, 1024, 0, side.get()>>>(rois, p.R, p.scale, p.H, p.W, p.N, order);
     const roialign::OrderArgs oa{rois, order_in_copy ? order : nullptr, static_cast<int>(p.R), p.scale, p.H, p.W, p.N,
                                  p.PH, p.PW, p.S, choice};
     // Few boxes on a large map: only what they can touch is copied (4 x 256 x 200 x 336 in fp32, adaptive

@@ -1142,7 +1142,7 @@ def test_rows_sorted_by_their_work_give_the_same_gradient(shape, layout):
 def test_adaptive_grids_at_the_edges_of_the_lists(dtype, C, pooled):
     """Bins of one to 17 pixels an axis: merged lists of 14 samples and one more, more pooled rows and columns than are
     listed at a time, rows staged in several passes; enough boxes for all of their pooled rows to stay with
-    one wavefront, on a map that is read in order of work and place."""
+    one wavefront, on a map that is read in order of place."""
     abi.set_impl('auto')
     rng = np.random.default_rng(C + pooled[1])
     N, H, W = 2, 17 * pooled[0] + 2, 17 * pooled[1] + 2
