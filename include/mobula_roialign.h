@@ -304,8 +304,8 @@ void mobula_hip_clear_error(void);
  * "conv_fp32_split": 1 (default) lets fp32 products of large layers be formed
  * from three bf16 parts of every operand, six products of parts for one of
  * fp32, where that is faster (results as near to exact ones as the fp32
- * kernels'; tensors with infinities, NaN, subnormals or products near the
- * ends of the range take those), 0 never, 2 wherever a product fits;
+ * kernels'; tensors with infinities, NaN, subnormals, or whose products or
+ * sums could come near the ends of the range, take those), 0 never, 2 wherever a product fits;
  * "roialign_tile_columns": 0 (default) lets the backward pass choose its tile
  * width from the size of the map, 56 or 28 fixes it; "roialign_row_split": 0
  * (default) lets it choose how many wavefronts share a tile row's work list,

@@ -68,16 +68,28 @@ struct GatherStep {
 };
 
 // Three bf16 parts stand for an fp32 value exactly, and their products for fp32 products, while no part
-// and no product of two parts leaves the normal range: biased exponents of 24 to 247 in either
-// operand, and the smallest two together at least 2^-100 (a product's last counted part is 2^-24 of it).
+// and no product of two parts leaves the normal range and no sum of them overflows: biased exponents of 24 to 247 in
+// either operand, the smallest two together at least 2^-100 (a product's last counted part is 2^-24 of it), and
+// the largest two small enough for a sum of as many terms as the product has.  (Where a sum overflows, the parts'
+// sums do so with either sign and give NaN for an infinity; just below, a head is rounded up past the end.)
 // Infinities and NaN are outside, so are subnormals.  The fp32 kernels take the product otherwise; both
 // are launched, and the tensors' words decide on the device which of them returns at once.
 struct SplitRange {
   const unsigned* a; const unsigned* b;   // exponent words of the operands; null: no choice to make
+  int most;                               // what eight times the highest bits of both may come to (most_exponents)
+  // An operand whose highest bit is h lies below 2^(8 h + 8 - 127), parts and all; `terms` products of two, in six
+  // products of parts that exceed them by a hundredth, stay below 2^128 while
+  // 8 (ha + hb) + 16 - 254 + log2(terms) <= 127.
+  __host__ static int most_exponents(long long terms) {
+    int log = 0;
+    while ((1ll << log) < terms) ++log;
+    return 127 + 254 - 16 - log;
+  }
   __device__ bool inside() const {
     const unsigned ea = *a, eb = *b, both = ea | eb;
     const int low_a = ea == 0u ? 31 : __builtin_ctz(ea), low_b = eb == 0u ? 31 : __builtin_ctz(eb);
-    return (both & 0x80000007u) == 0u && 8 * (low_a + low_b) >= 2 * 127 - 100;
+    const int high_a = ea == 0u ? 0 : 31 - __builtin_clz(ea), high_b = eb == 0u ? 0 : 31 - __builtin_clz(eb);
+    return (both & 0x80000007u) == 0u && 8 * (low_a + low_b) >= 2 * 127 - 100 && 8 * (high_a + high_b) <= most;
   }
   __device__ bool leaves_split() const { return a != nullptr && !inside(); }
   __device__ bool leaves_fp32() const { return a != nullptr && inside(); }

@@ -976,7 +976,7 @@ bool forward_split(const conv::Geometry& g, const float* x, const float* weight,
   char* const ws = static_cast<char*>(mobula_hip::workspace_if_possible(kWordBytes + f.prep.bytes + plan.bytes + kPieceBytes));
   if (ws == nullptr) return failed();
   unsigned* const words = reinterpret_cast<unsigned*>(ws);
-  const conv::SplitRange range{words, words + 1};
+  const conv::SplitRange range{words, words + 1, conv::SplitRange::most_exponents(g.C * taps)};
   char* const tables = f.place(ws + kWordBytes);
   float* const pieces = reinterpret_cast<float*>(tables + plan.bytes);
   conv::clear_words_kernel<<<1, 64, 0, stream>>>(words, 2);
@@ -1010,7 +1010,9 @@ bool gradients_split(const conv::Geometry& g, const float* dy, const float* x, c
   if (ws == nullptr) return failed();
   unsigned* const words = reinterpret_cast<unsigned*>(ws);   // dy, weights, x
   char* const tables = b.place(ws + kWordBytes);
-  const conv::SplitRange data_range{words, words + 1}, weight_range{words, words + 2};
+  const conv::SplitRange data_range{words, words + 1, conv::SplitRange::most_exponents(g.D * taps)};
+  const conv::SplitRange weight_range{words, words + 2,
+                                      conv::SplitRange::most_exponents(static_cast<long long>(g.N) * g.OH * g.OW)};
   conv::clear_words_kernel<<<1, 64, 0, stream>>>(words, 3);
   b.prep.launch<3>(stream, conv::ExponentWords{words + 1, words, words + 2});
   launch_gradients_b16<3>(b, tables + plan.bytes, stream, data_range, weight_range);

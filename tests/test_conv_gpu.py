@@ -711,3 +711,37 @@ def test_values_that_three_parts_do_not_stand_for(scale_x, scale_w, odd, split_a
             assert ((a[fine].double() - b[fine].double()).norm() / scale).item() <= 2e-6, what
         else:
             assert torch.equal(a[fine], b[fine]), what
+
+
+@pytest.mark.parametrize('place,a,b', [
+    # one product of two elements, the others of these tensors being zero
+    ('one', 1.005 * 2.0 ** 70, 2.0 ** 70),      # an infinity; of the parts' products +inf and -inf
+    ('one', -1.005 * 2.0 ** 70, 2.0 ** 70),
+    ('one', 1.998 * 2.0 ** 63, 2.0 ** 64),      # finite; with the head rounded up 2^128
+    ('one', 1.998 * 2.0 ** 50, 2.0 ** 50),      # finite, and formed from parts
+    # sums of terms of one size, of one sign (of both, what overflows on the way depends on the order of the sum,
+    # which neither way states): all overflow; none does
+    ('all', 2.0 ** 63, 2.0 ** 62), ('all', 2.0 ** 50, 2.0 ** 50),
+])
+def test_fp32_products_and_sums_that_overflow(place, a, b, split_always):
+    """Results are finite, infinite and NaN where the fp32 kernels' are, and these operands' (a product of
+    few bits, sums that are whole multiples of one) the same to the bit."""
+    N, C, H, W, D = 2, 64, 24, 28, 128
+    geo = _ci(N, C, H, W, D, 3, 3, 1, 1, 1, 1, 1, 1)
+    sign = (torch.arange(D, device='cuda') % 3 - 1.5).sign()   # of a filter's weights and of its dy
+
+    def make(value, *shape):
+        if place == 'all':
+            return torch.full(shape, value, device='cuda')
+        t = torch.zeros(shape, device='cuda')
+        t[0, 5, 1, 1] = value
+        return t
+    x, w = make(a, N, C, H, W), make(b, D, C, 3, 3) * sign.reshape(D, 1, 1, 1)
+    for dy in make(a, N, D, H, W), make(b, N, D, H, W):
+        dy *= sign.reshape(D, 1, 1)
+        native.set_option('conv_fp32_split', 2)
+        got = _three_products(geo, x, w, dy)
+        native.set_option('conv_fp32_split', 0)
+        for p, q, what in zip(got, _three_products(geo, x, w, dy), ('y', 'dx', 'dw')):
+            assert torch.equal(p.isnan(), q.isnan()) and torch.equal(p.nan_to_num(0.0), q.nan_to_num(0.0)), what
+            assert torch.equal(p.isinf(), q.isinf()), what
