@@ -297,15 +297,19 @@ void mobula_hip_clear_error(void);
  * "host_staging_device"; "kernel_timing": 0 off, 1 on; "side_stream": 1 (default)
  * lets helper kernels of a call run on a second stream of the device, 0 keeps
  * everything on the caller's stream; "conv_compute": 0 (default) multiplies the
- * convolution's fp32 operands as they are, 1 rounds them to bf16 and accumulates
- * in fp32 (results about 2e-3 off), 2 splits every operand into two bf16 and
- * forms three bf16 products per multiply-add (results about 5e-6 off; an
- * infinity gives NaN);
- * "conv_fp32_split": 1 (default) lets fp32 products of large layers be formed
- * from three bf16 parts of every operand, six products of parts for one of
- * fp32, where that is faster (results as near to exact ones as the fp32
- * kernels'; tensors with infinities, NaN, subnormals, or whose products or
- * sums could come near the ends of the range, take those), 0 never, 2 wherever a product fits;
+ * convolution's operands with all of their 24 bits (see "conv_fp32_split"), 1
+ * rounds them to bf16 and accumulates in fp32 (results about 2e-3 off), 2
+ * splits every operand into two bf16 and forms three bf16 products per
+ * multiply-add (results about 5e-6 off; an infinity gives NaN);
+ * "conv_fp32_split": 1 (default) lets fp32 products of large layers whose sums
+ * have sixteen terms and more be formed from three bf16 parts of every operand,
+ * six products of parts for one of fp32, where that is faster (over dense sums
+ * nearer to exact results than the fp32 kernels; a result that a single
+ * product makes up is off by a unit of the last place at most instead of half
+ * of one; tensors with infinities, NaN, subnormals, or whose products or sums
+ * could come near the ends of the range, take the fp32 kernels as a whole: one
+ * such element changes the time of its call and the last bits of all of its
+ * results, those of other images too), 0 never, 2 wherever a product fits;
  * "roialign_tile_columns": 0 (default) lets the backward pass choose its tile
  * width from the size of the map, 56 or 28 fixes it; "roialign_row_split": 0
  * (default) lets it choose how many wavefronts share a tile row's work list,

@@ -924,14 +924,26 @@ bool gradients_b16(const conv::Geometry& g, const float* dy, const float* x, con
 
 // ---- fp32 products from three bf16 parts per operand ---------------------------------------
 //
-// An fp32 value is three bf16 exactly, and six products of parts make an fp32 product but for terms of 2^-26
-// of it; sums are fp32 as before, with fewer roundings.  The matrix cores do sixteen times the bf16
+// An fp32 value is three bf16 exactly, and six products of parts make an fp32 product but for terms of at most
+// 2^-24 of it (two of the second part by the third: 2^-8 and 2^-17 of their values at most; 2^-27 in the mean square); sums
+// are fp32 as before, with fewer roundings.  The matrix cores do sixteen times the bf16
 // products per clock, so six cost less than one of fp32; the parts are written by a pass over the
 // tensors first.  At 32 x 256 x 56 x 56, 256 filters 3 x 3: forward 911 -> 600 us, both gradients 1890 -> 1166
-// (the products 535 to 580 us, 1.2 to 1.3 PFLOP/s of bf16, what a large bf16 product of a library
-// reaches on this device; the passes 45 and 90), errors against 64 bits 5.0e-7 -> 2.9e-7 (3.3e-7 -> 2.5e-7
-// for the weights' gradient).  The fp32 kernels follow every such product and return at once unless a
+// (the products 500 to 520 us, 1.36 to 1.42 PFLOP/s of bf16; the passes 93 each), errors against 64 bits 5.0e-7 -> 2.9e-7
+// (3.3e-7 -> 2.5e-7 for the weights' gradient).  The fp32 kernels follow every such product and return at once unless a
 // tensor holds values the parts do not stand for (conv::SplitRange).
+
+// Fewest terms of a sum that is formed from parts by choice.  What is left out of a product (up to half a unit of
+// its last place) counts where no rounding of a longer sum exceeds it: errors of parts against 64 bits are 1.02-1.03 of
+// the fp32 kernels' with one term, 0.84 with two, 0.66, 0.53, 0.43 with four, eight, sixteen, 0.3 to 0.8 beyond (pointwise
+// layers of 16 x 128 x 128 pixels).
+constexpr long long kLeastTerms = 16;
+// Taps along an axis that a pixel of the data gradient meets at least, if any.
+int least_taps(int K, int dil, int stride) {
+  int common = dil, rest = stride;
+  while (rest != 0) { const int r = common % rest; common = rest; rest = r; }
+  return std::max(1, K / (stride / common));
+}
 
 // option "conv_fp32_split": 1 = where it pays (default), 0 = never, 2 = wherever a product fits
 int split_choice() { return mobula_hip::option("conv_fp32_split", 1); }
@@ -961,7 +973,8 @@ SplitChoice choose_split(const conv::Geometry& g, bool dx, bool dw);
 bool forward_split(const conv::Geometry& g, const float* x, const float* weight, const float* bias, float* y,
                    double fp32_cost, hipStream_t stream) {
   ForwardB16<3> f;
-  if (split_choice() != 2 && forward_fp32_us(fp32_cost) < kSplitOverhead) return false;
+  const long long taps = g.KH * g.KW;
+  if (split_choice() != 2 && (forward_fp32_us(fp32_cost) < kSplitOverhead || g.C * taps < kLeastTerms)) return false;
   if (f.plan(g, x, weight, bias, y) != kFits) return false;
   if (split_choice() != 2) {
     double product = 0.0;
@@ -969,7 +982,6 @@ bool forward_split(const conv::Geometry& g, const float* x, const float* weight,
     if (product + parts_us(static_cast<long long>(g.N) * g.C * g.H * g.W) + kSplitOverhead > forward_fp32_us(fp32_cost)) return false;
   }
   GatherPlan plan;
-  const long long taps = g.KH * g.KW;
   if (!plan_gather(&plan, "conv2d_forward", g, weight, g.D, g.C, static_cast<long long>(g.C) * g.H * g.W,
                    g.OH * g.OW, g.W, +1, g.C * taps, taps))
     return true;
@@ -1032,6 +1044,9 @@ bool gradients_split(const conv::Geometry& g, const float* dy, const float* x, c
 SplitChoice choose_split(const conv::Geometry& g, bool dx, bool dw) {
   if (split_choice() == 0 || g.N == 0 || g.N >= 65536) return SplitChoice{false, false};
   if (split_choice() == 2) return SplitChoice{dx, dw};
+  const long long met = static_cast<long long>(least_taps(g.KH, g.dil_h, g.stride_h)) * least_taps(g.KW, g.dil_w, g.stride_w);
+  dx = dx && g.D * met >= kLeastTerms;
+  dw = dw && static_cast<long long>(g.N) * g.OH * g.OW >= kLeastTerms;
   // (what the fp32 ways take at most: most small layers end here)
   const double most_dx = data_fp32_us(gathered_product_cost(g.C, g.D, g.KH * g.KW, static_cast<long long>(g.N) * g.H * g.W),
                                       static_cast<size_t>(g.stride_h) * g.stride_w);

@@ -658,7 +658,7 @@ def _three_products(geo, x, w, dy, dx0=None, dw0=None):
     (5, 20, 7, 9, 130, (5, 5), (6, 2), (1, 3), (1, 1)),      # padding beyond the kernel
 ])
 def test_fp32_products_of_three_parts(shape, split_always):
-    """fp32 products from three bf16 parts per operand: exact products but for 2^-26 of them, and at most six fp32
+    """fp32 products from three bf16 parts per operand: exact products but for at most 2^-24 of them, and at most six fp32
     roundings for sixteen of K, each of 2^-24 of a sum no larger than the result's own scale."""
     N, C, H, W, D, kernel, pad, stride, dil = shape
     g = torch.Generator().manual_seed(91)
@@ -745,3 +745,70 @@ def test_fp32_products_and_sums_that_overflow(place, a, b, split_always):
         for p, q, what in zip(got, _three_products(geo, x, w, dy), ('y', 'dx', 'dw')):
             assert torch.equal(p.isnan(), q.isnan()) and torch.equal(p.nan_to_num(0.0), q.nan_to_num(0.0)), what
             assert torch.equal(p.isinf(), q.isinf()), what
+
+
+def _errors_of_both_ways(shape):
+    """Errors (2-norm, relative) against 64 bits of y, dx and dw of a layer, from parts and by the fp32 kernels."""
+    N, C, H, W, D, kernel, pad, stride, dil = shape
+    g = torch.Generator().manual_seed(94)
+    x, w = torch.randn(N, C, H, W, generator=g), torch.randn(D, C, *kernel, generator=g)
+    xr, wr = x.double().requires_grad_(True), w.double().requires_grad_(True)
+    y_ref = F.conv2d(xr, wr, None, stride=stride, padding=pad, dilation=dil)
+    dy = torch.randn(y_ref.shape, generator=g)
+    y_ref.backward(dy.double())
+    geo = _ci(N, C, H, W, D, kernel[0], kernel[1], pad[0], pad[1], stride[0], stride[1], dil[0], dil[1])
+    errors = []
+    for option in 2, 0:
+        native.set_option('conv_fp32_split', option)
+        got = _three_products(geo, x.cuda(), w.cuda(), dy.cuda())
+        errors.append([((a.cpu().double() - b).norm() / b.norm()).item() for a, b in zip(got, (y_ref.detach(), xr.grad, wr.grad))])
+    return errors
+
+
+@pytest.mark.parametrize('shape', [
+    # N, C, H, W, D, kernel, pad, stride, dilation: sums of sixteen terms (y, dx, dw in turn) and of more
+    (4, 16, 24, 28, 64, (1, 1), (0, 0), (1, 1), (1, 1)),
+    (4, 64, 24, 28, 16, (1, 1), (0, 0), (1, 1), (1, 1)),
+    (1, 64, 4, 4, 130, (1, 1), (0, 0), (1, 1), (1, 1)),
+    (2, 48, 23, 17, 64, (3, 3), (1, 1), (2, 2), (1, 1)),     # dx: 64 to 256 terms
+    (4, 64, 24, 28, 256, (3, 3), (1, 1), (1, 1), (1, 1)),
+    (2, 256, 20, 21, 130, (5, 5), (2, 2), (1, 1), (1, 1)),
+])
+def test_sums_of_parts_are_no_further_off_than_the_fp32_kernels(shape, split_always):
+    for parts, fp32, what in zip(*_errors_of_both_ways(shape), ('y', 'dx', 'dw')):
+        assert parts <= fp32, (what, parts, fp32)
+
+
+def test_one_product_of_parts_is_within_two_half_units(split_always):
+    """What six products of parts leave out of one of fp32 is at most 2^-24 of it, and the result's rounding another
+    2^-24 (the fp32 kernels': the rounding alone)."""
+    N, D, P = 1, 64, 64 * 64
+    g = torch.Generator().manual_seed(95)
+    x, w = torch.rand(N, 1, 64, 64, generator=g) + 1, torch.rand(D, 1, 1, 1, generator=g) + 1
+    y = torch.empty(N, D, 64, 64, device='cuda')
+    xd, wd = x.cuda(), w.cuda()
+    _call('conv2d_forward_c6a7aa85', ctypes.c_int(y.numel()), _ptr(xd), _ptr(wd), _ptr(wd), ctypes.c_int(0),
+          *_ci(N, 1, 64, 64, D, 1, 1, 0, 0, 1, 1, 1, 1), _ptr(y))
+    want = w.double().reshape(D, 1) * x.double().reshape(1, P)
+    off = ((y.cpu().double().reshape(D, P) - want) / want).abs().max().item()
+    assert off <= 2.0 ** -23 * (1 + 2.0 ** -7), off
+
+
+@pytest.mark.parametrize('filters', [1, 2])
+def test_sums_of_a_few_terms_are_not_formed_from_parts_by_choice(filters):
+    """At a stride of two a pixel of dx meets one to four taps: parts, which would be faster, lose bits of such sums."""
+    N, C, H, W = 16, 64, 97, 99
+    geo = _ci(N, C, H, W, filters, 3, 3, 1, 1, 2, 2, 1, 1)
+    g = torch.Generator(device='cuda').manual_seed(96)
+    dy = torch.randn(N, filters, 49, 50, generator=g, device='cuda')
+    w = torch.randn(filters, C, 3, 3, generator=g, device='cuda')
+    out = []
+    try:
+        for option in 1, 0:
+            native.set_option('conv_fp32_split', option)
+            out.append(torch.empty(N, C, H, W, device='cuda'))
+            _call('conv2d_backward_data_ecf81c91', ctypes.c_int(out[-1].numel()), _ptr(dy), _ptr(w), ctypes.c_int(0), *geo,
+                  _ptr(out[-1]))
+    finally:
+        native.set_option('conv_fp32_split', 1)
+    assert torch.equal(*out)
