@@ -397,7 +397,7 @@ __device__ __forceinline__ unsigned pack_bf16(float lo, float hi) {
 //   kBf16x3: every operand split into a bf16 head and a bf16 tail (a = ah + al
 //            to 16 significant bits); ah*bh + ah*bl + al*bh on the bf16 matrix
 //            cores, fp32 accumulation: fp32-like results (about 1e-5) at three
-//            bf16 products, which is still a sixth of the fp32 matrix-core time.
+//            bf16 products, a fifth of the fp32 matrix-core time.
 enum Compute { kFp32 = 0, kBf16 = 1, kBf16x3 = 2 };
 
 // Workgroup id -> tile, for a launch of tile_blocks(count) workgroups.

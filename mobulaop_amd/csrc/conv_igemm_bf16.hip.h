@@ -51,9 +51,9 @@ constexpr int kBlockB16 = 16;
 template <int PARTS>
 constexpr int kUnits = PARTS == 1 ? 2 : PARTS;
 
-// Part `part` of v as bf16: the head (v rounded to bf16), what the head leaves rounded to bf16, and
-// what both leave.  Two parts carry sixteen significant bits of v, three all 24 of them
-// (each difference is exact in fp32; |v| above 2^-103, below which the last part is no normal bf16).
+// The parts of a value as bf16: its head (the value rounded to bf16), what the head leaves rounded to bf16, and
+// what both leave.  Two parts carry sixteen significant bits of a value, three all 24 of them
+// (each difference is exact in fp32; values above 2^-103, below which the last part is no normal bf16).
 // split_bf16 packs the next part of two values like pack_bf16 and leaves the rest in them.
 __device__ __forceinline__ unsigned split_bf16(float& lo, float& hi) {
   const unsigned packed = pack_bf16(lo, hi);
@@ -63,7 +63,7 @@ __device__ __forceinline__ unsigned split_bf16(float& lo, float& hi) {
 }
 
 // Which binary exponents occur among the values of a tensor, eight to a bit (bit e / 8 for the biased
-// exponent e); zeros have none.  Kept by the conversions to three parts, see in_split_range().
+// exponent e); zeros have none.  Kept by the conversions to three parts for SplitRange::inside().
 __device__ __forceinline__ unsigned exponent_bit(float v) {
   const unsigned bits = __float_as_uint(v);
   return (bits << 1) != 0u ? 1u << ((bits >> 26) & 31u) : 0u;

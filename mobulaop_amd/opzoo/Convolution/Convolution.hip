@@ -83,11 +83,11 @@ void launch_igemm_mode(const Ops& ops, float* piece_buffer, conv::SplitRange ran
 }
 
 template <typename Ops>
-void launch_igemm(const Ops& ops, float* piece_buffer, hipStream_t stream, conv::SplitRange range = {}) {
+void launch_igemm(const Ops& ops, float* piece_buffer, hipStream_t stream) {
   switch (compute_mode()) {
-    case conv::kBf16: launch_igemm_mode<Ops, conv::kBf16>(ops, piece_buffer, range, stream); break;
-    case conv::kBf16x3: launch_igemm_mode<Ops, conv::kBf16x3>(ops, piece_buffer, range, stream); break;
-    default: launch_igemm_mode<Ops, conv::kFp32>(ops, piece_buffer, range, stream);
+    case conv::kBf16: launch_igemm_mode<Ops, conv::kBf16>(ops, piece_buffer, {}, stream); break;
+    case conv::kBf16x3: launch_igemm_mode<Ops, conv::kBf16x3>(ops, piece_buffer, {}, stream); break;
+    default: launch_igemm_mode<Ops, conv::kFp32>(ops, piece_buffer, {}, stream);
   }
 }
 
@@ -928,10 +928,10 @@ bool gradients_b16(const conv::Geometry& g, const float* dy, const float* x, con
 // 2^-24 of it (two of the second part by the third: 2^-8 and 2^-17 of their values at most; 2^-27 in the mean square); sums
 // are fp32 as before, with fewer roundings.  The matrix cores do sixteen times the bf16
 // products per clock, so six cost less than one of fp32; the parts are written by a pass over the
-// tensors first.  At 32 x 256 x 56 x 56, 256 filters 3 x 3: forward 911 -> 600 us, both gradients 1890 -> 1166
-// (the products 500 to 520 us, 1.36 to 1.42 PFLOP/s of bf16; the passes 93 each), errors against 64 bits 5.0e-7 -> 2.9e-7
-// (3.3e-7 -> 2.5e-7 for the weights' gradient).  The fp32 kernels follow every such product and return at once unless a
-// tensor holds values the parts do not stand for (conv::SplitRange).
+// tensors first.  At 32 x 256 x 56 x 56, 256 filters 3 x 3: forward 915 -> 600 us, both gradients in one call 1900 -> 1170
+// (the products 500 to 540 us, 1.3 to 1.4 PFLOP/s of bf16 by the clock that a device holds; the passes 93 each), errors
+// against 64 bits 8.5e-7 -> 2.9e-7 (8.7e-7 -> 5.3e-7 for the weights' gradient).  The fp32 kernels follow every such
+// product and return at once unless a tensor holds values the parts do not stand for (conv::SplitRange).
 
 // Fewest terms of a sum that is formed from parts by choice.  What is left out of a product (up to half a unit of
 // its last place) counts where no rounding of a longer sum exceeds it: errors of parts against 64 bits are 1.02-1.03 of
@@ -953,7 +953,8 @@ constexpr size_t kWordBytes = 256;
 
 // Microseconds of the fp32 ways from the CU clocks of their kernels (which know nothing of rounds that are not full)
 // and of what the split ways take besides their products: the passes over the tensors, and the
-// launches that clear words and find nothing to do.  Fitted to some fifty layers of 10 us to 3 ms.
+// launches that clear words and find nothing to do.  Fitted to some fifty layers of 10 us to 3 ms; of 26 others
+// (profiles/conv2d_parts_or_fp32.txt) a product takes the way that is slower by 12 us or 8 % at most.
 double forward_fp32_us(double clocks) { return clocks / (256 * 2300.0) + 15.0; }
 double data_fp32_us(double clocks, size_t classes) {
   return clocks / (256 * 2300.0) + 15.0 * std::max<size_t>(classes, 1);
@@ -963,9 +964,9 @@ double parts_us(long long elements) { return elements * 10 / 4.0e6; }
 constexpr double kSplitOverhead = 28.0;
 
 // Which of the wanted products split operands are faster for: those of some thirty us and more whose channels and
-// filters fill the tiles (forward, fp32 against split: 25 x 416 x 55 x 56, 168 filters 3 x 3: 1180 -> 563 us;
-// 5 x 96 x 119 x 109, 256: 263 -> 182; 8 x 432 x 8 x 9, 384: 50 against 93; 23 x 256 x 72 x 64, 32: 221
-// against 236).
+// filters fill the tiles (forward, fp32 against split: 25 x 416 x 55 x 56, 168 filters 3 x 3: 1175 -> 640 us;
+// 5 x 96 x 119 x 109, 256: 280 -> 190; 8 x 432 x 8 x 9, 384: 50 against 91; 23 x 256 x 72 x 64, 32: 230
+// against 238).
 struct SplitChoice { bool dx, dw; };
 SplitChoice choose_split(const conv::Geometry& g, bool dx, bool dw);
 
