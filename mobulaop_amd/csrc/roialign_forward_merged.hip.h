@@ -17,7 +17,7 @@
 // on scheduling; they differ from the per-sample order of the reference by
 // rounding only.
 //
-// Bound by vector instructions and the L1 path about alike (4 x 512 x 100 x 100 fp16, 6000 boxes, 7 x 7: busy 80 % and 78 % of
+// Bound by vector instructions and the L1 path about alike (4 x 512 x 100 x 100 fp16, 6000 boxes, 7 x 7: busy 75 % and 73 % of
 // the time): a multiply-add per pixel and channel, a 16-byte load per pixel and eight channels.  What is not
 // one of these is kept out of the loops: lists end in entries that load nothing, so a column takes a read and an
 // add; a row's entry is fetched from a lane that holds it; both axes' lists are made in one go; grids of up to
@@ -32,8 +32,11 @@ namespace roialign {
 
 struct FwdMerged {
   static constexpr int LCAP = 28;   // entries per merged list: two a sample
-  // Samples merged per list at a time: all of a grid of up to 14, else 11 (grids of up to 22 in two windows; in windows of
-  // 14 they take 7 % longer: 3000 boxes with bins of up to 23 pixels on 8 x 96 x 160 x 160, 499 and 534 us).
+  // Samples merged per list at a time: all of a grid of up to 14, else 11.  Lists of 14 samples for both axes and the
+  // staging area are 10016 bytes of the 10240 that let sixteen wavefronts share a CU; with lists of 16 fifteen do, and grids
+  // of 15 and 16 take 17 to 28 % less, all others 3 to 12 % more.  A window of n samples meets n + 1 pixels: 11 fill
+  // three blocks of four columns (fp16, 1500 boxes of one size on 2 x 128 x 256 x 256, windows of 11 against 14: grids of
+  // 18 points 394 and 438 us, 22 522 and 576, 24, three windows against two, 703 and 638, 30 1016 and 1051).
   static constexpr int WHOLE = 14, WS = 11;
   static constexpr int RPH = 8;     // pooled rows whose lists are held at a time
   // One wavefront per workgroup: the wavefronts are independent, and a slot is refilled as soon
