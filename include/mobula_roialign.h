@@ -302,14 +302,18 @@ void mobula_hip_clear_error(void);
  * splits every operand into two bf16 and forms three bf16 products per
  * multiply-add (results about 5e-6 off; an infinity gives NaN);
  * "conv_fp32_split": 1 (default) lets fp32 products of large layers whose sums
- * have sixteen terms and more be formed from three bf16 parts of every operand,
- * six products of parts for one of fp32, where that is faster (over dense sums
- * nearer to exact results than the fp32 kernels; a result that a single
- * product makes up is off by a unit of the last place at most instead of half
- * of one; tensors with infinities, NaN, subnormals, or whose products or sums
- * could come near the ends of the range, take the fp32 kernels as a whole: one
- * such element changes the time of its call and the last bits of all of its
- * results, those of other images too), 0 never, 2 wherever a product fits;
+ * have sixteen terms and more be formed from parts of every operand where that
+ * is faster (over dense sums nearer to exact results than the fp32 kernels):
+ * three bf16 parts, six products of parts for one of fp32 (a result that a
+ * single product makes up is off by a unit of the last place at most instead of
+ * half of one), or, for sums of 512 terms and more, two fp16 parts and three
+ * products (four units at most; tensors whose values lie too far apart for
+ * that, below 2^-23 of the largest and with no larger one beside them, take
+ * three parts).  Tensors with infinities, NaN, subnormals, or whose products or
+ * sums could come near the ends of the range, take the fp32 kernels as a whole:
+ * one such element changes the time of its call and the last bits of all of its
+ * results, those of other images too.  0 never, 2 three parts wherever a product
+ * fits, 3 two fp16 parts wherever one fits;
  * "roialign_tile_columns": 0 (default) lets the backward pass choose its tile
  * width from the size of the map, 56 or 28 fixes it; "roialign_row_split": 0
  * (default) lets it choose how many wavefronts share a tile row's work list,

@@ -72,11 +72,14 @@ struct GatherStep {
 // either operand, the smallest two together at least 2^-100 (a product's last counted part is 2^-24 of it), and
 // the largest two small enough for a sum of as many terms as the product has.  (Where a sum overflows, the parts'
 // sums do so with either sign and give NaN for an infinity; just below, a head is rounded up past the end.)
-// Infinities and NaN are outside, so are subnormals.  The fp32 kernels take the product otherwise; both
+// Infinities and NaN are outside, so are subnormals.  Where halves are tried first (conv_igemm_bf16.hip.h), three parts
+// are next, if the operands' words keep them from halves.  The fp32 kernels take the product otherwise; all
 // are launched, and the tensors' words decide on the device which of them returns at once.
 struct SplitRange {
   const unsigned* a; const unsigned* b;   // exponent words of the operands; null: no choice to make
   int most;                               // what eight times the highest bits of both may come to (most_exponents)
+  // two fp16 parts are tried first: the operands' words of what keeps them from that, and which of its bits matter
+  const unsigned* halves_a; const unsigned* halves_b; unsigned halves_mask;
   // An operand whose highest bit is h lies below 2^(8 h + 8 - 127), parts and all; `terms` products of two, in six
   // products of parts that exceed them by a hundredth, stay below 2^128 while
   // 8 (ha + hb) + 16 - 254 + log2(terms) <= 127.
@@ -91,8 +94,9 @@ struct SplitRange {
     const int high_a = ea == 0u ? 0 : 31 - __builtin_clz(ea), high_b = eb == 0u ? 0 : 31 - __builtin_clz(eb);
     return (both & 0x80000007u) == 0u && 8 * (low_a + low_b) >= 2 * 127 - 100 && 8 * (high_a + high_b) <= most;
   }
-  __device__ bool leaves_split() const { return a != nullptr && !inside(); }
-  __device__ bool leaves_fp32() const { return a != nullptr && inside(); }
+  __device__ bool halves_hold() const { return halves_a != nullptr && ((*halves_a | *halves_b) & halves_mask) == 0u; }
+  __device__ bool leaves_split() const { return halves_hold() || (a != nullptr && !inside()); }
+  __device__ bool leaves_fp32() const { return halves_hold() || (a != nullptr && inside()); }
 };
 
 // What a gathered product reads besides the gathered tensor, in one launch: out[m][tap][c] =
@@ -106,11 +110,9 @@ struct GatherTables {
   int KW, dil_h, dil_w, row, sign;
   unsigned weight_blocks, step_blocks;
 };
-__global__ void __launch_bounds__(256)
-gather_tables_kernel(GatherTables t, SplitRange range) {
-  if (range.leaves_fp32()) return;
-  if (blockIdx.x >= t.weight_blocks) {
-    const int s = (blockIdx.x - t.weight_blocks) * 256 + threadIdx.x, per_tap = t.Cpad / 16;
+__device__ __forceinline__ void gather_tables(const GatherTables& t, unsigned block) {
+  if (block >= t.weight_blocks) {
+    const int s = (block - t.weight_blocks) * 256 + threadIdx.x, per_tap = t.Cpad / 16;
     if (s >= t.taps * per_tap) return;
     const int tap = s / per_tap, kh = tap / t.KW, kw = tap - kh * t.KW;
     t.steps[s] = GatherStep{kh * t.dil_h, kw * t.dil_w, t.sign * (kh * t.dil_h * t.row + kw * t.dil_w) * 4,
@@ -118,11 +120,14 @@ gather_tables_kernel(GatherTables t, SplitRange range) {
     return;
   }
   const long long total = static_cast<long long>(t.Mpad) * t.taps * t.Cpad;
-  const long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
+  const long long i = static_cast<long long>(block) * 256 + threadIdx.x;
   if (i >= total) return;
   const int c = static_cast<int>(i % t.Cpad), tap = static_cast<int>((i / t.Cpad) % t.taps);
   const int m = static_cast<int>(i / (static_cast<long long>(t.Cpad) * t.taps));
   t.out[i] = (m < t.M && c < t.C) ? t.w[m * t.stride_m + c * t.stride_c + tap] : 0.0f;
+}
+__global__ void __launch_bounds__(256) gather_tables_kernel(GatherTables t, SplitRange range) {
+  if (!range.leaves_fp32()) gather_tables(t, blockIdx.x);
 }
 
 // ---- operand functors -------------------------------------------------------
@@ -245,12 +250,16 @@ struct BackwardDataOps {
 // offset of the channel plane in x and the dilated tap position.
 struct Tap { int off; short dh, dw; };
 
-__global__ void __launch_bounds__(256)
-build_taps_kernel(Tap* __restrict__ taps, int count, int KH, int KW, int plane, int dil_h, int dil_w) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void build_taps(Tap* __restrict__ taps, int count, int KH, int KW, int plane, int dil_h,
+                                           int dil_w, unsigned block) {
+  const int k = block * 256 + threadIdx.x;
   if (k >= count) return;
   const int kw = k % KW, kh = (k / KW) % KH, ch = k / (KW * KH);
   taps[k] = Tap{ch * plane, static_cast<short>(kh * dil_h), static_cast<short>(kw * dil_w)};
+}
+__global__ void __launch_bounds__(256)
+build_taps_kernel(Tap* __restrict__ taps, int count, int KH, int KW, int plane, int dil_h, int dil_w) {
+  build_taps(taps, count, KH, KW, plane, dil_h, dil_w, blockIdx.x);
 }
 
 // xp[plane][pad_h + ih][pad_w + iw] = x[plane][ih][iw], zeros around: planes of (H + 2 pad_h) x

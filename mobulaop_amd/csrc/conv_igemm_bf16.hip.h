@@ -1,5 +1,5 @@
-// The convolution's three products with bf16 operands in memory: operands rounded to bf16, or fp32
-// operands as two or three bf16 parts each.
+// The convolution's three products with 16-bit operands in memory: operands rounded to bf16, or fp32
+// operands as two or three bf16 parts or two fp16 parts each.
 //
 // conv_igemm.hip.h can round or split fp32 operands on their way into LDS; that is bound by fetching the
 // fp32 operands (sixteen 4-byte loads per lane and K step) and converting them, not by the matrix cores.
@@ -18,6 +18,14 @@
 // memory once and from LDS once for up to three products; walking K once per pair of parts takes
 // twice the loads and reads.
 // Plain bf16 operands bring two units of sixteen a step.
+// Halves: an fp32 value, scaled by a power of two that its tensor has in common, as an fp16 head (11 bits) and 2^11 times
+// what that leaves as an fp16 tail: 23 bits and the sign of the tail, so a quarter of the values lose their last
+// bit.  Three products of parts for one of fp32 where three bf16 parts take six: the tails' with the heads go into sums of
+// their own, 2^11 times as large; what the two tails' product adds, 2^-22 of a product at most, is left out.
+// Sums of the heads' products start anew every sixteen K steps and are added up in fp32, so that a long sum is rounded at its
+// own size only once for 256 terms: 32 x 256 x 56 x 56, 256 filters 3 x 3: errors against 64 bits 2.85e-7 -> 1.43e-7 (weight
+// gradient 5.3 -> 1.7), products 500 -> 340 us each, forward and both gradients 1819 -> 1157.  The device's power bounds them
+// (265 us each for tensors of zeros; without any load 193, without LDS reads 250).
 //
 // The forward and the data gradient gather the right operand: K runs over the taps of a channel block,
 // the blocks one after the other, and a column is an output pixel, whose sixteen channels at a tap are 32
@@ -28,7 +36,7 @@
 //
 // A workgroup owns a tile of 256, 192, 128 or 64 rows x 256 columns: eight wavefronts, two down and four
 // across, two to a SIMD so that one multiplies while the other waits, accumulating 32 x 32
-// fragments of v_mfma_f32_32x32x16_bf16.  256 x 256 needs half the bytes per matrix instruction of 128 x 128.
+// fragments of v_mfma_f32_32x32x16_bf16 or _f16.  256 x 256 needs half the bytes per matrix instruction of 128 x 128.
 //
 // Operands go from memory straight into LDS (buffer loads with the LDS flag, 16 bytes per lane: one
 // instruction moves 1 KB), three or four stages deep.  No register staging, no LDS store instructions.
@@ -37,6 +45,8 @@
 // Replaces, like conv_igemm.hip.h, the per-image im2col + matrix product of
 // opzoo/Convolution/Convolution.py:17-57.
 #pragma once
+#include <type_traits>
+
 #include "conv_igemm.hip.h"
 
 namespace conv {
@@ -44,12 +54,17 @@ namespace conv {
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 // Channels of a block in memory, and of a unit of K.
 constexpr int kBlockB16 = 16;
+// How operands are kept (the template argument FORM of what follows): one, two or three bf16 parts, or two fp16 parts.
+constexpr int kHalves = 4;
+template <int FORM>
+constexpr int kParts = FORM == kHalves ? 2 : FORM;
 // Units of sixteen in a K step: the parts of the operands, or two blocks of one part each.
-template <int PARTS>
-constexpr int kUnits = PARTS == 1 ? 2 : PARTS;
+template <int FORM>
+constexpr int kUnits = FORM == 1 ? 2 : kParts<FORM>;
 
 // The parts of a value as bf16: its head (the value rounded to bf16), what the head leaves rounded to bf16, and
 // what both leave.  Two parts carry sixteen significant bits of a value, three all 24 of them
@@ -60,6 +75,22 @@ __device__ __forceinline__ unsigned split_bf16(float& lo, float& hi) {
   lo -= __uint_as_float(packed << 16);
   hi -= __uint_as_float(packed & 0xffff0000u);
   return packed;
+}
+
+// Two fp16 parts of a value: the value times 2^shift rounded to fp16, and 2^11 times what that leaves.
+constexpr int kTailShift = 11;
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef float pair_f32 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ unsigned split_f16(float& lo, float& hi) {
+  const f16x2 packed = __builtin_convertvector(pair_f32{lo, hi}, f16x2);
+  lo = (lo - static_cast<float>(packed[0])) * static_cast<float>(1 << kTailShift);
+  hi = (hi - static_cast<float>(packed[1])) * static_cast<float>(1 << kTailShift);
+  return __builtin_bit_cast(unsigned, packed);
+}
+template <int FORM>
+__device__ __forceinline__ unsigned split_pair(float& lo, float& hi) {
+  if constexpr (FORM == kHalves) return split_f16(lo, hi);
+  else return split_bf16(lo, hi);
 }
 
 // Which binary exponents occur among the values of a tensor, eight to a bit (bit e / 8 for the biased
@@ -80,6 +111,66 @@ __global__ void __launch_bounds__(64) clear_words_kernel(unsigned* words, int co
   if (static_cast<int>(threadIdx.x) < count) words[threadIdx.x] = 0u;
 }
 
+// Scaled values of an operand in two fp16 parts lie below 2^16.  Both parts hold all 24 bits but for the last one of a
+// quarter of the values from 2^-12 on; a smaller value is off by up to 2^-36.
+constexpr float kLeastHalf = 0x1p-12f, kMostHalf = 65504.0f;
+constexpr unsigned kBeyondHalves = 1u, kLonePixel = 2u, kLoneChannel = 4u, kSmallForHalves = 8u, kLargeHalf = 16u;
+__device__ __forceinline__ unsigned half_range(float scaled) {
+  const float v = fabsf(scaled);
+  return (v <= kMostHalf ? 0u : kBeyondHalves) | (v < kLeastHalf && v != 0.0f ? kSmallForHalves : 0u);
+}
+
+// What is known of a tensor: its word of exponents (three parts) or of what keeps it from two halves, and behind that the
+// binary exponent its values are scaled by; the largest magnitudes of its pieces.
+constexpr int kMagnitudes = 256;
+struct TensorWords {
+  unsigned* word; unsigned* exponents; const unsigned* magnitudes;
+  int headroom;   // binary places between the largest value that was looked at and the largest there may be
+  // the power of two that brings the largest value below 2^15 (every wavefront of a conversion finds it)
+  __device__ int shift(bool keep) const {
+    const u32x4 m = reinterpret_cast<const u32x4*>(magnitudes)[threadIdx.x & 63];
+    unsigned most = max(max(m[0], m[1]), max(m[2], m[3]));
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) most = max(most, static_cast<unsigned>(__shfl_xor(most, d)));
+    const int exponent = static_cast<int>(most >> 23);   // (0: zeros and subnormals)
+    const int by = __builtin_amdgcn_readfirstlane(most == 0u ? 0 : 14 - headroom + 127 - max(exponent, 1));
+    if (keep && threadIdx.x == 0) word[1] = static_cast<unsigned>(by);
+    return by;
+  }
+};
+
+// The magnitudes of up to three tensors (blockIdx.y), and their words cleared.
+struct MagnitudeJob { const float* src[3]; long long count[3]; TensorWords words[3]; };
+__global__ void __launch_bounds__(1024) magnitudes_kernel(MagnitudeJob job) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  __shared__ unsigned waves[16];
+  const int t = blockIdx.y, tid = threadIdx.x;
+  const float* const src = job.src[t];
+  const long long count = job.count[t];
+  unsigned most = 0u;
+  // (a workgroup takes sixteen KB at a time: all of them, or one of every eight)
+  const int every = job.words[t].headroom == 0 ? 1 : 8;
+  const long long quads = reinterpret_cast<uintptr_t>(src) % 16 == 0 ? count / 4 : 0;
+  for (long long piece = blockIdx.x;; piece += kMagnitudes) {
+    const long long i = (piece * every + piece % every) * 1024 + tid;
+    if (i >= quads) break;
+    const f32x4 v = reinterpret_cast<const f32x4*>(src)[i];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) most = max(most, __float_as_uint(v[j]) & 0x7fffffffu);
+  }
+  for (long long i = 4 * quads + static_cast<long long>(blockIdx.x) * 1024 + tid; i < count; i += kMagnitudes * 1024)
+    most = max(most, __float_as_uint(src[i]) & 0x7fffffffu);
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) most = max(most, static_cast<unsigned>(__shfl_xor(most, d)));
+  if ((tid & 63) == 0) waves[tid >> 6] = most;
+  __syncthreads();
+  if (tid == 0) {
+    for (int w = 1; w < 16; ++w) most = max(most, waves[w]);
+    const_cast<unsigned*>(job.words[t].magnitudes)[blockIdx.x] = most;
+    if (blockIdx.x == 0) { *job.words[t].word = 0u; *job.words[t].exponents = 0u; }
+  }
+}
+
 // dst[part][n][c / 16][p][c % 16] = part `part` of src[n][c][p] for c < C, zero for C <= c < Cpad, the
 // parts `part` halves apart.  One workgroup: 64 pixels x 64 channels (four channel blocks) through LDS.  VEC: P
 // is a multiple of four and src 16-byte aligned, a lane reads four pixels at a time.  The source is
@@ -93,8 +184,8 @@ struct BlockedJob {
 
 constexpr int kPrepLdsWords = 64 * 65;   // what a job of prepare_b16_kernel finds in LDS
 
-template <int PARTS, bool VEC>
-__device__ __forceinline__ void to_blocked_bf16(const BlockedJob& job, unsigned block, float* lds, unsigned* exponents) {
+template <int FORM, bool VEC>
+__device__ __forceinline__ void to_blocked(const BlockedJob& job, unsigned block, float* lds, const TensorWords& words) {
   typedef float f32x4 __attribute__((ext_vector_type(4)));
   float (*const tile)[65] = reinterpret_cast<float (*)[65]>(lds);
   const int C = job.C, Cpad = job.Cpad, P = job.P;
@@ -104,6 +195,7 @@ __device__ __forceinline__ void to_blocked_bf16(const BlockedJob& job, unsigned 
   const unsigned row = block / job.tiles_p;
   const int n = row / job.tiles_c, c0 = (row - n * job.tiles_c) * 64, p0 = (block - row * job.tiles_p) * 64;
   const float* in = src + static_cast<size_t>(n) * C * P;
+  const int shift = FORM == kHalves ? words.shift(block == 0) : 0;
   if (VEC) {
     const int q = threadIdx.x & 15, r = threadIdx.x >> 4;   // 16 quads of pixels, 16 channels per pass
 #pragma unroll
@@ -135,19 +227,42 @@ __device__ __forceinline__ void to_blocked_bf16(const BlockedJob& job, unsigned 
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         f[j] = tile[cl + j][pl];
-        if (PARTS == 3) seen |= exponent_bit(f[j]);
+        if (FORM == 3) seen |= exponent_bit(f[j]);
+        if (FORM == kHalves) {
+          f[j] = ldexpf(f[j], shift);
+          seen |= half_range(f[j]);
+        }
       }
       unsigned short* const to = dst + ((static_cast<size_t>(n) * (Cpad / B) + c / B) * P + p) * B + 8 * cq;
 #pragma unroll
-      for (int part = 0; part < PARTS; ++part) {
+      for (int part = 0; part < kParts<FORM>; ++part) {
         u32x4 v;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = split_bf16(f[2 * j], f[2 * j + 1]);
+        for (int j = 0; j < 4; ++j) v[j] = split_pair<FORM>(f[2 * j], f[2 * j + 1]);
         *reinterpret_cast<u32x4*>(to + part * job.part) = v;
       }
     }
   }
-  if (PARTS == 3) add_exponents(exponents, seen);
+  if (FORM == 3) add_exponents(words.exponents, seen);
+  if (FORM == kHalves && __any(seen != 0u)) {
+    // a value that is small for the tensor does no harm where a larger one stands beside it: at its pixel for a sum
+    // over channels, in its channel for a sum over pixels
+    unsigned bad = seen & kBeyondHalves;
+    if (seen & kSmallForHalves) {
+      for (int k = 0; k < 2; ++k)
+        for (int j = 0; j < 8; ++j) {
+          const int cl = B * (2 * k + first) + 8 * cq + j;
+          if ((half_range(ldexpf(tile[cl][pl], shift)) & kSmallForHalves) == 0u) continue;
+          bool pixel = false, channel = false;
+          for (int i = 0; i < 64 && !(pixel && channel); ++i) {
+            pixel |= fabsf(ldexpf(tile[i][pl], shift)) >= kLeastHalf;
+            channel |= fabsf(ldexpf(tile[cl][i], shift)) >= kLeastHalf;
+          }
+          bad |= (pixel ? 0u : kLonePixel) | (channel ? 0u : kLoneChannel);
+        }
+    }
+    add_exponents(words.word, bad);
+  }
 }
 
 // The weights of a gathered product as they lie in LDS step by step.  Two or three parts: out[(c / 16) * taps +
@@ -159,48 +274,92 @@ struct ArrangeJob {
   unsigned blocks;
 };
 
-template <int PARTS>
-__device__ __forceinline__ void arrange_weights_bf16(const ArrangeJob& job, unsigned block, unsigned* exponents) {
-  constexpr int B = kBlockB16, BLOCKS = PARTS == 1 ? 2 : 1;   // channel blocks of a step
+template <int FORM>
+__device__ __forceinline__ void arrange_weights(const ArrangeJob& job, unsigned block, const TensorWords& words) {
+  constexpr int B = kBlockB16, BLOCKS = FORM == 1 ? 2 : 1, PARTS = kParts<FORM>;   // channel blocks of a step
   const long long total = static_cast<long long>(job.Mpad) * job.taps * job.Cpad / 2;   // pairs of channels
   const long long i = static_cast<long long>(block) * 256 + threadIdx.x;
   unsigned seen = 0u;
+  const int shift = FORM == kHalves ? words.shift(block == 0) : 0;
   if (i < total) {
     const int j = 2 * static_cast<int>(i % (B / 2)), m = static_cast<int>((i / (B / 2)) % job.Mpad);
     const int q = static_cast<int>(i / (B / 2 * static_cast<long long>(job.Mpad)));   // (step, block of the step)
     const int s = q / BLOCKS, cb = s / job.taps, tap = s - cb * job.taps, c = (cb * BLOCKS + q % BLOCKS) * B + j;
     float lo = (m < job.M && c < job.C) ? job.w[m * job.stride_m + c * job.stride_c + tap] : 0.0f;
     float hi = (m < job.M && c + 1 < job.C) ? job.w[m * job.stride_m + (c + 1) * job.stride_c + tap] : 0.0f;
-    seen = exponent_bit(lo) | exponent_bit(hi);
+    if (FORM == 3) seen = exponent_bit(lo) | exponent_bit(hi);
+    if (FORM == kHalves) {
+      lo = ldexpf(lo, shift); hi = ldexpf(hi, shift);
+      seen = half_range(lo) | half_range(hi) | (fmaxf(fabsf(lo), fabsf(hi)) >= kLeastHalf ? kLargeHalf : 0u);
+    }
     unsigned* const to = reinterpret_cast<unsigned*>(job.out) +
                          (static_cast<size_t>(q) * PARTS * job.Mpad + m) * (B / 2) + j / 2;
 #pragma unroll
-    for (int part = 0; part < PARTS; ++part) to[static_cast<size_t>(part) * job.Mpad * (B / 2)] = split_bf16(lo, hi);
+    for (int part = 0; part < PARTS; ++part) to[static_cast<size_t>(part) * job.Mpad * (B / 2)] = split_pair<FORM>(lo, hi);
   }
-  if (PARTS == 3) add_exponents(exponents, seen);
+  if (FORM == 3) add_exponents(words.exponents, seen);
+  if (FORM == kHalves && __any((seen & ~kLargeHalf) != 0u)) {
+    // (the eight lanes of a filter's sixteen channels at a tap look at each other)
+#pragma unroll
+    for (int d = 1; d < B / 2; d <<= 1) seen |= __shfl_xor(seen, d);
+    add_exponents(words.word, (seen & kBeyondHalves) |
+                                  ((seen & (kSmallForHalves | kLargeHalf)) == kSmallForHalves ? kLonePixel | kLoneChannel : 0u));
+  }
 }
 
 // Everything a call's products need, in one launch: the jobs do not depend on each other, and a small
 // layer's conversions take less time than their launches (a job with blocks == 0 is absent).
-// exponents (PARTS == 3): the words of the tensors the jobs read.
-struct ExponentWords { unsigned* weights; unsigned* first; unsigned* second; };
-template <int PARTS>
+// exponents (three parts, halves): the words of the tensors the jobs read.
+struct ExponentWords { TensorWords weights, first, second; };
+template <int FORM>
 __global__ void __launch_bounds__(256)
 prepare_b16_kernel(ArrangeJob weights, BlockedJob first, BlockedJob second, ExponentWords exponents) {
   __shared__ __attribute__((aligned(16))) float lds[kPrepLdsWords];
   unsigned block = blockIdx.x;
   if (block < first.blocks) {
-    if (first.vec) to_blocked_bf16<PARTS, true>(first, block, lds, exponents.first);
-    else to_blocked_bf16<PARTS, false>(first, block, lds, exponents.first);
+    if (first.vec) to_blocked<FORM, true>(first, block, lds, exponents.first);
+    else to_blocked<FORM, false>(first, block, lds, exponents.first);
     return;
   }
   block -= first.blocks;
   if (block < second.blocks) {
-    if (second.vec) to_blocked_bf16<PARTS, true>(second, block, lds, exponents.second);
-    else to_blocked_bf16<PARTS, false>(second, block, lds, exponents.second);
+    if (second.vec) to_blocked<FORM, true>(second, block, lds, exponents.second);
+    else to_blocked<FORM, false>(second, block, lds, exponents.second);
     return;
   }
-  arrange_weights_bf16<PARTS>(weights, block - second.blocks, exponents.weights);
+  arrange_weights<FORM>(weights, block - second.blocks, exponents.weights);
+}
+
+// The same for products that turn out not to be formed from halves: the three parts of their operands, and the tables of
+// the fp32 kernels behind those.
+struct TapsJob { Tap* taps; int count, KH, KW, plane, dil_h, dil_w; unsigned blocks; };
+__global__ void __launch_bounds__(256)
+prepare_again_kernel(ArrangeJob weights, BlockedJob first, BlockedJob second, ExponentWords exponents, GatherTables tables,
+                     TapsJob taps, SplitRange range, SplitRange other) {
+  if (range.halves_hold() && (other.halves_a == nullptr || other.halves_hold())) return;
+  __shared__ __attribute__((aligned(16))) float lds[kPrepLdsWords];
+  unsigned block = blockIdx.x;
+  if (block < first.blocks) {
+    to_blocked<3, false>(first, block, lds, exponents.first);
+    return;
+  }
+  block -= first.blocks;
+  if (block < second.blocks) {
+    to_blocked<3, false>(second, block, lds, exponents.second);
+    return;
+  }
+  block -= second.blocks;
+  if (block < weights.blocks) {
+    arrange_weights<3>(weights, block, exponents.weights);
+    return;
+  }
+  block -= weights.blocks;
+  if (block < tables.weight_blocks + tables.step_blocks) {
+    gather_tables(tables, block);
+    return;
+  }
+  block -= tables.weight_blocks + tables.step_blocks;
+  if (block < taps.blocks) build_taps(taps.taps, taps.count, taps.KH, taps.KW, taps.plane, taps.dil_h, taps.dil_w, block);
 }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of_bytes(const void* base, unsigned bytes) {
@@ -219,21 +378,24 @@ constexpr int kFarOutside = -(1 << 30);
 //     scalar one of 32 rows from m on;
 //   b_buffer(n0) / b_at(lane, unit) / b_from(unit): the right one, of the 32 columns of the wavefront
 //     (with the bit of kDead set: zeros; written as an or, so that no branch forms in the tile's loop);
-//   Column column(n) / store(column, m, v): where results of column n go.
+//   Column column(n) / store(column, m, v): where results of column n go; plain(): nothing is added to a result on
+//     its way out, which may be written at column.p + m * row_pitch().
 
 // A K step of a gathered product as (filter row, filter column, channel block); wavefront-uniform, kept in
 // scalar registers.
 struct StepCursor { int kh, kw, cb; };
 
 // What the gathered products have in common: the weights and the walk over K.
-template <int PARTS_>
+template <int FORM_>
 struct GatheredB16 {
-  static constexpr int PARTS = PARTS_, UNITS = kUnits<PARTS>, BLOCKS = PARTS == 1 ? 2 : 1;   // channel blocks of a step
+  static constexpr int FORM = FORM_, PARTS = kParts<FORM>, UNITS = kUnits<FORM>, BLOCKS = FORM == 1 ? 2 : 1;   // channel blocks of a step
   static constexpr bool kPixels = false;
   const unsigned short* __restrict__ wp;    // [K steps][UNITS][mpad][16]
   const unsigned short* __restrict__ src;   // [PARTS][images][cpad / 16][pixels][16]
   Geometry g; int M, Ncols, cpad, mpad;
   int source_part;                          // bytes from one part of the source to the next
+  const unsigned* weight_word; const unsigned* src_word;   // (halves: the operands' words)
+  __device__ int shift() const { return static_cast<int>(weight_word[1]) + static_cast<int>(src_word[1]); }
   __host__ __device__ int k_steps() const { return g.KH * g.KW * (cpad / (16 * BLOCKS)); }
   __device__ __amdgpu_buffer_rsrc_t a_buffer() const {
     return buffer_of_bytes(wp, static_cast<unsigned>(k_steps()) * UNITS * mpad * 32u);
@@ -266,9 +428,9 @@ __device__ __forceinline__ int lane_row() { return (threadIdx.x & 63) >> 1; }
 __device__ __forceinline__ int lane_chunk() { return (threadIdx.x & 1) ^ ((threadIdx.x >> 4) & 1); }
 
 // y[img, d, oh, ow] = bias[d] + sum over (c, kh, kw) of W[d, c, kh, kw] * x[img, c, ih, iw]
-template <int PARTS>
-struct ForwardOpsB16 : GatheredB16<PARTS> {
-  using Base = GatheredB16<PARTS>;
+template <int FORM>
+struct ForwardOpsB16 : GatheredB16<FORM> {
+  using Base = GatheredB16<FORM>;
   using Base::g; using Base::M; using Base::Ncols; using Base::cpad;
   const float* __restrict__ bias; float* __restrict__ y;
   struct Lane { StepCursor k; int anchor, ih0, iw0; };   // (a column past the last: ih0 far outside)
@@ -296,11 +458,13 @@ struct ForwardOpsB16 : GatheredB16<PARTS> {
                     (static_cast<unsigned>(iw) < static_cast<unsigned>(g.W));
     return (l.anchor + l.k.cb * Base::BLOCKS * plane_bytes() + (dh * g.W + dw) * 32) | (in ? 0 : kDead);
   }
-  __device__ int b_from(int unit) const { return unit * (PARTS == 1 ? plane_bytes() : Base::source_part); }
+  __device__ int b_from(int unit) const { return unit * (FORM == 1 ? plane_bytes() : Base::source_part); }
   __device__ Column column(int n) const {
     const int ohw = g.OH * g.OW, img = n / ohw, r = n - img * ohw;
     return Column{y + static_cast<size_t>(img) * g.D * ohw + r, n < Ncols};
   }
+  __device__ bool plain() const { return bias == nullptr; }
+  __device__ size_t row_pitch() const { return static_cast<size_t>(g.OH) * g.OW; }
   __device__ void store(const Column& c, int m, float v) const {
     if (m < M && c.ok) c.p[static_cast<size_t>(m) * (g.OH * g.OW)] = bias != nullptr ? v + bias[m] : v;
   }
@@ -308,9 +472,9 @@ struct ForwardOpsB16 : GatheredB16<PARTS> {
 
 // dx[img, c, ih, iw] = sum over (d, kh, kw) of W[d, c, kh, kw] * dy[img, d, oh, ow]
 // with oh * stride = ih + pad - kh * dil (and likewise for columns).
-template <int PARTS>
-struct BackwardDataOpsB16 : GatheredB16<PARTS> {
-  using Base = GatheredB16<PARTS>;
+template <int FORM>
+struct BackwardDataOpsB16 : GatheredB16<FORM> {
+  using Base = GatheredB16<FORM>;
   using Base::g; using Base::M; using Base::Ncols; using Base::cpad;
   float* __restrict__ dx; int accumulate;
   struct Lane { StepCursor k; int anchor, ihp, iwp; };   // (a column past the last: ihp far outside)
@@ -346,11 +510,13 @@ struct BackwardDataOpsB16 : GatheredB16<PARTS> {
                     (oh < g.OH) & (ow < g.OW);
     return (l.anchor + block + (oh * g.OW + ow) * 32) | (in ? 0 : kDead);
   }
-  __device__ int b_from(int unit) const { return unit * (PARTS == 1 ? plane_bytes() : Base::source_part); }
+  __device__ int b_from(int unit) const { return unit * (FORM == 1 ? plane_bytes() : Base::source_part); }
   __device__ Column column(int n) const {
     const int hw = g.H * g.W, img = n / hw, r = n - img * hw;
     return Column{dx + static_cast<size_t>(img) * g.C * hw + r, n < Ncols};
   }
+  __device__ bool plain() const { return !accumulate; }
+  __device__ size_t row_pitch() const { return static_cast<size_t>(g.H) * g.W; }
   __device__ void store(const Column& c, int m, float v) const {
     if (m >= M || !c.ok) return;
     float* p = c.p + static_cast<size_t>(m) * (g.H * g.W);
@@ -363,15 +529,17 @@ struct BackwardDataOpsB16 : GatheredB16<PARTS> {
 // instruction brings two blocks of rows (or columns) at sixteen pixels, 32 bytes each: of the block of
 // even lane halves in order, of the other with the fours of a pixel's number swapped pairwise (pixel p in
 // place p ^ 4), so that the transposed reads of both together meet every bank once.
-template <int PARTS_>
+template <int FORM_>
 struct WeightGradOpsB16 {
-  static constexpr int PARTS = PARTS_, UNITS = kUnits<PARTS>, STEP = PARTS == 1 ? 32 : 16;   // pixels of a step
+  static constexpr int FORM = FORM_, PARTS = kParts<FORM>, UNITS = kUnits<FORM>, STEP = FORM == 1 ? 32 : 16;   // pixels of a step
   static constexpr bool kPixels = true;
   const unsigned short* __restrict__ dys;   // [PARTS][N][dblocks][OH * OW][16]
   const unsigned short* __restrict__ xs;    // [PARTS][N][cblocks][H * W][16]
   float* __restrict__ dw;
   Geometry g; int M, Ncols, dblocks, cblocks, ctiles, accumulate;   // Ncols = KH * KW * ctiles * 16: channel blocks with channels
   int step_n, step_h, step_w;   // a step of pixels as images, rows and columns
+  const unsigned* dy_word; const unsigned* x_word;   // (halves: the operands' words)
+  __device__ int shift() const { return static_cast<int>(dy_word[1]) + static_cast<int>(x_word[1]); }
   struct Pixel { int n, oh, ow; };
   static constexpr int PIXELS = PARTS == 1 ? 2 : 1;
   struct Lane { Pixel p[PIXELS]; int a, b, dh, dw; };   // (a column past the last: dh far outside)
@@ -429,6 +597,8 @@ struct WeightGradOpsB16 {
     const int nb = n / 16, tap = nb / ctiles, c = (nb - tap * ctiles) * 16 + n % 16;
     return Column{dw + static_cast<size_t>(c) * (g.KH * g.KW) + tap, n < Ncols && c < g.C};
   }
+  __device__ bool plain() const { return !accumulate; }
+  __device__ size_t row_pitch() const { return static_cast<size_t>(g.C) * (g.KH * g.KW); }
   __device__ void store(const Column& c, int m, float v) const {
     if (m >= M || !c.ok) return;
     float* p = c.p + static_cast<size_t>(m) * g.C * (g.KH * g.KW);
@@ -464,12 +634,12 @@ __device__ __forceinline__ void workgroup_barrier() {
 // with one, 184 with two; with three parts the stages of two would be two deep: 267 filters 7 x 7 over
 // 28 x 48 x 47 x 52, data gradient 597 us with one, 800 with two).  At most 128 rows with three parts: two sets of
 // accumulators.
-template <int ROWS_, int PARTS>
+template <int ROWS_, int FORM>
 struct ShapeB16 {
-  static constexpr int PER_CU = ROWS_ <= 128 && PARTS < 3 ? 2 : 1;
-  static constexpr int STAGES = PARTS == 3 || PER_CU == 2 ? 3 : 4;
+  static constexpr int PER_CU = ROWS_ <= 128 && FORM < 3 ? 2 : 1;
+  static constexpr int STAGES = FORM == 3 || PER_CU == 2 ? 3 : 4;
   static constexpr int ROWS = ROWS_, COLS = 256, WAVES = 8, WM = 2, WN = 4, NI = ROWS / 64, NJ = 2;
-  static_assert(ROWS % 64 == 0 && ROWS <= (PARTS == 3 ? 128 : 256), "two wavefronts down, fragments of 32 rows");
+  static_assert(ROWS % 64 == 0 && ROWS <= (FORM >= 3 ? 128 : 256), "two wavefronts down, fragments of 32 rows");
 };
 
 // The products of a K step: which units of the operands they multiply, smallest parts first, and how
@@ -477,12 +647,14 @@ struct ShapeB16 {
 // read last, so that nothing of the stage is still to come from LDS at the barrier; with one part the second unit is
 // read under the only product before the barrier and waited for (32 x 256 x 56 x 56, 256 filters 3 x 3, forward and both
 // gradients: 446 us a step, 446 too with the reads in the product's first half).
-template <int PARTS>
+template <int FORM>
 struct ProductsB16;
 template <>
 struct ProductsB16<1> { static constexpr int COUNT = 2, BEFORE = 1, A[] = {0, 1}, B[] = {0, 1}; };
 template <>
 struct ProductsB16<2> { static constexpr int COUNT = 3, BEFORE = 2, A[] = {1, 0, 0}, B[] = {0, 1, 0}; };
+template <>
+struct ProductsB16<kHalves> : ProductsB16<2> {};
 template <>
 struct ProductsB16<3> { static constexpr int COUNT = 6, BEFORE = 3, A[] = {2, 0, 1, 1, 0, 0}, B[] = {0, 2, 1, 0, 1, 0}; };
 
@@ -492,7 +664,7 @@ struct ProductsB16<3> { static constexpr int COUNT = 6, BEFORE = 3, A[] = {2, 0,
 template <typename Ops, typename S>
 __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, int s_begin, int s_end,
                                                float* __restrict__ piece) {
-  using P = ProductsB16<Ops::PARTS>;
+  using P = ProductsB16<Ops::FORM>;
   constexpr int UNITS = Ops::UNITS, ROWS = S::ROWS, WAVES = S::WAVES, NI = S::NI, NJ = S::NJ;
   // a load instruction moves 32 rows x 32 bytes; those of the left operand past its rows bring zeros
   constexpr int A_PIECES = UNITS * ROWS / 32, A_LOADS = (A_PIECES + WAVES - 1) / WAVES, LOADS = A_LOADS + UNITS;
@@ -522,7 +694,7 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
                                                ops.a_from(s_issue < s_end ? s_issue : 0, unit, m0 + 32 * group), 0, 0);
     } else {
       const int unit = k - A_LOADS;
-      if (unit == 0 || (Ops::kPixels && Ops::PARTS == 1)) b_off = ops.b_at(state, unit) | dead;
+      if (unit == 0 || (Ops::kPixels && Ops::FORM == 1)) b_off = ops.b_at(state, unit) | dead;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(b_buf, base + A_HALVES + (unit * S::COLS + 32 * wave) * 16, 16, b_off,
                                                ops.b_from(unit), 0, 0);
     }
@@ -534,10 +706,11 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
   };
 
   bf16x8 fa[UNITS][NI], fb[UNITS][NJ], next_b[NJ];
-  // With three parts the heads' product has accumulators of its own: a rounding of the long sums for every sixteen of K
-  // (the fp32 instruction: eight), those of the others' sums are 2^-8 of them.
-  constexpr int SUMS = UNITS == 3 ? 2 : 1;
-  float16v acc[SUMS][NI][NJ];
+  // With three parts and with halves the heads' product has accumulators of its own: a rounding of the long sums for every
+  // sixteen of K (the fp32 instruction: eight), those of the others' sums are 2^-8 (halves: 2^-11) of them.
+  constexpr bool HALVES = Ops::FORM == kHalves;
+  constexpr int SUMS = UNITS == 3 || HALVES ? 2 : 1;
+  float16v acc[SUMS][NI][NJ], total[HALVES ? NI : 1][HALVES ? NJ : 1];
 #pragma unroll
   for (int q = 0; q < SUMS; ++q)
 #pragma unroll
@@ -545,10 +718,17 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
 #pragma unroll
       for (int j = 0; j < NJ; ++j)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[q][i][j][v] = 0.0f;
+        for (int v = 0; v < 16; ++v) {
+          acc[q][i][j][v] = 0.0f;
+          if constexpr (HALVES) total[i][j][v] = 0.0f;
+        }
   auto multiply = [&](int p, int i, int j) {
     float16v& sum = acc[SUMS == 2 && p == P::COUNT - 1 ? 1 : 0][i][j];
-    sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[P::A[p]][i], fb[P::B[p]][j], sum, 0, 0, 0);
+    if constexpr (HALVES)
+      sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, fa[P::A[p]][i]),
+                                                   __builtin_bit_cast(f16x8, fb[P::B[p]][j]), sum, 0, 0, 0);
+    else
+      sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[P::A[p]][i], fb[P::B[p]][j], sum, 0, 0, 0);
   };
 
   // ---- reading (offsets in halves): a fragment is row `col` of 32, its eight k of `half` ----
@@ -600,7 +780,26 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
   for (int i = 0; i < NI; ++i) fa[A_FIRST][i] = read_a(0, A_FIRST, i);
 #pragma unroll
   for (int j = 0; j < NJ; ++j) fb[0][j] = read_b(0, 0, j);
+  // Halves: the sums of the heads' products move into `total` after sixteen steps (eight where the sum is short: 1.30e-7 ->
+  // 1.20e-7 over 25 steps); of two wavefronts on a SIMD one does so half a chunk before the other, which multiplies
+  // meanwhile.  (In the loop's one body: a second one for the step that moves them spilled, 417 against 340 us.)
+  const int chunk = s_end - s_begin < 64 ? 8 : 16;
+  int s_move = s_begin + (wave < WAVES / 2 ? chunk : chunk / 2);
   for (int s = s_begin; s < s_end; ++s) {
+    if constexpr (HALVES) {
+      if (s == s_move) {
+        s_move += chunk;
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+              total[i][j][v] += acc[1][i][j][v];
+              acc[1][i][j][v] = 0.0f;
+            }
+      }
+    }
     const int next = stage + 1 == STAGES ? 0 : stage + 1;
 #pragma unroll
     for (int p = 0; p < P::BEFORE; ++p)
@@ -644,14 +843,36 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
 #pragma unroll
     for (int i = 0; i < NI; ++i)
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) acc[0][i][j] += acc[1][i][j];
+      for (int j = 0; j < NJ; ++j) {
+        if constexpr (HALVES) {
+          // (the pieces of a sum are added in the scaled operands' range)
+          const int by = piece == nullptr ? -ops.shift() : 0;
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            acc[0][i][j][v] = ldexpf(total[i][j][v] + acc[1][i][j][v] + acc[0][i][j][v] * (1.0f / (1 << kTailShift)), by);
+        } else {
+          acc[0][i][j] += acc[1][i][j];
+        }
+      }
   }
 
-  // accumulator register v of a lane: row 8 * (v / 4) + 4 * (lane / 32) + v % 4, column lane % 32
+  // accumulator register v of a lane: row 8 * (v / 4) + 4 * (lane / 32) + v % 4, column lane % 32.  Results of a tile
+  // whose rows all exist and that nothing is added to leave by one address and one store each.
+  const bool all_rows = m0 + ROWS <= ops.M, plain = all_rows && (piece != nullptr || ops.plain());
+  const size_t pitch = piece != nullptr ? S::COLS : ops.row_pitch();
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     const int column = wn + j * 32 + col;
-    if (piece != nullptr) {
+    const typename Ops::Column out = ops.column(n0 + column);
+    if (plain) {
+      float* const p = (piece != nullptr ? piece + column : out.p + m0 * pitch) + (wm + 4 * half) * pitch;
+      if (piece != nullptr ? n0 + column < ops.Ncols : out.ok) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) p[(i * 32 + 8 * (v >> 2) + (v & 3)) * pitch] = acc[0][i][j][v];
+      }
+    } else if (piece != nullptr) {
 #pragma unroll
       for (int i = 0; i < NI; ++i)
 #pragma unroll
@@ -660,7 +881,6 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
           if (m0 + row < ops.M && n0 + column < ops.Ncols) piece[row * S::COLS + column] = acc[0][i][j][v];
         }
     } else {
-      const typename Ops::Column out = ops.column(n0 + column);
 #pragma unroll
       for (int i = 0; i < NI; ++i)
 #pragma unroll
@@ -675,7 +895,7 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
 template <typename Ops, typename S>
 __global__ void __launch_bounds__(64 * S::WAVES, 2 * S::PER_CU)
 igemm_b16_kernel(Ops ops, int row_tiles, TileSplit split, float* __restrict__ piece_buffer, SplitRange range) {
-  if (range.leaves_split()) return;
+  if (Ops::FORM == kHalves ? !range.halves_hold() : range.leaves_split()) return;
   const int whole_blocks = tile_blocks(split.whole);
   int t, s_begin = 0, s_end = ops.k_steps();
   float* piece = nullptr;
@@ -701,7 +921,7 @@ struct PiecesB16 {
 };
 template <typename Ops>
 __device__ __forceinline__ void reduce_row_b16(const Ops& ops, const PiecesB16& p, unsigned block) {
-  if (p.range.leaves_split()) return;
+  if (Ops::FORM == kHalves ? !p.range.halves_hold() : p.range.leaves_split()) return;
   const int local = block / p.rows, row = block - local * p.rows, t = p.split.whole + local;
   const int m = (t % p.row_tiles) * p.rows + row, n = (t / p.row_tiles) * 256 + threadIdx.x;
   if (m >= ops.M || n >= ops.Ncols) return;
@@ -710,6 +930,7 @@ __device__ __forceinline__ void reduce_row_b16(const Ops& ops, const PiecesB16& 
   double sum = 0.0;
 #pragma unroll 8
   for (int i = 0; i < p.split.pieces; ++i) sum += static_cast<double>(at[i * tile]);
+  if constexpr (Ops::FORM == kHalves) sum = ldexp(sum, -ops.shift());
   ops.store(ops.column(n), m, static_cast<float>(sum));
 }
 template <typename Ops>
@@ -717,9 +938,9 @@ __global__ void __launch_bounds__(256) reduce_pieces_b16_kernel(Ops ops, PiecesB
   reduce_row_b16(ops, pieces, blockIdx.x);
 }
 // both gradients' pieces in one launch
-template <int PARTS>
+template <int FORM>
 __global__ void __launch_bounds__(256)
-reduce_gradients_b16_kernel(BackwardDataOpsB16<PARTS> data, PiecesB16 data_pieces, WeightGradOpsB16<PARTS> weight,
+reduce_gradients_b16_kernel(BackwardDataOpsB16<FORM> data, PiecesB16 data_pieces, WeightGradOpsB16<FORM> weight,
                             PiecesB16 weight_pieces) {
   if (blockIdx.x < data_pieces.blocks) reduce_row_b16(data, data_pieces, blockIdx.x);
   else reduce_row_b16(weight, weight_pieces, blockIdx.x - data_pieces.blocks);

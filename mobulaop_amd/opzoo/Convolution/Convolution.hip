@@ -122,8 +122,8 @@ conv::TileSplit split_b16(const Ops& ops, double* cost) {
   // and barriers that nothing hides cost what 64 rows do, 40 where two workgroups share a CU (and halve its
   // rate; one alone: a third more); three parts: 1.2 us for 128 rows, 0.68 for 64; two steps more to fill the
   // stages and write results
-  const double base = Ops::PARTS == 1 ? 0.97 : 1.1;
-  const double step = Ops::PARTS == 3 ? 2.24 * (S::ROWS + 20) / 276.0 : base * (S::ROWS + (S::PER_CU == 2 ? 40 : 64)) / 320.0;
+  const double base = Ops::FORM == 1 ? 0.97 : 1.1;
+  const double step = Ops::FORM == conv::kHalves ? 1.41 * (S::ROWS + 20) / 276.0 : Ops::FORM == 3 ? 2.24 * (S::ROWS + 20) / 276.0 : base * (S::ROWS + (S::PER_CU == 2 ? 40 : 64)) / 320.0;
   auto time = [&](int workgroups, int length) {
     return step * (length + 2) * (workgroups <= cus && S::PER_CU == 2 ? 1.33 : static_cast<double>((workgroups + cus - 1) / cus));
   };
@@ -155,31 +155,36 @@ conv::PiecesB16 launch_igemm_b16_shape(const Ops& ops, float* piece_buffer, conv
 // round that fills between half and three quarters of the device: one round of narrower tiles, 256 x 160,
 // over the same columns.  The two rounds then take as long as before -- the full round alone runs
 // slower than beside a half-empty one -- so there is one shape per product.)
+struct PlanB16 { int rows; double cost; int longest; };   // longest: K steps of the longest sum that is formed in one go
+template <typename Ops, int ROWS>
+void weigh_rows(const Ops& ops, PlanB16* best) {
+  double cost = 0.0;
+  const conv::TileSplit split = split_b16<Ops, conv::ShapeB16<ROWS, Ops::FORM>>(ops, &cost);
+  if (cost < best->cost) *best = PlanB16{ROWS, cost, split.whole > 0 ? ops.k_steps() : split.steps_per_piece};
+}
 template <typename Ops>
-int rows_b16(const Ops& ops, double* least) {
-  double cost[4] = {1e30, 1e30, 0.0, 0.0};
-  if constexpr (Ops::PARTS < 3) {
-    split_b16<Ops, conv::ShapeB16<256, Ops::PARTS>>(ops, cost);
-    split_b16<Ops, conv::ShapeB16<192, Ops::PARTS>>(ops, cost + 1);
+PlanB16 plan_b16(const Ops& ops) {
+  PlanB16 best{0, 1e30, 0};
+  if constexpr (Ops::FORM < 3) {
+    weigh_rows<Ops, 256>(ops, &best);
+    weigh_rows<Ops, 192>(ops, &best);
   }
-  split_b16<Ops, conv::ShapeB16<128, Ops::PARTS>>(ops, cost + 2);
-  split_b16<Ops, conv::ShapeB16<64, Ops::PARTS>>(ops, cost + 3);
-  const int best = static_cast<int>(std::min_element(cost, cost + 4) - cost);
-  if (least != nullptr) *least = cost[best];
-  return 256 - 64 * best;
+  weigh_rows<Ops, 128>(ops, &best);
+  weigh_rows<Ops, 64>(ops, &best);
+  return best;
 }
 template <typename Ops>
 conv::PiecesB16 launch_igemm_b16(const Ops& ops, float* piece_buffer, hipStream_t stream, conv::SplitRange range = {}) {
-  const int rows = rows_b16(ops, nullptr);
-  if constexpr (Ops::PARTS < 3) {
+  const int rows = plan_b16(ops).rows;
+  if constexpr (Ops::FORM < 3) {
     if (rows == 256)
-      return launch_igemm_b16_shape<Ops, conv::ShapeB16<256, Ops::PARTS>>(ops, piece_buffer, range, stream);
+      return launch_igemm_b16_shape<Ops, conv::ShapeB16<256, Ops::FORM>>(ops, piece_buffer, range, stream);
     if (rows == 192)
-      return launch_igemm_b16_shape<Ops, conv::ShapeB16<192, Ops::PARTS>>(ops, piece_buffer, range, stream);
+      return launch_igemm_b16_shape<Ops, conv::ShapeB16<192, Ops::FORM>>(ops, piece_buffer, range, stream);
   }
   if (rows == 128)
-    return launch_igemm_b16_shape<Ops, conv::ShapeB16<128, Ops::PARTS>>(ops, piece_buffer, range, stream);
-  return launch_igemm_b16_shape<Ops, conv::ShapeB16<64, Ops::PARTS>>(ops, piece_buffer, range, stream);
+    return launch_igemm_b16_shape<Ops, conv::ShapeB16<128, Ops::FORM>>(ops, piece_buffer, range, stream);
+  return launch_igemm_b16_shape<Ops, conv::ShapeB16<64, Ops::FORM>>(ops, piece_buffer, range, stream);
 }
 template <typename Ops>
 void reduce_b16(const Ops& ops, const conv::PiecesB16& pieces, hipStream_t stream) {
@@ -266,10 +271,13 @@ bool plan_gather(GatherPlan* plan, const char* what, const conv::Geometry& g, co
   return true;
 }
 
-// Fills the plan's tables, in the workspace at `at`; returns what follows them.
-char* build_gather(GatherPlan* plan, char* at, hipStream_t stream, conv::SplitRange range = {}) {
+void place_gather(GatherPlan* plan, char* at) {
   plan->tables.steps = reinterpret_cast<conv::GatherStep*>(at);
   plan->tables.out = reinterpret_cast<float*>(at + plan->step_bytes);
+}
+// Fills the plan's tables, in the workspace at `at`; returns what follows them.
+char* build_gather(GatherPlan* plan, char* at, hipStream_t stream, conv::SplitRange range = {}) {
+  place_gather(plan, at);
   conv::gather_tables_kernel<<<plan->tables.weight_blocks + plan->tables.step_blocks, 256, 0, stream>>>(plan->tables, range);
   return at + plan->bytes;
 }
@@ -281,25 +289,34 @@ struct PrepB16 {
   size_t bytes = 0;
   conv::ArrangeJob weights{};
   conv::BlockedJob first{}, second{};   // x of a forward pass; dy and x of a backward pass
-  template <int PARTS>
+  template <int FORM>
   void launch(hipStream_t stream, conv::ExponentWords exponents = {}) const {
     const unsigned blocks = first.blocks + second.blocks + weights.blocks;
-    if (blocks > 0) conv::prepare_b16_kernel<PARTS><<<blocks, 256, 0, stream>>>(weights, first, second, exponents);
+    if (blocks > 0) conv::prepare_b16_kernel<FORM><<<blocks, 256, 0, stream>>>(weights, first, second, exponents);
   }
 };
+
+// The three parts of operands whose products may not be formed from halves (range, other), and the fp32 kernels' tables.
+void launch_again(const PrepB16& prep, const conv::ExponentWords& words, const conv::GatherTables& tables,
+                  const conv::TapsJob& taps, conv::SplitRange range, conv::SplitRange other, hipStream_t stream) {
+  const unsigned blocks = prep.first.blocks + prep.second.blocks + prep.weights.blocks + tables.weight_blocks +
+                          tables.step_blocks + taps.blocks;
+  conv::prepare_again_kernel<<<blocks, 256, 0, stream>>>(prep.weights, prep.first, prep.second, words, tables, taps, range,
+                                                         other);
+}
 
 enum Fit { kFits, kOther, kError };   // kOther: the shape is for the caller's other kernels
 
 // A tensor as [part][images][channel block][pixels][16] bf16 (channels padded to whole K steps).
-template <int PARTS>
-int padded_channels(int channels) { return PARTS == 1 ? (channels + 31) / 32 * 32 : (channels + 15) / 16 * 16; }
-template <int PARTS>
+template <int FORM>
+int padded_channels(int channels) { return FORM == 1 ? (channels + 31) / 32 * 32 : (channels + 15) / 16 * 16; }
+template <int FORM>
 size_t blocked_bytes(int images, int channels, int pixels) {
-  return 2ull * PARTS * images * padded_channels<PARTS>(channels) * pixels;
+  return 2ull * conv::kParts<FORM> * images * padded_channels<FORM>(channels) * pixels;
 }
-template <int PARTS>
+template <int FORM>
 conv::BlockedJob blocked_job(const float* src, int images, int channels, int pixels) {
-  const int cpad = padded_channels<PARTS>(channels);
+  const int cpad = padded_channels<FORM>(channels);
   const unsigned tiles_p = (pixels + 63) / 64, tiles_c = (cpad + 63) / 64;
   return conv::BlockedJob{src, nullptr, channels, cpad, pixels, static_cast<size_t>(images) * cpad * pixels,
                           pixels % 4 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0, tiles_p, tiles_c,
@@ -312,11 +329,12 @@ char* place_blocked(conv::BlockedJob* job, size_t bytes, char* at) {
 
 // A gathered product of M rows over `channels` of the gathered tensor ([images][channels][src_pixels]): fills in
 // the fields of `ops` and `prep` but for the addresses and the tensor itself.
-template <int PARTS>
-Fit plan_gather_b16(conv::GatheredB16<PARTS>* ops, PrepB16* prep, const char* what, const conv::Geometry& g,
+template <int FORM>
+Fit plan_gather_b16(conv::GatheredB16<FORM>* ops, PrepB16* prep, const char* what, const conv::Geometry& g,
                     const float* w, int M, int channels, int images, int src_pixels, int columns_per_image,
                     long long stride_m, long long stride_c) {
-  const int taps = g.KH * g.KW, cpad = padded_channels<PARTS>(channels);
+  constexpr int PARTS = conv::kParts<FORM>;
+  const int taps = g.KH * g.KW, cpad = padded_channels<FORM>(channels);
   const long long image_bytes = static_cast<long long>(src_pixels) * cpad * 2;
   // a tile's columns span this many images at most; their byte offsets must stay below 2^31
   const long long span = 255 / std::max(columns_per_image, 1) + 2;
@@ -339,39 +357,39 @@ Fit plan_gather_b16(conv::GatheredB16<PARTS>* ops, PrepB16* prep, const char* wh
   prep->bytes += align_to_256(2 * PARTS * wcount);
   return kFits;
 }
-template <int PARTS>
-char* place_weights(conv::GatheredB16<PARTS>* ops, PrepB16* prep, char* at) {
+template <int FORM>
+char* place_weights(conv::GatheredB16<FORM>* ops, PrepB16* prep, char* at) {
   const conv::ArrangeJob& a = prep->weights;
   ops->wp = prep->weights.out = reinterpret_cast<unsigned short*>(at);
-  return at + align_to_256(2ull * PARTS * a.Mpad * a.taps * a.Cpad);
+  return at + align_to_256(2ull * conv::kParts<FORM> * a.Mpad * a.taps * a.Cpad);
 }
 
 // The products of a call and the operands they share.
-template <int PARTS>
+template <int FORM>
 struct ForwardB16 {
-  conv::ForwardOpsB16<PARTS> ops;
+  conv::ForwardOpsB16<FORM> ops;
   PrepB16 prep;
   size_t x_bytes;
   Fit plan(const conv::Geometry& g, const float* x, const float* w, const float* bias, float* y) {
     const long long taps = g.KH * g.KW;
     ops.bias = bias; ops.y = y; ops.Ncols = g.N * g.OH * g.OW;
-    prep.first = blocked_job<PARTS>(x, g.N, g.C, g.H * g.W);
-    x_bytes = blocked_bytes<PARTS>(g.N, g.C, g.H * g.W);
+    prep.first = blocked_job<FORM>(x, g.N, g.C, g.H * g.W);
+    x_bytes = blocked_bytes<FORM>(g.N, g.C, g.H * g.W);
     prep.bytes = align_to_256(x_bytes);
-    return plan_gather_b16<PARTS>(&ops, &prep, "conv2d_forward", g, w, g.D, g.C, g.N, g.H * g.W, g.OH * g.OW, g.C * taps,
+    return plan_gather_b16<FORM>(&ops, &prep, "conv2d_forward", g, w, g.D, g.C, g.N, g.H * g.W, g.OH * g.OW, g.C * taps,
                                   taps);
   }
   char* place(char* at) {
     at = place_blocked(&prep.first, x_bytes, at);
     ops.src = prep.first.dst;
-    return place_weights<PARTS>(&ops, &prep, at);
+    return place_weights<FORM>(&ops, &prep, at);
   }
 };
 
-template <int PARTS>
+template <int FORM>
 struct BackwardB16 {
-  conv::BackwardDataOpsB16<PARTS> data;
-  conv::WeightGradOpsB16<PARTS> weight;
+  conv::BackwardDataOpsB16<FORM> data;
+  conv::WeightGradOpsB16<FORM> weight;
   PrepB16 prep;
   size_t dy_bytes, x_bytes;
   bool with_dx, with_dw;
@@ -379,27 +397,27 @@ struct BackwardB16 {
   Fit plan(const conv::Geometry& g, const float* dy, const float* x, const float* w, int accumulate, float* dx, float* dw) {
     const long long taps = g.KH * g.KW;
     with_dx = dx != nullptr; with_dw = dw != nullptr;
-    prep.first = blocked_job<PARTS>(dy, g.N, g.D, g.OH * g.OW);
-    dy_bytes = blocked_bytes<PARTS>(g.N, g.D, g.OH * g.OW);
+    prep.first = blocked_job<FORM>(dy, g.N, g.D, g.OH * g.OW);
+    dy_bytes = blocked_bytes<FORM>(g.N, g.D, g.OH * g.OW);
     x_bytes = 0;
     prep.bytes = align_to_256(dy_bytes);
     if (with_dw) {
-      x_bytes = blocked_bytes<PARTS>(g.N, g.C, g.H * g.W);
+      x_bytes = blocked_bytes<FORM>(g.N, g.C, g.H * g.W);
       const long long cols = taps * ((g.C + 15) / 16 * 16), k = static_cast<long long>(g.N) * g.OH * g.OW;
       if (std::max(x_bytes, dy_bytes) >= (1ull << 31) || cols >= (1ll << 28) || g.N == 0) return kOther;
-      prep.second = blocked_job<PARTS>(x, g.N, g.C, g.H * g.W);
+      prep.second = blocked_job<FORM>(x, g.N, g.C, g.H * g.W);
       prep.bytes += align_to_256(x_bytes);
       weight.dw = dw; weight.accumulate = accumulate; weight.g = g; weight.M = g.D; weight.Ncols = static_cast<int>(cols);
-      weight.dblocks = padded_channels<PARTS>(g.D) / 16; weight.cblocks = padded_channels<PARTS>(g.C) / 16;
+      weight.dblocks = padded_channels<FORM>(g.D) / 16; weight.cblocks = padded_channels<FORM>(g.C) / 16;
       weight.ctiles = (g.C + 15) / 16;
-      const int step = conv::WeightGradOpsB16<PARTS>::STEP, rest = step % (g.OH * g.OW);
+      const int step = conv::WeightGradOpsB16<FORM>::STEP, rest = step % (g.OH * g.OW);
       weight.step_n = step / (g.OH * g.OW); weight.step_h = rest / g.OW; weight.step_w = rest % g.OW;
       if (k + 4 * step >= (1ll << 31)) return kOther;   // (pixels past the last are counted too)
     }
     if (!with_dx) return kFits;
     data.dx = dx; data.accumulate = accumulate; data.Ncols = g.N * g.H * g.W;
     // row m of the left operand is input channel m: element [m][tap][d] = weight[d][m][tap]
-    return plan_gather_b16<PARTS>(&data, &prep, "conv2d_backward_data", g, w, g.C, g.D, g.N, g.OH * g.OW, g.H * g.W, taps,
+    return plan_gather_b16<FORM>(&data, &prep, "conv2d_backward_data", g, w, g.C, g.D, g.N, g.OH * g.OW, g.H * g.W, taps,
                                   g.C * taps);
   }
   char* place(char* at) {
@@ -407,7 +425,7 @@ struct BackwardB16 {
     data.src = weight.dys = prep.first.dst;
     if (with_dw) at = place_blocked(&prep.second, x_bytes, at);
     weight.xs = prep.second.dst;
-    return with_dx ? place_weights<PARTS>(&data, &prep, at) : at;
+    return with_dx ? place_weights<FORM>(&data, &prep, at) : at;
   }
 };
 
@@ -839,15 +857,24 @@ bool plan_weight(WeightPlan* plan, const conv::Geometry& g) {
   return true;
 }
 
+conv::TapsJob taps_job(const WeightPlan& plan, const conv::Geometry& g, conv::Tap* taps) {
+  const int count = g.C * g.KH * g.KW;
+  return conv::TapsJob{taps, count, g.KH, g.KW, plan.padded ? plan.Hp * plan.Wp : g.H * g.W, g.dil_h, g.dil_w,
+                       static_cast<unsigned>(blocks_for_all(count))};
+}
+
+// (built: the plan's taps where they are made already)
 void run_weight(const WeightPlan& plan, const conv::Geometry& g, const float* dy, const float* x, int accumulate,
-                float* dw, char* ws, hipStream_t stream, conv::SplitRange range = {}) {
+                float* dw, char* ws, hipStream_t stream, conv::SplitRange range = {}, const conv::Tap* built = nullptr) {
   conv::BackwardWeightOps ops;
   ops.dy = dy; ops.x = x; ops.g = g;
   ops.M = g.D; ops.Ncols = g.C * g.KH * g.KW; ops.K = 0; ops.k_begin = 0;
-  conv::Tap* const taps = reinterpret_cast<conv::Tap*>(ws);
-  conv::build_taps_kernel<<<(ops.Ncols + 255) / 256, 256, 0, stream>>>(
-      taps, ops.Ncols, g.KH, g.KW, plan.padded ? plan.Hp * plan.Wp : g.H * g.W, g.dil_h, g.dil_w);
-  ops.taps = taps;
+  if (built == nullptr) {
+    const conv::TapsJob job = taps_job(plan, g, reinterpret_cast<conv::Tap*>(ws));
+    conv::build_taps_kernel<<<job.blocks, 256, 0, stream>>>(job.taps, job.count, job.KH, job.KW, job.plane, job.dil_h, job.dil_w);
+    built = job.taps;
+  }
+  ops.taps = built;
   ops.partial = reinterpret_cast<float*>(ws + plan.tap_bytes);
   ops.xp = nullptr; ops.Hp = plan.Hp; ops.Wp = plan.Wp;
   if (plan.padded) {
@@ -889,8 +916,8 @@ bool forward_b16(const conv::Geometry& g, const float* x, const float* weight, c
 
 // Launches the wanted products of a backward pass (operands prepared): one after the other, the pieces of both
 // added up by one kernel behind them.
-template <int PARTS>
-void launch_gradients_b16(const BackwardB16<PARTS>& b, char* piece_buffers, hipStream_t stream,
+template <int FORM>
+void launch_gradients_b16(const BackwardB16<FORM>& b, char* piece_buffers, hipStream_t stream,
                           conv::SplitRange data_range = {}, conv::SplitRange weight_range = {}) {
   float* const first = reinterpret_cast<float*>(piece_buffers);
   float* const second = b.with_dx ? first + kPieceBytes / sizeof(float) : first;
@@ -898,7 +925,7 @@ void launch_gradients_b16(const BackwardB16<PARTS>& b, char* piece_buffers, hipS
   if (b.with_dx) data = launch_igemm_b16(b.data, first, stream, data_range);
   if (b.with_dw) weight = launch_igemm_b16(b.weight, second, stream, weight_range);
   if (data.blocks > 0 && weight.blocks > 0)
-    conv::reduce_gradients_b16_kernel<PARTS><<<data.blocks + weight.blocks, 256, 0, stream>>>(b.data, data, b.weight, weight);
+    conv::reduce_gradients_b16_kernel<FORM><<<data.blocks + weight.blocks, 256, 0, stream>>>(b.data, data, b.weight, weight);
   else if (data.blocks > 0) reduce_b16(b.data, data, stream);
   else reduce_b16(b.weight, weight, stream);
 }
@@ -922,7 +949,7 @@ bool gradients_b16(const conv::Geometry& g, const float* dy, const float* x, con
   return true;
 }
 
-// ---- fp32 products from three bf16 parts per operand ---------------------------------------
+// ---- fp32 products from parts: three bf16 or two fp16 per operand ----------------------------
 //
 // An fp32 value is three bf16 exactly, and six products of parts make an fp32 product but for terms of at most
 // 2^-24 of it (two of the second part by the third: 2^-8 and 2^-17 of their values at most; 2^-27 in the mean square); sums
@@ -932,6 +959,12 @@ bool gradients_b16(const conv::Geometry& g, const float* dy, const float* x, con
 // (the products 500 to 540 us, 1.3 to 1.4 PFLOP/s of bf16 by the clock that a device holds; the passes 93 each), errors
 // against 64 bits 8.5e-7 -> 2.9e-7 (8.7e-7 -> 5.3e-7 for the weights' gradient).  The fp32 kernels follow every such
 // product and return at once unless a tensor holds values the parts do not stand for (conv::SplitRange).
+//
+// Two fp16 parts (halves) take half the matrix instructions: forward and both gradients of that layer 1819 -> 1157 us, errors
+// 1.4e-7 and 1.7e-7, as their sums start anew every 256 terms.  They need every value to lie within 2^27 of the tensor's
+// largest, or beside a value that does: in a group of 64 channels at its pixel where sums run over channels, of 64
+// pixels in its channel where they run over pixels.  What is found to lie further off while the halves are written sends
+// the product to three parts, and those to the fp32 kernels.
 
 // Fewest terms of a sum that is formed from parts by choice.  What is left out of a product (up to half a unit of
 // its last place) counts where no rounding of a longer sum exceeds it: errors of parts against 64 bits are 1.02-1.03 of
@@ -945,11 +978,42 @@ int least_taps(int K, int dil, int stride) {
   return std::max(1, K / (stride / common));
 }
 
-// option "conv_fp32_split": 1 = where it pays (default), 0 = never, 2 = wherever a product fits
+// option "conv_fp32_split": 1 = where it pays (default), 0 = never, 2 = three parts wherever a product fits, 3 = halves
 int split_choice() { return mobula_hip::option("conv_fp32_split", 1); }
 
-// Exponent words of x (or dy), the weights, and dy beside x, ahead of a call's operands.
-constexpr size_t kWordBytes = 256;
+// Fewest terms of a sum that is formed from halves by choice, in one go (not in shorter pieces of K).  An operand of two
+// halves is off by the last of its 24 bits for a quarter of the values, and what the product of both tails adds is left out:
+// 0.75e-7 of the result however long the sum; three parts lose less to that and more to long sums.  Errors of
+// halves and of three parts against 64 bits: 1.14e-7 and 0.78e-7 with 176 terms in one go, 1.20 and 1.14 with 400, 1.24 and
+// 1.47 with 704, 1.4 and 2.9 with 2304.
+constexpr long long kLeastTermsOfHalves = 512;
+
+// How a product of sums of `terms` terms may be formed: kHalves, three parts, or 0 (fp32 kernels).
+int form_of(long long terms) {
+  switch (split_choice()) {
+    case 0: return 0;
+    case 2: return 3;
+    case 3: return conv::kHalves;
+    default: return terms >= kLeastTermsOfHalves ? conv::kHalves : terms >= kLeastTerms ? 3 : 0;
+  }
+}
+// True where the product's sums are too short, as it would be cut along K.
+template <typename Ops>
+bool short_sums(const Ops& ops) {
+  return split_choice() == 1 && plan_b16(ops).longest * 16 < kLeastTermsOfHalves;
+}
+
+// What is kept of the tensors of a call ahead of its operands.
+constexpr size_t kWordBytes = 1024 + 3 * sizeof(unsigned) * conv::kMagnitudes;
+// Tensors of more elements are sampled for their magnitude (an eighth of them: 23 -> 6 us for 103 MB): the largest
+// value may be sixteen times the largest that was seen, else the product is formed from three parts.  (Those sixteen are
+// missing below: values within 2^23 of the tensor's largest.)
+constexpr long long kSampledElements = 1 << 20;
+conv::TensorWords tensor_words(char* ws, int t, long long elements) {
+  unsigned* const words = reinterpret_cast<unsigned*>(ws) + 4 * t;
+  return conv::TensorWords{words, words + 2, reinterpret_cast<const unsigned*>(ws + 1024) + t * conv::kMagnitudes,
+                           elements > kSampledElements ? 4 : 0};
+}
 
 // Microseconds of the fp32 ways from the CU clocks of their kernels (which know nothing of rounds that are not full)
 // and of what the split ways take besides their products: the passes over the tensors, and the
@@ -960,126 +1024,213 @@ double data_fp32_us(double clocks, size_t classes) {
   return clocks / (256 * 2300.0) + 15.0 * std::max<size_t>(classes, 1);
 }
 double weight_fp32_us(double clocks) { return 1.1 * clocks / (256 * 2300.0) + 30.0; }
-double parts_us(long long elements) { return elements * 10 / 4.0e6; }
+double parts_us(int form, long long elements) { return elements * (form == conv::kHalves ? 7 : 10) / 4.0e6; }
 constexpr double kSplitOverhead = 28.0;
 
-// Which of the wanted products split operands are faster for: those of some thirty us and more whose channels and
-// filters fill the tiles (forward, fp32 against split: 25 x 416 x 55 x 56, 168 filters 3 x 3: 1175 -> 640 us;
-// 5 x 96 x 119 x 109, 256: 280 -> 190; 8 x 432 x 8 x 9, 384: 50 against 91; 23 x 256 x 72 x 64, 32: 230
-// against 238).
-struct SplitChoice { bool dx, dw; };
-SplitChoice choose_split(const conv::Geometry& g, bool dx, bool dw);
+// The products of a forward pass, how they are made ready and in which workspace; the fp32 kernels behind them.
+struct ForwardFallback {
+  GatherPlan plan;
+  bool make(const conv::Geometry& g, const float* weight) {
+    const long long taps = g.KH * g.KW;
+    return plan_gather(&plan, "conv2d_forward", g, weight, g.D, g.C, static_cast<long long>(g.C) * g.H * g.W,
+                       g.OH * g.OW, g.W, +1, g.C * taps, taps);
+  }
+  void run(const conv::Geometry& g, const float* x, const float* bias, float* y, float* pieces, conv::SplitRange range,
+           hipStream_t stream) const {
+    conv::ForwardOps ops;
+    ops.x = x; ops.bias = bias; ops.y = y; ops.g = g; ops.M = g.D; ops.Ncols = g.N * g.OH * g.OW;
+    ops.wp = plan.tables.out; ops.steps = plan.tables.steps; ops.K = plan.K;
+    launch_igemm_mode<conv::ForwardOps, conv::kFp32>(ops, pieces, range, stream);
+  }
+};
 
 // True where the product is taken (or the call has failed).
 bool forward_split(const conv::Geometry& g, const float* x, const float* weight, const float* bias, float* y,
                    double fp32_cost, hipStream_t stream) {
-  ForwardB16<3> f;
-  const long long taps = g.KH * g.KW;
-  if (split_choice() != 2 && (forward_fp32_us(fp32_cost) < kSplitOverhead || g.C * taps < kLeastTerms)) return false;
-  if (f.plan(g, x, weight, bias, y) != kFits) return false;
-  if (split_choice() != 2) {
-    double product = 0.0;
-    rows_b16(f.ops, &product);
-    if (product + parts_us(static_cast<long long>(g.N) * g.C * g.H * g.W) + kSplitOverhead > forward_fp32_us(fp32_cost)) return false;
+  const long long taps = g.KH * g.KW, x_count = static_cast<long long>(g.N) * g.C * g.H * g.W;
+  const int form = form_of(g.C * taps);
+  const bool by_choice = split_choice() == 1;
+  if (form == 0 || (by_choice && forward_fp32_us(fp32_cost) < kSplitOverhead)) return false;
+  ForwardB16<3> parts;
+  ForwardB16<conv::kHalves> halves;
+  if (parts.plan(g, x, weight, bias, y) != kFits) return false;
+  const bool by_halves = form == conv::kHalves && halves.plan(g, x, weight, bias, y) == kFits && !short_sums(halves.ops);
+  if (by_choice) {
+    const double product = by_halves ? plan_b16(halves.ops).cost : plan_b16(parts.ops).cost;
+    if (product + parts_us(by_halves ? conv::kHalves : 3, x_count) + kSplitOverhead > forward_fp32_us(fp32_cost)) return false;
   }
-  GatherPlan plan;
-  if (!plan_gather(&plan, "conv2d_forward", g, weight, g.D, g.C, static_cast<long long>(g.C) * g.H * g.W,
-                   g.OH * g.OW, g.W, +1, g.C * taps, taps))
-    return true;
-  char* const ws = static_cast<char*>(mobula_hip::workspace_if_possible(kWordBytes + f.prep.bytes + plan.bytes + kPieceBytes));
+  ForwardFallback fp32;
+  if (!fp32.make(g, weight)) return true;
+  const size_t operands = std::max(parts.prep.bytes, by_halves ? halves.prep.bytes : 0);
+  char* const ws = static_cast<char*>(
+      mobula_hip::workspace_if_possible(kWordBytes + operands + fp32.plan.bytes + kPieceBytes));
   if (ws == nullptr) return failed();
-  unsigned* const words = reinterpret_cast<unsigned*>(ws);
-  const conv::SplitRange range{words, words + 1, conv::SplitRange::most_exponents(g.C * taps)};
-  char* const tables = f.place(ws + kWordBytes);
-  float* const pieces = reinterpret_cast<float*>(tables + plan.bytes);
-  conv::clear_words_kernel<<<1, 64, 0, stream>>>(words, 2);
-  f.prep.launch<3>(stream, conv::ExponentWords{words + 1, words, nullptr});
-  reduce_b16(f.ops, launch_igemm_b16(f.ops, pieces, stream, range), stream);
-  build_gather(&plan, tables, stream, range);
-  conv::ForwardOps ops;
-  ops.x = x; ops.bias = bias; ops.y = y; ops.g = g; ops.M = g.D; ops.Ncols = f.ops.Ncols;
-  ops.wp = plan.tables.out; ops.steps = plan.tables.steps; ops.K = plan.K;
-  launch_igemm_mode<conv::ForwardOps, conv::kFp32>(ops, pieces, range, stream);
+  const long long w_count = static_cast<long long>(g.D) * g.C * taps;
+  const conv::TensorWords x_words = tensor_words(ws, 0, x_count), w_words = tensor_words(ws, 1, w_count);
+  conv::SplitRange range{x_words.exponents, w_words.exponents, conv::SplitRange::most_exponents(g.C * taps)};
+  char* const tables = ws + kWordBytes + operands;
+  float* const pieces = reinterpret_cast<float*>(tables + fp32.plan.bytes);
+  const conv::ExponentWords words{w_words, x_words, {}};
+  parts.place(ws + kWordBytes);
+  place_gather(&fp32.plan, tables);
+  if (by_halves) {
+    range.halves_a = x_words.word; range.halves_b = w_words.word;
+    range.halves_mask = conv::kBeyondHalves | conv::kLonePixel;
+    halves.ops.src_word = x_words.word; halves.ops.weight_word = w_words.word;
+    halves.place(ws + kWordBytes);
+    const conv::MagnitudeJob job{{x, weight, nullptr}, {x_count, w_count, 0}, {x_words, w_words, {}}};
+    conv::magnitudes_kernel<<<dim3(conv::kMagnitudes, 2), 1024, 0, stream>>>(job);
+    halves.prep.launch<conv::kHalves>(stream, words);
+    reduce_b16(halves.ops, launch_igemm_b16(halves.ops, pieces, stream, range), stream);
+    launch_again(parts.prep, words, fp32.plan.tables, {}, range, {}, stream);
+  } else {
+    conv::clear_words_kernel<<<1, 64, 0, stream>>>(reinterpret_cast<unsigned*>(ws), 12);
+    parts.prep.launch<3>(stream, words);
+    build_gather(&fp32.plan, tables, stream, range);
+  }
+  reduce_b16(parts.ops, launch_igemm_b16(parts.ops, pieces, stream, range), stream);
+  fp32.run(g, x, bias, y, pieces, range, stream);
   MOBULA_HIP_TRY(hipGetLastError());
   return true;
 }
 
-// The gradients that are wanted (null: not).
-bool gradients_split(const conv::Geometry& g, const float* dy, const float* x, const float* weight, int accumulate,
-                     float* dx, float* dw, hipStream_t stream) {
-  BackwardB16<3> b;
+// The gradients that are wanted (null: not), from `form`.
+bool gradients_split(int form, const conv::Geometry& g, const float* dy, const float* x, const float* weight,
+                     int accumulate, float* dx, float* dw, hipStream_t stream) {
+  BackwardB16<3> parts;
+  BackwardB16<conv::kHalves> halves;
   GatherPlan plan{};
   WeightPlan weight_plan{};
   const long long taps = g.KH * g.KW;
-  if (b.plan(g, dy, x, weight, accumulate, dx, dw) != kFits) return false;
+  if (parts.plan(g, dy, x, weight, accumulate, dx, dw) != kFits) return false;
+  const bool by_halves = form == conv::kHalves && halves.plan(g, dy, x, weight, accumulate, dx, dw) == kFits;
   if (dx != nullptr && !plan_gather(&plan, "conv2d_backward_data", g, weight, g.C, g.D,
                                     static_cast<long long>(g.D) * g.OH * g.OW, g.H * g.W, g.OW, -1, taps, g.C * taps))
     return true;
   if (dw != nullptr && !plan_weight(&weight_plan, g)) return true;
   // (the fp32 weight gradient comes last: what it needs takes the place of the operands)
-  const size_t operands = b.prep.bytes + plan.bytes + (dx != nullptr && dw != nullptr ? 2 : 1) * kPieceBytes;
-  char* const ws = static_cast<char*>(
-      mobula_hip::workspace_if_possible(kWordBytes + std::max(operands, weight_plan.bytes)));
+  const size_t operands = std::max(parts.prep.bytes, by_halves ? halves.prep.bytes : 0);
+  const size_t first_bytes = operands + plan.bytes + (dx != nullptr && dw != nullptr ? 2 : 1) * kPieceBytes;
+  char* const ws = static_cast<char*>(mobula_hip::workspace_if_possible(
+      kWordBytes + weight_plan.tap_bytes + std::max(first_bytes, weight_plan.bytes)));
   if (ws == nullptr) return failed();
-  unsigned* const words = reinterpret_cast<unsigned*>(ws);   // dy, weights, x
-  char* const tables = b.place(ws + kWordBytes);
-  const conv::SplitRange data_range{words, words + 1, conv::SplitRange::most_exponents(g.D * taps)};
-  const conv::SplitRange weight_range{words, words + 2,
-                                      conv::SplitRange::most_exponents(static_cast<long long>(g.N) * g.OH * g.OW)};
-  conv::clear_words_kernel<<<1, 64, 0, stream>>>(words, 3);
-  b.prep.launch<3>(stream, conv::ExponentWords{words + 1, words, words + 2});
-  launch_gradients_b16<3>(b, tables + plan.bytes, stream, data_range, weight_range);
-  if (dx != nullptr) {
-    build_gather(&plan, tables, stream, data_range);
-    conv::BackwardDataOps ops;
-    ops.dy = dy; ops.dx = dx; ops.g = g; ops.accumulate = accumulate; ops.M = g.C; ops.Ncols = b.data.Ncols;
-    ops.wp = plan.tables.out; ops.steps = plan.tables.steps; ops.K = plan.K;
-    launch_igemm_mode<conv::BackwardDataOps, conv::kFp32>(ops, reinterpret_cast<float*>(tables + plan.bytes), data_range,
-                                                          stream);
+  const long long dy_count = static_cast<long long>(g.N) * g.D * g.OH * g.OW;
+  const long long x_count = dw != nullptr ? static_cast<long long>(g.N) * g.C * g.H * g.W : 0;
+  const long long w_count = dx != nullptr ? static_cast<long long>(g.D) * g.C * taps : 0;
+  const conv::TensorWords dy_words = tensor_words(ws, 0, dy_count), x_words = tensor_words(ws, 1, x_count),
+                          w_words = tensor_words(ws, 2, w_count);
+  conv::SplitRange data_range{dy_words.exponents, w_words.exponents, conv::SplitRange::most_exponents(g.D * taps)};
+  conv::SplitRange weight_range{dy_words.exponents, x_words.exponents,
+                                conv::SplitRange::most_exponents(static_cast<long long>(g.N) * g.OH * g.OW)};
+  conv::Tap* const built_taps = reinterpret_cast<conv::Tap*>(ws + kWordBytes);
+  char* const at = ws + kWordBytes + weight_plan.tap_bytes;
+  char* const tables = at + operands;
+  char* const pieces = tables + plan.bytes;
+  const conv::ExponentWords words{w_words, dy_words, x_words};
+  parts.place(at);
+  place_gather(&plan, tables);
+  const conv::TapsJob taps_of_weight = dw != nullptr ? taps_job(weight_plan, g, built_taps) : conv::TapsJob{};
+  if (by_halves) {
+    data_range.halves_a = weight_range.halves_a = dy_words.word;
+    data_range.halves_b = w_words.word; weight_range.halves_b = x_words.word;
+    data_range.halves_mask = conv::kBeyondHalves | conv::kLonePixel;
+    weight_range.halves_mask = conv::kBeyondHalves | conv::kLoneChannel;
+    halves.data.src_word = halves.weight.dy_word = dy_words.word;
+    halves.data.weight_word = w_words.word; halves.weight.x_word = x_words.word;
+    halves.place(at);
+    const conv::MagnitudeJob job{{dy, x, weight}, {dy_count, x_count, w_count}, {dy_words, x_words, w_words}};
+    conv::magnitudes_kernel<<<dim3(conv::kMagnitudes, 3), 1024, 0, stream>>>(job);
+    halves.prep.launch<conv::kHalves>(stream, words);
+    launch_gradients_b16<conv::kHalves>(halves, pieces, stream, data_range, weight_range);
+    launch_again(parts.prep, words, plan.tables, taps_of_weight, dx != nullptr ? data_range : weight_range,
+                 dx != nullptr && dw != nullptr ? weight_range : conv::SplitRange{}, stream);
+  } else {
+    conv::clear_words_kernel<<<1, 64, 0, stream>>>(reinterpret_cast<unsigned*>(ws), 12);
+    parts.prep.launch<3>(stream, words);
+    if (dx != nullptr) build_gather(&plan, tables, stream, data_range);
   }
-  if (dw != nullptr) run_weight(weight_plan, g, dy, x, accumulate, dw, ws + kWordBytes, stream, weight_range);
+  launch_gradients_b16<3>(parts, pieces, stream, data_range, weight_range);
+  if (dx != nullptr) {
+    conv::BackwardDataOps ops;
+    ops.dy = dy; ops.dx = dx; ops.g = g; ops.accumulate = accumulate; ops.M = g.C; ops.Ncols = parts.data.Ncols;
+    ops.wp = plan.tables.out; ops.steps = plan.tables.steps; ops.K = plan.K;
+    launch_igemm_mode<conv::BackwardDataOps, conv::kFp32>(ops, reinterpret_cast<float*>(pieces), data_range, stream);
+  }
+  if (dw != nullptr)
+    run_weight(weight_plan, g, dy, x, accumulate, dw, at, stream, weight_range, by_halves ? built_taps : nullptr);
   MOBULA_HIP_TRY(hipGetLastError());
   return true;
 }
 
+// Which of the wanted products split operands are faster for, and how they are formed (0: by the fp32 kernels): those of
+// some thirty us and more whose channels and filters fill the tiles (forward, fp32 against three parts: 25 x 416 x 55 x 56,
+// 168 filters 3 x 3: 1175 -> 640 us; 5 x 96 x 119 x 109, 256: 280 -> 190; 8 x 432 x 8 x 9, 384: 50 against 91;
+// 23 x 256 x 72 x 64, 32: 230 against 238).
+struct SplitChoice { int dx, dw; };
+
+// What the gradients that `form` may stand for cost (< 0: it may not).
+struct GradientCosts { double data, weight; };
+template <int FORM>
+GradientCosts gradient_costs(const conv::Geometry& g, bool dx, bool dw) {
+  GradientCosts cost{-1.0, -1.0};
+  BackwardB16<FORM> b;
+  float any;   // (for its address: nothing is written)
+  if (b.plan(g, &any, &any, &any, 0, dx ? &any : nullptr, dw ? &any : nullptr) != kFits) return cost;
+  if (dx && !(FORM == conv::kHalves && short_sums(b.data))) cost.data = plan_b16(b.data).cost;
+  if (dw && !(FORM == conv::kHalves && short_sums(b.weight))) cost.weight = plan_b16(b.weight).cost;
+  return cost;
+}
+
 SplitChoice choose_split(const conv::Geometry& g, bool dx, bool dw) {
-  if (split_choice() == 0 || g.N == 0 || g.N >= 65536) return SplitChoice{false, false};
-  if (split_choice() == 2) return SplitChoice{dx, dw};
+  if (split_choice() == 0 || g.N == 0 || g.N >= 65536) return SplitChoice{0, 0};
   const long long met = static_cast<long long>(least_taps(g.KH, g.dil_h, g.stride_h)) * least_taps(g.KW, g.dil_w, g.stride_w);
-  dx = dx && g.D * met >= kLeastTerms;
-  dw = dw && static_cast<long long>(g.N) * g.OH * g.OW >= kLeastTerms;
+  const int data_form = dx ? form_of(g.D * met) : 0;
+  const int weight_form = dw ? form_of(static_cast<long long>(g.N) * g.OH * g.OW) : 0;
+  if (split_choice() != 1) return SplitChoice{data_form, weight_form};
   // (what the fp32 ways take at most: most small layers end here)
   const double most_dx = data_fp32_us(gathered_product_cost(g.C, g.D, g.KH * g.KW, static_cast<long long>(g.N) * g.H * g.W),
                                       static_cast<size_t>(g.stride_h) * g.stride_w);
   const double most_dw = weight_fp32_us(weight_gathered_cost(g));
-  dx = dx && most_dx > kSplitOverhead;
-  dw = dw && most_dw > kSplitOverhead + 10.0;
-  if (!dx && !dw) return SplitChoice{false, false};
-  BackwardB16<3> b;
-  float any;   // (for its address: nothing is written)
-  if (b.plan(g, &any, &any, &any, 0, dx ? &any : nullptr, dw ? &any : nullptr) != kFits) return SplitChoice{false, false};
-  const double dy_parts = parts_us(static_cast<long long>(g.N) * g.D * g.OH * g.OW);
-  const double x_parts = parts_us(static_cast<long long>(g.N) * g.C * g.H * g.W);
-  double data = 0.0, weight = 0.0, data_fp32 = 0.0, weight_fp32 = 0.0;
+  dx = data_form != 0 && most_dx > kSplitOverhead;
+  dw = weight_form != 0 && most_dw > kSplitOverhead + 10.0;
+  if (!dx && !dw) return SplitChoice{0, 0};
+  const GradientCosts parts = gradient_costs<3>(g, dx, dw);
+  dx = dx && parts.data >= 0; dw = dw && parts.weight >= 0;
+  const GradientCosts halves = gradient_costs<conv::kHalves>(g, dx && data_form == conv::kHalves, dw && weight_form == conv::kHalves);
+  double data_fp32 = 0.0, weight_fp32 = 0.0;
   if (dx) {
-    rows_b16(b.data, &data);
     const DataPatches patches = data_patches(g, nullptr, nullptr, nullptr, 0);
     const size_t classes = data_patches_win(g, patches, &data_fp32) ? patches.classes.size() : 1;
     data_fp32 = data_fp32_us(data_fp32, classes);
   }
-  if (dw) {
-    rows_b16(b.weight, &weight);
-    weight_fp32 = weight_fp32_us(weight_fp32_cost(g));
-  }
-  const double only_dx = data + dy_parts + kSplitOverhead, only_dw = weight + dy_parts + x_parts + kSplitOverhead;
-  SplitChoice best{dx && only_dx < data_fp32, dw && only_dw < weight_fp32};
-  if (dx && dw) {   // the parts of dy are shared
-    const double both = data + weight + dy_parts + x_parts + 1.3 * kSplitOverhead, none = data_fp32 + weight_fp32;
-    const double one_dx = only_dx + weight_fp32, one_dw = only_dw + data_fp32;
-    best.dx = std::min(both, one_dx) < std::min(none, one_dw);
-    best.dw = std::min(both, one_dw) < std::min(none, one_dx);
-  }
-  return best;
+  if (dw) weight_fp32 = weight_fp32_us(weight_fp32_cost(g));
+  const long long dy_count = static_cast<long long>(g.N) * g.D * g.OH * g.OW;
+  const long long x_count = static_cast<long long>(g.N) * g.C * g.H * g.W;
+  // the products from their forms, each on its own, and from one form together, where they share the copy of dy
+  struct Way { SplitChoice choice; double cost; };
+  Way best{{0, 0}, data_fp32 + weight_fp32};
+  auto consider = [&](int a, int b, double cost) {
+    if (cost < best.cost) best = Way{{a, b}, cost};
+  };
+  const double dy3 = parts_us(3, dy_count), dy4 = parts_us(conv::kHalves, dy_count);
+  const double x3 = parts_us(3, x_count), x4 = parts_us(conv::kHalves, x_count);
+  if (dx) consider(3, 0, parts.data + dy3 + kSplitOverhead + weight_fp32);
+  if (dw) consider(0, 3, parts.weight + dy3 + x3 + kSplitOverhead + data_fp32);
+  if (dx && dw) consider(3, 3, parts.data + parts.weight + dy3 + x3 + 1.3 * kSplitOverhead);
+  // (what three parts win does not go to the fp32 kernels, whose sums lose more, for the sake of the other product)
+  const SplitChoice with_parts = best.choice;
+  auto upgrade = [&](int a, int b, double cost) {
+    if ((with_parts.dx == 0 || a != 0) && (with_parts.dw == 0 || b != 0)) consider(a, b, cost);
+  };
+  if (halves.data >= 0) upgrade(conv::kHalves, 0, halves.data + dy4 + kSplitOverhead + weight_fp32);
+  if (halves.weight >= 0) upgrade(0, conv::kHalves, halves.weight + dy4 + x4 + kSplitOverhead + data_fp32);
+  if (halves.data >= 0 && halves.weight >= 0)
+    upgrade(conv::kHalves, conv::kHalves, halves.data + halves.weight + dy4 + x4 + 1.3 * kSplitOverhead);
+  if (halves.weight >= 0 && dx)
+    upgrade(3, conv::kHalves, parts.data + dy3 + halves.weight + dy4 + x4 + 2 * kSplitOverhead);
+  if (halves.data >= 0 && dw)
+    upgrade(conv::kHalves, 3, halves.data + dy4 + parts.weight + dy3 + x3 + 2 * kSplitOverhead);
+  return best.choice;
 }
 
 // Both gradients in one go, sharing what prepares their operands; false: not taken, or only as far as *done says.
@@ -1089,10 +1240,15 @@ bool both_gradients(const conv::Geometry& g, const float* dy, const float* x, co
   if (compute_mode() == conv::kBf16) return gradients_b16<1>(g, dy, x, weight, 0, dx, dw, stream);
   if (compute_mode() == conv::kBf16x3) return gradients_b16<2>(g, dy, x, weight, 0, dx, dw, stream);
   const SplitChoice split = choose_split(g, true, true);
-  if ((split.dx || split.dw) &&
-      gradients_split(g, dy, x, weight, 0, split.dx ? dx : nullptr, split.dw ? dw : nullptr, stream))
+  if (split.dx != 0 && split.dw != 0 && split.dx != split.dw) {   // (no copy of dy serves both)
+    if (gradients_split(split.dx, g, dy, x, weight, 0, dx, nullptr, stream)) done->dx = split.dx;
+    if (!failed() && gradients_split(split.dw, g, dy, x, weight, 0, nullptr, dw, stream)) done->dw = split.dw;
+  } else if ((split.dx != 0 || split.dw != 0) &&
+             gradients_split(std::max(split.dx, split.dw), g, dy, x, weight, 0, split.dx != 0 ? dx : nullptr,
+                             split.dw != 0 ? dw : nullptr, stream)) {
     *done = split;
-  return done->dx && done->dw;
+  }
+  return done->dx != 0 && done->dw != 0;
 }
 
 // dx (+)= and dw (+)= as the launchers below say; allow_split: whether products of parts have yet to be weighed.
@@ -1108,9 +1264,8 @@ void data_gradient(const conv::Geometry& g, const float* dy, const float* weight
     if (taken) return;
   }
   if (compute_mode() == conv::kFp32) {
-    if (allow_split && choose_split(g, true, false).dx &&
-        gradients_split(g, dy, nullptr, weight, accumulate, dx, nullptr, stream))
-      return;
+    const int form = allow_split ? choose_split(g, true, false).dx : 0;
+    if (form != 0 && gradients_split(form, g, dy, nullptr, weight, accumulate, dx, nullptr, stream)) return;
     const DataPatches patches = data_patches(g, dy, weight, dx, accumulate);
     double cost = 0.0;
     if (data_patches_win(g, patches, &cost)) {
@@ -1151,9 +1306,8 @@ void weight_gradient(const conv::Geometry& g, const float* dy, const float* x, i
     if (taken) return;
   }
   if (compute_mode() == conv::kFp32 && wt > 0) {
-    if (allow_split && choose_split(g, false, true).dw &&
-        gradients_split(g, dy, x, nullptr, accumulate, nullptr, dw, stream))
-      return;
+    const int form = allow_split ? choose_split(g, false, true).dw : 0;
+    if (form != 0 && gradients_split(form, g, dy, x, nullptr, accumulate, nullptr, dw, stream)) return;
     if (weight_gradient_from_patches(g, dy, x, accumulate, dw, stream)) return;
   }
   WeightPlan plan;
@@ -1233,7 +1387,7 @@ MOBULA_KERNEL conv2d_forward_kernel(const int n, const T* x, const T* weight, co
     const PatchProduct patches = forward_patches(g, x, weight, bias, y);
     double cost = 0.0;
     const bool from_patches = forward_patches_win(g, patches, &cost);
-    if (split_choice() != 0 && forward_split(g, x, weight, bias, y, cost, stream)) return;
+    if (forward_split(g, x, weight, bias, y, cost, stream)) return;
     if (from_patches) {
       run_patch_product(patches, stream);
       return;

@@ -812,3 +812,146 @@ def test_sums_of_a_few_terms_are_not_formed_from_parts_by_choice(filters):
     finally:
         native.set_option('conv_fp32_split', 1)
     assert torch.equal(*out)
+
+
+@pytest.fixture
+def halves_always():
+    native.set_option('conv_fp32_split', 3)
+    yield
+    native.set_option('conv_fp32_split', 1)
+
+
+def _layer(shape, seed, scale=1.0):
+    """x, w, dy of a layer, its geometry, the three products in 64 bits, and the terms of their sums."""
+    N, C, H, W, D, kernel, pad, stride, dil = shape
+    g = torch.Generator().manual_seed(seed)
+    x, w = torch.randn(N, C, H, W, generator=g) * scale, torch.randn(D, C, *kernel, generator=g) / scale
+    xr, wr = x.double().requires_grad_(True), w.double().requires_grad_(True)
+    y_ref = F.conv2d(xr, wr, None, stride=stride, padding=pad, dilation=dil)
+    dy = torch.randn(y_ref.shape, generator=g)
+    y_ref.backward(dy.double())
+    geo = _ci(N, C, H, W, D, kernel[0], kernel[1], pad[0], pad[1], stride[0], stride[1], dil[0], dil[1])
+    terms = C * kernel[0] * kernel[1], D * kernel[0] * kernel[1], dy[:, 0].numel()
+    return (x.cuda(), w.cuda(), dy.cuda()), geo, (y_ref.detach(), xr.grad, wr.grad), terms
+
+
+@pytest.mark.parametrize('scale', [1.0, 2.0 ** -40, 2.0 ** 70])
+@pytest.mark.parametrize('shape', [
+    # N, C, H, W, D, kernel, pad, stride, dilation
+    (1, 1, 1, 1, 1, (1, 1), (0, 0), (1, 1), (1, 1)),         # one multiply-add
+    (3, 16, 5, 3, 64, (1, 1), (0, 0), (1, 1), (1, 1)),       # one step of K; 15 pixels an image
+    (40, 17, 2, 2, 65, (2, 2), (1, 1), (1, 1), (1, 1)),      # rows and channels one past a tile and a block
+    (2, 272, 9, 10, 128, (1, 1), (0, 0), (1, 1), (1, 1)),    # 17 steps: sums that move once, whole rows of tiles
+    (2, 33, 19, 21, 193, (3, 2), (2, 0), (1, 1), (1, 1)),    # odd planes: the element-wise conversion
+    (4, 128, 24, 28, 256, (3, 3), (1, 1), (1, 1), (1, 1)),   # 72 and more steps: sums that move every sixteen
+    (3, 48, 23, 17, 257, (3, 3), (0, 1), (2, 2), (1, 1)),    # strides: taps that reach no pixel
+    (2, 24, 30, 22, 40, (3, 2), (2, 1), (2, 1), (1, 2)),     # strides and dilation
+])
+def test_fp32_products_of_two_halves(shape, scale, halves_always):
+    """Operands of 23 bits and a sign (2^-23 of a value at most), the tails' product left out (2^-22), and up to six fp32
+    roundings for sixteen of K, each of 2^-24 of a sum no larger than the result's own scale: the latter add up as
+    their squares.  Operands of any scale."""
+    (x, w, dy), geo, want, terms = _layer(shape, 97, scale)
+    _leave_nan_patterns_in_the_workspace()
+    got = _three_products(geo, x, w, dy)
+    for a, b, k, what in zip(got, want, terms, ('y', 'dx', 'dw')):
+        error = ((a.cpu().double() - b).norm() / b.norm()).item()
+        assert error <= 2.0 ** -24 * (1 + 2 + 2 + 4 + (6 * (k / 16 + 1)) ** 0.5), (what, error)
+    start = [torch.randn(t.shape, generator=torch.Generator().manual_seed(98)).cuda() * t.abs().max() for t in (x, w)]
+    again = _three_products(geo, x, w, dy, *start)
+    assert torch.equal(again[0], got[0])
+    assert torch.equal(again[1], start[0] + got[1]) and torch.equal(again[2], start[1] + got[2])
+
+
+@pytest.mark.parametrize('odd', ['lone pixel', 'lone channel', 'small beside large', 'unseen', 'inf', 'nan', 'overflow'])
+def test_values_that_two_halves_do_not_stand_for(odd, halves_always):
+    """A tensor whose values lie too far apart for two halves is multiplied in three parts (the same bits as when they are
+    asked for) or by the fp32 kernels; small values beside large ones, and zeros, stay with the halves."""
+    shape = (2, 96, 80, 80, 64, (3, 3), (1, 1), (1, 1), (1, 1))     # x: 1.2 million elements, an eighth of them looked at
+    (x, w, dy), geo, _, _ = _layer(shape, 99)
+    dy[:, :, 10:30] = 0.0
+    if odd == 'lone pixel':            # 64 channels of a pixel, and what lies beside them, 2^-30 of the rest
+        x[1, :64, 7, 9] *= 2.0 ** -30
+        dy[0, :, 40, 3] *= 2.0 ** -30
+    elif odd == 'lone channel':
+        x[:, 5] *= 2.0 ** -30
+    elif odd == 'small beside large':
+        x[1, 3, 7, 9] *= 2.0 ** -60
+        dy[0, 1, 40, 3] = 1e-40
+    elif odd == 'unseen':              # (elements 4096 to 36863 are not looked at)
+        x.view(-1)[5000] = 1e5
+    elif odd == 'overflow':
+        x.abs_().mul_(2.0 ** 124), w.abs_().mul_(2.0 ** 20), dy.abs_().mul_(2.0 ** 60)   # (of one sign: whatever the order)
+    else:
+        x[1, 3, 7, 9] = float(odd)
+    got = _three_products(geo, x, w, dy)
+    native.set_option('conv_fp32_split', 2)
+    parts = _three_products(geo, x, w, dy)
+    native.set_option('conv_fp32_split', 0)
+    want = _three_products(geo, x, w, dy)
+    for a, b, what in zip(got, want, ('y', 'dx', 'dw')):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf()), what
+        fine = b.isfinite()
+        assert (a[fine].double() - b[fine].double()).norm() <= 2e-6 * b[fine].double().norm(), what
+    same = [torch.equal(a.nan_to_num(), b.nan_to_num()) for a, b in zip(got, parts)]
+    # which products left the halves: sums over channels where a pixel is far off, over pixels where a channel is
+    assert same == {'lone pixel': [True, True, False], 'lone channel': [False, False, True],
+                    'small beside large': [False, False, False], 'unseen': [True, False, True],
+                    'inf': [True, False, True], 'nan': [True, False, True], 'overflow': [True, False, True]}[odd]
+
+
+@pytest.mark.parametrize('shape', [
+    (4, 64, 24, 28, 256, (3, 3), (1, 1), (1, 1), (1, 1)),        # 576 terms, and pieces of K
+    (16, 64, 56, 56, 128, (3, 3), (1, 1), (1, 1), (1, 1)),
+    (2, 256, 60, 61, 130, (5, 5), (2, 2), (1, 1), (1, 1)),
+])
+def test_sums_formed_by_choice_are_no_further_off_than_those_of_three_parts_or_fp32(shape):
+    (x, w, dy), geo, want, _ = _layer(shape, 100)
+    errors = {}
+    try:
+        for option in 1, 2, 0:
+            native.set_option('conv_fp32_split', option)
+            errors[option] = [((a.cpu().double() - b).norm() / b.norm()).item()
+                              for a, b in zip(_three_products(geo, x, w, dy), want)]
+    finally:
+        native.set_option('conv_fp32_split', 1)
+    for chosen, parts, fp32, what in zip(errors[1], errors[2], errors[0], ('y', 'dx', 'dw')):
+        assert chosen <= 1.02 * max(parts, fp32), (what, chosen, parts, fp32)
+
+def test_halves_in_a_recorded_graph(halves_always):
+    """What is known of the operands is found anew by every replay: halves, three parts, halves again."""
+    shape = (2, 64, 24, 28, 128, (3, 3), (1, 1), (1, 1), (1, 1))
+    (x, w, dy), geo, _, _ = _layer(shape, 101)
+    usual, odd = x.clone(), x.clone()
+    odd[1, :, 7, 9] *= 2.0 ** -30
+    odd[0, 5] *= 2.0 ** -30
+    lib, stream = native.library(), torch.cuda.Stream()
+    y, dx, dw = torch.empty_like(dy), torch.empty_like(x), torch.empty_like(w)
+
+    def call(on=None):
+        native.begin_call(on, [])
+        lib.conv2d_forward_c6a7aa85(ctypes.c_int(0), ctypes.c_int(y.numel()), _ptr(x), _ptr(w), _ptr(w), ctypes.c_int(0),
+                                    *geo, _ptr(y))
+        lib.mobula_hip_conv2d_backward(ctypes.c_int(0), _ptr(dy), _ptr(x), _ptr(w), *geo, _ptr(dx), _ptr(dw))
+        native.end_call('conv2d')
+    try:
+        want = []
+        for values in usual, odd:
+            x.copy_(values)
+            call()
+            torch.cuda.synchronize()
+            want.append([t.clone() for t in (y, dx, dw)])
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            call(on=torch.cuda.current_stream().cuda_stream)
+        for which in (0, 1, 0, 0, 1):
+            x.copy_((usual, odd)[which])
+            for t in (y, dx, dw):
+                t.fill_(float('nan'))
+            graph.replay()
+            torch.cuda.synchronize()
+            for a, b in zip((y, dx, dw), want[which]):
+                assert torch.equal(a, b)
+        del graph
+    finally:
+        native.unpin_workspace()
