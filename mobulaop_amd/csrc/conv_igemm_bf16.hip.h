@@ -763,17 +763,41 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
   //   before the barrier, BEFORE products | the step's other fragments, each a product ahead of the one that needs it
   //   wait for the fragments and for stage s + 1 (all loads but those of later stages), barrier: everyone holds stage s
   //   in registers
-  //   behind it, the other products | requests for step s + STAGES into stage s, then the fragments the
-  //   next step begins with (those of the right operand into a spare set while the last products need theirs)
-  constexpr int SLOTS = NI * NJ, AFTER = P::COUNT - P::BEFORE, TAIL = LOADS + NI + NJ;
+  //   behind it, the other products | the fragments the next step begins with (those of the right operand
+  //   into a spare set while the last products need theirs)
+  //   and requests for loads.  One part and halves: for step s + STAGES - 1 into the stage of step s - 1, one every few
+  //   products throughout: a load that finds the address unit's queue full holds up whatever its wavefront has behind it, so
+  //   all of a step's at once, by eight wavefronts behind one barrier, do for the time of moving a stage (32 x 256 x 56 x 56,
+  //   256 filters 3 x 3, halves: forward 352 -> 324 us, data gradient 360 -> 347; one part: 137 -> 129, 140 -> 131; three to
+  //   six stages are all as fast).  Two and three parts, with more products to a load: for step s + STAGES into stage s, all
+  //   right behind the barrier (spread out: 1784 -> 1802 us for that layer in three parts).
+  constexpr bool SPREAD = Ops::FORM == 1 || HALVES;
+  constexpr int SLOTS = NI * NJ, AFTER = P::COUNT - P::BEFORE, ALL = P::COUNT * SLOTS;
+  constexpr int AHEAD = SPREAD ? STAGES - 1 : STAGES, TAIL = (SPREAD ? 0 : LOADS) + NI + NJ;
   constexpr int A_FIRST = P::A[0];   // the next step's first product: units A_FIRST and 0
+  auto load = [&](int q) {
+    request(q);
+    if (q == LOADS - 1) step_requested();
+  };
+  // load q goes behind product (2 q + 1) ALL / (2 LOADS) of the step
+  auto spread = [&](int at) {
+    if constexpr (SPREAD) {
 #pragma unroll
-  for (int k = 0; k < STAGES; ++k) {
+      for (int q = 0; q < LOADS; ++q)
+        if ((2 * q + 1) * ALL / (2 * LOADS) == at) load(q);
+    }
+  };
+  constexpr int EARLY = [] {   // those before the barrier
+    int n = 0;
+    for (int q = 0; q < LOADS; ++q) n += SPREAD && (2 * q + 1) * ALL / (2 * LOADS) < P::BEFORE * SLOTS;
+    return n;
+  }();
 #pragma unroll
-    for (int q = 0; q < LOADS; ++q) request(q);
-    step_requested();
+  for (int k = 0; k < AHEAD; ++k) {
+#pragma unroll
+    for (int q = 0; q < LOADS; ++q) load(q);
   }
-  wait_for_loads_but<(STAGES - 1) * LOADS>();
+  wait_for_loads_but<(AHEAD - 1) * LOADS>();
   workgroup_barrier();
   int stage = 0;
 #pragma unroll
@@ -814,9 +838,10 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
             else fa[ua][q - NJ] = read_a(stage, ua, q - NJ);
           }
         }
+        spread(p * SLOTS + k);
         __builtin_amdgcn_sched_barrier(0);
       }
-    wait_for_reads_and_loads_but<(STAGES - 2) * LOADS>();
+    wait_for_reads_and_loads_but<(AHEAD - 2) * LOADS + EARLY>();
     workgroup_barrier();
 #pragma unroll
     for (int p = 0; p < AFTER; ++p)
@@ -826,11 +851,12 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
         const int at = p * SLOTS + k;
 #pragma unroll
         for (int q = at * TAIL / (AFTER * SLOTS); q < (at + 1) * TAIL / (AFTER * SLOTS); ++q) {
-          if (q < LOADS) request(q);
-          else if (q < LOADS + NJ) next_b[q - LOADS] = read_b(next, 0, q - LOADS);
-          else fa[A_FIRST][q - LOADS - NJ] = read_a(next, A_FIRST, q - LOADS - NJ);
-          if (q == LOADS - 1) step_requested();
+          const int r = SPREAD ? q : q - LOADS;
+          if (r < 0) load(q);
+          else if (r < NJ) next_b[r] = read_b(next, 0, r);
+          else fa[A_FIRST][r - NJ] = read_a(next, A_FIRST, r - NJ);
         }
+        spread(P::BEFORE * SLOTS + at);
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
