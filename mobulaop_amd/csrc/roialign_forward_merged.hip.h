@@ -17,12 +17,17 @@
 // on scheduling; they differ from the per-sample order of the reference by
 // rounding only.
 //
-// Bound by vector instructions and the L1 path about alike (4 x 512 x 100 x 100 fp16, 6000 boxes, 7 x 7: busy 75 % and 73 % of
-// the time): a multiply-add per pixel and channel, a 16-byte load per pixel and eight channels.  What is not
-// one of these is kept out of the loops: lists end in entries that load nothing, so a column takes a read and an
-// add; a row's entry is fetched from a lane that holds it; both axes' lists are made in one go; grids of up to
-// 14 points in one window, so that only bins beyond 14 pixels are listed twice (4999 -> 4054 vector instructions a wavefront,
-// 573 -> 473 us a call).
+// A map row's merged columns are summed first, and that sum is then added to every pooled row the map row has a weight in: the
+// last rows of one pooled row are often the first of the next (34 rows of a box are read instead of 44 at 4 x 512 x
+// 100 x 100 fp16, 6000 boxes, 7 x 7), and a row takes one multiply-add per pixel and channel without a product of weights
+// before it.  Two rows at a time, three with four channels a lane: more sums do not fit 128 registers.
+//
+// Bound by the L1 path and vector instructions about alike (that shape: busy 85 % and 76 % of the time): a 16-byte load per
+// pixel and eight channels, a multiply-add per pixel and channel.  What is not one of these is kept out of the loops: lists
+// end in entries that load nothing, so a column takes a read and an add; a row's entry is fetched from a lane that holds it;
+// both axes' lists are made in one go; the number of points is divided by in the rows' weights; rows are read by code for two
+// (three) and for one, as a branch inside it costs moves of every sum (with it 453 us, with products of weights and no
+// shared rows 480, now 431; fp32, 256 channels: 436 -> 375).
 #pragma once
 #include <type_traits>
 
@@ -31,13 +36,22 @@
 namespace roialign {
 
 struct FwdMerged {
-  static constexpr int LCAP = 28;   // entries per merged list: two a sample
-  // Samples merged per list at a time: all of a grid of up to 14, else 11.  Lists of 14 samples for both axes and the
-  // staging area are 10016 bytes of the 10240 that let sixteen wavefronts share a CU; with lists of 16 fifteen do, and grids
-  // of 15 and 16 take 17 to 28 % less, all others 3 to 12 % more.  A window of n samples meets n + 1 pixels: 11 fill
-  // three blocks of four columns (fp16, 1500 boxes of one size on 2 x 128 x 256 x 256, windows of 11 against 14: grids of
-  // 18 points 394 and 438 us, 22 522 and 576, 24, three windows against two, 703 and 638, 30 1016 and 1051).
-  static constexpr int WHOLE = 14, WS = 11;
+  static constexpr int LCAP = 28;   // entries per merged list
+  // Samples merged per list at a time.  Where they lie at most a pixel apart (adaptive grids) 26 of them meet 28 pixels at
+  // most: a grid of up to 26 points is one list, larger ones are cut evenly (250 x 300 fp16, 1500 uniform boxes of up to 43 points:
+  // 2100 -> 1820 us against lists of 11 samples beyond 14, whose columns are listed anew for every pooled row and whose
+  // rows are not shared).  Samples further apart meet two pixels each: all of a grid of up to 14, else 11.
+  // Lists for both axes and the staging area are 10016 bytes of the 10240 that let sixteen wavefronts share a CU.
+  static constexpr int WHOLE = 14, WS = 11, DENSE = 26;
+  static_assert(2 * WHOLE <= LCAP && DENSE + 2 <= LCAP, "entries of a list");
+  // Samples merged at a time along an axis of `grid` points a bin.
+  __device__ static int window(int grid, float bin) {
+    if (bin <= static_cast<float>(grid)) {
+      const int windows = (grid + DENSE - 1) / DENSE;
+      return windows <= 1 ? DENSE : (grid + windows - 1) / windows;
+    }
+    return grid <= WHOLE ? WHOLE : WS;
+  }
   static constexpr int RPH = 8;     // pooled rows whose lists are held at a time
   // One wavefront per workgroup: the wavefronts are independent, and a slot is refilled as soon
   // as its wavefront ends instead of when the slowest of four does (boxes differ a lot in work
@@ -148,7 +162,7 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
   const int batch = uni_i(g.batch);
   const bool image_ok = batch >= 0 && batch < num_images;
   const int gh = uni_i(g.grid_h), gw = uni_i(g.grid_w);
-  const int ws_h = gh <= M::WHOLE ? M::WHOLE : M::WS, ws_w = gw <= M::WHOLE ? M::WHOLE : M::WS;
+  const int ws_h = uni_i(M::window(gh, g.bin_h)), ws_w = uni_i(M::window(gw, g.bin_w));
   // A box far larger than the map (or infinite) has up to 2^31 sample points per
   // bin, nearly all outside the map: forward_large_grid_kernel does those boxes.
   if (gh > kSearchedGrid || gw > kSearchedGrid) return;
@@ -229,6 +243,17 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
     for (int pwb = 0; pwb < PW; pwb += K::PWB) {
       const int pw = pwb + grp;
       const bool bin_on = pw < PW && quad_on;
+      // Column sums of the map rows read last: what the next pooled row begins with, where it begins with them
+      // (held < 0: no row).
+      constexpr int MOST = CPL == 4 ? 3 : 2;   // rows read at a time (eight channels a lane have registers for two)
+      int held[MOST];
+      float t[MOST][CPL];
+#pragma unroll
+      for (int r = 0; r < MOST; ++r) {
+        held[r] = -1;
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) t[r][i] = 0.0f;
+      }
 #pragma nounroll
       for (int ph = ph0; ph < ph0 + rp; ++ph) {
         float acc[CPL];
@@ -239,82 +264,92 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
           for (int iyw = 0; iyw < gh; iyw += ws_h) {
             need_rows(ph, iyw);
             const int nr = uni_i(rown[ph - row_p0]);
-            const MergedEntry row_of_lane = rowm[ph - row_p0][min(lane, M::LCAP - 1)];   // an entry a lane
+            // an entry a lane; the sum over a bin's points is divided by their number here (the reference divides the
+            // sum: the same but for the last bit where that number is no power of two)
+            const MergedEntry row_of_lane = rowm[ph - row_p0][min(lane, M::LCAP - 1)];
+            const float weight_of_lane = row_of_lane.w * inv_count;
+            auto row_off = [&](int r) { return __builtin_amdgcn_readlane(row_of_lane.off, r); };
+            auto add_row = [&](int r, const float (&sum)[CPL]) {
+              const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight_of_lane), r));
+#pragma unroll
+              for (int i = 0; i < CPL; ++i) acc[i] = fmaf(w, sum[i], acc[i]);
+            };
 #pragma nounroll
             for (int ixw = 0; ixw < gw; ixw += ws_w) {
               need_cols(pwb, ixw);
+              if (col_max == 0) continue;   // (no column of these eight has a point on the map)
               const MergedEntry* const clist = colm[grp];
-              // blocks of four map rows (scalar) x four or two map columns (per lane): the columns
-              // of a block are decoded once for all its rows; a last block of at most two columns
-              // is not padded to four
-              auto block = [&](const int (&roff)[4], const float (&rw)[4], const bool (&rlive)[4], const int (&coff)[4],
-                               const float (&cw)[4], auto width) {
-                constexpr int NC = decltype(width)::value;
-                typename LaneData<T>::type v[4][NC];
+              if (gw > ws_w) {   // (sums over other columns)
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                  if (rlive[r]) {
+                for (int r = 0; r < MOST; ++r) held[r] = -1;
+              }
+              int r0 = 0;
+              auto again = [&] {
+                const int off = row_off(r0);
+                if (off == held[0]) add_row(r0++, t[0]);
+                else if (off == held[1]) add_row(r0++, t[1]);
+                else if (off == held[MOST - 1]) add_row(r0++, t[MOST - 1]);
+                else return false;
+                return true;
+              };
+              if (nr > 0 && again() && nr > 1) (void)again();
+              // two map rows, or one (scalar), x four or two map columns (per lane) at a time
+              auto rows = [&](auto count) {
+                constexpr int ROWS = decltype(count)::value;
+                int roff[ROWS];
+#pragma unroll
+                for (int r = 0; r < ROWS; ++r) roff[r] = row_off(r0 + r);
+                auto block = [&](int cc, auto first, auto width) {
+                  constexpr bool FIRST = decltype(first)::value;
+                  constexpr int NC = decltype(width)::value;
+                  int coff[NC];
+                  float cw[NC];
+#pragma unroll
+                  for (int c = 0; c < NC; ++c) {
+                    const MergedEntry e = clist[cc + c];
+                    coff[c] = static_cast<int>(static_cast<unsigned>(e.off) + lane_off);
+                    cw[c] = e.w;
+                  }
+                  typename LaneData<T>::type v[ROWS][NC];
+#pragma unroll
+                  for (int r = 0; r < ROWS; ++r)
 #pragma unroll
                     for (int c = 0; c < NC; ++c) v[r][c] = buffer_load_lane<T>(plane, coff[c], roff[r]);
+#pragma unroll
+                  for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+                    for (int c = 0; c < NC; ++c)
+#pragma unroll
+                      for (int i = 0; i < CPL; ++i)   // (a multiply-add widens 16-bit values on the way, a product does not)
+                        t[r][i] = fmaf(cw[c], static_cast<float>(v[r][c][i]), FIRST && c == 0 ? 0.0f : t[r][i]);
+                };
+                const std::true_type yes;
+                const std::false_type no;
+                const std::integral_constant<int, 2> two;
+                const std::integral_constant<int, 4> four;
+                if (col_max <= 2) {   // (the same for every lane)
+                  block(0, yes, two);
+                } else {
+                  block(0, yes, four);
+#pragma nounroll
+                  for (int cc = 4; cc < col_max; cc += 4) {
+                    if (col_max - cc <= 2) block(cc, no, two);
+                    else block(cc, no, four);
                   }
+                }
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                  if (rlive[r]) {
-                    if constexpr (CPL > NC) {
-                      // more channels than columns per lane: the weight of a pixel first, then one
-                      // multiply-add per pixel and channel
-                      float w[NC];
-#pragma unroll
-                      for (int c = 0; c < NC; ++c) w[c] = rw[r] * cw[c];
-#pragma unroll
-                      for (int i = 0; i < CPL; ++i) {
-#pragma unroll
-                        for (int c = 0; c < NC; ++c) acc[i] = fmaf(w[c], static_cast<float>(v[r][c][i]), acc[i]);
-                      }
-                    } else {
-#pragma unroll
-                      for (int i = 0; i < CPL; ++i) {
-                        float t = cw[0] * static_cast<float>(v[r][0][i]);
-#pragma unroll
-                        for (int c = 1; c < NC; ++c) t = fmaf(cw[c], static_cast<float>(v[r][c][i]), t);
-                        acc[i] = fmaf(rw[r], t, acc[i]);
-                      }
-                    }
-                  }
+                for (int r = 0; r < ROWS; ++r) {
+                  held[r] = roff[r];
+                  add_row(r0 + r, t[r]);
+                }
               };
 #pragma nounroll
-              for (int cc = 0; cc < col_max; cc += 4) {
-                int coff[4];
-                float cw[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                  const MergedEntry e = clist[cc + k];
-                  coff[k] = static_cast<int>(static_cast<unsigned>(e.off) + lane_off);
-                  cw[k] = e.w;
-                }
-                const bool narrow = col_max - cc <= 2;   // (the same for every lane)
-#pragma nounroll
-                for (int r0 = 0; r0 < nr; r0 += 4) {
-                  int roff[4];
-                  float rw[4];
-                  bool rlive[4];
-#pragma unroll
-                  for (int k = 0; k < 4; ++k) {
-                    roff[k] = __builtin_amdgcn_readlane(row_of_lane.off, r0 + k);
-                    rw[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(row_of_lane.w), r0 + k));
-                    rlive[k] = r0 + k < nr;
-                  }
-                  if (narrow) block(roff, rw, rlive, coff, cw, std::integral_constant<int, 2>());
-                  else block(roff, rw, rlive, coff, cw, std::integral_constant<int, 4>());
-                }
-              }
+              for (; r0 + MOST <= nr; r0 += MOST) rows(std::integral_constant<int, MOST>());
+              if (MOST > 2 && r0 + 2 == nr) rows(std::integral_constant<int, 2>());
+              else if (r0 < nr) rows(std::integral_constant<int, 1>());
             }
           }
         }
-        // (the reference divides by the number of samples; multiplying by its reciprocal
-        // differs in the last bit only where that number is no power of two)
-#pragma unroll
-        for (int i = 0; i < CPL; ++i) acc[i] *= inv_count;
         if (NHWC) {
           // y[roi][ph][pw][C]: the lane's channels of its bin are 16 contiguous bytes
           if (bin_on) {

@@ -1160,6 +1160,31 @@ def test_adaptive_grids_at_the_edges_of_the_lists(dtype, C, pooled):
         assert_parity(part.float().cpu().numpy(), want, tol, 'y')
 
 
+@pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
+@pytest.mark.parametrize('dtype,C,S', [(np.float32, 36, 0), (np.float16, 72, 0), (np.float32, 36, 27), (np.float16, 72, 5)])
+def test_dense_grids_in_one_list_and_rows_that_pooled_rows_share(dtype, C, S, layout):
+    """Grids of up to 26 points no more than a pixel apart are one list, larger ones two and three; the map rows a
+    pooled row ends with are the first of the next, one or two of them, or all (bins below a pixel); fixed grids of
+    either kind.  Boxes on whole pixels (samples meet the map's lattice) and anywhere, also across its borders."""
+    abi.set_impl('auto')
+    rng = np.random.default_rng(C + S)
+    N, pooled = 2, (3, 5)
+    H, W = 66 * pooled[0], 66 * pooled[1]
+    sizes = (0.25, 1, 2, 3.5, 14, 15, 25.75, 26, 26.25, 27, 52, 52.5, 53, 64)
+    bins = np.array([[sizes[i], sizes[(5 * i + k) % len(sizes)]] for i in range(len(sizes)) for k in (0, 3)])
+    at = np.where(np.arange(len(bins))[:, None] % 3 == 0, 0.0, rng.uniform(-4, 4, bins.shape))
+    rois = np.stack([rng.integers(0, N, len(bins)), at[:, 0], at[:, 1], at[:, 0] + bins[:, 1] * pooled[1],
+                     at[:, 1] + bins[:, 0] * pooled[0]], 1).astype(np.float32)
+    x = rng.standard_normal((N, C, H, W)).astype(dtype)
+    want = oracle.forward(x.astype(np.float32), rois, pooled, 1.0, S).astype(dtype).astype(np.float32)
+    if layout == 'nchw':
+        y = abi.forward(abi.to_dev(x), abi.to_dev(rois), pooled, 1.0, S).float().cpu().numpy()
+    else:
+        y = abi.forward_nhwc(abi.to_dev(np.ascontiguousarray(x.transpose(0, 2, 3, 1))), abi.to_dev(rois), pooled, 1.0,
+                             S).float().cpu().numpy().transpose(0, 3, 1, 2)
+    assert_parity(y, want, FWD_TOL if dtype == np.float32 else FP16_TOL, 'y')
+
+
 @pytest.mark.parametrize('W', [200, 203])
 @pytest.mark.parametrize('dtype', [np.float32, np.float16])
 def test_few_boxes_on_a_large_map_copy_only_what_they_touch(W, dtype):
