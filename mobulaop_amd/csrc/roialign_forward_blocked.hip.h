@@ -24,7 +24,7 @@ namespace roialign {
 struct FwdBlocked {
   static constexpr int NW = 4;         // independent wavefronts per workgroup
   static constexpr int MAXT = 16;      // column samples held in LDS (two for each of 8 pooled columns)
-  static constexpr int ROWT = 64;      // row samples held in LDS at a time
+  static constexpr int ROWT = 16;      // pooled rows whose map rows are held in LDS at a time
   static constexpr int PWB = 8;        // pooled columns per step (one per group of 8 lanes)
   static constexpr int CELL = 32;      // side of the sorting cells in pixels
   static constexpr int MAXCELLS = 8192;
@@ -53,7 +53,8 @@ inline int blocked_rows_per_pass(int C, long long H, long long W, int PH, int PW
   // straightforward kernel, which touches no padding, is the better one)
   if (C < B::CPL || PW < 1 || B::CB * PW > stage) return 0;
   if (H * W * 128 >= (1ll << 31)) return 0;
-  return min(PH, stage / (B::CB * PW));
+  // (the plans of a pass's pooled rows lie in LDS at a time)
+  return min(merged ? PH : min(PH, FwdBlocked::ROWT), stage / (B::CB * PW));
 }
 
 struct OrderArgs {
@@ -261,11 +262,74 @@ roi_order_kernel(const float* __restrict__ rois, int R, float scale, int H, int 
   roi_order_body<1024, FwdBlocked::MAXCELLS>(hist, wave_sum, &carry, rois, R, scale, H, W, num_images, order);
 }
 
-// A row sample: byte offsets of its low and high row in a channel block's
-// plane (lo negative: the sample lies outside the map) and their weights.
-struct alignas(16) RowEntry { int lo, hi; float wl, wh; };
-// A column sample, likewise, with the offsets in bytes along a row.
+// What a pooled row takes from the map: up to four map rows (byte offsets in a channel block's plane) with their
+// weights, and the weights of the two rows that were fetched last before it.  `fetched`: how many rows are
+// fetched; kUsesOlder, kUsesNewer: whether the older and the newer of those two rows are used again.
+struct alignas(16) RowPlan {
+  static constexpr int kFetched = 7, kUsesOlder = 8, kUsesNewer = 16;
+  int off[4];
+  int code;
+  float older, newer, unused;
+  float w[4];
+};
+// A column sample: byte offsets along a row of its low and high column (lo negative: the sample lies outside the map)
+// and their weights.
 struct alignas(16) ColEntry { int lo, hi; float wl, wh; };
+
+// The plans of `count` <= 32 pooled rows from `first` on (at most two sample rows each; called by a whole wavefront, a lane
+// per sample row).  Samples less than a pixel apart share map rows: a row that both samples of a pooled row touch is
+// fetched once with the sum of its weights, and rows of the sample before this pooled row are still at hand (the caller
+// keeps the sums of the two rows it fetched last within a pass of `pass_rows`; 0: it keeps none).  A row whose weight is
+// exactly zero is multiplied by itself all the same (an infinity there makes the result NaN, as it does sample by
+// sample): such pooled rows share nothing.  (Decided for every pooled row as it came, with some forty branches: 827 against
+// 763 us for 8192 boxes of 256 channels, 14 x 14.)
+__device__ __forceinline__ void plan_pooled_rows(RowPlan* plans, const RoiGeom& g, int first, int count, int gh, int H,
+                                                 int row_bytes, int pass_rows) {
+  const int lane = threadIdx.x & 63, at = lane >> 1;
+  const AxisSample a = axis_sample(sample_coord(g.start_h, first + at, g.bin_h, lane & (gh - 1), gh), H);
+  const int low = a.valid ? a.low : -1;
+  const bool weighty = !a.valid || (a.l != 0.0f && a.h != 0.0f);
+  const int next_low = __shfl_down(low, 1), next_high = __shfl_down(a.high, 1), next_weighty = __shfl_down(weighty, 1);
+  const float next_l = __shfl_down(a.l, 1);
+  // the sample rows of the pooled row before: the last one, and the one before that
+  const int last_low = __shfl_up(low, 1), last_high = __shfl_up(a.high, 1), last_weighty = __shfl_up(weighty, 1);
+  const int before_low = __shfl_up(low, 2), before_weighty = __shfl_up(weighty, 2);
+  if ((lane & 1) != 0 || at >= count) return;
+  RowPlan* const plan = plans + at;
+  const bool both = gh > 1 && next_low >= 0;
+  int row[4] = {a.low, a.high, next_low, next_high};
+  float w[4] = {a.h, a.l, 1.0f - next_l, next_l};
+  bool on[4] = {a.valid, a.valid, both, both};
+  int code = 0;
+  float older = 0.0f, newer = 0.0f;
+  if (weighty && (next_weighty || !both)) {
+#pragma unroll
+    for (int k = 2; k < 4; ++k)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        if (on[k] && on[j] && row[k] == row[j]) { w[j] += w[k]; on[k] = false; }
+    // rows only go up: the two rows that were fetched last are those of the last sample
+    if (pass_rows > 0 && at % pass_rows != 0 && last_low >= 0 && last_weighty && before_weighty && before_low <= last_low &&
+        (!a.valid || last_low <= a.low) && (!both || (last_low <= next_low && low <= next_low))) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (on[k] && row[k] == last_low) { older = w[k]; code |= RowPlan::kUsesOlder; on[k] = false; }
+        if (on[k] && row[k] == last_high) { newer = w[k]; code |= RowPlan::kUsesNewer; on[k] = false; }
+      }
+    }
+  }
+  int n = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if (on[k]) {
+      plan->off[n] = row[k] * row_bytes;
+      plan->w[n] = w[k];
+      ++n;
+    }
+  plan->code = code | n;
+  plan->older = older;
+  plan->newer = newer;
+}
 
 // Sixteen bytes of consecutive channels as they lie in a lane's registers: four
 // fp32 or eight 16-bit values (kept packed; an element is widened where it is used).
@@ -364,7 +428,7 @@ forward_blocked_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
   constexpr int CPL = BlockOf<T>::CPL, CB = BlockOf<T>::CB, STAGE = BlockOf<T>::STAGE;
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
   constexpr int CWIN = K::MAXT / K::PWB;   // column samples per pooled column held at a time
-  __shared__ RowEntry rows_s[K::NW][K::ROWT];
+  __shared__ RowPlan rows_s[K::NW][K::ROWT];
   __shared__ ColEntry cols_s[K::NW][K::MAXT];
   __shared__ __attribute__((aligned(16))) T stage_s[K::NW][STAGE];
 
@@ -423,7 +487,7 @@ forward_blocked_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
   // count is a power of two for the usual sampling ratios: multiply by its exact reciprocal
   const bool pow2 = (gh & (gh - 1)) == 0 && (gw & (gw - 1)) == 0;
   const float inv_count = 1.0f / count;
-  RowEntry* const rows = rows_s[wave];
+  RowPlan* const rows = rows_s[wave];
   ColEntry* const cols = cols_s[wave];
   T* const stage = stage_s[wave];
   // NHWC: the caller's [N][H][W][C] map is read where it lies, a pixel's channels C * sizeof(T) apart
@@ -439,22 +503,13 @@ forward_blocked_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
   const __amdgpu_buffer_rsrc_t plane = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<char*>(plane_ptr), 0, H * row_bytes - (NHWC ? cb * 128 : 0), 0x00020000);
 
-  // LDS holds a window of the row samples (flat index ph * gh + iy) and, for the
-  // current block of 8 pooled columns, a window of CWIN column samples each.
-  // Both are refilled by the whole wavefront when a step leaves the window;
-  // with the usual grids one fill per ROI covers everything.
-  int row_s0 = 0, row_s1 = 0;
-  auto need_rows = [&](int s, int n) {
-    if (s < row_s0 || s + n > row_s1) {
-      row_s0 = s;
-      row_s1 = min(s + K::ROWT, PH * gh);
-      for (int i = lane; i < row_s1 - row_s0; i += 64) {
-        const int f = row_s0 + i, ph = f / gh, iy = f - ph * gh;
-        const AxisSample a = axis_sample(sample_coord(g.start_h, ph, g.bin_h, iy, gh), H);
-        rows[i] = RowEntry{a.valid ? a.low * row_bytes : -1, a.high * row_bytes, a.h, a.l};
-      }
-    }
-  };
+  // With eight channels per lane the sums of two rows would not fit the registers that four wavefronts
+  // per SIMD leave: 16-bit maps share rows within a pooled row only.
+  constexpr bool CARRY = CPL <= 4;
+  // LDS holds the plans of a window of pooled rows, filled where a pass leaves it, and, for the
+  // current block of 8 pooled columns, a window of CWIN column samples each, filled where a step does; with the
+  // usual pooled maps one fill per ROI covers everything.  (The first pooled row of a pass finds no sums kept.)
+  int row_p0 = 0, row_p1 = 0;
   int col_pwb = -1, col_x0 = 0, col_x1 = 0;
   auto need_cols = [&](int pwb, int ix, int n) {
     if (pwb != col_pwb || ix < col_x0 || ix + n > col_x1) {
@@ -472,6 +527,11 @@ forward_blocked_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
   const int staged = staged_pitch<T>(rows_per_pass, PH, PW, STAGE);
   for (int ph0 = ph_first; ph0 < ph_end; ph0 += rows_per_pass) {
     const int rp = min(rows_per_pass, ph_end - ph0), seg = rp * PW, pitch = rp == PH ? seg : staged;
+    if (image_ok && ph0 + rp > row_p1) {
+      row_p0 = ph0;
+      row_p1 = min(ph0 + K::ROWT, ph_end);
+      plan_pooled_rows(rows, g, ph0, row_p1 - row_p0, gh, H, row_bytes, CARRY ? rows_per_pass : 0);
+    }
     for (int pwb = 0; pwb < PW; pwb += K::PWB) {
       const int pw = pwb + grp;
       const bool bin_on = pw < PW && quad_on;
@@ -503,109 +563,79 @@ forward_blocked_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
       // pixel apart need three (two when both samples of every bin share their pixels)
       const int ncol = !image_ok ? 2 : __ballot(coff[3] != kDead) != 0 ? 4 : __ballot(coff[2] != kDead) != 0 ? 3 : 2;
       // A map row's contribution to this lane's pooled column, t(row) = sum over the column
-      // corners of weight x value, is the same for every sample that touches the row: samples
-      // less than a pixel apart share rows, within a bin and from one bin to the next (rows
-      // only go up), so t of the two rows of the last sample is carried along and a row is
-      // fetched once per pooled column however many samples use it.
-      // (With eight channels per lane the carried sums would not fit the registers that four
-      // wavefronts per SIMD leave: 16-bit maps share rows within a pooled row only.)
-      constexpr bool CARRY = CPL <= 4;
-      int carry_off[2] = {kDead, kDead};   // (no row has this offset)
-      float carry[2][CPL];
+      // corners of weight x value, is the same for every sample that touches the row: a row is fetched once per
+      // pooled column however many samples use it, and the sums of the two rows fetched last are kept.
+      float kept[2][CPL];
 #pragma unroll
-      for (int i = 0; i < CPL; ++i) carry[0][i] = carry[1][i] = 0.0f;
+      for (int i = 0; i < CPL; ++i) kept[0][i] = kept[1][i] = 0.0f;
       auto pooled_rows = [&](auto corner_slots) {
         constexpr int NC = decltype(corner_slots)::value;
+        // The plan of a pooled row is the same for every lane.  What steers the fetches sits in scalar registers
+        // and is read from LDS a pooled row ahead.
+        int off[4] = {}, code = 0;
+        float older = 0.0f, newer = 0.0f;
+        auto take = [&](int ph) {
+          const RowPlan& r = rows[ph - row_p0];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) off[k] = r.off[k];
+          code = r.code; older = r.older; newer = r.newer;
+        };
+        if (image_ok) take(ph0);
 #pragma nounroll
         for (int ph = ph0; ph < ph0 + rp; ++ph) {
           float acc[CPL];
 #pragma unroll
           for (int i = 0; i < CPL; ++i) acc[i] = 0.0f;
           if (image_ok) {
-            // Row corners of samples 0 and 1: the same for every lane, so they sit in scalar
-            // registers and steer uniform branches.
-            need_rows(ph * gh, gh);
-            int roff[4];
-            float rw[4];
-            int from[4];   // -1: no such corner; 0: loaded; 5, 6: the carried rows; 7: the sample's other row
-            {
-              int known[2] = {carry_off[0], carry_off[1]};   // the carried rows by the time of each sample
+            const int from[4] = {uni_i(off[0]), uni_i(off[1]), uni_i(off[2]), uni_i(off[3])}, steer = uni_i(code);
+            const float w_older = older, w_newer = newer;
+            float w[4];
 #pragma unroll
-              for (int a = 0; a < 2; ++a) {
-                const RowEntry e = rows[ph * gh + min(a, gh - 1) - row_s0];
-                const int lo = uni_i(e.lo), hi = uni_i(e.hi);
-                roff[2 * a] = lo; roff[2 * a + 1] = hi;
-                rw[2 * a] = uni_f(e.wl); rw[2 * a + 1] = uni_f(e.wh);
-                if (lo >= 0 && a < gh) {
-                  from[2 * a] = lo == known[0] ? 5 : lo == known[1] ? 6 : 0;
-                  from[2 * a + 1] = hi == lo ? 7 : hi == known[0] ? 5 : hi == known[1] ? 6 : 0;
-                  known[0] = lo; known[1] = hi;
-                } else {
-                  from[2 * a] = from[2 * a + 1] = -1;
+            for (int k = 0; k < 4; ++k) w[k] = rows[ph - row_p0].w[k];
+            if (ph + 1 < ph0 + rp) take(ph + 1);
+            // one straight line for every number of rows that are fetched: all loads, then the sums
+            auto fetch = [&](auto rows_fetched) {
+              constexpr int NR = decltype(rows_fetched)::value;
+              typename LaneData<T>::type v[NR > 0 ? NR : 1][NC];
+#pragma unroll
+              for (int r = 0; r < NR; ++r)
+#pragma unroll
+                for (int c = 0; c < NC; ++c) v[r][c] = buffer_load_lane<T>(plane, coff[c], from[r]);
+              if constexpr (CARRY) {
+                if (steer & RowPlan::kUsesOlder) {
+#pragma unroll
+                  for (int i = 0; i < CPL; ++i) acc[i] = w_older * kept[0][i];
+                }
+                if (steer & RowPlan::kUsesNewer) {
+#pragma unroll
+                  for (int i = 0; i < CPL; ++i) acc[i] = fmaf(w_newer, kept[1][i], acc[i]);
                 }
               }
-            }
-            // up to sixteen corners: four rows (scalar) x four columns (per lane)
-            typename LaneData<T>::type v[4][NC];
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (from[r] == 0) {
+              for (int r = 0; r < NR; ++r) {
 #pragma unroll
-                for (int c = 0; c < NC; ++c) v[r][c] = buffer_load_lane<T>(plane, coff[c], roff[r]);
-              }
-            if constexpr (CARRY) {
+                for (int i = 0; i < CPL; ++i) {
+                  float u = cw[0] * static_cast<float>(v[r][0][i]);
 #pragma unroll
-              for (int a = 0; a < 2; ++a) {
-                if (from[2 * a] < 0) continue;
-                float t[2][CPL];
-#pragma unroll
-                for (int k = 0; k < 2; ++k) {
-                  const int r = 2 * a + k;
-                  if (from[r] == 0) {
-#pragma unroll
-                    for (int i = 0; i < CPL; ++i) {
-                      float u = cw[0] * static_cast<float>(v[r][0][i]);
-#pragma unroll
-                      for (int c = 1; c < NC; ++c) u = fmaf(cw[c], static_cast<float>(v[r][c][i]), u);
-                      t[k][i] = u;
+                  for (int c = 1; c < NC; ++c) u = fmaf(cw[c], static_cast<float>(v[r][c][i]), u);
+                  acc[i] = fmaf(w[r], u, acc[i]);
+                  if constexpr (CARRY) {
+                    if (r == NR - 1) {
+                      if (NR == 1) kept[0][i] = kept[1][i];
+                      kept[1][i] = u;
+                    } else if (r == NR - 2) {
+                      kept[0][i] = u;
                     }
-                  } else if (from[r] == 5) {
-#pragma unroll
-                    for (int i = 0; i < CPL; ++i) t[k][i] = carry[0][i];
-                  } else if (from[r] == 6) {
-#pragma unroll
-                    for (int i = 0; i < CPL; ++i) t[k][i] = carry[1][i];
-                  } else {
-#pragma unroll
-                    for (int i = 0; i < CPL; ++i) t[k][i] = t[0][i];
-                  }
-#pragma unroll
-                  for (int i = 0; i < CPL; ++i) acc[i] = fmaf(rw[r], t[k][i], acc[i]);
-                }
-                carry_off[0] = roff[2 * a]; carry_off[1] = roff[2 * a + 1];
-#pragma unroll
-                for (int i = 0; i < CPL; ++i) { carry[0][i] = t[0][i]; carry[1][i] = t[1][i]; }
-              }
-            } else {
-              // a repeated row's weight goes to the corner that fetched the row
-              if (from[1] == 7) rw[0] += rw[1];
-              if (from[3] == 7) rw[2] += rw[3];
-#pragma unroll
-              for (int r = 2; r < 4; ++r) {
-                if (from[r] == 5) rw[0] += rw[r];
-                if (from[r] == 6) rw[1] += rw[r];
-              }
-#pragma unroll
-              for (int r = 0; r < 4; ++r)
-                if (from[r] == 0) {
-#pragma unroll
-                  for (int i = 0; i < CPL; ++i) {
-                    float u = cw[0] * static_cast<float>(v[r][0][i]);
-#pragma unroll
-                    for (int c = 1; c < NC; ++c) u = fmaf(cw[c], static_cast<float>(v[r][c][i]), u);
-                    acc[i] = fmaf(rw[r], u, acc[i]);
                   }
                 }
+              }
+            };
+            switch (steer & RowPlan::kFetched) {
+              case 4: fetch(std::integral_constant<int, 4>()); break;
+              case 3: fetch(std::integral_constant<int, 3>()); break;
+              case 2: fetch(std::integral_constant<int, 2>()); break;
+              case 1: fetch(std::integral_constant<int, 1>()); break;
+              default: fetch(std::integral_constant<int, 0>());
             }
           }
           if (pow2) {

@@ -1161,6 +1161,34 @@ def test_adaptive_grids_at_the_edges_of_the_lists(dtype, C, pooled):
 
 
 @pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
+@pytest.mark.parametrize('pooled,S', [((35, 3), 2), ((17, 7), 1), ((16, 14), 2), ((3, 2), 1)])
+def test_pooled_rows_that_share_map_rows_or_weigh_one_with_zero(pooled, S, layout):
+    """Pooled rows beyond the sixteen that are planned at a time, passes that start on a shared row, samples on the map's
+    lattice: the row above one has weight zero, and an infinity in it is a NaN in the bin, as in the reference."""
+    abi.set_impl('auto')
+    rng = np.random.default_rng(pooled[0] + S)
+    N, C, H, W = 2, 36, 41, 19
+    bins = np.array([0.25, 0.5, 1.0, 1.0, 1.5, 2.0, 0.7, 1.3] * 3, np.float32)   # height of a bin
+    at = np.concatenate([np.full(8, 0.25 if S == 2 else 0.5), np.full(8, -1.0), rng.uniform(-3, 30, 8)])
+    x1 = rng.uniform(0.31, 0.39, len(bins))   # (columns meet no lattice point: their weights are never zero)
+    rois = np.stack([rng.integers(0, N, len(bins)), x1, at, x1 + 0.7 * pooled[1], at + bins * pooled[0]], 1).astype(np.float32)
+    x = rng.standard_normal((N, C, H, W)).astype(np.float32)
+    for infinite in (False, True):
+        if infinite:
+            x[:, ::5, 3::6] = np.inf
+        want = oracle.forward(x, rois, pooled, 1.0, S)
+        if layout == 'nchw':
+            y = abi.forward(abi.to_dev(x), abi.to_dev(rois), pooled, 1.0, S).cpu().numpy()
+        else:
+            y = abi.forward_nhwc(abi.to_dev(np.ascontiguousarray(x.transpose(0, 2, 3, 1))), abi.to_dev(rois), pooled, 1.0,
+                                 S).cpu().numpy().transpose(0, 3, 1, 2)
+        assert (np.isnan(y) == np.isnan(want)).all() and (np.isposinf(y) == np.isposinf(want)).all()
+        assert infinite == bool(np.isnan(want).any())
+        finite = np.isfinite(want)
+        assert_parity(y[finite], want[finite], FWD_TOL, 'y')
+
+
+@pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
 @pytest.mark.parametrize('dtype,C,S', [(np.float32, 36, 0), (np.float16, 72, 0), (np.float32, 36, 27), (np.float16, 72, 5)])
 def test_dense_grids_in_one_list_and_rows_that_pooled_rows_share(dtype, C, S, layout):
     """Grids of up to 26 points no more than a pixel apart are one list, larger ones two and three; the map rows a
