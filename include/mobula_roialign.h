@@ -318,8 +318,10 @@ void mobula_hip_clear_error(void);
  * width from the size of the map, 56 or 28 fixes it; "roialign_row_split": 0
  * (default) lets it choose how many wavefronts share a tile row's work list,
  * 1 or 4 fixes it; "roialign_row_quads": 1 (default) lets it write rows of maps
- * whose width is a multiple of four 16 bytes at a time, 0 element by element --
- * all three for tests, the results do not depend on them beyond the order of
+ * whose width is a multiple of four 16 bytes at a time, 0 element by element;
+ * "roialign_few_boxes": 1 (default) lets a few boxes on a small map go back in
+ * one launch where that is faster, 0 never, 2 wherever it can (64 boxes) --
+ * all four for tests, the results do not depend on them beyond the order of
  * fp32 sums).  set returns 0, or -1 for an unknown name; get
  * returns -1 for a name never set. */
 int mobula_hip_set_option(const char* name, long long value);

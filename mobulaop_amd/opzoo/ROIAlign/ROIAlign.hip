@@ -14,6 +14,7 @@
 #include "roialign_naive.hip.h"
 #include "roialign_f64.hip.h"
 #include "roialign_backward_blocked.hip.h"
+#include "roialign_backward_few.hip.h"
 #include "roialign_forward_blocked.hip.h"
 #include "roialign_forward_merged.hip.h"
 
@@ -540,6 +541,19 @@ bool nhwc_backward_supported(const Problem& p) {
          static_cast<long long>(p.R) * p.PH * p.PW * p.C * 4 < (1ll << 31);
 }
 
+// Whether backward_few_kernel takes a call: option "roialign_few_boxes" 1 (default) where it is faster, 0 never, 2 wherever it can.
+bool takes_few_boxes(const Problem& p) {
+  using BF = roialign::BwdFew;
+  if (p.R < 1 || p.R > BF::kMostBoxes || (p.S != 1 && p.S != 2) || p.PH * p.S > BF::kMostSamples ||
+      p.PW * p.S > BF::kMostSamples)
+    return false;
+  const long long blocks = roialign::backward_few_blocks(p.N, p.C, p.H, p.W), bins = p.R * p.PH * p.PW;
+  if (p.N >= 65536 || (p.C + BF::CH - 1) / BF::CH >= 65536 || blocks >= (1ll << 31)) return false;
+  const long long option = mobula_hip::option("roialign_few_boxes", 1);
+  if (option == 0 || mobula_hip::option("roialign_impl", kAuto) != kAuto) return false;
+  return option == 2 || (bins <= BF::kMostBins && bins * blocks <= BF::kMostLooks && bins * p.R * blocks <= BF::kMostSteps);
+}
+
 template <typename T>
 void backward_device(const Problem& p, const T* dy, const float* rois, T* dx, bool assign,
                      hipStream_t stream) {
@@ -568,6 +582,16 @@ void backward_device(const Problem& p, const T* dy, const float* rois, T* dx, bo
         dy, dx, plan.ranges, plan.sorted, plan.class_counts(), plan.entries, plan.lists,
         plan.grid, plan.layout, p.C, p.H, p.W, p.PH, p.PW, cblk, dy_bytes,
         static_cast<unsigned>(plan.list_bytes), assign ? 1 : 0);
+    MOBULA_HIP_TRY(hipGetLastError());
+    return;
+  }
+  // a handful of boxes on a small map: one launch, no lists
+  if (takes_few_boxes(p)) {
+    const dim3 grid(static_cast<unsigned>((static_cast<long long>(p.H) * p.W + roialign::BwdFew::PIXELS - 1) / roialign::BwdFew::PIXELS),
+                    static_cast<unsigned>((p.C + roialign::BwdFew::CH - 1) / roialign::BwdFew::CH), static_cast<unsigned>(p.N));
+    mobula_hip::KernelTimer timer("backward_few_kernel", stream);
+    roialign::backward_few_kernel<T><<<grid, roialign::BwdFew::NW * 64, 0, stream>>>(
+        dy, rois, dx, p.scale, static_cast<int>(p.R), p.C, p.H, p.W, p.PH, p.PW, p.S, assign ? 1 : 0);
     MOBULA_HIP_TRY(hipGetLastError());
     return;
   }

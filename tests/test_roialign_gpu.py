@@ -812,6 +812,49 @@ def test_non_finite_gradient_of_one_roi_stays_in_its_cells(impl):
         assert not np.isfinite(got[..., :12]).all()
 
 
+@pytest.mark.parametrize('dtype', [np.float32, np.float16])
+@pytest.mark.parametrize('pooled,S', [((7, 7), 2), ((1, 1), 1), ((32, 3), 2), ((5, 32), 2), ((9, 17), 1)])
+@pytest.mark.parametrize('R,C,H,W', [(1, 3, 5, 7), (4, 8, 16, 16), (16, 13, 9, 71), (64, 9, 33, 31)])
+def test_backward_of_a_few_boxes_in_one_launch(R, C, H, W, pooled, S, dtype):
+    """Up to 64 boxes (by itself up to 16), channels and pixels that fill no workgroup, axes of up to 64 samples; boxes
+    across the borders, without extent, of no image, not finite, many on the same pixels; a gradient that is not finite
+    reaches the pixels of its bins and no others."""
+    native.set_option('roialign_few_boxes', 2)
+    try:
+        rng = np.random.default_rng(R + C + pooled[0])
+        N, scale = 3, 0.5
+        at = np.stack([rng.uniform(-4, W / scale, R), rng.uniform(-4, H / scale, R)], 1)
+        wh = np.stack([rng.uniform(0, W / scale, R), rng.uniform(0, H / scale, R)], 1) * rng.choice((0, 0.2, 1.0), (R, 1))
+        rois = np.concatenate([rng.integers(0, N, (R, 1)), at, at + wh], 1).astype(np.float32)
+        if R >= 16:
+            rois[3, 0], rois[5, 0] = N, -1
+            rois[7, 1:] = rois[8, 1:] = (0.0, 0.0, 1.0, 1.0)
+        shape = (N, C, H, W)
+        dy = rng.standard_normal((R, C) + pooled).astype(dtype)
+        tol = BWD_TOL if dtype == np.float32 else FP16_TOL
+        with_image = (rois[:, 0] >= 0) & (rois[:, 0] < N)
+        want = oracle.backward(dy[with_image].astype(np.float32), rois[with_image], shape, scale, S, impl='ordered')
+        got = abi.backward(abi.to_dev(dy), abi.to_dev(rois), shape, scale, S, assign=True).float().cpu().numpy()
+        assert_parity(got, want.astype(dtype).astype(np.float32), tol, 'assign')
+        base = rng.standard_normal(shape).astype(dtype)
+        got = abi.backward(abi.to_dev(dy), abi.to_dev(rois), shape, scale, S, dx=abi.to_dev(base)).float().cpu().numpy()
+        assert_parity(got, (want + base.astype(np.float32)).astype(dtype).astype(np.float32), tol, 'accumulate')
+        infinite = dy.copy()
+        infinite[0] = np.inf
+        got = abi.backward(abi.to_dev(infinite), abi.to_dev(rois), shape, scale, S, assign=True).float().cpu().numpy()
+        # (dy of one everywhere: which pixels the bins of the first box reach, weights of zero included)
+        touched = oracle.backward(np.full((1, C) + pooled, np.inf, np.float32), rois[:1], shape, scale, S, impl='ordered')
+        reached = ~np.isfinite(touched) if with_image[0] else np.zeros(shape, bool)
+        assert (np.isfinite(got) == ~reached).all()
+        assert_parity(got[~reached], want.astype(dtype).astype(np.float32)[~reached], tol, 'pixels that it does not reach')
+        rois[0, 1:] = np.nan   # (a box that is not a number ends; other images are as they were)
+        got = abi.backward(abi.to_dev(dy), abi.to_dev(rois), shape, scale, S, assign=True).float().cpu().numpy()
+        others = [n for n in range(N) if n != int(rois[0, 0])]
+        assert_parity(got[others], want.astype(dtype).astype(np.float32)[others], tol, 'other images')
+    finally:
+        native.set_option('roialign_few_boxes', 1)
+
+
 def test_workspace_can_be_given_back():
     """The scratch buffer grows with the largest call of the thread; a caller
     may release it between phases, and the next call allocates afresh."""
