@@ -273,6 +273,12 @@ void mobula_hip_conv2d_backward(const int device_id, const float* dy, const floa
                                 const int filters, const int kernel_h, const int kernel_w, const int pad_h,
                                 const int pad_w, const int stride_h, const int stride_w,
                                 const int dilation_h, const int dilation_w, float* dx, float* dw);
+/* The same with the bias's gradient db[filters] (null: not wanted), which rides in launches of the others. */
+void mobula_hip_conv2d_gradients(const int device_id, const float* dy, const float* x, const float* weight,
+                                 const int batch, const int channels, const int height, const int width,
+                                 const int filters, const int kernel_h, const int kernel_w, const int pad_h,
+                                 const int pad_w, const int stride_h, const int stride_w,
+                                 const int dilation_h, const int dilation_w, float* dx, float* dw, float* db);
 /* db[filters] (+)= sum of dy over images and pixels; n = filters. */
 void conv2d_backward_bias_cd239a08(const int device_id, const int n, const float* dy,
                                    const int accumulate, const int batch, const int pixels, float* db);

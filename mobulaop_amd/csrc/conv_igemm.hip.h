@@ -415,10 +415,11 @@ enum Compute { kFp32 = 0, kBf16 = 1, kBf16x3 = 2 };
 // contiguous range of tiles and the operand rows these share stay in its L2.
 // Returns -1 for the padding workgroups.
 __host__ __device__ inline int tile_blocks(int count) { return (count + 7) / 8 * 8; }
-__device__ __forceinline__ int tile_of_block(int count) {
-  const int per = (count + 7) / 8, t = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-  return (blockIdx.x >> 3) < per && t < count ? t : -1;
+__device__ __forceinline__ int tile_of_block(int count, unsigned block) {
+  const int per = (count + 7) / 8, t = (block & 7) * per + (block >> 3);
+  return static_cast<int>(block >> 3) < per && t < count ? t : -1;
 }
+__device__ __forceinline__ int tile_of_block(int count) { return tile_of_block(count, blockIdx.x); }
 
 // C[M, Ncols] = A[M, K] x B[K, Ncols], one 128x128 tile per workgroup, over the K
 // steps s_begin .. s_end - 1; results go through the operand functor, or (piece != nullptr: the tile
@@ -705,19 +706,23 @@ igemm_kernel(Ops ops, int row_tiles, TileSplit split, float* __restrict__ piece_
                         piece);
 }
 
-// Results of the split tiles: sum of their pieces, in piece order.
+// Results of the split tiles: sum of their pieces, in piece order.  The pieces of a product, as its launch cut them.
+struct PiecesF32 { const float* buffer; TileSplit split; int row_tiles; unsigned blocks; SplitRange range; };
 template <typename Ops>
-__global__ void __launch_bounds__(256)
-reduce_pieces_kernel(Ops ops, int row_tiles, TileSplit split, const float* __restrict__ piece_buffer, SplitRange range) {
-  if (range.leaves_fp32()) return;
+__device__ __forceinline__ void reduce_pieces_f32(const Ops& ops, const PiecesF32& p, unsigned block) {
+  if (p.range.leaves_fp32()) return;
   constexpr int TILE = Tile::BM * Tile::BN;
-  const int local = blockIdx.x / (TILE / 256), e = (blockIdx.x % (TILE / 256)) * 256 + threadIdx.x;
-  const int t = split.whole + local;
-  const float* p = piece_buffer + static_cast<size_t>(local) * split.pieces * TILE + e;
+  const int local = block / (TILE / 256), e = (block % (TILE / 256)) * 256 + threadIdx.x;
+  const int t = p.split.whole + local;
+  const float* at = p.buffer + static_cast<size_t>(local) * p.split.pieces * TILE + e;
   float sum = 0.0f;
-  for (int i = 0; i < split.pieces; ++i) sum += p[static_cast<size_t>(i) * TILE];
-  const int m = (t % row_tiles) * Tile::BM + e / Tile::BN, n = (t / row_tiles) * Tile::BN + e % Tile::BN;
+  for (int i = 0; i < p.split.pieces; ++i) sum += at[static_cast<size_t>(i) * TILE];
+  const int m = (t % p.row_tiles) * Tile::BM + e / Tile::BN, n = (t / p.row_tiles) * Tile::BN + e % Tile::BN;
   if (m < ops.M && n < ops.Ncols) ops.store(ops.column(n), m, sum);
+}
+template <typename Ops>
+__global__ void __launch_bounds__(256) reduce_pieces_kernel(Ops ops, PiecesF32 pieces) {
+  reduce_pieces_f32(ops, pieces, blockIdx.x);
 }
 
 // Slices of K times tiles, slice-major; every slice writes its own partial.
@@ -736,14 +741,66 @@ igemm_weight_kernel(BackwardWeightOps ops, int k_per_slice, int k_total, int row
                                       k_steps(ops.K), nullptr);
 }
 
+// db[d] = sum of dy[img, d, pixel] over images and pixels, in two steps that ride in launches of other work where there is
+// some (on their own they took 6 and 4 us of a first layer's 93, most of it launch): a wavefront per kPixels pixels of a
+// plane, their sums in the order of dy; then a wavefront per filter, which adds those up in 64 bits.
+struct BiasJob {
+  static constexpr int kPixels = 4096;
+  const float* dy; float* sums; float* db;
+  int N, D, ohw, runs, wide, accumulate;   // runs: of a plane; wide: planes are 16-byte aligned and whole quads
+  unsigned sum_blocks, total_blocks;       // workgroups of four wavefronts; 0: no such job
+};
+__device__ __forceinline__ void bias_sums(const BiasJob& job, unsigned block) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x & 63;
+  const long long unit = static_cast<long long>(block) * 4 + (threadIdx.x >> 6);
+  if (unit >= static_cast<long long>(job.N) * job.D * job.runs) return;
+  const long long plane = unit / job.runs;
+  const int first = static_cast<int>(unit - plane * job.runs) * BiasJob::kPixels, last = min(first + BiasJob::kPixels, job.ohw);
+  const float* const p = job.dy + plane * job.ohw;
+  float s = 0.0f;
+  if (job.wide) {
+    f32x4 v = 0.0f;
+#pragma unroll 4
+    for (int i = first + 4 * lane; i < last; i += 256) v += *reinterpret_cast<const f32x4*>(p + i);
+    s = (v[0] + v[1]) + (v[2] + v[3]);
+  } else {
+#pragma unroll 4
+    for (int i = first + lane; i < last; i += 64) s += p[i];
+  }
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) s += __shfl_xor(s, d);
+  if (lane == 0) job.sums[unit] = s;
+}
+__device__ __forceinline__ void bias_totals(const BiasJob& job, unsigned block) {
+  const int lane = threadIdx.x & 63, d = static_cast<int>(block) * 4 + (threadIdx.x >> 6);
+  if (d >= job.D) return;
+  double sum = 0.0;
+  const int count = job.N * job.runs;
+#pragma unroll 4
+  for (int i = lane; i < count; i += 64) {
+    const int img = i / job.runs;
+    sum += static_cast<double>(job.sums[(static_cast<long long>(img) * job.D + d) * job.runs + i - img * job.runs]);
+  }
+#pragma unroll
+  for (int k = 32; k > 0; k >>= 1) sum += __shfl_xor(sum, k);
+  if (lane == 0) job.db[d] = static_cast<float>(job.accumulate ? static_cast<double>(job.db[d]) + sum : sum);
+}
+__global__ void __launch_bounds__(256) bias_sums_kernel(BiasJob job) { bias_sums(job, blockIdx.x); }
+__global__ void __launch_bounds__(256) bias_totals_kernel(BiasJob job) { bias_totals(job, blockIdx.x); }
+
 // out[i] (+)= sum over slices of partial[s][i].  `groups` (a power of two) threads share an output: each
 // adds a contiguous run of slices, the runs are added in order.  V: outputs per thread (one 16-byte load
 // per slice for four).
 template <int V>
 __global__ void __launch_bounds__(256)
 reduce_slices_kernel(const float* __restrict__ partial, float* __restrict__ out, long long count,
-                     int slices, int groups, int accumulate, SplitRange range) {
+                     int slices, int groups, int accumulate, SplitRange range, BiasJob bias) {
   if (range.leaves_fp32()) return;
+  if (blockIdx.x >= gridDim.x - bias.total_blocks) {
+    bias_totals(bias, blockIdx.x - (gridDim.x - bias.total_blocks));
+    return;
+  }
   typedef float vec __attribute__((ext_vector_type(V)));
   __shared__ vec sums[256];
   const int per_block = 256 / groups, local = threadIdx.x % per_block, group = threadIdx.x / per_block;
@@ -765,16 +822,16 @@ reduce_slices_kernel(const float* __restrict__ partial, float* __restrict__ out,
   *to = accumulate ? *to + s : s;
 }
 
-// sums[part][d] (+)= sum of dy[img, d, :, :] over the images of the part (img = part, part + parts, ...);
-// grid (filters, parts).  V: pixels per load.
+// The same in one step, where there is no memory for sums in between: one workgroup to a filter.
+// db[d] (+)= sum of dy[img, d, :, :]; grid (filters).  V: pixels per load.
 template <int V>
 __global__ void __launch_bounds__(256)
-bias_grad_kernel(const float* __restrict__ dy, float* __restrict__ sums, int N, int D, int ohw, int accumulate) {
+bias_grad_kernel(const float* __restrict__ dy, float* __restrict__ db, int N, int D, int ohw, int accumulate) {
   typedef float vec __attribute__((ext_vector_type(V)));
   __shared__ float part[256];
   const int d = blockIdx.x;
   vec v = 0.0f;
-  for (int img = blockIdx.y; img < N; img += gridDim.y) {
+  for (int img = 0; img < N; ++img) {
     const float* p = dy + (static_cast<size_t>(img) * D + d) * ohw;
 #pragma unroll 4
     for (int i = threadIdx.x * V; i < ohw; i += 256 * V) v += *reinterpret_cast<const vec*>(p + i);
@@ -789,8 +846,7 @@ bias_grad_kernel(const float* __restrict__ dy, float* __restrict__ sums, int N, 
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    float* const to = sums + static_cast<size_t>(blockIdx.y) * D + d;
-    *to = accumulate ? *to + part[0] : part[0];
+    db[d] = accumulate ? db[d] + part[0] : part[0];
   }
 }
 

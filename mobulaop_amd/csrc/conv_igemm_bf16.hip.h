@@ -313,7 +313,7 @@ __device__ __forceinline__ void arrange_weights(const ArrangeJob& job, unsigned 
 struct ExponentWords { TensorWords weights, first, second; };
 template <int FORM>
 __global__ void __launch_bounds__(256)
-prepare_b16_kernel(ArrangeJob weights, BlockedJob first, BlockedJob second, ExponentWords exponents) {
+prepare_b16_kernel(ArrangeJob weights, BlockedJob first, BlockedJob second, ExponentWords exponents, BiasJob bias) {
   __shared__ __attribute__((aligned(16))) float lds[kPrepLdsWords];
   unsigned block = blockIdx.x;
   if (block < first.blocks) {
@@ -327,39 +327,46 @@ prepare_b16_kernel(ArrangeJob weights, BlockedJob first, BlockedJob second, Expo
     else to_blocked<FORM, false>(second, block, lds, exponents.second);
     return;
   }
-  arrange_weights<FORM>(weights, block - second.blocks, exponents.weights);
+  block -= second.blocks;
+  if (block < weights.blocks) {
+    arrange_weights<FORM>(weights, block, exponents.weights);
+    return;
+  }
+  bias_sums(bias, block - weights.blocks);
 }
 
 // The same for products that turn out not to be formed from halves: the three parts of their operands, and the tables of
 // the fp32 kernels behind those.
 struct TapsJob { Tap* taps; int count, KH, KW, plane, dil_h, dil_w; unsigned blocks; };
-__global__ void __launch_bounds__(256)
-prepare_again_kernel(ArrangeJob weights, BlockedJob first, BlockedJob second, ExponentWords exponents, GatherTables tables,
-                     TapsJob taps, SplitRange range, SplitRange other) {
-  if (range.halves_hold() && (other.halves_a == nullptr || other.halves_hold())) return;
-  __shared__ __attribute__((aligned(16))) float lds[kPrepLdsWords];
-  unsigned block = blockIdx.x;
-  if (block < first.blocks) {
-    to_blocked<3, false>(first, block, lds, exponents.first);
+struct AgainJob {
+  ArrangeJob weights; BlockedJob first, second; ExponentWords exponents; GatherTables tables; TapsJob taps;
+  SplitRange range, other;
+  unsigned blocks;
+};
+__device__ __forceinline__ void prepare_again(const AgainJob& job, unsigned block, float* lds) {
+  if (job.range.halves_hold() && (job.other.halves_a == nullptr || job.other.halves_hold())) return;
+  if (block < job.first.blocks) {
+    to_blocked<3, false>(job.first, block, lds, job.exponents.first);
     return;
   }
-  block -= first.blocks;
-  if (block < second.blocks) {
-    to_blocked<3, false>(second, block, lds, exponents.second);
+  block -= job.first.blocks;
+  if (block < job.second.blocks) {
+    to_blocked<3, false>(job.second, block, lds, job.exponents.second);
     return;
   }
-  block -= second.blocks;
-  if (block < weights.blocks) {
-    arrange_weights<3>(weights, block, exponents.weights);
+  block -= job.second.blocks;
+  if (block < job.weights.blocks) {
+    arrange_weights<3>(job.weights, block, job.exponents.weights);
     return;
   }
-  block -= weights.blocks;
-  if (block < tables.weight_blocks + tables.step_blocks) {
-    gather_tables(tables, block);
+  block -= job.weights.blocks;
+  if (block < job.tables.weight_blocks + job.tables.step_blocks) {
+    gather_tables(job.tables, block);
     return;
   }
-  block -= tables.weight_blocks + tables.step_blocks;
-  if (block < taps.blocks) build_taps(taps.taps, taps.count, taps.KH, taps.KW, taps.plane, taps.dil_h, taps.dil_w, block);
+  block -= job.tables.weight_blocks + job.tables.step_blocks;
+  const TapsJob& t = job.taps;
+  if (block < t.blocks) build_taps(t.taps, t.count, t.KH, t.KW, t.plane, t.dil_h, t.dil_w, block);
 }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of_bytes(const void* base, unsigned bytes) {
@@ -658,19 +665,28 @@ struct ProductsB16<kHalves> : ProductsB16<2> {};
 template <>
 struct ProductsB16<3> { static constexpr int COUNT = 6, BEFORE = 3, A[] = {2, 0, 1, 1, 0, 0}, B[] = {0, 2, 1, 0, 1, 0}; };
 
+// A stage of a tile in LDS (halves): a load instruction moves 32 rows x 32 bytes; those of the left operand past its rows
+// bring zeros.
+template <int FORM, typename S>
+struct StageB16 {
+  static constexpr int UNITS = kUnits<FORM>;
+  static constexpr int A_PIECES = UNITS * S::ROWS / 32, A_LOADS = (A_PIECES + S::WAVES - 1) / S::WAVES;
+  static constexpr int LOADS = A_LOADS + UNITS;
+  static constexpr int A_HALVES = A_LOADS * S::WAVES * 32 * 16, HALVES = A_HALVES + UNITS * S::COLS * 16;
+};
+
 // C[M, Ncols] = A[M, K] x B[K, Ncols], the tile of shape S at (m0, n0) over the K steps
 // s_begin .. s_end - 1 (s_begin < s_end).  piece == nullptr: results go through ops.store;
-// otherwise into the dense ROWS x 256 piece.
+// otherwise into the dense ROWS x 256 piece.  lds: S::STAGES stages.
 template <typename Ops, typename S>
 __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, int s_begin, int s_end,
-                                               float* __restrict__ piece) {
+                                               float* __restrict__ piece, unsigned short* lds) {
   using P = ProductsB16<Ops::FORM>;
+  using Stage = StageB16<Ops::FORM, S>;
   constexpr int UNITS = Ops::UNITS, ROWS = S::ROWS, WAVES = S::WAVES, NI = S::NI, NJ = S::NJ;
-  // a load instruction moves 32 rows x 32 bytes; those of the left operand past its rows bring zeros
-  constexpr int A_PIECES = UNITS * ROWS / 32, A_LOADS = (A_PIECES + WAVES - 1) / WAVES, LOADS = A_LOADS + UNITS;
-  constexpr int A_HALVES = A_LOADS * WAVES * 32 * 16, STAGE = A_HALVES + UNITS * S::COLS * 16;
+  constexpr int A_PIECES = Stage::A_PIECES, A_LOADS = Stage::A_LOADS, LOADS = Stage::LOADS;
+  constexpr int A_HALVES = Stage::A_HALVES, STAGE = Stage::HALVES;
   constexpr int STAGES = S::STAGES;
-  __shared__ __attribute__((aligned(1024))) unsigned short lds[STAGES * STAGE];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = (wave / S::WN) * (32 * NI), wn = (wave % S::WN) * (32 * NJ);
 
@@ -916,27 +932,49 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
   }
 }
 
-// The tiles of shape S in column-major order, whole tiles first,
+// A product's tiles of shape S in column-major order, whole tiles first,
 // then the tiles cut along K (see igemm_kernel).
+struct TilesB16 {
+  int row_tiles; TileSplit split; float* piece_buffer; SplitRange range;
+  int blocks;   // workgroups
+};
 template <typename Ops, typename S>
-__global__ void __launch_bounds__(64 * S::WAVES, 2 * S::PER_CU)
-igemm_b16_kernel(Ops ops, int row_tiles, TileSplit split, float* __restrict__ piece_buffer, SplitRange range) {
-  if (Ops::FORM == kHalves ? !range.halves_hold() : range.leaves_split()) return;
+__device__ __forceinline__ void igemm_block_b16(const Ops& ops, const TilesB16& tiles, int block, unsigned short* lds) {
+  if (Ops::FORM == kHalves ? !tiles.range.halves_hold() : tiles.range.leaves_split()) return;
+  const TileSplit& split = tiles.split;
   const int whole_blocks = tile_blocks(split.whole);
   int t, s_begin = 0, s_end = ops.k_steps();
   float* piece = nullptr;
-  if (static_cast<int>(blockIdx.x) < whole_blocks) {
-    t = tile_of_block(split.whole);
+  if (block < whole_blocks) {
+    t = tile_of_block(split.whole, block);
     if (t < 0) return;
   } else {
-    const int q = blockIdx.x - whole_blocks;
+    const int q = block - whole_blocks;
     t = split.whole + q / split.pieces;
     s_begin = (q % split.pieces) * split.steps_per_piece;
     s_end = min(s_end, s_begin + split.steps_per_piece);
-    piece = piece_buffer + static_cast<size_t>(q) * S::ROWS * S::COLS;
+    piece = tiles.piece_buffer + static_cast<size_t>(q) * S::ROWS * S::COLS;
   }
-  const int m0 = (t % row_tiles) * S::ROWS, n0 = (t / row_tiles) * S::COLS;
-  igemm_tile_b16<Ops, S>(ops, m0, n0, s_begin, s_end, piece);
+  const int m0 = (t % tiles.row_tiles) * S::ROWS, n0 = (t / tiles.row_tiles) * S::COLS;
+  igemm_tile_b16<Ops, S>(ops, m0, n0, s_begin, s_end, piece, lds);
+}
+template <typename Ops, typename S>
+__global__ void __launch_bounds__(64 * S::WAVES, 2 * S::PER_CU) igemm_b16_kernel(Ops ops, TilesB16 tiles) {
+  __shared__ __attribute__((aligned(1024))) unsigned short lds[S::STAGES * StageB16<Ops::FORM, S>::HALVES];
+  igemm_block_b16<Ops, S>(ops, tiles, blockIdx.x, lds);
+}
+// Both gradients in tiles of one shape, the weights' first (their sums are the longer ones): one launch instead of two, and
+// the last round of one is filled up by the other.  The first's workgroups are made up to a multiple of eight, so that the
+// other's keep their XCDs.  5 x 96 x 45 x 67, 130 filters 3 x 3, two parts: 22 + 25 us -> 43; 32 x 256 x 56 x 56, 256 filters,
+// halves: 335 + 325 -> 659, one part: 134 + 129 -> 257.
+template <int FORM, typename S>
+__global__ void __launch_bounds__(64 * S::WAVES, 2 * S::PER_CU)
+igemm_gradients_b16_kernel(WeightGradOpsB16<FORM> weight, TilesB16 weight_tiles, BackwardDataOpsB16<FORM> data,
+                           TilesB16 data_tiles) {
+  __shared__ __attribute__((aligned(1024))) unsigned short lds[S::STAGES * StageB16<FORM, S>::HALVES];
+  const int first = (weight_tiles.blocks + 7) / 8 * 8, block = blockIdx.x;
+  if (block >= first) igemm_block_b16<BackwardDataOpsB16<FORM>, S>(data, data_tiles, block - first, lds);
+  else if (block < weight_tiles.blocks) igemm_block_b16<WeightGradOpsB16<FORM>, S>(weight, weight_tiles, block, lds);
 }
 
 // Results of the split tiles: sum of their pieces, in piece order and in 64 bits (there may be hundreds, and
@@ -963,13 +1001,50 @@ template <typename Ops>
 __global__ void __launch_bounds__(256) reduce_pieces_b16_kernel(Ops ops, PiecesB16 pieces) {
   reduce_row_b16(ops, pieces, blockIdx.x);
 }
-// both gradients' pieces in one launch
-template <int FORM>
+// What follows the products of a call rides in as few launches as their order allows (one that finds nothing to do takes
+// 3 us of the device): halves' pieces and, if their operands kept them from halves, the conversions to three parts;
+template <typename Ops>
+__global__ void __launch_bounds__(256) reduce_or_again_kernel(Ops ops, PiecesB16 pieces, AgainJob again) {
+  __shared__ __attribute__((aligned(16))) float lds[kPrepLdsWords];
+  if (blockIdx.x < pieces.blocks) reduce_row_b16(ops, pieces, blockIdx.x);
+  else prepare_again(again, blockIdx.x - pieces.blocks, lds);
+}
+// three parts' pieces and those of the fp32 product that takes their place;
+template <typename Ops, typename Fp32Ops>
+__global__ void __launch_bounds__(256)
+reduce_parts_or_fp32_kernel(Ops ops, PiecesB16 pieces, Fp32Ops fp32, PiecesF32 fp32_pieces) {
+  if (blockIdx.x < pieces.blocks) reduce_row_b16(ops, pieces, blockIdx.x);
+  else reduce_pieces_f32(fp32, fp32_pieces, blockIdx.x - pieces.blocks);
+}
+// and both gradients' pieces, with the bias's sums.
+struct NoJob { unsigned blocks; };
+__device__ __forceinline__ void run_job(const NoJob&, unsigned, float*) {}
+__device__ __forceinline__ void run_job(const AgainJob& again, unsigned block, float* lds) { prepare_again(again, block, lds); }
+struct DataFp32Job { BackwardDataOps ops; PiecesF32 pieces; unsigned blocks; };
+__device__ __forceinline__ void run_job(const DataFp32Job& job, unsigned block, float*) {
+  reduce_pieces_f32(job.ops, job.pieces, block);
+}
+template <int FORM, typename Job>
 __global__ void __launch_bounds__(256)
 reduce_gradients_b16_kernel(BackwardDataOpsB16<FORM> data, PiecesB16 data_pieces, WeightGradOpsB16<FORM> weight,
-                            PiecesB16 weight_pieces) {
-  if (blockIdx.x < data_pieces.blocks) reduce_row_b16(data, data_pieces, blockIdx.x);
-  else reduce_row_b16(weight, weight_pieces, blockIdx.x - data_pieces.blocks);
+                            PiecesB16 weight_pieces, BiasJob bias, Job job) {
+  __shared__ __attribute__((aligned(16))) float lds[std::is_same<Job, AgainJob>::value ? kPrepLdsWords : 4];
+  unsigned block = blockIdx.x;
+  if (block < data_pieces.blocks) {
+    reduce_row_b16(data, data_pieces, block);
+    return;
+  }
+  block -= data_pieces.blocks;
+  if (block < weight_pieces.blocks) {
+    reduce_row_b16(weight, weight_pieces, block);
+    return;
+  }
+  block -= weight_pieces.blocks;
+  if (block < bias.total_blocks) {
+    bias_totals(bias, block);
+    return;
+  }
+  run_job(job, block - bias.total_blocks, lds);
 }
 
 }  // namespace conv

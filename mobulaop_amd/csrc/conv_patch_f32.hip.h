@@ -571,7 +571,13 @@ __device__ __forceinline__ void patch_weight_tile(const PatchWeightOps& ops, int
 // Slices of the chunks times tiles, slice-major; every slice writes its own partial.
 template <typename T, bool WIDE>
 __global__ void __launch_bounds__(T::NT, 2)
-patch_weight_kernel(PatchWeightOps ops, int chunks_per_slice, int chunks, int row_tiles, int tiles_per_slice, int count) {
+patch_weight_kernel(PatchWeightOps ops, int chunks_per_slice, int chunks, int row_tiles, int tiles_per_slice, int count,
+                    BiasJob bias) {
+  const int own = tile_blocks(count);
+  if (static_cast<int>(blockIdx.x) >= own) {
+    bias_sums(bias, blockIdx.x - own);
+    return;
+  }
   const int t = tile_of_block(count);
   if (t < 0) return;
   const int slice = t / tiles_per_slice, tile = t - slice * tiles_per_slice, q = slice * chunks_per_slice;

@@ -252,26 +252,22 @@ struct Conv2DBackward : public Node {
     const ConvArgs& a = args;
     const int dev = dy.device().index();
     const bool want_x = task_should_compute_output(0), want_w = task_should_compute_output(1);
-    if (want_x || want_w) {
+    const bool want_b = bias.defined() && task_should_compute_output(2);
+    if (want_x || want_w || want_b) {
       if (want_x) out[0] = at::empty_like(x);
       if (want_w) out[1] = at::empty_like(weight);
+      if (want_b) out[2] = at::empty_like(bias);
       auto dense = [](const Tensor& t) { return !t.defined() || t.is_contiguous() ? t : at::empty(t.sizes(), t.options()); };
-      const Tensor dx = dense(out[0]), dw = dense(out[1]), xd = x.contiguous(), w = weight.contiguous();
+      const Tensor dx = dense(out[0]), dw = dense(out[1]), db = want_b ? dense(out[2]) : Tensor(), xd = x.contiguous(), w = weight.contiguous();
       begin(dy, {});
-      mobula_hip_conv2d_backward(dev, dy.data_ptr<float>(), xd.data_ptr<float>(), w.data_ptr<float>(), GEOMETRY_OF(x, a),
-                                 want_x ? dx.data_ptr<float>() : nullptr, want_w ? dw.data_ptr<float>() : nullptr);
+      mobula_hip_conv2d_gradients(dev, dy.data_ptr<float>(), xd.data_ptr<float>(), w.data_ptr<float>(), GEOMETRY_OF(x, a),
+                                  want_x ? dx.data_ptr<float>() : nullptr, want_w ? dw.data_ptr<float>() : nullptr,
+                                  want_b ? db.data_ptr<float>() : nullptr);
       raise_if_failed("conv2d_backward");
       if (want_x && !dx.is_same(out[0])) out[0].copy_(dx);
       if (want_w && !dw.is_same(out[1])) out[1].copy_(dw);
+      if (want_b && !db.is_same(out[2])) out[2].copy_(db);
     }
-    if (bias.defined() && task_should_compute_output(2))
-      out[2] = filled_like(bias, [&](const Tensor& db) {
-        begin(dy, {-1, dy.numel(), -1, -1, -1, db.numel()});
-        conv2d_backward_bias_cd239a08(dev, static_cast<int>(db.numel()), dy.data_ptr<float>(), 0,
-                                      static_cast<int>(dy.size(0)), static_cast<int>(dy.size(2) * dy.size(3)),
-                                      db.data_ptr<float>());
-        raise_if_failed("conv2d_backward_bias");
-      });
     return out;
   }
 

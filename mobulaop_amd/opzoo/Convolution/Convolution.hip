@@ -69,17 +69,21 @@ conv::TileSplit split_tiles(int count, int steps, int resident, int room = kMaxP
   return split;
 }
 
+// A product; returns the pieces that are left to be added up.
 template <typename Ops, int MODE>
-void launch_igemm_mode(const Ops& ops, float* piece_buffer, conv::SplitRange range, hipStream_t stream) {
+conv::PiecesF32 launch_igemm_pieces(const Ops& ops, float* piece_buffer, conv::SplitRange range, hipStream_t stream) {
   const int row_tiles = (ops.M + conv::Tile::BM - 1) / conv::Tile::BM;
   const int count = row_tiles * ((ops.Ncols + conv::Tile::BN - 1) / conv::Tile::BN);
   const conv::TileSplit split = split_tiles(count, conv::k_steps(ops.K), resident_workgroups<Ops, MODE>());
   const int rest = count - split.whole;
   const dim3 grid(conv::tile_blocks(split.whole) + rest * split.pieces);
   conv::igemm_kernel<Ops, MODE><<<grid, conv::Tile::NT, 0, stream>>>(ops, row_tiles, split, piece_buffer, range);
-  if (rest > 0)
-    conv::reduce_pieces_kernel<Ops><<<rest * (conv::Tile::BM * conv::Tile::BN / 256), 256, 0, stream>>>(
-        ops, row_tiles, split, piece_buffer, range);
+  return conv::PiecesF32{piece_buffer, split, row_tiles, static_cast<unsigned>(rest) * (conv::Tile::BM * conv::Tile::BN / 256), range};
+}
+template <typename Ops, int MODE>
+void launch_igemm_mode(const Ops& ops, float* piece_buffer, conv::SplitRange range, hipStream_t stream) {
+  const conv::PiecesF32 pieces = launch_igemm_pieces<Ops, MODE>(ops, piece_buffer, range, stream);
+  if (pieces.blocks > 0) conv::reduce_pieces_kernel<Ops><<<pieces.blocks, 256, 0, stream>>>(ops, pieces);
 }
 
 template <typename Ops>
@@ -138,15 +142,21 @@ conv::TileSplit split_b16(const Ops& ops, double* cost) {
   return cut_wins ? cut : whole;
 }
 
-// A bf16 product in tiles of shape S; returns the pieces that are left to be added up.
+// A bf16 product as tiles of shape S, and the pieces that are left to be added up.
 template <typename Ops, typename S>
-conv::PiecesB16 launch_igemm_b16_shape(const Ops& ops, float* piece_buffer, conv::SplitRange range, hipStream_t stream) {
+conv::TilesB16 tiles_b16(const Ops& ops, float* piece_buffer, conv::SplitRange range, conv::PiecesB16* pieces) {
   const conv::TileSplit split = split_b16<Ops, S>(ops, nullptr);
   const int row_tiles = (ops.M + S::ROWS - 1) / S::ROWS;
   const int rest = row_tiles * ((ops.Ncols + S::COLS - 1) / S::COLS) - split.whole;
-  const dim3 grid(conv::tile_blocks(split.whole) + rest * split.pieces);
-  conv::igemm_b16_kernel<Ops, S><<<grid, 64 * S::WAVES, 0, stream>>>(ops, row_tiles, split, piece_buffer, range);
-  return conv::PiecesB16{piece_buffer, split, row_tiles, S::ROWS, static_cast<unsigned>(rest) * S::ROWS, range};
+  *pieces = conv::PiecesB16{piece_buffer, split, row_tiles, S::ROWS, static_cast<unsigned>(rest) * S::ROWS, range};
+  return conv::TilesB16{row_tiles, split, piece_buffer, range, conv::tile_blocks(split.whole) + rest * split.pieces};
+}
+template <typename Ops, typename S>
+conv::PiecesB16 launch_igemm_b16_shape(const Ops& ops, float* piece_buffer, conv::SplitRange range, hipStream_t stream) {
+  conv::PiecesB16 pieces;
+  const conv::TilesB16 tiles = tiles_b16<Ops, S>(ops, piece_buffer, range, &pieces);
+  conv::igemm_b16_kernel<Ops, S><<<tiles.blocks, 64 * S::WAVES, 0, stream>>>(ops, tiles);
+  return pieces;
 }
 
 // Tiles of the height that takes least: high ones where there are many, lower ones where the last row of tiles
@@ -290,19 +300,48 @@ struct PrepB16 {
   conv::ArrangeJob weights{};
   conv::BlockedJob first{}, second{};   // x of a forward pass; dy and x of a backward pass
   template <int FORM>
-  void launch(hipStream_t stream, conv::ExponentWords exponents = {}) const {
-    const unsigned blocks = first.blocks + second.blocks + weights.blocks;
-    if (blocks > 0) conv::prepare_b16_kernel<FORM><<<blocks, 256, 0, stream>>>(weights, first, second, exponents);
+  void launch(hipStream_t stream, conv::ExponentWords exponents = {}, const conv::BiasJob& bias = {}) const {
+    const unsigned blocks = first.blocks + second.blocks + weights.blocks + bias.sum_blocks;
+    if (blocks > 0) conv::prepare_b16_kernel<FORM><<<blocks, 256, 0, stream>>>(weights, first, second, exponents, bias);
   }
 };
 
 // The three parts of operands whose products may not be formed from halves (range, other), and the fp32 kernels' tables.
-void launch_again(const PrepB16& prep, const conv::ExponentWords& words, const conv::GatherTables& tables,
-                  const conv::TapsJob& taps, conv::SplitRange range, conv::SplitRange other, hipStream_t stream) {
-  const unsigned blocks = prep.first.blocks + prep.second.blocks + prep.weights.blocks + tables.weight_blocks +
-                          tables.step_blocks + taps.blocks;
-  conv::prepare_again_kernel<<<blocks, 256, 0, stream>>>(prep.weights, prep.first, prep.second, words, tables, taps, range,
-                                                         other);
+conv::AgainJob again_job(const PrepB16& prep, const conv::ExponentWords& words, const conv::GatherTables& tables,
+                         const conv::TapsJob& taps, conv::SplitRange range, conv::SplitRange other) {
+  return conv::AgainJob{prep.weights, prep.first, prep.second, words, tables, taps, range, other,
+                        prep.first.blocks + prep.second.blocks + prep.weights.blocks + tables.weight_blocks +
+                            tables.step_blocks + taps.blocks};
+}
+
+// The bias's gradient that rides in launches of a call's other work (db == nullptr: none), its sums at `at`.
+size_t bias_bytes(const conv::Geometry& g, const float* db) {
+  const long long runs = (static_cast<long long>(g.OH) * g.OW + conv::BiasJob::kPixels - 1) / conv::BiasJob::kPixels;
+  return db == nullptr ? 0 : align_to_256(sizeof(float) * static_cast<size_t>(g.N) * g.D * runs);
+}
+conv::BiasJob bias_job(int N, int D, int ohw, const float* dy, int accumulate, float* db, char* at) {
+  if (db == nullptr) return conv::BiasJob{};
+  const int runs = (ohw + conv::BiasJob::kPixels - 1) / conv::BiasJob::kPixels;
+  return conv::BiasJob{dy, reinterpret_cast<float*>(at), db, N, D, ohw, runs,
+                       ohw % 4 == 0 && reinterpret_cast<uintptr_t>(dy) % 16 == 0, accumulate,
+                       static_cast<unsigned>((static_cast<long long>(N) * D * runs + 3) / 4), static_cast<unsigned>((D + 3) / 4)};
+}
+// A call's workspace with `*bias_room` bytes for the bias's sums in front, or without them where that is too much (the bias
+// then has launches of its own).  optional: null where not even that can be had, else that is an error.
+char* workspace_with_bias(size_t bytes, bool optional, size_t* bias_room) {
+  if (*bias_room > 0) {
+    char* const ws = static_cast<char*>(mobula_hip::workspace_if_possible(bytes + *bias_room));
+    if (ws != nullptr || failed()) return ws;
+    *bias_room = 0;
+  }
+  return static_cast<char*>(optional ? mobula_hip::workspace_if_possible(bytes) : mobula_hip::workspace(bytes));
+}
+// The job for *db, which is then taken (null: none, or no room for it).
+conv::BiasJob take_bias(const conv::Geometry& g, const float* dy, float** db, size_t bias_room, char* at) {
+  if (bias_room == 0) return conv::BiasJob{};
+  float* const mine = *db;
+  *db = nullptr;
+  return bias_job(g.N, g.D, g.OH * g.OW, dy, 0, mine, at);
 }
 
 enum Fit { kFits, kOther, kError };   // kOther: the shape is for the caller's other kernels
@@ -738,17 +777,17 @@ WeightCut cut_weight(const conv::Geometry& g) {
 }
 
 void reduce_slices(const float* partial, float* out, long long count, int slices, int accumulate, hipStream_t stream,
-                   conv::SplitRange range = {}) {
+                   conv::SplitRange range = {}, const conv::BiasJob& bias = {}) {
   // groups of threads share an output's slices until the device has work; four outputs a thread
   // where they lie on 16-byte boundaries
   const int wide = count % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 ? 4 : 1;
   int groups = 1;
   while (groups < 32 && 2 * groups <= slices && count / wide * groups < 128 * 1024) groups *= 2;
-  const dim3 grid(static_cast<unsigned>((count / wide + 256 / groups - 1) / (256 / groups)));
+  const dim3 grid(static_cast<unsigned>((count / wide + 256 / groups - 1) / (256 / groups)) + bias.total_blocks);
   if (wide == 4)
-    conv::reduce_slices_kernel<4><<<grid, 256, 0, stream>>>(partial, out, count, slices, groups, accumulate, range);
+    conv::reduce_slices_kernel<4><<<grid, 256, 0, stream>>>(partial, out, count, slices, groups, accumulate, range, bias);
   else
-    conv::reduce_slices_kernel<1><<<grid, 256, 0, stream>>>(partial, out, count, slices, groups, accumulate, range);
+    conv::reduce_slices_kernel<1><<<grid, 256, 0, stream>>>(partial, out, count, slices, groups, accumulate, range, bias);
 }
 
 // CU clocks of igemm_weight_kernel: its steps span images and cost a little less than those from patches,
@@ -776,7 +815,7 @@ double weight_patch_cost(const conv::Geometry& g, const WeightCut& cut) {
 }
 
 template <typename T>
-bool weight_gradient_with(const conv::Geometry& g, const float* dy, const float* x, int accumulate, float* dw,
+bool weight_gradient_with(const conv::Geometry& g, const float* dy, const float* x, int accumulate, float* dw, float** db,
                           hipStream_t stream) {
   const WeightCut cut = cut_weight<T>(g);
   if (weight_patch_cost<T>(g, cut) < 0) return false;
@@ -791,20 +830,22 @@ bool weight_gradient_with(const conv::Geometry& g, const float* dy, const float*
   const int per_slice = (chunks + slices - 1) / slices;
   slices = (chunks + per_slice - 1) / per_slice;
   const long long wt = static_cast<long long>(g.D) * cols;
-  char* const ws = static_cast<char*>(mobula_hip::workspace(sizeof(float) * slices * wt));
+  size_t bias_room = bias_bytes(g, *db);
+  char* const ws = workspace_with_bias(sizeof(float) * slices * wt, false, &bias_room);
   if (failed()) return true;
-  conv::PatchWeightOps o{dy, x, reinterpret_cast<float*>(ws), g.N, g.C, g.H, g.W, g.D, g.OH, g.OW, g.stride_h, g.stride_w,
+  const conv::BiasJob bias = take_bias(g, dy, db, bias_room, ws);
+  conv::PatchWeightOps o{dy, x, reinterpret_cast<float*>(ws + bias_room), g.N, g.C, g.H, g.W, g.D, g.OH, g.OW, g.stride_h, g.stride_w,
                          g.pad_h, g.pad_w, g.dil_h, g.dil_w, g.KH, g.KW, cols, cut.px, chunks_per_image, cut.channels,
                          cut.plane, (g.OW - 1) * g.stride_w + (g.KW - 1) * g.dil_w + 1};
   const int count = static_cast<int>(tiles) * slices;
-  const dim3 grid(conv::tile_blocks(count));
+  const dim3 grid(conv::tile_blocks(count) + bias.sum_blocks);
   if (wide)
     conv::patch_weight_kernel<T, true><<<grid, T::NT, cut.lds, stream>>>(o, per_slice, chunks, row_tiles,
-                                                                        static_cast<int>(tiles), count);
+                                                                        static_cast<int>(tiles), count, bias);
   else
     conv::patch_weight_kernel<T, false><<<grid, T::NT, cut.lds, stream>>>(o, per_slice, chunks, row_tiles,
-                                                                         static_cast<int>(tiles), count);
-  reduce_slices(o.partial, dw, wt, slices, accumulate, stream);
+                                                                         static_cast<int>(tiles), count, bias);
+  reduce_slices(o.partial, dw, wt, slices, accumulate, stream, {}, bias);
   MOBULA_HIP_TRY(hipGetLastError());
   return true;
 }
@@ -818,10 +859,10 @@ double weight_fp32_cost(const conv::Geometry& g) {
 }
 
 bool weight_gradient_from_patches(const conv::Geometry& g, const float* dy, const float* x, int accumulate, float* dw,
-                                  hipStream_t stream) {
-  if (g.D > 64) return weight_gradient_with<conv::PatchTile128>(g, dy, x, accumulate, dw, stream);
-  if (g.D > 32) return weight_gradient_with<conv::PatchTile64>(g, dy, x, accumulate, dw, stream);
-  return weight_gradient_with<conv::PatchTile32>(g, dy, x, accumulate, dw, stream);
+                                  float** db, hipStream_t stream) {
+  if (g.D > 64) return weight_gradient_with<conv::PatchTile128>(g, dy, x, accumulate, dw, db, stream);
+  if (g.D > 32) return weight_gradient_with<conv::PatchTile64>(g, dy, x, accumulate, dw, db, stream);
+  return weight_gradient_with<conv::PatchTile32>(g, dy, x, accumulate, dw, db, stream);
 }
 
 // ---- fp32 weight gradient in slices of K (igemm_weight_kernel) --------------------------
@@ -914,37 +955,67 @@ bool forward_b16(const conv::Geometry& g, const float* x, const float* weight, c
   return true;
 }
 
-// Launches the wanted products of a backward pass (operands prepared): one after the other, the pieces of both
-// added up by one kernel behind them.
+// Launches the wanted products of a backward pass (operands prepared): together where their tiles have one shape, else one
+// after the other; what is left of them for one kernel behind.
 template <int FORM>
-void launch_gradients_b16(const BackwardB16<FORM>& b, char* piece_buffers, hipStream_t stream,
-                          conv::SplitRange data_range = {}, conv::SplitRange weight_range = {}) {
+struct GradientPieces { conv::PiecesB16 data{}, weight{}; };
+template <int FORM, int ROWS>
+bool launch_together(const BackwardB16<FORM>& b, int rows, float* first, float* second, hipStream_t stream,
+                     conv::SplitRange data_range, conv::SplitRange weight_range, GradientPieces<FORM>* pieces) {
+  if (rows != ROWS) return false;
+  using S = conv::ShapeB16<ROWS, FORM>;
+  const conv::TilesB16 data = tiles_b16<conv::BackwardDataOpsB16<FORM>, S>(b.data, first, data_range, &pieces->data);
+  const conv::TilesB16 weight = tiles_b16<conv::WeightGradOpsB16<FORM>, S>(b.weight, second, weight_range, &pieces->weight);
+  const int blocks = conv::tile_blocks(weight.blocks) + data.blocks;
+  conv::igemm_gradients_b16_kernel<FORM, S><<<blocks, 64 * S::WAVES, 0, stream>>>(b.weight, weight, b.data, data);
+  return true;
+}
+template <int FORM>
+GradientPieces<FORM> launch_gradients_b16(const BackwardB16<FORM>& b, char* piece_buffers, hipStream_t stream,
+                                          conv::SplitRange data_range = {}, conv::SplitRange weight_range = {}) {
   float* const first = reinterpret_cast<float*>(piece_buffers);
   float* const second = b.with_dx ? first + kPieceBytes / sizeof(float) : first;
-  conv::PiecesB16 data{}, weight{};
-  if (b.with_dx) data = launch_igemm_b16(b.data, first, stream, data_range);
-  if (b.with_dw) weight = launch_igemm_b16(b.weight, second, stream, weight_range);
-  if (data.blocks > 0 && weight.blocks > 0)
-    conv::reduce_gradients_b16_kernel<FORM><<<data.blocks + weight.blocks, 256, 0, stream>>>(b.data, data, b.weight, weight);
-  else if (data.blocks > 0) reduce_b16(b.data, data, stream);
-  else reduce_b16(b.weight, weight, stream);
+  GradientPieces<FORM> pieces;
+  if (b.with_dx && b.with_dw) {
+    const int rows = plan_b16(b.data).rows;
+    if (rows == plan_b16(b.weight).rows) {
+      if constexpr (FORM < 3) {
+        if (launch_together<FORM, 256>(b, rows, first, second, stream, data_range, weight_range, &pieces)) return pieces;
+        if (launch_together<FORM, 192>(b, rows, first, second, stream, data_range, weight_range, &pieces)) return pieces;
+      }
+      if (launch_together<FORM, 128>(b, rows, first, second, stream, data_range, weight_range, &pieces)) return pieces;
+      if (launch_together<FORM, 64>(b, rows, first, second, stream, data_range, weight_range, &pieces)) return pieces;
+    }
+  }
+  if (b.with_dx) pieces.data = launch_igemm_b16(b.data, first, stream, data_range);
+  if (b.with_dw) pieces.weight = launch_igemm_b16(b.weight, second, stream, weight_range);
+  return pieces;
+}
+// The pieces of both, the bias's sums and another job.
+template <int FORM, typename Job>
+void reduce_gradients_b16(const BackwardB16<FORM>& b, const GradientPieces<FORM>& pieces, const conv::BiasJob& bias, const Job& job,
+                          hipStream_t stream) {
+  const unsigned blocks = pieces.data.blocks + pieces.weight.blocks + bias.total_blocks + job.blocks;
+  if (blocks > 0)
+    conv::reduce_gradients_b16_kernel<FORM, Job><<<blocks, 256, 0, stream>>>(b.data, pieces.data, b.weight, pieces.weight, bias, job);
 }
 
-// The gradients that are wanted (null: not).  Both share the copy of dy; where the workspace cannot hold what both
-// need the caller takes one after the other.
+// The gradients that are wanted (null: not; the bias's only beside another).  dx and dw share the copy of dy; where the
+// workspace cannot hold what both need the caller takes one after the other.
 template <int PARTS>
 bool gradients_b16(const conv::Geometry& g, const float* dy, const float* x, const float* weight, int accumulate,
-                   float* dx, float* dw, hipStream_t stream) {
+                   float* dx, float* dw, float** db, hipStream_t stream) {
   BackwardB16<PARTS> b;
   const Fit fit = b.plan(g, dy, x, weight, accumulate, dx, dw);
   if (fit != kFits) return fit == kError;
-  const size_t bytes = b.prep.bytes + (dx != nullptr && dw != nullptr ? 2 : 1) * kPieceBytes;
-  char* const ws = static_cast<char*>(dx != nullptr && dw != nullptr ? mobula_hip::workspace_if_possible(bytes)
-                                                                     : mobula_hip::workspace(bytes));
+  const bool both = dx != nullptr && dw != nullptr;
+  size_t bias_room = bias_bytes(g, *db);
+  char* const ws = workspace_with_bias(b.prep.bytes + (both ? 2 : 1) * kPieceBytes, both, &bias_room);
   if (ws == nullptr || failed()) return failed();
-  char* const pieces = b.place(ws);
-  b.prep.template launch<PARTS>(stream);
-  launch_gradients_b16<PARTS>(b, pieces, stream);
+  const conv::BiasJob bias = take_bias(g, dy, db, bias_room, ws);
+  char* const pieces = b.place(ws + bias_room);
+  b.prep.template launch<PARTS>(stream, {}, bias);
+  reduce_gradients_b16<PARTS>(b, launch_gradients_b16<PARTS>(b, pieces, stream), bias, conv::NoJob{0}, stream);
   MOBULA_HIP_TRY(hipGetLastError());
   return true;
 }
@@ -1035,12 +1106,16 @@ struct ForwardFallback {
     return plan_gather(&plan, "conv2d_forward", g, weight, g.D, g.C, static_cast<long long>(g.C) * g.H * g.W,
                        g.OH * g.OW, g.W, +1, g.C * taps, taps);
   }
+  // (with the pieces of the parts' product that it stands in for)
   void run(const conv::Geometry& g, const float* x, const float* bias, float* y, float* pieces, conv::SplitRange range,
-           hipStream_t stream) const {
+           const conv::ForwardOpsB16<3>& parts, const conv::PiecesB16& parts_pieces, hipStream_t stream) const {
     conv::ForwardOps ops;
     ops.x = x; ops.bias = bias; ops.y = y; ops.g = g; ops.M = g.D; ops.Ncols = g.N * g.OH * g.OW;
     ops.wp = plan.tables.out; ops.steps = plan.tables.steps; ops.K = plan.K;
-    launch_igemm_mode<conv::ForwardOps, conv::kFp32>(ops, pieces, range, stream);
+    const conv::PiecesF32 left = launch_igemm_pieces<conv::ForwardOps, conv::kFp32>(ops, pieces, range, stream);
+    if (parts_pieces.blocks + left.blocks > 0)
+      conv::reduce_parts_or_fp32_kernel<conv::ForwardOpsB16<3>, conv::ForwardOps>
+          <<<parts_pieces.blocks + left.blocks, 256, 0, stream>>>(parts, parts_pieces, ops, left);
   }
 };
 
@@ -1081,22 +1156,24 @@ bool forward_split(const conv::Geometry& g, const float* x, const float* weight,
     const conv::MagnitudeJob job{{x, weight, nullptr}, {x_count, w_count, 0}, {x_words, w_words, {}}};
     conv::magnitudes_kernel<<<dim3(conv::kMagnitudes, 2), 1024, 0, stream>>>(job);
     halves.prep.launch<conv::kHalves>(stream, words);
-    reduce_b16(halves.ops, launch_igemm_b16(halves.ops, pieces, stream, range), stream);
-    launch_again(parts.prep, words, fp32.plan.tables, {}, range, {}, stream);
+    const conv::PiecesB16 left = launch_igemm_b16(halves.ops, pieces, stream, range);
+    const conv::AgainJob again = again_job(parts.prep, words, fp32.plan.tables, {}, range, {});
+    conv::reduce_or_again_kernel<conv::ForwardOpsB16<conv::kHalves>><<<left.blocks + again.blocks, 256, 0, stream>>>(
+        halves.ops, left, again);
   } else {
     conv::clear_words_kernel<<<1, 64, 0, stream>>>(reinterpret_cast<unsigned*>(ws), 12);
     parts.prep.launch<3>(stream, words);
     build_gather(&fp32.plan, tables, stream, range);
   }
-  reduce_b16(parts.ops, launch_igemm_b16(parts.ops, pieces, stream, range), stream);
-  fp32.run(g, x, bias, y, pieces, range, stream);
+  const conv::PiecesB16 left = launch_igemm_b16(parts.ops, pieces, stream, range);
+  fp32.run(g, x, bias, y, pieces, range, parts.ops, left, stream);
   MOBULA_HIP_TRY(hipGetLastError());
   return true;
 }
 
-// The gradients that are wanted (null: not), from `form`.
+// The gradients that are wanted (null: not; the bias's only beside another), from `form`.
 bool gradients_split(int form, const conv::Geometry& g, const float* dy, const float* x, const float* weight,
-                     int accumulate, float* dx, float* dw, hipStream_t stream) {
+                     int accumulate, float* dx, float* dw, float** db, hipStream_t stream) {
   BackwardB16<3> parts;
   BackwardB16<conv::kHalves> halves;
   GatherPlan plan{};
@@ -1111,9 +1188,11 @@ bool gradients_split(int form, const conv::Geometry& g, const float* dy, const f
   // (the fp32 weight gradient comes last: what it needs takes the place of the operands)
   const size_t operands = std::max(parts.prep.bytes, by_halves ? halves.prep.bytes : 0);
   const size_t first_bytes = operands + plan.bytes + (dx != nullptr && dw != nullptr ? 2 : 1) * kPieceBytes;
-  char* const ws = static_cast<char*>(mobula_hip::workspace_if_possible(
-      kWordBytes + weight_plan.tap_bytes + std::max(first_bytes, weight_plan.bytes)));
+  size_t bias_room = bias_bytes(g, *db);
+  char* const ws = workspace_with_bias(kWordBytes + weight_plan.tap_bytes + std::max(first_bytes, weight_plan.bytes), true,
+                                       &bias_room);
   if (ws == nullptr) return failed();
+  const conv::BiasJob bias = take_bias(g, dy, db, bias_room, ws + kWordBytes);
   const long long dy_count = static_cast<long long>(g.N) * g.D * g.OH * g.OW;
   const long long x_count = dw != nullptr ? static_cast<long long>(g.N) * g.C * g.H * g.W : 0;
   const long long w_count = dx != nullptr ? static_cast<long long>(g.D) * g.C * taps : 0;
@@ -1122,8 +1201,8 @@ bool gradients_split(int form, const conv::Geometry& g, const float* dy, const f
   conv::SplitRange data_range{dy_words.exponents, w_words.exponents, conv::SplitRange::most_exponents(g.D * taps)};
   conv::SplitRange weight_range{dy_words.exponents, x_words.exponents,
                                 conv::SplitRange::most_exponents(static_cast<long long>(g.N) * g.OH * g.OW)};
-  conv::Tap* const built_taps = reinterpret_cast<conv::Tap*>(ws + kWordBytes);
-  char* const at = ws + kWordBytes + weight_plan.tap_bytes;
+  conv::Tap* const built_taps = reinterpret_cast<conv::Tap*>(ws + kWordBytes + bias_room);
+  char* const at = ws + kWordBytes + bias_room + weight_plan.tap_bytes;
   char* const tables = at + operands;
   char* const pieces = tables + plan.bytes;
   const conv::ExponentWords words{w_words, dy_words, x_words};
@@ -1140,22 +1219,28 @@ bool gradients_split(int form, const conv::Geometry& g, const float* dy, const f
     halves.place(at);
     const conv::MagnitudeJob job{{dy, x, weight}, {dy_count, x_count, w_count}, {dy_words, x_words, w_words}};
     conv::magnitudes_kernel<<<dim3(conv::kMagnitudes, 3), 1024, 0, stream>>>(job);
-    halves.prep.launch<conv::kHalves>(stream, words);
-    launch_gradients_b16<conv::kHalves>(halves, pieces, stream, data_range, weight_range);
-    launch_again(parts.prep, words, plan.tables, taps_of_weight, dx != nullptr ? data_range : weight_range,
-                 dx != nullptr && dw != nullptr ? weight_range : conv::SplitRange{}, stream);
+    halves.prep.launch<conv::kHalves>(stream, words, bias);
+    const auto left = launch_gradients_b16<conv::kHalves>(halves, pieces, stream, data_range, weight_range);
+    reduce_gradients_b16<conv::kHalves>(
+        halves, left, bias,
+        again_job(parts.prep, words, plan.tables, taps_of_weight, dx != nullptr ? data_range : weight_range,
+                  dx != nullptr && dw != nullptr ? weight_range : conv::SplitRange{}), stream);
   } else {
     conv::clear_words_kernel<<<1, 64, 0, stream>>>(reinterpret_cast<unsigned*>(ws), 12);
-    parts.prep.launch<3>(stream, words);
+    parts.prep.launch<3>(stream, words, bias);
     if (dx != nullptr) build_gather(&plan, tables, stream, data_range);
   }
-  launch_gradients_b16<3>(parts, pieces, stream, data_range, weight_range);
+  // (the fp32 product's pieces may lie where the parts' product's do: one of the two is not formed)
+  const auto left = launch_gradients_b16<3>(parts, pieces, stream, data_range, weight_range);
+  conv::DataFp32Job data{};
   if (dx != nullptr) {
-    conv::BackwardDataOps ops;
+    conv::BackwardDataOps& ops = data.ops;
     ops.dy = dy; ops.dx = dx; ops.g = g; ops.accumulate = accumulate; ops.M = g.C; ops.Ncols = parts.data.Ncols;
     ops.wp = plan.tables.out; ops.steps = plan.tables.steps; ops.K = plan.K;
-    launch_igemm_mode<conv::BackwardDataOps, conv::kFp32>(ops, reinterpret_cast<float*>(pieces), data_range, stream);
+    data.pieces = launch_igemm_pieces<conv::BackwardDataOps, conv::kFp32>(ops, reinterpret_cast<float*>(pieces), data_range, stream);
+    data.blocks = data.pieces.blocks;
   }
+  reduce_gradients_b16<3>(parts, left, by_halves ? conv::BiasJob{} : bias, data, stream);
   if (dw != nullptr)
     run_weight(weight_plan, g, dy, x, accumulate, dw, at, stream, weight_range, by_halves ? built_taps : nullptr);
   MOBULA_HIP_TRY(hipGetLastError());
@@ -1235,37 +1320,38 @@ SplitChoice choose_split(const conv::Geometry& g, bool dx, bool dw) {
 
 // Both gradients in one go, sharing what prepares their operands; false: not taken, or only as far as *done says.
 bool both_gradients(const conv::Geometry& g, const float* dy, const float* x, const float* weight, float* dx, float* dw,
-                    SplitChoice* done) {
+                    float** db, SplitChoice* done) {
   hipStream_t stream = call_state().stream;
-  if (compute_mode() == conv::kBf16) return gradients_b16<1>(g, dy, x, weight, 0, dx, dw, stream);
-  if (compute_mode() == conv::kBf16x3) return gradients_b16<2>(g, dy, x, weight, 0, dx, dw, stream);
+  if (compute_mode() == conv::kBf16) return gradients_b16<1>(g, dy, x, weight, 0, dx, dw, db, stream);
+  if (compute_mode() == conv::kBf16x3) return gradients_b16<2>(g, dy, x, weight, 0, dx, dw, db, stream);
   const SplitChoice split = choose_split(g, true, true);
   if (split.dx != 0 && split.dw != 0 && split.dx != split.dw) {   // (no copy of dy serves both)
-    if (gradients_split(split.dx, g, dy, x, weight, 0, dx, nullptr, stream)) done->dx = split.dx;
-    if (!failed() && gradients_split(split.dw, g, dy, x, weight, 0, nullptr, dw, stream)) done->dw = split.dw;
+    if (gradients_split(split.dx, g, dy, x, weight, 0, dx, nullptr, db, stream)) done->dx = split.dx;
+    if (!failed() && gradients_split(split.dw, g, dy, x, weight, 0, nullptr, dw, db, stream)) done->dw = split.dw;
   } else if ((split.dx != 0 || split.dw != 0) &&
              gradients_split(std::max(split.dx, split.dw), g, dy, x, weight, 0, split.dx != 0 ? dx : nullptr,
-                             split.dw != 0 ? dw : nullptr, stream)) {
+                             split.dw != 0 ? dw : nullptr, db, stream)) {
     *done = split;
   }
   return done->dx != 0 && done->dw != 0;
 }
 
-// dx (+)= and dw (+)= as the launchers below say; allow_split: whether products of parts have yet to be weighed.
+// dx (+)= and dw (+)= as the launchers below say; allow_split: whether products of parts have yet to be weighed; *db: the
+// bias's gradient, null where none is wanted any more.
 void data_gradient(const conv::Geometry& g, const float* dy, const float* weight, int accumulate, float* dx,
-                   bool allow_split) {
+                   float** db, bool allow_split) {
   if (static_cast<long long>(g.N) * g.C * g.H * g.W == 0) return;
   hipStream_t stream = call_state().stream;
   mobula_hip::KernelTimer timer("conv2d_backward_data", stream);
   if (g.N < 65536) {
     bool taken = false;
-    if (compute_mode() == conv::kBf16) taken = gradients_b16<1>(g, dy, nullptr, weight, accumulate, dx, nullptr, stream);
-    if (compute_mode() == conv::kBf16x3) taken = gradients_b16<2>(g, dy, nullptr, weight, accumulate, dx, nullptr, stream);
+    if (compute_mode() == conv::kBf16) taken = gradients_b16<1>(g, dy, nullptr, weight, accumulate, dx, nullptr, db, stream);
+    if (compute_mode() == conv::kBf16x3) taken = gradients_b16<2>(g, dy, nullptr, weight, accumulate, dx, nullptr, db, stream);
     if (taken) return;
   }
   if (compute_mode() == conv::kFp32) {
     const int form = allow_split ? choose_split(g, true, false).dx : 0;
-    if (form != 0 && gradients_split(form, g, dy, nullptr, weight, accumulate, dx, nullptr, stream)) return;
+    if (form != 0 && gradients_split(form, g, dy, nullptr, weight, accumulate, dx, nullptr, db, stream)) return;
     const DataPatches patches = data_patches(g, dy, weight, dx, accumulate);
     double cost = 0.0;
     if (data_patches_win(g, patches, &cost)) {
@@ -1290,8 +1376,26 @@ void data_gradient(const conv::Geometry& g, const float* dy, const float* weight
   MOBULA_HIP_TRY(hipGetLastError());
 }
 
+// db (+)= sum of dy, on its own.
+void bias_gradient(int batch, int filters, int pixels, const float* dy, int accumulate, float* db, hipStream_t stream) {
+  const conv::BiasJob sizes = bias_job(batch, filters, pixels, dy, accumulate, db, nullptr);
+  const long long units = static_cast<long long>(batch) * filters * sizes.runs;
+  char* ws = nullptr;
+  if (units > 0 && units < (1ll << 31)) ws = static_cast<char*>(mobula_hip::workspace_if_possible(sizeof(float) * units));
+  if (failed()) return;
+  if (ws == nullptr) {   // (a first call under capture: one workgroup to a filter needs no memory)
+    (sizes.wide ? conv::bias_grad_kernel<4> : conv::bias_grad_kernel<1>)<<<filters, 256, 0, stream>>>(dy, db, batch, filters, pixels,
+                                                                                                 accumulate);
+  } else {
+    const conv::BiasJob job = bias_job(batch, filters, pixels, dy, accumulate, db, ws);
+    conv::bias_sums_kernel<<<job.sum_blocks, 256, 0, stream>>>(job);
+    conv::bias_totals_kernel<<<job.total_blocks, 256, 0, stream>>>(job);
+  }
+  MOBULA_HIP_TRY(hipGetLastError());
+}
+
 void weight_gradient(const conv::Geometry& g, const float* dy, const float* x, int accumulate, float* dw,
-                     bool allow_split) {
+                     float** db, bool allow_split) {
   const long long wt = static_cast<long long>(g.D) * g.C * g.KH * g.KW;
   if (static_cast<long long>(g.C) * g.H * g.W * 4 >= (1ll << 31)) {
     set_error("conv2d_backward_weight: images too large for 32-bit byte offsets");
@@ -1301,14 +1405,14 @@ void weight_gradient(const conv::Geometry& g, const float* dy, const float* x, i
   mobula_hip::KernelTimer timer("conv2d_backward_weight", stream);
   if (wt > 0) {
     bool taken = false;
-    if (compute_mode() == conv::kBf16) taken = gradients_b16<1>(g, dy, x, nullptr, accumulate, nullptr, dw, stream);
-    if (compute_mode() == conv::kBf16x3) taken = gradients_b16<2>(g, dy, x, nullptr, accumulate, nullptr, dw, stream);
+    if (compute_mode() == conv::kBf16) taken = gradients_b16<1>(g, dy, x, nullptr, accumulate, nullptr, dw, db, stream);
+    if (compute_mode() == conv::kBf16x3) taken = gradients_b16<2>(g, dy, x, nullptr, accumulate, nullptr, dw, db, stream);
     if (taken) return;
   }
   if (compute_mode() == conv::kFp32 && wt > 0) {
     const int form = allow_split ? choose_split(g, false, true).dw : 0;
-    if (form != 0 && gradients_split(form, g, dy, x, nullptr, accumulate, nullptr, dw, stream)) return;
-    if (weight_gradient_from_patches(g, dy, x, accumulate, dw, stream)) return;
+    if (form != 0 && gradients_split(form, g, dy, x, nullptr, accumulate, nullptr, dw, db, stream)) return;
+    if (weight_gradient_from_patches(g, dy, x, accumulate, dw, db, stream)) return;
   }
   WeightPlan plan;
   if (!plan_weight(&plan, g)) return;
@@ -1428,7 +1532,8 @@ MOBULA_KERNEL conv2d_backward_data_kernel(const int n, const T* dy, const T* wei
       !fits("conv2d_backward_data", 2, static_cast<long long>(g.D) * g.C * g.KH * g.KW) ||
       !fits("conv2d_backward_data", 17, in))
     return;
-  data_gradient(g, dy, weight, accumulate, dx, true);
+  float* no_bias = nullptr;
+  data_gradient(g, dy, weight, accumulate, dx, &no_bias, true);
 }
 
 // dw[D, C, KH, KW] (+)= the gradient with respect to the weights.  n is the
@@ -1450,7 +1555,8 @@ MOBULA_KERNEL conv2d_backward_weight_kernel(const int n, const T* dy, const T* x
       !fits("conv2d_backward_weight", 2, static_cast<long long>(g.N) * g.C * g.H * g.W) ||
       !fits("conv2d_backward_weight", 17, wt))
     return;
-  weight_gradient(g, dy, x, accumulate, dw, true);
+  float* no_bias = nullptr;
+  weight_gradient(g, dy, x, accumulate, dw, &no_bias, true);
 }
 
 // db[D] (+)= sum of dy over images and pixels.  n = D.
@@ -1462,22 +1568,7 @@ MOBULA_KERNEL conv2d_backward_bias_kernel(const int n, const T* dy, const int ac
   if (!fits("conv2d_backward_bias", 1, static_cast<long long>(batch) * n * pixels) ||
       !fits("conv2d_backward_bias", 5, n))
     return;
-  // planes of a filter dealt to as many workgroups as give the device about a thousand, their
-  // sums added in order by a second kernel (one workgroup per filter: 95 us for 64 filters of
-  // 8 x 112 x 112, the memory has 26 MB to give)
-  hipStream_t stream = call_state().stream;
-  int parts = std::max(1, std::min(batch, 1024 / n));
-  const bool wide = pixels % 4 == 0 && reinterpret_cast<uintptr_t>(dy) % 16 == 0;
-  float* sums = db;
-  if (parts > 1) {
-    sums = static_cast<float*>(mobula_hip::workspace_if_possible(sizeof(float) * static_cast<size_t>(parts) * n));
-    if (failed()) return;
-    if (sums == nullptr) { sums = db; parts = 1; }   // (a first call under capture: one workgroup per filter needs none)
-  }
-  (wide ? conv::bias_grad_kernel<4> : conv::bias_grad_kernel<1>)<<<dim3(n, parts), 256, 0, stream>>>(
-      dy, sums, batch, n, pixels, parts > 1 ? 0 : accumulate);
-  if (parts > 1) reduce_slices(sums, db, n, parts, accumulate, stream);
-  MOBULA_HIP_TRY(hipGetLastError());
+  bias_gradient(batch, n, pixels, dy, accumulate, db, call_state().stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -1552,25 +1643,32 @@ void conv2d_backward_weight_ecf81c91(const int device_id, const int n, const flo
   mobula_hip::finish_call();
 }
 
-// Both gradients of a backward pass (a null dx or dw: not wanted), which share the conversions of
-// their operands where the products have bf16 ones: one launch prepares dy for both, x and the weights.
-void mobula_hip_conv2d_backward(const int device_id, const float* dy, const float* x, const float* weight,
-                                CONV_GEOMETRY_PARAMS, float* dx, float* dw) {
+// The gradients of a backward pass (null: not wanted).  Those of x and the weights share the conversions of
+// their operands where the products have bf16 ones: one launch prepares dy for both, x and the weights; the bias's rides
+// in launches of theirs.
+void mobula_hip_conv2d_gradients(const int device_id, const float* dy, const float* x, const float* weight,
+                                 CONV_GEOMETRY_PARAMS, float* dx, float* dw, float* db) {
   if (!on_device("conv2d_backward", device_id)) return;
   mobula_hip::DeviceScope scope(device_id);
   conv::Geometry g;
   SplitChoice done{false, false};
-  if (scope.ok() && describe(&g, "conv2d_backward", CONV_GEOMETRY_ARGS) &&
-      !(dx != nullptr && dw != nullptr && g.N > 0 && g.N < 65536 && both_gradients(g, dy, x, weight, dx, dw, &done)) &&
-      !failed()) {
-    // (what was weighed for both together is not weighed again)
-    const bool weighed = dx != nullptr && dw != nullptr && compute_mode() == conv::kFp32;
-    if (dx != nullptr && !done.dx)
-      data_gradient(g, dy, weight, 0, dx, !weighed);
-    if (dw != nullptr && !done.dw && !failed())
-      weight_gradient(g, dy, x, 0, dw, !weighed);
+  if (scope.ok() && describe(&g, "conv2d_backward", CONV_GEOMETRY_ARGS)) {
+    if (!(dx != nullptr && dw != nullptr && g.N > 0 && g.N < 65536 && both_gradients(g, dy, x, weight, dx, dw, &db, &done)) &&
+        !failed()) {
+      // (what was weighed for both together is not weighed again)
+      const bool weighed = dx != nullptr && dw != nullptr && compute_mode() == conv::kFp32;
+      if (dx != nullptr && !done.dx)
+        data_gradient(g, dy, weight, 0, dx, &db, !weighed);
+      if (dw != nullptr && !done.dw && !failed())
+        weight_gradient(g, dy, x, 0, dw, &db, !weighed);
+    }
+    if (db != nullptr && !failed()) bias_gradient(g.N, g.D, g.OH * g.OW, dy, 0, db, call_state().stream);
   }
   mobula_hip::finish_call();
+}
+void mobula_hip_conv2d_backward(const int device_id, const float* dy, const float* x, const float* weight,
+                                CONV_GEOMETRY_PARAMS, float* dx, float* dw) {
+  mobula_hip_conv2d_gradients(device_id, dy, x, weight, CONV_GEOMETRY_ARGS, dx, dw, nullptr);
 }
 
 void conv2d_backward_bias_cd239a08(const int device_id, const int n, const float* dy, const int accumulate,

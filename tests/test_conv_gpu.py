@@ -530,6 +530,71 @@ def test_bias_gradient_can_be_recorded_first():
         dyd.add_(0)   # (ordinary work between the replays)
 
 
+@pytest.mark.parametrize('wanted', ['x w b', 'w b', 'b'])
+@pytest.mark.parametrize('shape', [
+    (2, 3, 70, 66, 7, 3, 1),       # planes of more than one run of 4096 pixels
+    (3, 16, 65, 63, 130, 1, 1),    # odd planes: no whole quads
+    (5, 34, 9, 7, 3, 3, 2),
+    (300, 16, 3, 3, 66, 3, 1),     # many small planes
+    (4, 64, 31, 33, 256, 3, 1),    # high tiles for both gradients
+])
+def test_bias_gradient_beside_the_others(shape, wanted, compute):
+    """The bias's gradient rides in launches of the other gradients where there are any: sums in pieces of a plane, 64 bits
+    behind those.  A piece's lane adds up to 64 values in fp32 and six levels more join the lanes: 70 roundings of half a unit
+    at most, of the sum of magnitudes."""
+    import mobulaop_amd as mobula
+    N, C, H, W, D, K, stride = shape
+    gen = torch.Generator().manual_seed(sum(shape))
+    x = torch.randn(N, C, H, W, generator=gen).cuda().requires_grad_('x' in wanted)
+    w = (torch.randn(D, C, K, K, generator=gen) / (C * K * K) ** 0.5).cuda().requires_grad_('w' in wanted)
+    b = torch.randn(D, generator=gen).cuda().requires_grad_(True)
+    y = mobula.op.Conv2D(x, w, b, channels=D, kernel_size=(K, K), strides=(stride, stride), padding=(K // 2, K // 2))
+    dy = torch.randn(y.shape, generator=gen).cuda() + 0.5
+    y.backward(dy)
+    exact, size = dy.double().sum((0, 2, 3)), dy.double().abs().sum((0, 2, 3))
+    assert ((b.grad.double() - exact).abs() <= 70 * 2.0 ** -24 * size).all()
+    xr, wr, br = (t.detach().cpu().requires_grad_(t.requires_grad) for t in (x, w, b))
+    F.conv2d(xr, wr, br, stride=stride, padding=K // 2).backward(dy.cpu())
+    if 'x' in wanted:
+        _close(x.grad, xr.grad, 'dx', compute)
+    if 'w' in wanted:
+        _close(w.grad, wr.grad, 'dw', compute)
+
+
+def test_bias_gradient_that_finds_no_room_beside_the_others():
+    """A recorded call cannot grow the workspace: one that was warmed up without a bias leaves none for its sums."""
+    import mobulaop_amd as mobula
+    gen = torch.Generator().manual_seed(8)
+    x, w = torch.randn(2, 3, 64, 64, generator=gen).cuda(), torch.randn(64, 3, 7, 7, generator=gen).cuda().requires_grad_(True)
+    b = torch.zeros(64, device='cuda', requires_grad=True)
+    dy = torch.randn(2, 64, 32, 32, generator=gen).cuda()
+
+    def gradients(*inputs):
+        y = mobula.op.Conv2D(*inputs, channels=64, kernel_size=(7, 7), strides=(2, 2), padding=(3, 3))
+        return torch.autograd.grad(y, inputs[1:], dy)
+
+    stream = torch.cuda.Stream()
+    try:
+        with torch.cuda.stream(stream):
+            native.release_workspace()
+            alone, = gradients(x, w)
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=stream):
+                dw, db = gradients(x, w, b)
+            for _ in range(3):
+                dw.zero_()
+                db.zero_()
+                torch.cuda.synchronize()
+                graph.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(dw, alone)
+                assert ((db.double() - dy.double().sum((0, 2, 3))).abs() <= 1e-4).all()
+            del graph
+    finally:
+        native.unpin_workspace()
+
+
 @pytest.mark.parametrize('mode', ['bf16', 'bf16x3'])
 def test_both_gradients_in_a_workspace_that_holds_the_operands_of_one(mode):
     """The gradients of one call share their operands where the workspace can hold both; where it cannot
