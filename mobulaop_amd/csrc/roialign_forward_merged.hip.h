@@ -104,7 +104,8 @@ __global__ void __launch_bounds__(FwdMerged::NW * 64, 4)
 forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
                       const int* __restrict__ order, T* __restrict__ y, float scale, int C, int H,
                       int W, int PH, int PW, int S, long long num_images, int cblk,
-                      int rows_per_pass, int rois_listed, int parts, const int* __restrict__ direct) {
+                      int rows_per_pass, int rois_listed, int parts, const int* __restrict__ direct,
+                      const T* __restrict__ x, unsigned jobs) {
   using K = FwdBlocked;
   using M = FwdMerged;
   constexpr int CPL = BlockOf<T>::CPL, CB = BlockOf<T>::CB, STAGE = BlockOf<T>::STAGE_MERGED;
@@ -114,6 +115,13 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
   __shared__ int rown_s[M::NW][M::RPH];
   __shared__ __attribute__((aligned(16))) T stage_s[M::NW][STAGE];
   if (direct != nullptr && *direct != 0) return;   // (forward_naive_kernel does the call: choose_direct_kernel)
+  // behind the jobs: boxes of larger grids, from the map itself (as a launch of their own, which found nothing to do for
+  // boxes on their map, they took 4 us a call)
+  if (blockIdx.x >= jobs) {
+    static_assert(M::NW == 1, "a wavefront for 64 boxes");
+    forward_large_grid<T, NHWC>(64ll * (blockIdx.x - jobs), rois_listed, x, scale, C, H, W, PH, PW, S, rois, y, num_images);
+    return;
+  }
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -164,7 +172,7 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
   const int gh = uni_i(g.grid_h), gw = uni_i(g.grid_w);
   const int ws_h = uni_i(M::window(gh, g.bin_h)), ws_w = uni_i(M::window(gw, g.bin_w));
   // A box far larger than the map (or infinite) has up to 2^31 sample points per
-  // bin, nearly all outside the map: forward_large_grid_kernel does those boxes.
+  // bin, nearly all outside the map: forward_large_grid does those boxes.
   if (gh > kSearchedGrid || gw > kSearchedGrid) return;
   const float inv_count = 1.0f / uni_f(g.count);
   MergedEntry (*const rowm)[M::LCAP] = rowm_s[wave];

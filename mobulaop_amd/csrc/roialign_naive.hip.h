@@ -72,18 +72,16 @@ forward_naive_kernel(long long n_out, const T* __restrict__ x, float scale, int 
   }
 }
 
-// The boxes forward_merged_kernel leaves out: those whose sampling grid has more
-// than kSearchedGrid points per bin along an axis.  One wavefront per ROI (it
-// returns at once for every other box); its lanes share out the ROI's outputs
+// The boxes that the merged lists leave out: those whose sampling grid has more
+// than kSearchedGrid points per bin along an axis.  One wavefront for the 64 ROIs from `first` on: a lane
+// looks at one, and for those it finds all lanes share out the outputs
 // and visit only the samples that can be valid.  NHWC: map [N][H][W][C] and
 // pooled tensor [R][PH][PW][C].
 template <typename T, bool NHWC>
-__global__ void __launch_bounds__(64)
-forward_large_grid_kernel(const T* __restrict__ x, float scale, int C, int H, int W, int PH, int PW, int S,
-                          const float* __restrict__ rois, T* __restrict__ y, long long num_images) {
-  const long long r = blockIdx.x;
+__device__ __forceinline__ void forward_large_box(long long r, const T* __restrict__ x, float scale, int C, int H, int W, int PH,
+                                                  int PW, int S, const float* __restrict__ rois, T* __restrict__ y,
+                                                  long long num_images) {
   const RoiGeom g = roi_geometry(rois + r * 5, scale, PH, PW, S);
-  if (g.grid_h <= kSearchedGrid && g.grid_w <= kSearchedGrid) return;
   const bool image_ok = g.batch >= 0 && g.batch < num_images;
   const int bins = PH * PW;
   for (int o = threadIdx.x; o < C * bins; o += 64) {
@@ -113,6 +111,20 @@ forward_large_grid_kernel(const T* __restrict__ x, float scale, int C, int H, in
     }
     y[r * C * bins + o] = from_float<T>(acc / g.count);
   }
+}
+
+template <typename T, bool NHWC>
+__device__ __forceinline__ void forward_large_grid(long long first, int R, const T* __restrict__ x, float scale, int C, int H,
+                                                   int W, int PH, int PW, int S, const float* __restrict__ rois,
+                                                   T* __restrict__ y, long long num_images) {
+  const long long mine = first + (threadIdx.x & 63);
+  bool large = false;
+  if (mine < R) {
+    const RoiGeom g = roi_geometry(rois + mine * 5, scale, PH, PW, S);
+    large = g.grid_h > kSearchedGrid || g.grid_w > kSearchedGrid;
+  }
+  for (unsigned long long left = __ballot(large); left != 0ull; left &= left - 1ull)
+    forward_large_box<T, NHWC>(first + __builtin_ctzll(left), x, scale, C, H, W, PH, PW, S, rois, y, num_images);
 }
 
 // TI: element type of dy; the sums go into an fp32 map.

@@ -291,6 +291,7 @@ __device__ __forceinline__ AxisUnit clip_unit(int bin, const AxisSample& a, int 
 // The wavefront also finds the ROI's box (the pixels any valid sample touches),
 // and stores it as tile ranges for build_tile_work_kernel.
 // `block`: index among the workgroups (of 256 threads) that build lists.
+constexpr long long kSharedItems = 4096;
 constexpr int kWorkClasses = 8;   // of tile rows by the length of their work lists (SortedRow)
 struct ListsArgs {
   const float* rois;
@@ -304,7 +305,14 @@ struct ListsArgs {
   int* cursors;
   AxisUnit* lists;
   const int* window_offsets;   // merged weights: the first item of every ROI (null: one item per ROI)
+  int parts_log;               // merged weights: log2 of the wavefronts that share an item's tiles (lists_parts_log)
 };
+// An item's tables are written tile row by tile row and tile column by tile column, for merged weights several hundred
+// dependent instructions each: with few items wavefronts deal the tiles of one out among them (301 boxes on 3 x 81 x 75 x 113,
+// adaptive grid: 21.6 -> 11.6 us with the search below).  Lists of samples are short beside what comes before their tiles
+// (512 boxes on 2 x 256 x 64 x 64: 12 us, 16 with four wavefronts to a box) and have one.
+inline int lists_parts_log(long long items) { return items <= kSharedItems / 4 ? 2 : items <= kSharedItems / 2 ? 1 : 0; }
+inline long long lists_blocks(long long items, int parts_log) { return std::max(1ll, ((items << parts_log) + 3) / 4); }
 
 __device__ __forceinline__ void build_lists_body(unsigned block, const ListsArgs& a) {
   const float* __restrict__ rois = a.rois;
@@ -465,17 +473,20 @@ __device__ __forceinline__ void build_window_lists_body(unsigned block, const Li
   const TileGrid tg = a.tg;
   const ListLayout ll = a.ll;
   if (block == 0 && threadIdx.x < 2 + kWorkClasses) a.cursors[threadIdx.x] = 0;
-  const int item = static_cast<int>((block * 256u + threadIdx.x) >> 6);
+  const int unit = static_cast<int>((block * 256u + threadIdx.x) >> 6), item = unit >> a.parts_log;
+  const int parts = 1 << a.parts_log, part = unit & (parts - 1);
   if (item >= items) return;
   const int lane = threadIdx.x & 63;
   int roi;
-  {   // the ROI whose items include this one
+  {   // the ROI whose items include this one, among 64 of the rest at a time (every look is a round trip to memory)
     int lo = 0, hi = R;
     while (hi - lo > 1) {
-      const int mid = (lo + hi) / 2;
-      if (a.window_offsets[mid] <= item) lo = mid; else hi = mid;
+      const int step = (hi - lo + 63) / 64, at = lo + step * (lane + 1);
+      const int upto = __popcll(__ballot(at < hi && a.window_offsets[min(at, hi - 1)] <= item));
+      lo += step * upto;
+      hi = min(hi, lo + step);
     }
-    roi = lo;
+    roi = __builtin_amdgcn_readfirstlane(lo);
   }
   const int j = item - a.window_offsets[roi];
   const RoiGeom g = roi_geometry(a.rois + static_cast<long long>(roi) * 5, a.scale, PH, PW, a.S_given);
@@ -499,7 +510,7 @@ __device__ __forceinline__ void build_window_lists_body(unsigned block, const Li
     col_lo = any ? clo : 0; col_hi = any ? chi : -1;
     const int ty0 = row_lo / tg.th, ty1 = any ? row_hi / tg.th : -1;
     const int tx0 = col_lo / tg.tw, tx1 = any ? col_hi / tg.tw : -1;
-    if (lane == 0) a.boxes[item] = TileBox{any ? g.batch : -1, ty0 | (ty1 << 16), tx0 | (tx1 << 16), roi};
+    if (lane == 0 && part == 0) a.boxes[item] = TileBox{any ? g.batch : -1, ty0 | (ty1 << 16), tx0 | (tx1 << 16), roi};
     if (!any) return;
   }
   AxisUnit* const base = a.lists + static_cast<long long>(item) * ll.roi_stride;
@@ -507,7 +518,7 @@ __device__ __forceinline__ void build_window_lists_body(unsigned block, const Li
   {
     // row taps: lane = tile row * 4 + k; the lane takes the pooled rows k, k + 4, ...
     const int r = lane >> 2, k4 = lane & 3;
-    for (int ty = row_lo / tg.th; ty <= row_hi / tg.th; ++ty) {
+    for (int ty = row_lo / tg.th + part; ty <= row_hi / tg.th; ty += parts) {
       const int row = ty * tg.th + r;
       WindowRowTable* const table = reinterpret_cast<WindowRowTable*>(base + ty * ll.row_stride);
       float w[8];
@@ -540,7 +551,7 @@ __device__ __forceinline__ void build_window_lists_body(unsigned block, const Li
     // windows: lane = pooled column (of eight) * 8 + dword of its ColWindow
     const int sub = lane >> 3, slot = (lane & 7) - 1;   // slot -1: the header
     int* const cols = reinterpret_cast<int*>(base + static_cast<long long>(ll.ty) * ll.row_stride);
-    for (int tx = col_lo / tg.tw; tx <= col_hi / tg.tw; ++tx) {
+    for (int tx = col_lo / tg.tw + part; tx <= col_hi / tg.tw; tx += parts) {
       for (int pw0 = 0; pw0 < ll.pw_padded; pw0 += 8) {
         const int pw = pw0 + sub;
         // (every lane takes part in the exchange: the lane asked may be one whose column does not exist)

@@ -195,7 +195,9 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
   const int nw = small_grid ? FB::NW : roialign::FwdMerged::NW;   // wavefronts per workgroup of the gather
   const int parts = roialign::forward_row_parts(p.R, cblk, p.PH, !small_grid);
   const long long grid = roialign::blocked_grid(static_cast<long long>(p.R) * parts, cblk, nw);
-  const bool fits = rpp > 0 && p.N > 0 && p.N < 65536 && cblk < 65536 && grid < (1ll << 31);
+  // boxes whose sampling grid has more than 64 points per axis have workgroups of their own behind the others
+  const long long large_blocks = !small_grid && (p.S <= 0 || p.S > roialign::kSearchedGrid) ? (p.R + 63) / 64 : 0;
+  const bool fits = rpp > 0 && p.N > 0 && p.N < 65536 && cblk < 65536 && grid + large_blocks < (1ll << 31);
   if (p.nhwc) {
     // the map is read where it lies: no copy, only the ROI ordering before the gather
     if (!fits || !nhwc_forward_supported<T>(p) || reinterpret_cast<size_t>(x) % 16 != 0 ||
@@ -218,13 +220,10 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
     } else {
       {
         mobula_hip::KernelTimer timer("forward_merged_kernel", stream);
-        roialign::forward_merged_kernel<T, true><<<static_cast<unsigned>(grid), nw * 64, 0, stream>>>(
-            x, rois, order, y, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, p.N, cblk, p.PH, p.R, parts, nullptr);
+        roialign::forward_merged_kernel<T, true><<<static_cast<unsigned>(grid + large_blocks), nw * 64, 0, stream>>>(
+            x, rois, order, y, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, p.N, cblk, p.PH, p.R, parts, nullptr, x,
+            static_cast<unsigned>(grid));
       }
-      // the boxes that kernel leaves out (sampling grids of more than 64 points per axis)
-      if (p.S <= 0 || p.S > roialign::kSearchedGrid)
-        roialign::forward_large_grid_kernel<T, true><<<static_cast<unsigned>(p.R), 64, 0, stream>>>(
-          x, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, rois, y, p.N);
     }
     MOBULA_HIP_TRY(hipGetLastError());
     return;
@@ -310,13 +309,10 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
       // every pixel of a bin is loaded once
       {
         mobula_hip::KernelTimer timer("forward_merged_kernel", stream, !fixed);
-        roialign::forward_merged_kernel<T, false><<<static_cast<unsigned>(grid), nw * 64, 0, stream>>>(
-            xt, rois, order, y, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, p.N, cblk, rpp, p.R, parts, choice);
+        roialign::forward_merged_kernel<T, false><<<static_cast<unsigned>(grid + large_blocks), nw * 64, 0, stream>>>(
+            xt, rois, order, y, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, p.N, cblk, rpp, p.R, parts, choice, x,
+            static_cast<unsigned>(grid));
       }
-      // the boxes that kernel leaves out (sampling grids of more than 64 points per axis), from the map itself
-      if (p.S <= 0 || p.S > roialign::kSearchedGrid)
-        roialign::forward_large_grid_kernel<T, false><<<static_cast<unsigned>(p.R), 64, 0, stream>>>(
-          x, p.scale, p.C, p.H, p.W, p.PH, p.PW, p.S, rois, y, p.N);
     }
     if (choice != nullptr)
       roialign::forward_naive_kernel<T><<<std::min(2048, grid_for(p.n_out, 256)), 256, 0, stream>>>(
@@ -475,8 +471,8 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
   // two kernels: per-item tables (which also resets the bump pointers), then per-tile lists
   const int n_items = static_cast<int>(items);
   const roialign::ListsArgs la{rois, n_items, p.R, p.scale, p.PH, p.PW, p.S, p.H, p.W, p.N, g, plan->layout,
-                               plan->boxes, plan->cursors, plan->lists, offsets};
-  const long long list_blocks = std::max(1ll, (items * 64 + 255) / 256);
+                               plan->boxes, plan->cursors, plan->lists, offsets, windows ? roialign::lists_parts_log(items) : 0};
+  const long long list_blocks = roialign::lists_blocks(items, la.parts_log);
   const DyLaunch dl = dy_launch<T>(p);
   if (fuse_dy != nullptr && with_dyb && dl.per > 0 && dl.blocks > 0 && dl.blocks + list_blocks < (1ll << 31)) {
     roialign::lists_and_dy_kernel<T><<<static_cast<unsigned>(dl.blocks + list_blocks), 256, dl.lds, stream>>>(

@@ -1256,6 +1256,38 @@ def test_dense_grids_in_one_list_and_rows_that_pooled_rows_share(dtype, C, S, la
     assert_parity(y, want, FWD_TOL if dtype == np.float32 else FP16_TOL, 'y')
 
 
+@pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
+@pytest.mark.parametrize('R', [1, 64, 65, 150, 1025, 2049])
+def test_adaptive_grids_with_items_shared_by_wavefronts_and_boxes_far_larger_than_the_map(R, layout):
+    """Up to 1024 list items have four wavefronts each, up to 2048 two, more one; boxes of more than 64 points per axis are
+    found 64 at a time, the first and the last of such a group among them (the backward pass then takes another way: it is
+    tried without them)."""
+    abi.set_impl('auto')
+    rng = np.random.default_rng(R)
+    N, C, H, W, pooled = 2, 12, 37, 61, (3, 4)
+    at = np.stack([rng.uniform(-3, W, R), rng.uniform(-3, H, R)], 1)
+    rois = np.concatenate([rng.integers(0, N, (R, 1)), at, at + rng.uniform(0, (W, H), (R, 2))], 1).astype(np.float32)
+    x = rng.standard_normal((N, C, H, W)).astype(np.float32)
+    dy = rng.standard_normal((R, C) + pooled).astype(np.float32)
+    nhwc = layout == 'nhwc'
+    if nhwc:
+        dx = abi.backward_nhwc(abi.to_dev(np.ascontiguousarray(dy.transpose(0, 2, 3, 1))), abi.to_dev(rois), (N, H, W, C), 1.0,
+                               0, assign=True).cpu().numpy().transpose(0, 3, 1, 2)
+    else:
+        dx = abi.backward(abi.to_dev(dy), abi.to_dev(rois), x.shape, 1.0, 0, assign=True).cpu().numpy()
+    assert_parity(dx, oracle.backward(dy, rois, x.shape, 1.0, 0, impl='ordered'), BWD_TOL, 'dx')
+    for r in (0, 63, 64, R - 1):
+        if r < R:
+            rois[r, 1:] = (-90.0, 2.0, 300.0, 30.0) if r % 2 else (3.0, -200.0, 40.0, 150.0)
+    want = oracle.forward(x, rois, pooled, 1.0, 0)
+    if nhwc:
+        y = abi.forward_nhwc(abi.to_dev(np.ascontiguousarray(x.transpose(0, 2, 3, 1))), abi.to_dev(rois), pooled, 1.0,
+                             0).cpu().numpy().transpose(0, 3, 1, 2)
+    else:
+        y = abi.forward(abi.to_dev(x), abi.to_dev(rois), pooled, 1.0, 0).cpu().numpy()
+    assert_parity(y, want, FWD_TOL, 'y')
+
+
 @pytest.mark.parametrize('W', [200, 203])
 @pytest.mark.parametrize('dtype', [np.float32, np.float16])
 def test_few_boxes_on_a_large_map_copy_only_what_they_touch(W, dtype):
