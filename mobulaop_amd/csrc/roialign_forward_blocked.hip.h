@@ -53,8 +53,7 @@ inline int blocked_rows_per_pass(int C, long long H, long long W, int PH, int PW
   // straightforward kernel, which touches no padding, is the better one)
   if (C < B::CPL || PW < 1 || B::CB * PW > stage) return 0;
   if (H * W * 128 >= (1ll << 31)) return 0;
-  // (the plans of a pass's pooled rows lie in LDS at a time)
-  return min(merged ? PH : min(PH, FwdBlocked::ROWT), stage / (B::CB * PW));
+  return min(PH, stage / (B::CB * PW));
 }
 
 struct OrderArgs {
@@ -503,6 +502,7 @@ forward_blocked_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
   const __amdgpu_buffer_rsrc_t plane = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<char*>(plane_ptr), 0, H * row_bytes - (NHWC ? cb * 128 : 0), 0x00020000);
 
+  rows_per_pass = min(rows_per_pass, K::ROWT);   // (the plans of a pass's pooled rows lie in LDS at a time)
   // With eight channels per lane the sums of two rows would not fit the registers that four wavefronts
   // per SIMD leave: 16-bit maps share rows within a pooled row only.
   constexpr bool CARRY = CPL <= 4;

@@ -260,6 +260,29 @@ def test_both_tile_widths_of_the_backward(cfg, down, columns, split, quads):
         assert_parity(got.cpu().numpy(), want, BWD_TOL, 'bwd channels-last')
 
 
+@pytest.mark.parametrize('S', [2, 1, 0])
+@pytest.mark.parametrize('split', [1, 4])
+@pytest.mark.parametrize('columns', [16, 20, 36, 60, 64, 0])
+@pytest.mark.parametrize('W', [5, 16, 61, 64, 65, 128])
+def test_every_kind_of_tile_width_of_the_backward(W, columns, split, S):
+    """Tiles as wide as the map, narrower than a window of merged weights and the dummies beside it take in all, cut so that
+    the last one has a column, or chosen by the map."""
+    abi.set_impl('tiled')
+    native.set_option('roialign_tile_columns', columns)
+    native.set_option('roialign_row_split', split)
+    rng = np.random.default_rng(W + columns)
+    N, C, H, R, pooled = 2, 36, 19, 60, (4, 9)
+    at = np.stack([rng.uniform(-3, W, R), rng.uniform(-3, H, R)], 1)
+    rois = np.concatenate([rng.integers(0, N, (R, 1)), at, at + rng.uniform(0, 1, (R, 2)) * (W, H)], 1).astype(np.float32)
+    dy = rng.standard_normal((R, C) + pooled).astype(np.float32)
+    want = oracle.backward(dy, rois, (N, C, H, W), 1.0, S, impl='ordered')
+    got = abi.backward(abi.to_dev(dy), abi.to_dev(rois), (N, C, H, W), 1.0, S, assign=True).cpu().numpy()
+    assert_parity(got, want, BWD_TOL, 'nchw')
+    got = abi.backward_nhwc(abi.to_dev(np.ascontiguousarray(dy.transpose(0, 2, 3, 1))), abi.to_dev(rois), (N, H, W, C), 1.0, S,
+                            assign=True).cpu().numpy().transpose(0, 3, 1, 2)
+    assert_parity(got, want, BWD_TOL, 'nhwc')
+
+
 @pytest.mark.parametrize('C', [1, 6, 35])
 def test_four_column_write_out_with_odd_channel_counts(C):
     """Maps whose width is a multiple of four are written four columns at a time
@@ -1229,6 +1252,26 @@ def test_pooled_rows_that_share_map_rows_or_weigh_one_with_zero(pooled, S, layou
         assert infinite == bool(np.isnan(want).any())
         finite = np.isfinite(want)
         assert_parity(y[finite], want[finite], FWD_TOL, 'y')
+
+
+@pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
+@pytest.mark.parametrize('dtype', [np.float32, np.float16])
+@pytest.mark.parametrize('pooled', [(16, 2), (17, 2), (35, 3), (28, 9)])
+def test_wavefronts_that_walk_more_pooled_rows_than_are_planned_at_a_time(pooled, dtype, layout):
+    """So many boxes that the rows of one are not dealt out: its wavefront plans them sixteen at a time."""
+    abi.set_impl('auto')
+    rng = np.random.default_rng(pooled[0])
+    N, C, H, W, R = 1, 264, 31, 24, 520
+    at = np.stack([rng.uniform(-2, W, R), rng.uniform(-2, H, R)], 1)
+    rois = np.concatenate([np.zeros((R, 1)), at, at + rng.uniform(0, 1, (R, 2)) * (W, H)], 1).astype(np.float32)
+    x = rng.standard_normal((N, C, H, W)).astype(dtype)
+    want = oracle.forward(x.astype(np.float32), rois, pooled, 1.0, 2).astype(dtype).astype(np.float32)
+    if layout == 'nchw':
+        y = abi.forward(abi.to_dev(x), abi.to_dev(rois), pooled, 1.0, 2).float().cpu().numpy()
+    else:
+        y = abi.forward_nhwc(abi.to_dev(np.ascontiguousarray(x.transpose(0, 2, 3, 1))), abi.to_dev(rois), pooled, 1.0,
+                             2).float().cpu().numpy().transpose(0, 3, 1, 2)
+    assert_parity(y, want, FWD_TOL if dtype == np.float32 else FP16_TOL, 'y')
 
 
 @pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
