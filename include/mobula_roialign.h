@@ -321,7 +321,7 @@ void mobula_hip_clear_error(void);
  * results, those of other images too.  0 never, 2 three parts wherever a product
  * fits, 3 two fp16 parts wherever one fits;
  * "roialign_tile_columns": 0 (default) lets the backward pass choose its tile
- * width from the size of the map, 56 or 28 fixes it; "roialign_row_split": 0
+ * width from the size of the map, a multiple of 4 from 16 to 64 fixes it; "roialign_row_split": 0
  * (default) lets it choose how many wavefronts share a tile row's work list,
  * 1 or 4 fixes it; "roialign_row_quads": 1 (default) lets it write rows of maps
  * whose width is a multiple of four 16 bytes at a time, 0 element by element;

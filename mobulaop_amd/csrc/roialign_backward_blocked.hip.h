@@ -25,6 +25,7 @@
 // load per lane fetches (eight pooled columns of) a pooled row, up to 1 KB; the
 // slab of a channel block is addressed with 32-bit offsets (up to 2 GiB each).
 #pragma once
+#include <algorithm>
 #include <type_traits>
 
 #include "roialign_taps.hip.h"
@@ -34,8 +35,8 @@ namespace roialign {
 struct BwdBlocked {
   static constexpr int TH = 1;           // rows of a band = wavefronts of a workgroup
   static constexpr int BANDS = kTileRows / TH;   // bands per tile
-  static constexpr int TW = 56;          // tile columns ...
-  static constexpr int TW_SMALL = 28;    // ... and for maps that give few tiles (see backward_tile_columns)
+  static constexpr int TW = 64;          // tile columns at most (see backward_tile_columns)
+  static constexpr int TW_LEAST = 16;    // (a window of merged weights and the dummies lie inside a row)
   static constexpr int CB = 32;          // channels per workgroup
   static constexpr int NW = TH;
   static constexpr int NT = NW * 64;
@@ -50,18 +51,32 @@ struct BwdBlocked {
 
 inline bool backward_blocked_supports(int PH, int PW, int S) { return lists_supported(PH, PW, S); }
 
-// Tile width for a map: narrow tiles double the number of (shorter) work lists,
-// which pays only while the wide ones would leave the SIMDs short of wavefronts
-// (measured: 2048 wavefronts 82 -> 65 us, 40000 wavefronts 222 -> 262 us).
-inline int backward_tile_columns(long long images, int H, int W, int cblk) {
-  const long long wide = images * ((H + kTileRows - 1) / kTileRows) * ((W + BwdBlocked::TW - 1) / BwdBlocked::TW);
-  return wide * kTileRows * cblk < 8192 ? BwdBlocked::TW_SMALL : BwdBlocked::TW;
+// Maps that give few tile rows of 56 columns: every row's work list is split, and tiles may be narrow.
+inline bool backward_few_tiles(long long images, int H, int W, int cblk) {
+  return images * ((H + kTileRows - 1) / kTileRows) * ((W + 55) / 56) * kTileRows * cblk < 8192;
 }
 
-// Wavefronts per tile row: the same maps also split every row's work list.
+// Tile width for a map: as few tiles as the widest allow, all about as wide (multiples of four columns: the four-column
+// write-out).  A box has an entry per row in every tile column that it reaches, and a last tile of a few columns costs its
+// rows' wavefronts like any other (tile owners, us: 4000 boxes on 4 x 256 x 200 x 320, 56 columns 208, 64: 184; 512 on
+// 2 x 256 x 64 x 64, 28: 42, 32: 38, 64: 34; 4000 on 4 x 256 x 100 x 100, 28: 237, 52: 169; 2000 on 8 x 64 x 40 x 120, 28: 42, 60: 31).
+// Narrower ones down to 32 columns where those give the device fewer wavefronts than it holds (300 boxes on 1 x 256 x 50 x
+// 84, 44: 24, 28: 23, 32: 21).  Windows of merged weights, whose rows are not split: 28 columns where tiles are few (301 boxes on
+// 3 x 81 x 75 x 113: 42; 32: 48; 64: 50), else up to 56 (1500 on 2 x 128 x 256 x 256: 52: 72, 56 and 64: 75).
+inline int backward_tile_columns(long long images, int H, int W, int cblk, bool windows) {
+  const bool few = backward_few_tiles(images, H, W, cblk);
+  if (windows && few) return 28;
+  const int most = windows ? 56 : BwdBlocked::TW;
+  auto width = [&](int tiles) { return std::max(BwdBlocked::TW_LEAST, ((W + tiles - 1) / tiles + 3) / 4 * 4); };
+  const long long rows = images * ((H + kTileRows - 1) / kTileRows) * kTileRows * cblk;
+  int tiles = (W + most - 1) / most;
+  while (few && rows * tiles * BwdBlocked::NSPLIT < 4096 && width(tiles) > 32) ++tiles;
+  return width(tiles);
+}
+
+// Wavefronts per tile row.
 inline int backward_row_split(long long images, int H, int W, int cblk) {
-  const long long wide = images * ((H + kTileRows - 1) / kTileRows) * ((W + BwdBlocked::TW - 1) / BwdBlocked::TW);
-  return wide * kTileRows * cblk < 8192 ? BwdBlocked::NSPLIT : 1;
+  return backward_few_tiles(images, H, W, cblk) ? BwdBlocked::NSPLIT : 1;
 }
 
 // dy[r][c][ph][pw] -> dyb[cb][r][ph][pw][32] (R: number of ROIs), zero where the channel does
@@ -190,7 +205,7 @@ __device__ __forceinline__ float lane_value(const unsigned __attribute__((ext_ve
 }
 
 // TO is the element type of dx (float, __half or bfloat16; sums are formed in fp32 and
-// rounded once).  TW: tile columns.  NSPLIT: wavefronts that share a tile row: each takes
+// rounded once).  NSPLIT: wavefronts that share a tile row: each takes
 // a contiguous part of the row's work list (whole items: an item belongs to the part its first
 // entry lies in) into a row of its own in LDS, and the parts are added in part order on the
 // way out -- for maps that give the SIMDs too few tile rows to keep them busy.
@@ -198,7 +213,9 @@ __device__ __forceinline__ float lane_value(const unsigned __attribute__((ext_ve
 // points per bin and axis) instead of pairs of sample columns.
 // dy_any: the blocked copy dyb, or for channels-last tensors the caller's dy[R][PH][PW][C] itself; of
 // dx's element type.
-template <bool NHWC, typename TO, int TW, int NSPLIT = 1, bool WIN = false>
+// Dynamic LDS: backward_blocked_lds(tg.tw, NSPLIT) bytes.
+inline size_t backward_blocked_lds(int tw, int nsplit) { return sizeof(float) * nsplit * (tw + 2) * BwdBlocked::CS; }
+template <bool NHWC, typename TO, int NSPLIT = 1, bool WIN = false>
 __global__ void __launch_bounds__(BwdBlocked::NT * NSPLIT)
 backward_blocked_kernel(const void* __restrict__ dy_any, TO* __restrict__ dx_any,
                         const WorkRange* __restrict__ ranges, const SortedRow* __restrict__ sorted,
@@ -207,10 +224,9 @@ backward_blocked_kernel(const void* __restrict__ dy_any, TO* __restrict__ dx_any
                         int W, int PH, int PW, int cblk, unsigned dyb_bytes, unsigned list_bytes,
                         int assign) {   // assign: bit 0 = overwrite dx (else add to it), bit 1 = rows may be written four columns at a time
   using K = BwdBlocked;
-  constexpr int RS = TW + 2;   // cells per row: one dummy on either side
+  const int TW = tg.tw, RS = TW + 2;   // cells per row: one dummy on either side
   static_assert(K::TH == 1, "the parts of a split row take the place of the rows of a band");
-  static_assert(TW % 4 == 0, "tiles start at multiples of four columns (the four-column write-out)");
-  __shared__ __attribute__((aligned(16))) float acc[NSPLIT * RS * K::CS];
+  extern __shared__ __attribute__((aligned(16))) float acc[];   // [NSPLIT][RS][CS]
 
   // Job decode.  Workgroups are dealt to the 8 XCDs round-robin, so blockIdx % 8
   // names the XCD: it takes the channel blocks b with b % 8 == xcd (their slice
@@ -616,8 +632,8 @@ backward_blocked_kernel(const void* __restrict__ dy_any, TO* __restrict__ dx_any
   // Any other row: one channel plane at a time, lanes along x.
   // LPC lanes per channel plane (a power of two that covers the tile's columns):
   // 64 / LPC planes are written per step
-  constexpr int LPC = TW <= 32 ? 32 : 64, PLANES = 64 / LPC;
-  const int col = lane & (LPC - 1), first = lane / LPC;
+  const int LPC = TW <= 32 ? 32 : 64, PLANES = 64 / LPC;
+  const int col = lane & (LPC - 1), first = TW <= 32 ? lane >> 5 : 0;
   if (col < cols) {
     const float* const src = acc + (col + 1) * K::CS;
     auto total = [&](int c) {

@@ -492,12 +492,12 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
 bool use_tiled() { return mobula_hip::option("roialign_impl", kAuto) != kNaive; }
 
 // Tile columns of the backward pass: chosen from the size of the map unless the
-// option "roialign_tile_columns" names one of the two widths (tests do).
+// option "roialign_tile_columns" names a width (tests do).
 int tile_columns(const Problem& p) {
   using BB = roialign::BwdBlocked;
   const long long forced = mobula_hip::option("roialign_tile_columns", 0);
-  if (forced == BB::TW || forced == BB::TW_SMALL) return static_cast<int>(forced);
-  return roialign::backward_tile_columns(p.N, p.H, p.W, (p.C + BB::CB - 1) / BB::CB);
+  if (forced >= BB::TW_LEAST && forced <= BB::TW && forced % 4 == 0) return static_cast<int>(forced);
+  return roialign::backward_tile_columns(p.N, p.H, p.W, (p.C + BB::CB - 1) / BB::CB, roialign::lists_in_windows(p.S));
 }
 
 // Wavefronts per tile row of the backward pass (1, or BwdBlocked::NSPLIT for maps with few tile
@@ -509,23 +509,18 @@ int row_split(const Problem& p) {
   return roialign::backward_row_split(p.N, p.H, p.W, (p.C + BB::CB - 1) / BB::CB);
 }
 
-// The tile owner for a problem: tile columns tw, nsplit wavefronts per tile row, sample lists or
+// The tile owner for a problem: nsplit wavefronts per tile row, sample lists or
 // windows of merged weights (which are not split: 47 us against 71 in four parts, 301 boxes on
 // 3 x 81 x 75 x 113).
 template <bool NHWC, typename T>
-auto owner_kernel(int tw, int* nsplit, bool windows) {
+auto owner_kernel(int* nsplit, bool windows) {
   using BB = roialign::BwdBlocked;
-  const bool wide = tw == BB::TW;
   if (windows) {
     *nsplit = 1;
-    return wide ? roialign::backward_blocked_kernel<NHWC, T, BB::TW, 1, true>
-                : roialign::backward_blocked_kernel<NHWC, T, BB::TW_SMALL, 1, true>;
+    return roialign::backward_blocked_kernel<NHWC, T, 1, true>;
   }
-  if (*nsplit > 1)
-    return wide ? roialign::backward_blocked_kernel<NHWC, T, BB::TW, BB::NSPLIT, false>
-                : roialign::backward_blocked_kernel<NHWC, T, BB::TW_SMALL, BB::NSPLIT, false>;
-  return wide ? roialign::backward_blocked_kernel<NHWC, T, BB::TW, 1, false>
-              : roialign::backward_blocked_kernel<NHWC, T, BB::TW_SMALL, 1, false>;
+  return *nsplit > 1 ? roialign::backward_blocked_kernel<NHWC, T, BB::NSPLIT, false>
+                     : roialign::backward_blocked_kernel<NHWC, T, 1, false>;
 }
 
 // Any sampling grid the lists take: fixed ones up to kSearchedGrid points, adaptive ones
@@ -573,8 +568,9 @@ void backward_device(const Problem& p, const T* dy, const float* rois, T* dx, bo
     const unsigned dy_bytes = static_cast<unsigned>(sizeof(T) * p.n_out);
     mobula_hip::KernelTimer timer("backward_blocked_kernel", stream);
     int nsplit = row_split(p);
-    const auto kernel = owner_kernel<true, T>(tw, &nsplit, plan.layout.windows != 0);
-    kernel<<<static_cast<unsigned>(roialign::backward_blocked_grid(plan.grid.total, cblk)), BB::NT * nsplit, 0, stream>>>(
+    const auto kernel = owner_kernel<true, T>(&nsplit, plan.layout.windows != 0);
+    kernel<<<static_cast<unsigned>(roialign::backward_blocked_grid(plan.grid.total, cblk)), BB::NT * nsplit,
+             roialign::backward_blocked_lds(tw, nsplit), stream>>>(
         dy, dx, plan.ranges, plan.sorted, plan.class_counts(), plan.entries, plan.lists,
         plan.grid, plan.layout, p.C, p.H, p.W, p.PH, p.PW, cblk, dy_bytes,
         static_cast<unsigned>(plan.list_bytes), assign ? 1 : 0);
@@ -624,8 +620,8 @@ void backward_device(const Problem& p, const T* dy, const float* rois, T* dx, bo
         // every row piece of dx starts at a multiple of four elements (tile widths are): four columns per store
         const bool quads = p.W % 4 == 0 && reinterpret_cast<size_t>(dx) % (4 * sizeof(T)) == 0 &&
                            mobula_hip::option("roialign_row_quads", 1) != 0;
-        const auto kernel = owner_kernel<false, T>(tw, &nsplit, plan.layout.windows != 0);
-        kernel<<<static_cast<unsigned>(grid), BB::NT * nsplit, 0, stream>>>(
+        const auto kernel = owner_kernel<false, T>(&nsplit, plan.layout.windows != 0);
+        kernel<<<static_cast<unsigned>(grid), BB::NT * nsplit, roialign::backward_blocked_lds(tw, nsplit), stream>>>(
             plan.dyb, dx, plan.ranges, plan.sorted, plan.class_counts(), plan.entries, plan.lists, plan.grid, plan.layout, p.C, p.H,
             p.W, p.PH, p.PW, cblk, static_cast<unsigned>(plan.dyb_bytes),
             static_cast<unsigned>(plan.list_bytes), (assign ? 1 : 0) | (quads ? 2 : 0));
