@@ -743,10 +743,11 @@ igemm_weight_kernel(BackwardWeightOps ops, int k_per_slice, int k_total, int row
 
 // db[d] = sum of dy[img, d, pixel] over images and pixels, in two steps that ride in launches of other work where there is
 // some (on their own they took 6 and 4 us of a first layer's 93, most of it launch): a wavefront per kPixels pixels of a
-// plane, their sums in the order of dy; then a wavefront per filter, which adds those up in 64 bits.
+// plane, their sums in the order of dy; then a wavefront per filter.  All in 64 bits: of a sum whose terms nearly cancel 32 lose
+// (15 x 29 x 81 x 65: 1.0e-7 with 16 terms a thread in 32 bits and a tree, 1.5e-7 with 64, 3e-8 now).
 struct BiasJob {
   static constexpr int kPixels = 4096;
-  const float* dy; float* sums; float* db;
+  const float* dy; double* sums; float* db;
   int N, D, ohw, runs, wide, accumulate;   // runs: of a plane; wide: planes are 16-byte aligned and whole quads
   unsigned sum_blocks, total_blocks;       // workgroups of four wavefronts; 0: no such job
 };
@@ -758,12 +759,13 @@ __device__ __forceinline__ void bias_sums(const BiasJob& job, unsigned block) {
   const long long plane = unit / job.runs;
   const int first = static_cast<int>(unit - plane * job.runs) * BiasJob::kPixels, last = min(first + BiasJob::kPixels, job.ohw);
   const float* const p = job.dy + plane * job.ohw;
-  float s = 0.0f;
+  double s = 0.0;
   if (job.wide) {
-    f32x4 v = 0.0f;
 #pragma unroll 4
-    for (int i = first + 4 * lane; i < last; i += 256) v += *reinterpret_cast<const f32x4*>(p + i);
-    s = (v[0] + v[1]) + (v[2] + v[3]);
+    for (int i = first + 4 * lane; i < last; i += 256) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(p + i);
+      s += (static_cast<double>(v[0]) + v[1]) + (static_cast<double>(v[2]) + v[3]);
+    }
   } else {
 #pragma unroll 4
     for (int i = first + lane; i < last; i += 64) s += p[i];
@@ -780,7 +782,7 @@ __device__ __forceinline__ void bias_totals(const BiasJob& job, unsigned block) 
 #pragma unroll 4
   for (int i = lane; i < count; i += 64) {
     const int img = i / job.runs;
-    sum += static_cast<double>(job.sums[(static_cast<long long>(img) * job.D + d) * job.runs + i - img * job.runs]);
+    sum += job.sums[(static_cast<long long>(img) * job.D + d) * job.runs + i - img * job.runs];
   }
 #pragma unroll
   for (int k = 32; k > 0; k >>= 1) sum += __shfl_xor(sum, k);

@@ -317,12 +317,12 @@ conv::AgainJob again_job(const PrepB16& prep, const conv::ExponentWords& words, 
 // The bias's gradient that rides in launches of a call's other work (db == nullptr: none), its sums at `at`.
 size_t bias_bytes(const conv::Geometry& g, const float* db) {
   const long long runs = (static_cast<long long>(g.OH) * g.OW + conv::BiasJob::kPixels - 1) / conv::BiasJob::kPixels;
-  return db == nullptr ? 0 : align_to_256(sizeof(float) * static_cast<size_t>(g.N) * g.D * runs);
+  return db == nullptr ? 0 : align_to_256(sizeof(double) * static_cast<size_t>(g.N) * g.D * runs);
 }
 conv::BiasJob bias_job(int N, int D, int ohw, const float* dy, int accumulate, float* db, char* at) {
   if (db == nullptr) return conv::BiasJob{};
   const int runs = (ohw + conv::BiasJob::kPixels - 1) / conv::BiasJob::kPixels;
-  return conv::BiasJob{dy, reinterpret_cast<float*>(at), db, N, D, ohw, runs,
+  return conv::BiasJob{dy, reinterpret_cast<double*>(at), db, N, D, ohw, runs,
                        ohw % 4 == 0 && reinterpret_cast<uintptr_t>(dy) % 16 == 0, accumulate,
                        static_cast<unsigned>((static_cast<long long>(N) * D * runs + 3) / 4), static_cast<unsigned>((D + 3) / 4)};
 }
@@ -1381,7 +1381,7 @@ void bias_gradient(int batch, int filters, int pixels, const float* dy, int accu
   const conv::BiasJob sizes = bias_job(batch, filters, pixels, dy, accumulate, db, nullptr);
   const long long units = static_cast<long long>(batch) * filters * sizes.runs;
   char* ws = nullptr;
-  if (units > 0 && units < (1ll << 31)) ws = static_cast<char*>(mobula_hip::workspace_if_possible(sizeof(float) * units));
+  if (units > 0 && units < (1ll << 31)) ws = static_cast<char*>(mobula_hip::workspace_if_possible(sizeof(double) * units));
   if (failed()) return;
   if (ws == nullptr) {   // (a first call under capture: one workgroup to a filter needs no memory)
     (sizes.wide ? conv::bias_grad_kernel<4> : conv::bias_grad_kernel<1>)<<<filters, 256, 0, stream>>>(dy, db, batch, filters, pixels,
