@@ -1,7 +1,7 @@
 // Backward ROIAlign: tile owners accumulate in LDS, 16 bytes per lane.
 //
-// dx is cut into tiles of 16 rows x 56 columns x 32 channels (28 columns for maps
-// that would give the SIMDs too few wavefronts otherwise), and a tile into
+// dx is cut into tiles of 16 rows x up to 64 columns x 32 channels (as few as cover a row, about
+// equally wide; narrower where the SIMDs would have too few wavefronts), and a tile into
 // bands of TH rows (TH = 1: single rows).  One workgroup owns one band, keeps
 // it in LDS as acc[row][column][channel] and is the only writer of that piece
 // of dx: no atomics anywhere and a summation order fixed by the ROI order.

@@ -2,7 +2,7 @@
 //
 // With a few boxes on a small map the gradient is a chain of launches and not work: per-box lists, per-tile lists and
 // the tile owners each take some six microseconds on the device, most of them waiting, and as much of the host.
-// Here a workgroup owns 64 neighbouring pixels of one plane's worth of eight channels, a lane a pixel, and looks at
+// Here a workgroup owns 64 neighbouring pixels in eight channels, a lane a pixel, and looks at
 // every box itself: a lane per box tells which boxes reach the pixels, the four wavefronts take one each, and what a
 // bin gives a pixel is dy times the sum of the row weights times the sum of the column weights that its samples
 // have there (opzoo/ROIAlign/ROIAlign.cpp:67-127: the sum over the samples' corners).  No lists, no atomics; the

@@ -32,7 +32,7 @@ struct FwdBlocked {
 
 // Per element type: channels per lane (16 bytes), channels per block of the
 // blocked layout (8 lanes: 128 bytes per pixel), staged outputs per wavefront
-// (8704 bytes: with the sample tables 39.9 KB per workgroup of four, four workgroups
+// (8704 bytes: with the sample tables 38.9 KB per workgroup of four, four workgroups
 // to a CU, which the registers allow anyway; 14 x 14 pooled maps go in four passes).
 template <typename T>
 struct BlockOf {
