@@ -23,14 +23,16 @@ struct BwdFew {
   // through the operator, us, lists and tile owners / this; 7 x 7 pooled: 1 x 64 x 32 x 32, 4 to 32 boxes 48 / 42, 64:
   // 48 / 51; 1 x 256 x 50 x 84, 16 boxes 49 / 44, 32: 49 / 57; 2 x 256 x 64 x 64, 8 boxes 34 / 28, 16: 33 / 37; 1 x 256 x 100 x 168,
   // 4 boxes 35 / 35, 8: 39 / 45.  14 x 14: 1 x 256 x 32 x 32, 8 boxes 51 / 45, 16: 51 / 65.  28 x 28, 4 boxes: 53 / 73.
+  // Channels last 48 / 42.  Three points per bin and axis, whose lists are windows of merged weights that the host waits for: 61 / 43.
   static constexpr long long kMostBins = 1600, kMostLooks = 1670000, kMostSteps = 29400000;
 };
 inline long long backward_few_blocks(long long N, int C, long long H, long long W) {
   return (H * W + BwdFew::PIXELS - 1) / BwdFew::PIXELS * ((C + BwdFew::CH - 1) / BwdFew::CH) * N;
 }
 
-// grid (runs of 64 pixels, groups of eight channels, images); S is 1 or 2, PH * S and PW * S at most 64, R at most 64.
-template <typename T>
+// grid (runs of 64 pixels, groups of eight channels, images); S is 1 to 4, PH * S and PW * S at most 64, R at most 64.
+// NHWC: dy [R][PH][PW][C], dx [N][H][W][C].
+template <typename T, bool NHWC>
 __global__ void __launch_bounds__(BwdFew::NW * 64)
 backward_few_kernel(const T* __restrict__ dy, const float* __restrict__ rois, T* __restrict__ dx, float scale, int R, int C,
                     int H, int W, int PH, int PW, int S, int assign) {
@@ -64,16 +66,17 @@ backward_few_kernel(const T* __restrict__ dy, const float* __restrict__ rois, T*
 #pragma unroll
   for (int c = 0; c < CH; ++c) acc[c] = 0.0f;
   const unsigned samples = (1u << S) - 1u;   // of a bin along an axis
-  const float inv_count = 1.0f / static_cast<float>(S * S);   // (a power of two)
+  const float count = static_cast<float>(S * S);
+  const int bin_of = lane / S, sample_of = lane - bin_of * S;   // the sample this lane weighs
   const unsigned long long hits = __ballot(hit);
   int turn = 0;
   for (unsigned long long m = hits; m != 0ull; m &= m - 1ull, ++turn) {
     if (turn % K::NW != wave) continue;
     const int r = __builtin_ctzll(m);
     // a lane per sample of either axis; one that contributes nothing lies at no pixel
-    auto sample = [&](float start, float bin, int count, int size) {
-      AxisSample a = axis_sample(sample_coord(start, lane >> (S - 1), bin, lane & (S - 1), S), size);
-      if (lane >= count || !a.valid) a.low = a.high = -1;
+    auto sample = [&](float start, float bin, int samples_of_axis, int size) {
+      AxisSample a = axis_sample(sample_coord(start, bin_of, bin, sample_of, S), size);
+      if (lane >= samples_of_axis || !a.valid) a.low = a.high = -1;
       return a;
     };
     const AxisSample row = sample(lane_f(g.start_h, r), lane_f(g.bin_h, r), PH * S, H);
@@ -93,27 +96,29 @@ backward_few_kernel(const T* __restrict__ dy, const float* __restrict__ rois, T*
       return touched;
     };
     for (int pwb = 0; pwb < PW && rows != 0ull; pwb += PWB) {
-      const unsigned here = static_cast<unsigned>(cols >> (pwb * S)) & ((1u << (PWB * S)) - 1u);
-      if (here == 0u) continue;
+      const unsigned long long here = (cols >> (pwb * S)) & ((1ull << (PWB * S)) - 1ull);
+      if (here == 0ull) continue;
       float wx[PWB];
       bool on_x[PWB];
 #pragma unroll
       for (int k = 0; k < PWB; ++k) {
         wx[k] = 0.0f; on_x[k] = false;
-        if ((here >> (k * S)) & samples) on_x[k] = weight(col, pwb + k, w, &wx[k]);
+        if (((here >> (k * S)) & samples) != 0ull) on_x[k] = weight(col, pwb + k, w, &wx[k]);
       }
       for (unsigned long long left = rows; left != 0ull;) {
-        const int ph = __builtin_ctzll(left) >> (S - 1);
+        const int ph = __builtin_ctzll(left) / S;
         left &= ~(static_cast<unsigned long long>(samples) << (ph * S));
         // eight channels x eight pooled columns of dy, a lane each
         const int c = c0 + (lane >> 3), pw = pwb + (lane & 7);
         float v = 0.0f;
-        if (c < C && pw < PW) v = to_float(dy[((static_cast<size_t>(r) * C + c) * PH + ph) * PW + pw]) * inv_count;
+        if (c < C && pw < PW)
+          v = to_float(dy[NHWC ? ((static_cast<size_t>(r) * PH + ph) * PW + pw) * C + c
+                               : ((static_cast<size_t>(r) * C + c) * PH + ph) * PW + pw]) / count;
         float wy;
         const bool on_y = weight(row, ph, h, &wy);
 #pragma unroll
         for (int k = 0; k < PWB; ++k) {
-          if (((here >> (k * S)) & samples) == 0u) continue;
+          if (((here >> (k * S)) & samples) == 0ull) continue;
           const float both = wy * wx[k];
           const bool touched = on_y && on_x[k];   // (elsewhere dy, finite or not, adds nothing)
 #pragma unroll
@@ -133,11 +138,16 @@ backward_few_kernel(const T* __restrict__ dy, const float* __restrict__ rois, T*
   } else if (!assign) {
     return;
   }
-  if (p >= plane) return;
-  for (int c = wave; c < CH && c0 + c < C; c += K::NW) {
-    const float sum = hits == 0ull ? 0.0f : ((part[0][c][lane] + part[1][c][lane]) + part[2][c][lane]) + part[3][c][lane];
-    T* const to = dx + (static_cast<size_t>(n) * C + c0 + c) * plane + p;
+  auto finish = [&](int c, int px, T* to) {
+    const float sum = hits == 0ull ? 0.0f : ((part[0][c][px] + part[1][c][px]) + part[2][c][px]) + part[3][c][px];
     *to = from_float<T>(assign ? sum : to_float(*to) + sum);
+  };
+  if (NHWC) {   // a pixel's channels are neighbours
+    const int c = threadIdx.x % CH;
+    for (int px = threadIdx.x / CH; px < K::PIXELS && first + px < plane && c0 + c < C; px += 64 * K::NW / CH)
+      finish(c, px, dx + (static_cast<size_t>(n) * plane + first + px) * C + c0 + c);
+  } else if (p < plane) {
+    for (int c = wave; c < CH && c0 + c < C; c += K::NW) finish(c, lane, dx + (static_cast<size_t>(n) * C + c0 + c) * plane + p);
   }
 }
 

@@ -535,7 +535,7 @@ bool nhwc_backward_supported(const Problem& p) {
 // Whether backward_few_kernel takes a call: option "roialign_few_boxes" 1 (default) where it is faster, 0 never, 2 wherever it can.
 bool takes_few_boxes(const Problem& p) {
   using BF = roialign::BwdFew;
-  if (p.R < 1 || p.R > BF::kMostBoxes || (p.S != 1 && p.S != 2) || p.PH * p.S > BF::kMostSamples ||
+  if (p.R < 1 || p.R > BF::kMostBoxes || p.S < 1 || p.S > 4 || p.PH * p.S > BF::kMostSamples ||
       p.PW * p.S > BF::kMostSamples)
     return false;
   const long long blocks = roialign::backward_few_blocks(p.N, p.C, p.H, p.W), bins = p.R * p.PH * p.PW;
@@ -543,6 +543,17 @@ bool takes_few_boxes(const Problem& p) {
   const long long option = mobula_hip::option("roialign_few_boxes", 1);
   if (option == 0 || mobula_hip::option("roialign_impl", kAuto) != kAuto) return false;
   return option == 2 || (bins <= BF::kMostBins && bins * blocks <= BF::kMostLooks && bins * p.R * blocks <= BF::kMostSteps);
+}
+
+template <bool NHWC, typename T>
+void launch_few_boxes(const Problem& p, const T* dy, const float* rois, T* dx, bool assign, hipStream_t stream) {
+  using BF = roialign::BwdFew;
+  const dim3 grid(static_cast<unsigned>((static_cast<long long>(p.H) * p.W + BF::PIXELS - 1) / BF::PIXELS),
+                  static_cast<unsigned>((p.C + BF::CH - 1) / BF::CH), static_cast<unsigned>(p.N));
+  mobula_hip::KernelTimer timer("backward_few_kernel", stream);
+  roialign::backward_few_kernel<T, NHWC><<<grid, BF::NW * 64, 0, stream>>>(
+      dy, rois, dx, p.scale, static_cast<int>(p.R), p.C, p.H, p.W, p.PH, p.PW, p.S, assign ? 1 : 0);
+  MOBULA_HIP_TRY(hipGetLastError());
 }
 
 template <typename T>
@@ -556,8 +567,13 @@ void backward_device(const Problem& p, const T* dy, const float* rois, T* dx, bo
     // dy and dx are used where they lie: only the pre-pass before the tile owners
     const int cblk = (p.C + BB::CB - 1) / BB::CB;
     const int tw = tile_columns(p);
-    if (!nhwc_backward_supported(p) || reinterpret_cast<size_t>(dy) % 16 != 0 ||
-        reinterpret_cast<size_t>(dx) % 16 != 0 ||
+    const bool taken = nhwc_backward_supported(p) && reinterpret_cast<size_t>(dy) % 16 == 0 &&
+                       reinterpret_cast<size_t>(dx) % 16 == 0;
+    if (taken && takes_few_boxes(p)) {
+      launch_few_boxes<true>(p, dy, rois, dx, assign, stream);
+      return;
+    }
+    if (!taken ||
         !plan_tiles<T>(p, rois, roialign::kTileRows, tw, /*with_dyb=*/false, stream, &plan) ||
         roialign::backward_blocked_grid(plan.grid.total, cblk) >= (1ll << 31)) {
       if (!failed())
@@ -579,12 +595,7 @@ void backward_device(const Problem& p, const T* dy, const float* rois, T* dx, bo
   }
   // a handful of boxes on a small map: one launch, no lists
   if (takes_few_boxes(p)) {
-    const dim3 grid(static_cast<unsigned>((static_cast<long long>(p.H) * p.W + roialign::BwdFew::PIXELS - 1) / roialign::BwdFew::PIXELS),
-                    static_cast<unsigned>((p.C + roialign::BwdFew::CH - 1) / roialign::BwdFew::CH), static_cast<unsigned>(p.N));
-    mobula_hip::KernelTimer timer("backward_few_kernel", stream);
-    roialign::backward_few_kernel<T><<<grid, roialign::BwdFew::NW * 64, 0, stream>>>(
-        dy, rois, dx, p.scale, static_cast<int>(p.R), p.C, p.H, p.W, p.PH, p.PW, p.S, assign ? 1 : 0);
-    MOBULA_HIP_TRY(hipGetLastError());
+    launch_few_boxes<false>(p, dy, rois, dx, assign, stream);
     return;
   }
   // the pre-pass (small, latency-bound kernels) runs beside the dy transposition, when that is

@@ -835,14 +835,25 @@ def test_non_finite_gradient_of_one_roi_stays_in_its_cells(impl):
         assert not np.isfinite(got[..., :12]).all()
 
 
+@pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
 @pytest.mark.parametrize('dtype', [np.float32, np.float16])
-@pytest.mark.parametrize('pooled,S', [((7, 7), 2), ((1, 1), 1), ((32, 3), 2), ((5, 32), 2), ((9, 17), 1)])
+@pytest.mark.parametrize('pooled,S', [((7, 7), 2), ((1, 1), 1), ((32, 3), 2), ((5, 32), 2), ((9, 17), 1), ((21, 7), 3), ((3, 16), 4)])
 @pytest.mark.parametrize('R,C,H,W', [(1, 3, 5, 7), (4, 8, 16, 16), (16, 13, 9, 71), (64, 9, 33, 31)])
-def test_backward_of_a_few_boxes_in_one_launch(R, C, H, W, pooled, S, dtype):
+def test_backward_of_a_few_boxes_in_one_launch(R, C, H, W, pooled, S, dtype, layout):
     """Up to 64 boxes (by itself up to 16), channels and pixels that fill no workgroup, axes of up to 64 samples; boxes
     across the borders, without extent, of no image, not finite, many on the same pixels; a gradient that is not finite
     reaches the pixels of its bins and no others."""
     native.set_option('roialign_few_boxes', 2)
+    if layout == 'nhwc':
+        C = (C + 3) // 4 * 4   # (what the channels-last entry points take)
+
+    def backward(dy, rois, shape, dx=None):
+        if layout == 'nchw':
+            return abi.backward(abi.to_dev(dy), abi.to_dev(rois), shape, scale, S, assign=dx is None,
+                                dx=None if dx is None else abi.to_dev(dx)).float().cpu().numpy()
+        last = lambda a: abi.to_dev(np.ascontiguousarray(a.transpose(0, 2, 3, 1)))   # noqa: E731
+        return abi.backward_nhwc(last(dy), abi.to_dev(rois), (shape[0], shape[2], shape[3], shape[1]), scale, S,
+                                 assign=dx is None, dx=None if dx is None else last(dx)).float().cpu().numpy().transpose(0, 3, 1, 2)
     try:
         rng = np.random.default_rng(R + C + pooled[0])
         N, scale = 3, 0.5
@@ -857,21 +868,21 @@ def test_backward_of_a_few_boxes_in_one_launch(R, C, H, W, pooled, S, dtype):
         tol = BWD_TOL if dtype == np.float32 else FP16_TOL
         with_image = (rois[:, 0] >= 0) & (rois[:, 0] < N)
         want = oracle.backward(dy[with_image].astype(np.float32), rois[with_image], shape, scale, S, impl='ordered')
-        got = abi.backward(abi.to_dev(dy), abi.to_dev(rois), shape, scale, S, assign=True).float().cpu().numpy()
+        got = backward(dy, rois, shape)
         assert_parity(got, want.astype(dtype).astype(np.float32), tol, 'assign')
         base = rng.standard_normal(shape).astype(dtype)
-        got = abi.backward(abi.to_dev(dy), abi.to_dev(rois), shape, scale, S, dx=abi.to_dev(base)).float().cpu().numpy()
+        got = backward(dy, rois, shape, base)
         assert_parity(got, (want + base.astype(np.float32)).astype(dtype).astype(np.float32), tol, 'accumulate')
         infinite = dy.copy()
         infinite[0] = np.inf
-        got = abi.backward(abi.to_dev(infinite), abi.to_dev(rois), shape, scale, S, assign=True).float().cpu().numpy()
+        got = backward(infinite, rois, shape)
         # (dy of one everywhere: which pixels the bins of the first box reach, weights of zero included)
         touched = oracle.backward(np.full((1, C) + pooled, np.inf, np.float32), rois[:1], shape, scale, S, impl='ordered')
         reached = ~np.isfinite(touched) if with_image[0] else np.zeros(shape, bool)
         assert (np.isfinite(got) == ~reached).all()
         assert_parity(got[~reached], want.astype(dtype).astype(np.float32)[~reached], tol, 'pixels that it does not reach')
         rois[0, 1:] = np.nan   # (a box that is not a number ends; other images are as they were)
-        got = abi.backward(abi.to_dev(dy), abi.to_dev(rois), shape, scale, S, assign=True).float().cpu().numpy()
+        got = backward(dy, rois, shape)
         others = [n for n in range(N) if n != int(rois[0, 0])]
         assert_parity(got[others], want.astype(dtype).astype(np.float32)[others], tol, 'other images')
     finally:
