@@ -303,8 +303,8 @@ void mobula_hip_clear_error(void);
  * "host_staging_device"; "kernel_timing": 0 off, 1 on; "side_stream": 1 (default)
  * lets helper kernels of a call run on a second stream of the device, 0 keeps
  * everything on the caller's stream; "conv_compute": 0 (default) multiplies the
- * convolution's operands with all of their 24 bits (see "conv_fp32_split"), 1
- * rounds them to bf16 and accumulates in fp32 (results about 2e-3 off), 2
+ * convolution's operands as fp32 values (with all of their 24 bits, or 23 and a
+ * sign: see "conv_fp32_split"), 1 rounds them to bf16 and accumulates in fp32 (results about 2e-3 off), 2
  * splits every operand into two bf16 and forms three bf16 products per
  * multiply-add (results about 5e-6 off; an infinity gives NaN);
  * "conv_fp32_split": 1 (default) lets fp32 products of large layers whose sums
@@ -313,13 +313,15 @@ void mobula_hip_clear_error(void);
  * three bf16 parts, six products of parts for one of fp32 (a result that a
  * single product makes up is off by a unit of the last place at most instead of
  * half of one), or, for sums of 512 terms and more, two fp16 parts and three
- * products (four units at most; tensors whose values lie too far apart for
- * that, below 2^-23 of the largest and with no larger one beside them, take
- * three parts).  Tensors with infinities, NaN, subnormals, or whose products or
- * sums could come near the ends of the range, take the fp32 kernels as a whole:
- * one such element changes the time of its call and the last bits of all of its
- * results, those of other images too.  0 never, 2 three parts wherever a product
- * fits, 3 two fp16 parts wherever one fits;
+ * products (four and a half units of the magnitudes that are added at most;
+ * values that fp16 does not span beside the tensor's largest, below some 2^-26 of
+ * it, are added from fp32 in 64 bits, up to 128 of a tensor; one with more takes
+ * three parts).  Tensors with infinities or NaN take the fp32 kernels as a
+ * whole; so do, where three parts are formed, those with subnormals or whose
+ * products or sums could come near the ends of the range.  One such element
+ * changes the time of its call and the last bits of all of its results, those
+ * of other images too.  0 never, 2 three parts wherever a product fits, 3 two
+ * fp16 parts wherever one fits;
  * "roialign_tile_columns": 0 (default) lets the backward pass choose its tile
  * width from the size of the map, a multiple of 4 from 16 to 64 fixes it; "roialign_row_split": 0
  * (default) lets it choose how many wavefronts share a tile row's work list,

@@ -78,8 +78,8 @@ struct GatherStep {
 struct SplitRange {
   const unsigned* a; const unsigned* b;   // exponent words of the operands; null: no choice to make
   int most;                               // what eight times the highest bits of both may come to (most_exponents)
-  // two fp16 parts are tried first: the operands' words of what keeps them from that, and which of its bits matter
-  const unsigned* halves_a; const unsigned* halves_b; unsigned halves_mask;
+  // two fp16 parts are tried first: the operands' words of what keeps them from that
+  const unsigned* halves_a; const unsigned* halves_b;
   // An operand whose highest bit is h lies below 2^(8 h + 8 - 127), parts and all; `terms` products of two, in six
   // products of parts that exceed them by a hundredth, stay below 2^128 while
   // 8 (ha + hb) + 16 - 254 + log2(terms) <= 127.
@@ -94,7 +94,7 @@ struct SplitRange {
     const int high_a = ea == 0u ? 0 : 31 - __builtin_clz(ea), high_b = eb == 0u ? 0 : 31 - __builtin_clz(eb);
     return (both & 0x80000007u) == 0u && 8 * (low_a + low_b) >= 2 * 127 - 100 && 8 * (high_a + high_b) <= most;
   }
-  __device__ bool halves_hold() const { return halves_a != nullptr && ((*halves_a | *halves_b) & halves_mask) == 0u; }
+  __device__ bool halves_hold() const { return halves_a != nullptr && (*halves_a | *halves_b) == 0u; }
   __device__ bool leaves_split() const { return halves_hold() || (a != nullptr && !inside()); }
   __device__ bool leaves_fp32() const { return halves_hold() || (a != nullptr && inside()); }
 };

@@ -21,7 +21,9 @@
 // Halves: an fp32 value, scaled by a power of two that its tensor has in common, as an fp16 head (11 bits) and 2^11 times
 // what that leaves as an fp16 tail: 23 bits and the sign of the tail, so a quarter of the values lose their last
 // bit.  Three products of parts for one of fp32 where three bf16 parts take six: the tails' with the heads go into sums of
-// their own, 2^11 times as large; what the two tails' product adds, 2^-22 of a product at most, is left out.
+// their own, 2^11 times as large; what the two tails' product adds, 2^-22 of a product at most, is left out.  So a result is
+// off by four and a half units of the magnitudes in it at most, whatever they are: values that fp16 does not span beside the tensor's
+// largest are kept apart (odd_values_kernel).
 // Sums of the heads' products start anew every sixteen K steps and are added up in fp32, so that a long sum is rounded at its
 // own size only once for 256 terms: 32 x 256 x 56 x 56, 256 filters 3 x 3: errors against 64 bits 2.85e-7 -> 1.43e-7 (weight
 // gradient 5.3 -> 1.7), products 500 -> 340 us each, forward and both gradients 1819 -> 1157.  The device's power bounds them
@@ -111,35 +113,62 @@ __global__ void __launch_bounds__(64) clear_words_kernel(unsigned* words, int co
   if (static_cast<int>(threadIdx.x) < count) words[threadIdx.x] = 0u;
 }
 
-// Scaled values of an operand in two fp16 parts lie below 2^16.  Both parts hold all 24 bits but for the last one of a
-// quarter of the values from 2^-12 on; a smaller value is off by up to 2^-36.
+// Scaled values from 2^-12 to the largest that fp16 holds have all of their 24 bits in two fp16 parts but for the last one of a
+// quarter of them.  Smaller ones would be off by up to 2^-36, whatever their size, and may be all that a result is made
+// of: the parts of a value outside are zero instead, and the value goes into the tensor's list (see odd_values_kernel).
 constexpr float kLeastHalf = 0x1p-12f, kMostHalf = 65504.0f;
-constexpr unsigned kBeyondHalves = 1u, kLonePixel = 2u, kLoneChannel = 4u, kSmallForHalves = 8u, kLargeHalf = 16u;
-__device__ __forceinline__ unsigned half_range(float scaled) {
-  const float v = fabsf(scaled);
-  return (v <= kMostHalf ? 0u : kBeyondHalves) | (v < kLeastHalf && v != 0.0f ? kSmallForHalves : 0u);
+constexpr int kMostOdd = 128;   // entries of a list; of 26 million normal values one to three are too small
+struct OddValue { int plane, at; float value; };   // (element plane * (elements of a plane) + at)
+__device__ __forceinline__ bool is_odd_half(float v, int shift) {
+  const float scaled = fabsf(ldexpf(v, shift));   // (may be zero for a v that is not)
+  return !(scaled >= kLeastHalf && scaled <= kMostHalf) && v != 0.0f;
 }
 
-// What is known of a tensor: its word of exponents (three parts) or of what keeps it from two halves, and behind that the
-// binary exponent its values are scaled by; the largest magnitudes of its pieces.
+// What is known of a tensor: whether anything keeps it from two halves (word[0] != 0: infinities or NaN, more odd values than
+// the list holds), the binary exponent its values are scaled by (word[1]), its word of exponents (three parts), how
+// many odd values it has, and which; the largest magnitudes of its pieces.
 constexpr int kMagnitudes = 256;
 struct TensorWords {
-  unsigned* word; unsigned* exponents; const unsigned* magnitudes;
-  int headroom;   // binary places between the largest value that was looked at and the largest there may be
-  // the power of two that brings the largest value below 2^15 (every wavefront of a conversion finds it)
+  unsigned* word; unsigned* exponents; unsigned* odd_count; const unsigned* magnitudes; OddValue* odd;
+  // the power of two that brings the largest value that was looked at below 2^15 (every wavefront of a conversion finds it)
   __device__ int shift(bool keep) const {
     const u32x4 m = reinterpret_cast<const u32x4*>(magnitudes)[threadIdx.x & 63];
     unsigned most = max(max(m[0], m[1]), max(m[2], m[3]));
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) most = max(most, static_cast<unsigned>(__shfl_xor(most, d)));
     const int exponent = static_cast<int>(most >> 23);   // (0: zeros and subnormals)
-    const int by = __builtin_amdgcn_readfirstlane(most == 0u ? 0 : 14 - headroom + 127 - max(exponent, 1));
+    const int by = __builtin_amdgcn_readfirstlane(most == 0u ? 0 : 14 + 127 - max(exponent, 1));
     if (keep && threadIdx.x == 0) word[1] = static_cast<unsigned>(by);
     return by;
   }
+  __device__ bool no_halves() const { return __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u; }
+  __device__ void set_no_halves() const { __hip_atomic_store(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+  // Room in the list for `mine` values of every lane of a wavefront (called by all of them); the first of this lane's,
+  // or -1 where the list is too short for the tensor.  (Wavefronts that alone have too many, or come when there are too many,
+  // leave the count alone: thousands of them take turns at one address.)
+  __device__ int reserve(int mine) const {
+    const int lane = threadIdx.x & 63;
+    int before = mine;   // (inclusive sums)
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int other = __shfl_up(before, d);
+      if (lane >= d) before += other;
+    }
+    const int all = __shfl(before, 63);
+    unsigned first = kMostOdd;
+    if (lane == 0 && !no_halves()) {
+      if (all <= kMostOdd) first = atomicAdd(odd_count, static_cast<unsigned>(all));
+      if (first + all > kMostOdd) set_no_halves();
+    }
+    first = __shfl(first, 0);
+    return first + all <= kMostOdd ? static_cast<int>(first) + before - mine : -1;
+  }
 };
 
-// The magnitudes of up to three tensors (blockIdx.y), and their words cleared.
+// The magnitudes of up to three tensors (blockIdx.y), and their words cleared.  Of large tensors one of every eight lines of
+// 128 bytes is looked at (103 MB: 28 us for all of them): values beyond the range that this gives are odd ones like those
+// below it.
+constexpr long long kSampledElements = 1 << 20;
 struct MagnitudeJob { const float* src[3]; long long count[3]; TensorWords words[3]; };
 __global__ void __launch_bounds__(1024) magnitudes_kernel(MagnitudeJob job) {
   typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -147,14 +176,14 @@ __global__ void __launch_bounds__(1024) magnitudes_kernel(MagnitudeJob job) {
   const int t = blockIdx.y, tid = threadIdx.x;
   const float* const src = job.src[t];
   const long long count = job.count[t];
+  const bool sampled = count > kSampledElements;
   unsigned most = 0u;
-  // (a workgroup takes sixteen KB at a time: all of them, or one of every eight)
-  const int every = job.words[t].headroom == 0 ? 1 : 8;
   const long long quads = reinterpret_cast<uintptr_t>(src) % 16 == 0 ? count / 4 : 0;
-  for (long long piece = blockIdx.x;; piece += kMagnitudes) {
-    const long long i = (piece * every + piece % every) * 1024 + tid;
-    if (i >= quads) break;
-    const f32x4 v = reinterpret_cast<const f32x4*>(src)[i];
+  const long long looks = sampled ? (quads + 63) / 64 * 8 : quads;
+  for (long long i = static_cast<long long>(blockIdx.x) * 1024 + tid; i < looks; i += kMagnitudes * 1024) {
+    const long long group = i >> 3, at = sampled ? group * 64 + ((group + (group >> 3)) & 7) * 8 + (i & 7) : i;
+    if (at >= quads) continue;
+    const f32x4 v = reinterpret_cast<const f32x4*>(src)[at];
 #pragma unroll
     for (int j = 0; j < 4; ++j) most = max(most, __float_as_uint(v[j]) & 0x7fffffffu);
   }
@@ -167,7 +196,7 @@ __global__ void __launch_bounds__(1024) magnitudes_kernel(MagnitudeJob job) {
   if (tid == 0) {
     for (int w = 1; w < 16; ++w) most = max(most, waves[w]);
     const_cast<unsigned*>(job.words[t].magnitudes)[blockIdx.x] = most;
-    if (blockIdx.x == 0) { *job.words[t].word = 0u; *job.words[t].exponents = 0u; }
+    if (blockIdx.x == 0) { *job.words[t].word = 0u; *job.words[t].exponents = 0u; *job.words[t].odd_count = 0u; }
   }
 }
 
@@ -191,11 +220,12 @@ __device__ __forceinline__ void to_blocked(const BlockedJob& job, unsigned block
   const int C = job.C, Cpad = job.Cpad, P = job.P;
   const float* const src = job.src;
   unsigned short* const dst = job.dst;
-  unsigned seen = 0u;
+  unsigned seen = 0u, odd = 0u;   // odd: bit 8 * k + j of what follows
   const unsigned row = block / job.tiles_p;
   const int n = row / job.tiles_c, c0 = (row - n * job.tiles_c) * 64, p0 = (block - row * job.tiles_p) * 64;
   const float* in = src + static_cast<size_t>(n) * C * P;
   const int shift = FORM == kHalves ? words.shift(block == 0) : 0;
+  const bool left = FORM == kHalves && words.no_halves();
   if (VEC) {
     const int q = threadIdx.x & 15, r = threadIdx.x >> 4;   // 16 quads of pixels, 16 channels per pass
 #pragma unroll
@@ -216,6 +246,8 @@ __device__ __forceinline__ void to_blocked(const BlockedJob& job, unsigned block
     }
   }
   __syncthreads();
+  // (a tensor that others have found to be none for halves is not written any more)
+  if (__any(left)) return;
   // a thread: one pixel, 8 channels (16 bytes); a channel block's threads cover a pixel of it
   constexpr int B = kBlockB16;
   const int cq = threadIdx.x & 1, pl = (threadIdx.x >> 1) & 63, first = threadIdx.x >> 7;
@@ -229,8 +261,9 @@ __device__ __forceinline__ void to_blocked(const BlockedJob& job, unsigned block
         f[j] = tile[cl + j][pl];
         if (FORM == 3) seen |= exponent_bit(f[j]);
         if (FORM == kHalves) {
-          f[j] = ldexpf(f[j], shift);
-          seen |= half_range(f[j]);
+          const bool is_odd = is_odd_half(f[j], shift);
+          odd |= is_odd ? 1u << (8 * k + j) : 0u;
+          f[j] = is_odd ? 0.0f : ldexpf(f[j], shift);
         }
       }
       unsigned short* const to = dst + ((static_cast<size_t>(n) * (Cpad / B) + c / B) * P + p) * B + 8 * cq;
@@ -244,24 +277,14 @@ __device__ __forceinline__ void to_blocked(const BlockedJob& job, unsigned block
     }
   }
   if (FORM == 3) add_exponents(words.exponents, seen);
-  if (FORM == kHalves && __any(seen != 0u)) {
-    // a value that is small for the tensor does no harm where a larger one stands beside it: at its pixel for a sum
-    // over channels, in its channel for a sum over pixels
-    unsigned bad = seen & kBeyondHalves;
-    if (seen & kSmallForHalves) {
-      for (int k = 0; k < 2; ++k)
-        for (int j = 0; j < 8; ++j) {
-          const int cl = B * (2 * k + first) + 8 * cq + j;
-          if ((half_range(ldexpf(tile[cl][pl], shift)) & kSmallForHalves) == 0u) continue;
-          bool pixel = false, channel = false;
-          for (int i = 0; i < 64 && !(pixel && channel); ++i) {
-            pixel |= fabsf(ldexpf(tile[i][pl], shift)) >= kLeastHalf;
-            channel |= fabsf(ldexpf(tile[cl][i], shift)) >= kLeastHalf;
-          }
-          bad |= (pixel ? 0u : kLonePixel) | (channel ? 0u : kLoneChannel);
-        }
+  if (FORM == kHalves && __any(odd != 0u)) {
+    int to = words.reserve(__popc(odd));
+    for (; odd != 0u; odd &= odd - 1u) {
+      const int q = __builtin_ctz(odd), cl = B * (2 * (q >> 3) + first) + 8 * cq + (q & 7);
+      const float v = tile[cl][pl];
+      if (!isfinite(v)) words.set_no_halves();
+      if (to >= 0) words.odd[to++] = OddValue{n * C + c0 + cl, p0 + pl, v};
     }
-    add_exponents(words.word, bad);
   }
 }
 
@@ -280,6 +303,8 @@ __device__ __forceinline__ void arrange_weights(const ArrangeJob& job, unsigned 
   const long long total = static_cast<long long>(job.Mpad) * job.taps * job.Cpad / 2;   // pairs of channels
   const long long i = static_cast<long long>(block) * 256 + threadIdx.x;
   unsigned seen = 0u;
+  float odd[2] = {0.0f, 0.0f};
+  long long at = 0;   // of the first of the pair in w
   const int shift = FORM == kHalves ? words.shift(block == 0) : 0;
   if (i < total) {
     const int j = 2 * static_cast<int>(i % (B / 2)), m = static_cast<int>((i / (B / 2)) % job.Mpad);
@@ -289,8 +314,11 @@ __device__ __forceinline__ void arrange_weights(const ArrangeJob& job, unsigned 
     float hi = (m < job.M && c + 1 < job.C) ? job.w[m * job.stride_m + (c + 1) * job.stride_c + tap] : 0.0f;
     if (FORM == 3) seen = exponent_bit(lo) | exponent_bit(hi);
     if (FORM == kHalves) {
-      lo = ldexpf(lo, shift); hi = ldexpf(hi, shift);
-      seen = half_range(lo) | half_range(hi) | (fmaxf(fabsf(lo), fabsf(hi)) >= kLeastHalf ? kLargeHalf : 0u);
+      odd[0] = is_odd_half(lo, shift) ? lo : 0.0f;
+      odd[1] = is_odd_half(hi, shift) ? hi : 0.0f;
+      lo = odd[0] != 0.0f ? 0.0f : ldexpf(lo, shift);
+      hi = odd[1] != 0.0f ? 0.0f : ldexpf(hi, shift);
+      at = m * job.stride_m + c * job.stride_c + tap;
     }
     unsigned* const to = reinterpret_cast<unsigned*>(job.out) +
                          (static_cast<size_t>(q) * PARTS * job.Mpad + m) * (B / 2) + j / 2;
@@ -298,12 +326,15 @@ __device__ __forceinline__ void arrange_weights(const ArrangeJob& job, unsigned 
     for (int part = 0; part < PARTS; ++part) to[static_cast<size_t>(part) * job.Mpad * (B / 2)] = split_pair<FORM>(lo, hi);
   }
   if (FORM == 3) add_exponents(words.exponents, seen);
-  if (FORM == kHalves && __any((seen & ~kLargeHalf) != 0u)) {
-    // (the eight lanes of a filter's sixteen channels at a tap look at each other)
-#pragma unroll
-    for (int d = 1; d < B / 2; d <<= 1) seen |= __shfl_xor(seen, d);
-    add_exponents(words.word, (seen & kBeyondHalves) |
-                                  ((seen & (kSmallForHalves | kLargeHalf)) == kSmallForHalves ? kLonePixel | kLoneChannel : 0u));
+  if (FORM == kHalves && __any(odd[0] != 0.0f || odd[1] != 0.0f)) {
+    int to = words.reserve((odd[0] != 0.0f) + (odd[1] != 0.0f));
+    for (int k = 0; k < 2; ++k)
+      if (to >= 0 && odd[k] != 0.0f) {
+        const long long element = at + k * job.stride_c;
+        const int plane = static_cast<int>(element / job.taps);
+        words.odd[to++] = OddValue{plane, static_cast<int>(element - static_cast<long long>(plane) * job.taps), odd[k]};
+      }
+    if (!isfinite(odd[0]) || !isfinite(odd[1])) words.set_no_halves();
   }
 }
 
@@ -975,6 +1006,201 @@ igemm_gradients_b16_kernel(WeightGradOpsB16<FORM> weight, TilesB16 weight_tiles,
   const int first = (weight_tiles.blocks + 7) / 8 * 8, block = blockIdx.x;
   if (block >= first) igemm_block_b16<BackwardDataOpsB16<FORM>, S>(data, data_tiles, block - first, lds);
   else if (block < weight_tiles.blocks) igemm_block_b16<WeightGradOpsB16<FORM>, S>(weight, weight_tiles, block, lds);
+}
+
+// What odd values add to a product of halves, in which they are zeros: of every pair of elements that holds one, the
+// product of both fp32 values in 64 bits, summed and added to the result once.  A product has two lists: a value of the
+// first (x, or dy for the data gradient) meets a few columns of the result, in every row; one of the second (the weights,
+// or dy for their gradient) meets every column of one row, where its pairs with odd values of the first are not
+// counted again.  A wavefront takes 64 rows of a column or 64 columns of a row, whose sum belongs to the first value that meets
+// it; the lists are sorted by place, so that results do not depend on who wrote them first.  A chain of a few round trips to
+// memory for the value or two of a tensor of tens of millions.
+enum Product { kForward, kData, kWeight };
+template <Product PRODUCT>
+struct OddJob {
+  Geometry g;
+  const float* first_partner; const float* second_partner;   // the tensors that values of the lists are multiplied with
+  float* out;
+  TensorWords first, second; SplitRange range;
+  unsigned blocks;   // workgroups: kOddGroups, or none
+};
+constexpr unsigned kOddGroups = 256;
+// An element as (a, b, h, w): of x image, channel, row, column; of dy image, filter, row, column; of the weights filter,
+// channel, tap's row and column.  A column of a result: of y and dx (image, -, row, column), of dw (channel, -, tap).
+struct OddSpot { int a, b, h, w; float value; };
+struct AxisOf { int stride, pad, dil; };
+__device__ __forceinline__ bool tap_of(const AxisOf& g, int in, int out, int size, int* tap) {
+  const int at = in + g.pad - out * g.stride;
+  *tap = at / g.dil;
+  return at >= 0 && at % g.dil == 0 && *tap < size;
+}
+__device__ __forceinline__ bool in_of(const AxisOf& g, int out, int tap, int size, int* in) {
+  *in = out * g.stride - g.pad + tap * g.dil;
+  return *in >= 0 && *in < size;
+}
+__device__ __forceinline__ bool out_of(const AxisOf& g, int in, int tap, int size, int* out) {
+  const int at = in + g.pad - tap * g.dil;
+  *out = at / g.stride;
+  return at >= 0 && at % g.stride == 0 && *out < size;
+}
+
+// Where value `s` of the first list meets column `c`: its partner in row m is element *at + m * *pitch.
+template <Product PRODUCT>
+__device__ __forceinline__ bool first_meets(const Geometry& g, const OddSpot& s, const OddSpot& c,
+                                            long long* at, long long* pitch) {
+  const AxisOf gh{g.stride_h, g.pad_h, g.dil_h}, gw{g.stride_w, g.pad_w, g.dil_w};
+  const int taps = g.KH * g.KW;
+  int h, w;
+  if (PRODUCT == kWeight) {   // x with dy
+    if (s.b != c.a || !out_of(gh, s.h, c.h, g.OH, &h) || !out_of(gw, s.w, c.w, g.OW, &w)) return false;
+    *pitch = static_cast<long long>(g.OH) * g.OW;
+    *at = s.a * g.D * *pitch + h * g.OW + w;
+    return true;
+  }
+  if (s.a != c.a) return false;
+  const bool forward = PRODUCT == kForward;   // x with the weights, dy with the weights
+  if (!tap_of(gh, forward ? s.h : c.h, forward ? c.h : s.h, g.KH, &h) ||
+      !tap_of(gw, forward ? s.w : c.w, forward ? c.w : s.w, g.KW, &w))
+    return false;
+  *pitch = forward ? static_cast<long long>(g.C) * taps : taps;
+  *at = static_cast<long long>(s.b) * (forward ? taps : g.C * taps) + h * g.KW + w;
+  return true;
+}
+// The row of the result that value `s` of the second list belongs to, and its partner in column `c`.
+template <Product PRODUCT>
+__device__ __forceinline__ int second_row(const OddSpot& s) { return PRODUCT == kForward ? s.a : s.b; }
+template <Product PRODUCT>
+__device__ __forceinline__ bool second_meets(const Geometry& g, const OddSpot& s, const OddSpot& c,
+                                             long long* at) {
+  const AxisOf gh{g.stride_h, g.pad_h, g.dil_h}, gw{g.stride_w, g.pad_w, g.dil_w};
+  int h, w;
+  if (PRODUCT == kData) {   // the weights with dy
+    if (!out_of(gh, c.h, s.h, g.OH, &h) || !out_of(gw, c.w, s.w, g.OW, &w)) return false;
+    *at = ((static_cast<long long>(c.a) * g.D + s.a) * g.OH + h) * g.OW + w;
+    return true;
+  }
+  const bool forward = PRODUCT == kForward;   // the weights with x, dy with x
+  if (!in_of(gh, forward ? c.h : s.h, forward ? s.h : c.h, g.H, &h) ||
+      !in_of(gw, forward ? c.w : s.w, forward ? s.w : c.w, g.W, &w))
+    return false;
+  const long long plane = forward ? static_cast<long long>(c.a) * g.C + s.b : static_cast<long long>(s.a) * g.C + c.a;
+  *at = (plane * g.H + h) * g.W + w;
+  return true;
+}
+
+// The column in which value `s` of the first list meets tap (h, w); false: none.
+template <Product PRODUCT>
+__device__ __forceinline__ bool column_of(const Geometry& g, const OddSpot& s, int h, int w, OddSpot* c) {
+  const AxisOf gh{g.stride_h, g.pad_h, g.dil_h}, gw{g.stride_w, g.pad_w, g.dil_w};
+  int at_h, at_w;
+  if (PRODUCT == kData) {
+    if (!in_of(gh, s.h, h, g.H, &at_h) || !in_of(gw, s.w, w, g.W, &at_w)) return false;
+  } else if (!out_of(gh, s.h, h, g.OH, &at_h) || !out_of(gw, s.w, w, g.OW, &at_w)) {
+    return false;
+  }
+  *c = PRODUCT == kWeight ? OddSpot{s.b, 0, h, w, 0.0f} : OddSpot{s.a, 0, at_h, at_w, 0.0f};
+  return true;
+}
+
+template <Product PRODUCT>
+__device__ __forceinline__ void add_odd_values(const OddJob<PRODUCT>& job, unsigned block, OddValue (*given)[kMostOdd],
+                                               OddSpot* first, OddSpot* second) {
+  const Geometry& g = job.g;
+  {
+    const int list = threadIdx.x / kMostOdd, i = threadIdx.x % kMostOdd;   // (half of the workgroup each)
+    static_assert(2 * kMostOdd == 256, "a thread per entry");
+    const OddValue mine = (list == 0 ? job.first.odd : job.second.odd)[i];   // (whether there is one or not)
+    const int count = static_cast<int>(*(list == 0 ? job.first.odd_count : job.second.odd_count));
+    if (!job.range.halves_hold()) return;   // (all of the workgroup)
+    given[list][i] = mine;
+    __syncthreads();
+    if (i < count) {
+      int rank = 0;
+      for (int k = 0; k < count; ++k)
+        rank += given[list][k].plane < mine.plane || (given[list][k].plane == mine.plane && given[list][k].at < mine.at);
+      const bool dy = PRODUCT == (list == 0 ? kData : kWeight), w = list == 1 && !dy;
+      const int per = dy ? g.D : g.C, width = dy ? g.OW : w ? g.KW : g.W;
+      (list == 0 ? first : second)[rank] =
+          OddSpot{mine.plane / per, mine.plane % per, mine.at / width, mine.at % width, mine.value};
+    }
+    __syncthreads();
+  }
+  const int n_first = static_cast<int>(*job.first.odd_count), n_second = static_cast<int>(*job.second.odd_count);
+  const int first_shift = static_cast<int>(job.first.word[1]), lane = threadIdx.x & 63, taps = g.KH * g.KW;
+  const int height = PRODUCT == kForward ? g.OH : PRODUCT == kData ? g.H : g.KH;
+  const int width = PRODUCT == kForward ? g.OW : PRODUCT == kData ? g.W : g.KW;
+  const int rows = PRODUCT == kData ? g.C : g.D;
+  const int columns = (PRODUCT == kWeight ? g.C : g.N) * height * width;
+  auto result = [&](int row, const OddSpot& c) {
+    const size_t plane = PRODUCT == kWeight ? static_cast<size_t>(row) * g.C + c.a : static_cast<size_t>(c.a) * rows + row;
+    return job.out + (plane * height + c.h) * width + c.w;
+  };
+  // which entries of a list pass a test (a lane per entry), and a walk over them
+  struct Entries { unsigned long long low, high; };
+  auto entries = [&](int count, auto test) {
+    return Entries{__ballot(lane < count && test(lane)), __ballot(64 + lane < count && test(64 + lane))};
+  };
+  auto first_of = [](const Entries& e) { return e.low != 0ull ? __builtin_ctzll(e.low) : 64 + __builtin_ctzll(e.high); };
+  auto for_each = [](Entries e, auto body) {
+    for (; e.low != 0ull; e.low &= e.low - 1ull) body(__builtin_ctzll(e.low));
+    for (; e.high != 0ull; e.high &= e.high - 1ull) body(64 + __builtin_ctzll(e.high));
+  };
+  auto from_second = [&](const Entries& which, int row, const OddSpot& c) {
+    double sum = 0.0;
+    for_each(which, [&](int k) {
+      long long at;
+      if (second_row<PRODUCT>(second[k]) != row || !second_meets<PRODUCT>(g, second[k], c, &at)) return;
+      const float v = job.second_partner[at];
+      if (!is_odd_half(v, first_shift)) sum += static_cast<double>(second[k].value) * v;
+    });
+    return sum;
+  };
+  const int row_chunks = (rows + 63) / 64, column_chunks = (columns + 63) / 64;
+  const long long column_tasks = static_cast<long long>(n_first) * taps * row_chunks;
+  const long long tasks = column_tasks + static_cast<long long>(n_second) * column_chunks;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (long long task = block * 4 + wave; task < tasks; task += kOddGroups * 4) {
+    long long at, pitch;
+    if (task < column_tasks) {   // a column that the first list meets: a lane per row
+      const int i = static_cast<int>(task / (taps * row_chunks)), rest = static_cast<int>(task - static_cast<long long>(i) * taps * row_chunks);
+      const int tap = rest / row_chunks, row0 = (rest - tap * row_chunks) * 64, row = row0 + lane;
+      OddSpot c;
+      if (!column_of<PRODUCT>(g, first[i], tap / g.KW, tap % g.KW, &c)) continue;
+      const Entries met = entries(n_first, [&](int k) { return first_meets<PRODUCT>(g, first[k], c, &at, &pitch); });
+      if (first_of(met) != i) continue;
+      const Entries there = entries(n_second, [&](int k) { return second_row<PRODUCT>(second[k]) / 64 == row0 / 64; });
+      if (row >= rows) continue;
+      float* const to = result(row, c);
+      const float before = *to;
+      double sum = 0.0;
+      for_each(met, [&](int k) {
+        (void)first_meets<PRODUCT>(g, first[k], c, &at, &pitch);
+        sum += static_cast<double>(first[k].value) * job.first_partner[at + row * pitch];
+      });
+      *to = static_cast<float>(before + (sum + from_second(there, row, c)));
+    } else {   // a row that the second list has values of, in columns that the first does not meet: a lane per column
+      const int i = static_cast<int>((task - column_tasks) / column_chunks), row = second_row<PRODUCT>(second[i]);
+      const int column = static_cast<int>(task - column_tasks - static_cast<long long>(i) * column_chunks) * 64 + lane;
+      const Entries there = entries(n_second, [&](int k) { return second_row<PRODUCT>(second[k]) == row; });
+      if (first_of(there) != i) continue;
+      if (column >= columns) continue;
+      const int a = column / (height * width), r = column - a * (height * width);
+      const OddSpot c{a, 0, r / width, r % width, 0.0f};
+      bool met = false;
+      for (int k = 0; k < n_first; ++k) met = met || first_meets<PRODUCT>(g, first[k], c, &at, &pitch);
+      if (met) continue;
+      float* const to = result(row, c);
+      *to = static_cast<float>(*to + from_second(there, row, c));
+    }
+  }
+}
+// (of one product, or of both gradients)
+template <Product ONE, Product OTHER>
+__global__ void __launch_bounds__(256) odd_values_kernel(OddJob<ONE> one, OddJob<OTHER> other) {
+  __shared__ OddValue given[2][kMostOdd];
+  __shared__ OddSpot first[kMostOdd], second[kMostOdd];
+  if (blockIdx.x < one.blocks) add_odd_values(one, blockIdx.x, given, first, second);
+  else add_odd_values(other, blockIdx.x - one.blocks, given, first, second);
 }
 
 // Results of the split tiles: sum of their pieces, in piece order and in 64 bits (there may be hundreds, and

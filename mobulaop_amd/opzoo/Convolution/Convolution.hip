@@ -1032,10 +1032,11 @@ bool gradients_b16(const conv::Geometry& g, const float* dy, const float* x, con
 // product and return at once unless a tensor holds values the parts do not stand for (conv::SplitRange).
 //
 // Two fp16 parts (halves) take half the matrix instructions: forward and both gradients of that layer 1819 -> 1157 us, errors
-// 1.4e-7 and 1.7e-7, as their sums start anew every 256 terms.  They need every value to lie within 2^27 of the tensor's
-// largest, or beside a value that does: in a group of 64 channels at its pixel where sums run over channels, of 64
-// pixels in its channel where they run over pixels.  What is found to lie further off while the halves are written sends
-// the product to three parts, and those to the fp32 kernels.
+// 1.4e-7 and 1.7e-7, as their sums start anew every 256 terms.  Both parts hold values within some 2^26 of the tensor's
+// largest; up to 128 others are added behind the product in 64 bits (conv::odd_values_kernel: 5 us where there is none or one, and
+// forward and both gradients of that layer 1120 us -> 1190 with 100 of x's, 1160 of dy's, 1530 of the weights', which each reach
+// a whole plane of every image; 1790 from three parts).  A tensor with more goes to three parts, and from there to the fp32
+// kernels: values all over 2^60, 3040 us with three parts tried first and 3230 with halves.
 
 // Fewest terms of a sum that is formed from parts by choice.  What is left out of a product (up to half a unit of
 // its last place) counts where no rounding of a longer sum exceeds it: errors of parts against 64 bits are 1.02-1.03 of
@@ -1075,15 +1076,14 @@ bool short_sums(const Ops& ops) {
 }
 
 // What is kept of the tensors of a call ahead of its operands.
-constexpr size_t kWordBytes = 1024 + 3 * sizeof(unsigned) * conv::kMagnitudes;
-// Tensors of more elements are sampled for their magnitude (an eighth of them: 23 -> 6 us for 103 MB): the largest
-// value may be sixteen times the largest that was seen, else the product is formed from three parts.  (Those sixteen are
-// missing below: values within 2^23 of the tensor's largest.)
-constexpr long long kSampledElements = 1 << 20;
-conv::TensorWords tensor_words(char* ws, int t, long long elements) {
+constexpr size_t kMagnitudeBytes = sizeof(unsigned) * conv::kMagnitudes, kListBytes = sizeof(conv::OddValue) * conv::kMostOdd;
+constexpr size_t kWordBytes = 1024 + 3 * (kMagnitudeBytes + kListBytes);
+static_assert(kWordBytes % 256 == 0, "operands on 256-byte boundaries");
+conv::TensorWords tensor_words(char* ws, int t) {
   unsigned* const words = reinterpret_cast<unsigned*>(ws) + 4 * t;
-  return conv::TensorWords{words, words + 2, reinterpret_cast<const unsigned*>(ws + 1024) + t * conv::kMagnitudes,
-                           elements > kSampledElements ? 4 : 0};
+  char* const behind = ws + 1024 + t * (kMagnitudeBytes + kListBytes);
+  return conv::TensorWords{words, words + 2, words + 3, reinterpret_cast<const unsigned*>(behind),
+                           reinterpret_cast<conv::OddValue*>(behind + kMagnitudeBytes)};
 }
 
 // Microseconds of the fp32 ways from the CU clocks of their kernels (which know nothing of rounds that are not full)
@@ -1141,7 +1141,7 @@ bool forward_split(const conv::Geometry& g, const float* x, const float* weight,
       mobula_hip::workspace_if_possible(kWordBytes + operands + fp32.plan.bytes + kPieceBytes));
   if (ws == nullptr) return failed();
   const long long w_count = static_cast<long long>(g.D) * g.C * taps;
-  const conv::TensorWords x_words = tensor_words(ws, 0, x_count), w_words = tensor_words(ws, 1, w_count);
+  const conv::TensorWords x_words = tensor_words(ws, 0), w_words = tensor_words(ws, 1);
   conv::SplitRange range{x_words.exponents, w_words.exponents, conv::SplitRange::most_exponents(g.C * taps)};
   char* const tables = ws + kWordBytes + operands;
   float* const pieces = reinterpret_cast<float*>(tables + fp32.plan.bytes);
@@ -1150,7 +1150,6 @@ bool forward_split(const conv::Geometry& g, const float* x, const float* weight,
   place_gather(&fp32.plan, tables);
   if (by_halves) {
     range.halves_a = x_words.word; range.halves_b = w_words.word;
-    range.halves_mask = conv::kBeyondHalves | conv::kLonePixel;
     halves.ops.src_word = x_words.word; halves.ops.weight_word = w_words.word;
     halves.place(ws + kWordBytes);
     const conv::MagnitudeJob job{{x, weight, nullptr}, {x_count, w_count, 0}, {x_words, w_words, {}}};
@@ -1160,6 +1159,8 @@ bool forward_split(const conv::Geometry& g, const float* x, const float* weight,
     const conv::AgainJob again = again_job(parts.prep, words, fp32.plan.tables, {}, range, {});
     conv::reduce_or_again_kernel<conv::ForwardOpsB16<conv::kHalves>><<<left.blocks + again.blocks, 256, 0, stream>>>(
         halves.ops, left, again);
+    const conv::OddJob<conv::kForward> odd{g, weight, x, y, x_words, w_words, range, conv::kOddGroups};
+    conv::odd_values_kernel<conv::kForward, conv::kForward><<<odd.blocks, 256, 0, stream>>>(odd, {});
   } else {
     conv::clear_words_kernel<<<1, 64, 0, stream>>>(reinterpret_cast<unsigned*>(ws), 12);
     parts.prep.launch<3>(stream, words);
@@ -1196,8 +1197,7 @@ bool gradients_split(int form, const conv::Geometry& g, const float* dy, const f
   const long long dy_count = static_cast<long long>(g.N) * g.D * g.OH * g.OW;
   const long long x_count = dw != nullptr ? static_cast<long long>(g.N) * g.C * g.H * g.W : 0;
   const long long w_count = dx != nullptr ? static_cast<long long>(g.D) * g.C * taps : 0;
-  const conv::TensorWords dy_words = tensor_words(ws, 0, dy_count), x_words = tensor_words(ws, 1, x_count),
-                          w_words = tensor_words(ws, 2, w_count);
+  const conv::TensorWords dy_words = tensor_words(ws, 0), x_words = tensor_words(ws, 1), w_words = tensor_words(ws, 2);
   conv::SplitRange data_range{dy_words.exponents, w_words.exponents, conv::SplitRange::most_exponents(g.D * taps)};
   conv::SplitRange weight_range{dy_words.exponents, x_words.exponents,
                                 conv::SplitRange::most_exponents(static_cast<long long>(g.N) * g.OH * g.OW)};
@@ -1212,8 +1212,6 @@ bool gradients_split(int form, const conv::Geometry& g, const float* dy, const f
   if (by_halves) {
     data_range.halves_a = weight_range.halves_a = dy_words.word;
     data_range.halves_b = w_words.word; weight_range.halves_b = x_words.word;
-    data_range.halves_mask = conv::kBeyondHalves | conv::kLonePixel;
-    weight_range.halves_mask = conv::kBeyondHalves | conv::kLoneChannel;
     halves.data.src_word = halves.weight.dy_word = dy_words.word;
     halves.data.weight_word = w_words.word; halves.weight.x_word = x_words.word;
     halves.place(at);
@@ -1225,6 +1223,9 @@ bool gradients_split(int form, const conv::Geometry& g, const float* dy, const f
         halves, left, bias,
         again_job(parts.prep, words, plan.tables, taps_of_weight, dx != nullptr ? data_range : weight_range,
                   dx != nullptr && dw != nullptr ? weight_range : conv::SplitRange{}), stream);
+    const conv::OddJob<conv::kData> odd_dx{g, weight, dy, dx, dy_words, w_words, data_range, dx != nullptr ? conv::kOddGroups : 0u};
+    const conv::OddJob<conv::kWeight> odd_dw{g, dy, x, dw, x_words, dy_words, weight_range, dw != nullptr ? conv::kOddGroups : 0u};
+    conv::odd_values_kernel<conv::kData, conv::kWeight><<<odd_dx.blocks + odd_dw.blocks, 256, 0, stream>>>(odd_dx, odd_dw);
   } else {
     conv::clear_words_kernel<<<1, 64, 0, stream>>>(reinterpret_cast<unsigned*>(ws), 12);
     parts.prep.launch<3>(stream, words, bias);

@@ -927,10 +927,12 @@ def test_fp32_products_of_two_halves(shape, scale, halves_always):
     assert torch.equal(again[1], start[0] + got[1]) and torch.equal(again[2], start[1] + got[2])
 
 
-@pytest.mark.parametrize('odd', ['lone pixel', 'lone channel', 'small beside large', 'unseen', 'inf', 'nan', 'overflow'])
+@pytest.mark.parametrize('odd', ['lone pixel', 'lone channel', 'small beside large', 'listed', 'one more', 'far larger', 'unseen', 'inf',
+                                 'nan', 'overflow'])
 def test_values_that_two_halves_do_not_stand_for(odd, halves_always):
-    """A tensor whose values lie too far apart for two halves is multiplied in three parts (the same bits as when they are
-    asked for) or by the fp32 kernels; small values beside large ones, and zeros, stay with the halves."""
+    """Up to 128 values of a tensor that are out of the range of two halves are listed and added behind the product; a tensor with
+    more is multiplied in three parts (the same bits as when they are asked for), one that is not finite by the fp32
+    kernels."""
     shape = (2, 96, 80, 80, 64, (3, 3), (1, 1), (1, 1), (1, 1))     # x: 1.2 million elements, an eighth of them looked at
     (x, w, dy), geo, _, _ = _layer(shape, 99)
     dy[:, :, 10:30] = 0.0
@@ -942,7 +944,11 @@ def test_values_that_two_halves_do_not_stand_for(odd, halves_always):
     elif odd == 'small beside large':
         x[1, 3, 7, 9] *= 2.0 ** -60
         dy[0, 1, 40, 3] = 1e-40
-    elif odd == 'unseen':              # (elements 4096 to 36863 are not looked at)
+    elif odd in ('listed', 'one more'):
+        x.view(-1)[:9000 * (128 + (odd == 'one more')):9000] *= 2.0 ** -40
+    elif odd == 'far larger':          # than all others: a thousand of them lie below 2^-27 of it
+        x.view(-1)[5024] = 1e5
+    elif odd == 'unseen':              # (the line of elements 4992 to 5023 is not looked at)
         x.view(-1)[5000] = 1e5
     elif odd == 'overflow':
         x.abs_().mul_(2.0 ** 124), w.abs_().mul_(2.0 ** 20), dy.abs_().mul_(2.0 ** 60)   # (of one sign: whatever the order)
@@ -958,10 +964,87 @@ def test_values_that_two_halves_do_not_stand_for(odd, halves_always):
         fine = b.isfinite()
         assert (a[fine].double() - b[fine].double()).norm() <= 2e-6 * b[fine].double().norm(), what
     same = [torch.equal(a.nan_to_num(), b.nan_to_num()) for a, b in zip(got, parts)]
-    # which products left the halves: sums over channels where a pixel is far off, over pixels where a channel is
-    assert same == {'lone pixel': [True, True, False], 'lone channel': [False, False, True],
-                    'small beside large': [False, False, False], 'unseen': [True, False, True],
-                    'inf': [True, False, True], 'nan': [True, False, True], 'overflow': [True, False, True]}[odd]
+    # which products left the halves
+    assert same == {'lone pixel': [False, False, False], 'lone channel': [True, False, True],
+                    'small beside large': [False, False, False], 'listed': [False, False, False], 'one more': [True, False, True],
+                    'far larger': [True, False, True], 'unseen': [False, False, False], 'inf': [True, False, True], 'nan': [True, False, True],
+                    'overflow': [True, False, True]}[odd]
+
+
+def _made_of_small_values(shape, which, scale, few, seed):
+    """x, w, dy of which `which` holds small values (scale times the rest; scale 0: subnormals) that make up whole results:
+    what would meet larger values beside them is zero in the other operand.  few: in a few places, else wherever there
+    are any of that kind."""
+    N, C, H, W, D, kernel, pad, stride, dil = shape
+    g = torch.Generator().manual_seed(seed)
+    x, w = torch.randn(N, C, H, W, generator=g), torch.randn(D, C, *kernel, generator=g)
+    dy = torch.randn(F.conv2d(x, w, None, stride=stride, padding=pad, dilation=dil).shape, generator=g)
+
+    def small(t):
+        return t.sign() * 2.0 ** -133 if scale == 0 else t * scale
+
+    def small_above(t, c):
+        """Channel c of t: small values in the rows above the eighth, larger ones from the twelfth on."""
+        kept = torch.zeros_like(t[:, c])
+        where = (slice(None), slice(3, 5), slice(4, 6)) if few else (slice(None), slice(0, 8))
+        kept[where] = small(t[:, c][where])
+        kept[:, 12:] = t[:, c, 12:]
+        t[:, c] = kept
+    if which == 'all':       # one value in twenty is not zero, and a few of those are small: they meet each other, too
+        for t in x, w, dy:
+            t.mul_(torch.rand(t.shape, generator=g) < 0.05)
+            flat = t.view(-1)
+            places = flat.nonzero().flatten()
+            places = places[torch.randperm(len(places), generator=g)[:40 if few else len(places) // 3]]
+            flat[places] = small(flat[places])
+    elif which == 'x':
+        small_above(x, 5)
+        w[:3, [c for c in range(C) if c != 5]] = 0.0   # filters that read this channel alone
+        dy[:, :3, 3:] = 0.0                            # and whose gradients do not meet its larger values
+    elif which == 'w':
+        index = (slice(1, 2), slice(7, 9)) if few else (slice(0, 2),)
+        w[index] = small(w[index])
+        x[:, [c for c in range(C) if c not in (7, 8)], :8] = 0.0   # where nothing but these channels is not zero
+        dy[:, [d for d in range(D) if d != 1], :8] = 0.0           # and nothing but this filter's gradient
+    else:
+        small_above(dy, 2)
+        w[[d for d in range(D) if d != 2], 1] = 0.0    # a channel that this filter alone reads
+        x[:, :2, 8:] = 0.0                             # and whose values do not meet the gradient's larger ones
+    return x, w, dy
+
+
+@pytest.mark.parametrize('few', [True, False])
+@pytest.mark.parametrize('scale', [2.0 ** 30, 2.0 ** -24, 2.0 ** -40, 0.0])
+@pytest.mark.parametrize('which', ['x', 'w', 'dy', 'all'])
+@pytest.mark.parametrize('shape', [
+    (2, 64, 16, 19, 64, (3, 3), (1, 1), (1, 1), (1, 1)),
+    (3, 33, 21, 18, 65, (3, 2), (2, 1), (2, 1), (1, 2)),         # strides, dilation, odd counts
+    (2, 96, 80, 80, 64, (3, 3), (1, 1), (1, 1), (1, 1)),         # more than a million elements
+])
+def test_results_that_small_values_alone_make_up(shape, which, scale, few, halves_always):
+    """A value that is small for its tensor makes up a result where the larger ones beside it meet zeros.  Element by element
+    against 64 bits: four and a half units of the magnitudes that are added (2^-23 of a value for either operand's last bit,
+    2^-22 for the product of the tails, 2^-24 for the result; the roundings within sums are far below that of so many
+    terms, but for a few values that are larger than all others: there every later one of up to six for sixteen
+    terms is 2^-24 of the whole).  Subnormal results
+    besides: half of 2^-149 for every product that is not zero (the fp32 kernels, which take tensors with many of
+    them, round each) and for the result."""
+    x, w, dy = _made_of_small_values(shape, which, scale, few, 107)
+    N, C, H, W, D, kernel, pad, stride, dil = shape
+    geo = _ci(N, C, H, W, D, kernel[0], kernel[1], pad[0], pad[1], stride[0], stride[1], dil[0], dil[1])
+    want, sizes, products = [], [], []
+    for out, f in (want, lambda t: t.double()), (sizes, lambda t: t.double().abs()), (products, lambda t: (t != 0).double()):
+        xr, wr = f(x).requires_grad_(True), f(w).requires_grad_(True)
+        y = F.conv2d(xr, wr, None, stride=stride, padding=pad, dilation=dil)
+        y.backward(f(dy))
+        out += [y.detach(), xr.grad, wr.grad]
+    _leave_nan_patterns_in_the_workspace()
+    got = _three_products(geo, x.cuda(), w.cuda(), dy.cuda())
+    terms = C * kernel[0] * kernel[1], D * kernel[0] * kernel[1], dy[:, 0].numel()
+    for a, b, size, count, k, what in zip(got, want, sizes, products, terms, ('y', 'dx', 'dw')):
+        units = 2.0 ** -21 + 2.0 ** -24 + (2.0 ** -24 * 6 * (k / 16 + 1) if scale > 1 else 0.0)
+        off = (a.cpu().double() - b).abs() - (units * size + 2.0 ** -150 * (count + 1))
+        assert (off <= 0).all(), (what, float((off / size.clamp_min(1e-300)).max()), int((off > 0).sum()))
 
 
 @pytest.mark.parametrize('shape', [
