@@ -1057,7 +1057,8 @@ int split_choice() { return mobula_hip::option("conv_fp32_split", 1); }
 // halves is off by the last of its 24 bits for a quarter of the values, and what the product of both tails adds is left out:
 // 0.75e-7 of the result however long the sum; three parts lose less to that and more to long sums.  Errors of
 // halves and of three parts against 64 bits: 1.14e-7 and 0.78e-7 with 176 terms in one go, 1.20 and 1.14 with 400, 1.24 and
-// 1.47 with 704, 1.4 and 2.9 with 2304.
+// 1.47 with 704, 1.4 and 2.9 with 2304.  The fp32 kernels are further off than halves from 512 terms on (1.34 and 1.17 for
+// the weight gradient of 8 x 432 x 8 x 9, 384 filters 3 x 3, 576 terms).
 constexpr long long kLeastTermsOfHalves = 512;
 
 // How a product of sums of `terms` terms may be formed: kHalves, three parts, or 0 (fp32 kernels).
@@ -1069,10 +1070,15 @@ int form_of(long long terms) {
     default: return terms >= kLeastTermsOfHalves ? conv::kHalves : terms >= kLeastTerms ? 3 : 0;
   }
 }
-// True where the product's sums are too short, as it would be cut along K.
+// True where the product's sums are too short for halves, as it would be cut along K: in themselves, or beside those
+// of three parts where these are the other way (`parts`: the K steps of their longest sum, 0: they are not).  Three parts are off
+// by some 0.058e-7 times the root of their longest sum's terms, halves by 1.2e-7 below a thousand terms, 1.4 with 1500, 1.9 with
+// 13000: weight gradient of 8 x 512 x 14 x 14, 512 filters 3 x 3, 1568 terms, 1.27e-7 in three parts, which cut it into three
+// (88 us), and 1.40 in halves, which do not (81).
 template <typename Ops>
-bool short_sums(const Ops& ops) {
-  return split_choice() == 1 && plan_b16(ops).longest * 16 < kLeastTermsOfHalves;
+bool short_sums(const Ops& ops, int parts) {
+  const int longest = plan_b16(ops).longest * 16;
+  return split_choice() == 1 && (longest < kLeastTermsOfHalves || (parts > 0 && parts * 16 < 480 + longest / 12));
 }
 
 // What is kept of the tensors of a call ahead of its operands.
@@ -1129,10 +1135,13 @@ bool forward_split(const conv::Geometry& g, const float* x, const float* weight,
   ForwardB16<3> parts;
   ForwardB16<conv::kHalves> halves;
   if (parts.plan(g, x, weight, bias, y) != kFits) return false;
-  const bool by_halves = form == conv::kHalves && halves.plan(g, x, weight, bias, y) == kFits && !short_sums(halves.ops);
+  bool by_halves = form == conv::kHalves && halves.plan(g, x, weight, bias, y) == kFits;
   if (by_choice) {
-    const double product = by_halves ? plan_b16(halves.ops).cost : plan_b16(parts.ops).cost;
-    if (product + parts_us(by_halves ? conv::kHalves : 3, x_count) + kSplitOverhead > forward_fp32_us(fp32_cost)) return false;
+    const double rest = forward_fp32_us(fp32_cost) - kSplitOverhead;   // what is left for a product and its operands
+    const PlanB16 with_parts = plan_b16(parts.ops);
+    const bool parts_win = with_parts.cost + parts_us(3, x_count) <= rest;
+    by_halves = by_halves && !short_sums(halves.ops, parts_win ? with_parts.longest : 0);
+    if (by_halves ? plan_b16(halves.ops).cost + parts_us(conv::kHalves, x_count) > rest : !parts_win) return false;
   }
   ForwardFallback fp32;
   if (!fp32.make(g, weight)) return true;
@@ -1254,16 +1263,23 @@ bool gradients_split(int form, const conv::Geometry& g, const float* dy, const f
 // 23 x 256 x 72 x 64, 32: 230 against 238).
 struct SplitChoice { int dx, dw; };
 
-// What the gradients that `form` may stand for cost (< 0: it may not).
-struct GradientCosts { double data, weight; };
+// What the gradients that FORM may stand for cost (< 0: it may not), and the K steps of their longest sums (parts_dx,
+// parts_dw: see short_sums).
+struct GradientCosts { double data, weight; int longest_data, longest_weight; };
 template <int FORM>
-GradientCosts gradient_costs(const conv::Geometry& g, bool dx, bool dw) {
-  GradientCosts cost{-1.0, -1.0};
+GradientCosts gradient_costs(const conv::Geometry& g, bool dx, bool dw, int parts_dx = 0, int parts_dw = 0) {
+  GradientCosts cost{-1.0, -1.0, 0, 0};
   BackwardB16<FORM> b;
   float any;   // (for its address: nothing is written)
   if (b.plan(g, &any, &any, &any, 0, dx ? &any : nullptr, dw ? &any : nullptr) != kFits) return cost;
-  if (dx && !(FORM == conv::kHalves && short_sums(b.data))) cost.data = plan_b16(b.data).cost;
-  if (dw && !(FORM == conv::kHalves && short_sums(b.weight))) cost.weight = plan_b16(b.weight).cost;
+  if (dx && !(FORM == conv::kHalves && short_sums(b.data, parts_dx))) {
+    const PlanB16 plan = plan_b16(b.data);
+    cost.data = plan.cost; cost.longest_data = plan.longest;
+  }
+  if (dw && !(FORM == conv::kHalves && short_sums(b.weight, parts_dw))) {
+    const PlanB16 plan = plan_b16(b.weight);
+    cost.weight = plan.cost; cost.longest_weight = plan.longest;
+  }
   return cost;
 }
 
@@ -1282,7 +1298,6 @@ SplitChoice choose_split(const conv::Geometry& g, bool dx, bool dw) {
   if (!dx && !dw) return SplitChoice{0, 0};
   const GradientCosts parts = gradient_costs<3>(g, dx, dw);
   dx = dx && parts.data >= 0; dw = dw && parts.weight >= 0;
-  const GradientCosts halves = gradient_costs<conv::kHalves>(g, dx && data_form == conv::kHalves, dw && weight_form == conv::kHalves);
   double data_fp32 = 0.0, weight_fp32 = 0.0;
   if (dx) {
     const DataPatches patches = data_patches(g, nullptr, nullptr, nullptr, 0);
@@ -1305,6 +1320,9 @@ SplitChoice choose_split(const conv::Geometry& g, bool dx, bool dw) {
   if (dx && dw) consider(3, 3, parts.data + parts.weight + dy3 + x3 + 1.3 * kSplitOverhead);
   // (what three parts win does not go to the fp32 kernels, whose sums lose more, for the sake of the other product)
   const SplitChoice with_parts = best.choice;
+  const GradientCosts halves = gradient_costs<conv::kHalves>(g, dx && data_form == conv::kHalves, dw && weight_form == conv::kHalves,
+                                                             with_parts.dx != 0 ? parts.longest_data : 0,
+                                                             with_parts.dw != 0 ? parts.longest_weight : 0);
   auto upgrade = [&](int a, int b, double cost) {
     if ((with_parts.dx == 0 || a != 0) && (with_parts.dw == 0 || b != 0)) consider(a, b, cost);
   };

@@ -1065,6 +1065,19 @@ def test_sums_formed_by_choice_are_no_further_off_than_those_of_three_parts_or_f
     for chosen, parts, fp32, what in zip(errors[1], errors[2], errors[0], ('y', 'dx', 'dw')):
         assert chosen <= 1.02 * max(parts, fp32), (what, chosen, parts, fp32)
 
+def test_sums_that_three_parts_cut_shorter_are_left_to_them():
+    """A weight gradient of few pixels, which is cut along K: shorter sums in three parts than in halves, and nearer."""
+    (x, w, dy), geo, want, _ = _layer((8, 512, 14, 14, 512) + ((3, 3), (1, 1), (1, 1), (1, 1)), 100)
+    errors = {}
+    try:
+        for option in 1, 2:
+            native.set_option('conv_fp32_split', option)
+            errors[option] = ((_three_products(geo, x, w, dy)[2].cpu().double() - want[2]).norm() / want[2].norm()).item()
+    finally:
+        native.set_option('conv_fp32_split', 1)
+    assert errors[1] <= 1.02 * errors[2]
+
+
 def test_halves_in_a_recorded_graph(halves_always):
     """What is known of the operands is found anew by every replay: halves, three parts, halves again."""
     shape = (2, 64, 24, 28, 128, (3, 3), (1, 1), (1, 1), (1, 1))
