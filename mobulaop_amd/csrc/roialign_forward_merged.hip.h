@@ -118,8 +118,8 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
   // behind the jobs: boxes of larger grids, from the map itself (as a launch of their own, which found nothing to do for
   // boxes on their map, they took 4 us a call)
   if (blockIdx.x >= jobs) {
-    static_assert(M::NW == 1, "a wavefront for 64 boxes");
-    forward_large_grid<T, NHWC>(64ll * (blockIdx.x - jobs), rois_listed, x, scale, C, H, W, PH, PW, S, rois, y, num_images);
+    static_assert(M::NW == 1, "a wavefront per box");
+    forward_large_grid<T, NHWC>(blockIdx.x - jobs, x, scale, C, H, W, PH, PW, S, rois, y, num_images);
     return;
   }
 

@@ -195,8 +195,8 @@ void forward_device(const Problem& p, const T* x, const float* rois, T* y, hipSt
   const int nw = small_grid ? FB::NW : roialign::FwdMerged::NW;   // wavefronts per workgroup of the gather
   const int parts = roialign::forward_row_parts(p.R, cblk, p.PH, !small_grid);
   const long long grid = roialign::blocked_grid(static_cast<long long>(p.R) * parts, cblk, nw);
-  // boxes whose sampling grid has more than 64 points per axis have workgroups of their own behind the others
-  const long long large_blocks = !small_grid && (p.S <= 0 || p.S > roialign::kSearchedGrid) ? (p.R + 63) / 64 : 0;
+  // boxes whose sampling grid has more than 64 points per axis: a workgroup each, behind the others
+  const long long large_blocks = !small_grid && (p.S <= 0 || p.S > roialign::kSearchedGrid) ? p.R : 0;
   const bool fits = rpp > 0 && p.N > 0 && p.N < 65536 && cblk < 65536 && grid + large_blocks < (1ll << 31);
   if (p.nhwc) {
     // the map is read where it lies: no copy, only the ROI ordering before the gather

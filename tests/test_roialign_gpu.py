@@ -1342,6 +1342,37 @@ def test_adaptive_grids_with_items_shared_by_wavefronts_and_boxes_far_larger_tha
     assert_parity(y, want, FWD_TOL, 'y')
 
 
+@pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
+@pytest.mark.parametrize('S', [0, 65])
+def test_boxes_of_large_grids_do_not_wait_for_each_other(S, layout):
+    """64 boxes of more than 64 points a bin take about as long as one (less than eight times, a wavefront each; one wavefront for
+    all of them 64 times)."""
+    abi.set_impl('auto')
+    rng = np.random.default_rng(S)
+    N, C, H, W, R, pooled = 1, 32, 80, 96, 64, (1, 1)
+    rois = np.concatenate([np.zeros((R, 1)), rng.uniform(0, 6, (R, 2)), rng.uniform(72, 79, (R, 2))], 1).astype(np.float32)
+    x = rng.standard_normal((N, C, H, W)).astype(np.float32)
+    want = oracle.forward(x, rois, pooled, 1.0, S)
+    xd = abi.to_dev(x if layout == 'nchw' else np.ascontiguousarray(x.transpose(0, 2, 3, 1)))
+    call = abi.forward if layout == 'nchw' else abi.forward_nhwc
+
+    def time_of(boxes):
+        rd, best = abi.to_dev(boxes), float('inf')
+        for _ in range(4):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            y = call(xd, rd, pooled, 1.0, S)
+            end.record()
+            torch.cuda.synchronize()
+            best = min(best, start.elapsed_time(end))
+        return best, y
+    one, _ = time_of(rois[:1])
+    all_of_them, y = time_of(rois)
+    y = y.cpu().numpy()
+    assert_parity(y if layout == 'nchw' else y.transpose(0, 3, 1, 2), want, FWD_TOL, 'y')
+    assert all_of_them < 8 * one
+
+
 @pytest.mark.parametrize('W', [200, 203])
 @pytest.mark.parametrize('dtype', [np.float32, np.float16])
 def test_few_boxes_on_a_large_map_copy_only_what_they_touch(W, dtype):
