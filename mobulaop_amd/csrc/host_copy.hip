@@ -232,8 +232,17 @@ class Copier {
     }
   }
 
+  // The lanes follow what the caller's stream has been given: it may use the memory that a transfer writes, or
+  // write what one reads.
+  void follow(hipStream_t stream) {
+    MOBULA_HIP_TRY(hipEventRecord(ordered_, stream));
+    for (const hipStream_t lane : lanes_)
+      if (!failed()) MOBULA_HIP_TRY(hipStreamWaitEvent(lane, ordered_, 0));
+  }
+
   void send(char* dev, hipStream_t stream) {
     int issued = 0, sent = 0;
+    follow(stream);
     while (issued < job_.transfers && !failed()) {
       bool moved = false;
       if (issued < sent + kSlots && job_.is_copied(issued)) {   // (beyond: the slot still counts the round before)
@@ -263,10 +272,7 @@ class Copier {
 
   void receive(const char* dev, hipStream_t stream) {
     int issued = 0, arrived = 0;
-    // the lanes follow what the caller's stream has been given
-    MOBULA_HIP_TRY(hipEventRecord(ordered_, stream));
-    for (const hipStream_t lane : lanes_)
-      if (!failed()) MOBULA_HIP_TRY(hipStreamWaitEvent(lane, ordered_, 0));
+    follow(stream);
     while (job_.finished.load(std::memory_order_acquire) < job_.pieces && !failed()) {
       bool moved = false;
       if (issued < job_.transfers && (issued < kSlots || job_.is_copied(issued - kSlots))) {
