@@ -824,32 +824,31 @@ reduce_slices_kernel(const float* __restrict__ partial, float* __restrict__ out,
   *to = accumulate ? *to + s : s;
 }
 
-// The same in one step, where there is no memory for sums in between: one workgroup to a filter.
+// The same in one step, where there is no memory for sums in between: one workgroup to a filter, 64-bit sums too.
 // db[d] (+)= sum of dy[img, d, :, :]; grid (filters).  V: pixels per load.
 template <int V>
 __global__ void __launch_bounds__(256)
 bias_grad_kernel(const float* __restrict__ dy, float* __restrict__ db, int N, int D, int ohw, int accumulate) {
   typedef float vec __attribute__((ext_vector_type(V)));
-  __shared__ float part[256];
+  __shared__ double part[256];
   const int d = blockIdx.x;
-  vec v = 0.0f;
+  double s = 0.0;
   for (int img = 0; img < N; ++img) {
     const float* p = dy + (static_cast<size_t>(img) * D + d) * ohw;
 #pragma unroll 4
-    for (int i = threadIdx.x * V; i < ohw; i += 256 * V) v += *reinterpret_cast<const vec*>(p + i);
-  }
-  float s = 0.0f;
+    for (int i = threadIdx.x * V; i < ohw; i += 256 * V) {
+      const vec v = *reinterpret_cast<const vec*>(p + i);
 #pragma unroll
-  for (int k = 0; k < V; ++k) s += v[k];
+      for (int k = 0; k < V; ++k) s += v[k];
+    }
+  }
   part[threadIdx.x] = s;
   __syncthreads();
   for (int off = 128; off > 0; off >>= 1) {
     if (threadIdx.x < off) part[threadIdx.x] += part[threadIdx.x + off];
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    db[d] = accumulate ? db[d] + part[0] : part[0];
-  }
+  if (threadIdx.x == 0) db[d] = static_cast<float>(accumulate ? static_cast<double>(db[d]) + part[0] : part[0]);
 }
 
 // The reference's unfold and fold (opzoo/Convolution/Convolution.cpp:13-90), one

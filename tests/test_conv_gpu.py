@@ -538,10 +538,10 @@ def test_bias_gradient_can_be_recorded_first():
     (300, 16, 3, 3, 66, 3, 1),     # many small planes
     (4, 64, 31, 33, 256, 3, 1),    # high tiles for both gradients
 ])
-def test_bias_gradient_beside_the_others(shape, wanted, compute):
+def test_bias_gradient_beside_the_others(mobula, shape, wanted, compute):
     """The bias's gradient rides in launches of the other gradients where there are any: 64-bit sums, rounded once (half a unit
     of the result; 2^-40 of the sum of magnitudes for the 64-bit additions, of which there are fewer than 2^12)."""
-    import mobulaop_amd as mobula
+    mobula.op.load('Convolution')
     N, C, H, W, D, K, stride = shape
     gen = torch.Generator().manual_seed(sum(shape))
     x = torch.randn(N, C, H, W, generator=gen).cuda().requires_grad_('x' in wanted)
@@ -560,16 +560,20 @@ def test_bias_gradient_beside_the_others(shape, wanted, compute):
         _close(w.grad, wr.grad, 'dw', compute)
 
 
-def test_bias_gradient_that_finds_no_room_beside_the_others():
-    """A recorded call cannot grow the workspace: one that was warmed up without a bias leaves none for its sums."""
-    import mobulaop_amd as mobula
+def test_bias_gradient_that_finds_no_room_beside_the_others(mobula):
+    """A recorded call cannot grow the workspace: one that was warmed up without a bias leaves none for its sums (an image of
+    one pixel has as many sums as filters).  They are 64-bit sums all the same (the bound of
+    test_bias_gradient_beside_the_others)."""
+    N, D = 65000, 336
+    mobula.op.load('Convolution')
     gen = torch.Generator().manual_seed(8)
-    x, w = torch.randn(2, 3, 64, 64, generator=gen).cuda(), torch.randn(64, 3, 7, 7, generator=gen).cuda().requires_grad_(True)
-    b = torch.zeros(64, device='cuda', requires_grad=True)
-    dy = torch.randn(2, 64, 32, 32, generator=gen).cuda()
+    x, w = torch.randn(N, 1, 1, 1, generator=gen).cuda(), torch.randn(D, 1, 1, 1, generator=gen).cuda().requires_grad_(True)
+    b = torch.zeros(D, device='cuda', requires_grad=True)
+    dy = torch.randn(N, D, 1, 1, generator=gen).cuda()
+    dy[1::2] = 1e-3 * dy[1::2] - dy[0::2]   # (terms that nearly cancel)
 
     def gradients(*inputs):
-        y = mobula.op.Conv2D(*inputs, channels=64, kernel_size=(7, 7), strides=(2, 2), padding=(3, 3))
+        y = mobula.op.Conv2D(*inputs, channels=D, kernel_size=(1, 1))
         return torch.autograd.grad(y, inputs[1:], dy)
 
     stream = torch.cuda.Stream()
@@ -578,6 +582,7 @@ def test_bias_gradient_that_finds_no_room_beside_the_others():
             native.release_workspace()
             alone, = gradients(x, w)
             torch.cuda.synchronize()
+            assert native.workspace_bytes() < 8 * N * D
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph, stream=stream):
                 dw, db = gradients(x, w, b)
@@ -588,7 +593,8 @@ def test_bias_gradient_that_finds_no_room_beside_the_others():
                 graph.replay()
                 torch.cuda.synchronize()
                 assert torch.equal(dw, alone)
-                assert ((db.double() - dy.double().sum((0, 2, 3))).abs() <= 1e-4).all()
+                exact, size = dy.double().sum((0, 2, 3)), dy.double().abs().sum((0, 2, 3))
+                assert ((db.double() - exact).abs() <= 2.0 ** -24 * exact.abs() + 2.0 ** -40 * size).all()
             del graph
     finally:
         native.unpin_workspace()
