@@ -226,20 +226,6 @@ struct ConvArgs {
       static_cast<int>((x).size(3)), (a).D, (a).kernel[0], (a).kernel[1], (a).pad[0], (a).pad[1],           \
       (a).stride[0], (a).stride[1], (a).dil[0], (a).dil[1]
 
-// A tensor laid out like `like`: what() fills it, or a dense one that is copied into it.
-template <typename F>
-Tensor filled_like(const Tensor& like, const F& fill) {
-  const Tensor out = at::empty_like(like);
-  if (out.is_contiguous()) {
-    fill(out);
-    return out;
-  }
-  const Tensor dense = at::empty(out.sizes(), out.options());
-  fill(dense);
-  out.copy_(dense);
-  return out;
-}
-
 struct Conv2DBackward : public Node {
   ConvArgs args;
   Tensor x, weight, bias;
@@ -258,7 +244,9 @@ struct Conv2DBackward : public Node {
       if (want_w) out[1] = at::empty_like(weight);
       if (want_b) out[2] = at::empty_like(bias);
       auto dense = [](const Tensor& t) { return !t.defined() || t.is_contiguous() ? t : at::empty(t.sizes(), t.options()); };
-      const Tensor dx = dense(out[0]), dw = dense(out[1]), db = want_b ? dense(out[2]) : Tensor(), xd = x.contiguous(), w = weight.contiguous();
+      const Tensor dx = dense(out[0]), dw = dense(out[1]), db = want_b ? dense(out[2]) : Tensor();
+      // (x is read for the weights' gradient, the weights for that of x)
+      const Tensor xd = want_w ? x.contiguous() : x, w = want_x ? weight.contiguous() : weight;
       begin(dy, {});
       mobula_hip_conv2d_gradients(dev, dy.data_ptr<float>(), xd.data_ptr<float>(), w.data_ptr<float>(), GEOMETRY_OF(x, a),
                                   want_x ? dx.data_ptr<float>() : nullptr, want_w ? dw.data_ptr<float>() : nullptr,

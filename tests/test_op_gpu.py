@@ -378,3 +378,27 @@ def test_host_arrays_of_several_sizes_and_from_several_threads(mobula, shape):
     for t in threads:
         t.join()
     assert not wrong
+
+
+@pytest.mark.parametrize('wanted', ['x', 'weight', 'bias'])
+def test_convolution_gradients_copy_only_what_they_read(mobula, wanted):
+    """x and weight in another order than dense are copied for the gradients that read them: x for the weight's, the weight for x's,
+    neither for the bias's."""
+    mobula.op.load('Convolution')
+    x = torch.randn(4, 64, 64, 64, device='cuda').to(memory_format=torch.channels_last)         # 4 MB
+    weight = torch.randn(512, 64, 9, 9, device='cuda').to(memory_format=torch.channels_last)    # 10 MB
+    inputs = dict(x=x, weight=weight, bias=torch.randn(512, device='cuda'))
+    inputs[wanted].requires_grad_(True)
+    y = mobula.op.Conv2D(*inputs.values(), channels=512, kernel_size=(9, 9), strides=(4, 4), padding=(4, 4))
+    dy = torch.randn_like(y)
+    y.backward(dy)   # (the workspace is there now)
+    y = mobula.op.Conv2D(*inputs.values(), channels=512, kernel_size=(9, 9), strides=(4, 4), padding=(4, 4))
+    torch.cuda.synchronize()
+    inputs[wanted].grad = None
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    y.backward(dy)
+    size = {k: 4 * t.numel() for k, t in inputs.items()}
+    # the gradient, once dense and once in its input's order, and the other operand
+    least = {'x': 2 * size['x'] + size['weight'], 'weight': 2 * size['weight'] + size['x'], 'bias': size['bias']}[wanted]
+    assert torch.cuda.max_memory_allocated() - before <= least + (1 << 20)
