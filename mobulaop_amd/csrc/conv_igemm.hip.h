@@ -742,13 +742,14 @@ igemm_weight_kernel(BackwardWeightOps ops, int k_per_slice, int k_total, int row
 }
 
 // db[d] = sum of dy[img, d, pixel] over images and pixels, in two steps that ride in launches of other work where there is
-// some (on their own they took 6 and 4 us of a first layer's 93, most of it launch): a wavefront per kPixels pixels of a
-// plane, their sums in the order of dy; then a wavefront per filter.  All in 64 bits: of a sum whose terms nearly cancel 32 lose
-// (15 x 29 x 81 x 65: 1.0e-7 with 16 terms a thread in 32 bits and a tree, 1.5e-7 with 64, 3e-8 now).
+// some (on their own they took 6 and 4 us of a first layer's 93, most of it launch): a wavefront per run of a plane's pixels,
+// their sums in the order of dy; then a wavefront per filter.  Runs are so short that there are some 4096 (4 x 200 planes of
+// 58 x 79, on their own: 11.2 us in runs of 4096 pixels, 64 loads a lane, 7.8 in runs of 512).  All in 64 bits: of a sum whose
+// terms nearly cancel 32 lose (15 x 29 x 81 x 65: 1.0e-7 with 16 terms a thread in 32 bits and a tree, 1.5e-7 with 64, 3e-8 now).
 struct BiasJob {
-  static constexpr int kPixels = 4096;
+  static constexpr int kMostPixels = 4096, kLeastPixels = 512, kWaves = 4096;
   const float* dy; double* sums; float* db;
-  int N, D, ohw, runs, wide, accumulate;   // runs: of a plane; wide: planes are 16-byte aligned and whole quads
+  int N, D, ohw, pixels, runs, wide, accumulate;   // pixels of a run, runs of a plane; wide: planes are 16-byte aligned and whole quads
   unsigned sum_blocks, total_blocks;       // workgroups of four wavefronts; 0: no such job
 };
 __device__ __forceinline__ void bias_sums(const BiasJob& job, unsigned block) {
@@ -757,7 +758,7 @@ __device__ __forceinline__ void bias_sums(const BiasJob& job, unsigned block) {
   const long long unit = static_cast<long long>(block) * 4 + (threadIdx.x >> 6);
   if (unit >= static_cast<long long>(job.N) * job.D * job.runs) return;
   const long long plane = unit / job.runs;
-  const int first = static_cast<int>(unit - plane * job.runs) * BiasJob::kPixels, last = min(first + BiasJob::kPixels, job.ohw);
+  const int first = static_cast<int>(unit - plane * job.runs) * job.pixels, last = min(first + job.pixels, job.ohw);
   const float* const p = job.dy + plane * job.ohw;
   double s = 0.0;
   if (job.wide) {

@@ -315,16 +315,19 @@ conv::AgainJob again_job(const PrepB16& prep, const conv::ExponentWords& words, 
 }
 
 // The bias's gradient that rides in launches of a call's other work (db == nullptr: none), its sums at `at`.
-size_t bias_bytes(const conv::Geometry& g, const float* db) {
-  const long long runs = (static_cast<long long>(g.OH) * g.OW + conv::BiasJob::kPixels - 1) / conv::BiasJob::kPixels;
-  return db == nullptr ? 0 : align_to_256(sizeof(double) * static_cast<size_t>(g.N) * g.D * runs);
-}
 conv::BiasJob bias_job(int N, int D, int ohw, const float* dy, int accumulate, float* db, char* at) {
   if (db == nullptr) return conv::BiasJob{};
-  const int runs = (ohw + conv::BiasJob::kPixels - 1) / conv::BiasJob::kPixels;
-  return conv::BiasJob{dy, reinterpret_cast<double*>(at), db, N, D, ohw, runs,
+  const long long planes = static_cast<long long>(N) * D;
+  int pixels = conv::BiasJob::kMostPixels;
+  auto runs = [&] { return (static_cast<long long>(ohw) + pixels - 1) / pixels; };
+  while (pixels > conv::BiasJob::kLeastPixels && planes * runs() < conv::BiasJob::kWaves) pixels /= 2;
+  return conv::BiasJob{dy, reinterpret_cast<double*>(at), db, N, D, ohw, pixels, static_cast<int>(runs()),
                        ohw % 4 == 0 && reinterpret_cast<uintptr_t>(dy) % 16 == 0, accumulate,
-                       static_cast<unsigned>((static_cast<long long>(N) * D * runs + 3) / 4), static_cast<unsigned>((D + 3) / 4)};
+                       static_cast<unsigned>((planes * runs() + 3) / 4), static_cast<unsigned>((D + 3) / 4)};
+}
+size_t bias_bytes(const conv::Geometry& g, float* db) {
+  return db == nullptr ? 0 : align_to_256(sizeof(double) * static_cast<size_t>(g.N) * g.D *
+                                          bias_job(g.N, g.D, g.OH * g.OW, nullptr, 0, db, nullptr).runs);
 }
 // A call's workspace with `*bias_room` bytes for the bias's sums in front, or without them where that is too much (the bias
 // then has launches of its own).  optional: null where not even that can be had, else that is an error.

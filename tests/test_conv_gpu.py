@@ -532,7 +532,7 @@ def test_bias_gradient_can_be_recorded_first():
 
 @pytest.mark.parametrize('wanted', ['x w b', 'w b', 'b'])
 @pytest.mark.parametrize('shape', [
-    (2, 3, 70, 66, 7, 3, 1),       # planes of more than one run of 4096 pixels
+    (2, 3, 70, 66, 7, 3, 1),       # planes of ten runs, the last of twelve pixels
     (3, 16, 65, 63, 130, 1, 1),    # odd planes: no whole quads
     (5, 34, 9, 7, 3, 3, 2),
     (300, 16, 3, 3, 66, 3, 1),     # many small planes

@@ -1314,7 +1314,7 @@ def test_dense_grids_in_one_list_and_rows_that_pooled_rows_share(dtype, C, S, la
 @pytest.mark.parametrize('R', [1, 64, 65, 150, 1025, 2049])
 def test_adaptive_grids_with_items_shared_by_wavefronts_and_boxes_far_larger_than_the_map(R, layout):
     """Up to 1024 list items have four wavefronts each, up to 2048 two, more one; boxes of more than 64 points per axis are
-    found 64 at a time, the first and the last of such a group among them (the backward pass then takes another way: it is
+    in workgroups of their own behind the others (the backward pass then takes another way: it is
     tried without them)."""
     abi.set_impl('auto')
     rng = np.random.default_rng(R)
