@@ -31,12 +31,14 @@ namespace {
 // the next one stands in the same queue: transfers take turns in two lanes, streams of the copier that follow the
 // caller's and that the caller's then follows.  Threads copy in smaller pieces, so that a slot is emptied by all of them.
 // (Both passes of the shape above, one lane: 2293 us with transfers of 2 MB, 2068 with 4, 2189 with 8; two lanes: 1880 with
-// 2 MB, 1900 with 4; three lanes of 2 MB 1890 to 2550, four of 1 MB 1940.)
+// 2 MB, 1900 with 4; three lanes of 2 MB 1890 to 2550, four of 1 MB 1940.)  Below some seven megabytes one lane, the caller's
+// stream, with transfers of 4 MB is faster (a forward pass with a map of 2.4 MB: 150 us, two lanes 178; 6.5: 259 and 274; 9: 354 and
+// 323; 20: 603 and 540).
 constexpr size_t kTransfer = 2u << 20;
 constexpr size_t kPiece = 256u << 10;
-constexpr int kPerTransfer = static_cast<int>(kTransfer / kPiece);
 constexpr int kSlots = 12;
 constexpr int kLanes = 2;
+constexpr size_t kLanesAbove = 7u << 20;
 // Below this hipMemcpy is as fast: waking the helpers costs some twenty microseconds.
 constexpr size_t kPipelinedBytes = 2u << 20;
 constexpr int kMostHelpers = 7;
@@ -51,28 +53,29 @@ struct Job {
   char* host = nullptr;
   size_t bytes = 0;
   bool to_device = false;
-  int pieces = 0, transfers = 0;
+  size_t transfer = kTransfer;   // bytes of one, and of a slot
+  int ring = kSlots, per_transfer = 0, pieces = 0, transfers = 0;
   char* slots = nullptr;
   std::atomic<int> next{0}, open{0}, finished{0};
   std::atomic<int> copied[kSlots];   // pieces of the slot's transfer that have been copied
 
-  size_t transfer_bytes(int t) const { return std::min(kTransfer, bytes - static_cast<size_t>(t) * kTransfer); }
-  int pieces_of(int t) const { return std::min(kPerTransfer, pieces - t * kPerTransfer); }
-  bool is_copied(int t) const { return copied[t % kSlots].load(std::memory_order_acquire) == pieces_of(t); }
-  char* slot(int t) const { return slots + static_cast<size_t>(t % kSlots) * kTransfer; }
+  size_t transfer_bytes(int t) const { return std::min(transfer, bytes - static_cast<size_t>(t) * transfer); }
+  int pieces_of(int t) const { return std::min(per_transfer, pieces - t * per_transfer); }
+  bool is_copied(int t) const { return copied[t % ring].load(std::memory_order_acquire) == pieces_of(t); }
+  char* slot(int t) const { return slots + static_cast<size_t>(t % ring) * transfer; }
   // Claims and copies one piece; false: none is open.
   bool help() {
     int i = next.load(std::memory_order_relaxed);
     do {
       if (i >= open.load(std::memory_order_acquire) || i >= pieces) return false;
     } while (!next.compare_exchange_weak(i, i + 1, std::memory_order_acq_rel));
-    const int t = i / kPerTransfer;
-    char* const there = slot(t) + static_cast<size_t>(i % kPerTransfer) * kPiece;
+    const int t = i / per_transfer;
+    char* const there = slot(t) + static_cast<size_t>(i % per_transfer) * kPiece;
     char* const mine = host + static_cast<size_t>(i) * kPiece;
     const size_t size = std::min(kPiece, bytes - static_cast<size_t>(i) * kPiece);
     if (to_device) std::memcpy(there, mine, size);
     else std::memcpy(mine, there, size);
-    copied[t % kSlots].fetch_add(1, std::memory_order_acq_rel);
+    copied[t % ring].fetch_add(1, std::memory_order_acq_rel);
     finished.fetch_add(1, std::memory_order_acq_rel);
     return true;
   }
@@ -95,15 +98,17 @@ class Copier {
     std::unique_lock<std::mutex> mine(busy_, std::try_to_lock);
     if (!mine.owns_lock() || !ready()) return false;
     job_.host = static_cast<char*>(host); job_.bytes = bytes; job_.to_device = to_device;
+    const int wide = bytes > kLanesAbove ? 1 : kLanes;   // (as many bytes in the ring)
+    job_.transfer = wide * kTransfer; job_.ring = kSlots / wide; job_.per_transfer = static_cast<int>(job_.transfer / kPiece);
     job_.pieces = static_cast<int>((bytes + kPiece - 1) / kPiece);
-    job_.transfers = static_cast<int>((bytes + kTransfer - 1) / kTransfer);
+    job_.transfers = static_cast<int>((bytes + job_.transfer - 1) / job_.transfer);
     job_.slots = slots_;
     for (auto& c : job_.copied) c.store(0, std::memory_order_relaxed);
     for (int k = 0; k < kSlots; ++k)   // slots that a previous copy to the device still reads
       if (pending_[k]) { MOBULA_HIP_TRY(hipEventSynchronize(events_[k])); pending_[k] = false; }
     if (failed()) return true;
     job_.next.store(0); job_.finished.store(0);
-    job_.open.store(to_device ? std::min(kSlots * kPerTransfer, job_.pieces) : 0);
+    job_.open.store(to_device ? std::min(job_.ring * job_.per_transfer, job_.pieces) : 0);
     wake();
     if (to_device) send(static_cast<char*>(dev), stream);
     else receive(static_cast<const char*>(dev), stream);
@@ -232,9 +237,11 @@ class Copier {
     }
   }
 
+  bool in_lanes() const { return job_.transfer == kTransfer; }
   // The lanes follow what the caller's stream has been given: it may use the memory that a transfer writes, or
   // write what one reads.
   void follow(hipStream_t stream) {
+    if (!in_lanes()) return;
     MOBULA_HIP_TRY(hipEventRecord(ordered_, stream));
     for (const hipStream_t lane : lanes_)
       if (!failed()) MOBULA_HIP_TRY(hipStreamWaitEvent(lane, ordered_, 0));
@@ -245,29 +252,29 @@ class Copier {
     follow(stream);
     while (issued < job_.transfers && !failed()) {
       bool moved = false;
-      if (issued < sent + kSlots && job_.is_copied(issued)) {   // (beyond: the slot still counts the round before)
-        const hipStream_t lane = lanes_[issued % kLanes];
-        MOBULA_HIP_TRY(hipMemcpyAsync(dev + static_cast<size_t>(issued) * kTransfer, job_.slot(issued),
+      if (issued < sent + job_.ring && job_.is_copied(issued)) {   // (beyond: the slot still counts the round before)
+        const hipStream_t lane = in_lanes() ? lanes_[issued % kLanes] : stream;
+        MOBULA_HIP_TRY(hipMemcpyAsync(dev + static_cast<size_t>(issued) * job_.transfer, job_.slot(issued),
                                       job_.transfer_bytes(issued), hipMemcpyHostToDevice, lane));
-        MOBULA_HIP_TRY(hipEventRecord(events_[issued % kSlots], lane));
-        pending_[issued % kSlots] = true;
+        MOBULA_HIP_TRY(hipEventRecord(events_[issued % job_.ring], lane));
+        pending_[issued % job_.ring] = true;
         ++issued;
         moved = true;
       }
       // a slot whose transfer has ended is free for the transfer a round later
-      if (sent < issued && sent + kSlots < job_.transfers && hipEventQuery(events_[sent % kSlots]) == hipSuccess) {
-        job_.copied[sent % kSlots].store(0, std::memory_order_relaxed);
+      if (sent < issued && sent + job_.ring < job_.transfers && hipEventQuery(events_[sent % job_.ring]) == hipSuccess) {
+        job_.copied[sent % job_.ring].store(0, std::memory_order_relaxed);
         ++sent;
-        job_.open.store(std::min(job_.pieces, (sent + kSlots) * kPerTransfer), std::memory_order_release);
+        job_.open.store(std::min(job_.pieces, (sent + job_.ring) * job_.per_transfer), std::memory_order_release);
         moved = true;
       }
       if (!moved && !job_.help()) relax();
     }
     if (failed()) finish_claimed();
     // the caller's stream goes on when the last transfer of every lane has ended
-    for (int t = std::max(0, issued - kLanes); t < issued && !failed(); ++t)
-      MOBULA_HIP_TRY(hipStreamWaitEvent(stream, events_[t % kSlots], 0));
-    if (failed()) wait_for_lanes();
+    for (int t = std::max(0, issued - kLanes); t < issued && in_lanes() && !failed(); ++t)
+      MOBULA_HIP_TRY(hipStreamWaitEvent(stream, events_[t % job_.ring], 0));
+    if (failed()) wait_for_lanes(stream);
   }
 
   void receive(const char* dev, hipStream_t stream) {
@@ -275,20 +282,20 @@ class Copier {
     follow(stream);
     while (job_.finished.load(std::memory_order_acquire) < job_.pieces && !failed()) {
       bool moved = false;
-      if (issued < job_.transfers && (issued < kSlots || job_.is_copied(issued - kSlots))) {
-        if (issued >= kSlots) job_.copied[issued % kSlots].store(0, std::memory_order_relaxed);
-        const hipStream_t lane = lanes_[issued % kLanes];
-        MOBULA_HIP_TRY(hipMemcpyAsync(job_.slot(issued), dev + static_cast<size_t>(issued) * kTransfer,
+      if (issued < job_.transfers && (issued < job_.ring || job_.is_copied(issued - job_.ring))) {
+        if (issued >= job_.ring) job_.copied[issued % job_.ring].store(0, std::memory_order_relaxed);
+        const hipStream_t lane = in_lanes() ? lanes_[issued % kLanes] : stream;
+        MOBULA_HIP_TRY(hipMemcpyAsync(job_.slot(issued), dev + static_cast<size_t>(issued) * job_.transfer,
                                       job_.transfer_bytes(issued), hipMemcpyDeviceToHost, lane));
-        MOBULA_HIP_TRY(hipEventRecord(events_[issued % kSlots], lane));
+        MOBULA_HIP_TRY(hipEventRecord(events_[issued % job_.ring], lane));
         ++issued;
         moved = true;
       }
       if (arrived < issued) {
-        const hipError_t state = hipEventQuery(events_[arrived % kSlots]);
+        const hipError_t state = hipEventQuery(events_[arrived % job_.ring]);
         if (state == hipSuccess) {
           ++arrived;
-          job_.open.store(std::min(job_.pieces, arrived * kPerTransfer), std::memory_order_release);
+          job_.open.store(std::min(job_.pieces, arrived * job_.per_transfer), std::memory_order_release);
           moved = true;
         } else if (state != hipErrorNotReady) {
           MOBULA_HIP_TRY(state);
@@ -297,11 +304,12 @@ class Copier {
       if (!moved && !job_.help()) relax();
     }
     if (failed()) {
-      wait_for_lanes();
+      wait_for_lanes(stream);
       finish_claimed();
     }
   }
-  void wait_for_lanes() {
+  void wait_for_lanes(hipStream_t stream) {
+    if (!in_lanes()) (void)hipStreamSynchronize(stream);
     for (const hipStream_t lane : lanes_) (void)hipStreamSynchronize(lane);
   }
   // After an error: nothing more is claimed, and what was claimed is finished.
