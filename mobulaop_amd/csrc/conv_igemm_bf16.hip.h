@@ -26,7 +26,7 @@
 // largest are kept apart (odd_values_kernel).
 // Sums of the heads' products start anew every sixteen K steps and are added up in fp32, so that a long sum is rounded at its
 // own size only once for 256 terms: 32 x 256 x 56 x 56, 256 filters 3 x 3: errors against 64 bits 2.85e-7 -> 1.43e-7 (weight
-// gradient 5.3 -> 1.7), products 500 -> 340 us each, forward and both gradients 1819 -> 1157.  The device's power bounds them
+// gradient 5.3 -> 1.7), products 500 -> 340 us each, forward and both gradients 1840 -> 1120.  The device's power bounds them
 // (265 us each for tensors of zeros; without any load 193, without LDS reads 250).
 //
 // The forward and the data gradient gather the right operand: K runs over the taps of a channel block,
@@ -166,7 +166,7 @@ struct TensorWords {
 };
 
 // The magnitudes of up to three tensors (blockIdx.y), and their words cleared.  Of large tensors one of every eight lines of
-// 128 bytes is looked at (103 MB: 28 us for all of them): values beyond the range that this gives are odd ones like those
+// 128 bytes is looked at (103 MB: 28 us for all of them, 6 for these): values beyond the range that this gives are odd ones like those
 // below it.
 constexpr long long kSampledElements = 1 << 20;
 struct MagnitudeJob { const float* src[3]; long long count[3]; TensorWords words[3]; };

@@ -1034,7 +1034,7 @@ bool gradients_b16(const conv::Geometry& g, const float* dy, const float* x, con
 // against 64 bits 8.5e-7 -> 2.9e-7 (8.7e-7 -> 5.3e-7 for the weights' gradient).  The fp32 kernels follow every such
 // product and return at once unless a tensor holds values the parts do not stand for (conv::SplitRange).
 //
-// Two fp16 parts (halves) take half the matrix instructions: forward and both gradients of that layer 1819 -> 1157 us, errors
+// Two fp16 parts (halves) take half the matrix instructions: forward and both gradients of that layer 1840 -> 1120 us, errors
 // 1.4e-7 and 1.7e-7, as their sums start anew every 256 terms.  Both parts hold values within some 2^26 of the tensor's
 // largest; up to 128 others are added behind the product in 64 bits (conv::odd_values_kernel: 5 us where there is none or one, and
 // forward and both gradients of that layer 1120 us -> 1190 with 100 of x's, 1160 of dy's, 1530 of the weights', which each reach

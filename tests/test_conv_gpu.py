@@ -1085,10 +1085,11 @@ def test_sums_that_three_parts_cut_shorter_are_left_to_them():
 
 
 def test_halves_in_a_recorded_graph(halves_always):
-    """What is known of the operands is found anew by every replay: halves, three parts, halves again."""
+    """What is known of the operands is found anew by every replay: halves, three parts, halves with a few listed values."""
     shape = (2, 64, 24, 28, 128, (3, 3), (1, 1), (1, 1), (1, 1))
     (x, w, dy), geo, _, _ = _layer(shape, 101)
-    usual, odd = x.clone(), x.clone()
+    usual, odd, few = x.clone(), x.clone(), x.clone()
+    few[1, 3, 7:9, 9] *= 2.0 ** -30
     odd[1, :, 7, 9] *= 2.0 ** -30
     odd[0, 5] *= 2.0 ** -30
     lib, stream = native.library(), torch.cuda.Stream()
@@ -1102,7 +1103,7 @@ def test_halves_in_a_recorded_graph(halves_always):
         native.end_call('conv2d')
     try:
         want = []
-        for values in usual, odd:
+        for values in usual, odd, few:
             x.copy_(values)
             call()
             torch.cuda.synchronize()
@@ -1110,8 +1111,8 @@ def test_halves_in_a_recorded_graph(halves_always):
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph, stream=stream):
             call(on=torch.cuda.current_stream().cuda_stream)
-        for which in (0, 1, 0, 0, 1):
-            x.copy_((usual, odd)[which])
+        for which in (0, 1, 2, 0, 0, 2, 1):
+            x.copy_((usual, odd, few)[which])
             for t in (y, dx, dw):
                 t.fill_(float('nan'))
             graph.replay()
