@@ -121,7 +121,7 @@ def cpu_baseline(w, budget_s=25.0, gpu_result=None):
             a, b = a.astype(np.float32), b.astype(np.float32)
             return float(np.abs(a - b).max() / max(float(np.abs(b).max()), 1e-30))
         y_gpu, dx_gpu = gpu_result(n)
-        if w['data'].dtype.itemsize == 2:   # 16-bit storage: the checker's result is rounded the same way
+        if w['data'].dtype.itemsize == 2:   # 16-bit storage: the oracle's result is rounded the same way
             y_cpu = y_cpu.astype(w['data'].dtype)
         out['gpu_vs_cpu'] = {'forward_max_rel': rel(y_gpu, y_cpu)}
         if dx_cpu is not None:

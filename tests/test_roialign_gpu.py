@@ -54,7 +54,7 @@ def test_golden_vectors(impl):
 @pytest.mark.skipif(not oracle.ref_available('serial'), reason='oracle/_ref is not built')
 def test_golden_inputs_against_the_compiled_reference():
     # the compiled reference kernels themselves (oracle/_ref, built in the development
-    # container from the reference's sources) as the checker, where they travelled along
+    # container from the reference's sources) as the oracle, where they travelled along
     for name in sorted(f for f in os.listdir(GOLDEN) if f.endswith('.npz')):
         z = np.load(os.path.join(GOLDEN, name))
         pooled = tuple(int(v) for v in z['pooled_size'])
@@ -163,7 +163,7 @@ def _round_bf16(a):
 @pytest.mark.parametrize('S', [2, 0])
 @pytest.mark.parametrize('C', [72, 64, 20])
 def test_bfloat16_storage(C, S):
-    """bfloat16 maps and gradients (fp32 boxes, fp32 arithmetic): the checker's fp32 result on
+    """bfloat16 maps and gradients (fp32 boxes, fp32 arithmetic): the oracle's fp32 result on
     the bfloat16-rounded operands, rounded to bfloat16.  NCHW and channels-last; C = 20 and the
     S = 0 backward go through the straightforward kernels."""
     abi.set_impl('auto')
@@ -211,7 +211,7 @@ def test_bfloat16_storage(C, S):
 @pytest.mark.parametrize('S', [2, 0])
 @pytest.mark.parametrize('C', [72, 20])
 def test_fp16_backward(C, S):
-    # fp16 gradients: the checker's fp32 result on the fp16-rounded dy, rounded to fp16;
+    # fp16 gradients: the oracle's fp32 result on the fp16-rounded dy, rounded to fp16;
     # S = 0 (and C = 20 in any case) goes through the straightforward kernel and an fp32 scratch map
     abi.set_impl('auto')
     rng = np.random.default_rng(300 * C + S)
