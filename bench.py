@@ -262,7 +262,7 @@ def short_conv_run(mode='fp32', steps=20, warmup=5):
             'frac': flops / (ms * 1e-3) / 1e12 / peak, 'bound': 'mfma ' + ('fp32' if mode == 'fp32' else 'bf16'),
             'tflops': flops / (ms * 1e-3) / 1e12,
             'parity_max_rel': parity,
-            # BASELINE.json asks for 1e-3 relative against the reference
+            # 1e-3 relative against the reference is asked for
             'within_1e-3': max(parity.values()) <= 1e-3,
             'parity_sample': 'first 2 images (outputs, data gradient) and the whole batch (weight gradient) '
                              'against torch conv2d on the CPU'}
@@ -612,7 +612,7 @@ def main():
             return y_n.cpu().numpy(), dx_n
         out['cpu_baseline'] = cpu_baseline(w, gpu_result=gpu_result)
     if args.workload == 'cfg2' and not args.no_other_configs and not nhwc and args.sampling_ratio is None:
-        # the other configurations of BASELINE.json, a few steps each (parity cases, shown
+        # the other configurations of the benchmark list, a few steps each (parity cases, shown
         # for orientation; `value` above is cfg2 alone)
         del x, dy, dx
         torch.cuda.empty_cache()

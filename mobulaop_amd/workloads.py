@@ -4,7 +4,7 @@ Each generator returns a dict with NumPy arrays `data` (NCHW), `rois`
 ([R,5] rows `[batch_idx, x1, y1, x2, y2]` in image pixels, always fp32), `dy`
 (N(0,1), shape [R,C,PH,PW]) and the operator parameters `pooled_size`,
 `spatial_scale`, `sampling_ratio`.  `scale_down` shrinks channel and ROI counts
-(not the geometry) so the CPU oracle finishes quickly in tests.
+(not the geometry) so a computation on the CPU finishes quickly in tests.
 """
 import numpy as np
 
