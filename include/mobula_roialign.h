@@ -328,9 +328,11 @@ void mobula_hip_clear_error(void);
  * 1 or 4 fixes it; "roialign_row_quads": 1 (default) lets it write rows of maps
  * whose width is a multiple of four 16 bytes at a time, 0 element by element;
  * "roialign_few_boxes": 1 (default) lets a few boxes on a small map go back in
- * one launch where that is faster, 0 never, 2 wherever it can (64 boxes) --
- * all four for tests, the results do not depend on them beyond the order of
- * fp32 sums).  set returns 0, or -1 for an unknown name; get
+ * one launch where that is faster, 0 never, 2 wherever it can (64 boxes);
+ * "roialign_patch": 4 or 12 fixes the wavefronts that share a patch of the
+ * gradient where sampling grids have more than two points per bin and axis, and
+ * takes other grids that way too, 1 (default) chooses -- all five for tests, the
+ * results do not depend on them beyond the order of fp32 sums).  set returns 0, or -1 for an unknown name; get
  * returns -1 for a name never set. */
 int mobula_hip_set_option(const char* name, long long value);
 long long mobula_hip_get_option(const char* name);

@@ -18,8 +18,7 @@
 // a pair of lane groups are taken one after the other by both groups, one group
 // adding the low corners and the other the high ones -- an LDS instruction
 // costs the same with eight active lanes as with 64, so nobody sits out.
-// Sampling grids of more than two points per bin come as windows of merged
-// weights instead (WIN): up to seven consecutive cells per pooled column.
+// Sampling grids of more than two points per bin and axis: roialign_backward_patch.hip.h.
 //
 // dy is read from a channel-blocked copy dyb[C/32][R][PH][PW][32]: one 16-byte
 // load per lane fetches (eight pooled columns of) a pooled row, up to 1 KB; the
@@ -36,7 +35,7 @@ struct BwdBlocked {
   static constexpr int TH = 1;           // rows of a band = wavefronts of a workgroup
   static constexpr int BANDS = kTileRows / TH;   // bands per tile
   static constexpr int TW = 64;          // tile columns at most (see backward_tile_columns)
-  static constexpr int TW_LEAST = 16;    // (a window of merged weights and the dummies lie inside a row)
+  static constexpr int TW_LEAST = 16;
   static constexpr int CB = 32;          // channels per workgroup
   static constexpr int NW = TH;
   static constexpr int NT = NW * 64;
@@ -61,12 +60,10 @@ inline bool backward_few_tiles(long long images, int H, int W, int cblk) {
 // rows' wavefronts like any other (tile owners, us: 4000 boxes on 4 x 256 x 200 x 320, 56 columns 208, 64: 184; 512 on
 // 2 x 256 x 64 x 64, 28: 42, 32: 38, 64: 34; 4000 on 4 x 256 x 100 x 100, 28: 237, 52: 169; 2000 on 8 x 64 x 40 x 120, 28: 42, 60: 31).
 // Narrower ones down to 32 columns where those give the device fewer wavefronts than it holds (300 boxes on 1 x 256 x 50 x
-// 84, 44: 24, 28: 23, 32: 21).  Windows of merged weights, whose rows are not split: 28 columns where tiles are few (301 boxes on
-// 3 x 81 x 75 x 113: 42; 32: 48; 64: 50), else up to 56 (1500 on 2 x 128 x 256 x 256: 52: 72, 56 and 64: 75).
-inline int backward_tile_columns(long long images, int H, int W, int cblk, bool windows) {
+// 84, 44: 24, 28: 23, 32: 21).
+inline int backward_tile_columns(long long images, int H, int W, int cblk) {
   const bool few = backward_few_tiles(images, H, W, cblk);
-  if (windows && few) return 28;
-  const int most = windows ? 56 : BwdBlocked::TW;
+  const int most = BwdBlocked::TW;
   auto width = [&](int tiles) { return std::max(BwdBlocked::TW_LEAST, ((W + tiles - 1) / tiles + 3) / 4 * 4); };
   const long long rows = images * ((H + kTileRows - 1) / kTileRows) * kTileRows * cblk;
   int tiles = (W + most - 1) / most;
@@ -172,10 +169,8 @@ template <typename T>
 __global__ void __launch_bounds__(256)
 lists_and_dy_kernel(ListsArgs lists, unsigned list_blocks, const T* __restrict__ dy, T* __restrict__ dyb,
                     int cblk, int per, int C) {
-  if (blockIdx.x < list_blocks) {
-    if (lists.window_offsets != nullptr) build_window_lists_body(blockIdx.x, lists);
-    else build_lists_body(blockIdx.x, lists);
-  }
+  if (blockIdx.x < list_blocks)
+    build_lists_body(blockIdx.x, lists);
   else
     transpose_dy_blocked_body<T>(blockIdx.x - list_blocks, dy, dyb, C, lists.PH, lists.PW, cblk, per, lists.R, 0);
 }
@@ -209,13 +204,11 @@ __device__ __forceinline__ float lane_value(const unsigned __attribute__((ext_ve
 // a contiguous part of the row's work list (whole items: an item belongs to the part its first
 // entry lies in) into a row of its own in LDS, and the parts are added in part order on the
 // way out -- for maps that give the SIMDs too few tile rows to keep them busy.
-// WIN: the list items are windows of merged column weights (sampling grids of more than two
-// points per bin and axis) instead of pairs of sample columns.
 // dy_any: the blocked copy dyb, or for channels-last tensors the caller's dy[R][PH][PW][C] itself; of
 // dx's element type.
 // Dynamic LDS: backward_blocked_lds(tg.tw, NSPLIT) bytes.
 inline size_t backward_blocked_lds(int tw, int nsplit) { return sizeof(float) * nsplit * (tw + 2) * BwdBlocked::CS; }
-template <bool NHWC, typename TO, int NSPLIT = 1, bool WIN = false>
+template <bool NHWC, typename TO, int NSPLIT = 1>
 __global__ void __launch_bounds__(BwdBlocked::NT * NSPLIT)
 backward_blocked_kernel(const void* __restrict__ dy_any, TO* __restrict__ dx_any,
                         const WorkRange* __restrict__ ranges, const SortedRow* __restrict__ sorted,
@@ -301,8 +294,6 @@ backward_blocked_kernel(const void* __restrict__ dy_any, TO* __restrict__ dx_any
       const_cast<AxisUnit*>(lists), 0, static_cast<int>(list_bytes), 0x00020000);
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
   typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-  // what a lane holds of an item's column list: one dword of a ColPair, or two of a ColWindow
-  typedef typename std::conditional<WIN, u32x2, unsigned>::type UT;
 
   // Each wavefront streams through the work list of its tile row: entries
   // (ROI, pooled row, weight) in ROI order, four at a time, double buffered:
@@ -313,30 +304,25 @@ backward_blocked_kernel(const void* __restrict__ dy_any, TO* __restrict__ dx_any
     const unsigned dy_fixed = (NHWC ? cb * K::CB * E : 0u) + pwb * dy_pw;
     const unsigned list_fixed = static_cast<unsigned>(
         (static_cast<long long>(ll.ty) * ll.row_stride + static_cast<long long>(tx) * ll.col_stride +
-         pwb * (WIN ? 2 : 1)) * sizeof(AxisUnit));
+         pwb) * sizeof(AxisUnit));
     // a lane whose pooled column or channels do not exist loads from outside the buffer (zero, no access)
     const int dy_lane = pwb + grp < PW && quad * 4 < nch ? static_cast<int>(grp * dy_pw + quad * 4 * E)
                                                          : static_cast<int>(0x80000000u);
     // The 16-byte column sample of the lane's pooled column comes as one dword per
     // lane (lane & 3 picks it; a 4-byte load costs the texture path half of a
     // 16-byte one) and is spread over the quad with DPP moves where it is used.
-    // (The 32-byte window of merged weights: two dwords per lane.)
-    const int list_lane = WIN ? grp * 32 + (lane & 3) * 8 : grp * 16 + (lane & 3) * 4;
-    auto issue = [&](const int16v& e, u32x4 (&d)[K::G], UT (&u)[K::G]) {
+    const int list_lane = grp * 16 + (lane & 3) * 4;
+    auto issue = [&](const int16v& e, u32x4 (&d)[K::G], unsigned (&u)[K::G]) {
 #pragma unroll
       for (int j = 0; j < K::G; ++j) {
-        // the item's lists, the dy of the ROI it belongs to
-        const unsigned roi = e[4 * j], ph = e[4 * j + 1], owner = static_cast<unsigned>(e[4 * j + 3]) >> 2;
+        const unsigned roi = e[4 * j], ph = e[4 * j + 1];
         if (E == 4) {
-          d[j] = __builtin_amdgcn_raw_buffer_load_b128(dy_buf, dy_lane, owner * dy_roi + ph * dy_ph + dy_fixed, 0);
+          d[j] = __builtin_amdgcn_raw_buffer_load_b128(dy_buf, dy_lane, roi * dy_roi + ph * dy_ph + dy_fixed, 0);
         } else {   // four 16-bit values: eight bytes
-          const u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(dy_buf, dy_lane, owner * dy_roi + ph * dy_ph + dy_fixed, 0);
+          const u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(dy_buf, dy_lane, roi * dy_roi + ph * dy_ph + dy_fixed, 0);
           d[j] = u32x4{w.x, w.y, 0u, 0u};
         }
-        if constexpr (WIN)
-          u[j] = __builtin_amdgcn_raw_buffer_load_b64(list_buf, list_lane, roi * list_roi + list_fixed, 0);
-        else
-          u[j] = __builtin_amdgcn_raw_buffer_load_b32(list_buf, list_lane, roi * list_roi + list_fixed, 0);
+        u[j] = __builtin_amdgcn_raw_buffer_load_b32(list_buf, list_lane, roi * list_roi + list_fixed, 0);
       }
     };
     float g[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -353,21 +339,7 @@ backward_blocked_kernel(const void* __restrict__ dy_any, TO* __restrict__ dx_any
       *reinterpret_cast<float4*>(a + K::CS) = hi;
     };
     bool mine = NSPLIT == 1, done = false;   // (uniform) inside an item of this part; past the part's last item
-    // adds g * w[i] to the cells a, a + 1, ... of the row (N of them; all reads before the first write)
-    auto add_cells = [&](float* a, const float* w, auto count) {
-      constexpr int N = decltype(count)::value;
-      float4 v[N];
-#pragma unroll
-      for (int i = 0; i < N; ++i) v[i] = *reinterpret_cast<const float4*>(a + i * K::CS);
-#pragma unroll
-      for (int i = 0; i < N; ++i) {
-        v[i].x = fmaf(g[0], w[i], v[i].x); v[i].y = fmaf(g[1], w[i], v[i].y);
-        v[i].z = fmaf(g[2], w[i], v[i].z); v[i].w = fmaf(g[3], w[i], v[i].w);
-      }
-#pragma unroll
-      for (int i = 0; i < N; ++i) *reinterpret_cast<float4*>(a + i * K::CS) = v[i];
-    };
-    auto process = [&](const int16v& e, const u32x4 (&d)[K::G], const UT (&u)[K::G], int at) {
+    auto process = [&](const int16v& e, const u32x4 (&d)[K::G], const unsigned (&u)[K::G], int at) {
 #pragma unroll
       for (int j = 0; j < K::G; ++j) {
         const float wy = __int_as_float(e[4 * j + 2]);
@@ -386,89 +358,7 @@ backward_blocked_kernel(const void* __restrict__ dy_any, TO* __restrict__ dx_any
 #pragma unroll
           for (int i = 0; i < 4; ++i) g[i] = lane_value<TI>(d[j], i) * wy;
         }
-        if constexpr (WIN) {
-          if ((fl & 2) != 0) {
-            // last tap of this item on this row: g times the weights of the window's cells.
-            // The lanes lane & 3 = k of a quad hold dwords 2k and 2k + 1 of the window:
-            // quad_perm [k, k, k, k] hands them to everyone
-            const int ulo = static_cast<int>(u[j][0]), uhi = static_cast<int>(u[j][1]);
-            const int header = __builtin_amdgcn_mov_dpp(ulo, 0x00, 0xf, 0xf, true);
-            const float w[kWindowCells] = {
-                __int_as_float(__builtin_amdgcn_mov_dpp(uhi, 0x00, 0xf, 0xf, true)),
-                __int_as_float(__builtin_amdgcn_mov_dpp(ulo, 0x55, 0xf, 0xf, true)),
-                __int_as_float(__builtin_amdgcn_mov_dpp(uhi, 0x55, 0xf, 0xf, true)),
-                __int_as_float(__builtin_amdgcn_mov_dpp(ulo, 0xaa, 0xf, 0xf, true)),
-                __int_as_float(__builtin_amdgcn_mov_dpp(uhi, 0xaa, 0xf, 0xf, true)),
-                __int_as_float(__builtin_amdgcn_mov_dpp(ulo, 0xff, 0xf, 0xf, true)),
-                __int_as_float(__builtin_amdgcn_mov_dpp(uhi, 0xff, 0xf, 0xf, true))};
-            float* const a = cell0 + (header & 0xffff) * K::CS;
-            const int turns = 1 << ((__builtin_amdgcn_readfirstlane(header) >> 16) & 3);
-            // (the eight lanes of a pooled column decide alike: a window that ends early costs the LDS nothing)
-            auto add_window = [&] {
-              if (w[0] != 0.0f || w[1] != 0.0f || w[2] != 0.0f || w[3] != 0.0f)
-                add_cells(a, w, std::integral_constant<int, 4>());
-              if (w[4] != 0.0f || w[5] != 0.0f || w[6] != 0.0f)
-                add_cells(a + 4 * K::CS, w + 4, std::integral_constant<int, 3>());
-            };
-            if (turns == 1) {
-              add_window();
-            } else {
-              // Neighbouring windows overlap.  An LDS instruction costs the same with few lanes as
-              // with all, so the two windows of a pair of lane groups (a row of 16 lanes) are taken
-              // one after the other by both groups together: one group adds the even cells, the
-              // other the odd ones (the gradient and the window of the other group: its lanes,
-              // eight further).
-              const int which = grp & 1, pair = grp >> 1, rounds = turns >> 1;
-              const int ulo_x = __builtin_amdgcn_mov_dpp(ulo, 0x128, 0xf, 0xf, true);   // row_ror:8
-              const int uhi_x = __builtin_amdgcn_mov_dpp(uhi, 0x128, 0xf, 0xf, true);
-              float gx[4];
-#pragma unroll
-              for (int i = 0; i < 4; ++i)
-                gx[i] = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(g[i]), 0x128, 0xf, 0xf, true));
-#pragma unroll
-              for (int t = 0; t < 2; ++t) {   // the pair's first window, then its second
-                const bool own = which == t;
-                const int vlo = own ? ulo : ulo_x, vhi = own ? uhi : uhi_x;
-                const float gg[4] = {own ? g[0] : gx[0], own ? g[1] : gx[1], own ? g[2] : gx[2], own ? g[3] : gx[3]};
-                const int hd = __builtin_amdgcn_mov_dpp(vlo, 0x00, 0xf, 0xf, true);
-                const float x0 = __int_as_float(__builtin_amdgcn_mov_dpp(vhi, 0x00, 0xf, 0xf, true));
-                const float x1 = __int_as_float(__builtin_amdgcn_mov_dpp(vlo, 0x55, 0xf, 0xf, true));
-                const float x2 = __int_as_float(__builtin_amdgcn_mov_dpp(vhi, 0x55, 0xf, 0xf, true));
-                const float x3 = __int_as_float(__builtin_amdgcn_mov_dpp(vlo, 0xaa, 0xf, 0xf, true));
-                const float x4 = __int_as_float(__builtin_amdgcn_mov_dpp(vhi, 0xaa, 0xf, 0xf, true));
-                const float x5 = __int_as_float(__builtin_amdgcn_mov_dpp(vlo, 0xff, 0xf, 0xf, true));
-                const float x6 = __int_as_float(__builtin_amdgcn_mov_dpp(vhi, 0xff, 0xf, 0xf, true));
-                const bool head = x0 != 0.0f || x1 != 0.0f || x2 != 0.0f || x3 != 0.0f;
-                const bool tail = x4 != 0.0f || x5 != 0.0f || x6 != 0.0f;
-                // this lane's cells: which, which + 2 of w[0..3]; 4 + which (and 6) of w[4..6]
-                float* const b = cell0 + ((hd & 0xffff) + which) * K::CS;
-                const float wa = which ? x1 : x0, wb = which ? x3 : x2, wc = which ? x5 : x4;
-                auto fold = [&](float4& v, float w) {
-                  v.x = fmaf(gg[0], w, v.x); v.y = fmaf(gg[1], w, v.y);
-                  v.z = fmaf(gg[2], w, v.z); v.w = fmaf(gg[3], w, v.w);
-                };
-                for (int r = 0; r < rounds; ++r)
-                  if ((pair & (rounds - 1)) == r) {
-                    if (head) {
-                      float4 va = *reinterpret_cast<const float4*>(b);
-                      float4 vb = *reinterpret_cast<const float4*>(b + 2 * K::CS);
-                      fold(va, wa); fold(vb, wb);
-                      *reinterpret_cast<float4*>(b) = va;
-                      *reinterpret_cast<float4*>(b + 2 * K::CS) = vb;
-                    }
-                    if (tail) {
-                      float4 vc = *reinterpret_cast<const float4*>(b + 4 * K::CS);
-                      float4 vd = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                      if (which == 0) vd = *reinterpret_cast<const float4*>(b + 6 * K::CS);
-                      fold(vc, wc); fold(vd, x6);
-                      *reinterpret_cast<float4*>(b + 4 * K::CS) = vc;
-                      if (which == 0) *reinterpret_cast<float4*>(b + 6 * K::CS) = vd;
-                    }
-                  }
-              }
-            }
-          }
-        } else if ((fl & 2) != 0) {
+        if ((fl & 2) != 0) {
           // last tap of this ROI on this row: spread g over the column samples
           // dword k of the quad's four: quad_perm [k, k, k, k]
           const int uj = static_cast<int>(u[j]);
@@ -543,7 +433,7 @@ backward_blocked_kernel(const void* __restrict__ dy_any, TO* __restrict__ dx_any
       const int w0 = first_entry >> 2;
       int16v e_cur = wl[w0], e_nx = wl[w0 + 1], e_n2;
       u32x4 d_a[K::G], d_b[K::G];
-      UT u_a[K::G], u_b[K::G];
+      unsigned u_a[K::G], u_b[K::G];
       issue(e_cur, d_a, u_a);
       // (a part goes on past its end until the item it is in has ended: to the next item start)
       for (int e0 = first_entry; e0 < n_entries && !done; e0 += 2 * K::G) {

@@ -23,7 +23,7 @@ struct BwdFew {
   // through the operator, us, lists and tile owners / this; 7 x 7 pooled: 1 x 64 x 32 x 32, 4 to 32 boxes 48 / 42, 64:
   // 48 / 51; 1 x 256 x 50 x 84, 16 boxes 49 / 44, 32: 49 / 57; 2 x 256 x 64 x 64, 8 boxes 34 / 28, 16: 33 / 37; 1 x 256 x 100 x 168,
   // 4 boxes 35 / 35, 8: 39 / 45.  14 x 14: 1 x 256 x 32 x 32, 8 boxes 51 / 45, 16: 51 / 65.  28 x 28, 4 boxes: 53 / 73.
-  // Channels last 48 / 42.  Three points per bin and axis, whose lists are windows of merged weights that the host waits for: 61 / 43.
+  // Channels last 48 / 42.
   static constexpr long long kMostBins = 1600, kMostLooks = 1670000, kMostSteps = 29400000;
 };
 inline long long backward_few_blocks(long long N, int C, long long H, long long W) {

@@ -56,6 +56,9 @@ __device__ __forceinline__ float sample_coord(float start, int p, float bin, int
 // than the map, or infinite, whose adaptive grid has up to 2^31 points per bin
 // of which only about `size` can be valid.
 constexpr int kSearchedGrid = 64;
+// Points per bin and axis up to which a grid's samples are numbered from coordinates, or merged a window at a time: beyond,
+// fp32 coordinates of neighbouring samples coincide.
+constexpr int kMergedGrid = 1 << 15;
 
 __device__ __forceinline__ void valid_sample_range(float start, int p, float bin, int grid, int size,
                                                    int* first, int* last) {

@@ -23,17 +23,8 @@
 //                           by tile row, then by sample order
 //   col list  of (roi, tx): one 16-byte ColPair per pooled column (padded to a
 //                           multiple of 8 columns): its one or two sample columns
-// These lists hold one or two sample points per bin and axis.  A larger sampling
-// grid (a ratio above 2, or the adaptive ceil(bin size)) is merged instead: the
-// gradient of a pixel is dy times (sum of the row weights its row gets from the
-// bin's sample rows) times (sum of the column weights its column gets from
-// the bin's sample columns), so a bin is described by one weight per row and one
-// per column it touches.  Rows become row taps as before (one per pooled row and
-// tile row, the weights of that pooled row's samples added up).  The columns of a
-// bin are cut into windows of kWindowCells cells, window j of every pooled column
-// together forming list item j of the ROI: its column list holds one 32-byte
-// ColWindow per pooled column, and the tile owners add the items up like so many
-// ROIs that share one dy.  `window_offsets_kernel` numbers the items.
+// These lists hold one or two sample points per bin and axis; larger sampling grids have weights
+// per cell instead (roialign_backward_patch.hip.h).
 // Sample coordinates come from roialign_geometry.h (reference operation order).
 #pragma once
 #include "roialign_tiles.hip.h"
@@ -77,199 +68,20 @@ struct ListLayout {
   int col_stride;        // 16-byte units per (item, tx) column list
   long long roi_stride;  // units per item: ty*row_stride + tx*col_stride
   int pw_padded;         // PW rounded up to 8: pooled columns of a column list
-  int windows;           // 1: merged weights (WindowRowTable, ColWindow), 0: sample lists (RowTapTable, ColPair)
 };
-
-constexpr int kWindowCells = 7;   // cells of a column window (with its header: eight dwords)
-
-inline bool lists_in_windows(int S) { return S != 1 && S != 2; }
 
 inline ListLayout make_list_layout(const TileGrid& tg, int PH, int PW, int S) {
   ListLayout l;
   l.ty = tg.ty; l.tx = tg.tx;
   l.pw_padded = (PW + 7) / 8 * 8;
-  l.windows = lists_in_windows(S) ? 1 : 0;
-  if (l.windows) {
-    l.row_stride = 4 + kTileRows * PH / 2 + 1;   // 64-byte index, then at most one tap per tile row and pooled row
-    l.col_stride = 2 * l.pw_padded;
-  } else {
-    l.row_stride = row_table_units(PH * (S == 1 ? 1 : 2));
-    l.col_stride = l.pw_padded;
-  }
+  l.row_stride = row_table_units(PH * (S == 1 ? 1 : 2));
+  l.col_stride = l.pw_padded;
   l.roi_stride = static_cast<long long>(l.ty) * l.row_stride + static_cast<long long>(l.tx) * l.col_stride;
   return l;
 }
 
 inline bool lists_supported(int PH, int PW, int S) {
   return PH * (S == 1 ? 1 : 2) <= kRowSlots && PW <= kMaxListPW;
-}
-
-// ---- merged weights (sampling grids of more than two points per bin and axis) ----
-
-// Grids up to this many points per axis are merged (sample numbers are found from
-// coordinates in fp32: beyond this the search margin of one sample would not do).
-constexpr int kMergedGrid = 1 << 15;
-
-// The cells the samples of pooled index p can touch along one axis, [*low, *low + *span):
-// a superset, found from the first and the last sample coordinate alone (coordinates never
-// decrease with the sample number), clamped the way the interpolation clamps them
-// (opzoo/ROIAlign/bilinear.h:15-40).
-__device__ __forceinline__ void bin_cells(float start, int p, float bin, int grid, int size, int* low,
-                                          int* span) {
-  const float c0 = sample_coord(start, p, bin, 0, grid), c1 = sample_coord(start, p, bin, grid - 1, grid);
-  *low = 0; *span = 0;
-  if (c1 < -1.0f || c0 > static_cast<float>(size)) return;   // every sample lies outside [-1, size]
-  // (a coordinate that is not a number passes the reference's test; fmaxf/fminf then give the bound)
-  const AxisSample a = axis_sample(fmaxf(c0, -1.0f), size), b = axis_sample(fminf(c1, static_cast<float>(size)), size);
-  *low = a.low;
-  *span = max(b.high - a.low + 1, 1);
-}
-
-// Sum of the weights that the valid samples of pooled index p give to `cell`
-// (samples in sample order; a sample whose two cells coincide at the border counts once).
-__device__ __forceinline__ float merged_weight(float start, int p, float bin, int grid, int size, int cell) {
-  // samples that can reach the cell have coordinates in (cell - 1, cell + 1); the border
-  // cells also take what is clamped onto them.  Sample numbers from coordinates, one to
-  // spare on either side; every candidate is then evaluated exactly.
-  const float lo = cell == 0 ? -1.0f : static_cast<float>(cell - 1);
-  const float hi = cell == size - 1 ? static_cast<float>(size) : static_cast<float>(cell + 1);
-  const float origin = start + static_cast<float>(p) * bin, step = bin / static_cast<float>(grid);
-  const float fa = (lo - origin) / step - 0.5f, fb = (hi - origin) / step - 0.5f;
-  int first = 0, last = grid;
-  if (fabsf(fa) < 1.0e9f && fabsf(fb) < 1.0e9f) {   // (false for coordinates that are not numbers)
-    first = max(0, static_cast<int>(floorf(fa)) - 1);
-    last = min(grid, static_cast<int>(ceilf(fb)) + 2);
-  }
-  float w = 0.0f;
-  for (int i = first; i < last; ++i) {
-    const AxisSample a = axis_sample(sample_coord(start, p, bin, i, grid), size);
-    if (!a.valid) continue;
-    if (a.low == cell) w += a.h;
-    if (a.high == cell && a.high != a.low) w += a.l;
-  }
-  return w;
-}
-
-// What the window items of one ROI need: their number (windows per pooled column), the
-// tile columns they span and an upper bound of the row taps of one of them.
-struct WindowCount { int windows; int tiles_x; int taps; };
-__device__ __forceinline__ WindowCount count_windows(const RoiGeom& g, int PH, int PW, int H, int W, int tw) {
-  WindowCount c{0, 0, 0};
-  int widest = 0, clo = W, chi = -1;
-  for (int pw = 0; pw < PW; ++pw) {
-    int low, span;
-    bin_cells(g.start_w, pw, g.bin_w, g.grid_w, W, &low, &span);
-    if (span > 0) { widest = max(widest, span); clo = min(clo, low); chi = max(chi, low + span - 1); }
-  }
-  for (int ph = 0; ph < PH; ++ph) {
-    int low, span;
-    bin_cells(g.start_h, ph, g.bin_h, g.grid_h, H, &low, &span);
-    c.taps += span;
-  }
-  if (widest == 0 || c.taps == 0) return WindowCount{0, 0, 0};
-  c.windows = (widest + kWindowCells - 1) / kWindowCells;
-  c.tiles_x = chi / tw - clo / tw + 1;
-  return c;
-}
-
-// Windows of ROI r (-1: its grid has more than kMergedGrid points along an axis) and an upper
-// bound of the work entries of its items.
-__device__ __forceinline__ int windows_of_roi(const float* __restrict__ rois, long long r, float scale, int PH, int PW,
-                                              int S, int H, int W, int tw, long long* work) {
-  const RoiGeom g = roi_geometry(rois + r * 5, scale, PH, PW, S);
-  *work = 0;
-  if (g.grid_h > kMergedGrid || g.grid_w > kMergedGrid || g.grid_h < 1 || g.grid_w < 1) return -1;
-  const WindowCount c = count_windows(g, PH, PW, H, W, tw);
-  *work = static_cast<long long>(c.windows) * c.tiles_x * c.taps;
-  return c.windows;
-}
-
-struct WindowArgs { const float* rois; int R; float scale; int PH, PW, S, H, W, tw; };
-
-// Window items, step 1 (many ROIs): their counts and work bounds, one thread per ROI.
-__global__ void __launch_bounds__(256)
-window_counts_kernel(WindowArgs a, int* __restrict__ counts, long long* __restrict__ work) {
-  for (long long r = blockIdx.x * 256ll + threadIdx.x; r < a.R; r += 256ll * gridDim.x)
-    counts[r] = windows_of_roi(a.rois, r, a.scale, a.PH, a.PW, a.S, a.H, a.W, a.tw, &work[r]);
-}
-
-// Up to this many ROIs are counted by the workgroup that adds the counts up: one launch less.
-constexpr int kCountedInOffsets = 2048;
-
-// Step 2: offsets[r] = number of the first window item of ROI r, offsets[R] = their total;
-// told[0] = the total, told[1] = 1 if some ROI's grid is too large to merge (the caller then takes
-// another path), told[2] = an upper bound of the work entries of all items (saturating at 2^30),
-// told[3] = ticket, written last: `told` is pinned host memory that the calling thread watches.
-// One workgroup of 1024 threads; every thread reads its share of the counts before any writes
-// (offsets may be that array).
-__global__ void __launch_bounds__(1024)
-window_offsets_kernel(WindowArgs a, const int* __restrict__ counts, const long long* __restrict__ work,
-                      int* __restrict__ offsets, volatile int* told, int ticket) {
-  __shared__ int part[16];
-  __shared__ long long entries[16];
-  __shared__ int too_big;
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, share = (a.R + 1023) / 1024;
-  const int first = min(a.R, t * share), last = min(a.R, first + share);
-  const bool counted = a.R > kCountedInOffsets;
-  if (t == 0) too_big = 0;
-  __syncthreads();
-  int few[kCountedInOffsets / 1024];
-  int sum = 0;
-  long long all = 0;
-  auto take = [&](int c, long long w) {
-    if (c < 0) too_big = 1;
-    sum += max(c, 0);
-    all += w;
-  };
-  if (counted) {
-    for (int r = first; r < last; ++r) take(counts[r], work[r]);
-  } else {
-#pragma unroll
-    for (int k = 0; k < kCountedInOffsets / 1024; ++k) {
-      few[k] = 0;
-      if (first + k < last) {
-        long long w = 0;
-        few[k] = windows_of_roi(a.rois, first + k, a.scale, a.PH, a.PW, a.S, a.H, a.W, a.tw, &w);
-        take(few[k], w);
-      }
-    }
-  }
-  int upto = sum;   // inclusive sum over the wavefront's lanes
-  for (int off = 1; off < 64; off <<= 1) {
-    const int up = __shfl_up(upto, off);
-    if (lane >= off) upto += up;
-    all += __shfl_xor(all, off);
-  }
-  if (lane == 63) { part[wave] = upto; entries[wave] = all; }
-  __syncthreads();
-  int at = upto - sum;
-  for (int w = 0; w < wave; ++w) at += part[w];
-  if (counted) {
-    for (int r = first; r < last; ++r) {
-      const int c = max(counts[r], 0);
-      offsets[r] = at;
-      at += c;
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < kCountedInOffsets / 1024; ++k)
-      if (first + k < last) {
-        offsets[first + k] = at;
-        at += max(few[k], 0);
-      }
-  }
-  if (t == 1023) {
-    offsets[a.R] = at;
-    if (told != nullptr) {
-      long long total = 0;
-      for (int w = 0; w < 16; ++w) total += entries[w];
-      told[0] = at;
-      told[1] = too_big;
-      told[2] = static_cast<int>(min(total, 1ll << 30));
-      __threadfence_system();
-      told[3] = ticket;
-    }
-  }
 }
 
 __device__ __forceinline__ AxisUnit clip_unit(int bin, const AxisSample& a, int t0, int tsize,
@@ -291,7 +103,6 @@ __device__ __forceinline__ AxisUnit clip_unit(int bin, const AxisSample& a, int 
 // The wavefront also finds the ROI's box (the pixels any valid sample touches),
 // and stores it as tile ranges for build_tile_work_kernel.
 // `block`: index among the workgroups (of 256 threads) that build lists.
-constexpr long long kSharedItems = 4096;
 constexpr int kWorkClasses = 8;   // of tile rows by the length of their work lists (SortedRow)
 struct ListsArgs {
   const float* rois;
@@ -304,15 +115,8 @@ struct ListsArgs {
   TileBox* boxes;
   int* cursors;
   AxisUnit* lists;
-  const int* window_offsets;   // merged weights: the first item of every ROI (null: one item per ROI)
-  int parts_log;               // merged weights: log2 of the wavefronts that share an item's tiles (lists_parts_log)
 };
-// An item's tables are written tile row by tile row and tile column by tile column, for merged weights several hundred
-// dependent instructions each: with few items wavefronts deal the tiles of one out among them (301 boxes on 3 x 81 x 75 x 113,
-// adaptive grid: 21.6 -> 11.6 us with the search below).  Lists of samples are short beside what comes before their tiles
-// (512 boxes on 2 x 256 x 64 x 64: 12 us, 16 with four wavefronts to a box) and have one.
-inline int lists_parts_log(long long items) { return items <= kSharedItems / 4 ? 2 : items <= kSharedItems / 2 ? 1 : 0; }
-inline long long lists_blocks(long long items, int parts_log) { return std::max(1ll, ((items << parts_log) + 3) / 4); }
+inline long long lists_blocks(long long items) { return std::max(1ll, (items + 3) / 4); }
 
 __device__ __forceinline__ void build_lists_body(unsigned block, const ListsArgs& a) {
   const float* __restrict__ rois = a.rois;
@@ -449,158 +253,18 @@ __device__ __forceinline__ void build_lists_body(unsigned block, const ListsArgs
   }
 }
 
-// Merged weights.  Row taps of one (item, tile row): per tile row start | count << 16, then the
-// taps by tile row and pooled row: at most one per pair, ListLayout::row_stride leaves room for all.
-struct alignas(16) WindowRowTable {
-  unsigned index[kTileRows];
-  RowTap taps[kTileRows * 32];
-};
-// The cells of one window of one pooled column inside one tile column band.
-//   header  cell | turns_log << 16: `cell` is the cell of w[0] in a tile row whose cell 0 is a
-//           dummy to the left of the tile (so the tile's first column is cell 1); the window is
-//           shifted so that all seven cells lie in the tile, cells it does not reach weigh zero.
-//           turns_log: log2 of the smallest power-of-two distance (in pooled columns, at most 8)
-//           at which the windows of this item never share a cell their owner touches (w[0..3]
-//           are added together, and so are w[4..6]: a group is skipped if all of it is zero).
-//   w       weight of cells cell .. cell + 6
-struct alignas(32) ColWindow { int header; float w[kWindowCells]; };
-static_assert(sizeof(ColWindow) == 32, "eight dwords: the tile owners load one per lane");
-
-// One wavefront per window item (ROI, j): the row taps of every tile row the ROI
-// touches -- the same for all windows of a ROI -- and window j of every pooled column.
-__device__ __forceinline__ void build_window_lists_body(unsigned block, const ListsArgs& a) {
-  const int items = a.items, R = a.R, PH = a.PH, PW = a.PW, H = a.H, W = a.W;
-  const TileGrid tg = a.tg;
-  const ListLayout ll = a.ll;
-  if (block == 0 && threadIdx.x < 2 + kWorkClasses) a.cursors[threadIdx.x] = 0;
-  const int unit = static_cast<int>((block * 256u + threadIdx.x) >> 6), item = unit >> a.parts_log;
-  const int parts = 1 << a.parts_log, part = unit & (parts - 1);
-  if (item >= items) return;
-  const int lane = threadIdx.x & 63;
-  int roi;
-  {   // the ROI whose items include this one, among 64 of the rest at a time (every look is a round trip to memory)
-    int lo = 0, hi = R;
-    while (hi - lo > 1) {
-      const int step = (hi - lo + 63) / 64, at = lo + step * (lane + 1);
-      const int upto = __popcll(__ballot(at < hi && a.window_offsets[min(at, hi - 1)] <= item));
-      lo += step * upto;
-      hi = min(hi, lo + step);
-    }
-    roi = __builtin_amdgcn_readfirstlane(lo);
-  }
-  const int j = item - a.window_offsets[roi];
-  const RoiGeom g = roi_geometry(a.rois + static_cast<long long>(roi) * 5, a.scale, PH, PW, a.S_given);
-  // lane p < 32: pooled row p and pooled column p
-  int rlow = 0, rspan = 0, clow = 0, cspan = 0;
-  if (lane < PH) bin_cells(g.start_h, lane, g.bin_h, g.grid_h, H, &rlow, &rspan);
-  if (lane < PW) bin_cells(g.start_w, lane, g.bin_w, g.grid_w, W, &clow, &cspan);
-  const int wlow_mine = clow + kWindowCells * j;                    // first cell of the window
-  const int wn_mine = max(0, min(kWindowCells, cspan - kWindowCells * j));   // its cells
-  int row_lo, row_hi, col_lo, col_hi;
-  {
-    int rlo = rspan > 0 ? rlow : H, rhi = rspan > 0 ? rlow + rspan - 1 : -1;
-    int clo = wn_mine > 0 ? wlow_mine : W, chi = wn_mine > 0 ? wlow_mine + wn_mine - 1 : -1;
-    for (int off = 32; off > 0; off >>= 1) {
-      rlo = min(rlo, __shfl_xor(rlo, off)); rhi = max(rhi, __shfl_xor(rhi, off));
-      clo = min(clo, __shfl_xor(clo, off)); chi = max(chi, __shfl_xor(chi, off));
-    }
-    const bool image_ok = g.batch >= 0 && g.batch < a.num_images;
-    const bool any = image_ok && rlo <= rhi && clo <= chi;
-    row_lo = any ? rlo : 0; row_hi = any ? rhi : -1;
-    col_lo = any ? clo : 0; col_hi = any ? chi : -1;
-    const int ty0 = row_lo / tg.th, ty1 = any ? row_hi / tg.th : -1;
-    const int tx0 = col_lo / tg.tw, tx1 = any ? col_hi / tg.tw : -1;
-    if (lane == 0 && part == 0) a.boxes[item] = TileBox{any ? g.batch : -1, ty0 | (ty1 << 16), tx0 | (tx1 << 16), roi};
-    if (!any) return;
-  }
-  AxisUnit* const base = a.lists + static_cast<long long>(item) * ll.roi_stride;
-  const float inv_count = 1.0f / g.count;
-  {
-    // row taps: lane = tile row * 4 + k; the lane takes the pooled rows k, k + 4, ...
-    const int r = lane >> 2, k4 = lane & 3;
-    for (int ty = row_lo / tg.th + part; ty <= row_hi / tg.th; ty += parts) {
-      const int row = ty * tg.th + r;
-      WindowRowTable* const table = reinterpret_cast<WindowRowTable*>(base + ty * ll.row_stride);
-      float w[8];
-      int at[8];
-      int mine = 0;   // taps of this lane's tile row so far
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        w[q] = 0.0f; at[q] = 0;
-        if (4 * q < PH) {   // (the same for every lane)
-          const int ph = 4 * q + k4;
-          if (ph < PH && row < H)
-            w[q] = merged_weight(g.start_h, ph, g.bin_h, g.grid_h, H, row) * inv_count;
-          const unsigned nib = static_cast<unsigned>(__ballot(w[q] != 0.0f) >> (4 * r)) & 15u;
-          at[q] = mine + __popc(nib & ((1u << k4) - 1u));
-          mine += __popc(nib);
-        }
-      }
-      int start = 0;
-      for (int q = 0; q < kTileRows; ++q) {
-        const int t = __shfl(mine, 4 * q);
-        if (q < r) start += t;
-      }
-#pragma unroll
-      for (int q = 0; q < 8; ++q)
-        if (w[q] != 0.0f) table->taps[start + at[q]] = RowTap{4 * q + k4, w[q]};
-      if (k4 == 0) table->index[r] = static_cast<unsigned>(start) | (static_cast<unsigned>(mine) << 16);
-    }
-  }
-  {
-    // windows: lane = pooled column (of eight) * 8 + dword of its ColWindow
-    const int sub = lane >> 3, slot = (lane & 7) - 1;   // slot -1: the header
-    int* const cols = reinterpret_cast<int*>(base + static_cast<long long>(ll.ty) * ll.row_stride);
-    for (int tx = col_lo / tg.tw + part; tx <= col_hi / tg.tw; tx += parts) {
-      for (int pw0 = 0; pw0 < ll.pw_padded; pw0 += 8) {
-        const int pw = pw0 + sub;
-        // (every lane takes part in the exchange: the lane asked may be one whose column does not exist)
-        const int wlow = __shfl(wlow_mine, pw & 63), wn_any = __shfl(wn_mine, pw & 63);
-        const int wn = pw < PW ? wn_any : 0;
-        // local cell of the window's first cell, and of w[0] once the window lies inside the tile
-        const int s0 = wlow - tx * tg.tw;
-        const int b = max(0, min(s0, tg.tw - kWindowCells));
-        const int cell = tx * tg.tw + b + slot;           // the cell this lane weighs
-        const int c = cell - wlow;                        // its place in the window
-        float w = 0.0f;
-        if (slot >= 0 && c >= 0 && c < wn && b + slot < tg.tw && cell < W)
-          w = merged_weight(g.start_w, pw, g.bin_w, g.grid_w, W, cell);
-        // The cells the tile owner reads and writes for this window (local): w[0..3] if one of
-        // them is not zero, w[4..6] likewise -- cells of weight zero among them included.
-        const unsigned live = static_cast<unsigned>(__ballot(w != 0.0f) >> (8 * sub)) & 0xffu;
-        const bool head = (live & 0x1eu) != 0, tail = (live & 0xe0u) != 0;
-        const int lo = head ? b : tail ? b + 4 : tg.tw;
-        const int hi = tail ? b + kWindowCells - 1 : head ? b + 3 : -1;
-        // smallest power-of-two distance at which no two windows of these eight columns share a cell
-        int lg = 0;
-#pragma unroll
-        for (int d = 1; d <= 4; d <<= 1) {
-          const int lo_d = __shfl_down(lo, 8 * d), hi_d = __shfl_down(hi, 8 * d);
-          const bool clash = sub + d < 8 && lo <= hi && lo_d <= hi_d && lo_d <= hi && lo <= hi_d;
-          if (__ballot(clash) != 0) lg = __builtin_ctz(d) + 1;
-        }
-        const int out = slot < 0 ? ((b + 1) | (lg << 16)) : __float_as_int(w);
-        cols[(static_cast<long long>(tx) * ll.col_stride + 2 * pw) * 4 + (lane & 7)] = out;
-      }
-    }
-  }
-}
-
 __global__ void __launch_bounds__(256) build_lists_kernel(ListsArgs a) {
-  if (a.window_offsets != nullptr) build_window_lists_body(blockIdx.x, a);
-  else build_lists_body(blockIdx.x, a);
+  build_lists_body(blockIdx.x, a);
 }
-
 
 // One wavefront's share of a tile: the (ROI, pooled row, weight) taps that land
 // on one tile row, in ROI order, so that the owner of that row streams through
 // them without looking anything up.
 struct alignas(16) WorkEntry {
-  int roi;     // the list item (its column pairs are read from its lists)
+  int roi;     // whose column pairs and dy are read
   int ph;
   float wy;
-  int flags;   // bit 0: continues the previous entry's item; bit 1: last entry of its item;
-               // bits 2..: the ROI whose dy the entry reads (the item itself, or the ROI it is a window of)
+  int flags;   // bit 0: continues the previous entry's ROI; bit 1: last entry of its ROI
 };
 struct WorkRange { int begin; int count; };
 
@@ -633,10 +297,8 @@ __device__ __forceinline__ SortedRow sorted_row(const SortedRow* __restrict__ so
 // sixteen lists comes from one bump-pointer allocation per tile (cursors[1]).
 // The order in which tiles take their space varies from run to run; what is
 // written into it does not.
-// WIN: the items are windows of merged weights (WindowRowTable) rather than sample lists.
 constexpr int kTileListCap = 4096;   // items of one tile that LDS holds (longer lists go through memory)
 
-template <bool WIN>
 __global__ void __launch_bounds__(kTileRows * 64)
 build_tile_work_kernel(const TileBox* __restrict__ boxes, int R, int* __restrict__ tile_rois,
                        const AxisUnit* __restrict__ lists, TileGrid tg, ListLayout ll,
@@ -645,10 +307,8 @@ build_tile_work_kernel(const TileBox* __restrict__ boxes, int R, int* __restrict
   __shared__ int hits[kTileRows];
   __shared__ int row_total[kTileRows];
   __shared__ int list_base, tile_base;
-  // the tile's items and the ROIs whose dy they read (<< 2, as the entries hold them), in item
-  // order: in LDS, so that the wavefronts below need not wait for memory to see the list
+  // the tile's ROIs in their order: in LDS, so that the wavefronts below need not wait for memory to see the list
   __shared__ int item_s[kTileListCap];
-  __shared__ int owner_s[kTileListCap];
   const long long tile = blockIdx.x;
   const int lane = threadIdx.x & 63, row = threadIdx.x >> 6;
   const int image = static_cast<int>(tile / tg.per_image);
@@ -658,10 +318,9 @@ build_tile_work_kernel(const TileBox* __restrict__ boxes, int R, int* __restrict
   // ---- the tile's item list ----
   const int share = ((R + kTileRows * 64 - 1) / (kTileRows * 64)) * 64;
   const int r_begin = row * share, r_end = min(R, r_begin + share);
-  auto hit_of = [&](int r, int* owner) {
+  auto hit_of = [&](int r) {
     if (r >= r_end) return false;
     const TileBox b = boxes[r];
-    *owner = b.roi << 2;
     return b.batch == image && ty >= (b.ty & 0xffff) && ty <= (b.ty >> 16) && tx >= (b.tx & 0xffff) &&
            tx <= (b.tx >> 16);
   };
@@ -669,18 +328,13 @@ build_tile_work_kernel(const TileBox* __restrict__ boxes, int R, int* __restrict
   // walk: with up to 4096 boxes in all that is every chunk, and the boxes are read once)
   constexpr int kKept = 4;
   bool kept_hit[kKept];
-  int kept_owner[kKept];
   int mine = 0;
 #pragma unroll
   for (int k = 0; k < kKept; ++k) {
-    kept_owner[k] = 0;
-    kept_hit[k] = hit_of(r_begin + 64 * k + lane, &kept_owner[k]);
+    kept_hit[k] = hit_of(r_begin + 64 * k + lane);
     mine += __popcll(__ballot(kept_hit[k]));
   }
-  for (int base = r_begin + 64 * kKept; base < r_end; base += 64) {
-    int unused_owner = 0;
-    mine += __popcll(__ballot(hit_of(base + lane, &unused_owner)));
-  }
+  for (int base = r_begin + 64 * kKept; base < r_end; base += 64) mine += __popcll(__ballot(hit_of(base + lane)));
   if (lane == 0) hits[row] = mine;
   __syncthreads();
   int written = 0, count = 0;
@@ -694,11 +348,11 @@ build_tile_work_kernel(const TileBox* __restrict__ boxes, int R, int* __restrict
     __syncthreads();
   }
   int* const long_list = tile_rois + (in_lds ? 0 : list_base);
-  auto put = [&](int base, bool hit, int owner) {
+  auto put = [&](int base, bool hit) {
     const unsigned long long mask = __ballot(hit);
     if (hit) {
       const int at = written + __popcll(mask & ((1ull << lane) - 1ull));
-      if (in_lds) { item_s[at] = base + lane; owner_s[at] = owner; }
+      if (in_lds) item_s[at] = base + lane;
       else long_list[at] = base + lane;
     }
     written += __popcll(mask);
@@ -706,27 +360,16 @@ build_tile_work_kernel(const TileBox* __restrict__ boxes, int R, int* __restrict
   };
 #pragma unroll
   for (int k = 0; k < kKept; ++k)
-    if (mine > 0) put(r_begin + 64 * k, kept_hit[k], kept_owner[k]);
-  for (int base = r_begin + 64 * kKept; base < r_end && mine > 0; base += 64) {
-    int owner = 0;
-    const bool hit = hit_of(base + lane, &owner);
-    put(base, hit, owner);
-  }
+    if (mine > 0) put(r_begin + 64 * k, kept_hit[k]);
+  for (int base = r_begin + 64 * kKept; base < r_end && mine > 0; base += 64) put(base, hit_of(base + lane));
   __syncthreads();   // the list is complete and visible to the whole workgroup
   auto item_at = [&](int i) { return in_lds ? item_s[i] : long_list[i]; };
-  auto owner_at = [&](int i, int item) { return in_lds ? owner_s[i] : boxes[item].roi << 2; };
 
   // ---- the work lists of the sixteen rows ----
   // taps of list item `roi` on this wavefront's tile row: where they start, how many
   auto taps_of = [&](int roi, const RowTap** taps) {
     const AxisUnit* const table = lists + static_cast<long long>(roi) * ll.roi_stride +
                                   static_cast<long long>(ty) * ll.row_stride;
-    if (WIN) {
-      const WindowRowTable* const tb = reinterpret_cast<const WindowRowTable*>(table);
-      const unsigned idx = tb->index[row];
-      *taps = tb->taps + (idx & 0xffffu);
-      return static_cast<int>(idx >> 16);
-    }
     const RowTapTable* const tb = reinterpret_cast<const RowTapTable*>(table);
     const unsigned idx = tb->index[row];
     *taps = tb->taps + (idx & 0xffu);
@@ -769,7 +412,7 @@ build_tile_work_kernel(const TileBox* __restrict__ boxes, int R, int* __restrict
     }
   }
   for (int base = 0; base < count; base += 64) {
-    int c = first_c, roi = first_item, owner = 0;
+    int c = first_c, roi = first_item;
     const RowTap* taps = first_taps;
     if (base > 0) {
       c = 0; roi = 0; taps = nullptr;
@@ -778,7 +421,6 @@ build_tile_work_kernel(const TileBox* __restrict__ boxes, int R, int* __restrict
         c = taps_of(roi, &taps);
       }
     }
-    if (base + lane < count) owner = owner_at(base + lane, roi);
     int incl = c;
     for (int off = 1; off < 64; off <<= 1) {
       const int up = __shfl_up(incl, off);
@@ -793,15 +435,14 @@ build_tile_work_kernel(const TileBox* __restrict__ boxes, int R, int* __restrict
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const int q = q0 + k;
-        if (q < c) dst[q] = WorkEntry{roi, four[k].ph, four[k].wy, (q > 0 ? 1 : 0) | (q == c - 1 ? 2 : 0) | owner};
+        if (q < c) dst[q] = WorkEntry{roi, four[k].ph, four[k].wy, (q > 0 ? 1 : 0) | (q == c - 1 ? 2 : 0)};
       }
     }
     out += __shfl(incl, 63);
   }
   // padding: taps of weight zero that continue the last ROI and never end it
   if (lane < reserved - total) {
-    const int item = item_at(count - 1);
-    entries[out + lane] = WorkEntry{item, 0, 0.0f, 1 | owner_at(count - 1, item)};
+    entries[out + lane] = WorkEntry{item_at(count - 1), 0, 0.0f, 1};
   }
 }
 

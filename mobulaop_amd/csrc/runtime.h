@@ -52,13 +52,6 @@ long long release_workspace();   // frees the calling thread's buffer on the cur
 void unpin_workspace();
 long long workspace_bytes();
 
-// A few words of pinned host memory of the calling thread, for a number the host needs from the device
-// before it can go on: a kernel writes words[0..2] and then, behind a system-wide fence, words[3] = ticket.
-struct Mailbox { int* words = nullptr; int ticket = 0; };
-Mailbox* mailbox();
-// Waits until words[3] holds box->ticket; false with an error set if the stream failed first.
-bool wait_for_mail(Mailbox* box, hipStream_t stream);
-
 long long option(const char* name, long long fallback);
 
 // Makes `device` current for the lifetime of the object (no-op for -1).

@@ -165,47 +165,6 @@ long long workspace_bytes() {
   return s == nullptr ? 0 : static_cast<long long>(s->bytes);
 }
 
-namespace {
-struct MailboxOfThread {
-  Mailbox box;
-  ~MailboxOfThread() {
-    if (box.words != nullptr) (void)hipHostFree(box.words);
-  }
-};
-}  // namespace
-
-Mailbox* mailbox() {
-  static thread_local MailboxOfThread mine;
-  if (mine.box.words == nullptr) {
-    void* p = nullptr;
-    MOBULA_HIP_TRY(hipHostMalloc(&p, 64, hipHostMallocPortable | hipHostMallocCoherent));
-    if (!failed()) {
-      std::memset(p, 0, 64);
-      mine.box.words = static_cast<int*>(p);
-    }
-  }
-  return &mine.box;
-}
-
-bool wait_for_mail(Mailbox* box, hipStream_t stream) {
-  const volatile int* const words = box->words;
-  for (unsigned spins = 0; words[3] != box->ticket; ++spins) {
-    __builtin_ia32_pause();
-    if (spins % 4096 != 4095) continue;
-    // (the stream has nothing left to do, or has failed: the mail is there, or will never be)
-    const hipError_t state = hipStreamQuery(stream);
-    if (state == hipErrorNotReady) {
-      (void)hipGetLastError();   // (an answer, no error of the call)
-      continue;
-    }
-    MOBULA_HIP_TRY(state);
-    if (!failed() && words[3] != box->ticket) set_error("a kernel ended without its message to the host");
-    break;
-  }
-  std::atomic_thread_fence(std::memory_order_acquire);
-  return !failed();
-}
-
 long long option(const char* name, long long fallback) {
   std::lock_guard<std::mutex> lock(g_mutex);
   auto it = g_options.find(name);
@@ -358,7 +317,7 @@ void mobula_hip_clear_error(void) { call_state().error.clear(); }
 int mobula_hip_set_option(const char* name, long long value) {
   static const char* known[] = {"roialign_impl", "host_staging_device", "kernel_timing", "side_stream",
                                 "conv_compute", "conv_fp32_split", "roialign_tile_columns", "roialign_row_split", "roialign_row_quads",
-                                "roialign_sort_rows", "roialign_few_boxes", nullptr};
+                                "roialign_sort_rows", "roialign_few_boxes", "roialign_patch", nullptr};
   for (int i = 0; known[i] != nullptr; ++i) {
     if (std::strcmp(known[i], name) == 0) {
       std::lock_guard<std::mutex> lock(mobula_hip::g_mutex);

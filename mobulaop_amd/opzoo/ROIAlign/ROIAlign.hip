@@ -15,6 +15,7 @@
 #include "roialign_f64.hip.h"
 #include "roialign_backward_blocked.hip.h"
 #include "roialign_backward_few.hip.h"
+#include "roialign_backward_patch.hip.h"
 #include "roialign_forward_blocked.hip.h"
 #include "roialign_forward_merged.hip.h"
 
@@ -371,45 +372,7 @@ DyLaunch dy_launch(const Problem& p) {
 template <typename T>
 bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_dyb,
                 hipStream_t stream, TilePlan* plan, const T* fuse_dy = nullptr) {
-  // List items: the ROIs, or for sampling grids of more than 2 x 2 points the
-  // windows of merged weights their bins are cut into.  How many depends on the
-  // boxes, so their number has to come back from the device (the host waits for it:
-  // not while the stream is being captured into a graph).
-  const bool windows = roialign::lists_in_windows(p.S);
-  long long items = p.R, window_entries = 0;
-  // the head of the workspace: offsets[R + 1], counts[R], work[R] (see window_offsets_kernel)
-  const size_t b_offsets = windows ? align_up(sizeof(int) * (2 * p.R + 1), 256) +
-                                         align_up(sizeof(long long) * p.R, 256) : 0;
-  char* head = nullptr;
-  const roialign::WindowArgs wa{rois, p.R, p.scale, p.PH, p.PW, p.S, p.H, p.W, tw};
-  auto number_windows = [&](char* at, int* told, int ticket) {
-    int* const offsets = reinterpret_cast<int*>(at);
-    int* const counts = offsets + p.R + 1;
-    long long* const work = reinterpret_cast<long long*>(at + align_up(sizeof(int) * (2 * p.R + 1), 256));
-    if (p.R > roialign::kCountedInOffsets)
-      roialign::window_counts_kernel<<<grid_for(p.R, 256), 256, 0, stream>>>(wa, counts, work);
-    roialign::window_offsets_kernel<<<1, 1024, 0, stream>>>(wa, counts, work, offsets, told, ticket);
-  };
-  if (p.S > roialign::kSearchedGrid) return false;   // (fixed grids of that size are not merged)
-  if (windows) {
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
-      (void)hipGetLastError();
-      return false;
-    }
-    head = static_cast<char*>(mobula_hip::workspace(b_offsets));
-    mobula_hip::Mailbox* const box = mobula_hip::mailbox();
-    if (failed()) return false;
-    // the numbers come back through pinned memory that this thread watches (a copy and a wait for
-    // the stream take some 25 us longer, with the device idle)
-    number_windows(head, box->words, ++box->ticket);
-    MOBULA_HIP_TRY(hipGetLastError());
-    if (failed() || !mobula_hip::wait_for_mail(box, stream)) return false;
-    const volatile int* const info = box->words;
-    if (info[1] != 0) return false;   // an adaptive grid too large to merge
-    items = info[0];
-    window_entries = info[2];
-  }
+  const long long items = p.R;
   if (items > (1ll << 22)) return false;
   roialign::TileGrid& g = plan->grid;
   g.th = th; g.tw = tw;
@@ -432,9 +395,7 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
   const size_t b_slab = with_dyb ? sizeof(T) * 32 * p.PW * p.R * p.PH : 0;
   const size_t b_dyt = align_up(b_slab * cblk, 256);
   // work lists: every tap of every ROI once per tile column it spans
-  // (windows: the bound that came back with their number)
-  const long long n_entries = (windows ? window_entries : items * 2 * p.PH * (p.S == 1 ? 1 : 2) * g.tx) +
-                              11 * roialign::kTileRows * g.total;
+  const long long n_entries = items * 2 * p.PH * (p.S == 1 ? 1 : 2) * g.tx + 11 * roialign::kTileRows * g.total;
   if (n_entries > (1ll << 27)) return false;
   // the consumer addresses both with 32-bit byte offsets
   if (b_slab >= (1ull << 31) || b_units >= (1ull << 31)) return false;
@@ -447,15 +408,9 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
   const bool sort_rows = g.total * roialign::kTileRows <= kSortedRows && sort_option != 0 &&
                          (sort_option == 2 || (!p.nhwc && cblk >= 5 && p.n_out >= kSortedAbove * p.N * p.C * p.H * p.W));
   const size_t b_sorted = sort_rows ? sizeof(roialign::SortedRow) * roialign::kWorkClasses * g.total * roialign::kTileRows : 0;
-  char* base = static_cast<char*>(mobula_hip::workspace(b_offsets + b_recs + b_cnt + b_list + b_units + b_dyt +
-                                                        b_ranges + b_entries + b_sorted + 256));
+  char* base = static_cast<char*>(mobula_hip::workspace(b_recs + b_cnt + b_list + b_units + b_dyt + b_ranges + b_entries +
+                                                        b_sorted + 256));
   if (failed()) return false;
-  int* offsets = nullptr;
-  if (windows) {
-    if (base != head) number_windows(base, nullptr, 0);   // the workspace has grown: it is another buffer now
-    offsets = reinterpret_cast<int*>(base);
-    base += b_offsets;
-  }
   plan->boxes = reinterpret_cast<roialign::TileBox*>(base);
   plan->cursors = reinterpret_cast<int*>(base + b_recs);
   plan->tile_rois = reinterpret_cast<int*>(base + b_recs + b_cnt);
@@ -471,8 +426,8 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
   // two kernels: per-item tables (which also resets the bump pointers), then per-tile lists
   const int n_items = static_cast<int>(items);
   const roialign::ListsArgs la{rois, n_items, p.R, p.scale, p.PH, p.PW, p.S, p.H, p.W, p.N, g, plan->layout,
-                               plan->boxes, plan->cursors, plan->lists, offsets, windows ? roialign::lists_parts_log(items) : 0};
-  const long long list_blocks = roialign::lists_blocks(items, la.parts_log);
+                               plan->boxes, plan->cursors, plan->lists};
+  const long long list_blocks = roialign::lists_blocks(items);
   const DyLaunch dl = dy_launch<T>(p);
   if (fuse_dy != nullptr && with_dyb && dl.per > 0 && dl.blocks > 0 && dl.blocks + list_blocks < (1ll << 31)) {
     roialign::lists_and_dy_kernel<T><<<static_cast<unsigned>(dl.blocks + list_blocks), 256, dl.lds, stream>>>(
@@ -481,10 +436,9 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
   } else {
     roialign::build_lists_kernel<<<static_cast<unsigned>(list_blocks), 256, 0, stream>>>(la);
   }
-  (windows ? roialign::build_tile_work_kernel<true> : roialign::build_tile_work_kernel<false>)
-      <<<static_cast<unsigned>(g.total), roialign::kTileRows * 64, 0, stream>>>(
-          plan->boxes, n_items, plan->tile_rois, plan->lists, g, plan->layout, plan->cursors, plan->ranges,
-          plan->entries, plan->sorted, p.H);
+  roialign::build_tile_work_kernel<<<static_cast<unsigned>(g.total), roialign::kTileRows * 64, 0, stream>>>(
+      plan->boxes, n_items, plan->tile_rois, plan->lists, g, plan->layout, plan->cursors, plan->ranges, plan->entries,
+      plan->sorted, p.H);
   MOBULA_HIP_TRY(hipGetLastError());
   return !failed();
 }
@@ -497,7 +451,7 @@ int tile_columns(const Problem& p) {
   using BB = roialign::BwdBlocked;
   const long long forced = mobula_hip::option("roialign_tile_columns", 0);
   if (forced >= BB::TW_LEAST && forced <= BB::TW && forced % 4 == 0) return static_cast<int>(forced);
-  return roialign::backward_tile_columns(p.N, p.H, p.W, (p.C + BB::CB - 1) / BB::CB, roialign::lists_in_windows(p.S));
+  return roialign::backward_tile_columns(p.N, p.H, p.W, (p.C + BB::CB - 1) / BB::CB);
 }
 
 // Wavefronts per tile row of the backward pass (1, or BwdBlocked::NSPLIT for maps with few tile
@@ -509,18 +463,11 @@ int row_split(const Problem& p) {
   return roialign::backward_row_split(p.N, p.H, p.W, (p.C + BB::CB - 1) / BB::CB);
 }
 
-// The tile owner for a problem: nsplit wavefronts per tile row, sample lists or
-// windows of merged weights (which are not split: 47 us against 71 in four parts, 301 boxes on
-// 3 x 81 x 75 x 113).
+// The tile owner for a problem: nsplit wavefronts per tile row.
 template <bool NHWC, typename T>
-auto owner_kernel(int* nsplit, bool windows) {
+auto owner_kernel(int nsplit) {
   using BB = roialign::BwdBlocked;
-  if (windows) {
-    *nsplit = 1;
-    return roialign::backward_blocked_kernel<NHWC, T, 1, true>;
-  }
-  return *nsplit > 1 ? roialign::backward_blocked_kernel<NHWC, T, BB::NSPLIT, false>
-                     : roialign::backward_blocked_kernel<NHWC, T, 1, false>;
+  return nsplit > 1 ? roialign::backward_blocked_kernel<NHWC, T, BB::NSPLIT> : roialign::backward_blocked_kernel<NHWC, T, 1>;
 }
 
 // Any sampling grid the lists take: fixed ones up to kSearchedGrid points, adaptive ones
@@ -556,6 +503,54 @@ void launch_few_boxes(const Problem& p, const T* dy, const float* rois, T* dx, b
   MOBULA_HIP_TRY(hipGetLastError());
 }
 
+// How backward_patch_kernel is launched: wavefronts of a workgroup (0: not at all), patches, workspace.
+struct PatchPlan { int waves; long long blocks; int tiles_x, tiles_y, hp, wp; size_t b_spans, b_records, b_dense; };
+
+// For sampling grids of more than two points per bin and axis; the option "roialign_patch" 4 or 12 names the wavefronts,
+// and takes grids of one and two points too (tests do).
+PatchPlan patch_plan(const Problem& p) {
+  using BP = roialign::BwdPatch;
+  PatchPlan plan{};
+  const long long option = mobula_hip::option("roialign_patch", 1);
+  const bool forced = option == 4 || option == 12;
+  if ((!forced && (p.S == 1 || p.S == 2)) || p.S > roialign::kSearchedGrid || p.PW > BP::BINS || p.PH > BP::MOST_PH) return plan;
+  plan.tiles_x = (p.W + BP::TX - 1) / BP::TX;
+  plan.tiles_y = (p.H + BP::TY - 1) / BP::TY;
+  plan.hp = (p.H + 15) / 16 * 16; plan.wp = (p.W + 15) / 16 * 16;
+  plan.b_spans = align_up(2 * sizeof(roialign::PatchSpan) * p.R, 256);
+  plan.b_records = align_up(sizeof(roialign::CellRecord) * p.R * (static_cast<long long>(plan.hp) + plan.wp), 256);
+  plan.b_dense = align_up(sizeof(float) * p.R * ((p.PH + 3) * p.PH + (p.PW + 3) * p.PW), 256);
+  const long long patches = p.N * plan.tiles_x * plan.tiles_y;
+  plan.blocks = patches * ((p.C + BP::CH - 1) / BP::CH);
+  if (plan.blocks >= (1ll << 31) || plan.b_records > (8ull << 30)) return plan;
+  // Twelve wavefronts to a patch where patches are few or their lists long (every one looks at all boxes and adds its sums up
+  // at the end).  Forward and backward with 4 and with 12, us: 126 patches times channel blocks of 2592 boxes (1 x 456 x 137 x
+  // 100) 1468 / 1396, 1152 of 1254 (4 x 80 x 41 x 248) 710 / 660, 770 of 482 (7 x 160 x 82 x 18) 286 / 296, 720 of 100 (3 x 81 x
+  // 75 x 113) 72 / 83, 5472 of 413 (4 x 256 x 148 x 131) 530 / 660, 576 of 671 (1 x 72 x 93 x 243) 190 / 169, 324 of 1295 (2 x 176 x
+  // 70 x 33) 337 / 220, 112 of 325 (4 x 32 x 49 x 56) 276 / 158, 120 of 736 (5 x 64 x 28 x 44) 405 / 208.
+  plan.waves = forced ? static_cast<int>(option)
+                      : plan.blocks <= 640 || (plan.blocks <= 2048 && p.R >= 8 * patches) ? 12 : 4;
+  return plan;
+}
+
+// False where there is no room for the weights (a stream being captured, a recorded graph with a smaller workspace).
+template <bool NHWC, typename T>
+bool launch_patches(const Problem& p, const PatchPlan& plan, const T* dy, const float* rois, T* dx, bool assign,
+                    hipStream_t stream) {
+  char* const ws = static_cast<char*>(mobula_hip::workspace_if_possible(plan.b_spans + plan.b_records + plan.b_dense + 256));
+  if (ws == nullptr || failed()) return false;
+  const roialign::PatchArgs pa{rois, static_cast<int>(p.R), p.scale, p.PH, p.PW, p.S, p.H, p.W, static_cast<int>(p.N), plan.hp, plan.wp,
+                               reinterpret_cast<roialign::PatchSpan*>(ws), reinterpret_cast<roialign::CellRecord*>(ws + plan.b_spans),
+                               reinterpret_cast<float*>(ws + plan.b_spans + plan.b_records)};
+  if (p.R > 0) roialign::patch_weights_kernel<<<(p.R + 1) / 2, 256, 0, stream>>>(pa);
+  const auto kernel = plan.waves == 4 ? roialign::backward_patch_kernel<T, NHWC, 4> : roialign::backward_patch_kernel<T, NHWC, 12>;
+  mobula_hip::KernelTimer timer("backward_blocked_kernel", stream);   // (whoever owns dx reports under this name)
+  kernel<<<static_cast<unsigned>(plan.blocks), plan.waves * 64, 0, stream>>>(dy, pa, dx, p.C, plan.tiles_x, plan.tiles_y,
+                                                                             assign ? 1 : 0);
+  MOBULA_HIP_TRY(hipGetLastError());
+  return true;
+}
+
 template <typename T>
 void backward_device(const Problem& p, const T* dy, const float* rois, T* dx, bool assign,
                      hipStream_t stream) {
@@ -573,7 +568,10 @@ void backward_device(const Problem& p, const T* dy, const float* rois, T* dx, bo
       launch_few_boxes<true>(p, dy, rois, dx, assign, stream);
       return;
     }
-    if (!taken ||
+    if (const PatchPlan patches = patch_plan(p);
+        taken && patches.waves > 0 && launch_patches<true>(p, patches, dy, rois, dx, assign, stream))
+      return;
+    if (!taken || (p.S != 1 && p.S != 2) ||
         !plan_tiles<T>(p, rois, roialign::kTileRows, tw, /*with_dyb=*/false, stream, &plan) ||
         roialign::backward_blocked_grid(plan.grid.total, cblk) >= (1ll << 31)) {
       if (!failed())
@@ -583,8 +581,8 @@ void backward_device(const Problem& p, const T* dy, const float* rois, T* dx, bo
     }
     const unsigned dy_bytes = static_cast<unsigned>(sizeof(T) * p.n_out);
     mobula_hip::KernelTimer timer("backward_blocked_kernel", stream);
-    int nsplit = row_split(p);
-    const auto kernel = owner_kernel<true, T>(&nsplit, plan.layout.windows != 0);
+    const int nsplit = row_split(p);
+    const auto kernel = owner_kernel<true, T>(nsplit);
     kernel<<<static_cast<unsigned>(roialign::backward_blocked_grid(plan.grid.total, cblk)), BB::NT * nsplit,
              roialign::backward_blocked_lds(tw, nsplit), stream>>>(
         dy, dx, plan.ranges, plan.sorted, plan.class_counts(), plan.entries, plan.lists,
@@ -598,12 +596,17 @@ void backward_device(const Problem& p, const T* dy, const float* rois, T* dx, bo
     launch_few_boxes<false>(p, dy, rois, dx, assign, stream);
     return;
   }
+  if (const PatchPlan patches = patch_plan(p);
+      use_tiled() && patches.waves > 0 && launch_patches<false>(p, patches, dy, rois, dx, assign, stream))
+    return;
+  if (failed()) return;
+  const bool lists = use_tiled() && (p.S == 1 || p.S == 2) && roialign::backward_blocked_supports(p.PH, p.PW, p.S);
   // the pre-pass (small, latency-bound kernels) runs beside the dy transposition, when that is
   // long enough to hide it: the transposition on the second stream, the pre-pass -- the longer of
   // the two beside a copy that saturates the memory -- on the caller's, so that the tile owners
   // follow it without waiting for a signal from another queue
   // (without a second stream the transposition shares the launch of the list builder instead)
-  const bool forked = static_cast<long long>(sizeof(T)) * p.n_out >= kSideStreamBytes &&
+  const bool forked = lists && static_cast<long long>(sizeof(T)) * p.n_out >= kSideStreamBytes &&
                       mobula_hip::option("side_stream", 1) != 0;
   if (forked) {
     // the helper stream forks from the caller's: whatever the caller's stream has to wait for
@@ -614,8 +617,7 @@ void backward_device(const Problem& p, const T* dy, const float* rois, T* dx, bo
   }
   mobula_hip::SideStream side(stream, forked);
   const int tw = tile_columns(p);
-  if (use_tiled() && roialign::backward_blocked_supports(p.PH, p.PW, p.S) &&
-      plan_tiles<T>(p, rois, roialign::kTileRows, tw, /*with_dyb=*/true, stream, &plan,
+  if (lists && plan_tiles<T>(p, rois, roialign::kTileRows, tw, /*with_dyb=*/true, stream, &plan,
                     side.get() == stream ? dy : nullptr)) {
     const int cblk = (p.C + BB::CB - 1) / BB::CB;
     const long long grid = roialign::backward_blocked_grid(plan.grid.total, cblk);
@@ -627,11 +629,11 @@ void backward_device(const Problem& p, const T* dy, const float* rois, T* dx, bo
       side.join();
       {
         mobula_hip::KernelTimer timer("backward_blocked_kernel", stream);
-        int nsplit = row_split(p);
+        const int nsplit = row_split(p);
         // every row piece of dx starts at a multiple of four elements (tile widths are): four columns per store
         const bool quads = p.W % 4 == 0 && reinterpret_cast<size_t>(dx) % (4 * sizeof(T)) == 0 &&
                            mobula_hip::option("roialign_row_quads", 1) != 0;
-        const auto kernel = owner_kernel<false, T>(&nsplit, plan.layout.windows != 0);
+        const auto kernel = owner_kernel<false, T>(nsplit);
         kernel<<<static_cast<unsigned>(grid), BB::NT * nsplit, roialign::backward_blocked_lds(tw, nsplit), stream>>>(
             plan.dyb, dx, plan.ranges, plan.sorted, plan.class_counts(), plan.entries, plan.lists, plan.grid, plan.layout, p.C, p.H,
             p.W, p.PH, p.PW, cblk, static_cast<unsigned>(plan.dyb_bytes),

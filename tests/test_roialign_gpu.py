@@ -889,6 +889,72 @@ def test_backward_of_a_few_boxes_in_one_launch(R, C, H, W, pooled, S, dtype, lay
         native.set_option('roialign_few_boxes', 1)
 
 
+@pytest.mark.parametrize('waves', [4, 12])
+@pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('R,C,H,W,pooled,S,scale', [
+    (1, 1, 1, 1, (1, 1), 0, 1.0),
+    (0, 33, 9, 17, (2, 2), 0, 0.5),
+    (13, 33, 8, 16, (7, 7), 3, 0.5),         # a patch, and a channel of the next block
+    (40, 31, 9, 33, (4, 8), 0, 0.25),        # rows and columns beyond it; all bins staged at once
+    (40, 36, 23, 15, (5, 8), 0, 0.25),       # one pooled row more than are staged at once
+    (25, 64, 40, 37, (32, 32), 5, 0.5),      # the most pooled rows and columns
+    (30, 4, 20, 200, (1, 17), 0, 1.0),       # wide bins
+    (30, 4, 200, 20, (17, 1), 64, 1.0),      # a dense fixed grid, dozens of weights to a cell
+    (3200, 5, 9, 12, (2, 3), 0, 0.25),       # more boxes than are looked at at a time
+    (50, 40, 33, 40, (14, 14), 2, 0.25),
+    (50, 40, 33, 40, (14, 14), 1, 0.25),
+])
+def test_backward_in_patches(R, C, H, W, pooled, S, scale, dtype, layout, waves):
+    """Edges of patches, of channel blocks and of what is staged; boxes below a pixel, across the borders, off the map, of no
+    image, far larger than the map and not a number."""
+    native.set_option('roialign_patch', waves)
+    native.set_option('roialign_few_boxes', 0)
+    if layout == 'nhwc':
+        C = (C + 3) // 4 * 4
+    try:
+        rng = np.random.default_rng(R + C + H + pooled[0])
+        N = 3
+        at = np.stack([rng.uniform(-0.2 * W, W, R), rng.uniform(-0.2 * H, H, R)], 1) / scale
+        wh = np.stack([rng.uniform(0, W, R), rng.uniform(0, H, R)], 1) / scale * rng.choice((0, 0.1, 1.0), (R, 1))
+        rois = np.concatenate([rng.integers(0, N, (R, 1)), at, at + wh], 1).astype(np.float32)
+        if R > 12:
+            rois[3, 0], rois[5, 0] = N, -1
+            rois[6, 1:] = (-3.0e5, -3.0e5, 3.0e5, 3.0e5)   # 2^15 points and more to a bin where the grid is adaptive
+            rois[7, 1:] = (-2.0 * W / scale, 0, -1.5 * W / scale, H / scale)
+        if S > 32:   # (the oracle takes a sample at a time)
+            rois, R = rois[:20], 20
+        dy = torch.from_numpy(rng.standard_normal((R, C) + pooled).astype(np.float32)).to(dtype)
+        shape = (N, C, H, W)
+        ok = (rois[:, 0] >= 0) & (rois[:, 0] < N)
+        if S <= 0:
+            ok &= (rois[:, 3] - rois[:, 1]) < 1e5
+            huge = ~ok & (rois[:, 0] >= 0) & (rois[:, 0] < N)
+            dy[torch.from_numpy(huge)] = 0   # (what the oracle would take hours for adds nothing)
+        want = oracle.backward(dy.float().numpy()[ok], rois[ok], shape, scale, S, impl='ordered')
+        tol = {torch.float32: BWD_TOL, torch.float16: FP16_TOL, torch.bfloat16: 1e-2}[dtype]
+
+        def backward(rois, dx=None):
+            last = layout == 'nhwc'
+            put = lambda a: (a.permute(0, 2, 3, 1) if last else a).contiguous().cuda()   # noqa: E731
+            call = abi.backward_nhwc if last else abi.backward
+            got = call(put(dy), abi.to_dev(rois), (N, H, W, C) if last else shape, scale, S, assign=dx is None,
+                       dx=None if dx is None else put(dx))
+            return (got.permute(0, 3, 1, 2) if last else got).float().cpu()
+        got = backward(rois)
+        assert_parity(got.numpy(), torch.from_numpy(want).to(dtype).float().numpy(), tol, 'assign')
+        assert torch.equal(got, backward(rois))
+        base = torch.from_numpy(rng.standard_normal(shape).astype(np.float32)).to(dtype)
+        assert_parity(backward(rois, base).numpy(), (torch.from_numpy(want) + base.float()).to(dtype).float().numpy(), tol, 'accumulate')
+        if R > 12:   # a box that is not a number, or infinite, ends; other images are as they were
+            rois[0, 1:], rois[1, 1:] = np.nan, (0, 0, np.inf, np.inf)
+            others = [n for n in range(N) if n not in rois[:2, 0]]
+            assert torch.equal(backward(rois)[others], got[others])
+    finally:
+        native.set_option('roialign_patch', 1)
+        native.set_option('roialign_few_boxes', 1)
+
+
 def test_workspace_can_be_given_back():
     """The scratch buffer grows with the largest call of the thread; a caller
     may release it between phases, and the next call allocates afresh."""
