@@ -99,7 +99,9 @@ __device__ __forceinline__ int merge_axis_samples(MergedEntry* out, float start,
   return count;
 }
 
-template <typename T, bool NHWC>
+// CLIP: boxes of grids up to kMergedGrid points take this way too (else up to kSearchedGrid), for bins so few that a box on the
+// map can have such a grid (forward_device).  Where it cannot, the test alone costs 1 % (4 x 512 x 100 x 100 fp16: 410 -> 415 us).
+template <typename T, bool NHWC, bool CLIP>
 __global__ void __launch_bounds__(FwdMerged::NW * 64, 4)
 forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
                       const int* __restrict__ order, T* __restrict__ y, float scale, int C, int H,
@@ -108,6 +110,7 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
                       const T* __restrict__ x, unsigned jobs) {
   using K = FwdBlocked;
   using M = FwdMerged;
+  constexpr int kMost = CLIP ? kMergedGrid : kSearchedGrid;
   constexpr int CPL = BlockOf<T>::CPL, CB = BlockOf<T>::CB, STAGE = BlockOf<T>::STAGE_MERGED;
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
   __shared__ __attribute__((aligned(16))) MergedEntry rowm_s[M::NW][M::RPH][M::LCAP];
@@ -115,11 +118,11 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
   __shared__ int rown_s[M::NW][M::RPH];
   __shared__ __attribute__((aligned(16))) T stage_s[M::NW][STAGE];
   if (direct != nullptr && *direct != 0) return;   // (forward_naive_kernel does the call: choose_direct_kernel)
-  // behind the jobs: boxes of larger grids, from the map itself (as a launch of their own, which found nothing to do for
+  // behind the jobs: boxes of the largest grids, from the map itself (as a launch of their own, which found nothing to do for
   // boxes on their map, they took 4 us a call)
   if (blockIdx.x >= jobs) {
     static_assert(M::NW == 1, "a wavefront per box");
-    forward_large_grid<T, NHWC>(blockIdx.x - jobs, x, scale, C, H, W, PH, PW, S, rois, y, num_images);
+    forward_large_grid<T, NHWC>(blockIdx.x - jobs, kMost, x, scale, C, H, W, PH, PW, S, rois, y, num_images);
     return;
   }
 
@@ -173,7 +176,7 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
   const int ws_h = uni_i(M::window(gh, g.bin_h)), ws_w = uni_i(M::window(gw, g.bin_w));
   // A box far larger than the map (or infinite) has up to 2^31 sample points per
   // bin, nearly all outside the map: forward_large_grid does those boxes.
-  if (gh > kSearchedGrid || gw > kSearchedGrid) return;
+  if (gh > kMost || gw > kMost) return;
   const float inv_count = 1.0f / uni_f(g.count);
   MergedEntry (*const rowm)[M::LCAP] = rowm_s[wave];
   MergedEntry (*const colm)[M::LCAP] = colm_s[wave];
@@ -191,18 +194,26 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
   const __amdgpu_buffer_rsrc_t plane = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<char*>(plane_ptr), 0, H * row_bytes - (NHWC ? cb * 128 : 0), 0x00020000);
 
+  // Of a large grid's bins only the points on the map, the windows counted from a bin's first one.
+  const bool clipped = CLIP && (gh > kSearchedGrid || gw > kSearchedGrid);
   // Lists held in LDS: rows of pooled rows row_p0 .. row_p0 + RPH - 1 for the
   // sample window starting at row_i0 (lane l builds the list of pooled row
   // row_p0 + l), columns of the pooled columns col_p0 .. col_p0 + 7 for the
   // window starting at col_i0.  With grids of up to WS points one build per
   // ROI (and block of pooled rows / columns) covers everything.
+  auto list = [&](MergedEntry* out, bool cols, int p, int i0) {
+    const float start = cols ? g.start_w : g.start_h, bin = cols ? g.bin_w : g.bin_h;
+    const int grid = cols ? gw : gh, size = cols ? W : H, window = cols ? ws_w : ws_h;
+    int first = 0, last = grid;
+    if (clipped) valid_sample_range(start, p, bin, grid, size, &first, &last);
+    return merge_axis_samples(out, start, p, bin, first + i0, min(window, last - first - i0), grid, size,
+                              cols ? px_bytes : row_bytes);
+  };
   int row_p0 = -1, row_i0 = -1;
   auto need_rows = [&](int ph, int i0) {
     if (i0 != row_i0 || ph < row_p0 || ph >= row_p0 + M::RPH) {
       row_p0 = ph; row_i0 = i0;
-      if (lane < M::RPH && ph + lane < PH)
-        rown[lane] = merge_axis_samples(rowm[lane], g.start_h, ph + lane, g.bin_h, i0, min(ws_h, gh - i0),
-                                        gh, H, row_bytes);
+      if (lane < M::RPH && ph + lane < PH) rown[lane] = list(rowm[lane], false, ph + lane, i0);
     }
   };
   int col_p0 = -1, col_i0 = -1, col_max = 0;
@@ -216,10 +227,7 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
     if (pwb != col_p0 || i0 != col_i0) {
       col_p0 = pwb; col_i0 = i0;
       int n = 0;
-      if (lane < K::PWB && pwb + lane < PW) {
-        n = merge_axis_samples(colm[lane], g.start_w, pwb + lane, g.bin_w, i0, min(ws_w, gw - i0), gw, W,
-                               px_bytes);
-      }
+      if (lane < K::PWB && pwb + lane < PW) n = list(colm[lane], true, pwb + lane, i0);
       const int own = n;
       for (int off = 4; off > 0; off >>= 1) n = max(n, __shfl_xor(n, off));
       col_max = uni_i(n);
@@ -231,12 +239,9 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
   if (image_ok) {
     static_assert(M::RPH == 8 && K::PWB == 8, "eight lanes an axis");
     const bool is_col = (lane & 8) != 0;
-    const int p = is_col ? lane & 7 : ph_first + lane, grid = is_col ? gw : gh;
+    const int p = is_col ? lane & 7 : ph_first + lane;
     int n = 0;
-    if (lane < 16 && p < (is_col ? PW : PH))
-      n = merge_axis_samples(is_col ? colm[lane & 7] : rowm[lane & 7], is_col ? g.start_w : g.start_h, p,
-                             is_col ? g.bin_w : g.bin_h, 0, min(is_col ? ws_w : ws_h, grid), grid, is_col ? W : H,
-                             is_col ? px_bytes : row_bytes);
+    if (lane < 16 && p < (is_col ? PW : PH)) n = list(is_col ? colm[lane & 7] : rowm[lane & 7], is_col, p, 0);
     if (lane < 8) rown[lane] = n;
     const int own = __shfl(n, (lane & 7) + 8);
     for (int off = 4; off > 0; off >>= 1) n = max(n, __shfl_xor(n, off));
@@ -245,12 +250,25 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
     row_p0 = ph_first; row_i0 = col_p0 = col_i0 = 0;
   }
 
+  // points of a bin that are visited
+  auto points = [&](bool cols, int p) {
+    if (!clipped) return cols ? gw : gh;
+    int first, last;
+    valid_sample_range(cols ? g.start_w : g.start_h, p, cols ? g.bin_w : g.bin_h, cols ? gw : gh, cols ? W : H, &first, &last);
+    return last - first;
+  };
   const int staged = staged_pitch<T>(rows_per_pass, PH, PW, STAGE);
   for (int ph0 = ph_first; ph0 < ph_end; ph0 += rows_per_pass) {
     const int rp = min(rows_per_pass, ph_end - ph0), seg = rp * PW, pitch = rp == PH ? seg : staged;
     for (int pwb = 0; pwb < PW; pwb += K::PWB) {
       const int pw = pwb + grp;
       const bool bin_on = pw < PW && quad_on;
+      int points_w = gw;   // of the bin with the most
+      if (clipped) {
+        points_w = points(true, min(pwb + (lane & 7), PW - 1));
+        for (int off = 4; off > 0; off >>= 1) points_w = max(points_w, __shfl_xor(points_w, off));
+        points_w = uni_i(points_w);
+      }
       // Column sums of the map rows read last: what the next pooled row begins with, where it begins with them
       // (held < 0: no row).
       constexpr int MOST = CPL == 4 ? 3 : 2;   // rows read at a time (eight channels a lane have registers for two)
@@ -269,7 +287,7 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
         for (int i = 0; i < CPL; ++i) acc[i] = 0.0f;
         if (image_ok) {
 #pragma nounroll
-          for (int iyw = 0; iyw < gh; iyw += ws_h) {
+          for (int iyw = 0, points_h = uni_i(points(false, ph)); iyw < points_h; iyw += ws_h) {
             need_rows(ph, iyw);
             const int nr = uni_i(rown[ph - row_p0]);
             // an entry a lane; the sum over a bin's points is divided by their number here (the reference divides the
@@ -283,11 +301,11 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
               for (int i = 0; i < CPL; ++i) acc[i] = fmaf(w, sum[i], acc[i]);
             };
 #pragma nounroll
-            for (int ixw = 0; ixw < gw; ixw += ws_w) {
+            for (int ixw = 0; ixw < points_w; ixw += ws_w) {
               need_cols(pwb, ixw);
               if (col_max == 0) continue;   // (no column of these eight has a point on the map)
               const MergedEntry* const clist = colm[grp];
-              if (gw > ws_w) {   // (sums over other columns)
+              if (points_w > ws_w) {   // (sums over other columns)
 #pragma unroll
                 for (int r = 0; r < MOST; ++r) held[r] = -1;
               }

@@ -73,18 +73,17 @@ forward_naive_kernel(long long n_out, const T* __restrict__ x, float scale, int 
 }
 
 // The boxes that the merged lists leave out: those whose sampling grid has more
-// than kSearchedGrid points per bin along an axis.  One wavefront per ROI (it returns at once for every other box); its lanes
-// share out the ROI's outputs and visit only the samples that can be valid.  Bound by one lane's chain of samples.  With few
-// bins across a wide map most boxes inside it are of this kind, and a fixed grid of more points makes all of them so: 400 boxes,
-// 1 x 1 pooled, adaptive, 2 x 256 x 200 x 336: 62 ms, and 660 where a wavefront looked at 64 boxes and took
-// those that it found one after the other.  Boxes of other grids pay 1 us for 6000 wavefronts that find nothing.
+// than `most` points per bin along an axis.  One wavefront per ROI (it returns at once for every other box); its lanes
+// share out the ROI's outputs and visit only the samples that can be valid.  Bound by one lane's chain of samples: for boxes
+// larger than the map only, and fixed grids of more than 64 points.  Boxes of other grids pay 1 us for 6000 wavefronts
+// that find nothing.
 // NHWC: map [N][H][W][C] and pooled tensor [R][PH][PW][C].
 template <typename T, bool NHWC>
-__device__ __forceinline__ void forward_large_grid(long long r, const T* __restrict__ x, float scale, int C, int H, int W, int PH,
+__device__ __forceinline__ void forward_large_grid(long long r, int most, const T* __restrict__ x, float scale, int C, int H, int W, int PH,
                                                   int PW, int S, const float* __restrict__ rois, T* __restrict__ y,
                                                   long long num_images) {
   const RoiGeom g = roi_geometry(rois + r * 5, scale, PH, PW, S);
-  if (g.grid_h <= kSearchedGrid && g.grid_w <= kSearchedGrid) return;
+  if (g.grid_h <= most && g.grid_w <= most) return;
   const bool image_ok = g.batch >= 0 && g.batch < num_images;
   const int bins = PH * PW;
   for (int o = threadIdx.x; o < C * bins; o += 64) {

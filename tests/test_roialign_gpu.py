@@ -889,6 +889,32 @@ def test_backward_of_a_few_boxes_in_one_launch(R, C, H, W, pooled, S, dtype, lay
         native.set_option('roialign_few_boxes', 1)
 
 
+@pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('C,H,W,pooled', [(8, 65, 3, (1, 1)), (40, 131, 7, (2, 9)), (72, 9, 200, (1, 3)), (8, 300, 300, (1, 1))])
+def test_bins_of_more_points_than_are_searched(C, H, W, pooled, dtype, layout):
+    """Bins of 64, 65, 78 and 79 points (one, two, three and four windows of a list), across either border, on a wide axis
+    beside a narrow one, boxes several times the map and beyond it."""
+    abi.set_impl('auto')
+    rng = np.random.default_rng(C + H)
+    N, scale = 2, 1.0
+    spans = [s * (pooled[0] if H > W else pooled[1]) for s in (64, 64.5, 78, 78.5, 130)]
+    boxes = [(0, 0, a, b) for a in spans for b in (5, a)] + [(-40, -40, W + 20, H + 20), (W * 0.3, -3, W * 9.0, H * 7.0),
+                                                             (-900, -900, 900, 900), (2 * W, 0, 300 * W, H), (0, 0, 2, 2)]
+    if H > W:
+        boxes = [(b[0], b[1], b[3], b[2]) if i < 10 else b for i, b in enumerate(boxes)]
+    rois = np.concatenate([rng.integers(0, N, (len(boxes), 1)), np.array(boxes)], 1).astype(np.float32)
+    x = torch.from_numpy(rng.standard_normal((N, C, H, W)).astype(np.float32)).to(dtype)
+    want = oracle.forward(x.float().numpy(), rois, pooled, scale, 0)
+    if layout == 'nhwc':
+        y = abi.forward_nhwc(x.permute(0, 2, 3, 1).contiguous().cuda(), abi.to_dev(rois), pooled, scale, 0).permute(0, 3, 1, 2)
+    else:
+        y = abi.forward(x.cuda(), abi.to_dev(rois), pooled, scale, 0)
+    # (sums of thousands of terms: FWD_TOL is of the largest result, as everywhere)
+    tol = {torch.float32: FWD_TOL, torch.float16: FP16_TOL, torch.bfloat16: 1e-2}[dtype]
+    assert_parity(y.float().cpu().numpy(), torch.from_numpy(want).to(dtype).float().numpy(), tol, 'fwd')
+
+
 @pytest.mark.parametrize('waves', [4, 12])
 @pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
