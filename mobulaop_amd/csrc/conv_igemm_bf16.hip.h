@@ -224,25 +224,31 @@ __device__ __forceinline__ void to_blocked(const BlockedJob& job, unsigned block
   const unsigned row = block / job.tiles_p;
   const int n = row / job.tiles_c, c0 = (row - n * job.tiles_c) * 64, p0 = (block - row * job.tiles_p) * 64;
   const float* in = src + static_cast<size_t>(n) * C * P;
+  // All loads first, without branches (an address for every lane: what lies past the tensor is cleared afterwards).  A guarded
+  // load each before its own store to LDS left one load in flight, four or sixteen round trips to memory a workgroup (x, dy and x
+  // of 13 x 364 x 163 x 163, 57 filters 1 x 1, one part: 403 -> 325 us, 5 TB/s; of 32 x 256 x 56 x 56, 256 filters: 87 -> 79).
+  constexpr int LOADS = VEC ? 4 : 16;
+  typename std::conditional<VEC, f32x4, float>::type v[LOADS];
+  const int lane_p = VEC ? 4 * (threadIdx.x & 15) : threadIdx.x & 63, lane_c = VEC ? threadIdx.x >> 4 : threadIdx.x >> 6;
+  const bool on_p = p0 + lane_p < P;
+  const float* const from = in + (on_p ? p0 + lane_p : 0);
+#pragma unroll
+  for (int k = 0; k < LOADS; ++k) {
+    const float* const at = from + static_cast<size_t>(min(c0 + lane_c + 64 / LOADS * k, C - 1)) * P;
+    if constexpr (VEC) v[k] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(at));
+    else v[k] = *at;
+  }
   const int shift = FORM == kHalves ? words.shift(block == 0) : 0;
   const bool left = FORM == kHalves && words.no_halves();
-  if (VEC) {
-    const int q = threadIdx.x & 15, r = threadIdx.x >> 4;   // 16 quads of pixels, 16 channels per pass
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int c = c0 + r + 16 * k, p = p0 + 4 * q;
-      f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (c < C && p < P)
-        v = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(in + static_cast<size_t>(c) * P + p));
+  for (int k = 0; k < LOADS; ++k) {
+    const int cl = lane_c + 64 / LOADS * k;
+    const bool on = on_p && c0 + cl < C;
+    if constexpr (VEC) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) tile[r + 16 * k][4 * q + i] = v[i];
-    }
-  } else {
-    const int px = threadIdx.x & 63, cr = threadIdx.x >> 6;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const int c = c0 + cr + 4 * k, p = p0 + px;
-      tile[cr + 4 * k][px] = (c < C && p < P) ? in[static_cast<size_t>(c) * P + p] : 0.0f;
+      for (int i = 0; i < 4; ++i) tile[cl][lane_p + i] = on ? v[k][i] : 0.0f;
+    } else {
+      tile[cl][lane_p] = on ? v[k] : 0.0f;
     }
   }
   __syncthreads();
