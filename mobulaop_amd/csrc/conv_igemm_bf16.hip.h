@@ -416,10 +416,10 @@ constexpr int kFarOutside = -(1 << 30);
 // Where a lane loads from.  A load instruction moves 1 KB into LDS, lane l to byte 16 * l of it: 32 rows of 32 bytes.
 // Operand functors of igemm_tile_b16:
 //   UNITS, kPixels: units of a K step; whether K runs over pixels (rows of LDS are pixels then);
-//   k_steps();
+//   k_steps(), k_steps_at(n0): of the longest sums, and of the columns from n0 on;
 //   Lane lane(m0, n0, s, wave): a lane's state before K step s; next(lane): one step on;
-//   a_buffer() / a_at(lane, unit) / a_from(lane, s, unit, m): the left operand, the lane's byte offset, and the
-//     scalar one of 32 rows from m on;
+//   a_buffer() / a_at(lane, unit) / a_from(lane, s, live, unit, m): the left operand, the lane's byte offset, and the
+//     scalar one of 32 rows from m on (of any step where it is not live: nothing is loaded);
 //   b_buffer(n0) / b_at(lane, unit) / b_from(unit): the right one, of the 32 columns of the wavefront
 //     (with the bit of kDead set: zeros; written as an or, so that no branch forms in the tile's loop);
 //   Column column(n) / store(column, m, v): where results of column n go; plain(): nothing is added to a result on
@@ -442,9 +442,12 @@ struct GatheredB16 {
   __device__ int shift() const { return static_cast<int>(weight_word[1]) + static_cast<int>(src_word[1]); }
   __host__ __device__ int k_steps() const { return g.KH * g.KW * (cpad / (16 * BLOCKS)); }
   __device__ __amdgpu_buffer_rsrc_t a_buffer() const {
-    return buffer_of_bytes(wp, static_cast<unsigned>(k_steps()) * UNITS * mpad * 32u);
+    return buffer_of_bytes(wp, static_cast<unsigned>(g.KH * g.KW * (cpad / (16 * BLOCKS))) * UNITS * mpad * 32u);
   }
-  __device__ int a_from(int s, int unit, int m) const { return ((s * UNITS + unit) * mpad + m) * 32; }
+  template <typename L>
+  __device__ int a_from(const L&, int s, bool live, int unit, int m) const { return (((live ? s : 0) * UNITS + unit) * mpad + m) * 32; }
+  __device__ int k_steps_at(int) const { return k_steps(); }
+  __host__ double mean_steps() const { return k_steps(); }
   __device__ StepCursor cursor(int s) const {
     const int taps = g.KH * g.KW, cb = s / taps, tap = s - cb * taps, kh = tap / g.KW;
     return StepCursor{__builtin_amdgcn_readfirstlane(kh), __builtin_amdgcn_readfirstlane(tap - kh * g.KW),
@@ -516,14 +519,27 @@ struct ForwardOpsB16 : GatheredB16<FORM> {
 
 // dx[img, c, ih, iw] = sum over (d, kh, kw) of W[d, c, kh, kw] * dy[img, d, oh, ow]
 // with oh * stride = ih + pad - kh * dil (and likewise for columns).
+//
+// STRIDED: columns are numbered by phases of the strides: the pixels y + i * stride_h, x + j * stride_w of all images, made up
+// to whole tiles, then those of the next phase.  They meet the same taps (every dkh'th row of the filter from kh on, every
+// dkw'th column from kw on, none at worst), at dy's pixels i + oy - t * ch, j + ox - u * cw, so K runs over these alone and a
+// strided product costs what its output pixels do.  (With all taps for every pixel and zeros where one falls between output
+// pixels, and now: 96 filters 5 x 5 at stride 2 over 19 x 64 x 196 x 182, one part, 339 and 148 us; both gradients of 80 over 17 x
+// 96 x 130 x 175, two parts, 622 and 355, of 120 over 1 x 214 x 175 x 217, one part, 167 and 81.)  Unit strides would be one
+// phase with all taps; in the one code for both they took 2 to 4 % more.
+constexpr int kMostPhases = 16;   // products of larger strides take all taps (phases == 0)
+struct PhaseOfDx { int first, rows, cols, y, x, kh, kw, nkh, nkw, oy, ox; };   // first: column; rows x cols pixels of an image
+struct PhaseSteps { int dkh, dkw, ch, cw; };
+template <int FORM, bool STRIDED>
+struct BackwardDataOpsB16;
+
 template <int FORM>
-struct BackwardDataOpsB16 : GatheredB16<FORM> {
+struct BackwardDataOpsB16<FORM, false> : GatheredB16<FORM> {
   using Base = GatheredB16<FORM>;
   using Base::g; using Base::M; using Base::Ncols; using Base::cpad;
   float* __restrict__ dx; int accumulate;
   struct Lane { StepCursor k; int anchor, ihp, iwp; };   // (a column past the last: ihp far outside)
   struct Column { float* p; bool ok; };
-  __device__ bool unit_stride() const { return g.stride_h == 1 && g.stride_w == 1; }
   __device__ int plane_bytes() const { return g.OH * g.OW * 32; }
   __device__ int image_bytes() const { return plane_bytes() * (cpad / 16); }
   __device__ __amdgpu_buffer_rsrc_t b_buffer(int n0) const {
@@ -535,16 +551,111 @@ struct BackwardDataOpsB16 : GatheredB16<FORM> {
     Lane l;
     l.k = Base::cursor(s);
     l.ihp = n < Ncols ? ih + g.pad_h : kFarOutside; l.iwp = iw + g.pad_w;
-    // stride 1: byte offset of dy[img, block 0, ihp, iwp]; otherwise of dy[img, block 0, 0, 0]
-    l.anchor = (img - first) * image_bytes() + (unit_stride() ? (l.ihp * g.OW + l.iwp) * 32 : 0) + lane_chunk() * 16;
+    // byte offset of dy[img, block 0, ihp, iwp]
+    l.anchor = (img - first) * image_bytes() + (l.ihp * g.OW + l.iwp) * 32 + lane_chunk() * 16;
     return l;
   }
   __device__ void next(Lane& l) const { Base::advance(l.k); }
   __device__ int a_at(const Lane&, int) const { return lane_row() * 32 + lane_chunk() * 16; }
-  __device__ int b_at(const Lane& l, int) const {
+  __device__ int b_at(const Lane& l, int) const {   // the tap's offset from the anchor pixel (ih + pad, iw + pad) of dy
     const int dh = l.k.kh * g.dil_h, dw = l.k.kw * g.dil_w, th = l.ihp - dh, tw = l.iwp - dw;
+    const bool in = (static_cast<unsigned>(th) < static_cast<unsigned>(g.OH)) &
+                    (static_cast<unsigned>(tw) < static_cast<unsigned>(g.OW));
+    return (l.anchor + l.k.cb * Base::BLOCKS * plane_bytes() - (dh * g.OW + dw) * 32) | (in ? 0 : kDead);
+  }
+  __device__ int b_from(int unit) const { return unit * (FORM == 1 ? plane_bytes() : Base::source_part); }
+  __device__ Column column(int n) const {
+    const int hw = g.H * g.W, img = n / hw, r = n - img * hw;
+    return Column{dx + static_cast<size_t>(img) * g.C * hw + r, n < Ncols};
+  }
+  __device__ bool plain() const { return !accumulate; }
+  __device__ size_t row_pitch() const { return static_cast<size_t>(g.H) * g.W; }
+  __device__ void store(const Column& c, int m, float v) const {
+    if (m >= M || !c.ok) return;
+    float* p = c.p + static_cast<size_t>(m) * (g.H * g.W);
+    *p = accumulate ? *p + v : v;
+  }
+};
+
+template <int FORM>
+struct BackwardDataOpsB16<FORM, true> : GatheredB16<FORM> {
+  using Base = GatheredB16<FORM>;
+  using Base::g; using Base::M; using Base::Ncols; using Base::cpad; using Base::mpad;
+  float* __restrict__ dx; int accumulate;
+  int phases; PhaseSteps by; PhaseOfDx phase[kMostPhases];
+  struct Cursor { int kh, kw, cb, step; };   // tap of the phase, channel block, step of the weights
+  struct Lane { Cursor k; int nkh, nkw, anchor, ihp, iwp; };   // (a column past the last: ihp far outside)
+  struct Column { float* p; bool ok; };
+  __host__ __device__ int blocks_of_k() const { return cpad / (16 * Base::BLOCKS); }
+  // K steps of the phase with most taps, and of the one that column n0 lies in
+  __host__ __device__ int k_steps() const { return phases == 0 ? Base::k_steps() : phase[0].nkh * phase[0].nkw * blocks_of_k(); }
+  __host__ double mean_steps() const {   // of a column
+    double sum = 0.0;
+    for (int f = 0; f < phases; ++f) sum += static_cast<double>(phase[f].nkh) * phase[f].nkw * phase[f].rows * phase[f].cols;
+    return phases == 0 ? k_steps() : sum * blocks_of_k() / (static_cast<double>(g.H) * g.W);
+  }
+  __device__ int phase_of(int n) const {   // (the same for a wavefront: phases are whole tiles)
+    n = __builtin_amdgcn_readfirstlane(n);
+    int f = 0;
+    while (f + 1 < phases && n >= phase[f + 1].first) ++f;
+    return f;
+  }
+  __device__ int k_steps_at(int n0) const {
+    if (phases == 0) return Base::k_steps();
+    const PhaseOfDx& f = phase[phase_of(n0)];
+    return f.nkh * f.nkw * blocks_of_k();
+  }
+  __device__ int plane_bytes() const { return g.OH * g.OW * 32; }
+  __device__ int image_bytes() const { return plane_bytes() * (cpad / 16); }
+  __device__ int first_image(int n0) const {
+    if (phases == 0) return n0 / (g.H * g.W);
+    const PhaseOfDx& f = phase[phase_of(n0)];
+    return (n0 - f.first) / (f.rows * f.cols);
+  }
+  __device__ __amdgpu_buffer_rsrc_t b_buffer(int n0) const {
+    return Base::images_from(__builtin_amdgcn_readfirstlane(first_image(n0)), image_bytes());
+  }
+  __device__ Lane lane(int, int n0, int s, int wave) const {
+    const int n = n0 + 32 * wave + lane_row();
+    Lane l;
+    if (phases == 0) {
+      const int hw = g.H * g.W, first = n0 / hw, img = n / hw, r = n - img * hw, ih = r / g.W, iw = r - ih * g.W;
+      l.nkh = g.KH; l.nkw = g.KW;
+      const StepCursor k = Base::cursor(s);
+      l.k = Cursor{k.kh, k.kw, k.cb, s};
+      l.ihp = n < Ncols ? ih + g.pad_h : kFarOutside; l.iwp = iw + g.pad_w;
+      l.anchor = (img - first) * image_bytes() + lane_chunk() * 16;   // of dy[img, block 0, 0, 0]
+      return l;
+    }
+    const PhaseOfDx& f = phase[phase_of(n0)];
+    const int hw = f.rows * f.cols, at = n - f.first, img = at / hw, r = at - img * hw, i = r / f.cols, j = r - i * f.cols;
+    const int taps = max(f.nkh * f.nkw, 1), cb = s / taps, tap = s - cb * taps, kh = tap / max(f.nkw, 1), kw = tap - kh * f.nkw;
+    l.nkh = f.nkh; l.nkw = f.nkw;
+    l.k = Cursor{__builtin_amdgcn_readfirstlane(kh), __builtin_amdgcn_readfirstlane(kw), __builtin_amdgcn_readfirstlane(cb),
+                 __builtin_amdgcn_readfirstlane((cb * g.KH + f.kh + kh * by.dkh) * g.KW + f.kw + kw * by.dkw)};
+    l.ihp = img < g.N ? i + f.oy : kFarOutside; l.iwp = j + f.ox;
+    l.anchor = (img - first_image(n0)) * image_bytes() + (l.ihp * g.OW + l.iwp) * 32 + lane_chunk() * 16;
+    return l;
+  }
+  __device__ void next(Lane& l) const {
+    l.k.step += by.dkw;
+    if (++l.k.kw == l.nkw) {
+      l.k.kw = 0;
+      l.k.step += by.dkh * g.KW - l.nkw * by.dkw;
+      if (++l.k.kh == l.nkh) {
+        l.k.kh = 0; ++l.k.cb;
+        l.k.step += (g.KH - l.nkh * by.dkh) * g.KW;
+      }
+    }
+  }
+  __device__ int a_at(const Lane&, int) const { return lane_row() * 32 + lane_chunk() * 16; }
+  __device__ int a_from(const Lane& l, int, bool live, int unit, int m) const {
+    return (((live ? l.k.step : 0) * Base::UNITS + unit) * mpad + m) * 32;
+  }
+  __device__ int b_at(const Lane& l, int) const {
+    const int dh = l.k.kh * by.ch, dw = l.k.kw * by.cw, th = l.ihp - dh, tw = l.iwp - dw;
     const int block = l.k.cb * Base::BLOCKS * plane_bytes();
-    if (unit_stride()) {   // the tap's offset from the anchor pixel (ih + pad, iw + pad) of dy
+    if (phases != 0) {   // the tap's offset from the anchor
       const bool in = (static_cast<unsigned>(th) < static_cast<unsigned>(g.OH)) &
                       (static_cast<unsigned>(tw) < static_cast<unsigned>(g.OW));
       return (l.anchor + block - (dh * g.OW + dw) * 32) | (in ? 0 : kDead);
@@ -556,8 +667,13 @@ struct BackwardDataOpsB16 : GatheredB16<FORM> {
   }
   __device__ int b_from(int unit) const { return unit * (FORM == 1 ? plane_bytes() : Base::source_part); }
   __device__ Column column(int n) const {
-    const int hw = g.H * g.W, img = n / hw, r = n - img * hw;
-    return Column{dx + static_cast<size_t>(img) * g.C * hw + r, n < Ncols};
+    if (phases == 0) {
+      const int hw = g.H * g.W, img = n / hw, r = n - img * hw;
+      return Column{dx + static_cast<size_t>(img) * g.C * hw + r, n < Ncols};
+    }
+    const PhaseOfDx& f = phase[phase_of(n)];
+    const int hw = f.rows * f.cols, at = n - f.first, img = at / hw, r = at - img * hw, i = r / f.cols, j = r - i * f.cols;
+    return Column{dx + (static_cast<size_t>(img) * g.C * g.H + f.y + i * g.stride_h) * g.W + f.x + j * g.stride_w, img < g.N};
   }
   __device__ bool plain() const { return !accumulate; }
   __device__ size_t row_pitch() const { return static_cast<size_t>(g.H) * g.W; }
@@ -589,6 +705,8 @@ struct WeightGradOpsB16 {
   struct Lane { Pixel p[PIXELS]; int a, b, dh, dw; };   // (a column past the last: dh far outside)
   struct Column { float* p; bool ok; };
   __host__ __device__ int k_steps() const { return (g.N * g.OH * g.OW + STEP - 1) / STEP; }
+  __device__ int k_steps_at(int) const { return k_steps(); }
+  __host__ double mean_steps() const { return k_steps(); }
   __device__ int dy_set() const { return g.N * dblocks * g.OH * g.OW * 32; }
   __device__ int x_set() const { return g.N * cblocks * g.H * g.W * 32; }
   __device__ __amdgpu_buffer_rsrc_t a_buffer() const { return buffer_of_bytes(dys, static_cast<unsigned>(PARTS) * dy_set()); }
@@ -628,7 +746,7 @@ struct WeightGradOpsB16 {
     return (l.a + ((p.n * dblocks * g.OH + p.oh) * g.OW + p.ow) * 32) | (p.n < g.N ? 0 : kDead);
   }
   // (rows past the last block are the next image's or zeros, and not stored)
-  __device__ int a_from(int, int unit, int m) const { return m / 16 * (g.OH * g.OW * 32) + (PIXELS == 2 ? 0 : unit * dy_set()); }
+  __device__ int a_from(const Lane&, int, bool, int unit, int m) const { return m / 16 * (g.OH * g.OW * 32) + (PIXELS == 2 ? 0 : unit * dy_set()); }
   __device__ int b_at(const Lane& l, int unit) const {
     const Pixel p = pixel(l, unit);
     const int ih = p.oh * g.stride_h + l.dh, iw = p.ow * g.stride_w + l.dw;
@@ -713,7 +831,7 @@ struct StageB16 {
 };
 
 // C[M, Ncols] = A[M, K] x B[K, Ncols], the tile of shape S at (m0, n0) over the K steps
-// s_begin .. s_end - 1 (s_begin < s_end).  piece == nullptr: results go through ops.store;
+// s_begin .. s_end - 1.  piece == nullptr: results go through ops.store;
 // otherwise into the dense ROWS x 256 piece.  lds: S::STAGES stages.
 template <typename Ops, typename S>
 __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, int s_begin, int s_end,
@@ -744,7 +862,7 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
       const int mine = past ? 0 : piece_a, unit = mine / (ROWS / 32), group = mine % (ROWS / 32);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(a_buf, base + piece_a * 512, 16,
                                                ops.a_at(state, unit) | dead | (past ? kDead : 0),
-                                               ops.a_from(s_issue < s_end ? s_issue : 0, unit, m0 + 32 * group), 0, 0);
+                                               ops.a_from(state, s_issue, s_issue < s_end, unit, m0 + 32 * group), 0, 0);
     } else {
       const int unit = k - A_LOADS;
       if (unit == 0 || (Ops::kPixels && Ops::FORM == 1)) b_off = ops.b_at(state, unit) | dead;
@@ -980,7 +1098,7 @@ __device__ __forceinline__ void igemm_block_b16(const Ops& ops, const TilesB16& 
   if (Ops::FORM == kHalves ? !tiles.range.halves_hold() : tiles.range.leaves_split()) return;
   const TileSplit& split = tiles.split;
   const int whole_blocks = tile_blocks(split.whole);
-  int t, s_begin = 0, s_end = ops.k_steps();
+  int t, s_begin = 0, s_end = 1 << 30;
   float* piece = nullptr;
   if (block < whole_blocks) {
     t = tile_of_block(split.whole, block);
@@ -989,11 +1107,12 @@ __device__ __forceinline__ void igemm_block_b16(const Ops& ops, const TilesB16& 
     const int q = block - whole_blocks;
     t = split.whole + q / split.pieces;
     s_begin = (q % split.pieces) * split.steps_per_piece;
-    s_end = min(s_end, s_begin + split.steps_per_piece);
+    s_end = s_begin + split.steps_per_piece;
     piece = tiles.piece_buffer + static_cast<size_t>(q) * S::ROWS * S::COLS;
   }
   const int m0 = (t % tiles.row_tiles) * S::ROWS, n0 = (t / tiles.row_tiles) * S::COLS;
-  igemm_tile_b16<Ops, S>(ops, m0, n0, s_begin, s_end, piece, lds);
+  s_end = min(s_end, ops.k_steps_at(n0));
+  igemm_tile_b16<Ops, S>(ops, m0, n0, s_begin, s_end, piece, lds);   // (no steps: zeros)
 }
 template <typename Ops, typename S>
 __global__ void __launch_bounds__(64 * S::WAVES, 2 * S::PER_CU) igemm_b16_kernel(Ops ops, TilesB16 tiles) {
@@ -1004,13 +1123,13 @@ __global__ void __launch_bounds__(64 * S::WAVES, 2 * S::PER_CU) igemm_b16_kernel
 // the last round of one is filled up by the other.  The first's workgroups are made up to a multiple of eight, so that the
 // other's keep their XCDs.  5 x 96 x 45 x 67, 130 filters 3 x 3, two parts: 22 + 25 us -> 43; 32 x 256 x 56 x 56, 256 filters,
 // halves: 335 + 325 -> 659, one part: 134 + 129 -> 257.
-template <int FORM, typename S>
+template <int FORM, bool STRIDED, typename S>
 __global__ void __launch_bounds__(64 * S::WAVES, 2 * S::PER_CU)
-igemm_gradients_b16_kernel(WeightGradOpsB16<FORM> weight, TilesB16 weight_tiles, BackwardDataOpsB16<FORM> data,
+igemm_gradients_b16_kernel(WeightGradOpsB16<FORM> weight, TilesB16 weight_tiles, BackwardDataOpsB16<FORM, STRIDED> data,
                            TilesB16 data_tiles) {
   __shared__ __attribute__((aligned(1024))) unsigned short lds[S::STAGES * StageB16<FORM, S>::HALVES];
   const int first = (weight_tiles.blocks + 7) / 8 * 8, block = blockIdx.x;
-  if (block >= first) igemm_block_b16<BackwardDataOpsB16<FORM>, S>(data, data_tiles, block - first, lds);
+  if (block >= first) igemm_block_b16<BackwardDataOpsB16<FORM, STRIDED>, S>(data, data_tiles, block - first, lds);
   else if (block < weight_tiles.blocks) igemm_block_b16<WeightGradOpsB16<FORM>, S>(weight, weight_tiles, block, lds);
 }
 
@@ -1256,9 +1375,9 @@ struct DataFp32Job { BackwardDataOps ops; PiecesF32 pieces; unsigned blocks; };
 __device__ __forceinline__ void run_job(const DataFp32Job& job, unsigned block, float*) {
   reduce_pieces_f32(job.ops, job.pieces, block);
 }
-template <int FORM, typename Job>
+template <int FORM, bool STRIDED, typename Job>
 __global__ void __launch_bounds__(256)
-reduce_gradients_b16_kernel(BackwardDataOpsB16<FORM> data, PiecesB16 data_pieces, WeightGradOpsB16<FORM> weight,
+reduce_gradients_b16_kernel(BackwardDataOpsB16<FORM, STRIDED> data, PiecesB16 data_pieces, WeightGradOpsB16<FORM> weight,
                             PiecesB16 weight_pieces, BiasJob bias, Job job) {
   __shared__ __attribute__((aligned(16))) float lds[std::is_same<Job, AgainJob>::value ? kPrepLdsWords : 4];
   unsigned block = blockIdx.x;

@@ -8,6 +8,7 @@
 // (opzoo/Convolution/Convolution.py:17-57), computed on the matrix cores
 // without a column buffer.
 #include <algorithm>
+#include <numeric>
 #include <type_traits>
 #include <vector>
 
@@ -128,14 +129,14 @@ conv::TileSplit split_b16(const Ops& ops, double* cost) {
   // stages and write results
   const double base = Ops::FORM == 1 ? 0.97 : 1.1;
   const double step = Ops::FORM == conv::kHalves ? 1.41 * (S::ROWS + 20) / 276.0 : Ops::FORM == 3 ? 2.24 * (S::ROWS + 20) / 276.0 : base * (S::ROWS + (S::PER_CU == 2 ? 40 : 64)) / 320.0;
-  auto time = [&](int workgroups, int length) {
+  auto time = [&](int workgroups, double length) {
     return step * (length + 2) * (workgroups <= cus && S::PER_CU == 2 ? 1.33 : static_cast<double>((workgroups + cus - 1) / cus));
   };
   const conv::TileSplit whole{count, 1, steps}, cut = split_tiles(count, steps, resident, room);
-  const double whole_time = time(count, steps);
+  const double whole_time = time(count, ops.mean_steps());
   const int rest = count - cut.whole, pieces = rest * cut.pieces;
   // pieces are written and read again at some 4 TB/s, and added up by a kernel of their own
-  const double cut_time = (cut.whole > 0 ? time(cut.whole, steps) : 0.0) + time(pieces, cut.steps_per_piece) +
+  const double cut_time = (cut.whole > 0 ? time(cut.whole, ops.mean_steps()) : 0.0) + time(pieces, cut.steps_per_piece) +
                           static_cast<double>(pieces) * S::ROWS * S::COLS * 8 / 4e6 + 5.0;
   const bool cut_wins = rest > 0 && cut_time < whole_time;
   if (cost != nullptr) *cost = cut_wins ? cut_time : whole_time;
@@ -428,9 +429,64 @@ struct ForwardB16 {
   }
 };
 
+// The phases of a data gradient's columns (conv::BackwardDataOpsB16), those with most taps first; returns the pixels of an
+// image in the smallest.
 template <int FORM>
+int plan_phases(conv::BackwardDataOpsB16<FORM, false>* data, const conv::Geometry& g) {
+  data->Ncols = g.N * g.H * g.W;
+  return g.H * g.W;
+}
+template <int FORM>
+int plan_phases(conv::BackwardDataOpsB16<FORM, true>* data, const conv::Geometry& g) {
+  const int sh = g.stride_h, sw = g.stride_w;
+  data->phases = 0;
+  data->by = conv::PhaseSteps{1, 1, g.dil_h, g.dil_w};
+  data->Ncols = g.N * g.H * g.W;
+  const long long columns = static_cast<long long>(g.N) * g.H * g.W + conv::kMostPhases * 256;
+  // (a single tap: nothing to leave out but zeros, whose pixels are then written apart from their neighbours; 106 filters 1 x 1
+  // at stride 2 over 17 x 142 x 61 x 74, two parts, the step 111.9 us and 113.3)
+  if (static_cast<long long>(sh) * sw > conv::kMostPhases || columns >= (1ll << 31) || g.KH * g.KW == 1) return g.H * g.W;
+  data->by = conv::PhaseSteps{sh / std::gcd(sh, g.dil_h), sw / std::gcd(sw, g.dil_w), g.dil_h / std::gcd(sh, g.dil_h),
+                              g.dil_w / std::gcd(sw, g.dil_w)};
+  // of the taps along an axis that meet the pixels at `at` the first, and how many there are
+  auto taps = [](int at, int pad, int dil, int stride, int step, int K, int* first) {
+    for (int k = 0; k < std::min(step, K); ++k)
+      if ((at + pad - k * dil) % stride == 0) { *first = k; return (K - k + step - 1) / step; }
+    *first = 0;
+    return 0;
+  };
+  std::vector<conv::PhaseOfDx> all;
+  for (int y = 0; y < std::min(sh, g.H); ++y)
+    for (int x = 0; x < std::min(sw, g.W); ++x) {
+      conv::PhaseOfDx f{};
+      f.y = y; f.x = x; f.rows = (g.H - y + sh - 1) / sh; f.cols = (g.W - x + sw - 1) / sw;
+      f.nkh = taps(y, g.pad_h, g.dil_h, sh, data->by.dkh, g.KH, &f.kh);
+      f.nkw = taps(x, g.pad_w, g.dil_w, sw, data->by.dkw, g.KW, &f.kw);
+      if (f.nkh == 0 || f.nkw == 0) f.nkh = f.nkw = 0;
+      f.oy = (y + g.pad_h - f.kh * g.dil_h) / sh; f.ox = (x + g.pad_w - f.kw * g.dil_w) / sw;
+      all.push_back(f);
+    }
+  std::stable_sort(all.begin(), all.end(),
+                   [](const conv::PhaseOfDx& a, const conv::PhaseOfDx& b) { return a.nkh * a.nkw > b.nkh * b.nkw; });
+  int least = g.H * g.W;
+  for (const conv::PhaseOfDx& f : all) least = std::min(least, f.rows * f.cols);
+  // (a tile spans more images where phases have few pixels of each: their byte offsets must stay below 2^31, see plan_gather_b16)
+  const long long image_bytes = static_cast<long long>(g.OH) * g.OW * padded_channels<FORM>(g.D) * 2;
+  if ((255 / least + 2 + (conv::kParts<FORM> > 1 ? static_cast<long long>(conv::kParts<FORM>) * g.N : 0)) * image_bytes >= (1ll << 31))
+    return g.H * g.W;
+  int at = 0;
+  for (conv::PhaseOfDx f : all) {
+    f.first = at;
+    data->phase[data->phases++] = f;
+    at += (g.N * f.rows * f.cols + 255) / 256 * 256;
+  }
+  data->Ncols = at;
+  return least;
+}
+
+template <int FORM, bool STRIDED>
 struct BackwardB16 {
-  conv::BackwardDataOpsB16<FORM> data;
+  conv::BackwardDataOpsB16<FORM, STRIDED> data;
   conv::WeightGradOpsB16<FORM> weight;
   PrepB16 prep;
   size_t dy_bytes, x_bytes;
@@ -457,9 +513,10 @@ struct BackwardB16 {
       if (k + 4 * step >= (1ll << 31)) return kOther;   // (pixels past the last are counted too)
     }
     if (!with_dx) return kFits;
-    data.dx = dx; data.accumulate = accumulate; data.Ncols = g.N * g.H * g.W;
+    data.dx = dx; data.accumulate = accumulate;
+    const int least = plan_phases(&data, g);
     // row m of the left operand is input channel m: element [m][tap][d] = weight[d][m][tap]
-    return plan_gather_b16<FORM>(&data, &prep, "conv2d_backward_data", g, w, g.C, g.D, g.N, g.OH * g.OW, g.H * g.W, taps,
+    return plan_gather_b16<FORM>(&data, &prep, "conv2d_backward_data", g, w, g.C, g.D, g.N, g.OH * g.OW, least, taps,
                                   g.C * taps);
   }
   char* place(char* at) {
@@ -962,19 +1019,19 @@ bool forward_b16(const conv::Geometry& g, const float* x, const float* weight, c
 // after the other; what is left of them for one kernel behind.
 template <int FORM>
 struct GradientPieces { conv::PiecesB16 data{}, weight{}; };
-template <int FORM, int ROWS>
-bool launch_together(const BackwardB16<FORM>& b, int rows, float* first, float* second, hipStream_t stream,
+template <int FORM, int ROWS, bool STRIDED>
+bool launch_together(const BackwardB16<FORM, STRIDED>& b, int rows, float* first, float* second, hipStream_t stream,
                      conv::SplitRange data_range, conv::SplitRange weight_range, GradientPieces<FORM>* pieces) {
   if (rows != ROWS) return false;
   using S = conv::ShapeB16<ROWS, FORM>;
-  const conv::TilesB16 data = tiles_b16<conv::BackwardDataOpsB16<FORM>, S>(b.data, first, data_range, &pieces->data);
+  const conv::TilesB16 data = tiles_b16<conv::BackwardDataOpsB16<FORM, STRIDED>, S>(b.data, first, data_range, &pieces->data);
   const conv::TilesB16 weight = tiles_b16<conv::WeightGradOpsB16<FORM>, S>(b.weight, second, weight_range, &pieces->weight);
   const int blocks = conv::tile_blocks(weight.blocks) + data.blocks;
-  conv::igemm_gradients_b16_kernel<FORM, S><<<blocks, 64 * S::WAVES, 0, stream>>>(b.weight, weight, b.data, data);
+  conv::igemm_gradients_b16_kernel<FORM, STRIDED, S><<<blocks, 64 * S::WAVES, 0, stream>>>(b.weight, weight, b.data, data);
   return true;
 }
-template <int FORM>
-GradientPieces<FORM> launch_gradients_b16(const BackwardB16<FORM>& b, char* piece_buffers, hipStream_t stream,
+template <int FORM, bool STRIDED>
+GradientPieces<FORM> launch_gradients_b16(const BackwardB16<FORM, STRIDED>& b, char* piece_buffers, hipStream_t stream,
                                           conv::SplitRange data_range = {}, conv::SplitRange weight_range = {}) {
   float* const first = reinterpret_cast<float*>(piece_buffers);
   float* const second = b.with_dx ? first + kPieceBytes / sizeof(float) : first;
@@ -995,20 +1052,20 @@ GradientPieces<FORM> launch_gradients_b16(const BackwardB16<FORM>& b, char* piec
   return pieces;
 }
 // The pieces of both, the bias's sums and another job.
-template <int FORM, typename Job>
-void reduce_gradients_b16(const BackwardB16<FORM>& b, const GradientPieces<FORM>& pieces, const conv::BiasJob& bias, const Job& job,
+template <int FORM, bool STRIDED, typename Job>
+void reduce_gradients_b16(const BackwardB16<FORM, STRIDED>& b, const GradientPieces<FORM>& pieces, const conv::BiasJob& bias, const Job& job,
                           hipStream_t stream) {
   const unsigned blocks = pieces.data.blocks + pieces.weight.blocks + bias.total_blocks + job.blocks;
   if (blocks > 0)
-    conv::reduce_gradients_b16_kernel<FORM, Job><<<blocks, 256, 0, stream>>>(b.data, pieces.data, b.weight, pieces.weight, bias, job);
+    conv::reduce_gradients_b16_kernel<FORM, STRIDED, Job><<<blocks, 256, 0, stream>>>(b.data, pieces.data, b.weight, pieces.weight, bias, job);
 }
 
 // The gradients that are wanted (null: not; the bias's only beside another).  dx and dw share the copy of dy; where the
 // workspace cannot hold what both need the caller takes one after the other.
-template <int PARTS>
-bool gradients_b16(const conv::Geometry& g, const float* dy, const float* x, const float* weight, int accumulate,
+template <int PARTS, bool STRIDED>
+bool gradients_b16_of(const conv::Geometry& g, const float* dy, const float* x, const float* weight, int accumulate,
                    float* dx, float* dw, float** db, hipStream_t stream) {
-  BackwardB16<PARTS> b;
+  BackwardB16<PARTS, STRIDED> b;
   const Fit fit = b.plan(g, dy, x, weight, accumulate, dx, dw);
   if (fit != kFits) return fit == kError;
   const bool both = dx != nullptr && dw != nullptr;
@@ -1018,9 +1075,17 @@ bool gradients_b16(const conv::Geometry& g, const float* dy, const float* x, con
   const conv::BiasJob bias = take_bias(g, dy, db, bias_room, ws);
   char* const pieces = b.place(ws + bias_room);
   b.prep.template launch<PARTS>(stream, {}, bias);
-  reduce_gradients_b16<PARTS>(b, launch_gradients_b16<PARTS>(b, pieces, stream), bias, conv::NoJob{0}, stream);
+  reduce_gradients_b16(b, launch_gradients_b16(b, pieces, stream), bias, conv::NoJob{0}, stream);
   MOBULA_HIP_TRY(hipGetLastError());
   return true;
+}
+// (the strides matter to the data gradient's tiles alone)
+bool strided(const conv::Geometry& g, const float* dx) { return dx != nullptr && (g.stride_h != 1 || g.stride_w != 1); }
+template <int PARTS>
+bool gradients_b16(const conv::Geometry& g, const float* dy, const float* x, const float* weight, int accumulate,
+                   float* dx, float* dw, float** db, hipStream_t stream) {
+  return (strided(g, dx) ? gradients_b16_of<PARTS, true> : gradients_b16_of<PARTS, false>)(g, dy, x, weight, accumulate, dx, dw,
+                                                                                           db, stream);
 }
 
 // ---- fp32 products from parts: three bf16 or two fp16 per operand ----------------------------
@@ -1185,10 +1250,11 @@ bool forward_split(const conv::Geometry& g, const float* x, const float* weight,
 }
 
 // The gradients that are wanted (null: not; the bias's only beside another), from `form`.
-bool gradients_split(int form, const conv::Geometry& g, const float* dy, const float* x, const float* weight,
-                     int accumulate, float* dx, float* dw, float** db, hipStream_t stream) {
-  BackwardB16<3> parts;
-  BackwardB16<conv::kHalves> halves;
+template <bool STRIDED>
+bool gradients_split_of(int form, const conv::Geometry& g, const float* dy, const float* x, const float* weight,
+                        int accumulate, float* dx, float* dw, float** db, hipStream_t stream) {
+  BackwardB16<3, STRIDED> parts;
+  BackwardB16<conv::kHalves, STRIDED> halves;
   GatherPlan plan{};
   WeightPlan weight_plan{};
   const long long taps = g.KH * g.KW;
@@ -1229,9 +1295,9 @@ bool gradients_split(int form, const conv::Geometry& g, const float* dy, const f
     halves.place(at);
     const conv::MagnitudeJob job{{dy, x, weight}, {dy_count, x_count, w_count}, {dy_words, x_words, w_words}};
     conv::magnitudes_kernel<<<dim3(conv::kMagnitudes, 3), 1024, 0, stream>>>(job);
-    halves.prep.launch<conv::kHalves>(stream, words, bias);
-    const auto left = launch_gradients_b16<conv::kHalves>(halves, pieces, stream, data_range, weight_range);
-    reduce_gradients_b16<conv::kHalves>(
+    halves.prep.template launch<conv::kHalves>(stream, words, bias);
+    const auto left = launch_gradients_b16(halves, pieces, stream, data_range, weight_range);
+    reduce_gradients_b16(
         halves, left, bias,
         again_job(parts.prep, words, plan.tables, taps_of_weight, dx != nullptr ? data_range : weight_range,
                   dx != nullptr && dw != nullptr ? weight_range : conv::SplitRange{}), stream);
@@ -1240,24 +1306,30 @@ bool gradients_split(int form, const conv::Geometry& g, const float* dy, const f
     conv::odd_values_kernel<conv::kData, conv::kWeight><<<odd_dx.blocks + odd_dw.blocks, 256, 0, stream>>>(odd_dx, odd_dw);
   } else {
     conv::clear_words_kernel<<<1, 64, 0, stream>>>(reinterpret_cast<unsigned*>(ws), 12);
-    parts.prep.launch<3>(stream, words, bias);
+    parts.prep.template launch<3>(stream, words, bias);
     if (dx != nullptr) build_gather(&plan, tables, stream, data_range);
   }
   // (the fp32 product's pieces may lie where the parts' product's do: one of the two is not formed)
-  const auto left = launch_gradients_b16<3>(parts, pieces, stream, data_range, weight_range);
+  const auto left = launch_gradients_b16(parts, pieces, stream, data_range, weight_range);
   conv::DataFp32Job data{};
   if (dx != nullptr) {
     conv::BackwardDataOps& ops = data.ops;
-    ops.dy = dy; ops.dx = dx; ops.g = g; ops.accumulate = accumulate; ops.M = g.C; ops.Ncols = parts.data.Ncols;
+    ops.dy = dy; ops.dx = dx; ops.g = g; ops.accumulate = accumulate; ops.M = g.C; ops.Ncols = g.N * g.H * g.W;
     ops.wp = plan.tables.out; ops.steps = plan.tables.steps; ops.K = plan.K;
     data.pieces = launch_igemm_pieces<conv::BackwardDataOps, conv::kFp32>(ops, reinterpret_cast<float*>(pieces), data_range, stream);
     data.blocks = data.pieces.blocks;
   }
-  reduce_gradients_b16<3>(parts, left, by_halves ? conv::BiasJob{} : bias, data, stream);
+  reduce_gradients_b16(parts, left, by_halves ? conv::BiasJob{} : bias, data, stream);
   if (dw != nullptr)
     run_weight(weight_plan, g, dy, x, accumulate, dw, at, stream, weight_range, by_halves ? built_taps : nullptr);
   MOBULA_HIP_TRY(hipGetLastError());
   return true;
+}
+
+bool gradients_split(int form, const conv::Geometry& g, const float* dy, const float* x, const float* weight,
+                     int accumulate, float* dx, float* dw, float** db, hipStream_t stream) {
+  return (strided(g, dx) ? gradients_split_of<true> : gradients_split_of<false>)(form, g, dy, x, weight, accumulate, dx, dw, db,
+                                                                                 stream);
 }
 
 // Which of the wanted products split operands are faster for, and how they are formed (0: by the fp32 kernels): those of
@@ -1269,10 +1341,10 @@ struct SplitChoice { int dx, dw; };
 // What the gradients that FORM may stand for cost (< 0: it may not), and the K steps of their longest sums (parts_dx,
 // parts_dw: see short_sums).
 struct GradientCosts { double data, weight; int longest_data, longest_weight; };
-template <int FORM>
-GradientCosts gradient_costs(const conv::Geometry& g, bool dx, bool dw, int parts_dx = 0, int parts_dw = 0) {
+template <int FORM, bool STRIDED>
+GradientCosts gradient_costs_of(const conv::Geometry& g, bool dx, bool dw, int parts_dx, int parts_dw) {
   GradientCosts cost{-1.0, -1.0, 0, 0};
-  BackwardB16<FORM> b;
+  BackwardB16<FORM, STRIDED> b;
   float any;   // (for its address: nothing is written)
   if (b.plan(g, &any, &any, &any, 0, dx ? &any : nullptr, dw ? &any : nullptr) != kFits) return cost;
   if (dx && !(FORM == conv::kHalves && short_sums(b.data, parts_dx))) {
@@ -1284,6 +1356,12 @@ GradientCosts gradient_costs(const conv::Geometry& g, bool dx, bool dw, int part
     cost.weight = plan.cost; cost.longest_weight = plan.longest;
   }
   return cost;
+}
+
+template <int FORM>
+GradientCosts gradient_costs(const conv::Geometry& g, bool dx, bool dw, int parts_dx = 0, int parts_dw = 0) {
+  return (dx && (g.stride_h != 1 || g.stride_w != 1) ? gradient_costs_of<FORM, true> : gradient_costs_of<FORM, false>)(
+      g, dx, dw, parts_dx, parts_dw);
 }
 
 SplitChoice choose_split(const conv::Geometry& g, bool dx, bool dw) {

@@ -404,6 +404,57 @@ def test_bf16_mode_is_exact_on_bf16_valued_operands(case):
     _close(dx2, 2 * xr.grad, 'dx accumulated', 1e-4)
 
 
+@pytest.mark.parametrize('mode', ['bf16', 'bf16x3', 'three parts', 'halves'])
+@pytest.mark.parametrize('case', [
+    # N, C, H, W, D, kernel, pad, stride, dilation
+    (2, 70, 23, 18, 40, (3, 3), (1, 1), (2, 2), (1, 1)),    # phases of one, two and four taps
+    (3, 20, 17, 31, 33, (5, 4), (2, 0), (2, 1), (1, 1)),
+    (2, 24, 20, 19, 48, (1, 1), (0, 0), (2, 2), (1, 1)),    # a single tap: all pixels in one go
+    (2, 24, 21, 20, 48, (3, 3), (2, 1), (2, 4), (2, 1)),    # a filter of every second row: odd rows meet no tap; four phases of columns
+    (2, 17, 19, 23, 20, (3, 4), (1, 2), (3, 2), (2, 3)),    # stride and dilation without a common factor
+    (300, 16, 3, 2, 20, (2, 2), (1, 0), (4, 2), (1, 1)),    # fewer rows than phases; a tile spans hundreds of images
+    (1, 130, 40, 37, 20, (7, 7), (3, 3), (4, 4), (1, 1)),   # sixteen phases, the most
+    (2, 18, 30, 30, 20, (6, 5), (2, 2), (5, 4), (1, 1)),    # twenty: all taps
+    (1, 600, 16, 16, 600, (3, 3), (1, 1), (2, 2), (1, 1)),  # cut along K: pieces past the end of a phase's
+])
+def test_data_gradient_of_strided_products(case, mode):
+    """Every phase of the strides with its own taps, against the products of the same operands in 64 bits; what the gradient
+    is added to; an infinite weight reaches no pixels of other phases."""
+    N, C, H, W, D, k, pad, stride, dil = case
+    g = torch.Generator().manual_seed(62)
+    w = torch.randn(D, C, *k, generator=g) * 0.1
+    shape = (N, C, H, W)
+    y_shape = F.conv2d(torch.zeros(1, C, H, W), w, padding=pad, stride=stride, dilation=dil).shape
+    dy = torch.randn((N,) + y_shape[1:], generator=g)
+    rnd = (lambda t: t.bfloat16().double()) if mode == 'bf16' else (lambda t: t.double())
+    want = torch.nn.grad.conv2d_input(shape, rnd(w), rnd(dy), stride=stride, padding=pad, dilation=dil)
+    # terms are rounded to 2^-16 of an operand with two parts, sums to fp32 otherwise; of the largest result
+    tol = 2e-5 if mode == 'bf16x3' else 2e-6
+    native.set_option('conv_compute', {'bf16': 1, 'bf16x3': 2}.get(mode, 0))
+    native.set_option('conv_fp32_split', {'three parts': 2, 'halves': 3}.get(mode, 1))
+    try:
+        _leave_nan_patterns_in_the_workspace()
+        geo = _ci(N, C, H, W, D, k[0], k[1], pad[0], pad[1], stride[0], stride[1], dil[0], dil[1])
+        dyd = dy.cuda()
+
+        def run(weight, dx, accumulate):
+            _call('conv2d_backward_data_ecf81c91', ctypes.c_int(dx.numel()), _ptr(dyd), _ptr(weight), ctypes.c_int(accumulate), *geo,
+                  _ptr(dx))
+            return dx
+        wd = w.cuda()
+        dx = run(wd, torch.full(shape, float('nan'), device='cuda'), 0)
+        _close(dx, want, 'dx', tol)
+        _close(run(wd, dx.clone(), 1), 2 * want, 'dx accumulated', tol)
+        if mode == 'bf16' and stride[0] * stride[1] <= 16 and k != (1, 1):   # (its phase it meets beyond dy's border, too)
+            wd[:, :, 0, 0] = float('inf')
+            got = run(wd, torch.empty(shape, device='cuda'), 0).cpu()
+            phase = ((torch.arange(H) + pad[0]) % stride[0] == 0)[:, None] & ((torch.arange(W) + pad[1]) % stride[1] == 0)
+            assert torch.isfinite(got[:, :, ~phase]).all()
+    finally:
+        native.set_option('conv_compute', 0)
+        native.set_option('conv_fp32_split', 1)
+
+
 def test_errors_surface_as_exceptions():
     x = torch.zeros(1, 1, 4, 4, device='cuda')
     w = torch.zeros(1, 1, 3, 3, device='cuda')
