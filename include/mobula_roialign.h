@@ -331,7 +331,9 @@ void mobula_hip_clear_error(void);
  * one launch where that is faster, 0 never, 2 wherever it can (64 boxes);
  * "roialign_patch": 4 or 12 fixes the wavefronts that share a patch of the
  * gradient where sampling grids have more than two points per bin and axis, and
- * takes other grids that way too, 1 (default) chooses -- all five for tests, the
+ * takes other grids that way too, 1 (default) chooses; "roialign_tile_groups": 1
+ * or 4 fixes the workgroups that make a tile's work lists, 0 (default) chooses --
+ * all six for tests, the
  * results do not depend on them beyond the order of fp32 sums).  set returns 0, or -1 for an unknown name; get
  * returns -1 for a name never set. */
 int mobula_hip_set_option(const char* name, long long value);

@@ -287,37 +287,44 @@ __device__ __forceinline__ SortedRow sorted_row(const SortedRow* __restrict__ so
   return SortedRow{-1, 0, 0, 0};
 }
 
-// One workgroup per tile, one wavefront per tile row.
+// GROUPS workgroups per tile, each sixteen wavefronts for 16 / GROUPS of its rows, GROUPS wavefronts to a row.
 // First the tile's ROI list: every wavefront takes a sixteenth of the ROIs,
 // counts those whose box covers the tile, and after one exchange writes them,
-// in increasing ROI index, into space taken from cursors[0] with one atomic.
-// Then the work lists: lane j looks at ROI j of the tile's list, takes its taps
-// for this wavefront's row from the row-tap table, and all lanes append theirs
-// in list order.  WorkRange::count includes the padding.  Space for the tile's
-// sixteen lists comes from one bump-pointer allocation per tile (cursors[1]).
-// The order in which tiles take their space varies from run to run; what is
+// in increasing ROI index, into LDS (GROUPS == 1: or, beyond kTileListCap, into space taken from
+// cursors[0] with one atomic).  Then the work lists: a wavefront takes a run of the list, lane j looks at ROI j of it, takes its
+// taps for this wavefront's row from the row-tap table, and all lanes append theirs
+// in list order.  WorkRange::count includes the padding.  Space for a workgroup's
+// lists comes from one bump-pointer allocation (cursors[1]).
+// The order in which workgroups take their space varies from run to run; what is
 // written into it does not.
-constexpr int kTileListCap = 4096;   // items of one tile that LDS holds (longer lists go through memory)
+//
+// Bound by the chain of dependent loads, once per 64 ROIs of a tile and row and twice over: where tiles are few, four wavefronts
+// share it (GROUPS 4).
+constexpr int kTileListCap = 4096;   // ROIs of one tile that LDS holds (longer lists go through memory)
+constexpr int kSharedListCap = 8192;   // ROIs of all up to which a tile may have several workgroups
 
+template <int GROUPS>
 __global__ void __launch_bounds__(kTileRows * 64)
 build_tile_work_kernel(const TileBox* __restrict__ boxes, int R, int* __restrict__ tile_rois,
                        const AxisUnit* __restrict__ lists, TileGrid tg, ListLayout ll,
                        int* __restrict__ cursors, WorkRange* __restrict__ ranges,
                        WorkEntry* __restrict__ entries, SortedRow* __restrict__ sorted, int H) {
+  constexpr int ROWS = kTileRows / GROUPS;   // of this workgroup
   __shared__ int hits[kTileRows];
-  __shared__ int row_total[kTileRows];
+  __shared__ int taken[kTileRows];   // entries of every wavefront, with a row's padding in its last
   __shared__ int list_base, tile_base;
   // the tile's ROIs in their order: in LDS, so that the wavefronts below need not wait for memory to see the list
-  __shared__ int item_s[kTileListCap];
-  const long long tile = blockIdx.x;
-  const int lane = threadIdx.x & 63, row = threadIdx.x >> 6;
+  __shared__ int item_s[GROUPS == 1 ? kTileListCap : kSharedListCap];
+  const long long tile = blockIdx.x / GROUPS;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, part = wave % GROUPS;
+  const int row = static_cast<int>(blockIdx.x % GROUPS) * ROWS + wave / GROUPS;
   const int image = static_cast<int>(tile / tg.per_image);
   const int t = static_cast<int>(tile % tg.per_image);
   const int ty = t / tg.tx, tx = t % tg.tx;
 
-  // ---- the tile's item list ----
+  // ---- the tile's ROI list ----
   const int share = ((R + kTileRows * 64 - 1) / (kTileRows * 64)) * 64;
-  const int r_begin = row * share, r_end = min(R, r_begin + share);
+  const int r_begin = wave * share, r_end = min(R, r_begin + share);
   auto hit_of = [&](int r) {
     if (r >= r_end) return false;
     const TileBox b = boxes[r];
@@ -335,14 +342,14 @@ build_tile_work_kernel(const TileBox* __restrict__ boxes, int R, int* __restrict
     mine += __popcll(__ballot(kept_hit[k]));
   }
   for (int base = r_begin + 64 * kKept; base < r_end; base += 64) mine += __popcll(__ballot(hit_of(base + lane)));
-  if (lane == 0) hits[row] = mine;
+  if (lane == 0) hits[wave] = mine;
   __syncthreads();
   int written = 0, count = 0;
   for (int r = 0; r < kTileRows; ++r) {
-    if (r < row) written += hits[r];
+    if (r < wave) written += hits[r];
     count += hits[r];
   }
-  const bool in_lds = count <= kTileListCap;   // (the same for the whole workgroup)
+  const bool in_lds = GROUPS > 1 || count <= kTileListCap;   // (the same for the whole workgroup)
   if (!in_lds) {
     if (threadIdx.x == 0) list_base = atomicAdd(cursors, count);
     __syncthreads();
@@ -365,8 +372,8 @@ build_tile_work_kernel(const TileBox* __restrict__ boxes, int R, int* __restrict
   __syncthreads();   // the list is complete and visible to the whole workgroup
   auto item_at = [&](int i) { return in_lds ? item_s[i] : long_list[i]; };
 
-  // ---- the work lists of the sixteen rows ----
-  // taps of list item `roi` on this wavefront's tile row: where they start, how many
+  // ---- the work lists of the rows ----
+  // taps of ROI `roi` on this wavefront's tile row: where they start, how many
   auto taps_of = [&](int roi, const RowTap** taps) {
     const AxisUnit* const table = lists + static_cast<long long>(roi) * ll.roi_stride +
                                   static_cast<long long>(ty) * ll.row_stride;
@@ -375,48 +382,60 @@ build_tile_work_kernel(const TileBox* __restrict__ boxes, int R, int* __restrict
     *taps = tb->taps + (idx & 0xffu);
     return static_cast<int>(idx >> 8);
   };
-  // (what the first 64 items gave is kept for the second walk: most tiles have no more)
+  // this wavefront's run of the list: whole chunks of 64
+  const int chunks = (count + 63) / 64, begin = part * chunks / GROUPS * 64, end = min(count, (part + 1) * chunks / GROUPS * 64);
+  // (what the first 64 ROIs gave is kept for the second walk: most runs have no more)
   int total = 0, first_c = 0, first_item = 0;
   const RowTap* first_taps = nullptr;
-  for (int base = 0; base < count; base += 64) {
+  for (int base = begin; base < end; base += 64) {
     int c = 0, item = 0;
     const RowTap* taps = nullptr;
-    if (base + lane < count) {
+    if (base + lane < end) {
       item = item_at(base + lane);
       c = taps_of(item, &taps);
     }
-    if (base == 0) { first_c = c; first_item = item; first_taps = taps; }
+    if (base == begin) { first_c = c; first_item = item; first_taps = taps; }
     for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off);
     total += c;
   }
+  if (lane == 0) taken[wave] = total;
+  __syncthreads();
+  int before = 0, row_total = 0;   // entries of the row's earlier runs, of all of them
+  for (int k = 0; k < GROUPS; ++k) {
+    const int n = taken[wave - part + k];
+    before += k < part ? n : 0;
+    row_total += n;
+  }
   // Lists are padded to a multiple of eight entries (one turn of the consumer's
   // double-buffered pipeline) plus four more that it prefetches but never uses.
-  const int padded = (total + 7) & ~7;
-  const int reserved = total > 0 ? padded + 4 : 0;
-  if (lane == 0) row_total[row] = reserved;
+  const int padded = (row_total + 7) & ~7;
+  const int reserved = row_total > 0 ? padded + 4 : 0;
+  if (GROUPS > 1) __syncthreads();   // (every wavefront has read what the others counted)
+  if (lane == 0) taken[wave] = part == GROUPS - 1 ? reserved - before : total;
   __syncthreads();
   if (threadIdx.x == 0) {
     int sum = 0;
-    for (int r = 0; r < kTileRows; ++r) sum += row_total[r];
+    for (int r = 0; r < kTileRows; ++r) sum += taken[r];
     tile_base = sum > 0 ? atomicAdd(cursors + 1, sum) : 0;
   }
   __syncthreads();
-  int out = tile_base;
-  for (int r = 0; r < row; ++r) out += row_total[r];
-  if (lane == 0) {
-    ranges[tile * kTileRows + row] = WorkRange{out, padded};
+  int row_at = tile_base;
+  for (int r = 0; r < wave - part; ++r) row_at += taken[r];
+  int out = row_at + before;
+  if (lane == 0 && part == 0) {
+    ranges[tile * kTileRows + row] = WorkRange{row_at, padded};
     if (sorted != nullptr && ty * tg.th + row < H) {
       const int c = work_class(padded);
       const int at = atomicAdd(cursors + 2 + c, 1);
-      sorted[c * tg.total * kTileRows + at] = SortedRow{static_cast<int>(tile) * kTileRows + row, out, padded, 0};
+      sorted[c * tg.total * kTileRows + at] = SortedRow{static_cast<int>(tile) * kTileRows + row, row_at, padded, 0};
     }
   }
-  for (int base = 0; base < count; base += 64) {
+  for (int base = begin; base < end; base += 64) {
     int c = first_c, roi = first_item;
     const RowTap* taps = first_taps;
-    if (base > 0) {
+    if (base > begin) {
       c = 0; roi = 0; taps = nullptr;
-      if (base + lane < count) {
+      if (base + lane < end) {
         roi = item_at(base + lane);
         c = taps_of(roi, &taps);
       }
@@ -441,9 +460,8 @@ build_tile_work_kernel(const TileBox* __restrict__ boxes, int R, int* __restrict
     out += __shfl(incl, 63);
   }
   // padding: taps of weight zero that continue the last ROI and never end it
-  if (lane < reserved - total) {
-    entries[out + lane] = WorkEntry{item_at(count - 1), 0, 0.0f, 1};
-  }
+  if (part == GROUPS - 1 && lane < reserved - row_total)
+    entries[row_at + row_total + lane] = WorkEntry{item_at(count - 1), 0, 0.0f, 1};
 }
 
 }  // namespace roialign

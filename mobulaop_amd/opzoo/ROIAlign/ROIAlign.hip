@@ -442,7 +442,13 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
   } else {
     roialign::build_lists_kernel<<<static_cast<unsigned>(list_blocks), 256, 0, stream>>>(la);
   }
-  roialign::build_tile_work_kernel<<<static_cast<unsigned>(g.total), roialign::kTileRows * 64, 0, stream>>>(
+  // Few tiles: four workgroups each (one and four, us, both passes: 8 tiles of 512 boxes, 2 x 256 x 64 x 64 77 / 72; 32 of
+  // 7830, 4 x 64 x 29 x 104 bfloat16 channels last, 28 x 28 pooled 1201 / 1153; 50 of 5480, 5 x 448 x 74 x 125 744 / 735; 312 of
+  // 4000, 4 x 256 x 200 x 336 545 / 555).  The option "roialign_tile_groups" names one of the two (tests do).
+  const long long groups = mobula_hip::option("roialign_tile_groups", 0);
+  const bool shared = items <= roialign::kSharedListCap && groups != 1 && (groups == 4 || g.total <= 128);
+  const auto tile_work = shared ? roialign::build_tile_work_kernel<4> : roialign::build_tile_work_kernel<1>;
+  tile_work<<<static_cast<unsigned>(g.total * (shared ? 4 : 1)), roialign::kTileRows * 64, 0, stream>>>(
       plan->boxes, n_items, plan->tile_rois, plan->lists, g, plan->layout, plan->cursors, plan->ranges, plan->entries,
       plan->sorted, p.H);
   MOBULA_HIP_TRY(hipGetLastError());

@@ -889,6 +889,30 @@ def test_backward_of_a_few_boxes_in_one_launch(R, C, H, W, pooled, S, dtype, lay
         native.set_option('roialign_few_boxes', 1)
 
 
+@pytest.mark.parametrize('R', [0, 1, 63, 64, 65, 129, 257, 4097, 8192, 9000])
+def test_work_lists_made_by_one_and_by_four_workgroups(R):
+    """A tile's boxes around the chunks that wavefronts take, around what is read once, and beyond what LDS holds (4096 boxes
+    of a tile by one workgroup, 8192 in all by four): the same lists, so the same bits."""
+    abi.set_impl('tiled')
+    rng = np.random.default_rng(R)
+    N, C, H, W, pooled, scale, S = 2, 8, 21, 40, (2, 3), 1.0, 2
+    x1, y1 = rng.uniform(-2, W, R), rng.uniform(-2, H, R)
+    rois = np.stack([rng.integers(0, N, R) * (R < 4000), x1, y1, x1 + rng.uniform(0.5, 30, R), y1 + rng.uniform(0.5, 25, R)],
+                    1).astype(np.float32)
+    dy = rng.standard_normal((R, C) + pooled).astype(np.float32)
+    want = oracle.backward(dy, rois, (N, C, H, W), scale, S, impl='ordered')
+    d_dy, d_rois = abi.to_dev(dy), abi.to_dev(rois)
+    try:
+        got = []
+        for groups in (1, 4, 0):
+            native.set_option('roialign_tile_groups', groups)
+            got.append(abi.backward(d_dy, d_rois, (N, C, H, W), scale, S, assign=True))
+    finally:
+        native.set_option('roialign_tile_groups', 0)
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+    assert_parity(got[0].cpu().numpy(), want, BWD_TOL, 'bwd')
+
+
 @pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize('C,H,W,pooled', [(8, 65, 3, (1, 1)), (40, 131, 7, (2, 9)), (72, 9, 200, (1, 3)), (8, 300, 300, (1, 1))])
