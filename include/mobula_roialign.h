@@ -273,6 +273,12 @@ void mobula_hip_conv2d_backward(const int device_id, const float* dy, const floa
                                 const int filters, const int kernel_h, const int kernel_w, const int pad_h,
                                 const int pad_w, const int stride_h, const int stride_w,
                                 const int dilation_h, const int dilation_w, float* dx, float* dw);
+/* dst[n][cols][rows] = src[n][rows][cols] for `planes` planes of 2- or 4-byte
+ * elements on device `device_id`, on the calling thread's stream (a tensor from
+ * one memory format to the other). */
+void mobula_hip_transpose_planes(const int device_id, const long long planes, const long long rows,
+                                 const long long cols, const int elem_bytes, const void* src, void* dst);
+
 /* The same with the bias's gradient db[filters] (null: not wanted), which rides in launches of the others. */
 void mobula_hip_conv2d_gradients(const int device_id, const float* dy, const float* x, const float* weight,
                                  const int batch, const int channels, const int height, const int width,

@@ -150,6 +150,30 @@ bool nhwc_taken(bool backward, const Tensor& map, const RoiAlignArgs& a, int64_t
                                             map.size(2), map.size(3), a.PH, a.PW, a.S, rois) != 0;
 }
 
+// dst = src where one is dense and the other channels-last (any other pair is torch's to copy).
+void copy_format(const Tensor& src, const Tensor& dst) {
+  const bool from_last = is_channels_last(src) && dst.is_contiguous();
+  const int64_t bytes = src.element_size();
+  const bool pair = from_last || (src.is_contiguous() && is_channels_last(dst));
+  if (!pair || src.dim() != 4 || (bytes != 2 && bytes != 4) || src.is_neg() || src._is_zerotensor() ||
+      src.size(0) >= (1ll << 28) || src.numel() >= (1ll << 38) || src.size(1) >= (1ll << 24) ||
+      src.size(2) * src.size(3) >= (1ll << 24)) {   // (what the library's kernel takes)
+    dst.copy_(src);
+    return;
+  }
+  const int64_t channels = src.size(1), pixels = src.size(2) * src.size(3);
+  begin(src, {});
+  mobula_hip_transpose_planes(src.device().index(), src.size(0), from_last ? pixels : channels, from_last ? channels : pixels,
+                              static_cast<int>(bytes), src.data_ptr(), dst.data_ptr());
+  raise_if_failed("transpose_planes");
+}
+Tensor in_format(const Tensor& t, at::MemoryFormat format) {
+  if (t.is_contiguous(format)) return t;
+  const Tensor out = at::empty(t.sizes(), t.options().memory_format(format));
+  copy_format(t, out);
+  return out;
+}
+
 Tensor roi_align_forward(const Tensor& x, const Tensor& rois, const RoiAlignArgs& a) {
   const bool keeps_format = is_channels_last(x);
   const Tensor y = at::empty({rois.size(0), x.size(1), a.PH, a.PW},
@@ -158,10 +182,10 @@ Tensor roi_align_forward(const Tensor& x, const Tensor& rois, const RoiAlignArgs
   const Tensor r = rois.contiguous();
   // (a pooled map of one bin is dense in both formats, and then not taken for a channels-last one)
   const bool nhwc = keeps_format && is_channels_last(y) && nhwc_taken(false, x, a, r.size(0));
-  const Tensor xd = nhwc ? x : x.contiguous();
+  const Tensor xd = nhwc ? x : in_format(x, at::MemoryFormat::Contiguous);
   const Tensor yd = nhwc || y.is_contiguous() ? y : at::empty(y.sizes(), x.options());
   with_symbols(x.scalar_type(), [&](const auto& s) { call_forward(s, nhwc, xd, r, yd, a); });
-  if (!yd.is_same(y)) y.copy_(yd);
+  if (!yd.is_same(y)) copy_format(yd, y);
   return y;
 }
 
@@ -183,15 +207,15 @@ struct RoiAlignBackward : public Node {
     const Tensor dx = at::empty_like(like);
     const Tensor r = rois.contiguous();
     if (is_channels_last(dx) && nhwc_taken(true, dx, args, r.size(0))) {
-      const Tensor d = dy.contiguous(at::MemoryFormat::ChannelsLast);
+      const Tensor d = in_format(dy, at::MemoryFormat::ChannelsLast);
       bool taken = false;
       with_symbols(dx.scalar_type(), [&](const auto& s) { taken = call_assign(s, true, d, r, dx, args); });
       if (taken) return dx;
     }
-    const Tensor d = dy.contiguous();
+    const Tensor d = in_format(dy, at::MemoryFormat::Contiguous);
     const Tensor dense = dx.is_contiguous() ? dx : at::empty(dx.sizes(), dx.options());
     with_symbols(dx.scalar_type(), [&](const auto& s) { call_assign(s, false, d, r, dense, args); });
-    if (!dense.is_same(dx)) dx.copy_(dense);
+    if (!dense.is_same(dx)) copy_format(dense, dx);
     return dx;
   }
 

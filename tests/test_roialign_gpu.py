@@ -1604,3 +1604,28 @@ def test_partly_copied_maps_of_several_channel_blocks(W, dtype, S):
     y = abi.forward(abi.to_dev(x), abi.to_dev(rois), pooled, scale, S).cpu().numpy()
     want = oracle.forward(x.astype(np.float32), rois, pooled, scale, S).astype(dtype)
     assert_parity(y.astype(np.float32), want.astype(np.float32), FWD_TOL if dtype == np.float32 else FP16_TOL, 'y')
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('C,W', [(1, 70), (63, 65), (65, 9), (130, 31), (3, 1)])
+def test_formats_of_channel_counts_that_need_a_conversion(C, W, dtype):
+    """Channels-last maps of counts that no lane takes whole pass through dense copies, tiles of 64 x 64 transposed:
+    the values are those of the dense call, bit for bit, in both directions, also from a gradient in either format."""
+    import mobulaop_amd as mobula
+    mobula.op.load('ROIAlign')
+    abi.set_impl('tiled')   # (sums in one order, whatever runs first)
+    g = torch.Generator().manual_seed(C)
+    x = torch.randn((3, C, 13, W), generator=g).cuda().to(dtype)
+    rois = torch.tensor([[0, -1, 2, 5, 9], [2, 0, 0, W, 13], [1, 3, 3, 3, 3.]], device='cuda')
+    results = []
+    for of_x in (torch.contiguous_format, torch.channels_last):
+        for of_dy in (torch.contiguous_format, torch.channels_last):
+            xs = x.contiguous(memory_format=of_x).detach().requires_grad_()
+            y = mobula.op.ROIAlign(xs, rois, pooled_size=(5, 7), spatial_scale=1.0, sampling_ratio=2)
+            assert y.is_contiguous(memory_format=of_x)
+            dy = torch.randn((3, C, 5, 7), generator=torch.Generator().manual_seed(1)).cuda().to(dtype)
+            y.backward(dy.contiguous(memory_format=of_dy))
+            results.append((y.detach(), xs.grad))
+    for y, dx in results[1:]:
+        assert torch.equal(y, results[0][0])
+        assert torch.equal(dx, results[0][1]), (dx.float() - results[0][1].float()).abs().max()
