@@ -335,7 +335,7 @@ void mobula_hip_clear_error(void);
  * whose width is a multiple of four 16 bytes at a time, 0 element by element;
  * "roialign_few_boxes": 1 (default) lets a few boxes on a small map go back in
  * one launch where that is faster, 0 never, 2 wherever it can (64 boxes);
- * "roialign_patch": 4 or 12 fixes the wavefronts that share a patch of the
+ * "roialign_patch": 2, 4 or 12 fixes the wavefronts that share a patch of the
  * gradient where sampling grids have more than two points per bin and axis, and
  * takes other grids that way too, 1 (default) chooses; "roialign_tile_groups": 1
  * or 4 fixes the workgroups that make a tile's work lists, 0 (default) chooses --

@@ -353,7 +353,7 @@ backward_patch_kernel(const T* __restrict__ dy, PatchArgs pa, T* __restrict__ dx
     }
   };
 
-  bool any = false;   // (the same for the whole workgroup)
+  int busy = 0;   // wavefronts that had a box (the same for the whole workgroup)
   for (int r0 = 0; r0 < R; r0 += CHUNK) {
     // the boxes that reach the patch, in their order
     bool hit[LOOK];
@@ -383,7 +383,7 @@ backward_patch_kernel(const T* __restrict__ dy, PatchArgs pa, T* __restrict__ dx
       upto += lane >= off ? before : 0;
     }
     const int total = __builtin_amdgcn_readlane(upto, 63), first_of = upto - own;
-    any = any || total > 0;
+    busy = max(busy, min(total, NW));
 #pragma unroll
     for (int j = 0; j < LOOK; ++j) {
       const unsigned long long m = __ballot(hit[j]);
@@ -445,7 +445,7 @@ backward_patch_kernel(const T* __restrict__ dy, PatchArgs pa, T* __restrict__ dx
   auto element = [&](int y, int x, int c) {
     return dx + (NHWC ? ((static_cast<size_t>(n) * H + y) * W + x) * C + c : ((static_cast<size_t>(n) * C + c) * H + y) * W + x);
   };
-  if (!any) {   // nothing to add up: 98 boxes on 6 x 416 x 228 x 193, forward and backward 350 -> 294 us
+  if (busy == 0) {   // nothing to add up: 98 boxes on 6 x 416 x 228 x 193, forward and backward 350 -> 294 us
     if (!assign) return;
     for (int u = tid; u < TY * TX * K::CH; u += NW * 64) {
       const int x = x0 + (NHWC ? (u >> 5) & 15 : u & 15), y = y0 + (NHWC ? u >> 9 : (u >> 4) & 7), c = c0 + (NHWC ? u & 31 : u >> 7);
@@ -460,7 +460,9 @@ backward_patch_kernel(const T* __restrict__ dy, PatchArgs pa, T* __restrict__ dx
   for (int r = 0; r < TY; ++r) {
     if (r % 2 == 0 && r > 0) __syncthreads();   // (what the last two rows left has been read)
 #pragma unroll
-    for (int i = 0; i < CR; ++i) stage[(r % 2 * CR + i) * SUMS + lane] = acc[r][i];
+    for (int i = 0; i < CR; ++i) {
+      if (wave < busy) stage[(r % 2 * CR + i) * SUMS + lane] = acc[r][i];
+    }
     if (r % 2 == 1) {
       __syncthreads();
       for (int u = tid; u < 2 * CR * 64; u += NW * 64) {
@@ -471,7 +473,7 @@ backward_patch_kernel(const T* __restrict__ dy, PatchArgs pa, T* __restrict__ dx
           const int at = (half * CR + i) * SUMS + g * TX + x;
           float sum = stage_s[0][at];
 #pragma unroll
-          for (int w = 1; w < NW; ++w) sum += stage_s[w][at];
+          for (int w = 1; w < NW; ++w) sum += w < busy ? stage_s[w][at] : 0.0f;
           T* const to = element(y, x0 + x, c);
           *to = from_float<T>(assign ? sum : to_float(*to) + sum);
         }

@@ -518,13 +518,13 @@ void launch_few_boxes(const Problem& p, const T* dy, const float* rois, T* dx, b
 // How backward_patch_kernel is launched: wavefronts of a workgroup (0: not at all), patches, workspace.
 struct PatchPlan { int waves; long long blocks; int tiles_x, tiles_y, hp, wp; size_t b_spans, b_records, b_dense; };
 
-// For sampling grids of more than two points per bin and axis; the option "roialign_patch" 4 or 12 names the wavefronts,
+// For sampling grids of more than two points per bin and axis; the option "roialign_patch" 2, 4 or 12 names the wavefronts,
 // and takes grids of one and two points too (tests do).
 PatchPlan patch_plan(const Problem& p) {
   using BP = roialign::BwdPatch;
   PatchPlan plan{};
   const long long option = mobula_hip::option("roialign_patch", 1);
-  const bool forced = option == 4 || option == 12;
+  const bool forced = option == 2 || option == 4 || option == 12;
   if ((!forced && (p.S == 1 || p.S == 2)) || p.S > roialign::kSearchedGrid || p.PW > BP::BINS || p.PH > BP::MOST_PH) return plan;
   plan.tiles_x = (p.W + BP::TX - 1) / BP::TX;
   plan.tiles_y = (p.H + BP::TY - 1) / BP::TY;
@@ -540,8 +540,13 @@ PatchPlan patch_plan(const Problem& p) {
   // 100) 1468 / 1396, 1152 of 1254 (4 x 80 x 41 x 248) 710 / 660, 770 of 482 (7 x 160 x 82 x 18) 286 / 296, 720 of 100 (3 x 81 x
   // 75 x 113) 72 / 83, 5472 of 413 (4 x 256 x 148 x 131) 530 / 660, 576 of 671 (1 x 72 x 93 x 243) 190 / 169, 324 of 1295 (2 x 176 x
   // 70 x 33) 337 / 220, 112 of 325 (4 x 32 x 49 x 56) 276 / 158, 120 of 736 (5 x 64 x 28 x 44) 405 / 208.
+  // Two where patches are many and the boxes of an image few, so that each reaches few patches (with 4 and with 2): 8400 of 23
+  // boxes in 3 images (3 x 421 x 196 x 116) 148 / 117, 4830 of 179 in 5 (5 x 64 x 178 x 331) 76 / 61, 6510 of 486 in 7 (7 x 144 x 242
+  // x 81) 147 / 123, 1512 of 57 in 3 (3 x 280 x 59 x 101) 95 / 86; but 1632 of 279 in 8 (8 x 40 x 44 x 266) 90 / 98, 840 of 33 in 7
+  // (7 x 128 x 79 x 43) 46 / 48, 5472 of 1651 in 4 530 / 564.
   plan.waves = forced ? static_cast<int>(option)
-                      : plan.blocks <= 640 || (plan.blocks <= 2048 && p.R >= 8 * patches) ? 12 : 4;
+               : plan.blocks <= 640 || (plan.blocks <= 2048 && p.R >= 8 * patches) ? 12
+               : plan.blocks >= 1280 && 64 * p.R <= p.N * plan.blocks ? 2 : 4;
   return plan;
 }
 
@@ -555,7 +560,9 @@ bool launch_patches(const Problem& p, const PatchPlan& plan, const T* dy, const 
                                reinterpret_cast<roialign::PatchSpan*>(ws), reinterpret_cast<roialign::CellRecord*>(ws + plan.b_spans),
                                reinterpret_cast<float*>(ws + plan.b_spans + plan.b_records)};
   if (p.R > 0) roialign::patch_weights_kernel<<<(p.R + 1) / 2, 256, 0, stream>>>(pa);
-  const auto kernel = plan.waves == 4 ? roialign::backward_patch_kernel<T, NHWC, 4> : roialign::backward_patch_kernel<T, NHWC, 12>;
+  const auto kernel = plan.waves == 2   ? roialign::backward_patch_kernel<T, NHWC, 2>
+                      : plan.waves == 4 ? roialign::backward_patch_kernel<T, NHWC, 4>
+                                        : roialign::backward_patch_kernel<T, NHWC, 12>;
   mobula_hip::KernelTimer timer("backward_blocked_kernel", stream);   // (whoever owns dx reports under this name)
   kernel<<<static_cast<unsigned>(plan.blocks), plan.waves * 64, 0, stream>>>(dy, pa, dx, p.C, plan.tiles_x, plan.tiles_y,
                                                                              assign ? 1 : 0);

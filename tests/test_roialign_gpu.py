@@ -939,7 +939,7 @@ def test_bins_of_more_points_than_are_searched(C, H, W, pooled, dtype, layout):
     assert_parity(y.float().cpu().numpy(), torch.from_numpy(want).to(dtype).float().numpy(), tol, 'fwd')
 
 
-@pytest.mark.parametrize('waves', [4, 12])
+@pytest.mark.parametrize('waves', [2, 4, 12])
 @pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize('R,C,H,W,pooled,S,scale', [
@@ -951,6 +951,8 @@ def test_bins_of_more_points_than_are_searched(C, H, W, pooled, dtype, layout):
     (25, 64, 40, 37, (32, 32), 5, 0.5),      # the most pooled rows and columns
     (30, 4, 20, 200, (1, 17), 0, 1.0),       # wide bins
     (30, 4, 200, 20, (17, 1), 64, 1.0),      # a dense fixed grid, dozens of weights to a cell
+    (90, 8, 44, 266, (14, 14), 0, 1.0),      # boxes of more cells than lanes, some of them of few samples
+    (90, 8, 44, 266, (14, 14), 3, 0.0625),
     (3200, 5, 9, 12, (2, 3), 0, 0.25),       # more boxes than are looked at at a time
     (50, 40, 33, 40, (14, 14), 2, 0.25),
     (50, 40, 33, 40, (14, 14), 1, 0.25),
