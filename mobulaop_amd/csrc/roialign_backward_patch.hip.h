@@ -81,6 +81,18 @@ patch_weights_kernel(PatchArgs a) {
     const float step = bin / static_cast<float>(grid);
     const int base = max(0, start > 0.0f ? static_cast<int>(fminf(start, last)) - 1 : 0);   // (of the dense table)
     int first_on = 1 << 20, last_on = -1;
+    // Up to 64 samples of the axis: a lane each, read from there by all cells.  (Each cell for itself took 42 samples of a box that
+    // is one cell wide, one after the other: 36 boxes, 14 x 14 bins of 3 x 3 points, 20 -> 13 us.)
+    const bool few = grid >= 1 && grid <= 64 && P * grid <= 64;
+    int low = -1, high = -1;   // cells of the lane's sample
+    float at_low = 0.0f, at_high = 0.0f;
+    if (few && lane < P * grid) {
+      const AxisSample s = axis_sample(sample_coord(start, lane / grid, bin, lane % grid, grid), size);
+      if (s.valid) {
+        low = s.low; at_low = s.h;
+        if (s.high != s.low) high = s.high, at_high = s.l;
+      }
+    }
     for (int cell = c0 + lane; cell <= c1; cell += 64) {
       CellRecord rec{};
       if (cell < size && image_ok) {
@@ -92,9 +104,10 @@ patch_weights_kernel(PatchArgs a) {
           w *= factor;
           if (w == 0.0f) return;
           if (n == 0) first = p;
-#pragma unroll
-          for (int k = 0; k < BwdPatch::kInline; ++k)
-            if (n == k) rec.w[k] = w;
+          static_assert(BwdPatch::kInline == 7, "one line each: a loop leaves the record in memory");
+          rec.w[0] = n == 0 ? w : rec.w[0]; rec.w[1] = n == 1 ? w : rec.w[1]; rec.w[2] = n == 2 ? w : rec.w[2];
+          rec.w[3] = n == 3 ? w : rec.w[3]; rec.w[4] = n == 4 ? w : rec.w[4]; rec.w[5] = n == 5 ? w : rec.w[5];
+          rec.w[6] = n == 6 ? w : rec.w[6];
           if (dense && rel >= 0 && rel < P + 3 && n < P) table[rel * P + n] = w;
           ++n;
         };
@@ -104,7 +117,16 @@ patch_weights_kernel(PatchArgs a) {
           if (s.low == cell) *w += s.h;
           if (s.high == cell && s.high != s.low) *w += s.l;
         };
-        if (grid >= 1 && grid <= kMergedGrid) {   // (the samples near the cell from its coordinate, one and more to spare)
+        if (few) {
+          for (int p = 0, q = 0; p < P; ++p) {
+            float w = 0.0f;
+            for (const int end_q = q + grid; q < end_q; ++q) {
+              if (__builtin_amdgcn_readlane(low, q) == cell) w += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(at_low), q));
+              if (__builtin_amdgcn_readlane(high, q) == cell) w += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(at_high), q));
+            }
+            put(p, w);
+          }
+        } else if (grid >= 1 && grid <= kMergedGrid) {   // (the samples near the cell from its coordinate, one and more to spare)
           const float fa = (from - start) / step - 0.5f, fb = (to_c - start) / step - 0.5f;
           int q = 0, q1 = P * grid;
           if (fabsf(fa) < 1.0e9f && fabsf(fb) < 1.0e9f) {
