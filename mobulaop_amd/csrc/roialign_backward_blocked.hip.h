@@ -177,12 +177,10 @@ lists_and_dy_kernel(ListsArgs lists, unsigned list_blocks, const T* __restrict__
 
 // Number of workgroups for `tiles` tiles and cblk channel blocks (job decode at
 // the top of backward_blocked_kernel).
-inline long long backward_blocked_grid(long long tiles, int cblk) {
-  tiles *= BwdBlocked::BANDS;   // one workgroup per band
-  long long per_xcd;
-  if (cblk >= 8) per_xcd = tiles * ((cblk + 7) / 8);
-  else per_xcd = (tiles + (8 / cblk) - 1) / (8 / cblk);
-  return 8 * per_xcd;
+// (sorted: the tile rows are taken longest first)
+inline long long backward_blocked_grid(long long tiles, int cblk, bool sorted) {
+  const long long rows = tiles * BwdBlocked::BANDS;   // one workgroup per band
+  return 8 * jobs_of_xcd(rows, cblk, sorted ? 1 : (rows + 7) / 8);
 }
 
 typedef int int16v __attribute__((ext_vector_type(16)));
@@ -221,26 +219,12 @@ backward_blocked_kernel(const void* __restrict__ dy_any, TO* __restrict__ dx_any
   static_assert(K::TH == 1, "the parts of a split row take the place of the rows of a band");
   extern __shared__ __attribute__((aligned(16))) float acc[];   // [NSPLIT][RS][CS]
 
-  // Job decode.  Workgroups are dealt to the 8 XCDs round-robin, so blockIdx % 8
-  // names the XCD: it takes the channel blocks b with b % 8 == xcd (their slice
-  // of dyb then stays in that XCD's L2) and walks the bands of the tiles in order; with
-  // fewer than 8 blocks the tiles of a block are split into 8 / cblk ranges.
-  const int xcd = blockIdx.x & 7;
-  const long long wi = blockIdx.x >> 3;
-  long long tile;
-  int cb;
-  if (cblk >= 8) {
-    const int nx = (cblk - xcd + 7) >> 3;
-    tile = wi / nx;
-    cb = xcd + 8 * static_cast<int>(wi % nx);
-  } else {
-    const int parts = 8 / cblk;
-    cb = xcd % cblk;
-    const int part = xcd / cblk;
-    const long long range = (tg.total * K::BANDS + parts - 1) / parts;
-    if (part >= parts || wi >= range) return;
-    tile = sorted != nullptr ? wi * parts + part : part * range + wi;
-  }
+  // Job decode: an XCD walks the bands of its channel blocks' tiles in order (job_of_xcd).
+  const unsigned rows = static_cast<unsigned>(tg.total * K::BANDS);
+  const XcdJob job = job_of_xcd(blockIdx.x & 7, blockIdx.x >> 3, cblk, sorted != nullptr ? 1 : (rows + 7) / 8);
+  const int cb = job.block;
+  long long tile = job.item;
+  if (cb >= cblk) return;
   if (tile >= tg.total * K::BANDS) return;
   static_assert(K::TH == 1 && K::BANDS == kTileRows, "a band is a tile row");
   WorkRange wr;

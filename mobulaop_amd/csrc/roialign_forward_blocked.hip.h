@@ -10,7 +10,7 @@
 // whole wavefront and live in scalar registers; a map row that several samples
 // of a pooled column touch (samples less than a pixel apart, within a bin or in
 // neighbouring bins) is fetched once and its weighted column sum reused.
-// Channel block b is only ever read by XCD b % 8 and ROIs are visited in
+// A channel block is read by one XCD or by a few (job_of_xcd) and ROIs are visited in
 // spatial order, so what one L2 has to hold is a 128-byte-per-pixel slice of
 // the neighbourhood the XCD is currently working in.
 #pragma once
@@ -351,10 +351,7 @@ __device__ __forceinline__ typename LaneData<T>::type buffer_load_lane(__amdgpu_
 // at the top of forward_blocked_kernel).
 // (nw: wavefronts per workgroup of the kernel that is launched)
 inline long long blocked_grid(long long R, int cblk, int nw = FwdBlocked::NW) {
-  long long per_xcd;
-  if (cblk >= 8) per_xcd = R * ((cblk + 7) / 8);
-  else per_xcd = (R + (8 / cblk) - 1) / (8 / cblk);
-  return 8 * ((per_xcd + nw - 1) / nw);
+  return 8 * ((jobs_of_xcd(R, cblk, (R + 7) / 8) + nw - 1) / nw);
 }
 
 // The same for channels-last maps (see the job decode).
@@ -435,10 +432,7 @@ forward_blocked_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   auto uni_i = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
   auto uni_f = [](float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); };
-  // Job decode.  Workgroups are dealt to the 8 XCDs round-robin, so blockIdx % 8
-  // names the XCD: it takes the channel blocks b with b % 8 == xcd and walks
-  // the sorted ROIs; with fewer than 8 blocks the ROIs of a block are split
-  // into 8 / cblk contiguous ranges instead.
+  // Job decode: an XCD walks the sorted ROIs of its channel blocks (job_of_xcd).
   // (with few ROIs the pooled rows of one are dealt to `parts` wavefronts, neighbours in this order)
   const int R = rois_listed * parts;
   const int xcd = blockIdx.x & 7;
@@ -453,17 +447,11 @@ forward_blocked_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
     cb = static_cast<int>(wi / range);
     if (cb >= cblk) return;
     slot = xcd * range + (wi - cb * range);
-  } else if (cblk >= 8) {
-    const int nx = (cblk - xcd + 7) >> 3;
-    slot = wi / nx;
-    cb = xcd + 8 * static_cast<int>(wi % nx);
   } else {
-    const int parts = 8 / cblk;
-    cb = xcd % cblk;
-    const int part = xcd / cblk;
-    const long long range = (R + parts - 1) / parts;
-    if (part >= parts || wi >= range) return;
-    slot = part * range + wi;
+    const XcdJob job = job_of_xcd(xcd, static_cast<unsigned>(wi), cblk, (static_cast<unsigned>(R) + 7) / 8);
+    cb = job.block;
+    slot = job.item;
+    if (cb >= cblk) return;
   }
   if (slot >= R) return;
   int ph_first = 0, ph_end = PH;

@@ -144,17 +144,11 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
     cb = static_cast<int>(wi / range);
     if (cb >= cblk) return;
     slot = xcd * range + (wi - cb * range);
-  } else if (cblk >= 8) {
-    const int nx = (cblk - xcd + 7) >> 3;
-    slot = wi / nx;
-    cb = xcd + 8 * static_cast<int>(wi % nx);
   } else {
-    const int parts = 8 / cblk;
-    cb = xcd % cblk;
-    const int part = xcd / cblk;
-    const long long range = (R + parts - 1) / parts;
-    if (part >= parts || wi >= range) return;
-    slot = part * range + wi;
+    const XcdJob job = job_of_xcd(xcd, static_cast<unsigned>(wi), cblk, (static_cast<unsigned>(R) + 7) / 8);
+    cb = job.block;
+    slot = job.item;
+    if (cb >= cblk) return;
   }
   if (slot >= R) return;
   int ph_first = 0, ph_end = PH;

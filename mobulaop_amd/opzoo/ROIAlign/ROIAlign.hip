@@ -592,7 +592,7 @@ void backward_device(const Problem& p, const T* dy, const float* rois, T* dx, bo
       return;
     if (!taken || (p.S != 1 && p.S != 2) ||
         !plan_tiles<T>(p, rois, roialign::kTileRows, tw, /*with_dyb=*/false, stream, &plan) ||
-        roialign::backward_blocked_grid(plan.grid.total, cblk) >= (1ll << 31)) {
+        roialign::backward_blocked_grid(plan.grid.total, cblk, plan.sorted != nullptr) >= (1ll << 31)) {
       if (!failed())
         set_error("roi_align_backward_nhwc: shape C=%d pooled %dx%d sampling_ratio %d (or the type or alignment "
                   "of the tensors) is not taken by the channels-last path", p.C, p.PH, p.PW, p.S);
@@ -602,7 +602,7 @@ void backward_device(const Problem& p, const T* dy, const float* rois, T* dx, bo
     mobula_hip::KernelTimer timer("backward_blocked_kernel", stream);
     const int nsplit = row_split(p);
     const auto kernel = owner_kernel<true, T>(nsplit);
-    kernel<<<static_cast<unsigned>(roialign::backward_blocked_grid(plan.grid.total, cblk)), BB::NT * nsplit,
+    kernel<<<static_cast<unsigned>(roialign::backward_blocked_grid(plan.grid.total, cblk, plan.sorted != nullptr)), BB::NT * nsplit,
              roialign::backward_blocked_lds(tw, nsplit), stream>>>(
         dy, dx, plan.ranges, plan.sorted, plan.class_counts(), plan.entries, plan.lists,
         plan.grid, plan.layout, p.C, p.H, p.W, p.PH, p.PW, cblk, dy_bytes,
@@ -639,7 +639,7 @@ void backward_device(const Problem& p, const T* dy, const float* rois, T* dx, bo
   if (lists && plan_tiles<T>(p, rois, roialign::kTileRows, tw, /*with_dyb=*/true, stream, &plan,
                     side.get() == stream ? dy : nullptr)) {
     const int cblk = (p.C + BB::CB - 1) / BB::CB;
-    const long long grid = roialign::backward_blocked_grid(plan.grid.total, cblk);
+    const long long grid = roialign::backward_blocked_grid(plan.grid.total, cblk, plan.sorted != nullptr);
     const DyLaunch dl = dy_launch<T>(p);
     if (grid < (1ll << 31) && dl.blocks < (1ll << 31) && (dl.per > 0 || dl.cap >= 4)) {
       if (p.R > 0 && !plan.dy_transposed)

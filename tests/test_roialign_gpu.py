@@ -1631,3 +1631,29 @@ def test_formats_of_channel_counts_that_need_a_conversion(C, W, dtype):
     for y, dx in results[1:]:
         assert torch.equal(y, results[0][0])
         assert torch.equal(dx, results[0][1]), (dx.float() - results[0][1].float()).abs().max()
+
+
+@pytest.mark.parametrize('sort', [0, 2])
+@pytest.mark.parametrize('R', [1, 37])
+@pytest.mark.parametrize('blocks', [1, 3, 4, 5, 7, 8, 9, 13, 16])
+def test_channel_blocks_shared_out_to_the_xcds(blocks, R, sort):
+    """Every box (tile row) of every channel block is taken once, by ranges and one by one, whatever the number of blocks."""
+    native.set_option('roialign_sort_rows', sort)
+    native.set_option('roialign_few_boxes', 0)
+    try:
+        abi.set_impl('tiled')
+        rng = np.random.default_rng(blocks)
+        N, C, H, W, pooled = 2, 32 * blocks - 5, 9, 21, (3, 5)
+        x = rng.standard_normal((N, C, H, W)).astype(np.float32)
+        c = rng.uniform(0, (W, H), (R, 2))
+        wh = rng.uniform(1, 9, (R, 2))
+        rois = np.concatenate([rng.integers(0, N, (R, 1)), c - wh / 2, c + wh / 2], 1).astype(np.float32)
+        dy = rng.standard_normal((R, C) + pooled).astype(np.float32)
+        for S in (2, 0):
+            y = abi.forward(abi.to_dev(x), abi.to_dev(rois), pooled, 1.0, S)
+            assert_parity(y.cpu().numpy(), oracle.forward(x, rois, pooled, 1.0, S), FWD_TOL, 'y')
+        dx = abi.backward(abi.to_dev(dy), abi.to_dev(rois), x.shape, 1.0, 2, assign=True)
+        assert_parity(dx.cpu().numpy(), oracle.backward(dy, rois, x.shape, 1.0, 2), BWD_TOL, 'dx')
+    finally:
+        native.set_option('roialign_sort_rows', 1)
+        native.set_option('roialign_few_boxes', 1)
