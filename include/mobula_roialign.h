@@ -331,7 +331,7 @@ void mobula_hip_clear_error(void);
  * "roialign_tile_columns": 0 (default) lets the backward pass choose its tile
  * width from the size of the map, a multiple of 4 from 16 to 64 fixes it; "roialign_row_split": 0
  * (default) lets it choose how many wavefronts share a tile row's work list,
- * 1 or 4 fixes it; "roialign_row_quads": 1 (default) lets it write rows of maps
+ * 1, 4 or 8 fixes it; "roialign_row_quads": 1 (default) lets it write rows of maps
  * whose width is a multiple of four 16 bytes at a time, 0 element by element;
  * "roialign_few_boxes": 1 (default) lets a few boxes on a small map go back in
  * one launch where that is faster, 0 never, 2 wherever it can (64 boxes);

@@ -51,8 +51,11 @@ struct BwdBlocked {
 inline bool backward_blocked_supports(int PH, int PW, int S) { return lists_supported(PH, PW, S); }
 
 // Maps that give few tile rows of 56 columns: every row's work list is split, and tiles may be narrow.
+inline long long backward_tile_rows(long long images, int H, int W, int cblk) {
+  return images * ((H + kTileRows - 1) / kTileRows) * ((W + 55) / 56) * kTileRows * cblk;
+}
 inline bool backward_few_tiles(long long images, int H, int W, int cblk) {
-  return images * ((H + kTileRows - 1) / kTileRows) * ((W + 55) / 56) * kTileRows * cblk < 8192;
+  return backward_tile_rows(images, H, W, cblk) < 8192;
 }
 
 // Tile width for a map: as few tiles as the widest allow, all about as wide (multiples of four columns: the four-column
@@ -71,9 +74,17 @@ inline int backward_tile_columns(long long images, int H, int W, int cblk) {
   return width(tiles);
 }
 
-// Wavefronts per tile row.
-inline int backward_row_split(long long images, int H, int W, int cblk) {
-  return backward_few_tiles(images, H, W, cblk) ? BwdBlocked::NSPLIT : 1;
+// Wavefronts per tile row.  `pooled` elements make the lists of `map` elements: where they are short and the rows more than the
+// device holds of undivided ones, parts only add their clearing and adding up (forward and backward, us, 4 parts and 1: 2592 rows,
+// 1.4 pooled elements to one of the map 97 / 77; 4800, 2.0 117 / 90; 2880, 0.2 102 / 79; 3584, 1.6 137 / 131; but 2496, 1.3 68 / 74;
+// 3024, 3.0 168 / 205).  A few rows with the lists of thousands of boxes are chains, and shorter in eight parts (4 and 8: 384
+// rows, 135 to one 325 / 223; 64, 125 290 / 209; 192, 75 147 / 112; but 640, 126 633 / 734; 384, 7 68 / 83; sixteen parts are slower
+// than four nearly everywhere).
+inline int backward_row_split(long long images, int H, int W, int cblk, long long pooled, long long map) {
+  if (!backward_few_tiles(images, H, W, cblk)) return 1;
+  const long long rows = backward_tile_rows(images, H, W, cblk);
+  if (rows >= 2560 && 2 * pooled <= 5 * map) return 1;
+  return rows <= 384 && pooled >= 50 * map ? 2 * BwdBlocked::NSPLIT : BwdBlocked::NSPLIT;
 }
 
 // dy[r][c][ph][pw] -> dyb[cb][r][ph][pw][32] (R: number of ROIs), zero where the channel does

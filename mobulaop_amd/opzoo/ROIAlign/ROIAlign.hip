@@ -466,20 +466,22 @@ int tile_columns(const Problem& p) {
   return roialign::backward_tile_columns(p.N, p.H, p.W, (p.C + BB::CB - 1) / BB::CB);
 }
 
-// Wavefronts per tile row of the backward pass (1, or BwdBlocked::NSPLIT for maps with few tile
-// rows); the option "roialign_row_split" names one of the two (tests do).
+// Wavefronts per tile row of the backward pass (1, 4 or 8: backward_row_split); the option "roialign_row_split"
+// names them (tests do).
 int row_split(const Problem& p) {
   using BB = roialign::BwdBlocked;
   const long long forced = mobula_hip::option("roialign_row_split", 0);
-  if (forced == 1 || forced == BB::NSPLIT) return static_cast<int>(forced);
-  return roialign::backward_row_split(p.N, p.H, p.W, (p.C + BB::CB - 1) / BB::CB);
+  if (forced == 1 || forced == BB::NSPLIT || forced == 2 * BB::NSPLIT) return static_cast<int>(forced);
+  return roialign::backward_row_split(p.N, p.H, p.W, (p.C + BB::CB - 1) / BB::CB, p.n_out, p.N * p.C * p.H * p.W);
 }
 
 // The tile owner for a problem: nsplit wavefronts per tile row.
 template <bool NHWC, typename T>
 auto owner_kernel(int nsplit) {
   using BB = roialign::BwdBlocked;
-  return nsplit > 1 ? roialign::backward_blocked_kernel<NHWC, T, BB::NSPLIT> : roialign::backward_blocked_kernel<NHWC, T, 1>;
+  return nsplit > BB::NSPLIT ? roialign::backward_blocked_kernel<NHWC, T, 2 * BB::NSPLIT>
+         : nsplit > 1        ? roialign::backward_blocked_kernel<NHWC, T, BB::NSPLIT>
+                             : roialign::backward_blocked_kernel<NHWC, T, 1>;
 }
 
 // Any sampling grid the lists take: fixed ones up to kSearchedGrid points, adaptive ones

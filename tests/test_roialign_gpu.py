@@ -1657,3 +1657,32 @@ def test_channel_blocks_shared_out_to_the_xcds(blocks, R, sort):
     finally:
         native.set_option('roialign_sort_rows', 1)
         native.set_option('roialign_few_boxes', 1)
+
+
+@pytest.mark.parametrize('S', [2, 1])
+@pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
+@pytest.mark.parametrize('W,R', [(5, 3), (61, 40), (65, 400)])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+def test_eight_wavefronts_to_a_tile_row(dtype, W, R, layout, S):
+    """Lists shorter than eight parts, items that reach over parts, long lists; against four wavefronts and the oracle."""
+    rng = np.random.default_rng(W)
+    N, C, H, pooled = 2, 36, 10, (5, 9)
+    c, half = rng.uniform(0, (W, H), (R, 2)), rng.uniform(1, 8, (R, 2))
+    rois = np.concatenate([rng.integers(0, N, (R, 1)), c - half, c + half], 1).astype(np.float32)
+    dy = torch.from_numpy(rng.standard_normal((R, C) + pooled).astype(np.float32)).to(dtype)
+    want = oracle.backward(dy.float().numpy(), rois, (N, C, H, W), 1.0, S, impl='ordered')
+    native.set_option('roialign_few_boxes', 0)
+    abi.set_impl('tiled')
+    try:
+        for split in (8, 4):
+            native.set_option('roialign_row_split', split)
+            if layout == 'nhwc':
+                got = abi.backward_nhwc(dy.permute(0, 2, 3, 1).contiguous().cuda(), abi.to_dev(rois), (N, H, W, C), 1.0, S, assign=True)
+                got = got.permute(0, 3, 1, 2)
+            else:
+                got = abi.backward(dy.cuda(), abi.to_dev(rois), (N, C, H, W), 1.0, S, assign=True)
+            # (bfloat16: sums in fp32, rounded once: half a unit of the last of 8 bits)
+            assert_parity(got.float().cpu().numpy(), want, BWD_TOL if dtype == torch.float32 else 2.0 ** -8, str(split))
+    finally:
+        native.set_option('roialign_row_split', 0)
+        native.set_option('roialign_few_boxes', 1)
