@@ -81,9 +81,11 @@ patch_weights_kernel(PatchArgs a) {
     const float step = bin / static_cast<float>(grid);
     const int base = max(0, start > 0.0f ? static_cast<int>(fminf(start, last)) - 1 : 0);   // (of the dense table)
     int first_on = 1 << 20, last_on = -1;
-    // Up to 64 samples of the axis: a lane each, read from there by all cells.  (Each cell for itself took 42 samples of a box that
-    // is one cell wide, one after the other: 36 boxes, 14 x 14 bins of 3 x 3 points, 20 -> 13 us.)
-    const bool few = grid >= 1 && grid <= 64 && P * grid <= 64;
+    // Up to 64 samples of the axis, close together: a lane each, read from there by all cells.  (Each cell for itself took 42 samples
+    // of a box that is one cell wide, one after the other: 36 boxes, 14 x 14 bins of 3 x 3 points, 20 -> 13 us.  Some ten
+    // instructions a sample and twenty a bin, against eighty for each of the samples around a cell: 2 / step and four to spare.)
+    const bool few = grid >= 1 && grid <= 64 && P * grid <= 64 &&
+                     static_cast<float>(P * (grid + 2)) * step <= 16.0f + 32.0f * step;
     int low = -1, high = -1;   // cells of the lane's sample
     float at_low = 0.0f, at_high = 0.0f;
     if (few && lane < P * grid) {
