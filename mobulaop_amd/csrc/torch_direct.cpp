@@ -120,7 +120,7 @@ void call_forward(const RoiAlignSymbols<T, B>& s, bool nhwc, const Tensor& x, co
   raise_if_failed(nhwc ? "roi_align_forward_nhwc" : "roi_align_forward");
 }
 
-// taken = false: the channels-last entry point refused a sampling grid that the other one takes
+// false: the channels-last entry point had no room for a larger grid's weights, where the other one falls back
 template <typename T, typename B>
 bool call_assign(const RoiAlignSymbols<T, B>& s, bool nhwc, const Tensor& dy, const Tensor& rois, const Tensor& dx,
                  const RoiAlignArgs& a) {

@@ -85,10 +85,9 @@ class ROIAlign:
                                                            _nhwc(dx), rois)
                 taken = True
             except RuntimeError:
-                # Sampling grids other than 1 or 2 points are merged into lists whose size
-                # depends on the boxes: an adaptive grid of more than 2^15 points per bin, or
-                # a stream that is being captured (the host waits for the size), is refused
-                # there.  The NCHW entry point below takes every grid.
+                # Sampling grids other than 1 or 2 points have their weights in a workspace; where
+                # it cannot be had (a stream that is being captured, a full device) the call is
+                # refused there.  The NCHW entry point below then takes the straightforward kernel.
                 if self.sampling_ratio in (1, 2):
                     raise
                 taken = False
