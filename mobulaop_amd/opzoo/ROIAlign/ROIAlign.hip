@@ -541,13 +541,14 @@ PatchPlan patch_plan(const Problem& p) {
   // at the end).  Forward and backward with 4 and with 12, us: 126 patches times channel blocks of 2592 boxes (1 x 456 x 137 x
   // 100) 1468 / 1396, 1152 of 1254 (4 x 80 x 41 x 248) 710 / 660, 770 of 482 (7 x 160 x 82 x 18) 286 / 296, 720 of 100 (3 x 81 x
   // 75 x 113) 72 / 83, 5472 of 413 (4 x 256 x 148 x 131) 530 / 660, 576 of 671 (1 x 72 x 93 x 243) 190 / 169, 324 of 1295 (2 x 176 x
-  // 70 x 33) 337 / 220, 112 of 325 (4 x 32 x 49 x 56) 276 / 158, 120 of 736 (5 x 64 x 28 x 44) 405 / 208.
+  // 70 x 33) 337 / 220, 112 of 325 (4 x 32 x 49 x 56) 276 / 158, 120 of 736 (5 x 64 x 28 x 44) 405 / 208; 600 of 107 boxes an image
+  // 117 / 126, 600 of 6 54 / 69, 576 of 5 35 / 48, 580 of 44 55 / 67, but 630 of 529 173 / 160, 350 of 221 82 / 71, 216 of 33 56 / 46.
   // Two where patches are many and the boxes of an image few, so that each reaches few patches (with 4 and with 2): 8400 of 23
   // boxes in 3 images (3 x 421 x 196 x 116) 148 / 117, 4830 of 179 in 5 (5 x 64 x 178 x 331) 76 / 61, 6510 of 486 in 7 (7 x 144 x 242
   // x 81) 147 / 123, 1512 of 57 in 3 (3 x 280 x 59 x 101) 95 / 86; but 1632 of 279 in 8 (8 x 40 x 44 x 266) 90 / 98, 840 of 33 in 7
   // (7 x 128 x 79 x 43) 46 / 48, 5472 of 1651 in 4 530 / 564.
   plan.waves = forced ? static_cast<int>(option)
-               : plan.blocks <= 640 || (plan.blocks <= 2048 && p.R >= 8 * patches) ? 12
+               : plan.blocks <= 320 || (plan.blocks <= 640 && p.R >= 160 * p.N) || (plan.blocks <= 2048 && p.R >= 8 * patches) ? 12
                : plan.blocks >= 1280 && 64 * p.R <= p.N * plan.blocks ? 2 : 4;
   return plan;
 }
