@@ -484,9 +484,9 @@ auto owner_kernel(int nsplit) {
                              : roialign::backward_blocked_kernel<NHWC, T, 1>;
 }
 
-// Fixed sampling grids up to kSearchedGrid points, and adaptive ones (where there is no room for the weights of
-// either the call fails: this path has no other kernel to fall back on).  The last line also keeps a box's dy within the
-// 32-bit byte offsets of both kernels.
+// Any sampling grid the lists take: fixed ones up to kSearchedGrid points, adaptive ones
+// (whether an adaptive one is small enough to merge depends on the boxes; if not the call
+// fails: this path has no other kernel to fall back on).
 bool nhwc_backward_supported(const Problem& p) {
   return roialign::backward_blocked_supports(p.PH, p.PW, p.S) && p.S <= roialign::kSearchedGrid &&
          p.C % 4 == 0 &&
