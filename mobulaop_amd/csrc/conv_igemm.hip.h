@@ -22,16 +22,11 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "conv_geometry.h"
+
 namespace conv {
 
 typedef float float16v __attribute__((ext_vector_type(16)));
-
-struct Geometry {
-  int N, C, H, W;        // input
-  int D, KH, KW;         // filters
-  int OH, OW;            // output
-  int pad_h, pad_w, stride_h, stride_w, dil_h, dil_w;
-};
 
 struct Tile {
   static constexpr int BM = 128, BN = 128, BK = 16;

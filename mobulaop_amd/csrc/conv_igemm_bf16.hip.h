@@ -520,16 +520,12 @@ struct ForwardOpsB16 : GatheredB16<FORM> {
 // dx[img, c, ih, iw] = sum over (d, kh, kw) of W[d, c, kh, kw] * dy[img, d, oh, ow]
 // with oh * stride = ih + pad - kh * dil (and likewise for columns).
 //
-// STRIDED: columns are numbered by phases of the strides: the pixels y + i * stride_h, x + j * stride_w of all images, made up
-// to whole tiles, then those of the next phase.  They meet the same taps (every dkh'th row of the filter from kh on, every
-// dkw'th column from kw on, none at worst), at dy's pixels i + oy - t * ch, j + ox - u * cw, so K runs over these alone and a
-// strided product costs what its output pixels do.  (With all taps for every pixel and zeros where one falls between output
+// STRIDED: columns are numbered by phases of the strides (conv_geometry.h), the pixels of a phase in all images made up to whole
+// tiles, then those of the next.  They meet the same taps, so K runs over these alone and a strided product costs what its
+// output pixels do.  (With all taps for every pixel and zeros where one falls between output
 // pixels, and now: 96 filters 5 x 5 at stride 2 over 19 x 64 x 196 x 182, one part, 339 and 148 us; both gradients of 80 over 17 x
 // 96 x 130 x 175, two parts, 622 and 355, of 120 over 1 x 214 x 175 x 217, one part, 167 and 81.)  Unit strides would be one
 // phase with all taps; in the one code for both they took 2 to 4 % more.
-constexpr int kMostPhases = 16;   // products of larger strides take all taps (phases == 0)
-struct PhaseOfDx { int first, rows, cols, y, x, kh, kw, nkh, nkw, oy, ox; };   // first: column; rows x cols pixels of an image
-struct PhaseSteps { int dkh, dkw, ch, cw; };
 template <int FORM, bool STRIDED>
 struct BackwardDataOpsB16;
 

@@ -8,7 +8,6 @@
 // (opzoo/Convolution/Convolution.py:17-57), computed on the matrix cores
 // without a column buffer.
 #include <algorithm>
-#include <numeric>
 #include <type_traits>
 #include <vector>
 
@@ -429,59 +428,21 @@ struct ForwardB16 {
   }
 };
 
-// The phases of a data gradient's columns (conv::BackwardDataOpsB16), those with most taps first; returns the pixels of an
-// image in the smallest.
+// A data gradient's columns; returns the pixels of an image that are neighbours among them at least.
 template <int FORM>
-int plan_phases(conv::BackwardDataOpsB16<FORM, false>* data, const conv::Geometry& g) {
+int plan_columns(conv::BackwardDataOpsB16<FORM, false>* data, const conv::Geometry& g) {
   data->Ncols = g.N * g.H * g.W;
   return g.H * g.W;
 }
 template <int FORM>
-int plan_phases(conv::BackwardDataOpsB16<FORM, true>* data, const conv::Geometry& g) {
-  const int sh = g.stride_h, sw = g.stride_w;
-  data->phases = 0;
-  data->by = conv::PhaseSteps{1, 1, g.dil_h, g.dil_w};
-  data->Ncols = g.N * g.H * g.W;
-  const long long columns = static_cast<long long>(g.N) * g.H * g.W + conv::kMostPhases * 256;
-  // (a single tap: nothing to leave out but zeros, whose pixels are then written apart from their neighbours; 106 filters 1 x 1
-  // at stride 2 over 17 x 142 x 61 x 74, two parts, the step 111.9 us and 113.3)
-  if (static_cast<long long>(sh) * sw > conv::kMostPhases || columns >= (1ll << 31) || g.KH * g.KW == 1) return g.H * g.W;
-  data->by = conv::PhaseSteps{sh / std::gcd(sh, g.dil_h), sw / std::gcd(sw, g.dil_w), g.dil_h / std::gcd(sh, g.dil_h),
-                              g.dil_w / std::gcd(sw, g.dil_w)};
-  // of the taps along an axis that meet the pixels at `at` the first, and how many there are
-  auto taps = [](int at, int pad, int dil, int stride, int step, int K, int* first) {
-    for (int k = 0; k < std::min(step, K); ++k)
-      if ((at + pad - k * dil) % stride == 0) { *first = k; return (K - k + step - 1) / step; }
-    *first = 0;
-    return 0;
-  };
-  std::vector<conv::PhaseOfDx> all;
-  for (int y = 0; y < std::min(sh, g.H); ++y)
-    for (int x = 0; x < std::min(sw, g.W); ++x) {
-      conv::PhaseOfDx f{};
-      f.y = y; f.x = x; f.rows = (g.H - y + sh - 1) / sh; f.cols = (g.W - x + sw - 1) / sw;
-      f.nkh = taps(y, g.pad_h, g.dil_h, sh, data->by.dkh, g.KH, &f.kh);
-      f.nkw = taps(x, g.pad_w, g.dil_w, sw, data->by.dkw, g.KW, &f.kw);
-      if (f.nkh == 0 || f.nkw == 0) f.nkh = f.nkw = 0;
-      f.oy = (y + g.pad_h - f.kh * g.dil_h) / sh; f.ox = (x + g.pad_w - f.kw * g.dil_w) / sw;
-      all.push_back(f);
-    }
-  std::stable_sort(all.begin(), all.end(),
-                   [](const conv::PhaseOfDx& a, const conv::PhaseOfDx& b) { return a.nkh * a.nkw > b.nkh * b.nkw; });
-  int least = g.H * g.W;
-  for (const conv::PhaseOfDx& f : all) least = std::min(least, f.rows * f.cols);
-  // (a tile spans more images where phases have few pixels of each: their byte offsets must stay below 2^31, see plan_gather_b16)
-  const long long image_bytes = static_cast<long long>(g.OH) * g.OW * padded_channels<FORM>(g.D) * 2;
-  if ((255 / least + 2 + (conv::kParts<FORM> > 1 ? static_cast<long long>(conv::kParts<FORM>) * g.N : 0)) * image_bytes >= (1ll << 31))
-    return g.H * g.W;
-  int at = 0;
-  for (conv::PhaseOfDx f : all) {
-    f.first = at;
-    data->phase[data->phases++] = f;
-    at += (g.N * f.rows * f.cols + 255) / 256 * 256;
-  }
-  data->Ncols = at;
-  return least;
+int plan_columns(conv::BackwardDataOpsB16<FORM, true>* data, const conv::Geometry& g) {
+  const conv::PhasePlan plan =
+      conv::plan_phases(g, static_cast<long long>(g.OH) * g.OW * padded_channels<FORM>(g.D) * 2, conv::kParts<FORM>);
+  data->phases = plan.phases;
+  data->by = plan.by;
+  data->Ncols = plan.columns;
+  std::copy(plan.phase, plan.phase + plan.phases, data->phase);
+  return plan.least;
 }
 
 template <int FORM, bool STRIDED>
@@ -514,7 +475,7 @@ struct BackwardB16 {
     }
     if (!with_dx) return kFits;
     data.dx = dx; data.accumulate = accumulate;
-    const int least = plan_phases(&data, g);
+    const int least = plan_columns(&data, g);
     // row m of the left operand is input channel m: element [m][tap][d] = weight[d][m][tap]
     return plan_gather_b16<FORM>(&data, &prep, "conv2d_backward_data", g, w, g.C, g.D, g.N, g.OH * g.OW, least, taps,
                                   g.C * taps);

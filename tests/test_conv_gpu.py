@@ -455,6 +455,26 @@ def test_data_gradient_of_strided_products(case, mode):
         native.set_option('conv_fp32_split', 1)
 
 
+def test_strided_data_gradient_where_phases_reach_too_far():
+    """So many images that the offsets of a phase's tiles would pass 2^31 and those of whole images do not: all taps, walked one
+    by one (tests/test_conv_phases.py has the rule)."""
+    N, C, H, W, D = 21398, 4, 14, 14, 512
+    g = torch.Generator(device='cuda').manual_seed(5)
+    w = torch.randn((D, C, 3, 3), generator=g, device='cuda') * 0.1
+    dy = torch.randn((N, D, 7, 7), generator=g, device='cuda')
+    dx = torch.full((N, C, H, W), float('nan'), device='cuda')
+    native.set_option('conv_compute', 2)
+    try:
+        _call('conv2d_backward_data_ecf81c91', ctypes.c_int(dx.numel()), _ptr(dy), _ptr(w), ctypes.c_int(0),
+              *_ci(N, C, H, W, D, 3, 3, 1, 1, 2, 2, 1, 1), _ptr(dx))
+    finally:
+        native.set_option('conv_compute', 0)
+    assert torch.isfinite(dx).all()
+    for n in (0, 1, N // 2, N - 1):
+        want = torch.nn.grad.conv2d_input((1, C, H, W), w.double().cpu(), dy[n:n + 1].double().cpu(), stride=2, padding=1)
+        _close(dx[n:n + 1], want, 'image %d' % n, 2e-5)   # (two parts: terms to 2^-16 of an operand)
+
+
 def test_errors_surface_as_exceptions():
     x = torch.zeros(1, 1, 4, 4, device='cuda')
     w = torch.zeros(1, 1, 3, 3, device='cuda')
