@@ -69,10 +69,12 @@ patch_weights_kernel(PatchArgs a) {
     const float start = axis ? g.start_w : g.start_h, bin = axis ? g.bin_w : g.bin_h;
     const int P = axis ? a.PW : a.PH, size = axis ? a.W : a.H, grid = axis ? g.grid_w : g.grid_h;
     const float end = start + bin * static_cast<float>(P);
-    // cells that may be touched, a cell to spare (what is not a number may touch every one), in whole patches
-    const float last = static_cast<float>(size - 1);
+    // cells that may be touched, a cell to spare (what is not a number may touch every one), in whole patches.  `far`: a sample
+    // on the map may lie beyond `end` by what both were rounded by, seven halves of a unit of the largest term, which is no larger
+    // than |start| + size.  (None lies before the start.)
+    const float last = static_cast<float>(size - 1), far = 5.0e-7f * (fabsf(start) + static_cast<float>(size));
     int c0 = start > 2.0f ? static_cast<int>(fminf(start, last)) - 2 : 0;
-    int c1 = end < last - 3.0f ? static_cast<int>(fmaxf(end, 0.0f)) + 3 : size - 1;
+    int c1 = end + far < last - 3.0f ? static_cast<int>(fmaxf(end + far, 0.0f)) + 3 : size - 1;
     c0 = max(c0, 0) & ~15; c1 = min(c1 | 15, (axis ? a.wp : a.hp) - 1);
     const bool dense = bin <= 1.0f;
     CellRecord* const to = a.records + static_cast<long long>(r) * (a.hp + a.wp) + (axis ? a.hp : 0);

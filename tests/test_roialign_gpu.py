@@ -1007,6 +1007,55 @@ def test_backward_in_patches(R, C, H, W, pooled, S, scale, dtype, layout, waves)
         native.set_option('roialign_few_boxes', 1)
 
 
+@pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
+@pytest.mark.parametrize('axis', [0, 1])
+@pytest.mark.parametrize('P', [1, 3])
+def test_patches_of_boxes_that_begin_far_off_the_map(P, axis, layout):
+    """A box whose far edge lies on the map and whose start is so far off that its samples' coordinates are rounded to whole
+    cells and more: some lie beyond its edge, and their cells have their part.  (Samples evaluated here, in fp32 and in the
+    order of the reference; the oracle would take all 2^27 of a bin.)"""
+    rng = np.random.default_rng(P)
+    f, R, C, size, other = np.float32, 48, 4, 300, 9
+    start, end = -(10 ** rng.uniform(7.0, 9.2, R)).astype(f), rng.uniform(5, 290, R).astype(f)
+    start[0], end[0] = -9.7e7, 148.8
+    rois = np.zeros((R, 5), f)
+    along, across = (1, 2) if axis else (2, 1)   # (columns of a row of five)
+    rois[:, along], rois[:, along + 2], rois[:, across], rois[:, across + 2] = start, end, 2.25, 3.25
+    dy = rng.standard_normal((R, C, 1, P) if axis else (R, C, P, 1)).astype(f)
+    shape = (1, C, other, size) if axis else (1, C, size, other)
+    want = np.zeros(shape)
+
+    def weights(v, cells):
+        """What samples at v give the cells."""
+        w = np.zeros(cells)
+        v = np.maximum(v[(v >= -1) & (v <= cells)], f(0))
+        low = np.minimum(v.astype(int), cells - 1)
+        part = np.where(low < cells - 1, v - low.astype(f), f(0)).astype(f)
+        np.add.at(w, low, f(1) - part)
+        np.add.at(w, np.minimum(low + 1, cells - 1), part)
+        return w
+    for r in range(R):
+        span = f(end[r] - start[r])
+        step, grid = f(span / f(P)), int(np.ceil(f(span / f(P))))
+        i = np.arange(grid - 4096, grid).astype(f)   # (the last bin's last ones: all that can be on the map)
+        v = f(start[r] + f(f(P - 1) * step)) + ((i + f(0.5)) * step).astype(f) / f(grid)
+        dy[r] *= grid / 256
+        across_weights = weights(f(2.25) + np.array([0.5], f), other)
+        share = weights(v, size) / np.float64(f(grid))
+        plane = np.outer(across_weights, share) if axis else np.outer(share, across_weights)
+        want[0] += dy[r].reshape(C, P)[:, -1].astype(np.float64)[:, None, None] * plane
+    last = layout == 'nhwc'
+    put = lambda a: np.ascontiguousarray(a.transpose(0, 2, 3, 1)) if last else a   # noqa: E731
+    native.set_option('roialign_patch', 4)
+    try:
+        got = (abi.backward_nhwc if last else abi.backward)(
+            abi.to_dev(put(dy)), abi.to_dev(rois), tuple(np.array(shape)[[0, 2, 3, 1]]) if last else shape, 1.0, 0,
+            assign=True).cpu().numpy()
+    finally:
+        native.set_option('roialign_patch', 1)
+    assert_parity(got.transpose(0, 3, 1, 2) if last else got, want.astype(f), BWD_TOL, 'dx')
+
+
 def test_workspace_can_be_given_back():
     """The scratch buffer grows with the largest call of the thread; a caller
     may release it between phases, and the next call allocates afresh."""
