@@ -1056,6 +1056,56 @@ def test_patches_of_boxes_that_begin_far_off_the_map(P, axis, layout):
     assert_parity(got.transpose(0, 3, 1, 2) if last else got, want.astype(f), BWD_TOL, 'dx')
 
 
+@pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
+@pytest.mark.parametrize('pooled', [(7, 7), (2, 3)])
+@pytest.mark.parametrize('S', [3, 0])
+def test_patches_put_what_is_not_finite_where_it_belongs(S, pooled, layout):
+    """One gradient that is not finite, in boxes on and off whole pixels: exactly the cells are lost that a sample of its bin
+    weighs with more than zero (computed from finite gradients).  Boxes that are not numbers, or infinite: the cells that the straightforward
+    kernel loses, no column or row beside them.  All others come out as without them."""
+    N, C, H, W = 1, 4, 40, 37
+    inf, nan = np.inf, np.nan
+    ordinary = [0, 22, 20, 33, 33]
+    rng = np.random.default_rng(1)
+    dy = rng.standard_normal((2, C) + pooled).astype(np.float32)
+    last = layout == 'nhwc'
+
+    def backward(dy, rois):
+        put = (lambda a: np.ascontiguousarray(a.transpose(0, 2, 3, 1))) if last else (lambda a: a)
+        got = (abi.backward_nhwc if last else abi.backward)(abi.to_dev(put(dy)), abi.to_dev(rois),
+                                                            (N, H, W, C) if last else (N, C, H, W), 1.0, S, assign=True)
+        return (got.permute(0, 3, 1, 2) if last else got).cpu().numpy()
+    native.set_option('roialign_patch', 4)
+    native.set_option('roialign_few_boxes', 0)
+    try:
+        for box in ([0, 4, 4, 11, 18], [0, 4.3, 4.2, 20.6, 18.9]):
+            rois = np.array([box, ordinary], np.float32)
+            want = oracle.backward(dy, rois, (N, C, H, W), 1.0, S, impl='ordered')
+            one = np.zeros_like(dy)
+            at = (0, 1, pooled[0] // 2, pooled[1] // 2)
+            one[at] = 1.0
+            lost = oracle.backward(one, rois, (N, C, H, W), 1.0, S, impl='ordered') != 0
+            for bad in (inf, -inf, nan):
+                worse = dy.copy()
+                worse[at] = bad
+                got = backward(worse, rois)
+                assert np.array_equal(np.isfinite(got), ~lost), (box, bad)
+                assert_parity(np.where(lost, 0, got), np.where(lost, 0, want), BWD_TOL, 'the others')
+        for box in ([0, nan, 3, 20, 30], [0, 3, nan, 20, 30], [0, 3, 3, nan, nan], [0, 2, 2, inf, 40], [0, -inf, 3, 20, 30],
+                    [0, -inf, -inf, inf, inf], [0, nan, nan, nan, nan]):
+            rois = np.array([box, ordinary], np.float32)
+            got = backward(dy, rois)
+            abi.set_impl('naive')
+            want = abi.backward(abi.to_dev(dy), abi.to_dev(rois), (N, C, H, W), 1.0, S, assign=True).cpu().numpy()
+            abi.set_impl('auto')
+            finite = np.isfinite(want)
+            assert np.array_equal(np.isfinite(got), finite), box
+            assert_parity(np.where(finite, got, 0), np.where(finite, want, 0), BWD_TOL, str(box))
+    finally:
+        native.set_option('roialign_patch', 1)
+        native.set_option('roialign_few_boxes', 1)
+
+
 def test_workspace_can_be_given_back():
     """The scratch buffer grows with the largest call of the thread; a caller
     may release it between phases, and the next call allocates afresh."""
