@@ -187,9 +187,10 @@ template <typename T> __device__ __forceinline__ float patch_value(float bits) {
 }
 
 // grid: patches x blocks of 32 channels.  dy: [R][C][PH][PW], or NHWC [R][PH][PW][C] (C a multiple of four, 16-byte aligned).
+// flags: 1 dx is overwritten, 2 four elements of dx from any multiple of four of a row (NHWC: of a pixel) on lie in it and aligned.
 template <typename T, bool NHWC, int NW>
 __global__ void __launch_bounds__(NW * 64, 3)
-backward_patch_kernel(const T* __restrict__ dy, PatchArgs pa, T* __restrict__ dx, int C, int tiles_x, int tiles_y, int assign) {
+backward_patch_kernel(const T* __restrict__ dy, PatchArgs pa, T* __restrict__ dx, int C, int tiles_x, int tiles_y, int flags) {
   using K = BwdPatch;
   constexpr int TX = K::TX, TY = K::TY, CR = K::CR, PITCH = K::PITCH;
   constexpr int LOOK = NW == 4 ? 8 : 4, CHUNK = NW * 64 * LOOK;   // boxes looked at at a time, by a thread and by all
@@ -203,6 +204,7 @@ backward_patch_kernel(const T* __restrict__ dy, PatchArgs pa, T* __restrict__ dx
   __shared__ int count_s[LOOK * NW];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int PH = pa.PH, PW = pa.PW, H = pa.H, W = pa.W, R = pa.R;
+  const bool assign = (flags & 1) != 0;
   // neighbouring patches on one XCD
   unsigned id = blockIdx.x;
   {
@@ -487,6 +489,17 @@ backward_patch_kernel(const T* __restrict__ dy, PatchArgs pa, T* __restrict__ dx
   };
   if (busy == 0) {   // nothing to add up: 98 boxes on 6 x 416 x 228 x 193, forward and backward 350 -> 294 us
     if (!assign) return;
+    // Most patches of a large map with a few boxes, and most of the launch: rows of the map, or its pixels, that are whole quads
+    // are written as such.  (Element by element and so, backward of 3 boxes on 7 x 457 x 94 x 188, fp16 68 -> 53 us, fp32 69 -> 56;
+    // of 3 on 4 x 256 x 200 x 336 68 -> 49, 70 -> 53.)
+    if ((flags & 2) != 0) {
+      typedef unsigned quad __attribute__((ext_vector_type(ES)));
+      for (int u = tid; u < TY * TX * K::CH / 4; u += NW * 64) {
+        const int x = x0 + (NHWC ? (u >> 3) & 15 : 4 * (u & 3)), y = y0 + (NHWC ? u >> 7 : (u >> 2) & 7), c = c0 + (NHWC ? 4 * (u & 7) : u >> 5);
+        if (y <= y1 && x <= x1 && c < C) *reinterpret_cast<quad*>(element(y, x, c)) = quad(0u);
+      }
+      return;
+    }
     for (int u = tid; u < TY * TX * K::CH; u += NW * 64) {
       const int x = x0 + (NHWC ? (u >> 5) & 15 : u & 15), y = y0 + (NHWC ? u >> 9 : (u >> 4) & 7), c = c0 + (NHWC ? u & 31 : u >> 7);
       if (y <= y1 && x <= x1 && c < C) *element(y, x, c) = from_float<T>(0.0f);

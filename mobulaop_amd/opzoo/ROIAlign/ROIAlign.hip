@@ -567,8 +567,10 @@ bool launch_patches(const Problem& p, const PatchPlan& plan, const T* dy, const 
                       : plan.waves == 4 ? roialign::backward_patch_kernel<T, NHWC, 4>
                                         : roialign::backward_patch_kernel<T, NHWC, 12>;
   mobula_hip::KernelTimer timer("backward_blocked_kernel", stream);   // (whoever owns dx reports under this name)
+  // (channels-last maps are taken with whole quads of channels only)
+  const bool quads = NHWC || (p.W % 4 == 0 && reinterpret_cast<size_t>(dx) % (4 * sizeof(T)) == 0);
   kernel<<<static_cast<unsigned>(plan.blocks), plan.waves * 64, 0, stream>>>(dy, pa, dx, p.C, plan.tiles_x, plan.tiles_y,
-                                                                             assign ? 1 : 0);
+                                                                             (assign ? 1 : 0) | (quads ? 2 : 0));
   MOBULA_HIP_TRY(hipGetLastError());
   return true;
 }

@@ -1106,6 +1106,39 @@ def test_patches_put_what_is_not_finite_where_it_belongs(S, pooled, layout):
         native.set_option('roialign_few_boxes', 1)
 
 
+@pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16])
+@pytest.mark.parametrize('C,H,W,aligned', [(33, 9, 36, True), (4, 17, 16, True), (40, 8, 37, True), (36, 25, 4, True), (33, 9, 36, False)])
+def test_patches_that_no_box_reaches(C, H, W, aligned, dtype, layout):
+    """They are cleared, four elements at a time where rows allow it, and nothing beside the map is written; a gradient that is
+    added to stays as it is."""
+    last = layout == 'nhwc'
+    if last:
+        C, aligned = (C + 3) // 4 * 4, True
+    N, R, pooled = 3, 2, (2, 3)
+    rois = np.array([[1, 2, 1, 3.5, 4], [1, 0, 3, 2, 5]], np.float32)
+    dy = np.random.default_rng(C).standard_normal((R, C) + pooled).astype(np.float32)
+    want = oracle.backward(torch.from_numpy(dy).to(dtype).float().numpy(), rois, (N, C, H, W), 1.0, 3, impl='ordered')
+    shape, n, pad = ((N, H, W, C) if last else (N, C, H, W)), N * C * H * W, 8 if aligned else 9
+    dyd = torch.from_numpy(dy).to(dtype)
+    dyd = (dyd.permute(0, 2, 3, 1) if last else dyd).contiguous().cuda()
+    native.set_option('roialign_patch', 2)
+    native.set_option('roialign_few_boxes', 0)
+    try:
+        for assign in (True, False):
+            room = torch.full((n + 2 * pad,), 3.0, dtype=dtype, device='cuda')
+            dx = room[pad:pad + n].view(shape)
+            (abi.backward_nhwc if last else abi.backward)(dyd, abi.to_dev(rois), shape, 1.0, 3, dx=dx, assign=assign)
+            got = (dx.permute(0, 3, 1, 2) if last else dx).float().cpu().numpy() - (0.0 if assign else 3.0)
+            assert np.abs(got[[0, 2]]).max() == 0 and np.abs(got[1, :, 8:]).max(initial=0) == 0
+            # (fp16: half a unit of 3 is 2^-10, of a gradient of about one)
+            assert_parity(got, want, 2 * FP16_TOL if dtype == torch.float16 else BWD_TOL, 'assign=%s' % assign)
+            assert (room[:pad] == 3.0).all() and (room[pad + n:] == 3.0).all()
+    finally:
+        native.set_option('roialign_patch', 1)
+        native.set_option('roialign_few_boxes', 1)
+
+
 def test_workspace_can_be_given_back():
     """The scratch buffer grows with the largest call of the thread; a caller
     may release it between phases, and the next call allocates afresh."""
