@@ -442,11 +442,12 @@ bool plan_tiles(const Problem& p, const float* rois, int th, int tw, bool with_d
   } else {
     roialign::build_lists_kernel<<<static_cast<unsigned>(list_blocks), 256, 0, stream>>>(la);
   }
-  // Few tiles: four workgroups each (one and four, us, both passes: 8 tiles of 512 boxes, 2 x 256 x 64 x 64 77 / 72; 32 of
-  // 7830, 4 x 64 x 29 x 104 bfloat16 channels last, 28 x 28 pooled 1201 / 1153; 50 of 5480, 5 x 448 x 74 x 125 744 / 735; 312 of
-  // 4000, 4 x 256 x 200 x 336 545 / 555).  The option "roialign_tile_groups" names one of the two (tests do).
+  // Few tiles: four workgroups each (one and four, us, both passes: 8 tiles of 512 boxes, 2 x 256 x 64 x 64 77 / 72; 64 of
+  // 6000, 16 x 32 x 64 x 64 119 / 114, of 4000 of 14 x 14, 4 x 256 x 128 x 128 1053 / 1049; 96 of 4000, 6 x 128 x 128 x 128 242 / 243;
+  // 120 of 5000 360 / 360; 128 of 8192 of 14 x 14, 8 x 256 x 128 x 128 2072 / 2095, of 8000, 8 x 64 x 128 x 128 261 / 266, of 300
+  // 141 / 145; 312 of 4000, 4 x 256 x 200 x 336 545 / 555).  The option "roialign_tile_groups" names one of the two (tests do).
   const long long groups = mobula_hip::option("roialign_tile_groups", 0);
-  const bool shared = items <= roialign::kSharedListCap && groups != 1 && (groups == 4 || g.total <= 128);
+  const bool shared = items <= roialign::kSharedListCap && groups != 1 && (groups == 4 || g.total <= 64);
   const auto tile_work = shared ? roialign::build_tile_work_kernel<4> : roialign::build_tile_work_kernel<1>;
   tile_work<<<static_cast<unsigned>(g.total * (shared ? 4 : 1)), roialign::kTileRows * 64, 0, stream>>>(
       plan->boxes, n_items, plan->tile_rois, plan->lists, g, plan->layout, plan->cursors, plan->ranges, plan->entries,
