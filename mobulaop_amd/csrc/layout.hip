@@ -83,7 +83,7 @@ transpose_planes_kernel(const T* __restrict__ src, T* __restrict__ dst, const Tr
 extern "C" void mobula_hip_transpose_planes(const int device_id, const long long planes, const long long rows,
                                             const long long cols, const int elem_bytes, const void* src, void* dst) {
   mobula_hip::begin_call();
-  constexpr long long kMost = 1ll << 24;   // (tiles of 64 x 64 have 32-bit offsets up to here)
+  constexpr long long kMost = 1ll << 24;   // (of the shapes that are weighed 64 x 64 has 32-bit offsets up to here)
   const bool known = device_id >= 0 && planes >= 0 && rows >= 0 && cols >= 0 && rows < kMost && cols < kMost &&
                      planes < (1ll << 31) && (elem_bytes == 2 || elem_bytes == 4);
   const bool any = known && planes > 0 && rows > 0 && cols > 0;

@@ -235,7 +235,6 @@ backward_blocked_kernel(const void* __restrict__ dy_any, TO* __restrict__ dx_any
   const XcdJob job = job_of_xcd(blockIdx.x & 7, blockIdx.x >> 3, cblk, sorted != nullptr ? 1 : (rows + 7) / 8);
   const int cb = job.block;
   long long tile = job.item;
-  if (cb >= cblk) return;
   if (tile >= tg.total * K::BANDS) return;
   static_assert(K::TH == 1 && K::BANDS == kTileRows, "a band is a tile row");
   WorkRange wr;

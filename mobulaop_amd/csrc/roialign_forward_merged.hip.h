@@ -148,7 +148,6 @@ forward_merged_kernel(const T* __restrict__ xt, const float* __restrict__ rois,
     const XcdJob job = job_of_xcd(xcd, static_cast<unsigned>(wi), cblk, (static_cast<unsigned>(R) + 7) / 8);
     cb = job.block;
     slot = job.item;
-    if (cb >= cblk) return;
   }
   if (slot >= R) return;
   int ph_first = 0, ph_end = PH;

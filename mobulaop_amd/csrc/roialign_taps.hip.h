@@ -157,7 +157,7 @@ __device__ __forceinline__ void build_lists_body(unsigned block, const ListsArgs
     rec.col_lo = any ? clo : 0; rec.col_hi = any ? chi : -1;
     const int ty0 = rec.row_lo / tg.th, ty1 = any ? rec.row_hi / tg.th : -1;
     const int tx0 = rec.col_lo / tg.tw, tx1 = any ? rec.col_hi / tg.tw : -1;
-    if (lane == 0) boxes[item] = TileBox{any ? g.batch : -1, ty0 | (ty1 << 16), tx0 | (tx1 << 16), roi};
+    if (lane == 0) boxes[item] = TileBox{any ? g.batch : -1, ty0 | (ty1 << 16), tx0 | (tx1 << 16), 0};
     if (!any) return;
   }
   AxisUnit* const base = lists + static_cast<long long>(item) * ll.roi_stride;

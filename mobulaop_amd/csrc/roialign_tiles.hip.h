@@ -17,9 +17,7 @@ struct TileGrid {
   long long total;   // per_image * num_images
 };
 
-// The tiles a ROI touches: image
-// (-1: none), first | last << 16 tile row, first | last << 16 tile column; and
-// the ROI it belongs to.
-struct alignas(16) TileBox { int batch; int ty; int tx; int roi; };
+// The tiles a ROI touches: image (-1: none), first | last << 16 tile row, first | last << 16 tile column.
+struct alignas(16) TileBox { int batch; int ty; int tx; int unused; };
 
 }  // namespace roialign

@@ -485,9 +485,9 @@ auto owner_kernel(int nsplit) {
                              : roialign::backward_blocked_kernel<NHWC, T, 1>;
 }
 
-// Any sampling grid the lists take: fixed ones up to kSearchedGrid points, adaptive ones
-// (whether an adaptive one is small enough to merge depends on the boxes; if not the call
-// fails: this path has no other kernel to fall back on).
+// Sampling grids of one and two points go through lists, others through patches: fixed ones up to kSearchedGrid points, and adaptive
+// ones whatever the boxes.  Without room for the lists or the patches' weights the call fails: this path has no other kernel
+// to fall back on.
 bool nhwc_backward_supported(const Problem& p) {
   return roialign::backward_blocked_supports(p.PH, p.PW, p.S) && p.S <= roialign::kSearchedGrid &&
          p.C % 4 == 0 &&
