@@ -30,6 +30,7 @@ def _announce(request):
     print('\n[case] {}'.format(request.node.nodeid), flush=True)
     yield
     abi.set_impl('auto')
+    native.set_option('roialign_few_boxes', 1)
     native.set_option('roialign_tile_columns', 0)
     native.set_option('roialign_row_split', 0)
     native.set_option('roialign_row_quads', 1)
@@ -265,8 +266,8 @@ def test_both_tile_widths_of_the_backward(cfg, down, columns, split, quads):
 @pytest.mark.parametrize('columns', [16, 20, 36, 60, 64, 0])
 @pytest.mark.parametrize('W', [5, 16, 61, 64, 65, 128])
 def test_every_kind_of_tile_width_of_the_backward(W, columns, split, S):
-    """Tiles as wide as the map, narrower than a window of merged weights and the dummies beside it take in all, cut so that
-    the last one has a column, or chosen by the map."""
+    """Tiles as wide as the map, as narrow as they come, cut so that the last one has a column, or chosen by the map (and
+    patches, which have none)."""
     abi.set_impl('tiled')
     native.set_option('roialign_tile_columns', columns)
     native.set_option('roialign_row_split', split)
@@ -398,10 +399,9 @@ def test_tiled_backward_beyond_two_gib_of_blocked_gradient():
 @pytest.mark.parametrize('columns', [56, 28])
 @pytest.mark.parametrize('S', [0, 3, 4, 5, 7, 65])
 def test_tiled_backward_with_larger_sampling_grids(S, columns):
-    """Sampling grids other than 1 or 2 points per bin are merged for the tiled
-    backward: one weight per row and per column a bin touches, the columns in
-    windows of seven cells (S = 0 gives every ROI its own grid; a fixed grid of
-    65 points is beyond what is merged and takes the plain kernel).
+    """Sampling grids other than 1 or 2 points per bin are gathered in patches from
+    weights per cell (S = 0 gives every ROI its own grid; a fixed grid of
+    65 points is beyond what is taken there and goes to the plain kernel).
     Boxes: tiny, ordinary, wider than the map, partly off the map."""
     abi.set_impl('tiled')
     native.set_option('roialign_tile_columns', columns)
@@ -647,30 +647,135 @@ def test_channels_last_rejects_what_it_does_not_take():
     assert abi.forward_nhwc(torch.zeros(1, 8, 8, 8, device='cuda'), rois, (2, 2), 1.0, 2).shape == (1, 2, 2, 8)
 
 
-def test_a_backward_with_a_dense_grid_can_be_recorded_too():
-    """The merged lists of a dense sampling grid are sized by a number that comes back from
-    the device, which a capturing stream cannot wait for: such a call is recorded with the
-    straightforward kernel (atomic adds: same sums, any order) and the replays give the
-    direct call's result within the tolerance."""
+def _dense_grid_case(S):
+    """Boxes, a gradient and what the oracle makes of them; few boxes go the way of many."""
+    native.set_option('roialign_few_boxes', 0)
     rng = np.random.default_rng(123)
-    N, C, H, W, R, pooled, scale, S = 2, 16, 40, 60, 50, (5, 6), 0.5, 3
+    N, C, H, W, R, pooled, scale = 2, 16, 40, 60, 50, (5, 6), 0.5
     ext = np.array([W / scale, H / scale])
     c = rng.uniform(0, 1, (R, 2)) * ext
     wh = rng.uniform(2, 60, (R, 2))
-    rois = abi.to_dev(np.concatenate([rng.integers(0, N, (R, 1)), c - wh / 2, c + wh / 2], 1).astype(np.float32))
-    dy = abi.to_dev(rng.standard_normal((R, C) + pooled).astype(np.float32))
-    dx = torch.empty((N, C, H, W), device='cuda')
-    want = abi.backward(dy, rois, dx.shape, scale, S, assign=True).clone()   # the tile owners
-    stream = torch.cuda.Stream()
-    graph = torch.cuda.CUDAGraph()
+    rois = np.concatenate([rng.integers(0, N, (R, 1)), c - wh / 2, c + wh / 2], 1).astype(np.float32)
+    dy = rng.standard_normal((R, C) + pooled).astype(np.float32)
+    return abi.to_dev(rois), abi.to_dev(dy), (N, C, H, W), scale, oracle.backward(dy, rois, (N, C, H, W), scale, S, impl='ordered')
+
+
+def _without_workspace():
+    torch.cuda.synchronize()
+    native.unpin_workspace()
+    native.release_workspace()
+
+
+@pytest.mark.parametrize('room', ['grown', 'none'])
+@pytest.mark.parametrize('S', [3, 0])
+def test_a_backward_with_a_dense_grid_can_be_recorded_too(S, room):
+    """The patches' weights lie in the workspace.  After an ordinary call of the shape they have it; where there is none, nothing
+    can be allocated while a stream is being captured: the call is recorded with the straightforward kernel (atomic adds, any
+    order), and the channels-last entry points refuse it."""
+    rois, dy, shape, scale, want = _dense_grid_case(S)
+    N, C, H, W = shape
+    dx = torch.empty(shape, device='cuda')
+    dy_last = dy.permute(0, 2, 3, 1).contiguous()
+    dx_last = torch.empty((N, H, W, C), device='cuda')
+    _without_workspace()
+    if room == 'grown':
+        abi.backward(dy, rois, shape, scale, S, assign=True)
+        torch.cuda.synchronize()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    held = native.workspace_bytes()
     with torch.cuda.graph(graph, stream=stream):
-        abi.backward(dy, rois, dx.shape, scale, S, dx=dx, assign=True, stream=torch.cuda.current_stream().cuda_stream)
-    for replay in range(3):
+        inner = torch.cuda.current_stream().cuda_stream
+        abi.backward(dy, rois, shape, scale, S, dx=dx, assign=True, stream=inner)
+        if room == 'grown':
+            abi.backward_nhwc(dy_last, rois, (N, H, W, C), scale, S, dx=dx_last, assign=True, stream=inner)
+        else:
+            with pytest.raises(RuntimeError, match='channels-last'):
+                abi.backward_nhwc(dy_last, rois, (N, H, W, C), scale, S, dx=dx_last, assign=True, stream=inner)
+    assert native.workspace_bytes() == held and (held > 0) == (room == 'grown')
+    first = None
+    for replay in range(4):
         dx.fill_(7.0)
+        dx_last.fill_(7.0)
         torch.cuda.synchronize()
         graph.replay()
         torch.cuda.synchronize()
-        assert_parity(dx.cpu().numpy(), want.cpu().numpy(), BWD_TOL, 'replay %d' % replay)
+        assert_parity(dx.cpu().numpy(), want, BWD_TOL, 'replay %d' % replay)
+        if room == 'grown':
+            assert_parity(dx_last.permute(0, 3, 1, 2).cpu().numpy(), want, BWD_TOL, 'channels-last, replay %d' % replay)
+            first = dx.clone() if first is None else first
+            assert torch.equal(dx, first)   # (patches add in one order)
+        if room == 'none':   # (an ordinary call between: it makes a workspace of its own)
+            assert_parity(abi.backward(dy, rois, shape, scale, S, assign=True).cpu().numpy(), want, BWD_TOL, 'between')
+    del graph
+    native.unpin_workspace()
+
+
+@pytest.mark.parametrize('S', [3, 0])
+def test_a_recorded_graph_with_a_small_workspace_leaves_dense_grids_their_kernels(S):
+    """A graph of a smaller call holds the workspace where it is: ordinary calls that need a larger one take the
+    straightforward kernel meanwhile, and the channels-last entry points refuse them."""
+    rois, dy, shape, scale, want = _dense_grid_case(S)
+    N, C, H, W = shape
+    _without_workspace()
+    small = (1, 4, 6, 6)
+    small_dy, small_rois, small_dx = dy[:1, :4].contiguous(), rois[:1].clone(), torch.empty(small, device='cuda')
+    small_rois[:, 0] = 0
+    abi.backward(small_dy, small_rois, small, scale, 3, dx=small_dx, assign=True)
+    torch.cuda.synchronize()
+    many, many_dy = rois.repeat(200, 1), dy.repeat(200, 1, 1, 1)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        abi.backward(small_dy, small_rois, small, scale, 3, dx=small_dx, assign=True, stream=torch.cuda.current_stream().cuda_stream)
+    held = native.workspace_bytes()
+    got = abi.backward(many_dy, many, shape, scale, S, assign=True).cpu().numpy()
+    assert native.workspace_bytes() == held > 0
+    assert_parity(got, 200 * want, BWD_TOL, 'many boxes')
+    with pytest.raises(RuntimeError, match='channels-last'):
+        abi.backward_nhwc(many_dy.permute(0, 2, 3, 1).contiguous(), many, (N, H, W, C), scale, S, assign=True)
+    del graph
+    native.unpin_workspace()
+    got = abi.backward(many_dy, many, shape, scale, S, assign=True).cpu().numpy()
+    assert native.workspace_bytes() > held
+    assert_parity(got, 200 * want, BWD_TOL, 'with room')
+
+
+@pytest.mark.parametrize('direct', [True, False])
+@pytest.mark.parametrize('S', [3, 0])
+def test_the_operator_goes_on_where_the_channels_last_entry_point_refuses(S, direct):
+    """Recorded without a workspace, the backward of a channels-last map with a dense grid is tried through the channels-last
+    entry point and taken by the other one."""
+    import mobulaop_amd as mobula
+    mobula.op.load('ROIAlign')
+    rois, dy, shape, scale, want = _dense_grid_case(S)
+    handle = mobula.op.ROIAlign
+    kw = dict(pooled_size=(5, 6), spatial_scale=scale, sampling_ratio=S)
+    g = torch.Generator(device='cuda').manual_seed(2)
+    x = torch.randn(shape, generator=g, device='cuda').contiguous(memory_format=torch.channels_last).requires_grad_()
+    handle(x.detach(), rois, **kw)   # (the direct call is bound with the first one)
+    stream, graph, way = torch.cuda.Stream(), torch.cuda.CUDAGraph(), handle.direct
+    assert way is not None
+    torch.cuda.synchronize()
+    try:
+        if not direct:
+            handle.direct = None
+        with torch.autograd.set_multithreading_enabled(False):   # (this thread's workspace)
+            with torch.cuda.stream(stream):
+                y = handle(x, rois, **kw)
+                torch.autograd.grad(y, x, dy, retain_graph=True)
+            torch.cuda.synchronize()
+            _without_workspace()
+            with torch.cuda.graph(graph, stream=stream):
+                (dx,) = torch.autograd.grad(y, x, dy, retain_graph=True)
+        assert native.workspace_bytes() == 0 and dx.is_contiguous(memory_format=torch.channels_last)
+        for replay in range(3):
+            dx.fill_(7.0)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert_parity(dx.cpu().numpy(), want, BWD_TOL, 'replay %d' % replay)
+    finally:
+        handle.direct = way
+    del graph
     native.unpin_workspace()
 
 
@@ -1438,7 +1543,7 @@ def test_sixteen_bit_gradients_through_the_blocked_copy(dtype, C, pooled, S):
     (2, 64, 100, 64, 400, (7, 7), 2), (1, 4, 5, 7, 3, (2, 3), 2)])
 def test_rows_sorted_by_their_work_give_the_same_gradient(shape, layout):
     """The tile owners in the order of their lists' lengths and in natural order: the same sums bit for bit, with
-    fewer and more than eight channel blocks, rows past the map's end, split rows, windows, boxes off the map."""
+    fewer and more than eight channel blocks, rows past the map's end, split rows, patches (which have no rows to sort), boxes off the map."""
     N, C, H, W, R, pooled, S = shape
     abi.set_impl('tiled')
     rng = np.random.default_rng(R)
@@ -1743,7 +1848,7 @@ def test_partly_copied_maps_of_several_channel_blocks(W, dtype, S):
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize('C,W', [(1, 70), (63, 65), (65, 9), (130, 31), (3, 1)])
 def test_formats_of_channel_counts_that_need_a_conversion(C, W, dtype):
-    """Channels-last maps of counts that no lane takes whole pass through dense copies, tiles of 64 x 64 transposed:
+    """Channels-last maps of counts that no lane takes whole pass through dense copies, transposed tile by tile:
     the values are those of the dense call, bit for bit, in both directions, also from a gradient in either format."""
     import mobulaop_amd as mobula
     mobula.op.load('ROIAlign')
