@@ -22,10 +22,12 @@ struct PhaseSteps { int dkh, dkw, ch, cw; };
 // of an image in the smallest phase.
 struct PhasePlan { int phases; PhaseSteps by; int columns, least; PhaseOfDx phase[kMostPhases]; };
 
+inline PhasePlan plan_all_taps(const Geometry& g) { return PhasePlan{0, {1, 1, g.dil_h, g.dil_w}, g.N * g.H * g.W, g.H * g.W, {}}; }
+
 // image_bytes, parts: of an image of dy in one part, and the parts.
 inline PhasePlan plan_phases(const Geometry& g, long long image_bytes, int parts) {
   const int sh = g.stride_h, sw = g.stride_w;
-  PhasePlan plan{0, {1, 1, g.dil_h, g.dil_w}, g.N * g.H * g.W, g.H * g.W, {}};
+  PhasePlan plan = plan_all_taps(g);
   const long long columns = static_cast<long long>(g.N) * g.H * g.W + kMostPhases * 256;
   // (a single tap: nothing to leave out but zeros, whose pixels are then written apart from their neighbours; 106 filters 1 x 1
   // at stride 2 over 17 x 142 x 61 x 74, two parts, the step 111.9 us and 113.3)

@@ -415,7 +415,7 @@ constexpr int kFarOutside = -(1 << 30);
 
 // Where a lane loads from.  A load instruction moves 1 KB into LDS, lane l to byte 16 * l of it: 32 rows of 32 bytes.
 // Operand functors of igemm_tile_b16:
-//   UNITS, kPixels: units of a K step; whether K runs over pixels (rows of LDS are pixels then);
+//   UNITS, kPixels, kStrided: units of a K step; whether K runs over pixels (rows of LDS are pixels then); whether columns have phases;
 //   k_steps(), k_steps_at(n0): of the longest sums, and of the columns from n0 on;
 //   Lane lane(m0, n0, s, wave): a lane's state before K step s; next(lane): one step on;
 //   a_buffer() / a_at(lane, unit) / a_from(lane, s, live, unit, m): the left operand, the lane's byte offset, and the
@@ -433,7 +433,7 @@ struct StepCursor { int kh, kw, cb; };
 template <int FORM_>
 struct GatheredB16 {
   static constexpr int FORM = FORM_, PARTS = kParts<FORM>, UNITS = kUnits<FORM>, BLOCKS = FORM == 1 ? 2 : 1;   // channel blocks of a step
-  static constexpr bool kPixels = false;
+  static constexpr bool kPixels = false, kStrided = false;
   const unsigned short* __restrict__ wp;    // [K steps][UNITS][mpad][16]
   const unsigned short* __restrict__ src;   // [PARTS][images][cpad / 16][pixels][16]
   Geometry g; int M, Ncols, cpad, mpad;
@@ -578,7 +578,9 @@ struct BackwardDataOpsB16<FORM, true> : GatheredB16<FORM> {
   using Base = GatheredB16<FORM>;
   using Base::g; using Base::M; using Base::Ncols; using Base::cpad; using Base::mpad;
   float* __restrict__ dx; int accumulate;
+  static constexpr bool kStrided = true;
   int phases; PhaseSteps by; PhaseOfDx phase[kMostPhases];
+  int pieces_of_all, longest_of_all;   // with phases, how the product of all taps would be cut: see split_b16 (0: not looked at)
   struct Cursor { int kh, kw, cb, step; };   // tap of the phase, channel block, step of the weights
   struct Lane { Cursor k; int nkh, nkw, anchor, ihp, iwp; };   // (a column past the last: ihp far outside)
   struct Column { float* p; bool ok; };
@@ -688,7 +690,7 @@ struct BackwardDataOpsB16<FORM, true> : GatheredB16<FORM> {
 template <int FORM_>
 struct WeightGradOpsB16 {
   static constexpr int FORM = FORM_, PARTS = kParts<FORM>, UNITS = kUnits<FORM>, STEP = FORM == 1 ? 32 : 16;   // pixels of a step
-  static constexpr bool kPixels = true;
+  static constexpr bool kPixels = true, kStrided = false;
   const unsigned short* __restrict__ dys;   // [PARTS][N][dblocks][OH * OW][16]
   const unsigned short* __restrict__ xs;    // [PARTS][N][cblocks][H * W][16]
   float* __restrict__ dw;
@@ -974,7 +976,10 @@ __device__ __forceinline__ void igemm_tile_b16(const Ops& ops, int m0, int n0, i
   // Halves: the sums of the heads' products move into `total` after sixteen steps (eight where the sum is short: 1.30e-7 ->
   // 1.20e-7 over 25 steps); of two wavefronts on a SIMD one does so half a chunk before the other, which multiplies
   // meanwhile.  (In the loop's one body: a second one for the step that moves them spilled, 417 against 340 us.)
-  const int chunk = s_end - s_begin < 64 ? 8 : 16;
+  // (phases: of the steps of all taps most are zeros; dx at stride 2, all taps / phases in chunks of 16 / of four and eight: 6 x 96 x
+  // 30 x 30, 192 filters 5 x 5 1.10 / 1.16 / 1.09e-7, 20 x 432 x 17 x 22, 448 5 x 5 1.36 / 1.45 / 1.33e-7)
+  int chunk = s_end - s_begin < 64 ? 8 : 16;
+  if constexpr (Ops::kStrided) chunk = ops.phases == 0 ? chunk : s_end - s_begin < 112 ? 4 : 8;
   int s_move = s_begin + (wave < WAVES / 2 ? chunk : chunk / 2);
   for (int s = s_begin; s < s_end; ++s) {
     if constexpr (HALVES) {
@@ -1094,7 +1099,7 @@ __device__ __forceinline__ void igemm_block_b16(const Ops& ops, const TilesB16& 
   if (Ops::FORM == kHalves ? !tiles.range.halves_hold() : tiles.range.leaves_split()) return;
   const TileSplit& split = tiles.split;
   const int whole_blocks = tile_blocks(split.whole);
-  int t, s_begin = 0, s_end = 1 << 30;
+  int t, s_begin = 0, at = 0;
   float* piece = nullptr;
   if (block < whole_blocks) {
     t = tile_of_block(split.whole, block);
@@ -1102,12 +1107,16 @@ __device__ __forceinline__ void igemm_block_b16(const Ops& ops, const TilesB16& 
   } else {
     const int q = block - whole_blocks;
     t = split.whole + q / split.pieces;
-    s_begin = (q % split.pieces) * split.steps_per_piece;
-    s_end = s_begin + split.steps_per_piece;
+    at = q % split.pieces;
     piece = tiles.piece_buffer + static_cast<size_t>(q) * S::ROWS * S::COLS;
   }
   const int m0 = (t % tiles.row_tiles) * S::ROWS, n0 = (t / tiles.row_tiles) * S::COLS;
-  s_end = min(s_end, ops.k_steps_at(n0));
+  int s_end = ops.k_steps_at(n0);
+  if (piece != nullptr) {   // (the columns of a short phase are cut like those of the longest: into shorter pieces, not into fewer)
+    const int length = Ops::kStrided ? (s_end + split.pieces - 1) / split.pieces : split.steps_per_piece;
+    s_begin = at * length;
+    s_end = min(s_end, s_begin + length);
+  }
   igemm_tile_b16<Ops, S>(ops, m0, n0, s_begin, s_end, piece, lds);   // (no steps: zeros)
 }
 template <typename Ops, typename S>

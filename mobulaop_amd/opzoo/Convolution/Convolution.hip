@@ -116,7 +116,11 @@ int resident_workgroups_b16() {
 }
 
 // How a bf16 product is cut into tiles of shape S and, where that is faster, the last round's along K; about
-// how long it takes (us).
+// how long it takes (us).  A strided data gradient in phases is cut into as many pieces as that of all taps would be: it is short
+// enough to be fastest in one go, and its sums would then be up to four times as long as they were with all taps (errors against
+// 64 bits, all taps / phases in one go / so, and us: 24 x 384 x 13 x 13, 500 filters 3 x 3 at stride 2, three parts 0.96 / 2.17 /
+// 0.96e-7, 177 / 163 / 131; 20 x 432 x 17 x 22, 448 5 x 5, three parts 2.24 / 3.24 / 2.24e-7, 475 / 267 / 265; 16 x 128 x 28 x 28, 512 3 x 3,
+// halves 1.08 / 1.34 / 1.07e-7, 93 / 92 / 88).
 template <typename Ops, typename S>
 conv::TileSplit split_b16(const Ops& ops, double* cost) {
   const int row_tiles = (ops.M + S::ROWS - 1) / S::ROWS, count = row_tiles * ((ops.Ncols + S::COLS - 1) / S::COLS);
@@ -132,13 +136,26 @@ conv::TileSplit split_b16(const Ops& ops, double* cost) {
     return step * (length + 2) * (workgroups <= cus && S::PER_CU == 2 ? 1.33 : static_cast<double>((workgroups + cus - 1) / cus));
   };
   const conv::TileSplit whole{count, 1, steps}, cut = split_tiles(count, steps, resident, room);
-  const double whole_time = time(count, ops.mean_steps());
-  const int rest = count - cut.whole, pieces = rest * cut.pieces;
+  // (of tiles that all run at once the longest counts)
+  const double whole_time = time(count, count <= cus ? steps : ops.mean_steps());
   // pieces are written and read again at some 4 TB/s, and added up by a kernel of their own
-  const double cut_time = (cut.whole > 0 ? time(cut.whole, ops.mean_steps()) : 0.0) + time(pieces, cut.steps_per_piece) +
-                          static_cast<double>(pieces) * S::ROWS * S::COLS * 8 / 4e6 + 5.0;
-  const bool cut_wins = rest > 0 && cut_time < whole_time;
-  if (cost != nullptr) *cost = cut_wins ? cut_time : whole_time;
+  auto cut_time = [&](const conv::TileSplit& split) {
+    const int pieces = (count - split.whole) * split.pieces;
+    return (split.whole > 0 ? time(split.whole, ops.mean_steps()) : 0.0) + time(pieces, split.steps_per_piece) +
+           static_cast<double>(pieces) * S::ROWS * S::COLS * 8 / 4e6 + 5.0;
+  };
+  if constexpr (Ops::kStrided) {
+    const int pieces = std::min(std::min(ops.pieces_of_all, steps), room / std::max(count, 1));
+    if (pieces > 1) {
+      const int length = (steps + pieces - 1) / pieces;
+      conv::TileSplit apart{0, (steps + length - 1) / length, length};
+      if (cut.whole == 0 && cut.pieces >= apart.pieces && cut_time(cut) < cut_time(apart)) apart = cut;
+      if (cost != nullptr) *cost = cut_time(apart);
+      return apart;
+    }
+  }
+  const bool cut_wins = count > cut.whole && cut_time(cut) < whole_time;
+  if (cost != nullptr) *cost = cut_wins ? cut_time(cut) : whole_time;
   return cut_wins ? cut : whole;
 }
 
@@ -181,6 +198,9 @@ PlanB16 plan_b16(const Ops& ops) {
   }
   weigh_rows<Ops, 128>(ops, &best);
   weigh_rows<Ops, 64>(ops, &best);
+  // (in K steps of all taps, so that short_sums chooses as it does for them: by its own terms 6 x 96 x 30 x 30, 192 filters 5 x 5 at
+  // stride 2 went to three parts, 109 us and 1.03e-7, instead of halves, 71 and 1.09)
+  if constexpr (Ops::kStrided) best.longest = ops.longest_of_all > 0 ? ops.longest_of_all : best.longest;
   return best;
 }
 template <typename Ops>
@@ -435,14 +455,17 @@ int plan_columns(conv::BackwardDataOpsB16<FORM, false>* data, const conv::Geomet
   return g.H * g.W;
 }
 template <int FORM>
-int plan_columns(conv::BackwardDataOpsB16<FORM, true>* data, const conv::Geometry& g) {
-  const conv::PhasePlan plan =
-      conv::plan_phases(g, static_cast<long long>(g.OH) * g.OW * padded_channels<FORM>(g.D) * 2, conv::kParts<FORM>);
+int plan_columns(conv::BackwardDataOpsB16<FORM, true>* data, const conv::PhasePlan& plan) {
+  data->pieces_of_all = data->longest_of_all = 0;
   data->phases = plan.phases;
   data->by = plan.by;
   data->Ncols = plan.columns;
   std::copy(plan.phase, plan.phase + plan.phases, data->phase);
   return plan.least;
+}
+template <int FORM>
+int plan_columns(conv::BackwardDataOpsB16<FORM, true>* data, const conv::Geometry& g) {
+  return plan_columns(data, conv::plan_phases(g, static_cast<long long>(g.OH) * g.OW * padded_channels<FORM>(g.D) * 2, conv::kParts<FORM>));
 }
 
 template <int FORM, bool STRIDED>
@@ -477,8 +500,24 @@ struct BackwardB16 {
     data.dx = dx; data.accumulate = accumulate;
     const int least = plan_columns(&data, g);
     // row m of the left operand is input channel m: element [m][tap][d] = weight[d][m][tap]
-    return plan_gather_b16<FORM>(&data, &prep, "conv2d_backward_data", g, w, g.C, g.D, g.N, g.OH * g.OW, least, taps,
-                                  g.C * taps);
+    const Fit fit = plan_gather_b16<FORM>(&data, &prep, "conv2d_backward_data", g, w, g.C, g.D, g.N, g.OH * g.OW, least, taps,
+                                          g.C * taps);
+    if constexpr (STRIDED && FORM != 1) {   // (one part: its operands' rounding hides the sums')
+      if (fit == kFits && data.phases != 0) {
+        conv::BackwardDataOpsB16<FORM, true> all = data;
+        plan_columns(&all, conv::plan_all_taps(g));
+        const PlanB16 of_all = plan_b16(all);
+        data.longest_of_all = of_all.longest;
+        data.pieces_of_all = (all.k_steps() + of_all.longest - 1) / std::max(of_all.longest, 1);
+        // A few images' phases, each made up to a tile, may take more than all taps do.  (Not with two parts, whose operands may
+        // hold infinities: times zero they are lost to other phases.  Those go in one go, 4.46e-6 off instead of 4.43.)
+        if (plan_b16(data).cost >= of_all.cost) {
+          if (FORM == 2) data.longest_of_all = data.pieces_of_all = 0;
+          else data = all;
+        }
+      }
+    }
+    return fit;
   }
   char* place(char* at) {
     at = place_blocked(&prep.first, dy_bytes, at);

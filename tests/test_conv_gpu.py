@@ -415,7 +415,9 @@ def test_bf16_mode_is_exact_on_bf16_valued_operands(case):
     (300, 16, 3, 2, 20, (2, 2), (1, 0), (4, 2), (1, 1)),    # fewer rows than phases; a tile spans hundreds of images
     (1, 130, 40, 37, 20, (7, 7), (3, 3), (4, 4), (1, 1)),   # sixteen phases, the most
     (2, 18, 30, 30, 20, (6, 5), (2, 2), (5, 4), (1, 1)),    # twenty: all taps
-    (1, 600, 16, 16, 600, (3, 3), (1, 1), (2, 2), (1, 1)),  # cut along K: pieces past the end of a phase's
+    (1, 600, 16, 16, 600, (3, 3), (1, 1), (2, 2), (1, 1)),  # cut along K; few pixels, all taps with three parts and halves
+    (4, 40, 40, 41, 130, (3, 3), (1, 1), (2, 2), (1, 1)),   # cut along K: phases of 36, 18 and nine steps into as many pieces
+    (9, 33, 45, 38, 44, (5, 5), (2, 2), (2, 2), (1, 1)),
 ])
 def test_data_gradient_of_strided_products(case, mode):
     """Every phase of the strides with its own taps, against the products of the same operands in 64 bits; what the gradient
@@ -914,6 +916,7 @@ def _errors_of_both_ways(shape):
     (2, 48, 23, 17, 64, (3, 3), (1, 1), (2, 2), (1, 1)),     # dx: 64 to 256 terms
     (4, 64, 24, 28, 256, (3, 3), (1, 1), (1, 1), (1, 1)),
     (2, 256, 20, 21, 130, (5, 5), (2, 2), (1, 1), (1, 1)),
+    (24, 384, 13, 13, 500, (3, 3), (1, 1), (2, 2), (1, 1)),   # dx: phases, whose sums are cut as those of all taps would be
 ])
 def test_sums_of_parts_are_no_further_off_than_the_fp32_kernels(shape, split_always):
     for parts, fp32, what in zip(*_errors_of_both_ways(shape), ('y', 'dx', 'dw')):
