@@ -211,7 +211,7 @@ struct BlockedJob {
   unsigned tiles_p, tiles_c, blocks;   // workgroups: (pixels / 64) x (channels / 64) x images
 };
 
-constexpr int kPrepLdsWords = 64 * 65;   // what a job of prepare_b16_kernel finds in LDS
+constexpr int kPrepLdsWords = 64 * 65 + 4;   // what a job of prepare_b16_kernel finds in LDS
 
 template <int FORM, bool VEC>
 __device__ __forceinline__ void to_blocked(const BlockedJob& job, unsigned block, float* lds, const TensorWords& words) {
@@ -221,34 +221,36 @@ __device__ __forceinline__ void to_blocked(const BlockedJob& job, unsigned block
   const float* const src = job.src;
   unsigned short* const dst = job.dst;
   unsigned seen = 0u, odd = 0u;   // odd: bit 8 * k + j of what follows
-  const unsigned row = block / job.tiles_p;
-  const int n = row / job.tiles_c, c0 = (row - n * job.tiles_c) * 64, p0 = (block - row * job.tiles_p) * 64;
-  const float* in = src + static_cast<size_t>(n) * C * P;
-  // All loads first, without branches (an address for every lane: what lies past the tensor is cleared afterwards).  A guarded
-  // load each before its own store to LDS left one load in flight, four or sixteen round trips to memory a workgroup (x, dy and x
-  // of 13 x 364 x 163 x 163, 57 filters 1 x 1, one part: 403 -> 325 us, 5 TB/s; of 32 x 256 x 56 x 56, 256 filters: 87 -> 79).
-  constexpr int LOADS = VEC ? 4 : 16;
+  const unsigned row = __builtin_amdgcn_readfirstlane(block / job.tiles_p);
+  const int n = __builtin_amdgcn_readfirstlane(row / job.tiles_c), c0 = (row - n * job.tiles_c) * 64, p0 = (block - row * job.tiles_p) * 64;
+  // All loads first, without branches: what lies past the tensor is loaded from the end of the buffer, which gives zeros and
+  // moves nothing.  A guarded load each before its own store to LDS left one load in flight, four or sixteen round trips to memory
+  // a workgroup (x, dy and x of 13 x 364 x 163 x 163, 57 filters 1 x 1, one part: 403 -> 325 us, 5 TB/s; of 32 x 256 x 56 x 56, 256
+  // filters: 87 -> 79); the last channel in the place of absent ones, a step: 28 x 32 x 160 x 206, 24 filters 1 x 1,
+  // fp32 451 -> 446, 16 x 20 x 160 x 206, 40 3 x 3 593 -> 575.
+  constexpr int LOADS = VEC ? 4 : 16, kNonTemporal = 2;
   typename std::conditional<VEC, f32x4, float>::type v[LOADS];
   const int lane_p = VEC ? 4 * (threadIdx.x & 15) : threadIdx.x & 63, lane_c = VEC ? threadIdx.x >> 4 : threadIdx.x >> 6;
-  const bool on_p = p0 + lane_p < P;
-  const float* const from = in + (on_p ? p0 + lane_p : 0);
+  const unsigned plane = static_cast<unsigned>(P) * 4u, end = min(64, C - c0) * plane;   // (of the tile's channels: below 2^32)
+  const __amdgpu_buffer_rsrc_t in = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(src + (static_cast<size_t>(n) * C + c0) * P), 0, end, 0x00020000);
 #pragma unroll
   for (int k = 0; k < LOADS; ++k) {
-    const float* const at = from + static_cast<size_t>(min(c0 + lane_c + 64 / LOADS * k, C - 1)) * P;
-    if constexpr (VEC) v[k] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(at));
-    else v[k] = *at;
+    const int cl = lane_c + 64 / LOADS * k;
+    const unsigned at = p0 + lane_p < P && c0 + cl < C ? cl * plane + (p0 + lane_p) * 4u : end;
+    if constexpr (VEC) v[k] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(in, at, 0, kNonTemporal));
+    else v[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(in, at, 0, 0));
   }
   const int shift = FORM == kHalves ? words.shift(block == 0) : 0;
   const bool left = FORM == kHalves && words.no_halves();
 #pragma unroll
   for (int k = 0; k < LOADS; ++k) {
     const int cl = lane_c + 64 / LOADS * k;
-    const bool on = on_p && c0 + cl < C;
     if constexpr (VEC) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) tile[cl][lane_p + i] = on ? v[k][i] : 0.0f;
+      for (int i = 0; i < 4; ++i) tile[cl][lane_p + i] = v[k][i];
     } else {
-      tile[cl][lane_p] = on ? v[k] : 0.0f;
+      tile[cl][lane_p] = v[k];
     }
   }
   __syncthreads();
@@ -282,7 +284,17 @@ __device__ __forceinline__ void to_blocked(const BlockedJob& job, unsigned block
       }
     }
   }
-  if (FORM == 3) add_exponents(words.exponents, seen);
+  if (FORM == 3) {
+    // (once a workgroup: all read one word, past the caches; where each of 57696 wavefronts did, they waited for one another longer
+    // than the copy takes, and the more the shorter that was: dy of 28 x 24 x 160 x 206 91 us with loads one by one, 124 with all
+    // first, 69 now)
+    unsigned* const of_waves = reinterpret_cast<unsigned*>(lds + 64 * 65);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) seen |= __shfl_xor(seen, d);
+    if ((threadIdx.x & 63) == 0) of_waves[threadIdx.x >> 6] = seen;
+    __syncthreads();
+    if (threadIdx.x < 64) add_exponents(words.exponents, threadIdx.x < 4 ? of_waves[threadIdx.x] : 0u);
+  }
   if (FORM == kHalves && __any(odd != 0u)) {
     int to = words.reserve(__popc(odd));
     for (; odd != 0u; odd &= odd - 1u) {

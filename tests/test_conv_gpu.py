@@ -923,6 +923,25 @@ def test_sums_of_parts_are_no_further_off_than_the_fp32_kernels(shape, split_alw
         assert parts <= fp32, (what, parts, fp32)
 
 
+@pytest.mark.parametrize('hw', [(8, 16), (11, 13)])
+@pytest.mark.parametrize('channel', [0, 15, 16, 40, 63, 64, 79])
+def test_every_wavefront_of_a_conversion_tells_what_it_found(channel, hw, split_always):
+    """An infinity anywhere in a tile of 64 pixels x 64 channels sends the product to the fp32 kernels, where it stays one (its
+    parts would make it NaN)."""
+    N, C, D = 2, 80, 64
+    g = torch.Generator(device='cuda').manual_seed(97)
+    w = torch.rand(D, C, 1, 1, generator=g, device='cuda') + 0.5
+    y = torch.empty(N, D, *hw, device='cuda')
+    for pixel in 0, 31, 32, 63, hw[0] * hw[1] - 1:
+        x = torch.randn(N, C, *hw, generator=g, device='cuda')
+        x.view(N, C, -1)[1, channel, pixel] = float('inf')
+        _call('conv2d_forward_c6a7aa85', ctypes.c_int(y.numel()), _ptr(x), _ptr(w), _ptr(w), ctypes.c_int(0),
+              *_ci(N, C, *hw, D, 1, 1, 0, 0, 1, 1, 1, 1), _ptr(y))
+        got = y.view(N, D, -1)
+        assert (got[1, :, pixel] == float('inf')).all()
+        assert torch.isfinite(got).sum().item() == got.numel() - D
+
+
 def test_one_product_of_parts_is_within_two_half_units(split_always):
     """What six products of parts leave out of one of fp32 is at most 2^-24 of it, and the result's rounding another
     2^-24 (the fp32 kernels': the rounding alone)."""
