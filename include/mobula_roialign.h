@@ -324,8 +324,8 @@ void mobula_hip_clear_error(void);
  * it, are added from fp32 in 64 bits, up to 128 of a tensor; one with more takes
  * three parts).  Data gradients of strided layers go by the terms of the pixels
  * that meet fewest taps; many take two fp16 parts, 23 bits of an operand where
- * the fp32 kernels have 24, for sums that come out nearer to exact (0.3 to 0.7 of
- * the error).  Tensors with infinities or NaN take the fp32 kernels as a
+ * the fp32 kernels have 24, for sums that come out nearer to exact (0.15 to 0.6
+ * of the error).  Tensors with infinities or NaN take the fp32 kernels as a
  * whole; so do, where three parts are formed, those with subnormals or whose
  * products or sums could come near the ends of the range.  One such element
  * changes the time of its call and the last bits of all of its results, those
