@@ -1163,7 +1163,8 @@ conv::TensorWords tensor_words(char* ws, int t) {
 // Microseconds of the fp32 ways from the CU clocks of their kernels (which know nothing of rounds that are not full)
 // and of what the split ways take besides their products: the passes over the tensors, and the
 // launches that clear words and find nothing to do.  Fitted to some fifty layers of 10 us to 3 ms; of 26 others
-// (profiles/conv2d_parts_or_fp32.txt) a product takes the way that is slower by 12 us or 8 % at most.
+// (profiles/conv2d_parts_or_fp32.txt) a few products of 65 to 100 us take the fp32 kernels where three parts would be faster by 15 us,
+// and some of 70 to 240 us where halves would take two thirds of the time.
 double forward_fp32_us(double clocks) { return clocks / (256 * 2300.0) + 15.0; }
 double data_fp32_us(double clocks, size_t classes) {
   return clocks / (256 * 2300.0) + 15.0 * std::max<size_t>(classes, 1);
